@@ -45,13 +45,32 @@ int check_shape(int64_t N, int64_t W, int32_t H, int32_t D, int32_t nd, int64_t 
     return S3D_OK;
 }
 
+// workspace of a forward call = plan: the sweep kernel's work list, then the tile kernel's where the shape may use it
+size_t fwd_workspace_bytes(int H, int64_t W, int64_t N)
+{
+    return align_up(attn_sweep_workspace_bytes(H, W, N), 256) + attn_tile_list_bytes(H, N, W);
+}
+void *tile_list_of(const AttnArgs &a)
+{
+    return static_cast<char *>(a.workspace) + align_up(attn_sweep_workspace_bytes(a.H, a.W, a.N), 256);
+}
+int launch_fwd(const AttnArgs &a, int dtype, hipStream_t stream, int what)
+{
+    if (!attn_tile_applies(a, dtype)) return launch_attn_sweep(a, dtype, stream, what);
+    if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), stream, what)) return rc;
+    if (!a.sizes_dev) return S3D_OK;
+    AttnArgs b = a;
+    b.leave_to_tiles = 1;
+    return launch_attn_sweep(b, dtype, stream, what);
+}
+
 }  // namespace
 }  // namespace s3d
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_attn_fwd_workspace_bytes(int32_t H, int64_t N, int64_t W)
 {
     if (H < 1 || N < 0 || W < 0) return 0;
-    return s3d::attn_sweep_workspace_bytes(H, W, N);
+    return s3d::fwd_workspace_bytes(H, W, N);
 }
 
 namespace s3d {
@@ -160,19 +179,19 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_fwd(
         return rc;
     if (empty) return S3D_OK;
     a.workspace = workspace;
-    const size_t need = attn_sweep_workspace_bytes(H, W, N);
+    const size_t need = fwd_workspace_bytes(H, W, N);
     if (!workspace || workspace_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_attn_fwd: workspace %zu B < required %zu B",
                     workspace ? workspace_bytes : size_t(0), need);
     // with a plan the work list is in the workspace already
-    return launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream),
-                             (flags & S3D_ATTN_PLANNED) ? kAttnSweep : (kAttnBuildList | kAttnSweep));
+    return launch_fwd(a, dtype, static_cast<hipStream_t>(stream),
+                      (flags & S3D_ATTN_PLANNED) ? kAttnSweep : (kAttnBuildList | kAttnSweep));
 }
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_attn_plan_bytes(int32_t H, int64_t N, int64_t W)
 {
     if (H < 1 || N < 0 || W < 0) return 0;
-    return s3d::attn_sweep_workspace_bytes(H, W, N);
+    return s3d::fwd_workspace_bytes(H, W, N);
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_attn_plan(
@@ -199,12 +218,16 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_plan(
     }
     if (N == 0 || W == 0) return S3D_OK;
     if (!w_sizes || !w2n) return fail(S3D_ERR_NULL_POINTER, "s3d_attn_plan: null device pointer");
-    const size_t need = attn_sweep_workspace_bytes(H, W, N);
+    const size_t need = fwd_workspace_bytes(H, W, N);
     if (!plan || plan_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_attn_plan: plan buffer %zu B < required %zu B", plan ? plan_bytes : size_t(0), need);
     a.w_sizes = w_sizes;
     a.w2n = w2n;
     a.workspace = plan;
+    // both lists where the shape may use either: the plan's caller may keep the table sizes on the device
+    if (D == 16 && attn_tile_shape(N, W, H, dtype == S3D_DTYPE_F32)) {
+        if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
+    }
     return launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream), kAttnBuildList);
 }
 
@@ -223,7 +246,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_fwd_noalloc(
                                    qkv_row_stride, dtype))
         return rc;
     if (empty) return S3D_OK;
-    const size_t need = attn_sweep_workspace_bytes(H, W, N);
+    const size_t need = fwd_workspace_bytes(H, W, N);
     if (need > kScratchBytes)
         return fail(S3D_ERR_WORKSPACE, "s3d_attn_fwd_noalloc: N = %lld voxels in W = %lld windows need %zu B of work "
                     "list, the built-in scratch holds %zu B; use s3d_attn_fwd with a workspace",
@@ -233,5 +256,5 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_fwd_noalloc(
     a.workspace = address;
     // the list kernels write every word of the work list that the sweep kernel reads (the queue counters
     // included), so nothing of an earlier call's contents is used
-    return launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream));
+    return launch_fwd(a, dtype, static_cast<hipStream_t>(stream), kAttnBuildList | kAttnSweep);
 }

@@ -20,12 +20,31 @@ struct AttnArgs {
     void *workspace;                       // the work list: queue counters, unit and window records
     int32_t block_shift;                   // the step target, a lane streams about 2^block_shift keys
     int32_t target_items;                  // wavefronts that serve one head group (sizes the finer units at the list's end)
+    int32_t leave_to_tiles;                // sizes_dev: the tile kernel was launched too and serves sizes that fit it
     int32_t spread_groups;                 // head groups take the workgroups in turn (else in runs of eight)
     int32_t H, D, nd, total_rows;
     int64_t N, W;
     int32_t rows[kMaxAxes];                // rows of each axis table
     int32_t base[kMaxAxes];                // first row of each axis table in the flat table
 };
+
+// Table rows of an axis that the tile kernel takes: of a position axis, of a colour or normal axis.
+constexpr int kTileRows = 64, kTileSignalRows = 32;
+template <typename Rows> __host__ __device__ inline bool rows_fit_tiles(const Rows &rows, int nd)
+{
+    for (int n = 0; n < nd; ++n)
+        if (rows[n] < 1 || rows[n] > (n < 3 ? kTileRows : kTileSignalRows)) return false;
+    return true;
+}
+#ifdef __HIPCC__
+// Rows of axis n by the caller's device tensor of table sizes, clipped so that every axis keeps a row inside the head's
+// table; `run`: rows of the axes before it.
+__device__ __forceinline__ int device_rows(const AttnArgs &a, int n, int nd, int run)
+{
+    const int rows = __builtin_amdgcn_readfirstlane(a.sizes_dev[n]) / (a.H * a.D);
+    return max(1, min(rows, a.total_rows - run - (nd - 1 - n)));
+}
+#endif
 
 // Persistent workgroups, one to three heads each with their table slices in LDS; lane = one query of some window,
 // which streams that window's keys; VALU math (packed fp16 dot products for fp16 I/O), any dtype, windows of any
@@ -35,6 +54,19 @@ size_t attn_sweep_workspace_bytes(int H, int64_t W, int64_t N);
 // work list that is already in a.workspace; the launch leaves it ready for the next one), or both.
 constexpr int kAttnBuildList = 1, kAttnSweep = 2;
 int launch_attn_sweep(const AttnArgs &a, int dtype, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
+
+// The tile kernel (attn_tile.hip): a workgroup works off tiles of up to 64 queries by 64 keys of a head, the table
+// products on the matrix pipe.  `list` is its unit list, attn_tile_list_bytes of device memory.
+// With sizes_dev the host cannot tell whether every axis fits: it launches the tile kernel and the sweep kernel, and each
+// works or returns by what it reads.
+bool attn_tile_shape(int64_t N, int64_t W, int H, bool fp32);
+bool attn_tile_applies(const AttnArgs &a, int dtype);
+size_t attn_tile_list_bytes(int H, int64_t N, int64_t W);
+int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
+
+// host side: a kernel's dynamic-LDS limit (see there), compute units of the current device
+int allow_dynamic_lds(const void *kernel, size_t bytes);
+int device_cus();
 
 // The pair sweeps of the backward on the sweep kernel's work list (built here, in b.f.workspace, which needs
 // attn_sweep_workspace_bytes): dq, dk, dv, and dL, P of every (pair, head) for the table-gradient kernels.

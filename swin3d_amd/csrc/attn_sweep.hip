@@ -25,6 +25,40 @@
 #include <vector>
 
 namespace s3d {
+
+// Raises a kernel's dynamic-LDS limit to `bytes`.  The runtime keeps the limit per function and device, so it is
+// set when a (function, device) pair first needs that much and not again: a call under stream capture then issues
+// kernel launches only (one eager call per shape and device has to come before the capture).
+int allow_dynamic_lds(const void *kernel, size_t bytes)
+{
+    struct Granted { const void *kernel; int device; size_t bytes; };
+    static std::mutex mutex;
+    static std::vector<Granted> granted;
+    int device = 0;
+    S3D_HIP_CHECK(hipGetDevice(&device));
+    std::lock_guard<std::mutex> lock(mutex);
+    for (Granted &g : granted) {
+        if (g.kernel == kernel && g.device == device) {
+            if (g.bytes >= bytes) return S3D_OK;
+            S3D_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+            g.bytes = bytes;
+            return S3D_OK;
+        }
+    }
+    S3D_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+    granted.push_back({kernel, device, bytes});
+    return S3D_OK;
+}
+
+int device_cus()
+{
+    int device = 0, v = 0;
+    if (hipGetDevice(&device) == hipSuccess &&
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && v > 0)
+        return v;
+    return 256;
+}
+
 namespace {
 
 using namespace sweep;
@@ -316,39 +350,6 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
     }
 }
 
-// Raises a kernel's dynamic-LDS limit to `bytes`.  The runtime keeps the limit per function and device, so it is
-// set when a (function, device) pair first needs that much and not again: a call under stream capture then issues
-// kernel launches only (one eager call per shape and device has to come before the capture).
-inline int allow_dynamic_lds(const void *kernel, size_t bytes)
-{
-    struct Granted { const void *kernel; int device; size_t bytes; };
-    static std::mutex mutex;
-    static std::vector<Granted> granted;
-    int device = 0;
-    S3D_HIP_CHECK(hipGetDevice(&device));
-    std::lock_guard<std::mutex> lock(mutex);
-    for (Granted &g : granted) {
-        if (g.kernel == kernel && g.device == device) {
-            if (g.bytes >= bytes) return S3D_OK;
-            S3D_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
-            g.bytes = bytes;
-            return S3D_OK;
-        }
-    }
-    S3D_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
-    granted.push_back({kernel, device, bytes});
-    return S3D_OK;
-}
-
-inline int device_cus()
-{
-    int device = 0, v = 0;
-    if (hipGetDevice(&device) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && v > 0)
-        return v;
-    return 256;
-}
-
 // Workgroup shapes.  A workgroup holds its heads' table slices once, so what fits a CU is set by registers and LDS:
 //   one head per wavefront: four workgroups of four wavefronts per CU at head_dim 8 (one wavefront of each on every
 //     SIMD), three at head_dim 16, two at head_dim 32 (an fp32 query, key, value and output row are 128 registers);
@@ -400,6 +401,12 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
     if (threadIdx.x == 0) group_exited = 0;
     const int H = a.H;
     const int HD = H * D;
+    if (a.leave_to_tiles) {
+        int rows[ND], run = 0;
+#pragma unroll
+        for (int n = 0; n < ND; ++n) run += rows[n] = device_rows(a, n, ND, run);
+        if (rows_fit_tiles(rows, ND)) return;
+    }
     // workgroups go to the XCDs in turn: consecutive runs of eight serve one head group, so every XCD gets every head
     // (or, with many head groups, the head groups take the workgroups in turn: see the launch)
     const int hg = a.spread_groups ? blockIdx.x % (H / HP) : (blockIdx.x / kQueues) % (H / HP);
@@ -449,8 +456,7 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
         for (int n = 0; n < ND; ++n) {
             int rows = a.rows[n], first = a.base[n];
             if (a.sizes_dev) {
-                rows = __builtin_amdgcn_readfirstlane(a.sizes_dev[n]) / HD;
-                rows = max(1, min(rows, a.total_rows - run - (ND - 1 - n)));
+                rows = device_rows(a, n, ND, run);
                 first = run;
                 run += rows;
             }

@@ -1,0 +1,473 @@
+// Sparse-voxel windowed self-attention with cRSE tables (gfx950): the tile kernel of the forward.
+#include "attn_tile.h"
+
+namespace s3d {
+namespace tile {
+namespace {
+
+constexpr int kListThreads = 1024;
+constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 32 and more tiles, then 64 .. 1 voxels
+
+__device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
+__device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
+
+// Unit list: windows in bins of equal size, largest first (a counting sort in LDS; the order inside a bin is of no
+// consequence, no result depends on which windows share a unit).
+__global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int32_t *__restrict__ w_sizes,
+                                                                 const int32_t *__restrict__ w2n, int W,
+                                                                 int32_t *__restrict__ total, int4 *__restrict__ units,
+                                                                 int32_t *__restrict__ entries)
+{
+    __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
+    const int t = threadIdx.x;
+    if (t < kListBins) windows[t] = big_units[t] = 0;
+    __syncthreads();
+    for (int w = t; w < W; w += kListThreads) {
+        const int n = w_sizes[w];
+        if (n <= 0) continue;
+        const int b = list_bin(n);
+        atomicAdd(&windows[b], 1);
+        if (n > kCols) atomicAdd(&big_units[b], tiles_of(n));
+    }
+    __syncthreads();
+    if (t == 0) {
+        int e = 0, u = 0;
+        for (int b = 0; b < kListBins; ++b) {
+            entry_at[b] = entry_first[b] = e;
+            unit_at[b] = u;
+            if (b < kBigBins) {
+                u += big_units[b];
+            } else {
+                const int per = kCols / (kCols - (b - kBigBins));
+                e += windows[b];
+                u += (windows[b] + per - 1) / per;
+            }
+        }
+        total[0] = u;
+    }
+    __syncthreads();
+    for (int w = t; w < W; w += kListThreads) {
+        const int n = w_sizes[w];
+        if (n <= 0) continue;
+        const int b = list_bin(n), at = w2n[w];
+        if (n > kCols) {
+            const int tiles = tiles_of(n), u = atomicAdd(&unit_at[b], tiles);
+            for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(at, n, q, tiles);
+        } else {
+            const int per = kCols / n, e = atomicAdd(&entry_at[b], 1), rank = e - entry_first[b];
+            entries[e] = at;
+            if (rank % per == 0) units[unit_at[b] + rank / per] = make_int4(e, n, min(per, windows[b] - rank), 0);
+        }
+    }
+}
+
+struct FwdArgs {
+    AttnArgs a;
+    UnitList list;
+};
+
+constexpr float kFix = 33554432.0f;        // 2^25: at most 64 weights of at most 1 meet in a cell
+constexpr float kCellScale = 1.0f / 1048576.0f;   // cells enter the products in units of 2^20
+constexpr float kOutScale = 1.0f / 32.0f;
+
+template <typename T, int D, int ND> struct FwdLayout {
+    static constexpr int kSt = Stages<ND>::kCount;
+    static constexpr uint32_t kSums = kCols * kStride * 4;                       // a [row][column] array of fp32 or u32
+    static constexpr uint32_t kKeys = kCols * kKeyStride * 4;                    // keys: coordinates and table products
+    static constexpr uint32_t kTableT = kSt * D * kStride * sizeof(T);           // value table, [stage][channel][row]
+    static constexpr uint32_t kValueT = D * kStride * sizeof(T);                 // values of the tile, [channel][key]
+    static constexpr uint32_t kCoords = ND * kCols * 4;
+    static constexpr uint32_t kMeta = 4 * kCols * 4;                             // rows of queries and keys, maxima, sums
+    static constexpr uint32_t kBytes = kSums + kKeys + kTableT + kValueT + kCoords + kMeta;
+};
+
+template <typename T, int D, int ND, bool kDeviceSizes>
+__global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
+{
+    using L = FwdLayout<T, D, ND>;
+    using S = Stages<ND>;
+    const AttnArgs &a = f.a;
+    extern __shared__ __align__(16) float smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int H = a.H, HD = H * D;
+    const int h = static_cast<int>(blockIdx.x) % H;
+    const int group = static_cast<int>(blockIdx.x) / H, groups = static_cast<int>(gridDim.x) / H;
+    const int total_units = f.list.total[0];
+    if (group >= total_units) return;
+    // rows and first row of every axis table: kernel arguments, or read from the caller's device tensor of table sizes.
+    // The host has not seen those: it launched the sweep kernel as well, and this kernel leaves the call to it when an
+    // axis has more rows than a stage holds.
+    int read_rows[ND], read_first[ND];
+    if constexpr (kDeviceSizes) {
+        int run = 0;
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+            read_first[n] = run;
+            run += read_rows[n] = device_rows(a, n, ND, run);
+        }
+        if (!rows_fit_tiles(read_rows, ND)) return;
+    }
+    auto rows_n = [&](int n) { return kDeviceSizes ? read_rows[n] : a.rows[n]; };
+    auto first_row = [&](int n) { return kDeviceSizes ? read_first[n] : a.base[n]; };
+
+    const uint32_t base = lds_base(smem);
+    const uint32_t sums = base, keys = sums + L::kSums, table_t = keys + L::kKeys, value_t = table_t + L::kTableT;
+    const uint32_t coords = value_t + L::kValueT, row_i = coords + L::kCoords, row_j = row_i + kCols * 4;
+    const uint32_t col_max = row_j + kCols * 4, col_sum = col_max + kCols * 4;
+
+    const T *gq = static_cast<const T *>(a.q), *gk = static_cast<const T *>(a.k), *gv = static_cast<const T *>(a.v);
+    const T *table_qk = static_cast<const T *>(wave < 4 ? a.table_q : a.table_k);
+    {
+        // the head's value table with the channels as rows, unused rows at zero
+        const T *tv = static_cast<const T *>(a.table_v);
+        for (int x = tid; x < L::kSt * kCols * (D / 8); x += kThreads) {
+            const int c8 = x % (D / 8), row = (x / (D / 8)) % kCols, st = x / (D / 8) / kCols;
+            const int axis = S::first(st) + (st >= 3 && row >= 32 ? 1 : 0);
+            const int r = st >= 3 ? row & 31 : row;
+            int axis_rows = 0, axis_first = 0;
+#pragma unroll
+            for (int n = 0; n < ND; ++n)
+                if (n == axis) { axis_rows = rows_n(n); axis_first = first_row(n); }
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+            if (r < axis_rows) load_row<8>(tv + static_cast<int64_t>(axis_first + r) * HD + h * D + c8 * 8, v);
+            T *to = reinterpret_cast<T *>(reinterpret_cast<char *>(smem) + (table_t - base)) +
+                    (st * D + c8 * 8) * kStride + (row & 32) + permuted_row(row & 31);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) to[e * kStride] = static_cast<T>(v[e]);
+        }
+    }
+
+    const int tile_c = wave & 1, tile_r = (wave >> 1) & 1;
+    const uint32_t row_stride = static_cast<uint32_t>(a.row_stride);
+    const int out_tile = wave & 3, out_half = wave >> 2;  // 16 queries, 32 of a stage's rows
+
+    for (int u = group; u < total_units; u += groups) {
+        const int4 unit = f.list.units[u];
+        const int n_w = __builtin_amdgcn_readfirstlane(unit.y);
+        const int tiles = __builtin_amdgcn_readfirstlane(unit.w);
+        const int at = __builtin_amdgcn_readfirstlane(unit.x), z = __builtin_amdgcn_readfirstlane(unit.z);
+        const bool small = tiles == 0;
+        const int size = small ? n_w : (n_w + tiles - 1) / tiles;
+        const int i0 = small ? 0 : z * size;
+        const int cols = small ? z * n_w : min(size, n_w - i0);
+        if (cols <= 0) continue;
+        const int reach = kThreads / cols;                // rows of threads: a thread takes every `reach`-th key
+        const int own = tid % cols, first = tid / cols;
+        const bool active = first < reach;
+        f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        float run_max = -INFINITY, run_sum = 0.0f;
+        for (int block = 0; block < (small ? 1 : tiles); ++block) {
+            const int j0 = small ? 0 : block * size;
+            const int keys_n = small ? cols : min(size, n_w - j0);
+            if (keys_n <= 0) break;
+            __syncthreads();
+            // the tile's voxels: threads 0..63 the queries, 64..127 the keys
+            if (tid < 2 * kCols) {
+                const bool is_key = tid >= kCols;
+                const int c = tid & (kCols - 1);
+                const int cc = min(c, (is_key ? keys_n : cols) - 1);
+                const int pos = small ? f.list.entries[at + cc / n_w] + cc % n_w : at + (is_key ? j0 : i0) + cc;
+                const int row = a.n2n ? a.n2n[pos] : pos;
+                lds_store_u32((is_key ? row_j : row_i) + c * 4, row);
+#pragma unroll
+                for (int n = 0; n < ND; ++n) {
+                    const float x = a.n_coords[static_cast<int64_t>(pos) * ND + n];
+                    lds_store(is_key ? keys + (c * kKeyStride + n) * 4 : coords + (n * kCols + c) * 4, x);
+                }
+                if (!is_key) {
+                    lds_store_u32(col_max + c * 4, 0x80000000u);
+                    lds_store_u32(col_sum + c * 4, 0u);
+                }
+            }
+            __syncthreads();
+            // (re-read per tile, so that what follows from the lane number does not sit in registers for the whole launch)
+            const int lane = opaque(tid & 63);
+            const int m32 = lane & 31, half32 = lane >> 5;       // row or column, and group of terms, of a 32x32 operand
+            const int n16 = lane & 15, group16 = lane >> 4;
+            const bool term_lane = D > 8 || half32 == 0;         // head_dim 8: the other half of the terms is zero
+            // operands that stay for all stages: queries (wavefronts 0..3) or keys
+            Operand<T> feat;
+            feat.clear();
+            if (term_lane) {
+                const int row = static_cast<int>(lds_load_u32((wave < 4 ? row_i : row_j) + (tile_c * 32 + m32) * 4));
+                feat.load((wave < 4 ? gq : gk) + static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_stride + h * D + half32 * 8);
+            }
+            if (wave < 4) {
+                // q . k of the tile, [key][query]
+                Operand<T> kf;
+                kf.clear();
+                if (term_lane) {
+                    const int row = static_cast<int>(lds_load_u32(row_j + (tile_r * 32 + m32) * 4));
+                    kf.load(gk + static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_stride + h * D + half32 * 8);
+                }
+                const f32x16 d = mfma32(kf, feat, f32x16{});
+                const uint32_t to = sums + ((tile_r * 32 + 4 * half32) * kStride + tile_c * 32 + m32) * 4;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) lds_store(to + mfma32_row(0, e) * kStride * 4, d[e]);
+            } else if (wave - 4 < D / 8) {
+                // values of the tile with the channels as rows; keys past the tile are zero
+                const int c8 = wave - 4;
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+                if (lane < keys_n)
+                    load_row<8>(gv + static_cast<uint64_t>(lds_load_u32(row_j + lane * 4)) * row_stride + h * D + c8 * 8, v);
+                T *to = reinterpret_cast<T *>(reinterpret_cast<char *>(smem) + (value_t - base)) + c8 * 8 * kStride +
+                        (lane & 32) + permuted_row(lane & 31);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) to[e * kStride] = static_cast<T>(v[e]);
+            }
+            __syncthreads();
+            // this thread's pairs: query `own`, keys key0 + first + s * reach
+            const int key0 = small ? own / n_w * n_w : 0;
+            const int per_query = small ? n_w : keys_n;
+            const int steps = (per_query + reach - 1) / reach;
+            float logit[kSteps];
+            uint32_t key_at[kSteps], packed[ND][2];
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                const int j = key0 + min(first + s * reach, per_query - 1);
+                key_at[s] = opaque(keys + j * (kKeyStride * 4));
+                logit[s] = lds_load(sums + (j * kStride + own) * 4);
+            }
+#pragma unroll
+            for (int n = 0; n < ND; ++n) packed[n][0] = packed[n][1] = 0;
+            // The stages: products of the queries and keys with all rows of the stage's axes, then every pair's own two.
+            // The table rows of the next stage are on their way while the pairs of this one are worked on.
+            auto stage_needed = [&](int st) {
+                return (st < 3 ? tile_r * 32 < rows_n(S::first(st)) : (tile_r == 0 || S::paired(st))) &&
+                       tile_c * 32 < (wave < 4 ? cols : keys_n);
+            };
+            auto stage_rows = [&](int st) {
+                const int one = S::first(st), other = one + (S::paired(st) ? 1 : 0);
+                const bool second = st >= 3 && tile_r == 1;
+                const int r = min((st < 3 ? tile_r * 32 : 0) + m32, (second ? rows_n(other) : rows_n(one)) - 1);
+                return table_qk + (__umul24((second ? first_row(other) : first_row(one)) + r, HD) + h * D + half32 * 8);
+            };
+            typename Operand<T>::Raw raw{};
+            if (stage_needed(0) && term_lane) raw = Operand<T>::fetch(stage_rows(0));
+#pragma unroll
+            for (int st = 0; st < S::kCount; ++st) {
+                __syncthreads();
+                if (stage_needed(st)) {
+                    Operand<T> rows;
+                    rows.clear();
+                    if (term_lane) rows.set(raw);
+                    // [row][query] for the queries, [key][row] for the keys (16-byte stores of four consecutive words a
+                    // lane, which the transposed product would give, met in more banks: +2 %)
+                    if (wave < 4) {
+                        const f32x16 d = mfma32(rows, feat, f32x16{});
+                        const uint32_t to = sums + ((tile_r * 32 + 4 * half32) * kStride + tile_c * 32 + m32) * 4;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) lds_store(to + mfma32_row(0, e) * kStride * 4, d[e]);
+                    } else {
+                        const f32x16 d = mfma32(feat, rows, f32x16{});
+                        const uint32_t to = keys + ((tile_c * 32 + 4 * half32) * kKeyStride + kCoordWords + tile_r * 32 + m32) * 4;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) lds_store(to + mfma32_row(0, e) * kKeyStride * 4, d[e]);
+                    }
+                }
+                if (st + 1 < S::kCount && stage_needed(st + 1) && term_lane) raw = Operand<T>::fetch(stage_rows(st + 1));
+                __syncthreads();
+#pragma unroll
+                for (int b = 0; b < (S::paired(st) ? 2 : 1); ++b) {
+                    const int axis = S::first(st) + b;
+                    const float half_rows = static_cast<float>(rows_n(axis) / 2), upper = crse_upper(rows_n(axis));
+                    const float ci = lds_load(coords + (axis * kCols + own) * 4);
+                    const uint32_t own_at = sums + own * 4 + b * 32 * kStride * 4;
+                    for_steps(steps, [&](int s) {
+                        const float cj = lds_load(key_at[s] + axis * 4);
+                        const uint32_t r = static_cast<uint32_t>(crse_row(ci, cj, half_rows, upper));
+                        packed[axis][s / 4] |= r << (8 * (s % 4));
+                        logit[s] += lds_load(__umul24(r, kStride * 4) + own_at) + lds_load(r * 4 + key_at[s] + (kCoordWords + b * 32) * 4);
+                    });
+                    // summed and packed now: the compiler would keep every gathered value until its sum is used
+#pragma unroll
+                    for (int s = 0; s < kSteps; ++s) asm volatile("" : "+v"(logit[s]));
+                    packed[axis][0] = opaque(packed[axis][0]);
+                    packed[axis][1] = opaque(packed[axis][1]);
+                }
+            }
+            // softmax of the tile: maxima per query, weights in fixed point.  Only the last step of a thread can lie
+            // past the window's keys.
+            const int my_steps = active ? (per_query - first + reach - 1) / reach : 0;
+            {
+                float top = -INFINITY;
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) top = s < my_steps ? fmaxf(top, logit[s]) : top;
+                if (active) lds_max(col_max + own * 4, float_order(top));
+            }
+            __syncthreads();
+            lds_zero<kCols * kStride>(sums, tid);
+            const float top = order_float(static_cast<int>(lds_load_u32(col_max + own * 4)));
+            uint32_t weight[kSteps];
+            uint32_t sum = 0;
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                weight[s] = s < my_steps ? static_cast<uint32_t>(__expf(logit[s] - top) * kFix + 0.5f) : 0u;
+                sum += weight[s];
+            }
+            if (active) lds_add(col_sum + own * 4, sum);
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s)
+                if (s < my_steps) lds_store_u32(sums + ((key0 + first + s * reach) * kStride + own) * 4, weight[s]);
+            f32x4_t tile_acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            const uint32_t cell_at = ((out_half * 32 + 2 * group16) * kStride + out_tile * 16 + n16) * 4;
+            auto read_out = [&](uint32_t cells, uint32_t operand, bool table) {
+                if (out_tile * 16 >= cols) return;
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    v[e] = static_cast<float>(lds_load_u32(cells + cell_at + ((e & 1) + 8 * (e >> 1)) * kStride * 4)) * kCellScale;
+                Cells<T> b;
+                // the weights of the values keep 21 bits; those of the table rows are rounded to the tables' type (what
+                // the sum of a pair's rows in that type costs elsewhere)
+                if (table) b.set_single(v); else b.set(v);
+                Operand<T> t;
+                t.load_lds(operand + ((D > 8 ? n16 : n16 & 7) * kStride + out_half * 32 + group16 * 8) * sizeof(T));
+                tile_acc = table ? mfma16_single(t, b, tile_acc) : mfma16(t, b, tile_acc);
+            };
+            __syncthreads();
+            read_out(sums, value_t, false);
+            lds_zero<kCols * kStride>(keys, tid);
+            __syncthreads();
+#pragma unroll
+            for (int st = 0; st < S::kCount; ++st) {
+                const uint32_t cells = st % 2 == 0 ? keys : sums, next = st % 2 == 0 ? sums : keys;
+#pragma unroll
+                for (int b = 0; b < (S::paired(st) ? 2 : 1); ++b) {
+                    const int axis = S::first(st) + b;
+                    const uint32_t own_at = cells + own * 4 + b * 32 * kStride * 4;
+                    for_steps(steps, [&](int s) {
+                        lds_add(__umul24((packed[axis][s / 4] >> (8 * (s % 4))) & 0xffu, kStride * 4) + own_at, weight[s]);
+                    });
+                }
+                __syncthreads();
+                if (st < 3 ? out_half * 32 < rows_n(S::first(st)) : (out_half == 0 || S::paired(st)))
+                    read_out(cells, table_t + st * D * kStride * sizeof(T), true);
+                if (st + 1 < S::kCount) {
+                    lds_zero<kCols * kStride>(next, tid);
+                    __syncthreads();
+                }
+            }
+            // into the query's running softmax state
+            const int i = out_tile * 16 + n16;
+            const float m_tile = order_float(static_cast<int>(lds_load_u32(col_max + i * 4)));
+            const float l_tile = static_cast<float>(lds_load_u32(col_sum + i * 4)) * (1.0f / kFix);
+            const float m_all = fmaxf(run_max, m_tile);
+            const float w_run = __expf(run_max - m_all), w_tile = __expf(m_tile - m_all);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = acc[e] * w_run + tile_acc[e] * w_tile;
+            run_sum = run_sum * w_run + l_tile * w_tile;
+            run_max = m_all;
+        }
+        // the two halves of the rows meet, and the result is stored
+        const int n16 = tid & 15, group16 = (tid & 63) >> 4;
+        __syncthreads();
+        const uint32_t meet = sums + (out_tile * 16 + n16) * 80 + group16 * 16;
+        if (out_half == 1) *(__attribute__((address_space(3))) f32x4_t *)(meet) = acc;
+        __syncthreads();
+        const int i = out_tile * 16 + n16;
+        if (out_half == 0 && i < cols) {
+            const f32x4_t other = *(__attribute__((address_space(3))) f32x4_t *)(meet);
+            const float inv = kOutScale / run_sum;
+            const int64_t row = static_cast<int>(lds_load_u32(row_i + i * 4));
+            if (group16 * 4 < D) {
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (acc[e] + other[e]) * inv;
+                T *to = static_cast<T *>(a.out) + row * HD + h * D + group16 * 4;
+                if constexpr (sizeof(T) == 2) {
+                    uint2 x;
+                    reinterpret_cast<__half2 *>(&x)[0] = __floats2half2_rn(o[0], o[1]);
+                    reinterpret_cast<__half2 *>(&x)[1] = __floats2half2_rn(o[2], o[3]);
+                    *reinterpret_cast<uint2 *>(to) = x;
+                } else {
+                    *reinterpret_cast<float4 *>(to) = make_float4(o[0], o[1], o[2], o[3]);
+                }
+            }
+            if (group16 == 0) {
+                if (a.out_max) a.out_max[row * H + h] = run_max;
+                if (a.out_sum) a.out_sum[row * H + h] = run_sum;
+            }
+        }
+    }
+}
+
+template <typename T, int D, int ND, bool kDeviceSizes>
+int launch_fwd(const AttnArgs &a, const UnitList &list, hipStream_t stream)
+{
+    using L = FwdLayout<T, D, ND>;
+    FwdArgs f;
+    f.a = a;
+    f.list = list;
+    constexpr uint32_t lds = L::kBytes;
+    auto kernel = attn_fwd_tile_kernel<T, D, ND, kDeviceSizes>;
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
+    const int per_cu = lds <= 80 * 1024 ? 2 : 1;
+    const int slots = per_cu * device_cus();
+    const int grid = slots >= a.H ? slots / a.H * a.H : a.H;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, f);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+}  // namespace
+
+int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, int64_t W, hipStream_t stream)
+{
+    hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(kListThreads), 0, stream, w_sizes, w2n, static_cast<int>(W),
+                       const_cast<int32_t *>(l.total), const_cast<int4 *>(l.units), const_cast<int32_t *>(l.entries));
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+}  // namespace tile
+
+// Where the tile kernel serves a forward (head_dim 16).  It leaves every tile's products, sums and histograms in LDS and
+// crosses some thirty barriers for them, which costs about what 64 x 64 pairs cost, so it needs windows of some size; on
+// these it spends 580 clocks of a CU on 64 pairs and a head where the sweep kernel spends 420 in fp16 and 690 in fp32.
+// But a window is spread over its queries' tiles and a tile's pairs over 512 threads, where the sweep gives a query at
+// most eight lanes: a launch that does not fill the chip ends when its longest unit ends, and that is a quarter as long.
+// Measured, sweep / tile kernel, by N^2 / W * H: fp16 76.7 / 44.7 us at 1.6 M, 108.6 / 87.2 at 3.5 M, 200 / 197 at 9.6 M,
+// 324 / 362 at 19 M; fp32 82 / 58 at 1.6 M, 330 / 282 at 9.6 M, 842 / 817 at 32 M, 1235 / 1254 at 46 M.
+constexpr int kTileMeanWindow = 40;
+constexpr double kTilePairsHalf = 8e6, kTilePairsFloat = 35e6;
+
+bool attn_tile_shape(int64_t N, int64_t W, int H, bool fp32)
+{
+    return W > 0 && N >= kTileMeanWindow * W &&
+           static_cast<double>(N) * N / W * H <= (fp32 ? kTilePairsFloat : kTilePairsHalf);
+}
+
+size_t attn_tile_list_bytes(int H, int64_t N, int64_t W)
+{
+    return attn_tile_shape(N, W, H, true) ? tile::list_bytes(N, W) : 0;
+}
+
+bool attn_tile_applies(const AttnArgs &a, int dtype)
+{
+    if (a.D != 16 || !attn_tile_shape(a.N, a.W, a.H, dtype == S3D_DTYPE_F32)) return false;
+    return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
+}
+
+int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t stream, int what)
+{
+    const tile::UnitList l = tile::list_at(list, a.N, a.W);
+    if (what & kAttnBuildList) {
+        if (int rc = tile::launch_list(l, a.w_sizes, a.w2n, a.W, stream)) return rc;
+    }
+    if (!(what & kAttnSweep)) return S3D_OK;
+#define S3D_CASE(TT, CODE, DD, NN)                                                        \
+    if (dtype == CODE && a.D == DD && a.nd == NN)                                         \
+        return a.sizes_dev ? tile::launch_fwd<TT, DD, NN, true>(a, l, stream) : tile::launch_fwd<TT, DD, NN, false>(a, l, stream);
+    S3D_CASE(__half, S3D_DTYPE_F16, 16, 3) S3D_CASE(__half, S3D_DTYPE_F16, 16, 6) S3D_CASE(__half, S3D_DTYPE_F16, 16, 9)
+    S3D_CASE(float, S3D_DTYPE_F32, 16, 3) S3D_CASE(float, S3D_DTYPE_F32, 16, 6) S3D_CASE(float, S3D_DTYPE_F32, 16, 9)
+#undef S3D_CASE
+    return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_fwd: head_dim %d, %d axes in the tile form", a.D, a.nd);
+}
+
+}  // namespace s3d
