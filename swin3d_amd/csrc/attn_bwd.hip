@@ -6,8 +6,9 @@
 //   dv_j  += P dout_i                              dTv[n][row_n(i,j)] += P dout_i
 //   dq_i  += dL (k_j + Tq(i,j))                    dTq[n][row_n(i,j)] += dL q_i
 //   dk_j  += dL (q_i + Tk(i,j))                    dTk[n][row_n(i,j)] += dL k_j
-// The reference adds every term with a global atomic.  Here every output element has ONE owner, and the call has two
-// forms.  With the window set's pair count it runs the pair sweeps of attn_sweep.hip (dq; dk and dv; on the
+// The reference adds every term with a global atomic.  Here every output element has ONE owner, and the call has three
+// forms.  With the window set's pair count it runs at head_dim 16 on tiles (attn_tile_bwd.hip: tables of up to 64 rows on
+// a position axis and 32 on a signal axis), otherwise the pair sweeps of attn_sweep.hip (dq; dk and dv; on the
 // forward's packed work list), which leave dL and P of every (pair, head) in the workspace, and the table-gradient
 // kernels below (attn_bwd_tables_kernel), which read them.  Without it, the fused sweeps (attn_bwd_sweep_kernel),
 // which recompute the logits and need no store:
@@ -1302,8 +1303,12 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_attn_bwd_workspace_
                bwd_row_map_bytes(N);
     size_t need = bwd_units_bytes(W, N, H, pairs) + bwd_delta_bytes(N, H) + bwd_tgrad_bytes(H, D, nd) +
                   bwd_pos_base_bytes(N) + bwd_row_map_bytes(N);
-    if (pairs > 0)
+    if (pairs > 0) {
         need += bwd_pd_bytes(H, pairs) + bwd_dlt_bytes(H, pairs) + align_up(attn_sweep_workspace_bytes(H, W, N), 256);
+        // the tile form works in the whole of it (whether it applies depends on the rows of the single axes)
+        const size_t tiles = D == 16 ? attn_tile_bwd_bytes(H, nd, N, W, pairs) + bwd_row_map_bytes(N) : 0;
+        if (need < tiles) need = tiles;
+    }
     return need;
 }
 
@@ -1416,6 +1421,8 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
         pr.pd = pd; pr.dl_t = dl_t; pr.pairs = pairs;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (N > 0 && W > 0 && attn_tile_bwd_applies(a.rows, nd, D, pairs))
+        return launch_attn_tile_bwd(pr, out, dtable_q, dtable_k, dtable_v, workspace, dtype, s);
     if (N == 0 || W == 0) {
         // nothing to differentiate: the table gradients are zero
         a.N = 0;

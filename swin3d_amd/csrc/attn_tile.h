@@ -39,14 +39,41 @@ __host__ __device__ constexpr int permuted_row(int row) { return ((row % 8) / 2)
 // several small windows of one size that fit 64 columns.  Windows of more than 64 voxels are cut into equal tiles.
 struct UnitList {
     const int32_t *total;      // [0]: units
-    const int4 *units;         // (first entry, voxels per window, windows, 0) or (first position, voxels, tile, tiles)
-    const int32_t *entries;    // first sorted positions of the windows of at most 64 voxels, by size
+    const int4 *units;         // (first entry, voxels per window, windows, 0) or (entry, voxels, tile, tiles)
+    const int2 *entries;       // windows by size: first sorted position, pairs (n^2) of the windows before it
+};
+// A unit, decoded: the tile's queries are `cols` voxels; with more than one tile the workgroup goes through the tiles
+// of the window's keys.
+struct Unit {
+    int entry, n_w, tile, tiles, size, cols;
+    bool small;
+    __device__ __forceinline__ Unit(const int4 u)
+    {
+        entry = __builtin_amdgcn_readfirstlane(u.x);
+        n_w = __builtin_amdgcn_readfirstlane(u.y);
+        const int z = __builtin_amdgcn_readfirstlane(u.z);
+        tiles = __builtin_amdgcn_readfirstlane(u.w);
+        small = tiles == 0;
+        size = small ? n_w : (n_w + tiles - 1) / tiles;
+        tile = small ? 0 : z;
+        cols = small ? z * n_w : min(size, n_w - z * size);
+    }
+    __device__ __forceinline__ int blocks() const { return small ? 1 : tiles; }
+    // keys of block b, and the entry, position inside the window and sorted position of column c of tile t
+    __device__ __forceinline__ int keys(int b) const { return small ? cols : min(size, n_w - b * size); }
+    __device__ __forceinline__ int2 entry_of(const UnitList &l, int c) const { return l.entries[small ? entry + c / n_w : entry]; }
+    __device__ __forceinline__ int inside(int t, int c) const { return small ? c % n_w : t * size + c; }
 };
 inline size_t list_round(size_t bytes) { return (bytes + 255) / 256 * 256; }
-inline size_t list_max_units(int64_t N, int64_t W) { return static_cast<size_t>(W > 0 ? W : 0) + static_cast<size_t>(N > 0 ? N : 0) / 32 + 1; }
+// a unit covers at least 32 voxels (a tile of a window of 65), but for the last one of each window size up to 32
+inline size_t list_max_units(int64_t N, int64_t W)
+{
+    (void)W;
+    return static_cast<size_t>(N > 0 ? N : 0) / 32 + kCols + 1;
+}
 inline size_t list_bytes(int64_t N, int64_t W)
 {
-    return 256 + list_round(sizeof(int4) * list_max_units(N, W)) + list_round(sizeof(int32_t) * static_cast<size_t>(W > 0 ? W : 1));
+    return 256 + list_round(sizeof(int4) * list_max_units(N, W)) + list_round(sizeof(int2) * static_cast<size_t>(W > 0 ? W : 1));
 }
 inline UnitList list_at(void *p, int64_t N, int64_t W)
 {
@@ -54,10 +81,90 @@ inline UnitList list_at(void *p, int64_t N, int64_t W)
     UnitList l;
     l.total = reinterpret_cast<const int32_t *>(base);
     l.units = reinterpret_cast<const int4 *>(base + 256);
-    l.entries = reinterpret_cast<const int32_t *>(base + 256 + list_round(sizeof(int4) * list_max_units(N, W)));
+    l.entries = reinterpret_cast<const int2 *>(base + 256 + list_round(sizeof(int4) * list_max_units(N, W)));
     return l;
 }
 int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, int64_t W, hipStream_t stream);
+
+constexpr int kListThreads = 1024;
+constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 32 and more tiles, then 64 .. 1 voxels
+
+__device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
+__device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
+
+// Unit list: windows in bins of equal size, largest first (a counting sort in LDS; the order inside a bin is of no
+// consequence, no result depends on which windows share a unit), and the pairs of the windows before each.
+__device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
+                                           int32_t *__restrict__ total, int4 *__restrict__ units, int2 *__restrict__ entries)
+{
+    __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
+    __shared__ int wave_pairs[kListThreads / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t < kListBins) windows[t] = big_units[t] = 0;
+    __syncthreads();
+    for (int w = t; w < W; w += kListThreads) {
+        const int n = w_sizes[w];
+        if (n <= 0) continue;
+        const int b = list_bin(n);
+        atomicAdd(&windows[b], 1);
+        if (n > kCols) atomicAdd(&big_units[b], tiles_of(n));
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // exclusive sums of windows and units over the bins, 64 at a time
+        int e_run = 0, u_run = 0;
+        for (int b0 = 0; b0 < kListBins; b0 += 64) {
+            const int b = b0 + lane;
+            const int count = b < kListBins ? windows[b] : 0;
+            const int per = b < kBigBins ? 1 : kCols / max(1, kCols - (b - kBigBins));
+            const int mine = b >= kListBins ? 0 : b < kBigBins ? big_units[b] : (count + per - 1) / per;
+            int e = count, u = mine;
+            for (int off = 1; off < 64; off <<= 1) {
+                const int ue = __shfl_up(e, off), uu = __shfl_up(u, off);
+                if (lane >= off) { e += ue; u += uu; }
+            }
+            if (b < kListBins) {
+                entry_at[b] = entry_first[b] = e_run + e - count;
+                unit_at[b] = u_run + u - mine;
+            }
+            e_run += __shfl(e, 63);
+            u_run += __shfl(u, 63);
+        }
+        if (lane == 0) total[0] = u_run;
+    }
+    __syncthreads();
+    int before = 0;                    // pairs of the windows that earlier rounds placed
+    for (int w0 = 0; w0 < W; w0 += kListThreads) {
+        const int w = w0 + t;
+        const int n = w < W ? w_sizes[w] : 0;
+        int incl = n > 0 ? n * n : 0;
+        const int own = incl;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off);
+            if (lane >= off) incl += up;
+        }
+        if (lane == 63) wave_pairs[wave] = incl;
+        __syncthreads();
+        int pairs = before + incl - own, all = 0;
+#pragma unroll
+        for (int v = 0; v < kListThreads / 64; ++v) {
+            pairs += v < wave ? wave_pairs[v] : 0;
+            all += wave_pairs[v];
+        }
+        before += all;
+        __syncthreads();
+        if (n <= 0) continue;
+        const int b = list_bin(n), e = atomicAdd(&entry_at[b], 1);
+        entries[e] = make_int2(w2n[w], pairs);
+        if (n > kCols) {
+            const int tiles = tiles_of(n), u = atomicAdd(&unit_at[b], tiles);
+            for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
+        } else {
+            const int per = kCols / n, rank = e - entry_first[b];
+            if (rank % per == 0) units[unit_at[b] + rank / per] = make_int4(e, n, min(per, windows[b] - rank), 0);
+        }
+    }
+}
 
 // ---- LDS --------------------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) float lds_f32;
@@ -68,6 +175,50 @@ __device__ __forceinline__ float lds_load(uint32_t addr) { return *(lds_f32 *)(a
 __device__ __forceinline__ uint32_t lds_load_u32(uint32_t addr) { return *(lds_u32 *)(addr); }
 __device__ __forceinline__ void lds_store(uint32_t addr, float v) { *(lds_f32 *)(addr) = v; }
 __device__ __forceinline__ void lds_store_u32(uint32_t addr, uint32_t v) { *(lds_u32 *)(addr) = v; }
+__device__ __forceinline__ float2 lds_load2(uint32_t addr)
+{
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const f32x2 v = *(__attribute__((address_space(3))) f32x2 *)(addr);
+    return make_float2(v[0], v[1]);
+}
+__device__ __forceinline__ void lds_store2(uint32_t addr, float a, float b)
+{
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    *(__attribute__((address_space(3))) f32x2 *)(addr) = f32x2{a, b};
+}
+__device__ __forceinline__ void lds_load8(uint32_t addr, float *v)
+{
+#pragma unroll
+    for (int c = 0; c < 8; c += 4) {
+        const f32x4_t q = *(lds_float4_t *)(addr + 4 * c);
+        v[c] = q[0]; v[c + 1] = q[1]; v[c + 2] = q[2]; v[c + 3] = q[3];
+    }
+}
+// eight 64-bit cells: low and high words
+__device__ __forceinline__ void lds_load_cells(uint32_t addr, uint32_t *lo, int *hi)
+{
+#pragma unroll
+    for (int c = 0; c < 8; c += 2) {
+        const u32x4_t q = *(lds_u32x4 *)(addr + 8 * c);
+        lo[c] = q[0]; hi[c] = static_cast<int>(q[1]); lo[c + 1] = q[2]; hi[c + 1] = static_cast<int>(q[3]);
+    }
+}
+// low word += lo (no carry: the sums of a cell stay below 2^32), high word += hi
+__device__ __forceinline__ void lds_add64(uint32_t addr, uint32_t lo, int hi)
+{
+    typedef __attribute__((address_space(3))) uint64_t lds_u64;
+    const uint64_t v = (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | lo;
+    __hip_atomic_fetch_add((lds_u64 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// four channels of a row
+__device__ __forceinline__ void store4(float *p, const float *v) { *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void store4(__half *p, const float *v)
+{
+    uint2 x;
+    reinterpret_cast<__half2 *>(&x)[0] = __floats2half2_rn(v[0], v[1]);
+    reinterpret_cast<__half2 *>(&x)[1] = __floats2half2_rn(v[2], v[3]);
+    *reinterpret_cast<uint2 *>(p) = x;
+}
 __device__ __forceinline__ void lds_store4(uint32_t addr, float a, float b, float c, float d)
 {
     *(__attribute__((address_space(3))) f32x4_t *)(addr) = f32x4_t{a, b, c, d};
@@ -80,6 +231,12 @@ __device__ __forceinline__ void lds_max(uint32_t addr, int v)
 {
     __hip_atomic_fetch_max((lds_i32 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+// exponent e with |x| < 2^e, and 2^e
+__device__ __forceinline__ int exponent_of(float x)
+{
+    return x != 0.0f ? max(-100, static_cast<int>((__float_as_uint(x) >> 23) & 0xff) - 126) : -100;
+}
+__device__ __forceinline__ float power2(int e) { return ldexpf(1.0f, e); }
 // order-preserving integer image of a float
 __device__ __forceinline__ int float_order(float f)
 {
@@ -87,6 +244,14 @@ __device__ __forceinline__ int float_order(float f)
     return i >= 0 ? i : i ^ 0x7fffffff;
 }
 __device__ __forceinline__ float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff); }
+// Barrier of the workgroup for what it shares in LDS.  __syncthreads() also waits for every load from memory that is under
+// way, among them what a stage has asked for ahead of its use.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 // a value that the compiler cannot follow
 __device__ __forceinline__ int opaque(int x)
 {
@@ -148,6 +313,11 @@ template <> struct Operand<__half> {
     __device__ __forceinline__ void load(const __half *p) { x = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4 *>(p)); }
     __device__ __forceinline__ void load_lds(uint32_t addr) { x = __builtin_bit_cast(f16x8, *(lds_u32x4 *)(addr)); }
     __device__ __forceinline__ void clear() { x = f16x8{}; }
+    __device__ __forceinline__ void set_values(const __half *v)
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __builtin_bit_cast(_Float16, v[e]);
+    }
 };
 template <> struct Operand<float> {
     bf16x8 s[3];
@@ -181,7 +351,8 @@ template <> struct Operand<float> {
 #pragma unroll
         for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(bf16x8, out[k]);
     }
-    __device__ __forceinline__ void load(const float *p)
+    __device__ __forceinline__ void set_values(const float *v) { split(v); }
+    template <typename TF> __device__ __forceinline__ void load(const TF *p)
     {
         float v[8];
         load_row<8>(p, v);
@@ -226,30 +397,32 @@ __device__ __forceinline__ int mfma32_row(int lane, int e) { return 4 * (lane >>
 template <typename T> struct Cells;
 template <> struct Cells<__half> {
     f16x8 hi, lo;
-    // rounded to one fp16 number each
-    __device__ __forceinline__ void set_single(const float *v)
+    // v * scale, rounded to one fp16 number each
+    __device__ __forceinline__ void set_single(const float *v, float scale)
     {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) hi[e] = static_cast<_Float16>(v[e]);
+        for (int e = 0; e < 8; ++e) hi[e] = static_cast<_Float16>(v[e] * scale);
     }
-    __device__ __forceinline__ void set(const float *v)
+    // v * scale as the sum of two fp16 numbers
+    __device__ __forceinline__ void set(const float *v, float scale)
     {
-        u32x4 h, l;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const auto p = __builtin_amdgcn_cvt_pkrtz(v[2 * e], v[2 * e + 1]);
-            h[e] = __builtin_bit_cast(uint32_t, p);
-            const float r0 = v[2 * e] - static_cast<float>(p[0]), r1 = v[2 * e + 1] - static_cast<float>(p[1]);
-            l[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(r0, r1));
+        for (int e = 0; e < 8; ++e) {
+            hi[e] = static_cast<_Float16>(v[e] * scale);
+            lo[e] = static_cast<_Float16>(__builtin_fmaf(v[e], scale, -static_cast<float>(hi[e])));
         }
-        hi = __builtin_bit_cast(f16x8, h);
-        lo = __builtin_bit_cast(f16x8, l);
     }
 };
 template <> struct Cells<float> {
     Operand<float> x;
-    __device__ __forceinline__ void set(const float *v) { x.split(v); }
-    __device__ __forceinline__ void set_single(const float *v) { x.split(v); }
+    __device__ __forceinline__ void set(const float *v, float scale)
+    {
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = v[e] * scale;
+        x.split(y);
+    }
+    __device__ __forceinline__ void set_single(const float *v, float scale) { set(v, scale); }
 };
 __device__ __forceinline__ f32x4_t mfma16(const Operand<__half> &a, const Cells<__half> &b, f32x4_t c)
 {
@@ -271,6 +444,49 @@ __device__ __forceinline__ f32x4_t mfma16(const Operand<float> &a, const Cells<f
 }
 
 __device__ __forceinline__ f32x4_t mfma16_single(const Operand<float> &a, const Cells<float> &b, f32x4_t c) { return mfma16(a, b, c); }
+
+// fp32 values beside fp16 ones: the sum of two fp16 numbers (23 bits) of the values times a power of two that brings the
+// largest of them to 2^14
+struct Pair16 {
+    f16x8 hi, lo;
+    __device__ __forceinline__ void set_values(const float *v, float scale)
+    {
+        Cells<__half> c;
+        c.set(v, scale);
+        hi = c.hi;
+        lo = c.lo;
+    }
+};
+__device__ __forceinline__ f32x16 mfma32(const Pair16 &a, const Operand<__half> &b, f32x16 c)
+{
+    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.lo, b.x, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.hi, b.x, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 mfma32(const Operand<__half> &a, const Pair16 &b, f32x16 c)
+{
+    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.lo, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.hi, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t mfma16(const Pair16 &a, const Cells<__half> &b, f32x4_t c)
+{
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo, b.hi, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.lo, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.hi, c, 0, 0, 0);
+}
+
+// ... with the cells as A (their columns are the terms) and exact values as B
+template <typename T> struct CellsA : Cells<T> {};
+__device__ __forceinline__ f32x4_t mfma16(const CellsA<__half> &a, const Operand<__half> &b, f32x4_t c)
+{
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo, b.x, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.x, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t mfma16(const CellsA<float> &a, const Operand<float> &b, f32x4_t c)
+{
+    Cells<float> x;
+    x.x = b;
+    return mfma16(a.x, x, c);
+}
 
 }  // namespace tile
 }  // namespace s3d

@@ -5,60 +5,10 @@ namespace s3d {
 namespace tile {
 namespace {
 
-constexpr int kListThreads = 1024;
-constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 32 and more tiles, then 64 .. 1 voxels
-
-__device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
-__device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
-
-// Unit list: windows in bins of equal size, largest first (a counting sort in LDS; the order inside a bin is of no
-// consequence, no result depends on which windows share a unit).
-__global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int32_t *__restrict__ w_sizes,
-                                                                 const int32_t *__restrict__ w2n, int W,
-                                                                 int32_t *__restrict__ total, int4 *__restrict__ units,
-                                                                 int32_t *__restrict__ entries)
+__global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int32_t *w_sizes, const int32_t *w2n, int W, int32_t *total,
+                                                                 int4 *units, int2 *entries)
 {
-    __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
-    const int t = threadIdx.x;
-    if (t < kListBins) windows[t] = big_units[t] = 0;
-    __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n <= 0) continue;
-        const int b = list_bin(n);
-        atomicAdd(&windows[b], 1);
-        if (n > kCols) atomicAdd(&big_units[b], tiles_of(n));
-    }
-    __syncthreads();
-    if (t == 0) {
-        int e = 0, u = 0;
-        for (int b = 0; b < kListBins; ++b) {
-            entry_at[b] = entry_first[b] = e;
-            unit_at[b] = u;
-            if (b < kBigBins) {
-                u += big_units[b];
-            } else {
-                const int per = kCols / (kCols - (b - kBigBins));
-                e += windows[b];
-                u += (windows[b] + per - 1) / per;
-            }
-        }
-        total[0] = u;
-    }
-    __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n <= 0) continue;
-        const int b = list_bin(n), at = w2n[w];
-        if (n > kCols) {
-            const int tiles = tiles_of(n), u = atomicAdd(&unit_at[b], tiles);
-            for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(at, n, q, tiles);
-        } else {
-            const int per = kCols / n, e = atomicAdd(&entry_at[b], 1), rank = e - entry_first[b];
-            entries[e] = at;
-            if (rank % per == 0) units[unit_at[b] + rank / per] = make_int4(e, n, min(per, windows[b] - rank), 0);
-        }
-    }
+    build_list(w_sizes, w2n, W, total, units, entries);
 }
 
 struct FwdArgs {
@@ -144,31 +94,25 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
     const int out_tile = wave & 3, out_half = wave >> 2;  // 16 queries, 32 of a stage's rows
 
     for (int u = group; u < total_units; u += groups) {
-        const int4 unit = f.list.units[u];
-        const int n_w = __builtin_amdgcn_readfirstlane(unit.y);
-        const int tiles = __builtin_amdgcn_readfirstlane(unit.w);
-        const int at = __builtin_amdgcn_readfirstlane(unit.x), z = __builtin_amdgcn_readfirstlane(unit.z);
-        const bool small = tiles == 0;
-        const int size = small ? n_w : (n_w + tiles - 1) / tiles;
-        const int i0 = small ? 0 : z * size;
-        const int cols = small ? z * n_w : min(size, n_w - i0);
+        const Unit unit(f.list.units[u]);
+        const int cols = unit.cols, n_w = unit.n_w;
+        const bool small = unit.small;
         if (cols <= 0) continue;
         const int reach = kThreads / cols;                // rows of threads: a thread takes every `reach`-th key
         const int own = tid % cols, first = tid / cols;
         const bool active = first < reach;
         f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
         float run_max = -INFINITY, run_sum = 0.0f;
-        for (int block = 0; block < (small ? 1 : tiles); ++block) {
-            const int j0 = small ? 0 : block * size;
-            const int keys_n = small ? cols : min(size, n_w - j0);
+        for (int block = 0; block < unit.blocks(); ++block) {
+            const int keys_n = unit.keys(block);
             if (keys_n <= 0) break;
-            __syncthreads();
+            lds_barrier();
             // the tile's voxels: threads 0..63 the queries, 64..127 the keys
             if (tid < 2 * kCols) {
                 const bool is_key = tid >= kCols;
                 const int c = tid & (kCols - 1);
                 const int cc = min(c, (is_key ? keys_n : cols) - 1);
-                const int pos = small ? f.list.entries[at + cc / n_w] + cc % n_w : at + (is_key ? j0 : i0) + cc;
+                const int pos = unit.entry_of(f.list, cc).x + unit.inside(is_key ? block : unit.tile, cc);
                 const int row = a.n2n ? a.n2n[pos] : pos;
                 lds_store_u32((is_key ? row_j : row_i) + c * 4, row);
 #pragma unroll
@@ -181,7 +125,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     lds_store_u32(col_sum + c * 4, 0u);
                 }
             }
-            __syncthreads();
+            lds_barrier();
             // (re-read per tile, so that what follows from the lane number does not sit in registers for the whole launch)
             const int lane = opaque(tid & 63);
             const int m32 = lane & 31, half32 = lane >> 5;       // row or column, and group of terms, of a 32x32 operand
@@ -219,7 +163,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) to[e * kStride] = static_cast<T>(v[e]);
             }
-            __syncthreads();
+            lds_barrier();
             // this thread's pairs: query `own`, keys key0 + first + s * reach
             const int key0 = small ? own / n_w * n_w : 0;
             const int per_query = small ? n_w : keys_n;
@@ -250,7 +194,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             if (stage_needed(0) && term_lane) raw = Operand<T>::fetch(stage_rows(0));
 #pragma unroll
             for (int st = 0; st < S::kCount; ++st) {
-                __syncthreads();
+                lds_barrier();
                 if (stage_needed(st)) {
                     Operand<T> rows;
                     rows.clear();
@@ -270,7 +214,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     }
                 }
                 if (st + 1 < S::kCount && stage_needed(st + 1) && term_lane) raw = Operand<T>::fetch(stage_rows(st + 1));
-                __syncthreads();
+                lds_barrier();
 #pragma unroll
                 for (int b = 0; b < (S::paired(st) ? 2 : 1); ++b) {
                     const int axis = S::first(st) + b;
@@ -299,7 +243,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 for (int s = 0; s < kSteps; ++s) top = s < my_steps ? fmaxf(top, logit[s]) : top;
                 if (active) lds_max(col_max + own * 4, float_order(top));
             }
-            __syncthreads();
+            lds_barrier();
             lds_zero<kCols * kStride>(sums, tid);
             const float top = order_float(static_cast<int>(lds_load_u32(col_max + own * 4)));
             uint32_t weight[kSteps];
@@ -310,7 +254,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 sum += weight[s];
             }
             if (active) lds_add(col_sum + own * 4, sum);
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int s = 0; s < kSteps; ++s)
                 if (s < my_steps) lds_store_u32(sums + ((key0 + first + s * reach) * kStride + own) * 4, weight[s]);
@@ -321,19 +265,19 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 float v[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    v[e] = static_cast<float>(lds_load_u32(cells + cell_at + ((e & 1) + 8 * (e >> 1)) * kStride * 4)) * kCellScale;
+                    v[e] = static_cast<float>(lds_load_u32(cells + cell_at + ((e & 1) + 8 * (e >> 1)) * kStride * 4));
                 Cells<T> b;
                 // the weights of the values keep 21 bits; those of the table rows are rounded to the tables' type (what
                 // the sum of a pair's rows in that type costs elsewhere)
-                if (table) b.set_single(v); else b.set(v);
+                if (table) b.set_single(v, kCellScale); else b.set(v, kCellScale);
                 Operand<T> t;
                 t.load_lds(operand + ((D > 8 ? n16 : n16 & 7) * kStride + out_half * 32 + group16 * 8) * sizeof(T));
                 tile_acc = table ? mfma16_single(t, b, tile_acc) : mfma16(t, b, tile_acc);
             };
-            __syncthreads();
+            lds_barrier();
             read_out(sums, value_t, false);
             lds_zero<kCols * kStride>(keys, tid);
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int st = 0; st < S::kCount; ++st) {
                 const uint32_t cells = st % 2 == 0 ? keys : sums, next = st % 2 == 0 ? sums : keys;
@@ -345,12 +289,12 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                         lds_add(__umul24((packed[axis][s / 4] >> (8 * (s % 4))) & 0xffu, kStride * 4) + own_at, weight[s]);
                     });
                 }
-                __syncthreads();
+                lds_barrier();
                 if (st < 3 ? out_half * 32 < rows_n(S::first(st)) : (out_half == 0 || S::paired(st)))
                     read_out(cells, table_t + st * D * kStride * sizeof(T), true);
                 if (st + 1 < S::kCount) {
                     lds_zero<kCols * kStride>(next, tid);
-                    __syncthreads();
+                    lds_barrier();
                 }
             }
             // into the query's running softmax state
@@ -366,10 +310,10 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
         }
         // the two halves of the rows meet, and the result is stored
         const int n16 = tid & 15, group16 = (tid & 63) >> 4;
-        __syncthreads();
+        lds_barrier();
         const uint32_t meet = sums + (out_tile * 16 + n16) * 80 + group16 * 16;
         if (out_half == 1) *(__attribute__((address_space(3))) f32x4_t *)(meet) = acc;
-        __syncthreads();
+        lds_barrier();
         const int i = out_tile * 16 + n16;
         if (out_half == 0 && i < cols) {
             const f32x4_t other = *(__attribute__((address_space(3))) f32x4_t *)(meet);
@@ -420,7 +364,7 @@ int launch_fwd(const AttnArgs &a, const UnitList &list, hipStream_t stream)
 int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, int64_t W, hipStream_t stream)
 {
     hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(kListThreads), 0, stream, w_sizes, w2n, static_cast<int>(W),
-                       const_cast<int32_t *>(l.total), const_cast<int4 *>(l.units), const_cast<int32_t *>(l.entries));
+                       const_cast<int32_t *>(l.total), const_cast<int4 *>(l.units), const_cast<int2 *>(l.entries));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

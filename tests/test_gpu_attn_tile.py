@@ -38,3 +38,48 @@ def test_forward_stages_and_row_limits(oracle_lib, hip_lib, dtype, ws, cRSE, hea
     assert np.allclose(omax, ref[1], rtol=0, atol=2e-5 * np.abs(ref[1]).max() if dtype == torch.float32 else 1e-3)
     assert np.allclose(osum, ref[2], rtol=1e-4 if dtype == torch.float32 else 3e-3)
     assert np.array_equal(run_attention(case, dtype, device_sizes=True), got)
+
+
+def _backward(case, dtype, tables, dout, spare=0, part=1):
+    import swin3d_amd
+    dev = torch.device("cuda")
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    i = case.index
+    args = [t(x).to(dtype) for x in (case.q, case.k, case.v)] + [t(x) for x in (case.tq, case.tk, case.tv)]
+    rest = (t(case.table_sizes), t(i["w_sizes"]), t(i["w2n"]), t(i["n2n"]), t(case.n_coords))
+    out, omax, osum = swin3d_amd.window_attention_forward(*args[:3], *[x.to(dtype) for x in args[3:]], *rest, return_stats=True)
+    pairs = int((torch.as_tensor(i["w_sizes"]).long() ** 2).sum()) // part + spare
+    return swin3d_amd.window_attention_backward(*args[:3], *[x.to(tables) for x in args[3:]], *rest, out, omax, osum,
+                                                t(dout).to(dtype), pairs=pairs)
+
+
+@pytest.mark.parametrize("dtype,tables", [(torch.float32, torch.float32), (torch.float16, torch.float16), (torch.float16, torch.float32)])
+@pytest.mark.parametrize("ws,cRSE,heads,fill", [
+    (8, "XYZ_RGB_NORM", 3, 0.75),     # 64 rows on the position axes; windows of six tiles
+    (7, "XYZ_RGB", 2, 0.3),           # an odd number of signal axes; windows of two tiles
+    (5, "XYZ", 1, 0.2),               # no signal axes; several windows in a tile
+    (10, "XYZ", 2, 0.5),              # 80 rows: beyond a stage, the pair sweeps'
+])
+def test_backward_stages_and_row_limits(oracle_lib, hip_lib, dtype, tables, ws, cRSE, heads, fill):
+    from test_gpu_attn_bwd import _assert_close
+    half = (ws, ws, (ws + 1) // 2)
+    n = int(fill * 8 * half[0] * half[1] * half[2])
+    case = make_attn_case(oracle_lib, seed=ws, n=n, ws=ws, quant=4, heads=heads, dim=16, cRSE=cRSE, extent=half)
+    case.v *= np.float32(0.4)
+    case.tv *= np.float32(0.2)
+    if dtype == torch.float16:
+        to_half_and_back(case)
+    dout = np.random.default_rng(ws).standard_normal(case.q.shape).astype(np.float16).astype(np.float32)
+    got = _backward(case, dtype, tables, dout)
+    _assert_close([g.double().cpu().numpy() for g in got], oracle_lib.attn_bwd(*case.oracle_args(), dout), dtype)
+    if ws == 10:
+        return
+    # the same bits again, also with room to spare in the store
+    for again in (_backward(case, dtype, tables, dout), _backward(case, dtype, tables, dout, spare=4321)):
+        assert all(torch.equal(x, y) for x, y in zip(got[:3], again[:3]))
+    # too small a store: the windows beyond it and every table gradient say so
+    short = _backward(case, dtype, tables, dout, part=2)
+    assert all(bool(torch.isnan(g).all()) for g in short[3:])
+    for g, whole in zip(short[:3], got[:3]):
+        bad = torch.isnan(g.float()).flatten(1).any(1)
+        assert bool(bad.any()) and torch.equal(g[~bad], whole[~bad])
