@@ -387,6 +387,51 @@ int s3d_add_layernorm(const float *x, const void *residual, int32_t residual_dty
                       const float *beta, float eps, float *x_out, void *y, int32_t y_dtype, int64_t N, int32_t C,
                       void *stream);
 
+/*
+ * y = x w^T + bias, then GELU (the exact form) where gelu is not zero; fp16 operands and result, fp32 accumulation, bias
+ * and GELU, one rounding at the end.  x device [M,K], w device [N,K] (torch.nn.Linear's weight), bias device [N] or null,
+ * y device [M,N], all dense and 16-byte aligned; N a multiple of 8, K of 16.
+ */
+int s3d_linear(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, int32_t gelu,
+               void *stream);
+
+/*
+ * The Swin blocks of a stage at inference (Swin3D/modules/swin3d_layers.py:563-625): per block
+ *   x = x + proj(attention(qkv(LayerNorm(x))));  x = x + fc2(GELU(fc1(LayerNorm(x))))
+ * with the residual stream in fp32 and the branches in fp16, in one host call.  Block i works on window set i % num_sets.
+ *
+ *   x              device [N,C] fp32, C = H*D; left as it is
+ *   x_out          device [N,C] fp32, and
+ *   pending        device [N,C] fp16: the result is x_out + pending (the sum is the next LayerNorm's, which can make it
+ *                  on its way)
+ *   table_sizes    HOST [nd], as for s3d_attn_fwd
+ *   sets, blocks   HOST arrays of the structs below, which hold device pointers
+ * C and hidden multiples of 16, C at most 1024; head_dim, axes and tables as for s3d_attn_fwd in fp16.
+ */
+typedef struct {
+    const int32_t *w_sizes, *w2n, *n2n;      /* as for s3d_attn_fwd (n2n may be null) */
+    const float *n_coords;
+    int64_t num_windows;
+    void *plan;                              /* of s3d_attn_plan for these windows, H, D and fp16; where planned is 0, as */
+    size_t plan_bytes;                       /* much memory, and every block makes its own list there */
+    int32_t planned;
+} s3d_window_set;
+
+typedef struct {
+    const float *norm1_weight, *norm1_bias, *norm2_weight, *norm2_bias;   /* fp32 [C] */
+    const void *qkv_weight, *qkv_bias;       /* fp16 [3C,C] (the q rows scaled by D^-0.5), [3C] or null */
+    const void *table_q, *table_k, *table_v; /* fp16 [table_len] */
+    const void *proj_weight, *proj_bias;     /* fp16 [C,C], [C] or null */
+    const void *fc1_weight, *fc1_bias;       /* fp16 [hidden,C], [hidden] or null */
+    const void *fc2_weight, *fc2_bias;       /* fp16 [C,hidden], [C] or null */
+    float norm1_eps, norm2_eps;
+} s3d_swin_block;
+
+size_t s3d_swin_blocks_workspace_bytes(int64_t N, int32_t C, int32_t hidden);
+int s3d_swin_blocks(const float *x, float *x_out, void *pending, int64_t N, int32_t H, int32_t D, int32_t hidden,
+                    const int32_t *table_sizes, int32_t nd, int64_t table_len, const s3d_window_set *sets, int32_t num_sets,
+                    const s3d_swin_block *blocks, int32_t num_blocks, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

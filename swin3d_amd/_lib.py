@@ -22,6 +22,18 @@ _vp = ctypes.c_void_p
 _i32 = ctypes.c_int32
 _i64 = ctypes.c_int64
 
+
+class WindowSet(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("w_sizes", "w2n", "n2n", "n_coords")] + [
+        ("num_windows", _i64), ("plan", _vp), ("plan_bytes", ctypes.c_size_t), ("planned", _i32)]
+
+
+class SwinBlock(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("norm1_weight", "norm1_bias", "norm2_weight", "norm2_bias", "qkv_weight", "qkv_bias",
+                                   "table_q", "table_k", "table_v", "proj_weight", "proj_bias", "fc1_weight", "fc1_bias",
+                                   "fc2_weight", "fc2_bias")] + [("norm1_eps", ctypes.c_float), ("norm2_eps", ctypes.c_float)]
+
+
 # name -> (restype, argtypes); mirrors include/swin3d_amd.h
 SIGNATURES = {
     "s3d_version": (ctypes.c_int, []),
@@ -51,6 +63,11 @@ SIGNATURES = {
     "s3d_knn_interpolate": (ctypes.c_int, [_vp, _vp, _i32, _i64, _vp, _i64, _i32, _i32, _vp, _vp]),
     "s3d_knn_max_pool": (ctypes.c_int, [_vp, _i32, _i64, _vp, _i64, _i32, _i32, _vp, _vp]),
     "s3d_add_layernorm": (ctypes.c_int, [_vp, _vp, _i32, _vp, _vp, ctypes.c_float, _vp, _vp, _i32, _i64, _i32, _vp]),
+    "s3d_linear": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp]),
+    "s3d_swin_blocks_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32]),
+    # x x_out pending | N H D hidden | table sizes nd len | sets blocks | ws bytes stream
+    "s3d_swin_blocks": (ctypes.c_int, [_vp] * 3 + [_i64, _i32, _i32, _i32] + [_vp, _i32, _i64] + [_vp, _i32] * 2 +
+                        [_vp, ctypes.c_size_t, _vp]),
 }
 
 

@@ -1,0 +1,194 @@
+// Y = X W^T + b, with GELU on request: fp16 operands, fp32 accumulation and fp32 bias and GELU, one rounding to fp16
+// (gfx950).  The projections of a Swin block at inference (Swin3D/modules/swin3d_layers.py:153-176, 382-560): tall X
+// (rows = voxels), K and N a few dozen to a few thousand.
+//
+// Both operands are contiguous along K, which is how a lane of v_mfma_f32_32x32x16 wants them: eight consecutive numbers
+// of a row.  A workgroup stages 64 numbers of K of its rows of X and W in LDS (the next 64 on their way in registers
+// meanwhile) with the 16-byte pieces of a row in an order that depends on the row, so that the lanes' reads of 32 rows
+// spread over all banks; W goes in as the first operand, so that a lane ends up with four neighbouring outputs of one
+// row, and the tile leaves through LDS as whole rows.
+//
+// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 219 us against
+// 416 us as product and GELU apart, at 2.2 of the 5.1 TB/s that a copy reaches; 80 -> 240, 125 us against 207.  At the
+// deepest the tiles are few and a tile's chain of chunks is what counts: 811 rows, 384 -> 384, 5 us against 18 through
+// torch, whose launch alone takes the host that long.
+#include "linear.h"
+
+namespace s3d {
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kThreads = 256;
+constexpr int kChunk = 64;        // numbers of K staged at a time
+constexpr int kPieces = kChunk / 8;
+
+// x Phi(x).  Phi by Abramowitz and Stegun 7.1.26 in its complementary form, erfc(z) = t (a1 + .. + a5 t^4) exp(-z^2),
+// t = 1 / (1 + p z): |error| < 1.5e-7, far below the rounding to fp16 that follows.
+__device__ __forceinline__ float gelu(float x)
+{
+    const float z = fabsf(x) * 0.70710678118654752f;
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
+    float poly = fmaf(1.061405429f, t, -1.453152027f);
+    poly = fmaf(poly, t, 1.421413741f);
+    poly = fmaf(poly, t, -0.284496736f);
+    poly = fmaf(poly, t, 0.254829592f);
+    const float tail = 0.5f * poly * t * __expf(-z * z);      // Phi(-|x|)
+    return x * (x > 0.0f ? 1.0f - tail : tail);
+}
+
+// The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
+__device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
+
+// WM x WN wavefronts of TM x TN products of 32 x 32
+template <int WM, int WN, int TM, int TN> struct Tile {
+    static_assert(WM * WN == kThreads / 64, "four wavefronts");
+    static constexpr int kWM = WM, kTM = TM, kTN = TN;
+    static constexpr int kM = 32 * WM * TM, kN = 32 * WN * TN;
+    static constexpr int kStage = (kM + kN) * kChunk * 2;             // bytes of one staged chunk
+    static constexpr int kPitch = kN + 8;                             // of the finished tile
+    static constexpr int kLds = 2 * kStage > kM * kPitch * 2 ? 2 * kStage : kM * kPitch * 2;
+    static constexpr int kLoads = (kM + kN) * kPieces / kThreads;     // pieces per thread and chunk
+};
+
+template <typename L, bool GELU>
+__global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
+                                                             const _Float16 *__restrict__ bias, _Float16 *__restrict__ y,
+                                                             int M, int N, int K, int tiles_n, int tiles)
+{
+    constexpr int TM = L::kTM, TN = L::kTN;
+    __shared__ __align__(16) char smem[L::kLds];
+    // workgroups b, b + 8, .. run on one XCD: they get neighbouring tiles, which share rows of X
+    const int share = (tiles + 7) / 8, tile = static_cast<int>(blockIdx.x) % 8 * share + static_cast<int>(blockIdx.x) / 8;
+    if (tile >= tiles) return;
+    const int m0 = tile / tiles_n * L::kM, n0 = tile % tiles_n * L::kN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave % L::kWM * (32 * TM), wave_n = wave / L::kWM * (32 * TN);
+    const int r32 = lane & 31, half = lane >> 5;
+
+    // this thread's pieces of a chunk: row (tid / 8 + 32 i) of [X rows, W rows], piece tid % 8
+    const int piece = tid % kPieces, row = tid / kPieces;
+    const _Float16 *from[L::kLoads];
+#pragma unroll
+    for (int i = 0; i < L::kLoads; ++i) {
+        const int r = row + i * (kThreads / kPieces);
+        from[i] = (r < L::kM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r - L::kM, N - 1)) * K) + piece * 8;
+    }
+    uint4 held[L::kLoads];
+    auto fetch = [&](int k0) {
+        if (k0 + piece * 8 < K) {
+#pragma unroll
+            for (int i = 0; i < L::kLoads; ++i) held[i] = *reinterpret_cast<const uint4 *>(from[i] + k0);
+        }
+    };
+    auto put = [&](int buffer) {
+        uint4 *to = reinterpret_cast<uint4 *>(smem + buffer * L::kStage);
+#pragma unroll
+        for (int i = 0; i < L::kLoads; ++i) to[placed(row + i * (kThreads / kPieces), piece)] = held[i];
+    };
+    f32x16 acc[TM][TN] = {};
+    auto multiply = [&](int buffer, int steps) {
+        const half8 *at = reinterpret_cast<const half8 *>(smem + buffer * L::kStage);
+#pragma unroll
+        for (int s = 0; s < kChunk / 16; ++s) {
+            if (s >= steps) break;
+            half8 a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[i] = at[placed(wave_m + i * 32 + r32, 2 * s + half)];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[j] = at[placed(L::kM + wave_n + j * 32 + r32, 2 * s + half)];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[j], a[i], acc[i][j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < L::kLoads; ++i) held[i] = make_uint4(0, 0, 0, 0);
+    fetch(0);
+    put(0);
+    __syncthreads();
+    const int whole = (K - 1) / kChunk;      // chunks before the last one
+    for (int c = 0; c < whole; ++c) {
+        fetch((c + 1) * kChunk);
+        multiply(c & 1, kChunk / 16);
+        put((c + 1) & 1);
+        __syncthreads();
+    }
+    multiply(whole & 1, (K - whole * kChunk) / 16);
+    __syncthreads();
+
+    // a lane's outputs: row r32 of X, columns 8 g + 4 half .. + 3 of W's 32
+    _Float16 *out = reinterpret_cast<_Float16 *>(smem);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int n = wave_n + j * 32 + 8 * g + 4 * half;
+            half4 b = {0, 0, 0, 0};
+            if (bias) b = *reinterpret_cast<const half4 *>(bias + min(n0 + n, N - 4));
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                half4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = acc[i][j][4 * g + e] + static_cast<float>(b[e]);
+                    o[e] = static_cast<_Float16>(GELU ? gelu(v) : v);
+                }
+                *reinterpret_cast<half4 *>(out + (wave_m + i * 32 + r32) * L::kPitch + n) = o;
+            }
+        }
+    __syncthreads();
+    constexpr int kRowPieces = L::kN / 8;
+#pragma unroll
+    for (int t = tid; t < L::kM * kRowPieces; t += kThreads) {
+        const int r = t / kRowPieces, n = t % kRowPieces * 8;
+        if (m0 + r < M && n0 + n < N)
+            *reinterpret_cast<uint4 *>(y + static_cast<int64_t>(m0 + r) * N + n0 + n) = *reinterpret_cast<const uint4 *>(out + r * L::kPitch + n);
+    }
+}
+
+template <typename L>
+int launch(const LinearArgs &a, hipStream_t stream)
+{
+    const int tiles_n = (a.N + L::kN - 1) / L::kN;
+    const int64_t tiles = ceil_div(a.M, L::kM) * tiles_n;
+    if (tiles > (1 << 30)) return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M = %lld rows", (long long)a.M);
+    const dim3 grid(static_cast<unsigned>(ceil_div(tiles, 8) * 8));
+    auto kernel = a.gelu ? linear_kernel<L, true> : linear_kernel<L, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, static_cast<const _Float16 *>(a.x), static_cast<const _Float16 *>(a.w),
+                       static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<int>(a.M), a.N, a.K, tiles_n,
+                       static_cast<int>(tiles));
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+}  // namespace
+
+int launch_linear(const LinearArgs &a, hipStream_t stream)
+{
+    if (a.M < 0 || a.M > 0x7fffffff || a.N < 8 || a.N % 8 || a.K < 16 || a.K % 16)
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M=%lld N=%d K=%d (N a multiple of 8, K of 16)", (long long)a.M, a.N, a.K);
+    if (a.M == 0) return S3D_OK;
+    if (!a.x || !a.w || !a.y) return fail(S3D_ERR_NULL_POINTER, "s3d_linear: null device pointer");
+    // Tiles of 64 x 64 as long as larger ones would leave CUs without work; then 128 rows by the width that pads N least,
+    // the widest of those that still give every CU two tiles.  192 columns take most of a wavefront's registers: with
+    // GELU only where the tile is the whole row.
+    if (ceil_div(a.M, 64) * ((a.N + 63) / 64) < 1024) return launch<Tile<2, 2, 1, 1>>(a, stream);
+    auto padded = [&](int width) { return (a.N + width - 1) / width * width; };
+    auto enough = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width) >= 512; };
+    const int least = padded(64);
+    if (padded(192) == least && enough(192) && (!a.gelu || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
+    if (padded(128) == least && enough(128)) return launch<Tile<2, 2, 2, 2>>(a, stream);
+    return launch<Tile<2, 2, 2, 1>>(a, stream);
+}
+
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_linear(
+    const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, int32_t gelu, void *stream)
+{
+    return s3d::launch_linear(s3d::LinearArgs{x, w, bias, y, M, N, K, gelu != 0}, static_cast<hipStream_t>(stream));
+}

@@ -35,6 +35,7 @@ from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
 from .fused_norm import add_layernorm
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .sparse_dl.knn import KNN, KNNInterpolate, knn_max_pool, knn_query
+from .swin_blocks import linear_rows, swin_blocks
 from .window_index import build_window_indices, get_index01, index_arguments, window_signals
 
 
@@ -251,6 +252,8 @@ def drop_inference_copies(model):
     for m in model.modules():
         if hasattr(m, "_s3d_cast"):
             del m._s3d_cast
+        if hasattr(m, "_s3d_blocks"):
+            del m._s3d_blocks
         if isinstance(m, WindowAttention):
             m._cache = None
 
@@ -262,6 +265,12 @@ def _linear(layer, x):
     epoch = _cache_epoch()
     if torch.is_grad_enabled() or not torch.is_autocast_enabled() or not x.is_cuda:
         return layer(x)
+    weight, bias = _autocast_copy(layer, epoch)
+    out = linear_rows(x, weight, bias)
+    return F.linear(x, weight, bias) if out is None else out
+
+
+def _autocast_copy(layer, epoch):
     dtype = torch.get_autocast_dtype("cuda")
     w, b = layer.weight, layer.bias
     key = (epoch, dtype, w.data_ptr(), w._version, None if b is None else (b.data_ptr(), b._version))
@@ -269,7 +278,7 @@ def _linear(layer, x):
     if kept is None or kept[0] != key:
         kept = (key, w.detach().to(dtype), None if b is None else b.detach().to(dtype))
         layer._s3d_cast = kept
-    return F.linear(x, kept[1], kept[2])
+    return kept[1], kept[2]
 
 
 class Mlp(nn.Module):
@@ -462,15 +471,17 @@ class Stage(nn.Module):
             shifts.append((self.downsample.factor, 0))      # the downsample's cells: the same host wait
         indices = build_window_indices(coords, stride, self.window_size, shifts)
         cell_index = indices.pop() if pooled else None
-        args = [index_arguments(index, local, extra) for index in indices]
-        if rows_in_window_order and args:
-            args[0] = args[0][:5] + (None,) + args[0][6:]      # (.., w2n, n2n, w2m, ..): no row map
         if len(self.blocks) > 0:
             # the quantiser scaling of the signals is the same for every block of the stage: once per index set,
-            # fused with the gather into window order
+            # fused with the gather into window order (and in place of the unscaled signals, which nobody reads)
             attn = self.blocks[0].attn
-            args = [tuple(a) + (window_signals(index, local, extra, crse_num_axes(attn.cRSE) - 3, attn.quant_size,
-                                               2 * attn.quant_size),) for a, index in zip(args, indices)]
+            args = [(None, None, None, index.w_sizes, index.w2n, index.n2n, None, None,
+                     window_signals(index, local, extra, crse_num_axes(attn.cRSE) - 3, attn.quant_size, 2 * attn.quant_size))
+                    for index in indices]
+        else:
+            args = [index_arguments(index, local, extra) for index in indices]
+        if rows_in_window_order and args:
+            args[0] = args[0][:5] + (None,) + args[0][6:]      # (.., w2n, n2n, w2m, ..): no row map
         down = (self.downsample.plan(coords, stride, signals, num_batches, cell_index)
                 if self.downsample is not None else None)
         return args, down
@@ -482,8 +493,14 @@ class Stage(nn.Module):
         feats = voxels.feats
         pending = None
         if len(self.blocks) > 0 and self.blocks[0]._fused_path(feats):
-            for i, block in enumerate(self.blocks):
-                feats, pending = block.forward_fused(feats, pending, args[i % len(args)])
+            epoch = _cache_epoch()
+            done = swin_blocks(self, self.blocks._modules.values(), (SwinBlock, WindowAttention, Mlp), feats, args, epoch,
+                               lambda layer: _autocast_copy(layer, epoch))
+            if done is not None:
+                feats, pending = done
+            else:
+                for i, block in enumerate(self.blocks):
+                    feats, pending = block.forward_fused(feats, pending, args[i % len(args)])
             if self.downsample is None or not feats.is_contiguous():
                 feats, pending = feats + pending, None
             # else: the downsample's LayerNorm kernel adds the last MLP output, in place
@@ -518,7 +535,7 @@ def window_order(coords, stride, window_size):
     return n2n.long()      # coordinates out of the sort's range are reported by the stage's own index build
 
 
-def geometry_steps(stem_coords, stride, signals, layers, window_ordered=False):
+def geometry_steps(stem_coords, stride, signals, layers, window_ordered=False, num_batches=None):
     """Generator over the geometry of a forward pass, in the order the feature pass needs it: with window_ordered
     the permutation of the input rows (or None), then the stem convolution's neighbour rows, then the plan of every
     stage (finest first).  None of it depends on features.
@@ -536,7 +553,8 @@ def geometry_steps(stem_coords, stride, signals, layers, window_ordered=False):
             ordered = True
         yield order, coords, signals
     yield conv3x3x3_neighbours(coords, stride)
-    num_batches = int(coords[-1, 0]) + 1 if coords.shape[0] else 0    # batch ids are ascending: one read
+    if num_batches is None:
+        num_batches = count_batches(coords)
     for level, layer in enumerate(layers):
         plan = layer.plan(coords, stride, signals, num_batches, rows_in_window_order=ordered)
         ordered = False
@@ -555,16 +573,21 @@ def geometry_steps(stem_coords, stride, signals, layers, window_ordered=False):
             stride = stride * layer.downsample.factor
 
 
-def plan_stages(stem_coords, stride, signals, layers):
+def count_batches(coords):
+    """Batch elements of a voxel set: batch ids are ascending, so one read of the last row's."""
+    return int(coords[-1, 0]) + 1 if coords.shape[0] else 0
+
+
+def plan_stages(stem_coords, stride, signals, layers, num_batches=None):
     """(stem neighbours, [stage plans]) computed up front on the current stream."""
-    steps = list(geometry_steps(stem_coords, stride, signals, layers))
+    steps = list(geometry_steps(stem_coords, stride, signals, layers, num_batches=num_batches))
     return steps[0], steps[1:]
 
 
-def plan_stages_window_ordered(voxels, signals, layers):
+def plan_stages_window_ordered(voxels, signals, layers, num_batches=None):
     """As plan_stages, with every level in the order of its regular windows: -> (input voxels and signals in
     that order, the permutation applied to the input rows (long [N], or None), stem neighbours, [stage plans])."""
-    steps = list(geometry_steps(voxels.coords, voxels.stride, signals, layers, window_ordered=True))
+    steps = list(geometry_steps(voxels.coords, voxels.stride, signals, layers, window_ordered=True, num_batches=num_batches))
     order, coords, signals = steps[0]
     if order is not None:
         voxels = SparseVoxels(coords, voxels.feats[order], voxels.stride)
@@ -652,18 +675,19 @@ class Upsample(nn.Module):
         """LayerNorm + Linear; for inference under fp16 autocast the norm is the fused kernel that writes fp16."""
         if _fused_norm_applies(feats):
             _, normed = add_layernorm(feats, None, block[0])
-            return block[1](normed)
+            return _linear(block[1], normed)
         return block(feats)
 
-    def forward(self, voxels, signals, voxels_up, signals_up, plan_up=None):
+    def forward(self, voxels, signals, voxels_up, signals_up, plan_up=None, num_batches=None):
         """(voxels, signals): the coarse level; (voxels_up, signals_up): the finer level it feeds.  plan_up: a
         stage plan of the finer level's voxel set with the same window size (the encoder's, whose regular window
-        set is the one this level's attention block needs), so that the index is not built a second time."""
+        set is the one this level's attention block needs), so that the index is not built a second time.
+        num_batches: batch elements of both, where the caller knows it: the host then waits for nothing."""
         xyz = signals[:, 1:4].detach().contiguous().float()
         support_xyz = signals_up[:, 1:4].detach().contiguous().float()
         feats = self._norm_linear(self.linear1, voxels_up.feats) + knn_linear_interpolation(
             xyz, support_xyz, self._norm_linear(self.linear2, voxels.feats).float(),
-            segment_offsets(voxels.coords[:, 0]), segment_offsets(voxels_up.coords[:, 0]), K=self.up_k)
+            segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches), K=self.up_k)
         voxels_up = voxels_up.with_feats(feats.float())
         if self.attn:
             if plan_up is not None:
@@ -727,10 +751,11 @@ class Swin3DUNet(nn.Module):
     def forward(self, voxels, signals):
         """-> logits [N, num_classes] on the input voxels."""
         order = None
+        num_batches = count_batches(voxels.coords)
         if self.window_ordered:
-            voxels, signals, order, neighbours, plans = plan_stages_window_ordered(voxels, signals, self.layers)
+            voxels, signals, order, neighbours, plans = plan_stages_window_ordered(voxels, signals, self.layers, num_batches)
         else:
-            neighbours, plans = plan_stages(voxels.coords, voxels.stride, signals, self.layers)
+            neighbours, plans = plan_stages(voxels.coords, voxels.stride, signals, self.layers, num_batches)
         voxels = self.stem_layer(voxels, neighbours)
         levels = []
         for layer, plan in zip(self.layers, plans):
@@ -741,7 +766,7 @@ class Swin3DUNet(nn.Module):
         for level, upsample in zip(range(len(levels) - 1, -1, -1), self.upsamples):
             voxels_up, signals_up = levels.pop()
             # the decoder level works on the encoder level's voxels with the same window size: same window index
-            voxels = upsample(voxels, signals, voxels_up, signals_up, plans[level])
+            voxels = upsample(voxels, signals, voxels_up, signals_up, plans[level], num_batches)
             signals = signals_up
         logits = self.classifier(voxels.feats.float())
         if order is None:

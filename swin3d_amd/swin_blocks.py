@@ -1,0 +1,166 @@
+"""The Swin blocks of a stage at inference under fp16 autocast as one library call (s3d_swin_blocks): the host's share of
+a block through torch is some fifteen dispatches, several times what its kernels take on a small scan."""
+import ctypes
+
+import torch
+import torch.nn as nn
+from torch.nn.modules import module as _module_hooks
+
+from . import _lib
+from .sparse_dl.attn import attn_coff
+
+
+def _plain(m, kind):
+    """m is a `kind` (no subclass: it may compute something else) and nothing watches or replaces its forward."""
+    return type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+
+
+def _parts(block, kinds):
+    """(block, norm1, attn, qkv, proj, norm2, mlp, fc1, act, fc2), or None where one of them is not what it was built as."""
+    m = block._modules
+    attn, mlp = m["attn"], m["mlp"]
+    if not (_plain(block, kinds[0]) and _plain(attn, kinds[1]) and _plain(mlp, kinds[2])):
+        return None
+    a, f = attn._modules, mlp._modules
+    parts = (block, m["norm1"], attn, a["qkv"], a["proj"], m["norm2"], mlp, f["fc1"], f["act"], f["fc2"])
+    if not (_plain(parts[1], nn.LayerNorm) and _plain(parts[5], nn.LayerNorm) and _plain(parts[8], nn.GELU)
+            and parts[8].approximate == "none" and all(_plain(parts[i], nn.Linear) for i in (3, 4, 7, 9))):
+        return None
+    return parts
+
+
+def _stamp(parts):
+    """Addresses and versions of the parameters of the blocks."""
+    return [x for block in parts for i in (1, 2, 3, 4, 5, 7, 9) for p in block[i]._parameters.values() if p is not None
+            for x in (p.data_ptr(), p._version)]
+
+
+def _descriptions(parts, half_copy):
+    """The blocks as the library takes them, and the tensors they point to.  half_copy: (layer) -> its (weight, bias) in
+    fp16."""
+    kept, blocks = [], (_lib.SwinBlock * len(parts))()
+
+    def at(t):
+        if t is None:
+            return None
+        kept.append(t)
+        return t.data_ptr()
+
+    for b, (_, norm1, attn, _, proj, norm2, _, fc1, _, fc2) in zip(blocks, parts):
+        weight, bias, tables = attn._prepared()
+        b.qkv_weight, b.qkv_bias = at(weight.contiguous()), at(bias)
+        b.table_q, b.table_k, b.table_v = (at(t) for t in tables)
+        for name, layer in (("proj", proj), ("fc1", fc1), ("fc2", fc2)):
+            w, bias = half_copy(layer)
+            setattr(b, name + "_weight", at(w.contiguous()))
+            setattr(b, name + "_bias", at(bias))
+        for name, norm in (("norm1", norm1), ("norm2", norm2)):
+            setattr(b, name + "_weight", at(norm.weight.detach().float().contiguous()))
+            setattr(b, name + "_bias", at(norm.bias.detach().float().contiguous()))
+            setattr(b, name + "_eps", norm.eps)
+    return blocks, kept
+
+
+def _applicable(parts, channels):
+    attn, fc1 = parts[0][2], parts[0][7]
+    if attn.fp16_mode not in (1, 2) or attn.head_dim not in (8, 16, 32) or channels % 16 or fc1.out_features % 16:
+        return False
+    for _, norm1, a, qkv, proj, norm2, _, f1, _, f2 in parts:
+        if (a.num_heads, a.head_dim, a.fp16_mode, a.dim) != (attn.num_heads, attn.head_dim, attn.fp16_mode, channels) \
+                or list(a.table_sizes) != list(attn.table_sizes):
+            return False
+        for norm in (norm1, norm2):
+            if tuple(norm.normalized_shape) != (channels,) or norm.weight is None or norm.bias is None:
+                return False
+        shapes = [(qkv, channels, 3 * channels), (proj, channels, channels), (f1, channels, fc1.out_features),
+                  (f2, fc1.out_features, channels)]
+        if any((m.in_features, m.out_features) != (i, o) for m, i, o in shapes):
+            return False
+        # the fp16 copies of fp32 parameters on one device
+        if any(p.dtype != torch.float32 or p.device != qkv.weight.device
+               for m in (norm1, a, qkv, proj, norm2, f1, f2) for p in m._parameters.values() if p is not None):
+            return False
+    return True
+
+
+def linear_rows(x, weight, bias, gelu=False):
+    """x @ weight.T + bias (then GELU) of fp16 rows on the library's kernel (s3d_linear); None where it does not take the
+    operands."""
+    if x.dim() != 2 or any(t is not None and (t.dtype != torch.float16 or t.device != x.device) for t in (x, weight, bias)) \
+            or x.shape[1] % 16 or weight.shape[0] % 8 or not x.is_contiguous() or not weight.is_contiguous() \
+            or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return None
+    out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
+    with torch.cuda.device(x.device):
+        status = _lib.lib().s3d_linear(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
+                                       x.shape[0], weight.shape[0], x.shape[1], int(gelu),
+                                       torch.cuda.current_stream(x.device).cuda_stream)
+    _lib.check(status, "s3d_linear")
+    return out
+
+
+def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
+    """(feats, pending) behind the blocks, as their `forward_fused` one after the other would give it, or None where the
+    library call does not stand for them.
+
+    owner       the module that keeps the descriptions of the blocks between calls (`_s3d_blocks`), made anew when a
+                parameter, its version or `epoch` has changed
+    kinds       (block, attention, MLP) types the blocks have to be of
+    feats       fp32 [N,C]; left as it is
+    index_sets  per window set what index_arguments and window_signals give
+    """
+    n, channels = feats.shape
+    if n == 0 or _module_hooks._global_forward_hooks or _module_hooks._global_forward_pre_hooks:
+        return None
+    if type(feats) is not torch.Tensor or any(len(s) < 9 for s in index_sets):
+        return None
+    parts = [_parts(b, kinds) for b in blocks]
+    if any(p is None for p in parts):
+        return None
+    key = (epoch, _stamp(parts), [m for p in parts for m in p])
+    kept = getattr(owner, "_s3d_blocks", None)
+    if kept is None or kept[0] != key:
+        kept = (key, _descriptions(parts, half_copy) if _applicable(parts, channels) else None)
+        owner._s3d_blocks = kept
+    if kept[1] is None:
+        return None
+    described, tensors = kept[1]
+    dev = feats.device
+    if tensors[0].device != dev:
+        return None
+    attn, hidden = parts[0][2], parts[0][7].out_features
+    heads, dim, sizes = attn.num_heads, attn.head_dim, attn.table_sizes
+    nd, table_len = len(sizes), sum(sizes)
+    c_sizes = (ctypes.c_int32 * nd)(*sizes)
+    lib = _lib.lib()
+    feats = feats.contiguous()
+    out = torch.empty_like(feats)
+    pending = torch.empty((n, channels), dtype=torch.float16, device=dev)
+    ws_bytes = lib.s3d_swin_blocks_workspace_bytes(n, channels, hidden)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    sets = (_lib.WindowSet * len(index_sets))()
+    held = []
+    with torch.cuda.device(dev):
+        stream = torch.cuda.current_stream(dev).cuda_stream
+        for s, args in zip(sets, index_sets):
+            _, _, _, w_sizes_in, w2n_in, n2n, _, _, coords = args[:9]
+            w_sizes, w2n = (attn_coff._as_int32(name, t, dev) for name, t in (("w_sizes", w_sizes_in), ("w2n", w2n_in)))
+            n2n = None if n2n is None else attn_coff._as_int32("n2n", n2n, dev)
+            coords = coords.float().contiguous()
+            if w_sizes.dim() != 1 or w2n.shape != w_sizes.shape or coords.shape != (n, nd) or coords.device != dev \
+                    or (n2n is not None and n2n.shape != (n,)):
+                return None
+            plan = attn_coff._plan_for(lib, w_sizes_in, w2n_in, w_sizes, w2n, c_sizes, sizes, nd, table_len, n, heads, dim,
+                                       _lib.S3D_DTYPE_F16, stream) if attn_coff.REUSE_PLANS else None
+            s.planned = plan is not None
+            if plan is None:
+                plan = torch.empty(lib.s3d_attn_plan_bytes(heads, n, w_sizes.numel()), dtype=torch.uint8, device=dev)
+            held.append((w_sizes, w2n, n2n, coords, plan))
+            s.w_sizes, s.w2n, s.n_coords = w_sizes.data_ptr(), w2n.data_ptr(), coords.data_ptr()
+            s.n2n = None if n2n is None else n2n.data_ptr()
+            s.num_windows, s.plan, s.plan_bytes = w_sizes.numel(), plan.data_ptr(), plan.numel()
+        status = lib.s3d_swin_blocks(
+            feats.data_ptr(), out.data_ptr(), pending.data_ptr(), n, heads, dim, hidden, c_sizes, nd, table_len, sets,
+            len(sets), described, len(described), workspace.data_ptr(), ws_bytes, stream)
+    _lib.check(status, "s3d_swin_blocks")
+    return out, pending

@@ -1,0 +1,69 @@
+"""s3d_linear against an fp32 product at the edges of its tiles and of its dispatch, and the blocks of a stage in one call
+against the blocks one by one."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from swin3d_amd import _lib, encoder, synth
+from swin3d_amd.swin_blocks import linear_rows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 16), (63, 48, 48), (65, 144, 80), (200, 72, 640),       # 64 x 64 tiles, remainders on every side
+    (66000, 48, 64), (40001, 80, 48),                              # 128 x 64 and 128 x 128
+    (45000, 192, 96), (33000, 144, 16),                            # 128 x 192
+    (9001, 640, 80), (4100, 1152, 192),                            # several columns of tiles
+])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear(hip_lib, m, n, k, gelu):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w, b = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k), (n,)))
+    w = (w.float() * k ** -0.5).half()
+    ref = F.linear(x.float(), w.float(), b.float())
+    for bias, want in ((b, ref), (None, ref - b.float())):
+        want = F.gelu(want) if gelu else want
+        got = linear_rows(x, w, bias, gelu).float()
+        assert float((got - want).abs().max()) <= 1e-3 * float(want.abs().max())
+        assert bool(((got - want).abs() <= 6e-4 * want.abs() + 2e-6 * float(want.abs().max()) + 6e-7).all())
+
+
+def test_linear_refuses_what_it_cannot_do(hip_lib):
+    x, w = torch.randn(5, 24, device="cuda").half(), torch.randn(8, 24, device="cuda").half()
+    assert linear_rows(x, w, None) is None and linear_rows(x.float(), w.float(), None) is None
+    assert _lib.lib().s3d_linear(x.data_ptr(), w.data_ptr(), None, x.data_ptr(), 5, 8, 24, 0, None) < 0
+
+
+@pytest.mark.parametrize("heads,dim,window,mode", [(6, 8, 5, 2), (5, 16, 7, 1)])
+def test_blocks_in_one_call_equal_single_blocks(hip_lib, heads, dim, window, mode):
+    """Same launches but for the GELU (fused with fc1, which then is not rounded in between) and the products' order of
+    summation; hooks and changed parameters are noticed."""
+    dev = torch.device("cuda")
+    scene = synth.make_room((3.0, 3.0, 2.0), 4, 5000, seed=5)
+    coords = torch.from_numpy(scene.coords).to(dev)
+    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)
+    torch.manual_seed(1)
+    stage = encoder.Stage(heads * dim, 3, heads, window, 4, downsample=False, cRSE="XYZ_RGB_NORM", fp16_mode=mode).to(dev).eval()
+    for name, p in stage.named_parameters():
+        if "table" in name or "bias" in name:
+            torch.nn.init.normal_(p, std=0.1)
+    feats = torch.randn(coords.shape[0], heads * dim, device=dev)
+    kept, calls = feats.clone(), []
+
+    def both():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            plan = stage.plan(coords, 1, signals)
+            one, _, _ = stage(encoder.SparseVoxels(coords, feats, 1), signals, plan)
+            hook = stage.blocks[1].mlp.act.register_forward_hook(lambda *_: calls.append(1))
+            single, _, _ = stage(encoder.SparseVoxels(coords, feats, 1), signals, plan)
+            hook.remove()
+        assert (one.feats - single.feats).abs().max() <= 2e-3 * single.feats.abs().max()
+        return one.feats
+
+    first = both()
+    assert len(calls) == 1 and torch.equal(feats, kept) and hasattr(stage, "_s3d_blocks")
+    assert torch.equal(both(), first)
+    with torch.no_grad():
+        stage.blocks[2].mlp.fc2.weight.mul_(3.0)
+    assert (both() - first).abs().max() > 1e-2 * first.abs().max()
