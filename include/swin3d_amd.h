@@ -250,7 +250,7 @@ int s3d_window_index(const int32_t *coords, int64_t N, int32_t stride, int32_t w
 /*
  * The same index by a counting sort over the lattice of windows, for scenes whose windows fit a dense lattice of
  * at most max(4096, 2 N) cells (capped at 2^24): the bounding box of (batch, wx, wy, wz) over the voxels.  Room-sized
- * scenes do; the call is then five launches of a few microseconds instead of a sort of all voxels.  Same arguments
+ * scenes do; the call is then six launches of a few microseconds instead of a sort of all voxels.  Same arguments
  * and outputs as s3d_window_index (the results are identical, rows of equal coordinates in row order); own
  * workspace size.  When the lattice is too large, counts[3] has bit 1 (value 2) set and NO output is written: call
  * s3d_window_index instead.  counts[3] bit 0 (value 1): coordinates out of range, as for s3d_window_index.
@@ -259,6 +259,19 @@ size_t s3d_window_index_grid_workspace_bytes(int64_t N);
 int s3d_window_index_grid(const int32_t *coords, int64_t N, int32_t stride, int32_t window,
                           int32_t shift, int32_t *n2n, int32_t *w_w_id, int32_t *w_sizes, int32_t *w2n,
                           int64_t *counts, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * s3d_window_index_grid for up to four window sets of the same voxels in one run of launches.  sets: HOST array.
+ */
+typedef struct {
+    int32_t *n2n, *w_w_id, *w_sizes, *w2n;   /* device int32 [N] out, as for s3d_window_index_grid */
+    int64_t *counts;                         /* device int64 [4] out */
+    int32_t window, shift;
+} s3d_window_index_set;
+
+size_t s3d_window_indices_workspace_bytes(int64_t N, int32_t num_sets);
+int s3d_window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets,
+                       void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * Representative voxel of every cell of a window sort: the member whose signal row is nearest (Euclidean, fp32) to
@@ -334,6 +347,10 @@ int s3d_knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz,
             const int32_t *src_offset, const int32_t *query_offset, int32_t B, int32_t *ret_idx,
             float *ret_dist2, float cell_size, void *workspace, size_t workspace_bytes,
             void *stream);
+/* The same with Euclidean distances (the square roots, sqrt(S3D_KNN_PAD_DIST2) for padded slots) in ret_dist. */
+int s3d_knn_distances(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int64_t Nq,
+                      const int32_t *src_offset, const int32_t *query_offset, int32_t B, int32_t *ret_idx,
+                      float *ret_dist, float cell_size, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * Inverse-distance interpolation of source features at the queries, from the result of s3d_knn.

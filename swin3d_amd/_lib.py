@@ -3,8 +3,11 @@
 There is no fallback: if the shared library is missing or a call fails, a
 RuntimeError is raised.
 """
+import contextlib
 import ctypes
 import os
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libswin3d_amd.so")
@@ -26,6 +29,10 @@ _i64 = ctypes.c_int64
 class WindowSet(ctypes.Structure):
     _fields_ = [(n, _vp) for n in ("w_sizes", "w2n", "n2n", "n_coords")] + [
         ("num_windows", _i64), ("plan", _vp), ("plan_bytes", ctypes.c_size_t), ("planned", _i32)]
+
+
+class WindowIndexSet(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("n2n", "w_w_id", "w_sizes", "w2n", "counts")] + [("window", _i32), ("shift", _i32)]
 
 
 class SwinBlock(ctypes.Structure):
@@ -53,12 +60,16 @@ SIGNATURES = {
     "s3d_window_index": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),
     "s3d_window_index_grid_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_window_index_grid": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),
+    "s3d_window_indices_workspace_bytes": (ctypes.c_size_t, [_i64, _i32]),
+    "s3d_window_indices": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_cell_representatives": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp, _vp]),
     "s3d_key_neighbours": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i32, _vp, _vp]),
     "s3d_window_signals": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _i32, _i32, ctypes.c_float, ctypes.c_float, _vp,
                                           _i64, _vp]),
     "s3d_knn_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i32]),
     "s3d_knn": (ctypes.c_int, [_i32, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _vp, _vp, ctypes.c_float,
+                               _vp, ctypes.c_size_t, _vp]),
+    "s3d_knn_distances": (ctypes.c_int, [_i32, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _vp, _vp, ctypes.c_float,
                                _vp, ctypes.c_size_t, _vp]),
     "s3d_knn_interpolate": (ctypes.c_int, [_vp, _vp, _i32, _i64, _vp, _i64, _i32, _i32, _vp, _vp]),
     "s3d_knn_max_pool": (ctypes.c_int, [_vp, _i32, _i64, _vp, _i64, _i32, _i32, _vp, _vp]),
@@ -86,6 +97,20 @@ def lib():
             fn.argtypes = argtypes
         _lib = handle
     return _lib
+
+
+_HERE_ALREADY = contextlib.nullcontext()
+
+
+def on(device):
+    """Context with `device` (that of a CUDA tensor) as the current one; nothing to do where it is so already, which is
+    a tenth of what torch.cuda.device costs the host."""
+    return _HERE_ALREADY if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def stream(device):
+    """The current stream of `device` as the library takes it."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def check(status, what):

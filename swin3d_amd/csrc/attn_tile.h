@@ -92,13 +92,15 @@ constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 
 __device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
 __device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
 
-// Unit list: windows in bins of equal size, largest first (a counting sort in LDS; the order inside a bin is of no
-// consequence, no result depends on which windows share a unit), and the pairs of the windows before each.
+// Unit list: windows in bins of equal size, largest first (a counting sort in LDS), and the pairs of the windows before
+// each.  Inside a bin the windows keep their order: where a window lies in its unit decides in which order the matrix pipe
+// adds its products, and a result is to be the same bits on every call.
 __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
                                            int32_t *__restrict__ total, int4 *__restrict__ units, int2 *__restrict__ entries)
 {
     __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
-    __shared__ int wave_pairs[kListThreads / 64];
+    constexpr int kWavesOfList = kListThreads / 64;
+    __shared__ int wave_pairs[kWavesOfList], of_wave[kWavesOfList][kListBins];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (t < kListBins) windows[t] = big_units[t] = 0;
     __syncthreads();
@@ -144,25 +146,52 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
             if (lane >= off) incl += up;
         }
         if (lane == 63) wave_pairs[wave] = incl;
+        for (int i = t; i < kWavesOfList * kListBins; i += kListThreads) of_wave[0][i] = 0;
         __syncthreads();
+        // a window's place among those of its bin: in its wavefront, then behind the wavefronts before
+        const int b = n > 0 ? list_bin(n) : -1;
+        int rank = 0;
+        for (unsigned long long left = __ballot(b >= 0); left;) {
+            const int bin = __builtin_amdgcn_readlane(b, __ffsll(static_cast<long long>(left)) - 1);
+            const unsigned long long same = __ballot(b == bin);
+            if (b == bin) rank = __popcll(same & ((1ull << lane) - 1));
+            if (lane == 0) of_wave[wave][bin] = __popcll(same);
+            left &= ~same;
+        }
         int pairs = before + incl - own, all = 0;
 #pragma unroll
-        for (int v = 0; v < kListThreads / 64; ++v) {
+        for (int v = 0; v < kWavesOfList; ++v) {
             pairs += v < wave ? wave_pairs[v] : 0;
             all += wave_pairs[v];
         }
         before += all;
         __syncthreads();
-        if (n <= 0) continue;
-        const int b = list_bin(n), e = atomicAdd(&entry_at[b], 1);
-        entries[e] = make_int2(w2n[w], pairs);
-        if (n > kCols) {
-            const int tiles = tiles_of(n), u = atomicAdd(&unit_at[b], tiles);
-            for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
-        } else {
-            const int per = kCols / n, rank = e - entry_first[b];
-            if (rank % per == 0) units[unit_at[b] + rank / per] = make_int4(e, n, min(per, windows[b] - rank), 0);
+        if (t < kListBins) {
+            int count[kWavesOfList], run = entry_at[t];
+#pragma unroll
+            for (int v = 0; v < kWavesOfList; ++v) count[v] = of_wave[v][t];
+#pragma unroll
+            for (int v = 0; v < kWavesOfList; ++v) {
+                of_wave[v][t] = run;
+                run += count[v];
+            }
+            entry_at[t] = run;
         }
+        __syncthreads();
+        if (b >= 0) {
+            const int e = of_wave[wave][b] + rank, in_bin = e - entry_first[b];
+            entries[e] = make_int2(w2n[w], pairs);
+            if (n > kCols) {
+                const int tiles = tiles_of(n);
+                // (the windows of the first bin differ in their tiles)
+                const int u = b > 0 ? unit_at[b] + in_bin * tiles : atomicAdd(&unit_at[b], tiles);
+                for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
+            } else {
+                const int per = kCols / n;
+                if (in_bin % per == 0) units[unit_at[b] + in_bin / per] = make_int4(e, n, min(per, windows[b] - in_bin), 0);
+            }
+        }
+        __syncthreads();
     }
 }
 

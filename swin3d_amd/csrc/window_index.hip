@@ -163,11 +163,28 @@ __global__ __launch_bounds__(kThreads) void segment_size_kernel(const int32_t *_
 // lattice is the bounding box of the window coordinates), a window is a lattice cell and the index is a counting
 // sort: every voxel draws a slot in its cell, a scan over the cells gives every non-empty cell its rank (= window
 // number, ascending (batch, wx, wy, wz) because the cell number is) and its first position, the voxels are placed
-// there, and each window's few voxels are put in (local id, row) order by one wavefront.  Five launches of a few
+// there, and each window's few voxels are put in (local id, row) order by one wavefront.  Six launches of a few
 // microseconds instead of a block sort and eight merge passes.
+//
+// Up to kMaxSets window sets of the same voxels are built together (blockIdx.y = set): what bounds a set alone is the
+// launches, each with too little work for the card (199,327 voxels, two sets: 46 us of kernels instead of 73).  The lattices come from one bounding box of the coordinates (a
+// window coordinate does not decrease with its voxel's), and one scan runs over the cells of all sets.
 constexpr int kGridBoxes = 128;          // workgroups of the bounding-box pass
 constexpr int kSlotBits = 20;            // a voxel's slot in its cell, below its local id in one word
 constexpr int kBadRange = 1, kNoGrid = 2;   // counts[3]: coordinates out of range / lattice too large for the grid path
+
+constexpr int kMaxSets = 4;
+
+struct GridSet {
+    int window, shift;
+    int32_t *n2n, *w_w_id, *w_sizes, *w2n;
+    int64_t *counts;
+};
+
+struct GridSets {
+    GridSet set[kMaxSets];
+    int num;
+};
 
 struct GridPlan {
     int lo[4], dim[4];   // batch, wx, wy, wz: lowest value and extent of the lattice
@@ -206,19 +223,20 @@ size_t grid_scan_temp_bytes(int64_t n)
     return bytes;
 }
 
-GridLayout make_grid_layout(int64_t N)
+// plans, cells, scan, place and keys: one of each per set, one behind the other
+GridLayout make_grid_layout(int64_t N, int sets)
 {
     GridLayout L{};
     L.cells_cap = grid_cells_cap(N);
-    const size_t n = static_cast<size_t>(N > 0 ? N : 1), cells = static_cast<size_t>(L.cells_cap) + 1;
+    const size_t n = static_cast<size_t>(N > 0 ? N : 1) * sets, cells = (static_cast<size_t>(L.cells_cap) + 1) * sets;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
         off = align_up(off + bytes, 256);
         return at;
     };
-    L.plan = take(sizeof(GridPlan));
-    L.partials = take(sizeof(int32_t) * 9 * kGridBoxes);
+    L.plan = take(sizeof(GridPlan) * sets);
+    L.partials = take(sizeof(int32_t) * 8 * kGridBoxes);
     L.cells = take(cells * sizeof(int32_t));
     L.scan = take(cells * sizeof(uint64_t));
     L.place = take(n * sizeof(int2));
@@ -248,26 +266,26 @@ __device__ __forceinline__ bool window_of(const int4 c, int stride, int window, 
     return !bad;
 }
 
-// partial bounding boxes of the window coordinates (one per workgroup, no atomics), the cell counters and the
-// call's totals and status word at zero (the later launches only ever OR bits into the status word)
-__global__ __launch_bounds__(kThreads) void grid_bbox_kernel(const int32_t *__restrict__ coords, int64_t N, int stride,
-                                                             int window, int shift, int32_t *__restrict__ partials,
-                                                             int32_t *__restrict__ cells, int64_t num_cells,
-                                                             int64_t *__restrict__ counts)
+// partial bounding boxes of the coordinates (one per workgroup, no atomics), the cell counters and the sets' totals and
+// status words at zero (the later launches only ever OR bits into a status word)
+__global__ __launch_bounds__(kThreads) void grid_bbox_kernel(const int32_t *__restrict__ coords, int64_t N, GridSets sets,
+                                                             int32_t *__restrict__ partials, int32_t *__restrict__ cells,
+                                                             int64_t num_cells)
 {
-    if (blockIdx.x == 0 && threadIdx.x < 4) counts[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 4)
+        for (int s = 0; s < sets.num; ++s) sets.set[s].counts[threadIdx.x] = 0;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < num_cells;
          i += static_cast<int64_t>(gridDim.x) * kThreads)
         cells[i] = 0;
-    int lo[4], hi[4], bad = 0;
+    int lo[4], hi[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) { lo[a] = 0x7fffffff; hi[a] = static_cast<int>(0x80000000u); }
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < N;
          i += static_cast<int64_t>(gridDim.x) * kThreads) {
-        int w[4], local;
-        if (!window_of(reinterpret_cast<const int4 *>(coords)[i], stride, window, shift, w, &local)) bad = 1;
+        const int4 c = reinterpret_cast<const int4 *>(coords)[i];
+        const int x[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
-        for (int a = 0; a < 4; ++a) { lo[a] = min(lo[a], w[a]); hi[a] = max(hi[a], w[a]); }
+        for (int a = 0; a < 4; ++a) { lo[a] = min(lo[a], x[a]); hi[a] = max(hi[a], x[a]); }
     }
     for (int off = 32; off > 0; off >>= 1) {
 #pragma unroll
@@ -275,69 +293,66 @@ __global__ __launch_bounds__(kThreads) void grid_bbox_kernel(const int32_t *__re
             lo[a] = min(lo[a], __shfl_down(lo[a], off));
             hi[a] = max(hi[a], __shfl_down(hi[a], off));
         }
-        bad |= __shfl_down(bad, off);
     }
-    __shared__ int part[kThreads / 64][9];
+    __shared__ int part[kThreads / 64][8];
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int a = 0; a < 4; ++a) { part[threadIdx.x >> 6][a] = lo[a]; part[threadIdx.x >> 6][4 + a] = hi[a]; }
-        part[threadIdx.x >> 6][8] = bad;
     }
     __syncthreads();
-    if (threadIdx.x < 9) {
+    if (threadIdx.x < 8) {
         int v = part[0][threadIdx.x];
         for (int wv = 1; wv < kThreads / 64; ++wv)
-            v = threadIdx.x < 4 ? min(v, part[wv][threadIdx.x]) : max(v, part[wv][threadIdx.x]);   // the flag: max = or
-        partials[blockIdx.x * 9 + threadIdx.x] = v;
+            v = threadIdx.x < 4 ? min(v, part[wv][threadIdx.x]) : max(v, part[wv][threadIdx.x]);
+        partials[threadIdx.x * kGridBoxes + blockIdx.x] = v;
     }
 }
 
-// Every workgroup reduces the partial boxes to the lattice (workgroup 0 records it and its bits of the status word);
-// then every voxel draws a slot in its cell - neighbouring lanes of one cell with one atomic.  A cell that runs
-// out of slot numbers (more than 2^kSlotBits voxels in one window: only with masses of equal coordinates) sets the
+// Every workgroup reduces the partial boxes to its set's lattice (workgroup 0 of a set records it and its bits of the
+// status word); then every voxel draws a slot in its cell - neighbouring lanes of one cell with one atomic.  A cell that
+// runs out of slot numbers (more than 2^kSlotBits voxels in one window: only with masses of equal coordinates) sets the
 // "no grid" bit as well: the status word was zeroed by the launch before this one and every writer ORs into it, so
 // no bit is lost whichever workgroup comes first, and the later launches of the call write nothing once it is set.
 __global__ __launch_bounds__(kThreads) void grid_count_kernel(
-    const int32_t *__restrict__ coords, int64_t N, int stride, int window, int shift,
-    const int32_t *__restrict__ partials, int64_t cells_cap, GridPlan *__restrict__ plan_out,
-    int32_t *__restrict__ cells, int2 *__restrict__ place, int64_t *__restrict__ counts)
+    const int32_t *__restrict__ coords, int64_t N, int stride, GridSets sets, const int32_t *__restrict__ partials,
+    int64_t cells_cap, GridPlan *__restrict__ plan_out, int32_t *__restrict__ cells, int2 *__restrict__ place)
 {
     __shared__ GridPlan plan;
-    __shared__ int part[kThreads / 64][9];
+    __shared__ int box[8];
+    const int set = blockIdx.y, window = sets.set[set].window, shift = sets.set[set].shift;
+    int64_t *counts = sets.set[set].counts;
+    cells += set * (cells_cap + 1);
+    place += set * N;
     {
-        int v[9];
+        // eight numbers by 32 lanes each
+        static_assert(kThreads == 8 * 32 && kGridBoxes % 32 == 0, "a thread per part of a number");
+        const int a = threadIdx.x >> 5;
+        int v = partials[a * kGridBoxes + (threadIdx.x & 31)];
 #pragma unroll
-        for (int a = 0; a < 9; ++a) v[a] = a < 4 ? 0x7fffffff : static_cast<int>(0x80000000u);
-        for (int t = threadIdx.x; t < kGridBoxes; t += kThreads)
-#pragma unroll
-            for (int a = 0; a < 9; ++a) v[a] = a < 4 ? min(v[a], partials[t * 9 + a]) : max(v[a], partials[t * 9 + a]);
-#pragma unroll
-        for (int a = 0; a < 9; ++a)
-            for (int off = 32; off > 0; off >>= 1) {
-                const int o = __shfl_down(v[a], off);
-                v[a] = a < 4 ? min(v[a], o) : max(v[a], o);
-            }
-        if ((threadIdx.x & 63) == 0)
-#pragma unroll
-            for (int a = 0; a < 9; ++a) part[threadIdx.x >> 6][a] = v[a];
+        for (int t = 32; t < kGridBoxes; t += 32) {
+            const int o = partials[a * kGridBoxes + t + (threadIdx.x & 31)];
+            v = a < 4 ? min(v, o) : max(v, o);
+        }
+        for (int off = 16; off > 0; off >>= 1) {
+            const int o = __shfl_down(v, off, 32);
+            v = a < 4 ? min(v, o) : max(v, o);
+        }
+        if ((threadIdx.x & 31) == 0) box[a] = v;
         __syncthreads();
         if (threadIdx.x == 0) {
-            int r[9];
-            for (int a = 0; a < 9; ++a) {
-                r[a] = part[0][a];
-                for (int wv = 1; wv < kThreads / 64; ++wv) r[a] = a < 4 ? min(r[a], part[wv][a]) : max(r[a], part[wv][a]);
-            }
+            int lo[4], hi[4], local;
+            const bool good = window_of(make_int4(box[0], box[1], box[2], box[3]), stride, window, shift, lo, &local) &
+                              window_of(make_int4(box[4], box[5], box[6], box[7]), stride, window, shift, hi, &local);
             double total = 1.0;
-            for (int a = 0; a < 4; ++a) {
-                plan.lo[a] = r[a];
-                plan.dim[a] = r[4 + a] - r[a] + 1;
-                total *= static_cast<double>(plan.dim[a]);
+            for (int x = 0; x < 4; ++x) {
+                plan.lo[x] = lo[x];
+                plan.dim[x] = hi[x] - lo[x] + 1;
+                total *= static_cast<double>(plan.dim[x]);
             }
-            const bool bad = r[8] > 0;
-            plan.ok = !bad && total <= static_cast<double>(cells_cap);
+            plan.ok = good && total <= static_cast<double>(cells_cap);
             if (blockIdx.x == 0) {
-                *plan_out = plan;
-                const unsigned long long bits = (bad ? kBadRange : 0) | (plan.ok ? 0 : kNoGrid);
+                plan_out[set] = plan;
+                const unsigned long long bits = (good ? 0 : kBadRange) | (plan.ok ? 0 : kNoGrid);
                 if (bits) atomicOr(reinterpret_cast<unsigned long long *>(counts + 3), bits);
             }
         }
@@ -371,24 +386,30 @@ __global__ __launch_bounds__(kThreads) void grid_count_kernel(
 }
 
 // every voxel to its window's segment (slot order); the voxel in slot 0 also records the window
-__global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__restrict__ place, int64_t N,
+__global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__restrict__ place, int64_t N, GridSets sets,
                                                               const GridPlan *__restrict__ plan,
                                                               const uint64_t *__restrict__ scan, int64_t cells_cap,
-                                                              uint64_t *__restrict__ keys, int32_t *__restrict__ w2n,
-                                                              int32_t *__restrict__ w_sizes, int64_t *__restrict__ counts)
+                                                              uint64_t *__restrict__ keys)
 {
-    if (!plan->ok || (counts[3] & kNoGrid)) return;
+    const int set = blockIdx.y;
+    int64_t *counts = sets.set[set].counts;
+    int32_t *w2n = sets.set[set].w2n, *w_sizes = sets.set[set].w_sizes;
+    if (!plan[set].ok || (counts[3] & kNoGrid)) return;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i == 0) counts[0] = static_cast<int64_t>(scan[cells_cap] >> 32);   // non-empty cells before the end = windows
+    scan += set * (cells_cap + 1);
+    place += set * N;
+    keys += set * N;
+    const uint64_t before = scan[0];       // windows and voxels of the sets before this one
+    if (i == 0) counts[0] = static_cast<int64_t>((scan[cells_cap] - before) >> 32);   // non-empty cells = windows
     if (i >= N) return;
     const int2 p = place[i];
-    const uint64_t here = scan[p.x];
+    const uint64_t here = scan[p.x] - before;
     const int start = static_cast<int>(here & 0xffffffffu), slot = p.y & ((1 << kSlotBits) - 1);
     keys[start + slot] = (static_cast<uint64_t>(p.y >> kSlotBits) << 32) | static_cast<uint32_t>(i);
     if (slot == 0) {
         const int rank = static_cast<int>(here >> 32);
         w2n[rank] = start;
-        w_sizes[rank] = static_cast<int>(scan[p.x + 1] & 0xffffffffu) - start;
+        w_sizes[rank] = static_cast<int>((scan[p.x + 1] - before) & 0xffffffffu) - start;
     }
 }
 
@@ -396,13 +417,14 @@ __global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__rest
 // the number of smaller ones, counted against every element of the window (a few dozen to a few hundred voxels).
 // Also the totals: sum of squared sizes and the largest size, one pair of atomics per workgroup.
 __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__restrict__ plan,
-                                                              const uint64_t *__restrict__ keys,
-                                                              const int32_t *__restrict__ w2n,
-                                                              const int32_t *__restrict__ w_sizes,
-                                                              int32_t *__restrict__ n2n, int32_t *__restrict__ w_w_id,
-                                                              int64_t *__restrict__ counts)
+                                                              const uint64_t *__restrict__ keys, int64_t N, GridSets sets)
 {
-    if (!plan->ok || (counts[3] & kNoGrid)) return;
+    const int set = blockIdx.y;
+    const int32_t *w2n = sets.set[set].w2n, *w_sizes = sets.set[set].w_sizes;
+    int32_t *n2n = sets.set[set].n2n, *w_w_id = sets.set[set].w_w_id;
+    int64_t *counts = sets.set[set].counts;
+    if (!plan[set].ok || (counts[3] & kNoGrid)) return;
+    keys += set * N;
     constexpr int kOrderStage = 512;                       // keys of a window staged in LDS at a time, per wavefront
     constexpr int kTotalGroups = 32;
     __shared__ uint64_t stage_all[kThreads / 64][kOrderStage];
@@ -479,28 +501,32 @@ __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__
     }
 }
 
-// one thread per (sorted position, column); the add and the multiply stay separate roundings, as in the
-// reference's tensor statement (sum, then scale)
+// A thread per sorted position reads its voxel's row; the matrix leaves through LDS, a workgroup's rows in one piece (a
+// thread per element divides by the columns and reads n2n nine times: 10.7 us for 199,327 x 9).  The add and the multiply
+// stay separate roundings, as in the reference's tensor statement (sum, then scale).
 __global__ __launch_bounds__(kThreads) void window_signals_kernel(
     const int32_t *__restrict__ w_w_id, const int32_t *__restrict__ n2n, const float *__restrict__ frac,
     const float *__restrict__ signals, int64_t signals_stride, int columns, int window, float xyz_scale,
-    float other_scale, float *__restrict__ out, int64_t N)
+    float other_scale, float *__restrict__ out, int64_t N, int rows)
 {
 #pragma clang fp contract(off)
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (t >= N * columns) return;
-    const int64_t p = t / columns;
-    const int c = static_cast<int>(t - p * columns);
-    const int64_t row = n2n[p];
-    float v;
-    if (c < 3) {
+    extern __shared__ float tile[];
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * rows, p = p0 + threadIdx.x;
+    if (static_cast<int>(threadIdx.x) < rows && p < N) {
+        float *to = tile + threadIdx.x * columns;
+        const int64_t row = n2n[p];
         const int id = w_w_id[p];
-        const int cell = c == 0 ? id / (window * window) : c == 1 ? (id / window) % window : id % window;
-        v = (static_cast<float>(cell) + frac[row * 3 + c]) * xyz_scale;
-    } else {
-        v = signals[row * signals_stride + (c - 3)] * other_scale;
+        const int x = id / (window * window), rest = id - x * (window * window), y = rest / window, z = rest - y * window;
+        to[0] = (static_cast<float>(x) + frac[row * 3]) * xyz_scale;
+        to[1] = (static_cast<float>(y) + frac[row * 3 + 1]) * xyz_scale;
+        to[2] = (static_cast<float>(z) + frac[row * 3 + 2]) * xyz_scale;
+        const float *from = signals + row * signals_stride;
+#pragma unroll 6
+        for (int c = 3; c < columns; ++c) to[c] = from[c - 3] * other_scale;
     }
-    out[t] = v;
+    __syncthreads();
+    const int here = static_cast<int>(min(static_cast<int64_t>(rows), N - p0)) * columns;
+    for (int t = threadIdx.x; t < here; t += kThreads) out[p0 * columns + t] = tile[t];
 }
 
 // one thread per (sorted voxel, offset): binary search of key + delta in the sorted keys
@@ -618,9 +644,13 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_signals(
     if (!w_w_id || !n2n || !frac || !out || (num_signals > 0 && !signals))
         return fail(S3D_ERR_NULL_POINTER, "s3d_window_signals: null device pointer");
     const int columns = 3 + num_signals;
-    const dim3 grid(static_cast<unsigned>(ceil_div(N * columns, kThreads)));
-    hipLaunchKernelGGL(window_signals_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), w_w_id, n2n,
-                       frac, signals, signals_stride, columns, window, xyz_scale, other_scale, out, N);
+    // as many rows a workgroup as half of the LDS of a launch without special attributes takes
+    if (columns > 8192) return fail(S3D_ERR_BAD_SHAPE, "s3d_window_signals: num_signals=%d", num_signals);
+    const int rows = columns <= 8192 / kThreads ? kThreads : 8192 / columns;
+    const dim3 grid(static_cast<unsigned>(ceil_div(N, rows)));
+    const uint32_t lds = rows * columns * sizeof(float);
+    hipLaunchKernelGGL(window_signals_kernel, grid, dim3(kThreads), lds, static_cast<hipStream_t>(stream), w_w_id, n2n,
+                       frac, signals, signals_stride, columns, window, xyz_scale, other_scale, out, N, rows);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
@@ -681,35 +711,43 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_index(const int
     return S3D_OK;
 }
 
-extern "C" __attribute__((visibility("default"))) size_t s3d_window_index_grid_workspace_bytes(int64_t N)
+extern "C" __attribute__((visibility("default"))) size_t s3d_window_indices_workspace_bytes(int64_t N, int32_t num_sets)
 {
-    return s3d::make_grid_layout(N).total;
+    return num_sets < 1 || num_sets > s3d::kMaxSets ? 0 : s3d::make_grid_layout(N, num_sets).total;
 }
 
-extern "C" __attribute__((visibility("default"))) int s3d_window_index_grid(
-    const int32_t *coords, int64_t N, int32_t stride, int32_t window, int32_t shift, int32_t *n2n, int32_t *w_w_id,
-    int32_t *w_sizes, int32_t *w2n, int64_t *counts, void *workspace, size_t workspace_bytes, void *stream)
+extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
+    const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *jobs, int32_t num_sets, void *workspace,
+    size_t workspace_bytes, void *stream)
 {
     using namespace s3d;
-    if (N < 0 || N > 0x7fffffffLL)
-        return fail(S3D_ERR_BAD_SHAPE, "s3d_window_index_grid: N=%lld out of range", (long long)N);
-    if (stride < 1 || window < 1 || window > 10 || shift < 0 || shift >= window)
-        return fail(S3D_ERR_BAD_SHAPE, "s3d_window_index_grid: stride=%d window=%d shift=%d (need stride>=1, "
-                    "1<=window<=10, 0<=shift<window)", stride, window, shift);
-    if (!counts) return fail(S3D_ERR_NULL_POINTER, "s3d_window_index_grid: counts is null");
+    if (N < 0 || N > 0x7fffffffLL || num_sets < 1 || num_sets > kMaxSets || N * num_sets > 0xffffffffLL)
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_window_indices: N=%lld voxels, %d sets (1..%d)", (long long)N, num_sets, kMaxSets);
+    if (!jobs) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: sets is null");
+    GridSets sets{};
+    sets.num = num_sets;
+    for (int i = 0; i < num_sets; ++i) {
+        const s3d_window_index_set &j = jobs[i];
+        if (stride < 1 || j.window < 1 || j.window > 10 || j.shift < 0 || j.shift >= j.window)
+            return fail(S3D_ERR_BAD_SHAPE, "s3d_window_indices: stride=%d window=%d shift=%d (need stride>=1, "
+                        "1<=window<=10, 0<=shift<window)", stride, j.window, j.shift);
+        if (!j.counts) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: counts is null");
+        if (N > 0 && (!j.n2n || !j.w_w_id || !j.w_sizes || !j.w2n))
+            return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: null device pointer");
+        sets.set[i] = GridSet{j.window, j.shift, j.n2n, j.w_w_id, j.w_sizes, j.w2n, j.counts};
+    }
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (N == 0) {
-        hipLaunchKernelGGL(init_counts_kernel, dim3(1), dim3(64), 0, s, counts);
+        for (int i = 0; i < num_sets; ++i) hipLaunchKernelGGL(init_counts_kernel, dim3(1), dim3(64), 0, s, sets.set[i].counts);
         S3D_HIP_CHECK(hipGetLastError());
         return S3D_OK;
     }
-    if (!coords || !n2n || !w_w_id || !w_sizes || !w2n || !workspace)
-        return fail(S3D_ERR_NULL_POINTER, "s3d_window_index_grid: null device pointer");
+    if (!coords || !workspace) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: null device pointer");
     if (reinterpret_cast<uintptr_t>(coords) % 16 != 0)
-        return fail(S3D_ERR_BAD_SHAPE, "s3d_window_index_grid: coords must be 16-byte aligned");
-    const GridLayout L = make_grid_layout(N);
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_window_indices: coords must be 16-byte aligned");
+    const GridLayout L = make_grid_layout(N, num_sets);
     if (workspace_bytes < L.total)
-        return fail(S3D_ERR_WORKSPACE, "s3d_window_index_grid: workspace %zu B < required %zu B", workspace_bytes, L.total);
+        return fail(S3D_ERR_WORKSPACE, "s3d_window_indices: workspace %zu B < required %zu B", workspace_bytes, L.total);
     char *base = static_cast<char *>(workspace);
     GridPlan *plan = reinterpret_cast<GridPlan *>(base + L.plan);
     int32_t *partials = reinterpret_cast<int32_t *>(base + L.partials);
@@ -718,24 +756,36 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_index_grid(
     int2 *place = reinterpret_cast<int2 *>(base + L.place);
     uint64_t *keys = reinterpret_cast<uint64_t *>(base + L.keys);
     size_t temp_bytes = L.temp_bytes;
-    const int64_t num_cells = L.cells_cap + 1;
-    const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)));
-    hipLaunchKernelGGL(grid_bbox_kernel, dim3(kGridBoxes), dim3(kThreads), 0, s, coords, N, stride, window, shift, partials,
-                       cells, num_cells, counts);
+    const int64_t num_cells = (L.cells_cap + 1) * num_sets;
+    const unsigned per_set = static_cast<unsigned>(num_sets);
+    const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)), per_set);
+    hipLaunchKernelGGL(grid_bbox_kernel, dim3(kGridBoxes), dim3(kThreads), 0, s, coords, N, sets, partials, cells, num_cells);
     S3D_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(grid_count_kernel, grid, dim3(kThreads), 0, s, coords, N, stride, window, shift, partials,
-                       L.cells_cap, plan, cells, place, counts);
+    hipLaunchKernelGGL(grid_count_kernel, grid, dim3(kThreads), 0, s, coords, N, stride, sets, partials, L.cells_cap, plan,
+                       cells, place);
     S3D_HIP_CHECK(hipGetLastError());
     S3D_HIP_CHECK(rocprim::exclusive_scan(base + L.temp, temp_bytes, CellWordIterator(cells, CellWord()), scan, uint64_t(0),
                                           static_cast<size_t>(num_cells), rocprim::plus<uint64_t>(), s));
-    hipLaunchKernelGGL(grid_place_kernel, grid, dim3(kThreads), 0, s, place, N, plan, scan, L.cells_cap, keys, w2n, w_sizes,
-                       counts);
+    hipLaunchKernelGGL(grid_place_kernel, grid, dim3(kThreads), 0, s, place, N, sets, plan, scan, L.cells_cap, keys);
     S3D_HIP_CHECK(hipGetLastError());
     // about one window per wavefront if the windows hold 16 voxels on average, more in turn otherwise
     int64_t order_blocks = ceil_div(N, 64);
     order_blocks = order_blocks < 32 ? 32 : (order_blocks > 4096 ? 4096 : order_blocks);
-    hipLaunchKernelGGL(grid_order_kernel, dim3(static_cast<unsigned>(order_blocks)), dim3(kThreads), 0, s, plan, keys, w2n,
-                       w_sizes, n2n, w_w_id, counts);
+    hipLaunchKernelGGL(grid_order_kernel, dim3(static_cast<unsigned>(order_blocks), per_set), dim3(kThreads), 0, s, plan, keys,
+                       N, sets);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
+}
+
+extern "C" __attribute__((visibility("default"))) size_t s3d_window_index_grid_workspace_bytes(int64_t N)
+{
+    return s3d_window_indices_workspace_bytes(N, 1);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_window_index_grid(
+    const int32_t *coords, int64_t N, int32_t stride, int32_t window, int32_t shift, int32_t *n2n, int32_t *w_w_id,
+    int32_t *w_sizes, int32_t *w2n, int64_t *counts, void *workspace, size_t workspace_bytes, void *stream)
+{
+    const s3d_window_index_set set{n2n, w_w_id, w_sizes, w2n, counts, window, shift};
+    return s3d_window_indices(coords, N, stride, &set, 1, workspace, workspace_bytes, stream);
 }

@@ -82,9 +82,9 @@ def conv3x3x3_neighbours(coords, stride):
                            for dz in (-1, 0, 1)], dtype=torch.long, device=coords.device) * stride
     if coords.is_cuda:
         out = torch.empty((n, 27), dtype=torch.long, device=coords.device)
-        with torch.cuda.device(coords.device):
+        with _lib.on(coords.device):
             status = _lib.lib().s3d_key_neighbours(sorted_keys.data_ptr(), order.data_ptr(), n, deltas.data_ptr(), 27,
-                                                   out.data_ptr(), torch.cuda.current_stream(coords.device).cuda_stream)
+                                                   out.data_ptr(), _lib.stream(coords.device))
         _lib.check(status, "s3d_key_neighbours")
         return out
     queries = sorted_keys.unsqueeze(0) + deltas.unsqueeze(1)                    # [27, N], rows ascending
@@ -155,11 +155,11 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
             if sig.stride(1) != 1:
                 sig = sig.contiguous()
             pick = torch.empty(index.num_windows, dtype=torch.long, device=coords.device)
-            with torch.cuda.device(coords.device):
+            with _lib.on(coords.device):
                 status = _lib.lib().s3d_cell_representatives(
                     index.n2n.data_ptr(), index.w2n.data_ptr(), index.w_sizes.data_ptr(), index.num_windows,
                     sig.data_ptr(), sig.stride(0), sig.shape[1], pick.data_ptr(),
-                    torch.cuda.current_stream(coords.device).cuda_stream)
+                    _lib.stream(coords.device))
             _lib.check(status, "s3d_cell_representatives")
             return members, pick
     coarse, cell_of_row = pool_coordinates(coords, stride, factor)
@@ -525,12 +525,12 @@ def window_order(coords, stride, window_size):
     n2n, wwid, w_sizes, w2n = (torch.empty(n, dtype=torch.int32, device=dev) for _ in range(4))
     counts = torch.empty(4, dtype=torch.int64, device=dev)
     lib = _lib.lib()
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         ws_bytes = lib.s3d_window_index_workspace_bytes(n)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         status = lib.s3d_window_index(coords.data_ptr(), n, int(stride), int(window_size), 0, n2n.data_ptr(),
                                       wwid.data_ptr(), w_sizes.data_ptr(), w2n.data_ptr(), counts.data_ptr(),
-                                      workspace.data_ptr(), ws_bytes, torch.cuda.current_stream(dev).cuda_stream)
+                                      workspace.data_ptr(), ws_bytes, _lib.stream(dev))
     _lib.check(status, "s3d_window_index")
     return n2n.long()      # coordinates out of the sort's range are reported by the stage's own index build
 

@@ -33,8 +33,8 @@ def add_layernorm(x, residual, norm, out_dtype=torch.float16, inplace=False):
         summed = x if inplace else torch.empty_like(x)
     y = torch.empty((n, c), dtype=out_dtype, device=x.device)
     gamma, beta = norm.weight.detach().float().contiguous(), norm.bias.detach().float().contiguous()
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream(x.device).cuda_stream
+    with _lib.on(x.device):
+        stream = _lib.stream(x.device)
         status = _lib.lib().s3d_add_layernorm(x.data_ptr(), res_ptr, res_code, gamma.data_ptr(), beta.data_ptr(),
                                              float(norm.eps), summed.data_ptr() if residual is not None else None,
                                              y.data_ptr(), _DTYPE_CODE[out_dtype], n, c, stream)

@@ -187,18 +187,25 @@ def window_attention_forward(q, k, v, table_q, table_k, table_v, table_sizes, w_
     dev = q.device
     if q.dim() != 3:
         raise ValueError(f"query must be [N,H,D], got {tuple(q.shape)}")
-    n, h, d = q.shape
     if q.dtype not in _DTYPE_CODE:
         raise TypeError(f"unsupported feature dtype {q.dtype} (float16 or float32)")
     for name, t in (("key", k), ("value", v)):
         _require_cuda(name, t, dev, strided_rows=True)
         if t.shape != q.shape or t.dtype != q.dtype:
             raise ValueError(f"{name} must match query: {tuple(t.shape)} {t.dtype}")
+    return _attention(q, k, v, [_row_stride(t) for t in (q, k, v)], table_q, table_k, table_v, table_sizes, w_sizes, w2n, n2n,
+                      n_coords, return_stats)
+
+
+def _attention(q, k, v, strides, table_q, table_k, table_v, table_sizes, w_sizes, w2n, n2n, n_coords, return_stats):
+    """window_attention_forward behind the checks of q, k, v, whose row strides (or None) are `strides`."""
+    dev = q.device
+    n, h, d = q.shape
     # q, k, v are read in place when they share one row stride (views of one projection output)
-    strides = {_row_stride(t) for t in (q, k, v)}
-    if len(strides) != 1 or None in strides:
+    row_stride = strides[0]
+    if row_stride is None or strides[1] != row_stride or strides[2] != row_stride:
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    row_stride = _row_stride(q)
+        row_stride = _row_stride(q)
     if d not in (8, 16, 32):
         raise ValueError(f"head_dim must be 8, 16 or 32, got {d}")
     if _sizes_stay_on_device(table_sizes):
@@ -245,8 +252,8 @@ def window_attention_forward(q, k, v, table_q, table_k, table_v, table_sizes, w_
     code = _DTYPE_CODE[q.dtype]
     num_w = w_sizes.numel()
     flags = _lib.S3D_ATTN_SIZES_ON_DEVICE if sizes is None else 0
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with _lib.on(dev):
+        stream = _lib.stream(dev)
         # the work list depends on the window set only: it is built once and kept on the caller's w_sizes
         # tensor, so the blocks that share a window set share it
         plan = None if not REUSE_PLANS else _plan_for(lib, w_sizes_in, w2n_in, w_sizes, w2n, c_sizes, sizes,
@@ -354,10 +361,10 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
     lib = _lib.lib()
     tensors = [t.contiguous() for t in (q, k, v, table_q, table_k, table_v)]
     out, dout, out_max, out_sum, n_coords = (t.contiguous() for t in (out, dout, out_max, out_sum, n_coords))
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         ws_bytes = lib.s3d_attn_bwd_workspace_bytes(h, d, nd, table_len, n, w_sizes.numel(), pairs)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        stream = _lib.stream(dev)
         status = lib.s3d_attn_bwd(
             *(t.data_ptr() for t in tensors), c_sizes, nd, table_len, w_sizes.data_ptr(), w2n.data_ptr(),
             None if n2n is None else n2n.data_ptr(), n_coords.data_ptr(), out.data_ptr(), out_max.data_ptr(),
@@ -394,8 +401,11 @@ class SelfAttnAIOFunction(Function):
             raise NotImplementedError(f"compute dtype {c_dtype} is not supported (float16 / float32)")
         _, w_sizes, _, w2n, n2n, n_coords = indices
         raw = (raw_query_feats, raw_key_feats, raw_value_feats, query_table, key_table, value_table)
-        feats = [t.to(c_dtype) for t in raw[:3]]
-        feats = [t if _row_stride(t) is not None else t.contiguous() for t in feats]
+        feats = [t if t.dtype == c_dtype else t.to(c_dtype) for t in raw[:3]]
+        strides = [_row_stride(t) for t in feats]
+        if None in strides:
+            feats = [t.contiguous() if s is None else t for t, s in zip(feats, strides)]
+            strides = [_row_stride(t) for t in feats]
         tables = [t.to(c_dtype).contiguous() for t in raw[3:]]
         n_coords = n_coords.to(torch.float32).contiguous()
         needs_grad = any(ctx.needs_input_grad[:6])
@@ -405,8 +415,12 @@ class SelfAttnAIOFunction(Function):
                 raise NotImplementedError(
                     f"attention backward supports head_dim 8, 16 and 32, got {raw_query_feats.shape[2]}; run the "
                     "forward under torch.no_grad()")
-        res = window_attention_forward(*feats, *tables, table_offsets, w_sizes, w2n, n2n, n_coords,
-                                       return_stats=needs_grad)
+        q, k, v = feats
+        if not (q.is_cuda and q.dim() == 3 and q.shape == k.shape == v.shape and q.device == k.device == v.device):
+            # (what is wrong with them, in words)
+            res = window_attention_forward(*feats, *tables, table_offsets, w_sizes, w2n, n2n, n_coords, return_stats=needs_grad)
+        else:
+            res = _attention(q, k, v, strides, *tables, table_offsets, w_sizes, w2n, n2n, n_coords, needs_grad)
         if not needs_grad:
             return res
         out, omax, osum = res

@@ -11,8 +11,9 @@ from torch.autograd.function import Function
 from ... import _lib
 
 
-def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0):
-    """-> (idx int32 [Nq,K], SQUARED distances fp32 [Nq,K]).  cell_size <= 0: chosen from the data."""
+def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0, squared=True):
+    """-> (idx int32 [Nq,K], SQUARED distances fp32 [Nq,K], or the distances with squared=False).  cell_size <= 0: chosen
+    from the data."""
     K = int(K)
     if not 1 <= K <= _lib.KNN_KMAX:
         raise ValueError(f"K must be in 1..{_lib.KNN_KMAX}, got {K}")
@@ -40,14 +41,15 @@ def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0):
     idx = torch.empty((nq, K), dtype=torch.int32, device=dev)
     dist2 = torch.empty((nq, K), dtype=torch.float32, device=dev)
     lib = _lib.lib()
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         ws_bytes = lib.s3d_knn_workspace_bytes(ns, nq, b)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        stream = torch.cuda.current_stream(dev).cuda_stream
-        status = lib.s3d_knn(K, src_xyz.data_ptr(), ns, query_xyz.data_ptr(), nq,
-                             src_offset.data_ptr(), query_offset.data_ptr(), b, idx.data_ptr(),
-                             dist2.data_ptr(), float(cell_size), workspace.data_ptr(), ws_bytes,
-                             stream)
+        stream = _lib.stream(dev)
+        fn = lib.s3d_knn if squared else lib.s3d_knn_distances
+        status = fn(K, src_xyz.data_ptr(), ns, query_xyz.data_ptr(), nq,
+                    src_offset.data_ptr(), query_offset.data_ptr(), b, idx.data_ptr(),
+                    dist2.data_ptr(), float(cell_size), workspace.data_ptr(), ws_bytes,
+                    stream)
     _lib.check(status, "s3d_knn")
     return idx, dist2
 
@@ -58,8 +60,7 @@ class KNN(Function):
 
     @staticmethod
     def forward(ctx, K, src_xyz, query_xyz, src_offset, query_offset):
-        idx, dist2 = knn_query(K, src_xyz, query_xyz, src_offset, query_offset, KNN.cell_size)
-        dist = torch.sqrt(dist2)
+        idx, dist = knn_query(K, src_xyz, query_xyz, src_offset, query_offset, KNN.cell_size, squared=False)
         ctx.mark_non_differentiable(idx, dist)
         return idx, dist
 
@@ -81,8 +82,8 @@ def knn_interpolate(idx, dist2, src_feat):
     nq, k = idx.shape
     ns, c = src_feat.shape
     out = torch.empty((nq, c), dtype=src_feat.dtype, device=src_feat.device)
-    with torch.cuda.device(src_feat.device):
-        stream = torch.cuda.current_stream(src_feat.device).cuda_stream
+    with _lib.on(src_feat.device):
+        stream = _lib.stream(src_feat.device)
         status = _lib.lib().s3d_knn_interpolate(idx.data_ptr(), dist2.data_ptr(), k, nq, src_feat.data_ptr(), ns, c,
                                                 _FEAT_DTYPE[src_feat.dtype], out.data_ptr(), stream)
     _lib.check(status, "s3d_knn_interpolate")
@@ -104,8 +105,8 @@ def knn_max_pool(idx, src_feat):
     nq, k = idx.shape
     ns, c = src_feat.shape
     out = torch.empty((nq, c), dtype=src_feat.dtype, device=src_feat.device)
-    with torch.cuda.device(src_feat.device):
-        stream = torch.cuda.current_stream(src_feat.device).cuda_stream
+    with _lib.on(src_feat.device):
+        stream = _lib.stream(src_feat.device)
         status = _lib.lib().s3d_knn_max_pool(idx.data_ptr(), k, nq, src_feat.data_ptr(), ns, c,
                                              _FEAT_DTYPE[src_feat.dtype], out.data_ptr(), stream)
     _lib.check(status, "s3d_knn_max_pool")

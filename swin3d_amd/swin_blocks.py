@@ -91,10 +91,10 @@ def linear_rows(x, weight, bias, gelu=False):
             or x.data_ptr() % 16 or weight.data_ptr() % 16:
         return None
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         status = _lib.lib().s3d_linear(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
                                        x.shape[0], weight.shape[0], x.shape[1], int(gelu),
-                                       torch.cuda.current_stream(x.device).cuda_stream)
+                                       _lib.stream(x.device))
     _lib.check(status, "s3d_linear")
     return out
 
@@ -140,8 +140,8 @@ def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     sets = (_lib.WindowSet * len(index_sets))()
     held = []
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with _lib.on(dev):
+        stream = _lib.stream(dev)
         for s, args in zip(sets, index_sets):
             _, _, _, w_sizes_in, w2n_in, n2n, _, _, coords = args[:9]
             w_sizes, w2n = (attn_coff._as_int32(name, t, dev) for name, t in (("w_sizes", w_sizes_in), ("w2n", w2n_in)))

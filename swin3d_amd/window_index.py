@@ -15,6 +15,7 @@ from . import _lib
 
 # s3d_window_index_grid (counting sort over the window lattice) where it applies; False: always the sort of all voxels
 USE_GRID_PATH = True
+GRID_SETS = 4      # window sets that one such call builds at most
 
 
 @dataclass
@@ -57,29 +58,48 @@ def build_window_indices(coords, stride, window_size, shifts):
     counts = torch.empty((len(sets), 4), dtype=torch.int64, device=dev)
     lib = _lib.lib()
     outputs = []
+    pitch = (n + 63) // 64 * 64
 
-    def enqueue(i, window, shift, grid):
-        fn, size_fn = ((lib.s3d_window_index_grid, lib.s3d_window_index_grid_workspace_bytes) if grid else
-                       (lib.s3d_window_index, lib.s3d_window_index_workspace_bytes))
-        ws_bytes = size_fn(n)
+    def enqueue_grid(first, some):
+        """The sets `some` (numbers from `first` on) by the counting sort, together."""
+        out = torch.empty((4 * len(some), pitch), dtype=torch.int32, device=dev)
+        jobs = (_lib.WindowIndexSet * len(some))()
+        at, step = out.data_ptr(), 4 * pitch
+        for i, (job, (window, shift)) in enumerate(zip(jobs, some)):
+            job.n2n, job.w_w_id, job.w_sizes, job.w2n = (at + (4 * i + k) * step for k in range(4))
+            job.counts = counts.data_ptr() + 32 * (first + i)
+            job.window, job.shift = int(window), int(shift)
+        ws_bytes = lib.s3d_window_indices_workspace_bytes(n, len(some))
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        status = lib.s3d_window_indices(coords.data_ptr(), n, int(stride), jobs, len(some), workspace.data_ptr(), ws_bytes,
+                                        _lib.stream(dev))
+        _lib.check(status, "s3d_window_indices")
+        rows = out[:, :n].unbind(0)
+        return [rows[4 * i:4 * i + 4] for i in range(len(some))]
+
+    def enqueue(i, window, shift):
+        ws_bytes = lib.s3d_window_index_workspace_bytes(n)
         n2n, wwid, w_sizes, w2n = (torch.empty(n, dtype=torch.int32, device=dev) for _ in range(4))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        status = fn(coords.data_ptr(), n, int(stride), int(window), int(shift), n2n.data_ptr(), wwid.data_ptr(),
-                    w_sizes.data_ptr(), w2n.data_ptr(), counts[i].data_ptr(), workspace.data_ptr(), ws_bytes,
-                    torch.cuda.current_stream(dev).cuda_stream)
-        _lib.check(status, fn.__name__)
+        status = lib.s3d_window_index(coords.data_ptr(), n, int(stride), int(window), int(shift), n2n.data_ptr(), wwid.data_ptr(),
+                                      w_sizes.data_ptr(), w2n.data_ptr(), counts[i].data_ptr(), workspace.data_ptr(), ws_bytes,
+                                      _lib.stream(dev))
+        _lib.check(status, "s3d_window_index")
         return n2n, wwid, w_sizes, w2n
 
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         # the counting sort over the window lattice first; a set whose lattice is too large for it (bit 1 of its
         # status word) is built again by the sort of all voxels, at the price of a second wait
-        for i, (window, shift) in enumerate(sets):
-            outputs.append(enqueue(i, window, shift, grid=USE_GRID_PATH))
+        if USE_GRID_PATH:
+            for first in range(0, len(sets), GRID_SETS):
+                outputs += enqueue_grid(first, sets[first:first + GRID_SETS])
+        else:
+            outputs = [enqueue(i, window, shift) for i, (window, shift) in enumerate(sets)]
         host_counts = counts.tolist()
         redo = [i for i, c in enumerate(host_counts) if c[3] & 2]
         if redo:
             for i in redo:
-                outputs[i] = enqueue(i, sets[i][0], sets[i][1], grid=False)
+                outputs[i] = enqueue(i, sets[i][0], sets[i][1])
             host_counts = counts.tolist()
     result = []
     for (n2n, wwid, w_sizes, w2n), (num_w, num_m, max_w, err), (window, _) in zip(outputs, host_counts, sets):
@@ -119,12 +139,12 @@ def window_signals(index, local_xyz, colors, num_signals=None, xyz_scale=1.0, ot
         raise ValueError(f"local_xyz must be [{n},3] and colors [{n},*], got {tuple(frac.shape)} and "
                          f"{tuple(colors.shape)}")
     out = torch.empty((n, 3 + num_signals), dtype=torch.float32, device=frac.device)
-    with torch.cuda.device(frac.device):
+    with _lib.on(frac.device):
         status = _lib.lib().s3d_window_signals(
             index.w_w_id.data_ptr(), index.n2n.data_ptr(), frac.data_ptr(),
             colors.data_ptr() if num_signals > 0 else None, colors.stride(0) if num_signals > 0 else 0,
             int(num_signals), int(index.window_size), float(xyz_scale), float(other_scale), out.data_ptr(), n,
-            torch.cuda.current_stream(frac.device).cuda_stream)
+            _lib.stream(frac.device))
     _lib.check(status, "s3d_window_signals")
     return out
 

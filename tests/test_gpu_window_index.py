@@ -159,3 +159,18 @@ def test_lattice_too_large_falls_back_to_the_sort(oracle_lib, hip_lib, index_pat
         torch.cuda.synchronize()
         assert int(counts[3]) & 2
         assert all(bool((o == -7).all()) for o in outs)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 5000])
+def test_several_sets_in_one_call(hip_lib, n):
+    """Sets of their own window sizes built together, more than one run of launches takes, one of them (window 1) with a
+    lattice too large for the counting sort."""
+    from swin3d_amd import window_index
+    coords = torch.from_numpy(random_scene(np.random.default_rng(n), n, extent=(24, 24, 12), batches=2, stride=2)).cuda()
+    sets = [(5, 0), (5, 2), (2, 0), (7, 3), (1, 0), (10, 9)]
+    together = window_index.build_window_indices(coords, 2, 5, sets)
+    for (window, shift), got in zip(sets, together):
+        alone = window_index.build_window_index(coords, 2, window, shift)
+        assert (got.num_windows, got.num_pairs, got.max_window_voxels) == (alone.num_windows, alone.num_pairs, alone.max_window_voxels)
+        for name in ("n2n", "w_w_id", "w_sizes", "w2n"):
+            assert torch.equal(getattr(got, name), getattr(alone, name)), (name, window, shift)
