@@ -35,7 +35,7 @@ from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
 from .fused_norm import add_layernorm
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .sparse_dl.knn import KNN, KNNInterpolate, knn_max_pool, knn_query
-from .swin_blocks import linear_rows, swin_blocks
+from .swin_blocks import linear_rows, plain, swin_blocks
 from .window_index import build_window_indices, get_index01, index_arguments, window_signals
 
 
@@ -675,7 +675,7 @@ class Upsample(nn.Module):
         """LayerNorm + Linear; for inference under fp16 autocast the norm is the fused kernel that writes fp16."""
         if _fused_norm_applies(feats):
             _, normed = add_layernorm(feats, None, block[0])
-            return _linear(block[1], normed)
+            return _linear(block[1], normed) if plain(block[1], nn.Linear) else block[1](normed)
         return block(feats)
 
     def forward(self, voxels, signals, voxels_up, signals_up, plan_up=None, num_batches=None):

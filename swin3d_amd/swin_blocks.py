@@ -4,35 +4,55 @@ import ctypes
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _module_hooks
 
 from . import _lib
 from .sparse_dl.attn import attn_coff
 
 
-def _plain(m, kind):
+def plain(m, kind):
     """m is a `kind` (no subclass: it may compute something else) and nothing watches or replaces its forward."""
-    return type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+    return (type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+            and not _module_hooks._global_forward_hooks and not _module_hooks._global_forward_pre_hooks)
+
+
+def _data_only(x):
+    """x is its data and nothing follows what is done to it: no subclass, no transform, forward-mode derivative, dispatch
+    mode or tracer, all of which a call by address would pass by."""
+    return (type(x) is torch.Tensor and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._len_torch_dispatch_stack() and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
 def _parts(block, kinds):
     """(block, norm1, attn, qkv, proj, norm2, mlp, fc1, act, fc2), or None where one of them is not what it was built as."""
     m = block._modules
     attn, mlp = m["attn"], m["mlp"]
-    if not (_plain(block, kinds[0]) and _plain(attn, kinds[1]) and _plain(mlp, kinds[2])):
+    if not (plain(block, kinds[0]) and plain(attn, kinds[1]) and plain(mlp, kinds[2])):
         return None
     a, f = attn._modules, mlp._modules
     parts = (block, m["norm1"], attn, a["qkv"], a["proj"], m["norm2"], mlp, f["fc1"], f["act"], f["fc2"])
-    if not (_plain(parts[1], nn.LayerNorm) and _plain(parts[5], nn.LayerNorm) and _plain(parts[8], nn.GELU)
-            and parts[8].approximate == "none" and all(_plain(parts[i], nn.Linear) for i in (3, 4, 7, 9))):
+    if not (plain(parts[1], nn.LayerNorm) and plain(parts[5], nn.LayerNorm) and plain(parts[8], nn.GELU)
+            and parts[8].approximate == "none" and all(plain(parts[i], nn.Linear) for i in (3, 4, 7, 9))):
         return None
     return parts
 
 
 def _stamp(parts):
-    """Addresses and versions of the parameters of the blocks."""
+    """Addresses and versions of the parameters of the blocks, and the norms' epsilons."""
     return [x for block in parts for i in (1, 2, 3, 4, 5, 7, 9) for p in block[i]._parameters.values() if p is not None
-            for x in (p.data_ptr(), p._version)]
+            for x in (p.data_ptr(), p._version)] + [block[i].eps for block in parts for i in (1, 5)]
+
+
+class _Kept:
+    """What swin_blocks keeps on its owner: key, descriptions (or None) and the tensors they point to.  Addresses are
+    worth nothing in another place: a copy of the owner, or one read from a file, starts with None."""
+
+    def __init__(self, key, described, tensors):
+        self.key, self.described, self.tensors = key, described, tensors
+
+    def __reduce__(self):
+        return type(None), ()
 
 
 def _descriptions(parts, half_copy):
@@ -86,9 +106,11 @@ def _applicable(parts, channels):
 def linear_rows(x, weight, bias, gelu=False):
     """x @ weight.T + bias (then GELU) of fp16 rows on the library's kernel (s3d_linear); None where it does not take the
     operands."""
-    if x.dim() != 2 or any(t is not None and (t.dtype != torch.float16 or t.device != x.device) for t in (x, weight, bias)) \
-            or x.shape[1] % 16 or weight.shape[0] % 8 or not x.is_contiguous() or not weight.is_contiguous() \
-            or x.data_ptr() % 16 or weight.data_ptr() % 16:
+    if not _data_only(x) or x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] \
+            or any(t is not None and (t.dtype != torch.float16 or t.device != x.device or not t.is_contiguous()
+                                      or t.data_ptr() % 16) for t in (x, weight, bias)) \
+            or x.shape[1] % 16 or x.shape[1] == 0 or weight.shape[0] % 8 or weight.shape[0] == 0 \
+            or (bias is not None and bias.shape != weight.shape[:1]):
         return None
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
     with _lib.on(x.device):
@@ -110,21 +132,19 @@ def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
     index_sets  per window set what index_arguments and window_signals give
     """
     n, channels = feats.shape
-    if n == 0 or _module_hooks._global_forward_hooks or _module_hooks._global_forward_pre_hooks:
-        return None
-    if type(feats) is not torch.Tensor or any(len(s) < 9 for s in index_sets):
+    if n == 0 or not _data_only(feats) or any(len(s) < 9 for s in index_sets):
         return None
     parts = [_parts(b, kinds) for b in blocks]
     if any(p is None for p in parts):
         return None
     key = (epoch, _stamp(parts), [m for p in parts for m in p])
     kept = getattr(owner, "_s3d_blocks", None)
-    if kept is None or kept[0] != key:
-        kept = (key, _descriptions(parts, half_copy) if _applicable(parts, channels) else None)
+    if kept is None or kept.key != key:
+        kept = _Kept(key, *(_descriptions(parts, half_copy) if _applicable(parts, channels) else (None, None)))
         owner._s3d_blocks = kept
-    if kept[1] is None:
+    if kept.described is None:
         return None
-    described, tensors = kept[1]
+    described, tensors = kept.described, kept.tensors
     dev = feats.device
     if tensors[0].device != dev:
         return None
