@@ -33,6 +33,7 @@ import torch.nn.functional as F
 from . import _lib
 from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
 from .fused_norm import add_layernorm
+from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .sparse_dl.knn import KNN, KNNInterpolate, knn_max_pool, knn_query
 from .swin_blocks import linear_rows, plain, swin_blocks
@@ -264,7 +265,8 @@ def _linear(layer, x):
     long as its context, and the encoder has about seventy such layers."""
     epoch = _cache_epoch()
     if torch.is_grad_enabled() or not torch.is_autocast_enabled() or not x.is_cuda:
-        return layer(x)
+        out = trained_linear(x, layer.weight, layer.bias) if plain(layer, nn.Linear) else None
+        return layer(x) if out is None else out
     weight, bias = _autocast_copy(layer, epoch)
     out = linear_rows(x, weight, bias)
     return F.linear(x, weight, bias) if out is None else out
@@ -400,8 +402,10 @@ class WindowAttention(nn.Module):
         _, _, m2w, w_sizes, w2n, n2n, w2m, n_coords = attn_args[:8]
         weight, bias, tables = self._prepared()
         # q, k, v stay slices of the [N, 3C] projection output, which the attention kernels read in place
-        qkv = F.linear(feats, weight, bias).view(n, 3, self.num_heads, self.head_dim)
-        query, key, value = qkv[:, 0], qkv[:, 1], qkv[:, 2]
+        qkv = trained_linear(feats, weight, bias)
+        qkv = F.linear(feats, weight, bias) if qkv is None else qkv
+        # (unbind: its gradient is one stack, that of three slices three zeroed buffers and their sum)
+        query, key, value = qkv.view(n, 3, self.num_heads, self.head_dim).unbind(1)
         # the scaled signals of the index set, when the caller prepared them once for all blocks that share it
         n_crse = attn_args[8] if len(attn_args) > 8 else scale_crse_coords(n_coords, self.quant_size, self.cRSE)
         precision = (PrecisionMode.HALF_NONE, PrecisionMode.HALF_FORWARD, PrecisionMode.HALF_ALL)[self.fp16_mode]
@@ -676,6 +680,8 @@ class Upsample(nn.Module):
         if _fused_norm_applies(feats):
             _, normed = add_layernorm(feats, None, block[0])
             return _linear(block[1], normed) if plain(block[1], nn.Linear) else block[1](normed)
+        if torch.is_grad_enabled() and plain(block, nn.Sequential):
+            return _linear(block[1], block[0](feats))
         return block(feats)
 
     def forward(self, voxels, signals, voxels_up, signals_up, plan_up=None, num_batches=None):

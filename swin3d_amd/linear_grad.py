@@ -1,0 +1,70 @@
+"""Dense layers in training under fp16 autocast: the product and its gradients on the library's kernels (s3d_linear,
+s3d_linear_grad).  Tall rows and small weights are what the networks have, where a product that does not split the sum
+over the rows leaves most of the chip idle."""
+import torch
+import torch.nn.functional as F
+from torch.autograd.function import Function
+
+from . import _lib
+from .swin_blocks import data_only, linear_rows
+
+
+def _weight_gradients(dy, x, want_weight, want_bias):
+    """(dy.T @ x, dy.sum(0)) of fp16 rows as far as they are wanted; None where the kernel does not take them."""
+    if not (data_only(dy) and data_only(x)) or dy.dtype != torch.float16 or dy.data_ptr() % 16 or x.data_ptr() % 16:
+        return None
+    (m, n), k, dev = dy.shape, x.shape[1], dy.device
+    dw = torch.empty((n, k), dtype=torch.float16, device=dev) if want_weight else None
+    db = torch.empty(n, dtype=torch.float16, device=dev) if want_bias else None
+    lib = _lib.lib()
+    with _lib.on(dev):
+        ws_bytes = lib.s3d_linear_grad_workspace_bytes(m, n, k)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        status = lib.s3d_linear_grad(dy.data_ptr(), x.data_ptr(), None if dw is None else dw.data_ptr(),
+                                     None if db is None else db.data_ptr(), m, n, k, workspace.data_ptr(), ws_bytes,
+                                     _lib.stream(dev))
+    _lib.check(status, "s3d_linear_grad")
+    return dw, db
+
+
+class _Linear(Function):
+    """F.linear of fp16 rows."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        out = linear_rows(x, weight, bias)
+        return F.linear(x, weight, bias) if out is None else out
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        need_x, need_weight, need_bias = ctx.needs_input_grad
+        if torch.is_grad_enabled():      # a graph of the gradients is wanted: operations that have one
+            return (dy.mm(weight) if need_x else None, dy.t().mm(x) if need_weight else None, dy.sum(0) if need_bias else None)
+        dy = dy.contiguous()
+        dx = dw = db = None
+        if need_x:
+            dx = linear_rows(dy, weight.t().contiguous(), None)
+            dx = dy.mm(weight) if dx is None else dx
+        if need_weight or need_bias:
+            grads = _weight_gradients(dy, x.contiguous(), need_weight, need_bias)
+            dw, db = grads if grads is not None else (dy.t().mm(x) if need_weight else None, dy.sum(0) if need_bias else None)
+        return dx, dw, db
+
+
+def trained_linear(x, weight, bias):
+    """F.linear(x, weight, bias) as autocast computes it, with the gradients above; None where this does not apply: outside
+    of training under fp16 autocast, and for operands that the kernels do not take."""
+    if not (torch.is_grad_enabled() and x.is_cuda and torch.is_autocast_enabled()
+            and torch.get_autocast_dtype("cuda") == torch.float16):
+        return None
+    operands = (x, weight) if bias is None else (x, weight, bias)
+    if not all((data_only(t) or type(t) is torch.nn.Parameter and data_only(t.data)) and t.device == x.device
+               and t.dtype in (torch.float16, torch.float32) for t in operands):
+        return None
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[0] == 0 or x.shape[1] != weight.shape[1] or x.shape[1] % 16 \
+            or x.shape[1] == 0 or weight.shape[0] == 0 or weight.shape[0] % 8 or max(weight.shape) > 16384 \
+            or (bias is not None and bias.shape != weight.shape[:1]):
+        return None
+    return _Linear.apply(*(t.to(torch.float16) for t in operands), *([None] if bias is None else []))

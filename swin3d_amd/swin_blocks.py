@@ -14,10 +14,12 @@ from .sparse_dl.attn import attn_coff
 def plain(m, kind):
     """m is a `kind` (no subclass: it may compute something else) and nothing watches or replaces its forward."""
     return (type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
-            and not _module_hooks._global_forward_hooks and not _module_hooks._global_forward_pre_hooks)
+            and not m._backward_hooks and not m._backward_pre_hooks
+            and not _module_hooks._global_forward_hooks and not _module_hooks._global_forward_pre_hooks
+            and not _module_hooks._global_backward_hooks and not _module_hooks._global_backward_pre_hooks)
 
 
-def _data_only(x):
+def data_only(x):
     """x is its data and nothing follows what is done to it: no subclass, no transform, forward-mode derivative, dispatch
     mode or tracer, all of which a call by address would pass by."""
     return (type(x) is torch.Tensor and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
@@ -106,7 +108,7 @@ def _applicable(parts, channels):
 def linear_rows(x, weight, bias, gelu=False):
     """x @ weight.T + bias (then GELU) of fp16 rows on the library's kernel (s3d_linear); None where it does not take the
     operands."""
-    if not _data_only(x) or x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] \
+    if not data_only(x) or x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] \
             or any(t is not None and (t.dtype != torch.float16 or t.device != x.device or not t.is_contiguous()
                                       or t.data_ptr() % 16) for t in (x, weight, bias)) \
             or x.shape[1] % 16 or x.shape[1] == 0 or weight.shape[0] % 8 or weight.shape[0] == 0 \
@@ -132,7 +134,7 @@ def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
     index_sets  per window set what index_arguments and window_signals give
     """
     n, channels = feats.shape
-    if n == 0 or not _data_only(feats) or any(len(s) < 9 for s in index_sets):
+    if n == 0 or not data_only(feats) or any(len(s) < 9 for s in index_sets):
         return None
     parts = [_parts(b, kinds) for b in blocks]
     if any(p is None for p in parts):

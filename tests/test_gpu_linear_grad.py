@@ -1,0 +1,71 @@
+"""s3d_linear_grad against fp32 sums at the edges of its tiles and splits, and the layer in training against F.linear."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from swin3d_amd import encoder
+from swin3d_amd.linear_grad import _weight_gradients, trained_linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 16), (63, 48, 48), (65, 144, 48), (257, 72, 640),      # one part, remainders on every side
+    (1025, 240, 80), (3100, 1536, 384), (12421, 320, 320),        # several tiles and parts
+    (66001, 96, 192), (199327, 48, 48),                           # as many parts as there are
+])
+def test_weight_gradients(hip_lib, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    dy, x = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, n), (m, k)))
+    dw, db = _weight_gradients(dy, x, True, True)
+    # half a unit of the result's last place, and the sums in fp32: m additions of products below 36, at most
+    # sqrt(m) eps off for random signs
+    for got, want, terms in ((dw, dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()),
+                             (db, dy.double().sum(0), dy.double().abs().sum(0))):
+        assert bool(((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -24 * terms + 1e-7).all())
+    again = _weight_gradients(dy, x, True, True)
+    assert torch.equal(again[0], dw) and torch.equal(again[1], db)
+    assert _weight_gradients(dy, x, False, True)[0] is None and torch.equal(_weight_gradients(dy, x, True, False)[0], dw)
+
+
+def test_weight_gradients_show_what_is_not_finite(hip_lib):
+    dy, x = torch.ones(300, 48, device="cuda").half(), torch.ones(300, 64, device="cuda").half()
+    dy[123, 5], x[7, 9] = float("inf"), float("nan")
+    dw, db = _weight_gradients(dy, x, True, True)
+    want = dy.float().t() @ x.float()
+    assert torch.equal(dw.isnan(), want.isnan()) and torch.equal(dw.isinf(), want.isinf()) and db[5].isinf()
+
+
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_layer_in_training(hip_lib, bias, dtype):
+    torch.manual_seed(3)
+    layer = nn.Linear(96, 40, bias=bias).cuda()
+    x = torch.randn(2500, 96, device="cuda").to(dtype).requires_grad_()
+    leaves = [x, *layer.parameters()]
+    grad = torch.randn(2500, 40, device="cuda").half()
+    with torch.autocast("cuda", dtype=torch.float16):
+        out, ref = encoder._linear(layer, x), F.linear(x, layer.weight, layer.bias)
+        assert trained_linear(x, layer.weight, layer.bias) is not None
+        layer.weight.requires_grad_(False)
+        only_x = torch.autograd.grad(encoder._linear(layer, x), x, grad)[0]
+        layer.weight.requires_grad_(True)
+    assert type(out.grad_fn).__name__ == "_LinearBackward" and out.dtype == ref.dtype
+    got, want = (torch.autograd.grad(o, leaves, grad, retain_graph=True) for o in (out, ref))
+    for a, b in ((out, ref), *zip(got, want)):
+        # one rounding to fp16 on either side
+        assert a.dtype == b.dtype and bool(((a - b).abs() <= 2.0 ** -10 * b.abs() + 1e-4 * b.abs().max()).all())
+    assert torch.equal(only_x, got[0])
+    # gradients of gradients
+    first = [torch.autograd.grad(o, x, grad.float().to(o.dtype).requires_grad_(), create_graph=True)[0] for o in (out, ref)]
+    second = [torch.autograd.grad(f.float().square().sum(), layer.weight)[0] for f in first]
+    assert (second[0] - second[1]).abs().max() <= 2e-3 * second[1].abs().max()
+
+
+def test_layer_keeps_its_hooks_in_training(hip_lib):
+    layer, calls = nn.Linear(32, 32).cuda(), []
+    layer.register_full_backward_hook(lambda *_: calls.append(1))
+    with torch.autocast("cuda", dtype=torch.float16):
+        encoder._linear(layer, torch.randn(8, 32, device="cuda", requires_grad=True)).sum().backward()
+    assert calls == [1]
