@@ -405,6 +405,16 @@ int s3d_add_layernorm(const float *x, const void *residual, int32_t residual_dty
                       void *stream);
 
 /*
+ * The gradients of that call with y in fp16: dx = dsum + the gradient of LayerNorm in fp32, dresidual the same in fp16,
+ * dgamma and dbeta [C] in fp32.  sum device [N,C] is the call's x_out (x without a residual), dsum fp32 [N,C] or null,
+ * dy fp16 [N,C]; dx and dresidual may be null; all dense and 16-byte aligned.  The same bits on every call.
+ */
+size_t s3d_layernorm_grad_workspace_bytes(int64_t N, int32_t C);
+int s3d_layernorm_grad(const float *sum, const float *dsum, const void *dy, const float *gamma, float eps, float *dx,
+                       void *dresidual, float *dgamma, float *dbeta, int64_t N, int32_t C, void *workspace,
+                       size_t workspace_bytes, void *stream);
+
+/*
  * y = x w^T + bias, then GELU (the exact form) where gelu is not zero; fp16 operands and result, fp32 accumulation, bias
  * and GELU, one rounding at the end.  x device [M,K], w device [N,K] (torch.nn.Linear's weight), bias device [N] or null,
  * y device [M,N], all dense and 16-byte aligned; N a multiple of 8, K of 16.

@@ -144,3 +144,181 @@ extern "C" __attribute__((visibility("default"))) int s3d_add_layernorm(
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
+
+// The gradients of (sum, y) = (x + residual, LayerNorm(x + residual)):  with h = (sum - mean) rstd and g = dy gamma,
+//   d = dsum + rstd (g - mean(g) - h mean(g h)),  dgamma = column sums of dy h,  dbeta = those of dy;
+// d goes to x in fp32 and to the residual in its fp16.
+//
+// Memory bound: the rows of sum, dsum, dy once in, d (and its fp16 copy) once out.  Mean and deviation are taken again from
+// the row, which is read anyway.  A lane keeps its channels' share of dgamma and dbeta in registers over all the rows that
+// its group draws; the groups of a workgroup add theirs in LDS and leave a part per workgroup, in a fixed order.
+// 199,327 rows of 48: 24 us (153 MB moved, 6.5 TB/s), 12,421 of 192: 12 us and the parts' sum 5; through torch the same
+// three gradients took 300 us and 40, with two more passes for the sum with dsum and the fp16 copy.
+namespace s3d {
+namespace {
+
+struct LnGradArgs {
+    const float *sum, *dsum;
+    const __half *dy;
+    const float *gamma;
+    float eps;
+    float *dx;
+    __half *dres;
+    float *parts;      // [workgroups][2 C]
+    int64_t N;
+    int C;
+};
+
+__device__ __forceinline__ float4 load_half4(const __half *p)
+{
+    const uint2 raw = *reinterpret_cast<const uint2 *>(p);
+    const float2 lo = __half22float2(*reinterpret_cast<const __half2 *>(&raw.x)), hi = __half22float2(*reinterpret_cast<const __half2 *>(&raw.y));
+    return make_float4(lo.x, lo.y, hi.x, hi.y);
+}
+
+// G lanes a row, CH chunks of four channels a lane
+template <int G, int CH> __global__ __launch_bounds__(kLnThreads) void layernorm_grad_kernel(LnGradArgs a)
+{
+    constexpr int kGroups = kLnThreads / G;
+    __shared__ float shared[kGroups][G * CH * 4];
+    const int lane = threadIdx.x % G, group = threadIdx.x / G, chunks = a.C / 4;
+    const float over = 1.0f / static_cast<float>(a.C);
+    float gamma[CH][4], dgamma[CH][4] = {}, dbeta[CH][4] = {};
+    bool mine[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        mine[i] = lane + i * G < chunks;
+        *reinterpret_cast<float4 *>(gamma[i]) = mine[i] ? *reinterpret_cast<const float4 *>(a.gamma + 4 * (lane + i * G)) : make_float4(0, 0, 0, 0);
+    }
+    const int64_t step = static_cast<int64_t>(gridDim.x) * kGroups;
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * kGroups + group; row < a.N; row += step) {      // (a group stays together)
+        float v[CH][4], dy[CH][4], ds[CH][4];
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int64_t at = row * a.C + 4 * (lane + i * G);
+            float4 x = make_float4(0, 0, 0, 0), y = x, s = x;
+            if (mine[i]) {
+                x = *reinterpret_cast<const float4 *>(a.sum + at);
+                y = load_half4(a.dy + at);
+                if (a.dsum) s = *reinterpret_cast<const float4 *>(a.dsum + at);
+            }
+            *reinterpret_cast<float4 *>(v[i]) = x;
+            *reinterpret_cast<float4 *>(dy[i]) = y;
+            *reinterpret_cast<float4 *>(ds[i]) = s;
+            sum += (x.x + x.y) + (x.z + x.w);
+        }
+        const float mean = group_sum<G>(sum) * over;
+        float sq = 0.0f, sum_g = 0.0f, sum_gh = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[i][e] = mine[i] ? v[i][e] - mean : 0.0f;
+                sq += v[i][e] * v[i][e];
+                sum_g += dy[i][e] * gamma[i][e];
+                sum_gh += dy[i][e] * gamma[i][e] * v[i][e];
+            }
+        const float rstd = rsqrtf(group_sum<G>(sq) * over + a.eps);
+        const float mean_g = group_sum<G>(sum_g) * over, mean_gh = group_sum<G>(sum_gh) * rstd * over;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            if (!mine[i]) continue;
+            const int64_t at = row * a.C + 4 * (lane + i * G);
+            float d[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float h = v[i][e] * rstd;
+                dgamma[i][e] += dy[i][e] * h;
+                dbeta[i][e] += dy[i][e];
+                d[e] = ds[i][e] + rstd * (dy[i][e] * gamma[i][e] - mean_g - h * mean_gh);
+            }
+            if (a.dx) *reinterpret_cast<float4 *>(a.dx + at) = make_float4(d[0], d[1], d[2], d[3]);
+            if (a.dres) {
+                uint2 packed;
+                *reinterpret_cast<__half2 *>(&packed.x) = __floats2half2_rn(d[0], d[1]);
+                *reinterpret_cast<__half2 *>(&packed.y) = __floats2half2_rn(d[2], d[3]);
+                *reinterpret_cast<uint2 *>(a.dres + at) = packed;
+            }
+        }
+    }
+    float *part = a.parts + static_cast<int64_t>(blockIdx.x) * 2 * a.C;
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+        if (which) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) shared[group][4 * (lane + i * G) + e] = which ? dbeta[i][e] : dgamma[i][e];
+        __syncthreads();
+        for (int c = threadIdx.x; c < a.C; c += kLnThreads) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) sum += shared[g][c];
+            part[which * a.C + c] = sum;
+        }
+    }
+}
+
+// The sum of the parts: 16 numbers a workgroup, sixteen shares of the parts each.
+__global__ __launch_bounds__(kLnThreads) void layernorm_grad_sum_kernel(const float *__restrict__ parts, int count, int C,
+                                                                        float *__restrict__ dgamma, float *__restrict__ dbeta)
+{
+    __shared__ float shared[kLnThreads];
+    const int e = threadIdx.x & 15, share = threadIdx.x >> 4, c = static_cast<int>(blockIdx.x) * 16 + e, at = min(c, 2 * C - 1);
+    float sum = 0.0f;
+#pragma unroll 8
+    for (int p = share; p < count; p += 16) sum += parts[static_cast<int64_t>(p) * 2 * C + at];
+    shared[threadIdx.x] = sum;
+    __syncthreads();
+    if (share > 0 || c >= 2 * C) return;
+    sum = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) sum += shared[16 * s + e];
+    (c < C ? dgamma[c] : dbeta[c - C]) = sum;
+}
+
+// lanes a row: as few as hold it in two chunks each
+int ln_lanes(int C) { return C <= 128 ? 16 : C <= 256 ? 32 : 64; }
+
+// four rows a group at least, four workgroups a CU at most
+int64_t ln_parts(int64_t N, int C)
+{
+    const int64_t wanted = ceil_div(N, 4 * (kLnThreads / ln_lanes(C)));
+    return wanted < 1024 ? wanted : 1024;
+}
+
+bool ln_fits(int64_t N, int32_t C) { return N >= 1 && C >= 4 && C % 4 == 0 && C <= 4 * kMaxChunks * 64; }
+
+}  // namespace
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) size_t s3d_layernorm_grad_workspace_bytes(int64_t N, int32_t C)
+{
+    return s3d::ln_fits(N, C) ? static_cast<size_t>(s3d::ln_parts(N, C)) * 2 * C * sizeof(float) : 0;
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_layernorm_grad(
+    const float *sum, const float *dsum, const void *dy, const float *gamma, float eps, float *dx, void *dresidual, float *dgamma,
+    float *dbeta, int64_t N, int32_t C, void *workspace, size_t workspace_bytes, void *stream)
+{
+    using namespace s3d;
+    if (!ln_fits(N, C))
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_layernorm_grad: N=%lld C=%d (C a multiple of 4, 4..%d)", (long long)N, C, 4 * kMaxChunks * 64);
+    if (!sum || !dy || !gamma || !dgamma || !dbeta) return fail(S3D_ERR_NULL_POINTER, "s3d_layernorm_grad: null device pointer");
+    const size_t need = s3d_layernorm_grad_workspace_bytes(N, C);
+    if (!workspace || workspace_bytes < need)
+        return fail(S3D_ERR_WORKSPACE, "s3d_layernorm_grad: workspace %zu B < required %zu B", workspace ? workspace_bytes : size_t(0), need);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const LnGradArgs args{sum, dsum, static_cast<const __half *>(dy), gamma, eps, dx, static_cast<__half *>(dresidual),
+                          static_cast<float *>(workspace), N, C};
+    const int parts = static_cast<int>(ln_parts(N, C));
+    auto kernel = C <= 64 ? layernorm_grad_kernel<16, 1> : C <= 128 ? layernorm_grad_kernel<16, 2> : C <= 256 ? layernorm_grad_kernel<32, 2>
+                  : C <= 512 ? layernorm_grad_kernel<64, 2> : layernorm_grad_kernel<64, 4>;
+    hipLaunchKernelGGL(kernel, dim3(parts), dim3(kLnThreads), 0, s, args);
+    S3D_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(layernorm_grad_sum_kernel, dim3(static_cast<unsigned>(ceil_div(2 * C, 16))), dim3(kLnThreads), 0, s,
+                       args.parts, parts, C, dgamma, dbeta);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}

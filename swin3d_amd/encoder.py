@@ -32,7 +32,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
-from .fused_norm import add_layernorm
+from .fused_norm import add_layernorm, trained_add_norm
 from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .sparse_dl.knn import KNN, KNNInterpolate, knn_max_pool, knn_query
@@ -305,6 +305,12 @@ def _fused_norm_applies(feats):
             and feats.shape[1] % 4 == 0 and feats.shape[1] <= 1024)
 
 
+def _norm(norm, x):
+    """norm(x) for a dense layer that follows: in fp16 where autocast would give it that."""
+    done = trained_add_norm(x, None, norm)
+    return norm(x) if done is None else done[1]
+
+
 class GridKNNDownsample(nn.Module):
     """Coarse voxel = stride-2 cell; its feature = max over the K=16 nearest fine points of
     Linear(LayerNorm(feature)); its coordinate signals = those of the picked representative."""
@@ -339,7 +345,7 @@ class GridKNNDownsample(nn.Module):
         else:
             if pending is not None:
                 voxels.feats += pending
-            normed = self.norm(voxels.feats)
+            normed = _norm(self.norm, voxels.feats)
         projected = _linear(self.linear, normed)
         if not torch.is_grad_enabled() and projected.is_cuda and projected.dtype in (torch.float16, torch.float32):
             feats = knn_max_pool(idx, projected)      # one kernel, no [Nq, K, C] intermediate
@@ -429,6 +435,14 @@ class SwinBlock(nn.Module):
         if self._fused_path(feats):
             feats, pending = self.forward_fused(feats, None, attn_args)
             return feats + pending
+        if plain(self.attn, WindowAttention) and plain(self.mlp, Mlp):
+            done = trained_add_norm(feats, None, self.norm1)
+            if done is not None:
+                feats, normed = done
+                branch = self.attn(normed, attn_args)
+                done = trained_add_norm(feats, branch, self.norm2)
+                feats, normed = (feats + branch, None) if done is None else done
+                return feats + self.mlp(self.norm2(feats) if normed is None else normed)
         feats = feats + self.attn(self.norm1(feats), attn_args)      # fp32 + fp16 promotes to fp32
         return feats + self.mlp(self.norm2(feats))
 
@@ -681,7 +695,7 @@ class Upsample(nn.Module):
             _, normed = add_layernorm(feats, None, block[0])
             return _linear(block[1], normed) if plain(block[1], nn.Linear) else block[1](normed)
         if torch.is_grad_enabled() and plain(block, nn.Sequential):
-            return _linear(block[1], block[0](feats))
+            return _linear(block[1], _norm(block[0], feats))
         return block(feats)
 
     def forward(self, voxels, signals, voxels_up, signals_up, plan_up=None, num_batches=None):

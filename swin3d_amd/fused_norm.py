@@ -1,8 +1,11 @@
 """Residual add fused with LayerNorm (HIP kernel s3d_add_layernorm) for the Swin block around the
 attention operator (Swin3D/modules/swin3d_layers.py:617-623)."""
 import torch
+import torch.nn as nn
+from torch.autograd.function import Function
 
 from . import _lib
+from .swin_blocks import data_only, plain
 
 _DTYPE_CODE = {torch.float32: _lib.S3D_DTYPE_F32, torch.float16: _lib.S3D_DTYPE_F16}
 
@@ -40,3 +43,69 @@ def add_layernorm(x, residual, norm, out_dtype=torch.float16, inplace=False):
                                              y.data_ptr(), _DTYPE_CODE[out_dtype], n, c, stream)
     _lib.check(status, "s3d_add_layernorm")
     return summed, y
+
+
+class _AddNorm(Function):
+    """(x + residual, LayerNorm of it in fp16); x itself in the first place without a residual."""
+
+    @staticmethod
+    def forward(ctx, x, residual, weight, bias, norm):
+        ctx.set_materialize_grads(False)
+        summed, y = add_layernorm(x, residual, norm)
+        ctx.save_for_backward(summed, weight)
+        ctx.eps, ctx.residual = norm.eps, residual is not None
+        return summed, y
+
+    @staticmethod
+    def backward(ctx, dsum, dy):
+        summed, weight = ctx.saved_tensors
+        need_x, need_residual, need_weight, need_bias, _ = ctx.needs_input_grad
+        if dy is None:
+            return dsum, dsum.half() if need_residual and dsum is not None else None, None, None, None
+        given = [dy] if dsum is None else [dy, dsum]
+        if torch.is_grad_enabled() or not all(data_only(t) for t in given) or dy.dtype != torch.float16 \
+                or (dsum is not None and dsum.dtype != torch.float32):
+            # a graph of the gradients is wanted, or something follows them: operations that have one
+            g = dy.float()
+            h = summed - summed.mean(1, keepdim=True)
+            rstd = (h.square().mean(1, keepdim=True) + ctx.eps).rsqrt()
+            h, gw = h * rstd, g * weight
+            dx = rstd * (gw - gw.mean(1, keepdim=True) - h * (gw * h).mean(1, keepdim=True))
+            dx = dx if dsum is None else dx + dsum
+            return (dx if need_x else None, dx.half() if need_residual else None, (g * h).sum(0) if need_weight else None,
+                    g.sum(0) if need_bias else None, None)
+        dy, dsum = (t if t is None or t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+                    for t in (dy, dsum))
+        (n, c), dev = summed.shape, summed.device
+        dx = torch.empty_like(summed) if need_x else None
+        dres = torch.empty_like(dy) if need_residual else None
+        dgamma, dbeta = (torch.empty(c, dtype=torch.float32, device=dev) for _ in range(2))
+        lib = _lib.lib()
+        with _lib.on(dev):
+            ws_bytes = lib.s3d_layernorm_grad_workspace_bytes(n, c)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            status = lib.s3d_layernorm_grad(
+                summed.data_ptr(), None if dsum is None else dsum.data_ptr(), dy.data_ptr(), weight.data_ptr(), ctx.eps,
+                None if dx is None else dx.data_ptr(), None if dres is None else dres.data_ptr(), dgamma.data_ptr(),
+                dbeta.data_ptr(), n, c, workspace.data_ptr(), ws_bytes, _lib.stream(dev))
+        _lib.check(status, "s3d_layernorm_grad")
+        return dx, dres, dgamma if need_weight else None, dbeta if need_bias else None, None
+
+
+def trained_add_norm(x, residual, norm):
+    """(x + residual, norm(x + residual) in fp16) with gradients, for training under fp16 autocast where a dense layer takes
+    the rows; None where it does not apply."""
+    if not (torch.is_grad_enabled() and x.is_cuda and torch.is_autocast_enabled()
+            and torch.get_autocast_dtype("cuda") == torch.float16 and plain(norm, nn.LayerNorm)):
+        return None
+    weight, bias = norm.weight, norm.bias
+    if weight is None or bias is None or x.dim() != 2 or x.shape[0] == 0 or tuple(norm.normalized_shape) != (x.shape[1],) \
+            or x.shape[1] % 4 or x.shape[1] > 1024:
+        return None
+    for t, dtype in ((x, torch.float32), (weight, torch.float32), (bias, torch.float32), (residual, torch.float16)):
+        if t is not None and not ((data_only(t) or type(t) is nn.Parameter and data_only(t.data)) and t.dtype == dtype
+                                  and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            return None
+    if residual is not None and residual.shape != x.shape:
+        return None
+    return _AddNorm.apply(x, residual, weight, bias, norm)
