@@ -13,6 +13,10 @@ def _weight_gradients(dy, x, want_weight, want_bias):
     """(dy.T @ x, dy.sum(0)) of fp16 rows as far as they are wanted; None where the kernel does not take them."""
     if not (data_only(dy) and data_only(x)) or dy.dtype != torch.float16 or dy.data_ptr() % 16 or x.data_ptr() % 16:
         return None
+    if dy.shape[1] % 8:      # (the number of classes)
+        extra = -dy.shape[1] % 8
+        return tuple(g if g is None else g[:-extra].clone() for g in
+                     _weight_gradients(F.pad(dy, (0, extra)), x, want_weight, want_bias))
     (m, n), k, dev = dy.shape, x.shape[1], dy.device
     dw = torch.empty((n, k), dtype=torch.float16, device=dev) if want_weight else None
     db = torch.empty(n, dtype=torch.float16, device=dev) if want_bias else None
@@ -63,8 +67,8 @@ def trained_linear(x, weight, bias):
     if not all((data_only(t) or type(t) is torch.nn.Parameter and data_only(t.data)) and t.device == x.device
                and t.dtype in (torch.float16, torch.float32) for t in operands):
         return None
-    if x.dim() != 2 or weight.dim() != 2 or x.shape[0] == 0 or x.shape[1] != weight.shape[1] or x.shape[1] % 16 \
-            or x.shape[1] == 0 or weight.shape[0] == 0 or weight.shape[0] % 8 or max(weight.shape) > 16384 \
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[0] == 0 or x.shape[1] != weight.shape[1] or x.shape[1] % 8 \
+            or x.shape[1] == 0 or weight.shape[0] == 0 or max(weight.shape) > 16384 \
             or (bias is not None and bias.shape != weight.shape[:1]):
         return None
     return _Linear.apply(*(t.to(torch.float16) for t in operands), *([None] if bias is None else []))

@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
     (1, 8, 16), (63, 48, 48), (65, 144, 48), (257, 72, 640),      # one part, remainders on every side
     (1025, 240, 80), (3100, 1536, 384), (12421, 320, 320),        # several tiles and parts
     (66001, 96, 192), (199327, 48, 48),                           # as many parts as there are
+    (5000, 13, 48), (700, 1, 24),                                 # columns that do not fill a load
 ])
 def test_weight_gradients(hip_lib, m, n, k):
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
