@@ -424,12 +424,12 @@ int s3d_linear(const void *x, const void *w, const void *bias, void *y, int64_t 
 
 /*
  * The gradients of that layer's weight and bias: dw = dy^T x [N,K] and db = column sums of dy [N], either may be null.
- * dy device [M,N], x device [M,K], fp16, dense and 16-byte aligned; dw, db fp16 (fp32 sums, one rounding); N and K
- * multiples of 8, M at least 1.  The same bits on every call.
+ * dy device [M,N], x device [M,K], fp16, dense and 16-byte aligned; dw, db of grad_dtype (fp32 sums, rounded once for
+ * fp16); N and K multiples of 8, M at least 1.  The same bits on every call.
  */
 size_t s3d_linear_grad_workspace_bytes(int64_t M, int32_t N, int32_t K);
-int s3d_linear_grad(const void *dy, const void *x, void *dw, void *db, int64_t M, int32_t N, int32_t K, void *workspace,
-                    size_t workspace_bytes, void *stream);
+int s3d_linear_grad(const void *dy, const void *x, void *dw, void *db, int32_t grad_dtype, int64_t M, int32_t N, int32_t K,
+                    void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * The Swin blocks of a stage at inference (Swin3D/modules/swin3d_layers.py:563-625): per block

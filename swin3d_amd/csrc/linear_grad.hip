@@ -1,5 +1,5 @@
 // The gradients of a dense layer's weight and bias: dW = dY^T X, db = the column sums of dY; fp16 operands, fp32
-// accumulation, one rounding to fp16 (gfx950).  The projections of a Swin block in training
+// accumulation, results in the parameters' type (gfx950).  The projections of a Swin block in training
 // (Swin3D/modules/swin3d_layers.py:153-176, 382-560): dW is N x K, a few dozen to a few hundred each, and the sum runs
 // over the voxels.
 //
@@ -134,8 +134,9 @@ __global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
 }
 
 // The sum of the parts: 64 numbers a workgroup, its four wavefronts share the parts.
+template <typename T>
 __global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(const float *__restrict__ parts, int splits, int64_t products,
-                                                                   int64_t total, _Float16 *__restrict__ dw, _Float16 *__restrict__ db)
+                                                                   int64_t total, T *__restrict__ dw, T *__restrict__ db)
 {
     __shared__ float shared[kThreads];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -148,9 +149,9 @@ __global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(const float *
     if (wave > 0 || e >= total) return;
     sum = (shared[lane] + shared[lane + 64]) + (shared[lane + 128] + shared[lane + 192]);
     if (e < products) {
-        if (dw) dw[e] = static_cast<_Float16>(sum);
+        if (dw) dw[e] = static_cast<T>(sum);
     } else if (db) {
-        db[e - products] = static_cast<_Float16>(sum);
+        db[e - products] = static_cast<T>(sum);
     }
 }
 
@@ -187,12 +188,14 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_linear_grad_workspa
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
-    const void *dy, const void *x, void *dw, void *db, int64_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
-    void *stream)
+    const void *dy, const void *x, void *dw, void *db, int32_t grad_dtype, int64_t M, int32_t N, int32_t K, void *workspace,
+    size_t workspace_bytes, void *stream)
 {
     using namespace s3d;
     if (!fits(M, N, K))
         return fail(S3D_ERR_BAD_SHAPE, "s3d_linear_grad: M=%lld N=%d K=%d (N and K multiples of 8, at most 16384)", (long long)M, N, K);
+    if (grad_dtype != S3D_DTYPE_F32 && grad_dtype != S3D_DTYPE_F16)
+        return fail(S3D_ERR_BAD_DTYPE, "s3d_linear_grad: grad_dtype %d (0 = fp32, 1 = fp16)", grad_dtype);
     if (!dy || !x || !(dw || db)) return fail(S3D_ERR_NULL_POINTER, "s3d_linear_grad: null device pointer");
     const size_t need = s3d_linear_grad_workspace_bytes(M, N, K);
     if (!workspace || workspace_bytes < need)
@@ -206,8 +209,13 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
     hipLaunchKernelGGL(kernel, dim3(split.tiles, split.count), dim3(kThreads), 0, s, args);
     S3D_HIP_CHECK(hipGetLastError());
     const int64_t products = static_cast<int64_t>(N) * K, total = products + N;
-    hipLaunchKernelGGL(linear_grad_sum_kernel, dim3(static_cast<unsigned>(ceil_div(total, 64))), dim3(kThreads), 0, s,
-                       args.parts, split.count, products, total, static_cast<_Float16 *>(dw), static_cast<_Float16 *>(db));
+    const dim3 sums(static_cast<unsigned>(ceil_div(total, 64)));
+    if (grad_dtype == S3D_DTYPE_F32)
+        hipLaunchKernelGGL(linear_grad_sum_kernel<float>, sums, dim3(kThreads), 0, s, args.parts, split.count, products, total,
+                           static_cast<float *>(dw), static_cast<float *>(db));
+    else
+        hipLaunchKernelGGL(linear_grad_sum_kernel<_Float16>, sums, dim3(kThreads), 0, s, args.parts, split.count, products, total,
+                           static_cast<_Float16 *>(dw), static_cast<_Float16 *>(db));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

@@ -9,52 +9,62 @@ from . import _lib
 from .swin_blocks import data_only, linear_rows
 
 
-def _weight_gradients(dy, x, want_weight, want_bias):
-    """(dy.T @ x, dy.sum(0)) of fp16 rows as far as they are wanted; None where the kernel does not take them."""
+_DTYPE_CODE = {torch.float32: _lib.S3D_DTYPE_F32, torch.float16: _lib.S3D_DTYPE_F16}
+
+
+def _weight_gradients(dy, x, want_weight, want_bias, dtype=torch.float32):
+    """(dy.T @ x, dy.sum(0)) of fp16 rows in `dtype`, as far as they are wanted; None where the kernel does not take them."""
     if not (data_only(dy) and data_only(x)) or dy.dtype != torch.float16 or dy.data_ptr() % 16 or x.data_ptr() % 16:
         return None
     if dy.shape[1] % 8:      # (the number of classes)
         extra = -dy.shape[1] % 8
         return tuple(g if g is None else g[:-extra].clone() for g in
-                     _weight_gradients(F.pad(dy, (0, extra)), x, want_weight, want_bias))
+                     _weight_gradients(F.pad(dy, (0, extra)), x, want_weight, want_bias, dtype))
     (m, n), k, dev = dy.shape, x.shape[1], dy.device
-    dw = torch.empty((n, k), dtype=torch.float16, device=dev) if want_weight else None
-    db = torch.empty(n, dtype=torch.float16, device=dev) if want_bias else None
+    dw = torch.empty((n, k), dtype=dtype, device=dev) if want_weight else None
+    db = torch.empty(n, dtype=dtype, device=dev) if want_bias else None
     lib = _lib.lib()
     with _lib.on(dev):
         ws_bytes = lib.s3d_linear_grad_workspace_bytes(m, n, k)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         status = lib.s3d_linear_grad(dy.data_ptr(), x.data_ptr(), None if dw is None else dw.data_ptr(),
-                                     None if db is None else db.data_ptr(), m, n, k, workspace.data_ptr(), ws_bytes,
-                                     _lib.stream(dev))
+                                     None if db is None else db.data_ptr(), _DTYPE_CODE[dtype], m, n, k, workspace.data_ptr(),
+                                     ws_bytes, _lib.stream(dev))
     _lib.check(status, "s3d_linear_grad")
     return dw, db
 
 
 class _Linear(Function):
-    """F.linear of fp16 rows."""
+    """F.linear in fp16 of fp16 rows and parameters in fp16 or fp32, whose gradients come in their own type: autocast would
+    round them to fp16 on the way."""
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        ctx.save_for_backward(x, weight)
-        out = linear_rows(x, weight, bias)
-        return F.linear(x, weight, bias) if out is None else out
+        half = weight.to(torch.float16)
+        ctx.save_for_backward(x, weight, half)
+        ctx.bias_dtype = None if bias is None else bias.dtype
+        bias = None if bias is None else bias.to(torch.float16)
+        out = linear_rows(x, half, bias)
+        return F.linear(x, half, bias) if out is None else out
 
     @staticmethod
     def backward(ctx, dy):
-        x, weight = ctx.saved_tensors
+        x, weight, half = ctx.saved_tensors
         need_x, need_weight, need_bias = ctx.needs_input_grad
-        if torch.is_grad_enabled():      # a graph of the gradients is wanted: operations that have one
-            return (dy.mm(weight) if need_x else None, dy.t().mm(x) if need_weight else None, dy.sum(0) if need_bias else None)
-        dy = dy.contiguous()
-        dx = dw = db = None
-        if need_x:
-            dx = linear_rows(dy, weight.t().contiguous(), None)
-            dx = dy.mm(weight) if dx is None else dx
-        if need_weight or need_bias:
-            grads = _weight_gradients(dy, x.contiguous(), need_weight, need_bias)
-            dw, db = grads if grads is not None else (dy.t().mm(x) if need_weight else None, dy.sum(0) if need_bias else None)
-        return dx, dw, db
+        dx = grads = None
+        if not torch.is_grad_enabled():
+            dy = dy.contiguous()
+            if need_x:
+                dx = linear_rows(dy, half.t().contiguous(), None)
+                dx = dy.mm(half) if dx is None else dx
+            if need_weight or need_bias:
+                grads = _weight_gradients(dy, x.contiguous(), need_weight, need_bias, weight.dtype if need_weight else ctx.bias_dtype)
+        elif need_x:      # a graph of the gradients is wanted: operations that have one
+            dx = dy.mm(weight.to(torch.float16))
+        if grads is None:
+            grads = dy.t().mm(x) if need_weight else None, dy.sum(0) if need_bias else None
+        dw, db = grads
+        return dx, dw if dw is None else dw.to(weight.dtype), db if db is None else db.to(ctx.bias_dtype)
 
 
 def trained_linear(x, weight, bias):
@@ -71,4 +81,4 @@ def trained_linear(x, weight, bias):
             or x.shape[1] == 0 or weight.shape[0] == 0 or max(weight.shape) > 16384 \
             or (bias is not None and bias.shape != weight.shape[:1]):
         return None
-    return _Linear.apply(*(t.to(torch.float16) for t in operands), *([None] if bias is None else []))
+    return _Linear.apply(x.to(torch.float16), weight, bias)

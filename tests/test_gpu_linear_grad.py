@@ -16,18 +16,21 @@ pytestmark = pytest.mark.gpu
     (66001, 96, 192), (199327, 48, 48),                           # as many parts as there are
     (5000, 13, 48), (700, 1, 24),                                 # columns that do not fill a load
 ])
-def test_weight_gradients(hip_lib, m, n, k):
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_weight_gradients(hip_lib, m, n, k, dtype):
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
     dy, x = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, n), (m, k)))
-    dw, db = _weight_gradients(dy, x, True, True)
-    # half a unit of the result's last place, and the sums in fp32: m additions of products below 36, at most
-    # sqrt(m) eps off for random signs
+    dw, db = _weight_gradients(dy, x, True, True, dtype)
+    # half a unit of the result's last place for fp16, and the sums in fp32: of terms of random sign a partial sum stays
+    # below 4 sqrt(m), so one of its at most m roundings (or truncations, twice that) below 2^-23 4 sqrt(m), and m of them, of
+    # random sign too, below 2^-21 m sqrt(m) / sqrt(m) = 2^-21 m, where the sum of the terms' sizes is 0.64 m or more
     for got, want, terms in ((dw, dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()),
                              (db, dy.double().sum(0), dy.double().abs().sum(0))):
-        assert bool(((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -24 * terms + 1e-7).all())
-    again = _weight_gradients(dy, x, True, True)
+        assert bool(((got.double() - want).abs() <= (2.0 ** -11 if dtype == torch.float16 else 0.0) * want.abs() + 2.0 ** -20 * terms + 1e-7).all())
+    again = _weight_gradients(dy, x, True, True, dtype)
     assert torch.equal(again[0], dw) and torch.equal(again[1], db)
-    assert _weight_gradients(dy, x, False, True)[0] is None and torch.equal(_weight_gradients(dy, x, True, False)[0], dw)
+    assert _weight_gradients(dy, x, False, True, dtype)[0] is None
+    assert torch.equal(_weight_gradients(dy, x, True, False, dtype)[0], dw)
 
 
 def test_weight_gradients_show_what_is_not_finite(hip_lib):
