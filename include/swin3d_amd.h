@@ -380,6 +380,16 @@ int s3d_knn_distances(int32_t K, const float *src_xyz, int64_t Ns, const float *
 int s3d_knn_max_pool(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C,
                      int32_t dtype, void *out, void *stream);
 
+/*
+ * The gradient of that call for src_feat: every query's dout goes in equal shares to the rows of its list that hold the
+ * maximum `out`; a maximum that is not a number gives NaN to all of them.  dsrc_feat device [Ns,C] of `dtype`, written
+ * whole; Nq and Ns at least 1.
+ */
+size_t s3d_knn_max_pool_grad_workspace_bytes(int64_t Nq, int32_t K, int64_t Ns, int32_t C, int32_t dtype);
+int s3d_knn_max_pool_grad(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C,
+                          int32_t dtype, const void *out, const void *dout, void *dsrc_feat, void *workspace,
+                          size_t workspace_bytes, void *stream);
+
 int s3d_knn_interpolate(const int32_t *idx, const float *dist2, int32_t K, int64_t Nq, const void *src_feat,
                         int64_t Ns, int32_t C, int32_t dtype, void *out, void *stream);
 

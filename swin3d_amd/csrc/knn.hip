@@ -628,7 +628,7 @@ __global__ __launch_bounds__(kThreads) void knn_max_pool_kernel(const int32_t *_
 #pragma unroll
         for (int i = 0; i < kAhead; ++i)
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) best[e] = (i0 + i == 0 || v[i][e] > best[e]) ? v[i][e] : best[e];
+            for (int e = 0; e < VEC; ++e) best[e] = (i0 + i == 0 || v[i][e] > best[e] || v[i][e] != v[i][e]) ? v[i][e] : best[e];
     }
     if constexpr (VEC * sizeof(T) == 16)
         *reinterpret_cast<uint4 *>(out + qi * C + c0) = *reinterpret_cast<const uint4 *>(best);

@@ -35,8 +35,8 @@ from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
 from .fused_norm import add_layernorm, trained_add_norm
 from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
-from .sparse_dl.knn import KNN, KNNInterpolate, knn_max_pool, knn_query
-from .swin_blocks import linear_rows, plain, swin_blocks
+from .sparse_dl.knn import KNN, KNNInterpolate, KNNMaxPool, knn_max_pool, knn_query
+from .swin_blocks import data_only, linear_rows, plain, swin_blocks
 from .window_index import build_window_indices, get_index01, index_arguments, window_signals
 
 
@@ -355,6 +355,9 @@ class GridKNNDownsample(nn.Module):
         projected = _linear(self.linear, normed)
         if not torch.is_grad_enabled() and projected.is_cuda and projected.dtype in (torch.float16, torch.float32):
             feats = knn_max_pool(idx, projected)      # one kernel, no [Nq, K, C] intermediate
+        elif (projected.is_cuda and projected.dtype in (torch.float16, torch.float32) and data_only(projected)
+              and idx.is_cuda and idx.dtype == torch.int32 and idx.numel() > 0 and projected.shape[0] > 0):
+            feats = KNNMaxPool.apply(idx, projected)
         else:
             rows = idx.view(-1).long().clamp_(min=0)
             feats = projected[rows].view(coarse.shape[0], self.k, projected.shape[1]).amax(dim=1)

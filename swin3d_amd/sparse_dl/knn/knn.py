@@ -9,6 +9,7 @@ import torch
 from torch.autograd.function import Function
 
 from ... import _lib
+from ...swin_blocks import data_only
 
 
 def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0, squared=True):
@@ -94,7 +95,7 @@ def knn_max_pool(idx, src_feat):
     """Channel-wise maximum of src_feat [Ns,C] over the K nearest sources of every query (idx int32 [Nq,K] of a
     knn_query result) -> [Nq,C] in the dtype of src_feat: the gather + max of the KNN downsample
     (Swin3D/modules/swin3d_layers.py:292-312) without the [Nq,K,C] intermediate.  Padded slots (row -1) read
-    row 0, as the clamped gather does.  No autograd (inference)."""
+    row 0, as the clamped gather does.  No autograd: KNNMaxPool has it."""
     if not (idx.is_cuda and src_feat.is_cuda):
         raise RuntimeError("idx and src_feat must be CUDA (HIP) tensors")
     if idx.dtype != torch.int32 or idx.dim() != 2:
@@ -111,6 +112,42 @@ def knn_max_pool(idx, src_feat):
                                              _FEAT_DTYPE[src_feat.dtype], out.data_ptr(), stream)
     _lib.check(status, "s3d_knn_max_pool")
     return out
+
+
+class KNNMaxPool(Function):
+    """Differentiable (w.r.t. the features) knn_max_pool: KNNMaxPool.apply(idx, src_feat).  Rows that share a maximum share
+    its gradient, as under torch's amax."""
+
+    @staticmethod
+    def forward(ctx, idx, src_feat):
+        idx, src_feat = idx.contiguous(), src_feat.contiguous()
+        out = knn_max_pool(idx, src_feat)
+        ctx.save_for_backward(idx, src_feat, out)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        idx, src_feat, out = ctx.saved_tensors
+        if torch.is_grad_enabled() or not data_only(dout) or dout.dtype != src_feat.dtype:
+            # a graph of the gradient is wanted, or something follows it: operations that have one
+            rows = idx.reshape(-1).long().clamp(min=0)
+            gathered = src_feat[rows].view(*idx.shape, src_feat.shape[1])
+            held = (gathered == out.unsqueeze(1)).to(dout.dtype)
+            given = (dout / held.sum(1)).unsqueeze(1) * held
+            return None, torch.zeros_like(src_feat).index_add(0, rows, given.reshape(-1, src_feat.shape[1]).to(src_feat.dtype))
+        dout = dout.contiguous()
+        (nq, k), (ns, c) = idx.shape, src_feat.shape
+        grad = torch.empty_like(src_feat)
+        code = _FEAT_DTYPE[src_feat.dtype]
+        lib = _lib.lib()
+        with _lib.on(src_feat.device):
+            ws_bytes = lib.s3d_knn_max_pool_grad_workspace_bytes(nq, k, ns, c, code)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=src_feat.device)
+            status = lib.s3d_knn_max_pool_grad(idx.data_ptr(), k, nq, src_feat.data_ptr(), ns, c, code, out.data_ptr(),
+                                               dout.data_ptr(), grad.data_ptr(), workspace.data_ptr(), ws_bytes,
+                                               _lib.stream(src_feat.device))
+        _lib.check(status, "s3d_knn_max_pool_grad")
+        return None, grad
 
 
 class KNNInterpolate(Function):
