@@ -103,9 +103,18 @@ def sparse_conv3x3x3(voxels, weight, neighbours=None):
     n, cin = feats.shape
     if neighbours is None:
         neighbours = conv3x3x3_neighbours(voxels.coords, voxels.stride)
+    if (feats.is_cuda and feats.dtype == torch.float32 and not feats.requires_grad and torch.is_autocast_enabled()
+            and torch.get_autocast_dtype("cuda") == torch.float16):
+        feats = feats.to(torch.float16)      # as the product takes it: the 27 copies are half as large
     padded = torch.cat([feats, feats.new_zeros(1, cin)], 0)   # row n = zeros for missing neighbours
     gathered = padded[neighbours.reshape(-1)].view(n, 27 * cin)
-    return gathered @ weight.reshape(27 * cin, -1).to(gathered.dtype)
+    weight = weight.reshape(27 * cin, -1)
+    if torch.is_grad_enabled() and feats.is_cuda and torch.is_autocast_enabled():
+        extra = (0, -27 * cin % 16)          # whole 16-byte pieces of a row
+        out = trained_linear(F.pad(gathered, extra), F.pad(weight.t(), extra), None)
+        if out is not None:
+            return out
+    return gathered @ weight.to(gathered.dtype)
 
 
 def pool_coordinates(coords, stride, factor):

@@ -5,7 +5,7 @@ import torch.nn as nn
 from torch.autograd.function import Function
 
 from . import _lib
-from .swin_blocks import data_only, plain
+from .swin_blocks import data_only, followed, plain
 
 _DTYPE_CODE = {torch.float32: _lib.S3D_DTYPE_F32, torch.float16: _lib.S3D_DTYPE_F16}
 
@@ -95,7 +95,7 @@ class _AddNorm(Function):
 def trained_add_norm(x, residual, norm):
     """(x + residual, norm(x + residual) in fp16) with gradients, for training under fp16 autocast where a dense layer takes
     the rows; None where it does not apply."""
-    if not (torch.is_grad_enabled() and x.is_cuda and torch.is_autocast_enabled()
+    if followed() or not (torch.is_grad_enabled() and x.is_cuda and torch.is_autocast_enabled()
             and torch.get_autocast_dtype("cuda") == torch.float16 and plain(norm, nn.LayerNorm)):
         return None
     weight, bias = norm.weight, norm.bias
@@ -103,8 +103,8 @@ def trained_add_norm(x, residual, norm):
             or x.shape[1] % 4 or x.shape[1] > 1024:
         return None
     for t, dtype in ((x, torch.float32), (weight, torch.float32), (bias, torch.float32), (residual, torch.float16)):
-        if t is not None and not ((data_only(t) or type(t) is nn.Parameter and data_only(t.data)) and t.dtype == dtype
-                                  and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0):
+        if t is not None and not (type(t) in (torch.Tensor, nn.Parameter) and t.dtype == dtype and t.device == x.device
+                                  and t.is_contiguous() and t.data_ptr() % 16 == 0):
             return None
     if residual is not None and residual.shape != x.shape:
         return None

@@ -6,7 +6,7 @@ import torch.nn.functional as F
 from torch.autograd.function import Function
 
 from . import _lib
-from .swin_blocks import data_only, linear_rows
+from .swin_blocks import data_only, followed, linear_rows
 
 
 _DTYPE_CODE = {torch.float32: _lib.S3D_DTYPE_F32, torch.float16: _lib.S3D_DTYPE_F16}
@@ -73,12 +73,12 @@ def trained_linear(x, weight, bias):
     if not (torch.is_grad_enabled() and x.is_cuda and torch.is_autocast_enabled()
             and torch.get_autocast_dtype("cuda") == torch.float16):
         return None
-    operands = (x, weight) if bias is None else (x, weight, bias)
-    if not all((data_only(t) or type(t) is torch.nn.Parameter and data_only(t.data)) and t.device == x.device
-               and t.dtype in (torch.float16, torch.float32) for t in operands):
-        return None
+    for t in (x, weight, bias):
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device != x.device
+                              or t.dtype not in (torch.float16, torch.float32)):
+            return None
     if x.dim() != 2 or weight.dim() != 2 or x.shape[0] == 0 or x.shape[1] != weight.shape[1] or x.shape[1] % 8 \
             or x.shape[1] == 0 or weight.shape[0] == 0 or max(weight.shape) > 16384 \
-            or (bias is not None and bias.shape != weight.shape[:1]):
+            or (bias is not None and bias.shape != weight.shape[:1]) or followed():
         return None
     return _Linear.apply(x.to(torch.float16), weight, bias)

@@ -19,11 +19,16 @@ def plain(m, kind):
             and not _module_hooks._global_backward_hooks and not _module_hooks._global_backward_pre_hooks)
 
 
+def followed():
+    """Something follows what is done to tensors, which a call by address would pass by: a transform, a forward-mode
+    derivative, a dispatch mode or a tracer."""
+    return (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
 def data_only(x):
-    """x is its data and nothing follows what is done to it: no subclass, no transform, forward-mode derivative, dispatch
-    mode or tracer, all of which a call by address would pass by."""
-    return (type(x) is torch.Tensor and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and not torch._C._len_torch_dispatch_stack() and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+    """x is its data (no subclass) and nothing follows what is done to it."""
+    return type(x) is torch.Tensor and not followed()
 
 
 def _parts(block, kinds):
