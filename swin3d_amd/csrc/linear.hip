@@ -8,8 +8,8 @@
 // spread over all banks; W goes in as the first operand, so that a lane ends up with four neighbouring outputs of one
 // row, and the tile leaves through LDS as whole rows.
 //
-// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 219 us against
-// 416 us as product and GELU apart, at 2.2 of the 5.1 TB/s that a copy reaches; 80 -> 240, 125 us against 207.  At the
+// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 202 us (178
+// without GELU) against 416 us as product and GELU apart, at 2.4 of the 4.7 TB/s that a copy reaches; 80 -> 240, 125 us against 207.  At the
 // deepest the tiles are few and a tile's chain of chunks is what counts: 811 rows, 384 -> 384, 5 us against 18 through
 // torch, whose launch alone takes the host that long.
 #include "linear.h"
@@ -25,18 +25,21 @@ constexpr int kThreads = 256;
 constexpr int kChunk = 64;        // numbers of K staged at a time
 constexpr int kPieces = kChunk / 8;
 
-// x Phi(x).  Phi by Abramowitz and Stegun 7.1.26 in its complementary form, erfc(z) = t (a1 + .. + a5 t^4) exp(-z^2),
-// t = 1 / (1 + p z): |error| < 1.5e-7, far below the rounding to fp16 that follows.
+// x Phi(x) = (x + |x|) / 2 - |x| Phi(-|x|), with 2 Phi(-u) = 2^p(u): the logarithm of the normal distribution's tail is
+// close to a parabola, and the polynomial of degree 7 with p(0) = 0 that fits it best for |x| Phi(-|x|) over [0, 5.8] (least
+// squares at Chebyshev nodes) is 2.5e-7 off, the rounding of fp32; from 5.8 on the tail is below fp16's smallest number.
+// Fifteen instruction slots where a rational form with an exponential took 22, and small results keep fp16's relative
+// precision.  Infinities and NaN as x Phi(x) has them: the first sum is NaN for -infinity.
 __device__ __forceinline__ float gelu(float x)
 {
-    const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
-    float poly = fmaf(1.061405429f, t, -1.453152027f);
-    poly = fmaf(poly, t, 1.421413741f);
-    poly = fmaf(poly, t, -0.284496736f);
-    poly = fmaf(poly, t, 0.254829592f);
-    const float tail = 0.5f * poly * t * __expf(-z * z);      // Phi(-|x|)
-    return x * (x > 0.0f ? 1.0f - tail : tail);
+    const float u = fabsf(x), c = fminf(u, 5.8f);
+    float p = fmaf(-7.429386528e-7f, c, 4.341329259e-5f);
+    p = fmaf(p, c, -8.166006301e-4f);
+    p = fmaf(p, c, 8.171264082e-3f);
+    p = fmaf(p, c, -5.347365886e-2f);
+    p = fmaf(p, c, -4.587851465e-1f);
+    p = fmaf(p, c, -1.151172519f);
+    return 0.5f * fmaf(-c, __builtin_amdgcn_exp2f(p * c), x + u);
 }
 
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.

@@ -29,6 +29,23 @@ def test_linear(hip_lib, m, n, k, gelu):
         assert bool(((got - want).abs() <= 6e-4 * want.abs() + 2e-6 * float(want.abs().max()) + 6e-7).all())
 
 
+def test_gelu_of_every_number(hip_lib):
+    """All finite fp16 numbers through the identity: half a place of rounding, and the approximation, which is fp32's own
+    rounding and below 2^-25 where the result is too small for fp16."""
+    x = torch.arange(-32768, 32768, device="cuda").to(torch.int16).view(torch.float16)
+    x = torch.where(x.isfinite(), x, 0).view(-1, 16)
+    got = linear_rows(x, torch.eye(16, device="cuda").half(), None, True).double()
+    wide = x.double()
+    want = 0.5 * wide * torch.special.erfc(-wide * 0.5 ** 0.5)
+    assert bool(((got - want).abs() <= 2.0 ** -11 * 1.02 * want.abs() + 2.0 ** -25 * 1.7).all())
+    assert got.isfinite().all()
+    x = torch.zeros(3, 16, device="cuda").half()
+    x[0, 0], x[1, 0], x[2, 0] = float("inf"), float("-inf"), float("nan")
+    w = torch.ones(8, 16, device="cuda").half()
+    got = linear_rows(x, w, None, True)
+    assert bool((got[0] == float("inf")).all()) and bool(got[1:].isnan().all())
+
+
 def test_linear_refuses_what_it_cannot_do(hip_lib):
     x, w = torch.randn(5, 24, device="cuda").half(), torch.randn(8, 24, device="cuda").half()
     assert linear_rows(x, w, None) is None and linear_rows(x.float(), w.float(), None) is None
