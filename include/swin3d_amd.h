@@ -373,7 +373,8 @@ int s3d_knn_distances(int32_t K, const float *src_xyz, int64_t Ns, const float *
  * Replaces the gather + max of the KNN downsample (Swin3D/modules/swin3d_layers.py:292-312: query_knn_feature
  * builds [Nq,K,C], then max over K) with one kernel that never writes the gathered copies:
  *   out[q][c] = max_i src_feat[max(idx[q][i], 0)][c]
- * A slot padded with row -1 reads row 0, exactly as the clamped index of the tensor statement does.
+ * A slot padded with row -1 reads row 0, exactly as the clamped index of the tensor statement does;
+ * NaN in one of the rows gives NaN, as under torch's amax.
  *   idx        device int32 [Nq,K] as written by s3d_knn
  *   src_feat   device [Ns,C] of `dtype` (Ns >= 1)        out   device [Nq,C] of `dtype`
  */
