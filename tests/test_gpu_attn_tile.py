@@ -37,7 +37,10 @@ def test_forward_stages_and_row_limits(oracle_lib, hip_lib, dtype, ws, cRSE, hea
     assert_attn_close(got, ref[0], dtype)
     assert np.allclose(omax, ref[1], rtol=0, atol=2e-5 * np.abs(ref[1]).max() if dtype == torch.float32 else 1e-3)
     assert np.allclose(osum, ref[2], rtol=1e-4 if dtype == torch.float32 else 3e-3)
-    assert np.array_equal(run_attention(case, dtype, device_sizes=True), got)
+    # (with statistics the sweep kernel runs, without them the tiles)
+    plain = run_attention(case, dtype)
+    assert_attn_close(plain, ref[0], dtype)
+    assert np.array_equal(run_attention(case, dtype, device_sizes=True), plain)
 
 
 def _backward(case, dtype, tables, dout, spare=0, part=1):
