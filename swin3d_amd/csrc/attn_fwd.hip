@@ -56,9 +56,9 @@ void *tile_list_of(const AttnArgs &a)
 }
 int launch_fwd(const AttnArgs &a, int dtype, hipStream_t stream, int what)
 {
-    // A call that leaves softmax statistics is a training step's, and stays on the sweep: a network's gradients go through
-    // maxima over neighbours, and another rounding of the features (2.7e-4 between the kernels, neither further from exact)
-    // moves which of two close ones wins, which is 2 % of the encoder's gradients on scans of 20,000 voxels.
+    // A call that leaves softmax statistics is a training step's, and stays on the sweep: the two kernels differ by fp16
+    // roundings of the features (2.7e-4, neither further from exact), and on scans of 20,000 voxels that gives another
+    // sample of the 2 to 5 % by which fp16 activations move the gradients of an encoder (2 % between the two).
     if (a.out_max || a.out_sum || !attn_tile_applies(a, dtype)) return launch_attn_sweep(a, dtype, stream, what);
     if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), stream, what)) return rc;
     if (!a.sizes_dev) return S3D_OK;

@@ -110,8 +110,7 @@ def sparse_conv3x3x3(voxels, weight, neighbours=None):
     gathered = padded[neighbours.reshape(-1)].view(n, 27 * cin)
     weight = weight.reshape(27 * cin, -1)
     if torch.is_grad_enabled() and feats.is_cuda and torch.is_autocast_enabled():
-        extra = (0, -27 * cin % 16)          # whole 16-byte pieces of a row
-        out = trained_linear(F.pad(gathered, extra), F.pad(weight.t(), extra), None)
+        out = trained_linear(gathered, weight.t(), None, any_width=True)
         if out is not None:
             return out
     return gathered @ weight.to(gathered.dtype)

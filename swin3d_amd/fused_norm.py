@@ -52,8 +52,8 @@ class _AddNorm(Function):
     @staticmethod
     def forward(ctx, x, residual, weight, bias, norm):
         ctx.set_materialize_grads(False)
-        # torch's own forward: a rounding of the mean elsewhere in fp32 moves single fp16 roundings, with them the winners
-        # of the maxima over neighbours, and a fiftieth of the encoder's gradients on scans of 20,000 voxels
+        # torch's own forward: a rounding of the mean elsewhere in fp32 moves single fp16 roundings of the rows, and with
+        # them the gradients of an encoder on scans of 20,000 voxels by a fiftieth (see linear_grad.py)
         summed = x if residual is None else x + residual.to(x.dtype)
         y = F.layer_norm(summed, norm.normalized_shape, weight, bias, norm.eps).to(torch.float16)
         ctx.save_for_backward(summed, weight)
