@@ -405,7 +405,7 @@ class WindowAttention(nn.Module):
         names = ("xyz", "rgb", "norm")[: crse_num_axes(self.cRSE) // 3]
         params = [self.qkv.weight, self.qkv.bias] + [getattr(self, f"{k}_{n}_table") for k in ("query", "key", "value")
                                                      for n in names]
-        key = (_cache_epoch(), dtype) + tuple((p.data_ptr(), p._version) for p in params if p is not None)
+        key = (_cache_epoch(), dtype, self.scale, self.cRSE) + tuple((p.data_ptr(), p._version) for p in params if p is not None)
         if caching and self._cache is not None and self._cache[0] == key:
             return self._cache[1]
         # q scale folded into the projection (a C x C multiply instead of an N x C one)

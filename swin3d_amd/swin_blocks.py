@@ -46,9 +46,15 @@ def _parts(block, kinds):
 
 
 def _stamp(parts):
-    """Addresses and versions of the parameters of the blocks, and the norms' epsilons."""
-    return [x for block in parts for i in (1, 2, 3, 4, 5, 7, 9) for p in block[i]._parameters.values() if p is not None
-            for x in (p.data_ptr(), p._version)] + [block[i].eps for block in parts for i in (1, 5)]
+    """What the descriptions of the blocks, and the decision that there are any, follow from: addresses and versions of the
+    parameters, and the plain attributes of the layers, which a program may set at any time."""
+    stamp = [x for block in parts for i in (1, 2, 3, 4, 5, 7, 9) for p in block[i]._parameters.values() if p is not None
+             for x in (p.data_ptr(), p._version)]
+    for _, norm1, attn, qkv, proj, norm2, _, fc1, _, fc2 in parts:
+        stamp += [attn.fp16_mode, attn.num_heads, attn.head_dim, attn.dim, attn.scale, attn.cRSE, *attn.table_sizes]
+        stamp += [x for norm in (norm1, norm2) for x in (norm.eps, *norm.normalized_shape)]
+        stamp += [x for layer in (qkv, proj, fc1, fc2) for x in (layer.in_features, layer.out_features)]
+    return stamp
 
 
 class _Kept:
@@ -133,7 +139,7 @@ def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
     library call does not stand for them.
 
     owner       the module that keeps the descriptions of the blocks between calls (`_s3d_blocks`), made anew when a
-                parameter, its version or `epoch` has changed
+                parameter, its version, an attribute of a layer or `epoch` has changed
     kinds       (block, attention, MLP) types the blocks have to be of
     feats       fp32 [N,C]; left as it is
     index_sets  per window set what index_arguments and window_signals give

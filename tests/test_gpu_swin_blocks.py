@@ -84,3 +84,26 @@ def test_blocks_in_one_call_equal_single_blocks(hip_lib, heads, dim, window, mod
     with torch.no_grad():
         stage.blocks[2].mlp.fc2.weight.mul_(3.0)
     assert (both() - first).abs().max() > 1e-2 * first.abs().max()
+
+
+def test_a_precision_set_after_a_call_is_followed(hip_lib):
+    """fp16_mode 0 is not the library call's: the blocks then run one by one, the attention in fp32."""
+    dev = torch.device("cuda")
+    scene = synth.make_room((3.0, 3.0, 2.0), 4, 5000, seed=5)
+    coords = torch.from_numpy(scene.coords).to(dev)
+    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)
+    torch.manual_seed(1)
+    stage = encoder.Stage(48, 2, 6, 5, 4, downsample=False, cRSE="XYZ_RGB_NORM", fp16_mode=2).to(dev).eval()
+    feats = torch.randn(coords.shape[0], 48, device=dev)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            return stage(encoder.SparseVoxels(coords, feats, 1), signals)[0].feats
+
+    run()
+    for block in stage.blocks:
+        block.attn.fp16_mode = 0
+    got = run()
+    del stage._s3d_blocks
+    assert torch.equal(got, run())
+    assert stage._s3d_blocks.described is None

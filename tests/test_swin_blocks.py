@@ -56,9 +56,24 @@ def test_upsample_projection_keeps_its_hooks(monkeypatch):
     assert calls == [1]
 
 
-def test_stamp_has_the_epsilons():
-    block = encoder.SwinBlock(16, 2, 5, 4)
+@pytest.mark.parametrize("layer,name,value", [
+    ("norm2", "eps", 1e-3), ("norm1", "normalized_shape", (4, 4)), ("attn", "fp16_mode", 0), ("attn", "scale", 0.1),
+    ("attn", "num_heads", 4), ("attn", "head_dim", 4), ("attn", "dim", 8), ("attn", "cRSE", "XYZ"),
+    ("attn", "table_sizes", [16] * 6), ("mlp.fc1", "out_features", 32),
+])
+def test_stamp_has_what_the_descriptions_follow_from(layer, name, value):
+    block = encoder.SwinBlock(16, 2, 5, 4, cRSE="XYZ_RGB", fp16_mode=2)
     parts = [swin_blocks._parts(block, (encoder.SwinBlock, encoder.WindowAttention, encoder.Mlp))]
     before = swin_blocks._stamp(parts)
-    block.norm2.eps = 1e-3
+    assert swin_blocks._stamp(parts) == before
+    setattr(block.get_submodule(layer), name, value)
     assert swin_blocks._stamp(parts) != before
+
+
+def test_a_scale_set_after_a_call_reaches_the_projection():
+    attn = encoder.WindowAttention(16, 5, 4, 2, cRSE="XYZ")
+    with torch.no_grad():
+        first = attn._prepared()[0]
+        attn.scale *= 2
+        second = attn._prepared()[0]
+    assert torch.equal(second[:16], 2 * first[:16]) and torch.equal(second[16:], first[16:])
