@@ -507,12 +507,12 @@ __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__
 __global__ __launch_bounds__(kThreads) void window_signals_kernel(
     const int32_t *__restrict__ w_w_id, const int32_t *__restrict__ n2n, const float *__restrict__ frac,
     const float *__restrict__ signals, int64_t signals_stride, int columns, int window, float xyz_scale,
-    float other_scale, float *__restrict__ out, int64_t N, int rows)
+    float other_scale, float *__restrict__ out, int64_t N)
 {
 #pragma clang fp contract(off)
     extern __shared__ float tile[];
-    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * rows, p = p0 + threadIdx.x;
-    if (static_cast<int>(threadIdx.x) < rows && p < N) {
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kThreads, p = p0 + threadIdx.x;
+    if (p < N) {
         float *to = tile + threadIdx.x * columns;
         const int64_t row = n2n[p];
         const int id = w_w_id[p];
@@ -525,8 +525,29 @@ __global__ __launch_bounds__(kThreads) void window_signals_kernel(
         for (int c = 3; c < columns; ++c) to[c] = from[c - 3] * other_scale;
     }
     __syncthreads();
-    const int here = static_cast<int>(min(static_cast<int64_t>(rows), N - p0)) * columns;
+    const int here = static_cast<int>(min(static_cast<int64_t>(kThreads), N - p0)) * columns;
     for (int t = threadIdx.x; t < here; t += kThreads) out[p0 * columns + t] = tile[t];
+}
+
+// The same for rows too wide for a workgroup's LDS: a thread per element.
+__global__ __launch_bounds__(kThreads) void window_signals_wide_kernel(
+    const int32_t *__restrict__ w_w_id, const int32_t *__restrict__ n2n, const float *__restrict__ frac,
+    const float *__restrict__ signals, int64_t signals_stride, int columns, int window, float xyz_scale,
+    float other_scale, float *__restrict__ out, int64_t N)
+{
+#pragma clang fp contract(off)
+    const int64_t step = static_cast<int64_t>(gridDim.x) * kThreads;
+    for (int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; t < N * columns; t += step) {
+        const int64_t p = t / columns, row = n2n[p];
+        const int c = static_cast<int>(t - p * columns);
+        if (c < 3) {
+            const int id = w_w_id[p];
+            const int cell = c == 0 ? id / (window * window) : c == 1 ? (id / window) % window : id % window;
+            out[t] = (static_cast<float>(cell) + frac[row * 3 + c]) * xyz_scale;
+        } else {
+            out[t] = signals[row * signals_stride + (c - 3)] * other_scale;
+        }
+    }
 }
 
 // one thread per (sorted voxel, offset): binary search of key + delta in the sorted keys
@@ -644,13 +665,19 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_signals(
     if (!w_w_id || !n2n || !frac || !out || (num_signals > 0 && !signals))
         return fail(S3D_ERR_NULL_POINTER, "s3d_window_signals: null device pointer");
     const int columns = 3 + num_signals;
-    // as many rows a workgroup as half of the LDS of a launch without special attributes takes
-    if (columns > 8192) return fail(S3D_ERR_BAD_SHAPE, "s3d_window_signals: num_signals=%d", num_signals);
-    const int rows = columns <= 8192 / kThreads ? kThreads : 8192 / columns;
-    const dim3 grid(static_cast<unsigned>(ceil_div(N, rows)));
-    const uint32_t lds = rows * columns * sizeof(float);
+    // a row per thread while a workgroup's rows fit half of the LDS of a launch without special attributes
+    if (columns > 8192 / kThreads) {
+        const int64_t groups = ceil_div(N * columns, kThreads);
+        hipLaunchKernelGGL(window_signals_wide_kernel, dim3(static_cast<unsigned>(groups < 65536 ? groups : 65536)), dim3(kThreads), 0,
+                           static_cast<hipStream_t>(stream), w_w_id, n2n, frac, signals, signals_stride, columns, window, xyz_scale,
+                           other_scale, out, N);
+        S3D_HIP_CHECK(hipGetLastError());
+        return S3D_OK;
+    }
+    const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)));
+    const uint32_t lds = kThreads * columns * sizeof(float);
     hipLaunchKernelGGL(window_signals_kernel, grid, dim3(kThreads), lds, static_cast<hipStream_t>(stream), w_w_id, n2n,
-                       frac, signals, signals_stride, columns, window, xyz_scale, other_scale, out, N, rows);
+                       frac, signals, signals_stride, columns, window, xyz_scale, other_scale, out, N);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

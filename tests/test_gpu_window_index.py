@@ -123,6 +123,21 @@ def test_window_signals_match_the_tensor_statement(hip_lib, num_signals):
     assert torch.equal(got, ref * scale)
 
 
+@pytest.mark.parametrize("num_signals", [29, 30, 400, 9000])
+def test_window_signals_of_wide_rows(hip_lib, num_signals):
+    """32 columns are the last that a workgroup holds a row per thread of; there is no most."""
+    import swin3d_amd
+    rng = np.random.default_rng(num_signals)
+    n = 300 if num_signals > 1000 else 3000
+    coords = torch.from_numpy(random_scene(rng, n, extent=(30, 30, 10), batches=2)).cuda()
+    frac = torch.rand((n, 3), device="cuda")
+    colors = torch.rand((n, num_signals + 2), device="cuda")
+    index = swin3d_amd.build_window_index(coords, 1, 5)
+    order = index.n2n.long()
+    got = swin3d_amd.window_signals(index, frac, colors, num_signals, 4, 8)
+    assert torch.equal(got, torch.cat([(index.local_xyz().float() + frac[order]) * 4, colors[order, :num_signals] * 8], 1))
+
+
 def test_several_window_sets_in_one_call(oracle_lib, hip_lib):
     """build_window_indices enqueues all sets before its one host wait; each equals its single build."""
     import swin3d_amd
