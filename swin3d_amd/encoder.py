@@ -25,6 +25,7 @@ anything in the reference; here pooled voxels are sorted by (batch, x, y, z) and
 the lower row.  Stochastic depth is inference-time identity.
 """
 from dataclasses import dataclass
+from functools import partial
 
 import torch
 import torch.nn as nn
@@ -422,7 +423,7 @@ class WindowAttention(nn.Module):
 
     def forward(self, feats, attn_args):
         n = feats.shape[0]
-        _, _, m2w, w_sizes, w2n, n2n, w2m, n_coords = attn_args[:8]
+        _, _, m2w, w_sizes, w2n, n2n, w2m = attn_args[:7]
         weight, bias, tables = self._prepared()
         # q, k, v stay slices of the [N, 3C] projection output, which the attention kernels read in place
         qkv = trained_linear(feats, weight, bias)
@@ -430,7 +431,7 @@ class WindowAttention(nn.Module):
         # (unbind: its gradient is one stack, that of three slices three zeroed buffers and their sum)
         query, key, value = qkv.view(n, 3, self.num_heads, self.head_dim).unbind(1)
         # the scaled signals of the index set, when the caller prepared them once for all blocks that share it
-        n_crse = attn_args[8] if len(attn_args) > 8 else scale_crse_coords(n_coords, self.quant_size, self.cRSE)
+        n_crse = attn_args[8] if len(attn_args) > 8 else scale_crse_coords(attn_args[7], self.quant_size, self.cRSE)
         precision = (PrecisionMode.HALF_NONE, PrecisionMode.HALF_FORWARD, PrecisionMode.HALF_ALL)[self.fp16_mode]
         out = SelfAttnAIOFunction.apply(
             query, key, value, *tables, self.table_sizes, [m2w, w_sizes, w2m, w2n, n2n, n_crse], PosEmb.SEPARATE,
@@ -484,6 +485,41 @@ class SwinBlock(nn.Module):
         return _fused_norm_applies(feats)
 
 
+class StageArguments(tuple):
+    """What a block's attention takes for one window set: the tuple of index_arguments and, behind it, the scaled signals,
+    which is what the attention of this file reads.  The unscaled signals (the eighth entry) are made when they are asked
+    for: a kernel per window set of a pass that only blocks with an attention of their own need."""
+
+    UNSCALED = 7
+
+    def __new__(cls, index, n2n, scaled, unscaled):
+        self = super().__new__(cls, (None, None, None, index.w_sizes, index.w2n, n2n, None, None, scaled))
+        self._make = unscaled
+        return self
+
+    def _whole(self):
+        if self._make is not None:
+            self._made = self._make()
+            self._make = None
+        items = list(tuple.__iter__(self))
+        items[self.UNSCALED] = self._made
+        return tuple(items)
+
+    def __getitem__(self, at):
+        asked = range(len(self))[at]
+        needs = self.UNSCALED in asked if isinstance(at, slice) else asked == self.UNSCALED
+        return self._whole()[at] if needs else tuple.__getitem__(self, at)
+
+    def __iter__(self):
+        return iter(self._whole())
+
+    def __add__(self, other):
+        return self._whole() + other
+
+    def __reduce__(self):
+        return tuple, (self._whole(),)
+
+
 class Stage(nn.Module):
     """`depth` Swin blocks on one resolution (regular / shifted windows alternate), then an
     optional KNN downsample."""
@@ -516,15 +552,16 @@ class Stage(nn.Module):
         cell_index = indices.pop() if pooled else None
         if len(self.blocks) > 0:
             # the quantiser scaling of the signals is the same for every block of the stage: once per index set,
-            # fused with the gather into window order (and in place of the unscaled signals, which nobody reads)
+            # fused with the gather into window order
             attn = self.blocks[0].attn
-            args = [(None, None, None, index.w_sizes, index.w2n, index.n2n, None, None,
-                     window_signals(index, local, extra, crse_num_axes(attn.cRSE) - 3, attn.quant_size, 2 * attn.quant_size))
-                    for index in indices]
+            args = [StageArguments(index, index.n2n if i > 0 or not rows_in_window_order else None,      # (None: no row map)
+                                   window_signals(index, local, extra, crse_num_axes(attn.cRSE) - 3, attn.quant_size,
+                                                  2 * attn.quant_size), partial(window_signals, index, local, extra))
+                    for i, index in enumerate(indices)]
         else:
             args = [index_arguments(index, local, extra) for index in indices]
-        if rows_in_window_order and args:
-            args[0] = args[0][:5] + (None,) + args[0][6:]      # (.., w2n, n2n, w2m, ..): no row map
+            if rows_in_window_order and args:
+                args[0] = args[0][:5] + (None,) + args[0][6:]      # (.., w2n, n2n, w2m, ..): no row map
         down = (self.downsample.plan(coords, stride, signals, num_batches, cell_index)
                 if self.downsample is not None else None)
         return args, down

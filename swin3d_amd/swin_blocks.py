@@ -176,7 +176,7 @@ def swin_blocks(owner, blocks, kinds, feats, index_sets, epoch, half_copy):
     with _lib.on(dev):
         stream = _lib.stream(dev)
         for s, args in zip(sets, index_sets):
-            _, _, _, w_sizes_in, w2n_in, n2n, _, _, coords = args[:9]
+            w_sizes_in, w2n_in, n2n, coords = args[3], args[4], args[5], args[8]
             w_sizes, w2n = (attn_coff._as_int32(name, t, dev) for name, t in (("w_sizes", w_sizes_in), ("w2n", w2n_in)))
             n2n = None if n2n is None else attn_coff._as_int32("n2n", n2n, dev)
             coords = coords.float().contiguous()

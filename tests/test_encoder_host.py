@@ -190,3 +190,19 @@ def test_state_dict_names_are_the_reference_checkpoints(tmp_path):
     with pytest.raises(RuntimeError, match="mlp.fc1"):
         model.load_pretrained_model(str(tmp_path / "renamed.pth"), verbose=False)
     assert model.load_pretrained_model(str(tmp_path / "renamed.pth"), verbose=False, strict_encoder=False)
+
+
+def test_stage_arguments_make_the_unscaled_signals_when_asked():
+    import copy
+    from types import SimpleNamespace
+    calls = []
+    make = lambda: calls.append(1) or "unscaled"
+    index = SimpleNamespace(w_sizes="sizes", w2n="starts")
+    args = encoder.StageArguments(index, "rows", "scaled", make)
+    assert isinstance(args, tuple) and len(args) == 9
+    assert (args[3], args[4], args[5], args[8], args[-1], args[:7][5], args[8:]) == ("sizes", "starts", "rows", "scaled", "scaled", "rows", ("scaled",))
+    assert not calls
+    whole = (None, None, None, "sizes", "starts", "rows", None, "unscaled", "scaled")
+    assert args[7] == args[-2] == "unscaled" and args[:8] == whole[:8] and tuple(args) == whole and args + (1,) == whole + (1,)
+    *_, n_coords, scaled = args
+    assert (n_coords, scaled, len(calls)) == ("unscaled", "scaled", 1) and copy.copy(args) == whole
