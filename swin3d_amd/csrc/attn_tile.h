@@ -10,6 +10,7 @@ namespace tile {
 
 using namespace sweep;
 
+constexpr int D = 16;                    // channels of a head
 constexpr int kThreads = 512;            // eight wavefronts; two workgroups share a CU (LDS, 128 registers)
 constexpr int kWaves = kThreads / 64;
 constexpr int kCols = 64;                // voxels on either side of a tile
@@ -66,14 +67,10 @@ struct Unit {
 };
 inline size_t list_round(size_t bytes) { return (bytes + 255) / 256 * 256; }
 // a unit covers at least 32 voxels (a tile of a window of 65), but for the last one of each window size up to 32
-inline size_t list_max_units(int64_t N, int64_t W)
-{
-    (void)W;
-    return static_cast<size_t>(N > 0 ? N : 0) / 32 + kCols + 1;
-}
+inline size_t list_max_units(int64_t N) { return static_cast<size_t>(N > 0 ? N : 0) / 32 + kCols + 1; }
 inline size_t list_bytes(int64_t N, int64_t W)
 {
-    return 256 + list_round(sizeof(int4) * list_max_units(N, W)) + list_round(sizeof(int2) * static_cast<size_t>(W > 0 ? W : 1));
+    return 256 + list_round(sizeof(int4) * list_max_units(N)) + list_round(sizeof(int2) * static_cast<size_t>(W > 0 ? W : 1));
 }
 inline UnitList list_at(void *p, int64_t N, int64_t W)
 {
@@ -81,7 +78,7 @@ inline UnitList list_at(void *p, int64_t N, int64_t W)
     UnitList l;
     l.total = reinterpret_cast<const int32_t *>(base);
     l.units = reinterpret_cast<const int4 *>(base + 256);
-    l.entries = reinterpret_cast<const int2 *>(base + 256 + list_round(sizeof(int4) * list_max_units(N, W)));
+    l.entries = reinterpret_cast<const int2 *>(base + 256 + list_round(sizeof(int4) * list_max_units(N)));
     return l;
 }
 int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, int64_t W, hipStream_t stream);
@@ -248,10 +245,6 @@ __device__ __forceinline__ void store4(__half *p, const float *v)
     reinterpret_cast<__half2 *>(&x)[1] = __floats2half2_rn(v[2], v[3]);
     *reinterpret_cast<uint2 *>(p) = x;
 }
-__device__ __forceinline__ void lds_store4(uint32_t addr, float a, float b, float c, float d)
-{
-    *(__attribute__((address_space(3))) f32x4_t *)(addr) = f32x4_t{a, b, c, d};
-}
 __device__ __forceinline__ void lds_add(uint32_t addr, uint32_t v)
 {
     __hip_atomic_fetch_add((lds_u32 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -341,7 +334,6 @@ template <> struct Operand<__half> {
     __device__ __forceinline__ void set(const Raw &r) { x = __builtin_bit_cast(f16x8, r.v); }
     __device__ __forceinline__ void load(const __half *p) { x = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4 *>(p)); }
     __device__ __forceinline__ void load_lds(uint32_t addr) { x = __builtin_bit_cast(f16x8, *(lds_u32x4 *)(addr)); }
-    __device__ __forceinline__ void clear() { x = f16x8{}; }
     __device__ __forceinline__ void set_values(const __half *v)
     {
 #pragma unroll
@@ -396,11 +388,6 @@ template <> struct Operand<float> {
             v[c] = q[0]; v[c + 1] = q[1]; v[c + 2] = q[2]; v[c + 3] = q[3];
         }
         split(v);
-    }
-    __device__ __forceinline__ void clear()
-    {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(bf16x8, u32x4{});
     }
 };
 // a 32 x 32 result over 16 terms: A row lane % 32, B column lane % 32, terms 8 (lane / 32) + 0..7; the result's column

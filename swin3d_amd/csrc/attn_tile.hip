@@ -20,7 +20,7 @@ constexpr float kFix = 33554432.0f;        // 2^25: at most 64 weights of at mos
 constexpr float kCellScale = 1.0f / 1048576.0f;   // cells enter the products in units of 2^20
 constexpr float kOutScale = 1.0f / 32.0f;
 
-template <typename T, int D, int ND> struct FwdLayout {
+template <typename T, int ND> struct FwdLayout {
     static constexpr int kSt = Stages<ND>::kCount;
     static constexpr uint32_t kSums = kCols * kStride * 4;                       // a [row][column] array of fp32 or u32
     static constexpr uint32_t kKeys = kCols * kKeyStride * 4;                    // keys: coordinates and table products
@@ -31,10 +31,10 @@ template <typename T, int D, int ND> struct FwdLayout {
     static constexpr uint32_t kBytes = kSums + kKeys + kTableT + kValueT + kCoords + kMeta;
 };
 
-template <typename T, int D, int ND, bool kDeviceSizes>
+template <typename T, int ND, bool kDeviceSizes>
 __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
 {
-    using L = FwdLayout<T, D, ND>;
+    using L = FwdLayout<T, ND>;
     using S = Stages<ND>;
     const AttnArgs &a = f.a;
     extern __shared__ __align__(16) float smem[];
@@ -130,22 +130,17 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             const int lane = opaque(tid & 63);
             const int m32 = lane & 31, half32 = lane >> 5;       // row or column, and group of terms, of a 32x32 operand
             const int n16 = lane & 15, group16 = lane >> 4;
-            const bool term_lane = D > 8 || half32 == 0;         // head_dim 8: the other half of the terms is zero
             // operands that stay for all stages: queries (wavefronts 0..3) or keys
             Operand<T> feat;
-            feat.clear();
-            if (term_lane) {
+            {
                 const int row = static_cast<int>(lds_load_u32((wave < 4 ? row_i : row_j) + (tile_c * 32 + m32) * 4));
                 feat.load((wave < 4 ? gq : gk) + static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_stride + h * D + half32 * 8);
             }
             if (wave < 4) {
                 // q . k of the tile, [key][query]
                 Operand<T> kf;
-                kf.clear();
-                if (term_lane) {
-                    const int row = static_cast<int>(lds_load_u32(row_j + (tile_r * 32 + m32) * 4));
-                    kf.load(gk + static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_stride + h * D + half32 * 8);
-                }
+                const int row = static_cast<int>(lds_load_u32(row_j + (tile_r * 32 + m32) * 4));
+                kf.load(gk + static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_stride + h * D + half32 * 8);
                 const f32x16 d = mfma32(kf, feat, f32x16{});
                 const uint32_t to = sums + ((tile_r * 32 + 4 * half32) * kStride + tile_c * 32 + m32) * 4;
 #pragma unroll
@@ -191,14 +186,13 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 return table_qk + (__umul24((second ? first_row(other) : first_row(one)) + r, HD) + h * D + half32 * 8);
             };
             typename Operand<T>::Raw raw{};
-            if (stage_needed(0) && term_lane) raw = Operand<T>::fetch(stage_rows(0));
+            if (stage_needed(0)) raw = Operand<T>::fetch(stage_rows(0));
 #pragma unroll
             for (int st = 0; st < S::kCount; ++st) {
                 lds_barrier();
                 if (stage_needed(st)) {
                     Operand<T> rows;
-                    rows.clear();
-                    if (term_lane) rows.set(raw);
+                    rows.set(raw);
                     // [row][query] for the queries, [key][row] for the keys (16-byte stores of four consecutive words a
                     // lane, which the transposed product would give, met in more banks: +2 %)
                     if (wave < 4) {
@@ -213,7 +207,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                         for (int e = 0; e < 16; ++e) lds_store(to + mfma32_row(0, e) * kKeyStride * 4, d[e]);
                     }
                 }
-                if (st + 1 < S::kCount && stage_needed(st + 1) && term_lane) raw = Operand<T>::fetch(stage_rows(st + 1));
+                if (st + 1 < S::kCount && stage_needed(st + 1)) raw = Operand<T>::fetch(stage_rows(st + 1));
                 lds_barrier();
 #pragma unroll
                 for (int b = 0; b < (S::paired(st) ? 2 : 1); ++b) {
@@ -271,7 +265,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 // the sum of a pair's rows in that type costs elsewhere)
                 if (table) b.set_single(v, kCellScale); else b.set(v, kCellScale);
                 Operand<T> t;
-                t.load_lds(operand + ((D > 8 ? n16 : n16 & 7) * kStride + out_half * 32 + group16 * 8) * sizeof(T));
+                t.load_lds(operand + (n16 * kStride + out_half * 32 + group16 * 8) * sizeof(T));
                 tile_acc = table ? mfma16_single(t, b, tile_acc) : mfma16(t, b, tile_acc);
             };
             lds_barrier();
@@ -319,37 +313,23 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             const f32x4_t other = *(__attribute__((address_space(3))) f32x4_t *)(meet);
             const float inv = kOutScale / run_sum;
             const int64_t row = static_cast<int>(lds_load_u32(row_i + i * 4));
-            if (group16 * 4 < D) {
-                float o[4];
+            float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = (acc[e] + other[e]) * inv;
-                T *to = static_cast<T *>(a.out) + row * HD + h * D + group16 * 4;
-                if constexpr (sizeof(T) == 2) {
-                    uint2 x;
-                    reinterpret_cast<__half2 *>(&x)[0] = __floats2half2_rn(o[0], o[1]);
-                    reinterpret_cast<__half2 *>(&x)[1] = __floats2half2_rn(o[2], o[3]);
-                    *reinterpret_cast<uint2 *>(to) = x;
-                } else {
-                    *reinterpret_cast<float4 *>(to) = make_float4(o[0], o[1], o[2], o[3]);
-                }
-            }
-            if (group16 == 0) {
-                if (a.out_max) a.out_max[row * H + h] = run_max;
-                if (a.out_sum) a.out_sum[row * H + h] = run_sum;
-            }
+            for (int e = 0; e < 4; ++e) o[e] = (acc[e] + other[e]) * inv;
+            store4(static_cast<T *>(a.out) + row * HD + h * D + group16 * 4, o);
         }
     }
 }
 
-template <typename T, int D, int ND, bool kDeviceSizes>
+template <typename T, int ND, bool kDeviceSizes>
 int launch_fwd(const AttnArgs &a, const UnitList &list, hipStream_t stream)
 {
-    using L = FwdLayout<T, D, ND>;
+    using L = FwdLayout<T, ND>;
     FwdArgs f;
     f.a = a;
     f.list = list;
     constexpr uint32_t lds = L::kBytes;
-    auto kernel = attn_fwd_tile_kernel<T, D, ND, kDeviceSizes>;
+    auto kernel = attn_fwd_tile_kernel<T, ND, kDeviceSizes>;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
     const int per_cu = lds <= 80 * 1024 ? 2 : 1;
     const int slots = per_cu * device_cus();
@@ -394,7 +374,7 @@ size_t attn_tile_list_bytes(int H, int64_t N, int64_t W)
 
 bool attn_tile_applies(const AttnArgs &a, int dtype)
 {
-    if (a.D != 16 || !attn_tile_shape(a.N, a.W, a.H, dtype == S3D_DTYPE_F32)) return false;
+    if (a.D != tile::D || !attn_tile_shape(a.N, a.W, a.H, dtype == S3D_DTYPE_F32)) return false;
     return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
 }
 
@@ -405,11 +385,11 @@ int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t strea
         if (int rc = tile::launch_list(l, a.w_sizes, a.w2n, a.W, stream)) return rc;
     }
     if (!(what & kAttnSweep)) return S3D_OK;
-#define S3D_CASE(TT, CODE, DD, NN)                                                        \
-    if (dtype == CODE && a.D == DD && a.nd == NN)                                         \
-        return a.sizes_dev ? tile::launch_fwd<TT, DD, NN, true>(a, l, stream) : tile::launch_fwd<TT, DD, NN, false>(a, l, stream);
-    S3D_CASE(__half, S3D_DTYPE_F16, 16, 3) S3D_CASE(__half, S3D_DTYPE_F16, 16, 6) S3D_CASE(__half, S3D_DTYPE_F16, 16, 9)
-    S3D_CASE(float, S3D_DTYPE_F32, 16, 3) S3D_CASE(float, S3D_DTYPE_F32, 16, 6) S3D_CASE(float, S3D_DTYPE_F32, 16, 9)
+#define S3D_CASE(TT, CODE, NN)                                                            \
+    if (dtype == CODE && a.D == tile::D && a.nd == NN)                                    \
+        return a.sizes_dev ? tile::launch_fwd<TT, NN, true>(a, l, stream) : tile::launch_fwd<TT, NN, false>(a, l, stream);
+    S3D_CASE(__half, S3D_DTYPE_F16, 3) S3D_CASE(__half, S3D_DTYPE_F16, 6) S3D_CASE(__half, S3D_DTYPE_F16, 9)
+    S3D_CASE(float, S3D_DTYPE_F32, 3) S3D_CASE(float, S3D_DTYPE_F32, 6) S3D_CASE(float, S3D_DTYPE_F32, 9)
 #undef S3D_CASE
     return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_fwd: head_dim %d, %d axes in the tile form", a.D, a.nd);
 }

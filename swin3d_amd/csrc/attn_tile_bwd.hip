@@ -31,7 +31,6 @@ namespace s3d {
 namespace tile {
 namespace {
 
-constexpr int D = 16;
 constexpr float kFixWeight = 33554432.0f;     // 2^25: P <= 1, at most 64 meet in a cell of 32 unsigned bits
 constexpr float kFixGrad = 16777216.0f;       // 2^24: |dL| <= 1 after scaling, at most 64 in a cell of 32 signed bits
 constexpr float kWeightCell = 1.0f / kFixWeight, kGradCell = 1.0f / kFixGrad;
@@ -810,7 +809,7 @@ int launch_bwd(const BwdTileArgs &b0, hipStream_t stream)
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(gradients), lds_g)) return rc;
     const dim3 grid(static_cast<unsigned>(b.groups * a.H));
     hipLaunchKernelGGL((tile_setup_kernel<T, TF, ND>), dim3(static_cast<unsigned>(1 + 5 * a.H)), dim3(kListThreads), 0, stream, b);
-    const int64_t most_units = static_cast<int64_t>(list_max_units(a.N, a.W));
+    const int64_t most_units = static_cast<int64_t>(list_max_units(a.N));
     hipLaunchKernelGGL(tile_columns_kernel<ND>, dim3(static_cast<unsigned>(ceil_div(most_units, 4))), dim3(256), 0, stream, b);
     hipLaunchKernelGGL(records, grid, dim3(kThreads), lds_r, stream, b);
     hipLaunchKernelGGL(gradients, grid, dim3(kThreads), lds_g, stream, b);
@@ -830,7 +829,7 @@ size_t slots_bytes(int H, int nd)
 }
 
 // row, first pair and coordinates of the units' columns
-size_t columns_bytes(int64_t N, int64_t W, int nd) { return align_up(sizeof(int32_t) * list_max_units(N, W) * kCols * (2 + static_cast<size_t>(nd)), 256); }
+size_t columns_bytes(int64_t N, int nd) { return align_up(sizeof(int32_t) * list_max_units(N) * kCols * (2 + static_cast<size_t>(nd)), 256); }
 
 // tables as operands, at most 48 bytes a lane, and their scales
 size_t operand_bytes(int H, int nd)
@@ -855,7 +854,7 @@ size_t attn_tile_bwd_bytes(int H, int nd, int64_t N, int64_t W, int64_t pairs)
 {
     return align_up(sizeof(float2) * static_cast<size_t>(H) * pairs, 256) +
            align_up(sizeof(float) * static_cast<size_t>(pairs / 64 + N) * H * 2 * tile::D, 256) + tile::slots_bytes(H, nd) +
-           tile::operand_bytes(H, nd) + tile::columns_bytes(N, W, nd) + tile::list_bytes(N, W);
+           tile::operand_bytes(H, nd) + tile::columns_bytes(N, nd) + tile::list_bytes(N, W);
 }
 
 int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, float *dtk, float *dtv, void *workspace, int dtype,
@@ -874,11 +873,11 @@ int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, floa
     b.operands = at;
     at += tile::operand_bytes(H, nd);
     b.scales = reinterpret_cast<float *>(at - align_up(sizeof(float) * 5 * static_cast<size_t>(H), 256));
-    const size_t columns = tile::list_max_units(p.f.N, p.f.W) * tile::kCols;
+    const size_t columns = tile::list_max_units(p.f.N) * tile::kCols;
     b.rows = reinterpret_cast<int32_t *>(at);
     b.first_pair = b.rows + columns;
     b.coords = reinterpret_cast<float *>(b.first_pair + columns);
-    at += tile::columns_bytes(p.f.N, p.f.W, nd);
+    at += tile::columns_bytes(p.f.N, nd);
     b.list = tile::list_at(at, p.f.N, p.f.W);
     b.dout = p.dout;
     b.out = out;
