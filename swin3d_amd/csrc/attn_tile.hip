@@ -16,9 +16,18 @@ struct FwdArgs {
     UnitList list;
 };
 
-constexpr float kFix = 33554432.0f;        // 2^25: at most 64 weights of at most 1 meet in a cell
-constexpr float kCellScale = 1.0f / 1048576.0f;   // cells enter the products in units of 2^20
-constexpr float kOutScale = 1.0f / 32.0f;
+// Softmax weights in a tile.  A query's weights are at most 1 and sum to less than 2^e (e from their sum l).
+//  * their sum: 64-bit integers in units of 2^-57, which hold a thread's partial sum in fp32 as it is;
+//  * summed by table row: 32-bit integers in units of 2^(e-31), below 2^-31 of the sum of all weights, so that a cell keeps
+//    what fp32 would whatever else falls into it, and no order of additions shows;
+//  * beside a value: as they are, in fp32.
+// They enter the matrix products over 2^(e - kLift): beside fp16 operands as two fp16 numbers, 23 bits from 2^15 down to
+// 2^-3 and units of 2^-25 below, which is 2^-40 of the sum; beside fp32 in full.
+constexpr float kSumFix = 33554432.0f;               // 2^25: the high word of a sum, at most 64 weights
+constexpr float kSumLow = 1.0f / 4294967296.0f;
+constexpr int kCellBits = 31;
+template <typename T> constexpr int kLift = sizeof(T) == 2 ? 15 : 0;      // (fp32 values may be as large as fp32 is)
+template <typename T> constexpr float kCellScale = sizeof(T) == 2 ? 1.0f / 65536.0f : 1.0f / 2147483648.0f;   // 2^(kLift - kCellBits)
 
 template <typename T, int ND> struct FwdLayout {
     static constexpr int kSt = Stages<ND>::kCount;
@@ -27,7 +36,7 @@ template <typename T, int ND> struct FwdLayout {
     static constexpr uint32_t kTableT = kSt * D * kStride * sizeof(T);           // value table, [stage][channel][row]
     static constexpr uint32_t kValueT = D * kStride * sizeof(T);                 // values of the tile, [channel][key]
     static constexpr uint32_t kCoords = ND * kCols * 4;
-    static constexpr uint32_t kMeta = 4 * kCols * 4;                             // rows of queries and keys, maxima, sums
+    static constexpr uint32_t kMeta = 5 * kCols * 4;                             // sums (64 bits), rows of queries and keys, maxima
     static constexpr uint32_t kBytes = kSums + kKeys + kTableT + kValueT + kCoords + kMeta;
 };
 
@@ -62,8 +71,12 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
 
     const uint32_t base = lds_base(smem);
     const uint32_t sums = base, keys = sums + L::kSums, table_t = keys + L::kKeys, value_t = table_t + L::kTableT;
-    const uint32_t coords = value_t + L::kValueT, row_i = coords + L::kCoords, row_j = row_i + kCols * 4;
-    const uint32_t col_max = row_j + kCols * 4, col_sum = col_max + kCols * 4;
+    const uint32_t coords = value_t + L::kValueT, col_sum = coords + L::kCoords, row_i = col_sum + kCols * 8;
+    const uint32_t row_j = row_i + kCols * 4, col_max = row_j + kCols * 4;
+    auto sum_of = [&](int c) {
+        return fmaf(static_cast<float>(lds_load_u32(col_sum + c * 8)), kSumLow / kSumFix,
+                    static_cast<float>(lds_load_u32(col_sum + c * 8 + 4)) * (1.0f / kSumFix));
+    };
 
     const T *gq = static_cast<const T *>(a.q), *gk = static_cast<const T *>(a.k), *gv = static_cast<const T *>(a.v);
     const T *table_qk = static_cast<const T *>(wave < 4 ? a.table_q : a.table_k);
@@ -122,7 +135,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                 }
                 if (!is_key) {
                     lds_store_u32(col_max + c * 4, 0x80000000u);
-                    lds_store_u32(col_sum + c * 4, 0u);
+                    lds_store2(col_sum + c * 8, 0.0f, 0.0f);
                 }
             }
             lds_barrier();
@@ -228,7 +241,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     packed[axis][1] = opaque(packed[axis][1]);
                 }
             }
-            // softmax of the tile: maxima per query, weights in fixed point.  Only the last step of a thread can lie
+            // softmax of the tile: maxima per query, weights and their sum.  Only the last step of a thread can lie
             // past the window's keys.
             const int my_steps = active ? (per_query - first + reach - 1) / reach : 0;
             {
@@ -240,33 +253,43 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             lds_barrier();
             lds_zero<kCols * kStride>(sums, tid);
             const float top = order_float(static_cast<int>(lds_load_u32(col_max + own * 4)));
-            uint32_t weight[kSteps];
-            uint32_t sum = 0;
+            float p[kSteps], sum = 0.0f;
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
-                weight[s] = s < my_steps ? static_cast<uint32_t>(__expf(logit[s] - top) * kFix + 0.5f) : 0u;
-                sum += weight[s];
+                p[s] = s < my_steps ? __expf(logit[s] - top) : 0.0f;
+                sum += p[s];
             }
-            if (active) lds_add(col_sum + own * 4, sum);
+            if (active) {
+                const float fixed = sum * kSumFix, whole = floorf(fixed);
+                lds_add64(col_sum + own * 8, static_cast<uint32_t>((fixed - whole) / kSumLow), static_cast<int>(whole));
+            }
             lds_barrier();
+            uint32_t weight[kSteps];
+            {
+                const float scale = power2(kCellBits - exponent_of(sum_of(own)));
 #pragma unroll
-            for (int s = 0; s < kSteps; ++s)
-                if (s < my_steps) lds_store_u32(sums + ((key0 + first + s * reach) * kStride + own) * 4, weight[s]);
-            f32x4_t tile_acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                for (int s = 0; s < kSteps; ++s) {
+                    weight[s] = static_cast<uint32_t>(rintf(p[s] * scale));
+                    if (s < my_steps) lds_store(sums + ((key0 + first + s * reach) * kStride + own) * 4, p[s]);
+                }
+            }
+            f32x4_t tile_acc = {0.0f, 0.0f, 0.0f, 0.0f}, tile_small = {0.0f, 0.0f, 0.0f, 0.0f};
             const uint32_t cell_at = ((out_half * 32 + 2 * group16) * kStride + out_tile * 16 + n16) * 4;
+            const float l_tile = sum_of(out_tile * 16 + n16);
+            const int exponent = exponent_of(l_tile) - kLift<T>;
             auto read_out = [&](uint32_t cells, uint32_t operand, bool table) {
                 if (out_tile * 16 >= cols) return;
                 float v[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    v[e] = static_cast<float>(lds_load_u32(cells + cell_at + ((e & 1) + 8 * (e >> 1)) * kStride * 4));
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t at = cells + cell_at + ((e & 1) + 8 * (e >> 1)) * kStride * 4;
+                    v[e] = table ? static_cast<float>(lds_load_u32(at)) : lds_load(at);
+                }
                 Cells<T> b;
-                // the weights of the values keep 21 bits; those of the table rows are rounded to the tables' type (what
-                // the sum of a pair's rows in that type costs elsewhere)
-                if (table) b.set_single(v, kCellScale); else b.set(v, kCellScale);
+                b.set(v, table ? kCellScale<T> : power2(-exponent));
                 Operand<T> t;
                 t.load_lds(operand + (n16 * kStride + out_half * 32 + group16 * 8) * sizeof(T));
-                tile_acc = table ? mfma16_single(t, b, tile_acc) : mfma16(t, b, tile_acc);
+                mfma16(t, b, tile_acc, tile_small);
             };
             lds_barrier();
             read_out(sums, value_t, false);
@@ -294,11 +317,10 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             // into the query's running softmax state
             const int i = out_tile * 16 + n16;
             const float m_tile = order_float(static_cast<int>(lds_load_u32(col_max + i * 4)));
-            const float l_tile = static_cast<float>(lds_load_u32(col_sum + i * 4)) * (1.0f / kFix);
             const float m_all = fmaxf(run_max, m_tile);
-            const float w_run = __expf(run_max - m_all), w_tile = __expf(m_tile - m_all);
+            const float w_run = __expf(run_max - m_all), w_tile = __expf(m_tile - m_all), w_acc = w_tile * power2(exponent);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = acc[e] * w_run + tile_acc[e] * w_tile;
+            for (int e = 0; e < 4; ++e) acc[e] = acc[e] * w_run + (tile_acc[e] + tile_small[e]) * w_acc;
             run_sum = run_sum * w_run + l_tile * w_tile;
             run_max = m_all;
         }
@@ -311,7 +333,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
         const int i = out_tile * 16 + n16;
         if (out_half == 0 && i < cols) {
             const f32x4_t other = *(__attribute__((address_space(3))) f32x4_t *)(meet);
-            const float inv = kOutScale / run_sum;
+            const float inv = 1.0f / run_sum;
             const int64_t row = static_cast<int>(lds_load_u32(row_i + i * 4));
             float o[4];
 #pragma unroll

@@ -43,6 +43,36 @@ def test_forward_stages_and_row_limits(oracle_lib, hip_lib, dtype, ws, cRSE, hea
     assert np.array_equal(run_attention(case, dtype, device_sizes=True), plain)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("ws,fill", [(5, 0.75), (7, 0.75)])     # a tile a window, and several
+def test_forward_weights_keep_their_bits(oracle_lib, hip_lib, dtype, ws, fill):
+    from gpu_helpers import run_attention
+    case = _case(oracle_lib, ws, "XYZ", 2, dtype, fill)
+    # the rows of two axes cancel: what is left of 1000 is the rounding of the weights and of their sums in fp32.  Weights
+    # of 23 bits leave 2^-24 of the 2000 that the terms' sizes add up to, and the (at most 128) terms of a sum 2^-24 each of
+    # partial sums below 1000, of random sign: sqrt(128) of them at one standard deviation
+    case.v[:], case.tq[:], case.tk[:] = 0, 0, 0
+    for rows, value in zip(case.axis_tables(case.tv), (1000, -1000, 0)):
+        rows[:] = value
+    got = run_attention(case, dtype)
+    assert np.abs(got).max() <= 1000 * 2.0 ** -24 * (2 + 4 * 128 ** 0.5)
+    # a key of each window with a weight of e^-19 beside its value alone
+    case.tv[:], case.q[:], case.k[:] = 0, 0, 0
+    case.q[:, :, 0] = 1
+    light = case.index["n2n"][case.index["w2n"]]
+    case.k[light, :, 0], case.v[light] = -19, 30000
+    got = run_attention(case, dtype)
+    others = np.empty(case.N)
+    others[case.index["n2n"]] = np.repeat(case.index["w_sizes"], case.index["w_sizes"]) - 1
+    want = np.exp(-19.0) * 30000 / (others + np.exp(-19.0))
+    want[light] = 30000 * np.exp(-19.0) / (others[light] + np.exp(-19.0))
+    # fp32: 27 units of 2^-24 in the exponent (of 2) of a logit of -19, twice, and the softmax's roundings; fp16: half a unit
+    # of its smallest numbers, and a weight's unit of 2^-40 of the sum beside 30000
+    bound = 4e-6 * want if dtype == torch.float32 else 2.0 ** -25 + 30000 * 2.0 ** -40 + 1e-5 * want
+    some = others > 0
+    assert (np.abs(got - want[:, None, None]) <= bound[:, None, None])[some].all()
+
+
 def _backward(case, dtype, tables, dout, spare=0, part=1):
     import swin3d_amd
     dev = torch.device("cuda")
