@@ -249,10 +249,15 @@ __device__ __forceinline__ void lds_add(uint32_t addr, uint32_t v)
 {
     __hip_atomic_fetch_add((lds_u32 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void lds_or(uint32_t addr, uint32_t v)
+{
+    __hip_atomic_fetch_or((lds_u32 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 __device__ __forceinline__ void lds_max(uint32_t addr, int v)
 {
     __hip_atomic_fetch_max((lds_i32 *)(addr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
 // exponent e with |x| < 2^e, and 2^e
 __device__ __forceinline__ int exponent_of(float x)
 {

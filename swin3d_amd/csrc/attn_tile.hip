@@ -36,9 +36,78 @@ template <typename T, int ND> struct FwdLayout {
     static constexpr uint32_t kTableT = kSt * D * kStride * sizeof(T);           // value table, [stage][channel][row]
     static constexpr uint32_t kValueT = D * kStride * sizeof(T);                 // values of the tile, [channel][key]
     static constexpr uint32_t kCoords = ND * kCols * 4;
-    static constexpr uint32_t kMeta = 5 * kCols * 4;                             // sums (64 bits), rows of queries and keys, maxima
+    static constexpr uint32_t kMeta = 5 * kCols * 4 + 48;                        // sums (64 bits), rows of queries and keys, maxima, masks
     static constexpr uint32_t kBytes = kSums + kKeys + kTableT + kValueT + kCoords + kMeta;
 };
+
+// A NaN or an infinity stays in its window, as on the sweep, though a matrix product takes the keys of a whole unit and all
+// rows of a table, zero weights among them: a value or a value table's entry that is not finite goes into its operand as
+// zero, and the queries that it belongs to - those of its window, all of the head - are marked, as is a query with a logit
+// that is not finite.  A marked query's result is stored as NaN, and a workgroup that has marked any goes through its units
+// once more and does over, pair by pair, what is NaN.  (Done over inside the loop over units, it took the tiles 3 us of 45,
+// in registers.)
+template <typename T, int ND, typename Rows, typename First>
+__device__ __forceinline__ void exact_query(const AttnArgs &a, int h, int64_t row, int pos0, int n_w, int sub, const float *own, Rows rows_n, First first_row)
+{
+    // eight neighbouring lanes a query, which take every eighth key
+    const int HD = a.H * D;
+    const T *gq = static_cast<const T *>(a.q) + h * D, *gk = static_cast<const T *>(a.k) + h * D, *gv = static_cast<const T *>(a.v) + h * D;
+    const T *table_q = static_cast<const T *>(a.table_q) + h * D, *table_k = static_cast<const T *>(a.table_k) + h * D;
+    const T *table_v = static_cast<const T *>(a.table_v) + h * D;
+    float q[D], acc[D], m = -INFINITY, l = 0.0f;
+    load_row<D>(gq + row * a.row_stride, q);
+#pragma unroll
+    for (int c = 0; c < D; ++c) acc[c] = 0.0f;
+    for (int j = sub; j < n_w; j += 8) {
+        const int pos = pos0 + j;
+        const int64_t key = a.n2n ? a.n2n[pos] : pos;
+        float k[D], x[D], logit = 0.0f;
+        int at[ND];
+        load_row<D>(gk + key * a.row_stride, k);
+#pragma unroll
+        for (int c = 0; c < D; ++c) logit = fmaf(q[c], k[c], logit);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+            const float cj = a.n_coords[static_cast<int64_t>(pos) * ND + n];
+            at[n] = (first_row(n) + crse_row(own[n], cj, static_cast<float>(rows_n(n) / 2), crse_upper(rows_n(n)))) * HD;
+            float part = 0.0f;
+            load_row<D>(table_q + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) part = fmaf(q[c], x[c], part);
+            load_row<D>(table_k + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) part = fmaf(k[c], x[c], part);
+            logit += part;
+        }
+        const float top = fmaxf(m, logit);
+        const float scale = m == -INFINITY ? 0.0f : __expf(m - top), p = logit == -INFINITY ? 0.0f : __expf(logit - top);
+        m = top;
+        l = fmaf(l, scale, p);
+        load_row<D>(gv + key * a.row_stride, x);
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c] * scale);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+            load_row<D>(table_v + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c]);
+        }
+    }
+#pragma unroll
+    for (int other = 1; other < 8; other <<= 1) {
+        const float m_o = __shfl_xor(m, other), l_o = __shfl_xor(l, other), top = fmaxf(m, m_o);
+        const float w = m == -INFINITY ? 0.0f : __expf(m - top), w_o = m_o == -INFINITY ? 0.0f : __expf(m_o - top);
+        l = l * w + l_o * w_o;
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = acc[c] * w + __shfl_xor(acc[c], other) * w_o;
+        m = top;
+    }
+    if (sub > 0) return;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int c = 0; c < D; ++c) acc[c] *= inv;
+    store_row<D>(static_cast<T *>(a.out) + row * HD + h * D, acc);
+}
 
 template <typename T, int ND, bool kDeviceSizes>
 __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
@@ -73,6 +142,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
     const uint32_t sums = base, keys = sums + L::kSums, table_t = keys + L::kKeys, value_t = table_t + L::kTableT;
     const uint32_t coords = value_t + L::kValueT, col_sum = coords + L::kCoords, row_i = col_sum + kCols * 8;
     const uint32_t row_j = row_i + kCols * 4, col_max = row_j + kCols * 4;
+    const uint32_t marked = col_max + kCols * 4, bad_keys = marked + 8, bad_head = marked + 16;   // 64 bits, 64 bits, 8 words
     auto sum_of = [&](int c) {
         return fmaf(static_cast<float>(lds_load_u32(col_sum + c * 8)), kSumLow / kSumFix,
                     static_cast<float>(lds_load_u32(col_sum + c * 8 + 4)) * (1.0f / kSumFix));
@@ -82,6 +152,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
     const T *table_qk = static_cast<const T *>(wave < 4 ? a.table_q : a.table_k);
     {
         // the head's value table with the channels as rows, unused rows at zero
+        bool bad_table = false;
         const T *tv = static_cast<const T *>(a.table_v);
         for (int x = tid; x < L::kSt * kCols * (D / 8); x += kThreads) {
             const int c8 = x % (D / 8), row = (x / (D / 8)) % kCols, st = x / (D / 8) / kCols;
@@ -98,13 +169,20 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             T *to = reinterpret_cast<T *>(reinterpret_cast<char *>(smem) + (table_t - base)) +
                     (st * D + c8 * 8) * kStride + (row & 32) + permuted_row(row & 31);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) to[e * kStride] = static_cast<T>(v[e]);
+            for (int e = 0; e < 8; ++e) {
+                bad_table = bad_table || !finite(v[e]);
+                to[e * kStride] = static_cast<T>(finite(v[e]) ? v[e] : 0.0f);
+            }
         }
+        // (a word per wavefront, cleared by its first lane: as a value of the thread it would sit in registers throughout)
+        if ((tid & 63) == 0) lds_store_u32(bad_head + wave * 4, 0u);
+        if (bad_table) lds_store_u32(bad_head + wave * 4, 1u);
     }
 
     const int tile_c = wave & 1, tile_r = (wave >> 1) & 1;
     const uint32_t row_stride = static_cast<uint32_t>(a.row_stride);
     const int out_tile = wave & 3, out_half = wave >> 2;  // 16 queries, 32 of a stage's rows
+    bool again = false;
 
     for (int u = group; u < total_units; u += groups) {
         const Unit unit(f.list.units[u]);
@@ -120,6 +198,14 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             const int keys_n = unit.keys(block);
             if (keys_n <= 0) break;
             lds_barrier();
+            if (tid < 4 && (tid >= 2 || block == 0)) {
+                uint32_t all = 0;
+                if (tid < 2) {
+#pragma unroll
+                    for (int w = 0; w < kWaves; ++w) all |= lds_load_u32(bad_head + w * 4);
+                }
+                lds_store_u32(marked + tid * 4, all ? 0xffffffffu : 0u);
+            }
             // the tile's voxels: threads 0..63 the queries, 64..127 the keys
             if (tid < 2 * kCols) {
                 const bool is_key = tid >= kCols;
@@ -168,8 +254,13 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     load_row<8>(gv + static_cast<uint64_t>(lds_load_u32(row_j + lane * 4)) * row_stride + h * D + c8 * 8, v);
                 T *to = reinterpret_cast<T *>(reinterpret_cast<char *>(smem) + (value_t - base)) + c8 * 8 * kStride +
                         (lane & 32) + permuted_row(lane & 31);
+                bool bad = false;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) to[e * kStride] = static_cast<T>(v[e]);
+                for (int e = 0; e < 8; ++e) {
+                    bad = bad || !finite(v[e]);
+                    to[e * kStride] = static_cast<T>(finite(v[e]) ? v[e] : 0.0f);
+                }
+                if (bad) lds_or(bad_keys + (lane >> 5) * 4, 1u << (lane & 31));
             }
             lds_barrier();
             // this thread's pairs: query `own`, keys key0 + first + s * reach
@@ -240,6 +331,15 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     packed[axis][0] = opaque(packed[axis][0]);
                     packed[axis][1] = opaque(packed[axis][1]);
                 }
+            }
+            {
+                bool bad = false;
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) bad = bad || !finite(logit[s]);
+                // the values of the query's keys: bits key0 .. key0 + per_query - 1
+                const uint64_t of_tile = static_cast<uint64_t>(lds_load_u32(bad_keys + 4)) << 32 | lds_load_u32(bad_keys);
+                bad = bad || (of_tile >> key0) << (kCols - per_query) != 0;
+                if (bad) lds_or(marked + (own >> 5) * 4, 1u << (own & 31));
             }
             // softmax of the tile: maxima per query, weights and their sum.  Only the last step of a thread can lie
             // past the window's keys.
@@ -331,15 +431,32 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
         if (out_half == 1) *(__attribute__((address_space(3))) f32x4_t *)(meet) = acc;
         lds_barrier();
         const int i = out_tile * 16 + n16;
+        again = again || (lds_load_u32(marked + 4) | lds_load_u32(marked)) != 0;
         if (out_half == 0 && i < cols) {
+            const bool mark = (lds_load_u32(marked + (i >> 5) * 4) >> (i & 31) & 1) != 0;
             const f32x4_t other = *(__attribute__((address_space(3))) f32x4_t *)(meet);
             const float inv = 1.0f / run_sum;
             const int64_t row = static_cast<int>(lds_load_u32(row_i + i * 4));
             float o[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (acc[e] + other[e]) * inv;
+            for (int e = 0; e < 4; ++e) o[e] = mark ? __int_as_float(0x7fc00000) : (acc[e] + other[e]) * inv;
             store4(static_cast<T *>(a.out) + row * HD + h * D + group16 * 4, o);
         }
+    }
+    if (!again) return;
+    __syncthreads();      // the workgroup's stores
+    for (int u = group; u < total_units; u += groups) {
+        const Unit unit(f.list.units[u]);
+        const int i = tid >> 3;
+        if (i >= unit.cols) continue;
+        const int first = unit.entry_of(f.list, i).x, pos = first + unit.inside(unit.tile, i);
+        const int64_t row = a.n2n ? a.n2n[pos] : pos;
+        const float out = to_float(static_cast<const volatile T *>(a.out)[row * HD + h * D]);
+        if (out == out) continue;
+        float ci[ND];
+#pragma unroll
+        for (int n = 0; n < ND; ++n) ci[n] = a.n_coords[static_cast<int64_t>(pos) * ND + n];
+        exact_query<T, ND>(a, h, row, first, unit.n_w, tid & 7, ci, rows_n, first_row);
     }
 }
 

@@ -73,6 +73,72 @@ def test_forward_weights_keep_their_bits(oracle_lib, hip_lib, dtype, ws, fill):
     assert (np.abs(got - want[:, None, None]) <= bound[:, None, None])[some].all()
 
 
+def _windows_case(oracle_lib, sizes, cRSE, heads, seed, ws=7):
+    """Windows of the given numbers of voxels, in rows of a random order."""
+    from conftest import random_scene
+    from helpers import AttnCase, n_coords_from_scene
+    from swin3d_amd import crse, synth
+    rng = np.random.default_rng(seed)
+    cells = np.stack(np.meshgrid(*[np.arange(ws)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    coords = np.concatenate([np.concatenate([np.zeros((n, 1), np.int64), cells[rng.permutation(ws ** 3)[:n]] + [w * ws, 0, 0]], 1)
+                             for w, n in enumerate(sizes)]).astype(np.int32)
+    coords = coords[rng.permutation(coords.shape[0])]
+    n = coords.shape[0]
+    frac = rng.random((n, 3)).astype(np.float32)
+    sig = rng.uniform(-1, 1, (n, crse.crse_num_axes(cRSE) - 3)).astype(np.float32)
+    index, n_coords = n_coords_from_scene(oracle_lib, coords, frac, sig, 1, ws, 4, cRSE)
+    assert sorted(index["w_sizes"]) == sorted(sizes)
+    table_sizes = crse.crse_table_sizes(ws, 4, heads, 16, cRSE)
+    q, k, v, tables = synth.layer_inputs(n, heads * 16, heads, int(sum(table_sizes)), seed=seed, recipe="sharp")
+    return AttnCase(coords, 1, ws, 4, heads, 16, cRSE, index, n_coords, q, k, 0.4 * v, (0.3 * tables[0], 0.3 * tables[1], 0.2 * tables[2]),
+                    table_sizes)
+
+
+def _kinds(x):
+    """0 finite, 1 and -1 infinite, 2 not a number"""
+    return np.where(np.isnan(x), 2, np.where(np.isinf(x), np.sign(x), 0))
+
+
+# units of several windows of 20, 16 and 9 voxels, windows of a tile and of several; as many voxels in larger windows that
+# the mean is 40
+SIZES = [20] * 5 + [16] * 4 + [9] * 8 + [64, 65, 120, 150, 150, 150, 200, 200]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("cRSE", ["XYZ", "XYZ_RGB_NORM"])
+@pytest.mark.parametrize("where,value", [("q", np.nan), ("k", np.nan), ("k", np.inf), ("k masked", -np.inf), ("v", np.nan),
+                                         ("v", np.inf), ("v", -np.inf), ("tq", np.inf), ("tk", np.nan), ("tv", np.inf), ("tv", np.nan)])
+def test_forward_keeps_what_is_not_finite_in_its_window(oracle_lib, hip_lib, dtype, cRSE, where, value):
+    """The same elements as in the oracle are NaN, plus and minus infinity and finite, and windows without such a voxel have
+    the bits of a call without it."""
+    from gpu_helpers import assert_attn_close, run_attention
+    case = _windows_case(oracle_lib, SIZES, cRSE, 2, seed=9)
+    if dtype == torch.float16:
+        to_half_and_back(case)
+    case.tk[:] = np.abs(case.tk)
+    clean = run_attention(case, dtype)
+    w_sizes, w2n, n2n = (case.index[x] for x in ("w_sizes", "w2n", "n2n"))
+    touched = np.zeros(case.N, bool)
+    for size in (9, 20, 64, 200):
+        w = int(np.flatnonzero(w_sizes == size)[0])
+        rows = n2n[w2n[w]:w2n[w] + size]
+        touched[rows] = True
+        if where[0] in "qkv":
+            getattr(case, where[0])[rows[-1], 1, 3] = value
+        if where == "k masked":
+            case.q[rows, 1, 3] = np.abs(case.q[rows, 1, 3]) + 0.1
+    if where[0] == "t":
+        case.axis_tables(getattr(case, where))[1][5, 1, 3] = value
+        touched[:] = True
+    got, ref = run_attention(case, dtype), oracle_lib.attn_fwd(*case.oracle_args())
+    assert np.array_equal(got[~touched], clean[~touched])
+    assert np.array_equal(run_attention(case, dtype, device_sizes=True), got, equal_nan=True)
+    assert not np.isfinite(got).all() or where == "k masked"
+    assert np.array_equal(_kinds(got), _kinds(ref))
+    same = np.isfinite(ref)
+    assert_attn_close(np.where(same, got, 0), np.where(same, ref, 0), dtype)
+
+
 def _backward(case, dtype, tables, dout, spare=0, part=1):
     import swin3d_amd
     dev = torch.device("cuda")
