@@ -325,12 +325,16 @@ template <typename Fn> __device__ __forceinline__ void for_steps(int steps, Fn f
 // ---- matrix operands --------------------------------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Eight values of an operand.  fp16 as they are; fp32 as a sum of three bf16 numbers, which hold its 24 bits exactly:
-// the six largest of the nine partial products keep a product to 2^-24 of itself, what fp32 arithmetic rounds to, at
-// a third of the time of fp32 matrix instructions.
+// Eight values of an operand.  fp16 as they are; fp32 as a sum of three bf16 numbers, which hold its 24 bits exactly: of the
+// nine partial products the six largest are taken, at a third of the time of fp32 matrix instructions.  What is left out of
+// a product is 2^-25 of it, half of what fp32 arithmetic rounds to, and of either sign as long as one of its operands is
+// split into the nearest numbers (split); the other may be cut off (cut, cheaper by a sixth), but with both cut off what is
+// left out has the product's sign, and the backward's errors against 64 bits are a third larger.
 template <typename T> struct Operand;
 template <> struct Operand<__half> {
     f16x8 x;
@@ -355,9 +359,24 @@ template <> struct Operand<float> {
     __device__ __forceinline__ void set(const Raw &r)
     {
         const float v[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
-        split(v);
+        cut(v);
     }
     __device__ __forceinline__ void split(const float *v)
+    {
+        u32x4 out[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f32x2 x = {v[2 * e], v[2 * e + 1]};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                out[k][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
+                if (k < 2) x -= f32x2{__uint_as_float(out[k][e] << 16), __uint_as_float(out[k][e] & 0xffff0000u)};
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(bf16x8, out[k]);
+    }
+    __device__ __forceinline__ void cut(const float *v)
     {
         u32x4 out[3];
 #pragma unroll
@@ -392,7 +411,7 @@ template <> struct Operand<float> {
             const f32x4_t q = *(lds_float4_t *)(addr + 4 * c);
             v[c] = q[0]; v[c + 1] = q[1]; v[c + 2] = q[2]; v[c + 3] = q[3];
         }
-        split(v);
+        cut(v);
     }
 };
 // a 32 x 32 result over 16 terms: A row lane % 32, B column lane % 32, terms 8 (lane / 32) + 0..7; the result's column
@@ -419,7 +438,7 @@ template <typename T> struct Cells;
 template <> struct Cells<__half> {
     f16x8 hi, lo;
     // v * scale as the sum of two fp16 numbers
-    __device__ __forceinline__ void set(const float *v, float scale)
+    template <bool kNearest = true> __device__ __forceinline__ void set(const float *v, float scale)
     {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -430,12 +449,12 @@ template <> struct Cells<__half> {
 };
 template <> struct Cells<float> {
     Operand<float> x;
-    __device__ __forceinline__ void set(const float *v, float scale)
+    template <bool kNearest = true> __device__ __forceinline__ void set(const float *v, float scale)
     {
         float y[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[e] = v[e] * scale;
-        x.split(y);
+        if constexpr (kNearest) x.split(y); else x.cut(y);
     }
 };
 __device__ __forceinline__ f32x4_t mfma16(const Operand<__half> &a, const Cells<__half> &b, f32x4_t c)
@@ -443,31 +462,19 @@ __device__ __forceinline__ f32x4_t mfma16(const Operand<__half> &a, const Cells<
     c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.x, b.lo, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.x, b.hi, c, 0, 0, 0);
 }
+// (the six partial products meet before they join the sum, which is then rounded once a product: the forward's error against
+// 64 bits on 3000 voxels of near-uniform weights is 1.0e-7 so, 2.4e-7 one after the other, 1.9e-7 in the sweep)
 __device__ __forceinline__ f32x4_t mfma16(const Operand<float> &a, const Cells<float> &b, f32x4_t c)
 {
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[2], b.x.s[0], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[1], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[2], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[0], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[1], c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[0], c, 0, 0, 0);
-}
-
-// ... into a sum over many products.  Beside fp32 operands the small partial products have a sum of their own, so that the
-// large one is rounded once a product and not six times: the forward's error against 64 bits on 3000 voxels of near-uniform
-// weights is 1.0e-7 so, 2.4e-7 in one sum, 1.9e-7 in the sweep.
-__device__ __forceinline__ void mfma16(const Operand<__half> &a, const Cells<__half> &b, f32x4_t &sum, f32x4_t &)
-{
-    sum = mfma16(a, b, sum);
-}
-__device__ __forceinline__ void mfma16(const Operand<float> &a, const Cells<float> &b, f32x4_t &sum, f32x4_t &small)
-{
-    small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[2], b.x.s[0], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[1], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[2], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[0], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[1], small, 0, 0, 0);
-    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[0], sum, 0, 0, 0);
+    f32x4_t p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[2], b.x.s[0], f32x4_t{}, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[1], p, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[2], p, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[1], b.x.s[0], p, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[1], p, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.s[0], b.x.s[0], p, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] += p[e];
+    return c;
 }
 
 // fp32 values beside fp16 ones: the sum of two fp16 numbers (23 bits) of the values times a power of two that brings the

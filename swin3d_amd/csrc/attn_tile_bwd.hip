@@ -7,7 +7,7 @@
 //    head): 8 bytes at [head][pairs before the window + j n + i].
 //  * tile_gradients_kernel: everything that is a sum over pairs.  Per axis the pairs' dL and P are added up by table row
 //    into histograms over the rows, one column per query (dL and P in one 64-bit cell) and one per key (dL): integers on
-//    a fixed-point image, scaled per query or key by its largest |dL|, so no order of additions shows in a result.  A
+//    a fixed-point image, scaled per query or key by its sum of |dL|, so no order of additions shows in a result.  A
 //    histogram H then gives, by matrix products,
 //        dT[row][c] += sum_columns H[row][column] x[column][c]   (x = q, dout, k: the three table gradients)
 //        dx[column][c] += sum_rows H[row][column] T[row][c]      (dq from Tq, dk from Tk)
@@ -31,9 +31,20 @@ namespace s3d {
 namespace tile {
 namespace {
 
-constexpr float kFixWeight = 33554432.0f;     // 2^25: P <= 1, at most 64 meet in a cell of 32 unsigned bits
-constexpr float kFixGrad = 16777216.0f;       // 2^24: |dL| <= 1 after scaling, at most 64 in a cell of 32 signed bits
-constexpr float kWeightCell = 1.0f / kFixWeight, kGradCell = 1.0f / kFixGrad;
+// dL and P in the gradients kernel.
+//  * Summed by table row they are integers in cells of 32 bits: P in units of 2^-29 (a query's weights sum to 1 but for
+//    rounding, also of fp16 tables in a forward whose backward has fp32 ones; there is room for 8), dL in units of 2^(e-30),
+//    2^e the least power above the sum of |dL| of its query (by key: of its key) in the tile.  A cell keeps what fp32 would,
+//    and no order of additions shows.
+//  * They enter the products over 2^-kLiftP and 2^(e-kLift), the cells and the pairs' own alike: beside fp16 operands as two
+//    fp16 numbers, 23 bits down to 2^-3 and units of 2^-24 below, that is 2^-36 of P and 2^-39 of the sum of |dL|.
+constexpr float kFixWeight = 536870912.0f;
+constexpr int kFixGrad = 30;
+template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // (fp32 features may be as large as fp32 is)
+template <typename TF> constexpr float kLiftP = sizeof(TF) == 2 ? 4096.0f : 1.0f;
+template <typename TF> constexpr float kWeightCell = kLiftP<TF> / kFixWeight;
+template <typename TF> constexpr float kGradCell = (sizeof(TF) == 2 ? 32768.0f : 1.0f) / 1073741824.0f;
+constexpr int kLiftFeature = 15;              // exponent of the tile's largest q or k in the table gradients
 
 // What the matrix products are made of: features (TF) as they are, and tables (T) in the same type, or fp32 tables beside
 // fp16 features as pairs of fp16 numbers.
@@ -299,7 +310,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
                         const uint32_t r = static_cast<uint32_t>(crse_row(ci, cj, half_rows, upper));
                         const float2 x = lds_load2(__umul24(r, kStride * 8) + own_at);
                         const float k = lds_load(r * 4 + key_at[s] + (kCoordWords + p * 32) * 4);
-                        logit[s] = fmaf(k, scale_k, fmaf(x.x, scale_q, logit[s]));
+                        logit[s] += fmaf(k, scale_k, x.x * scale_q);      // (the long sum is rounded once an axis)
                         dp[s] = fmaf(x.y, scale_v, dp[s]);
                     });
                 }
@@ -449,14 +460,14 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             // cells as an operand: a row's eight columns, a column's eight rows
             const uint32_t row_at = (quarter * 16 + n16) * kStride + term_at, column_at = 2 * group16 * kStride + column;
             const uint32_t channel_at = (n16 * kStride + term_at) * sizeof(TF);
-            f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};           // dk (wavefronts 0..3) or dq, over 2^exponent
+            f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};           // dk (wavefronts 0..3) or dq, over 2^(exponent - kLift)
             f32x4_t table_acc = {0.0f, 0.0f, 0.0f, 0.0f};     // ... the tables' part, over table_scale as well
             f32x4_t dv_acc = {0.0f, 0.0f, 0.0f, 0.0f};
             int exponent;
             {
-                // a column of dL per lane (the other lane groups hold its other terms), its exponent, and the products
+                // a column of dL per lane (the other lane groups hold its other terms), its sum's exponent, and the products
                 // dk_j += sum_i dL q_i, dv_j += sum_i P dout_i; dq_i += sum_j dL k_j
-                float v[2][8], top = 0.0f;
+                float v[2][8], all = 0.0f;
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) {
                     if (low) {
@@ -466,16 +477,16 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                         for (int e = 0; e < 8; ++e) v[ks][e] = lds_load(tile + (term_at * kStride + column) * 4 + (ks * 32 + e) * kStride * 4);
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[ks][e]));
+                    for (int e = 0; e < 8; ++e) all += fabsf(v[ks][e]);
                 }
-                top = fmaxf(top, __shfl_xor(top, 16));
-                top = fmaxf(top, __shfl_xor(top, 32));
-                exponent = exponent_of(top);
+                all += __shfl_xor(all, 16);
+                all += __shfl_xor(all, 32);
+                exponent = exponent_of(all);
                 if (group16 == 0) {
                     lds_store_u32((low ? exp_j : exp_i) + column * 4, exponent);
                     lds_max(exp_top + (low ? 4 : 0), exponent);
                 }
-                const float scale = power2(-exponent);
+                const float scale = power2(kLift<TF> - exponent);
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) {
                     Cells<TF> c;
@@ -486,7 +497,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                     if (low) {
                         float w[8];
                         lds_load8(cells + row_at * 4 + ks * 128, w);
-                        c.set(w, 1.0f);
+                        c.set(w, kLiftP<TF>);
                         x.load_lds(feat_d + channel_at + ks * 32 * sizeof(TF));
                         dv_acc = mfma16(x, c, dv_acc);
                     }
@@ -497,18 +508,18 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             uint32_t fix_p[kSteps];
             int fix_l[kSteps];
             {
-                const float scale = power2(-static_cast<int>(lds_load_u32(exp_i + own * 4))) * kFixGrad;
+                const int up = kFixGrad - static_cast<int>(lds_load_u32(exp_i + own * 4));
 #pragma unroll
                 for (int s = 0; s < kSteps; ++s) {
-                    fix_l[s] = static_cast<int>(rintf(grad[s] * scale));
-                    fix_p[s] = static_cast<uint32_t>(weight[s] * kFixWeight + 0.5f);
+                    fix_l[s] = static_cast<int>(rintf(ldexpf(grad[s], up)));
+                    fix_p[s] = static_cast<uint32_t>(rintf(weight[s] * kFixWeight));
                 }
             }
             const int top_i = static_cast<int>(lds_load_u32(exp_top)), top_j = static_cast<int>(lds_load_u32(exp_top + 4));
-            const int lift_q = 8 - static_cast<int>(lds_load_u32(exp_top + 8)), lift_k = 8 - static_cast<int>(lds_load_u32(exp_top + 12));
+            const int lift_q = kLiftFeature - static_cast<int>(lds_load_u32(exp_top + 8)), lift_k = kLiftFeature - static_cast<int>(lds_load_u32(exp_top + 12));
             {
                 // q and k over the tile's largest exponent of a query or key, for the table gradients; the largest value
-                // near 2^8, far from where fp16 numbers lose bits
+                // below 2^15, as far as can be from where fp16 numbers lose bits
                 TF *fq = reinterpret_cast<TF *>(reinterpret_cast<char *>(smem) + (feat_q - cells));
                 TF *fk = reinterpret_cast<TF *>(reinterpret_cast<char *>(smem) + (feat_k - cells));
                 const int c = tid & 63;
@@ -521,7 +532,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                     fk[at] = static_cast<TF>(static_cast<float>(fk[at]) * sj);
                 }
             }
-            const float grad_i = power2(top_i - lift_q), grad_j = power2(top_j - lift_k);
+            const float grad_i = power2(top_i - lift_q - kLift<TF>), grad_j = power2(top_j - lift_k - kLift<TF>);
             const int steps = (per_query + reach - 1) / reach;
             uint32_t other_at[kSteps];           // coordinates of the pairs' other side
 #pragma unroll
@@ -583,18 +594,19 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                             Operand<TF> x;
 #pragma unroll
                             for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(l[e]);
-                            c.set(v, kGradCell);
+                            c.set(v, kGradCell<TF>);
                             x.load_lds(feat_q + channel_at + ks * 32 * sizeof(TF));
                             gq = mfma16(c, x, gq);
 #pragma unroll
                             for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(w[e]);
-                            c.set(v, kWeightCell);
+                            c.set(v, kWeightCell<TF>);
                             x.load_lds(feat_d + channel_at + ks * 32 * sizeof(TF));
                             gv = mfma16(c, x, gv);
                         }
                         slot_at[st * kStageSlot] = make_float4(fmaf(gq[0], grad_i, old_q.x), fmaf(gq[1], grad_i, old_q.y),
                                                                fmaf(gq[2], grad_i, old_q.z), fmaf(gq[3], grad_i, old_q.w));
-                        slot_at[2 * kKind / 4 + st * kStageSlot] = make_float4(old_v.x + gv[0], old_v.y + gv[1], old_v.z + gv[2], old_v.w + gv[3]);
+                        slot_at[2 * kKind / 4 + st * kStageSlot] = make_float4(fmaf(gv[0], 1.0f / kLiftP<TF>, old_v.x), fmaf(gv[1], 1.0f / kLiftP<TF>, old_v.y),
+                                                                             fmaf(gv[2], 1.0f / kLiftP<TF>, old_v.z), fmaf(gv[3], 1.0f / kLiftP<TF>, old_v.w));
                     }
                 } else if (quarter * 16 < cols) {
 #pragma unroll
@@ -605,7 +617,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                         for (int e = 0; e < 8; ++e)
                             v[e] = static_cast<float>(static_cast<int>(lds_load_u32(cells + column_at * 8 + (ks * 32 + (e & 1) + 8 * (e >> 1)) * kStride * 8 + 4)));
                         Cells<TF> c;
-                        c.set(v, kGradCell);
+                        c.template set<false>(v, kGradCell<TF>);      // (the table's operand is the nearest)
                         table_acc = mfma16(x[ks], c, table_acc);
                     }
                 }
@@ -621,13 +633,13 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             const int query0 = small ? own_k / n_w * n_w : 0;
             const int steps_k = (per_key + reach_k - 1) / reach_k;
             {
-                const float scale = power2(-static_cast<int>(lds_load_u32(exp_j + own_k * 4))) * kFixGrad;
+                const int up = kFixGrad - static_cast<int>(lds_load_u32(exp_j + own_k * 4));
 #pragma unroll
                 for (int s = 0; s < kSteps; ++s) {
                     const int i = first_k + s * reach_k, at = query0 + min(i, per_key - 1);
                     const float x = lds_load(tile + (own_k * kStride + at) * 4);
                     other_at[s] = coords_i + at * 4;
-                    fix_l[s] = first_k < reach_k && i < per_key ? static_cast<int>(rintf(x * scale)) : 0;
+                    fix_l[s] = first_k < reach_k && i < per_key ? static_cast<int>(rintf(ldexpf(x, up))) : 0;
                 }
             }
             lds_zero<kCols * kStride>(cells, tid);
@@ -669,7 +681,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
 #pragma unroll
                             for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(__float_as_int(v[e]));
                             CellsA<TF> c;
-                            c.set(v, kGradCell);
+                            c.set(v, kGradCell<TF>);
                             Operand<TF> x;
                             x.load_lds(feat_k + channel_at + ks * 32 * sizeof(TF));
                             gk = mfma16(c, x, gk);
@@ -686,7 +698,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                         for (int e = 0; e < 8; ++e)
                             v[e] = static_cast<float>(static_cast<int>(lds_load_u32(here + column_at * 4 + (ks * 32 + (e & 1) + 8 * (e >> 1)) * kStride * 4)));
                         Cells<TF> c;
-                        c.set(v, kGradCell);
+                        c.template set<false>(v, kGradCell<TF>);      // (the table's operand is the nearest)
                         table_acc = mfma16(x[ks], c, table_acc);
                     }
                 }
@@ -697,7 +709,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             for (int st = 0; st < 3; ++st) by_key(st, std::false_type{});
 #pragma unroll 1
             for (int st = 3; st < S::kCount; ++st) by_key(st, std::true_type{});
-            const float back = power2(exponent);
+            const float back = power2(exponent - kLift<TF>);
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = fmaf(table_acc[e], table_scale, acc[e]);
             if (!low) {
@@ -705,7 +717,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                 for (int e = 0; e < 4; ++e) dq_sum[e] += acc[e] * back;
             } else if (column < keys_n) {
                 const float o[4] = {acc[0] * back, acc[1] * back, acc[2] * back, acc[3] * back};
-                const float w[4] = {dv_acc[0], dv_acc[1], dv_acc[2], dv_acc[3]};
+                const float w[4] = {dv_acc[0] / kLiftP<TF>, dv_acc[1] / kLiftP<TF>, dv_acc[2] / kLiftP<TF>, dv_acc[3] / kLiftP<TF>};
                 if (unit.tiles > 1) {
                     const int2 entry = b.list.entries[unit.entry];
                     if (window_fits(entry, n_w, b.pairs)) {

@@ -67,7 +67,7 @@ def test_forward_weights_keep_their_bits(oracle_lib, hip_lib, dtype, ws, fill):
     want = np.exp(-19.0) * 30000 / (others + np.exp(-19.0))
     want[light] = 30000 * np.exp(-19.0) / (others[light] + np.exp(-19.0))
     # fp32: 27 units of 2^-24 in the exponent (of 2) of a logit of -19, twice, and the softmax's roundings; fp16: half a unit
-    # of its smallest numbers, and a weight's unit of 2^-40 of the sum beside 30000
+    # of its smallest numbers, and half of a weight's unit of 2^-39 of the sum beside 30000
     bound = 4e-6 * want if dtype == torch.float32 else 2.0 ** -25 + 30000 * 2.0 ** -40 + 1e-5 * want
     some = others > 0
     assert (np.abs(got - want[:, None, None]) <= bound[:, None, None])[some].all()
@@ -182,3 +182,40 @@ def test_backward_stages_and_row_limits(oracle_lib, hip_lib, dtype, tables, ws, 
     for g, whole in zip(short[:3], got[:3]):
         bad = torch.isnan(g.float()).flatten(1).any(1)
         assert bool(bad.any()) and torch.equal(g[~bad], whole[~bad])
+
+
+@pytest.mark.parametrize("dtype,tables", [(torch.float32, torch.float32), (torch.float16, torch.float16), (torch.float16, torch.float32)])
+@pytest.mark.parametrize("ws,fill", [(7, 0.75), (5, 0.3)])       # several tiles a window; a tile
+def test_backward_weights_keep_their_bits(oracle_lib, hip_lib, dtype, tables, ws, fill):
+    """A key of each window with a weight of e^-14 / n beside every query."""
+    case = _case(oracle_lib, ws, "XYZ", 2, torch.float16, fill) if fill > 0.5 else \
+        to_half_and_back(make_attn_case(oracle_lib, seed=ws, n=int(fill * 1000), ws=ws, quant=4, heads=2, dim=16, cRSE="XYZ", extent=(5, 5, 3)))
+    for x in (case.q, case.k, case.tq, case.tk, case.tv):
+        x[:] = 0
+    light = case.index["n2n"][case.index["w2n"]]
+    case.q[:, :, 0], case.k[light, :, 0] = 1, -14
+    dout = (1000 * (1 + np.random.default_rng(ws).random(case.q.shape))).astype(np.float16).astype(np.float32)
+    ref = oracle_lib.attn_bwd(*case.oracle_args(), dout)
+    dv = _backward(case, dtype, tables, dout)[2].double().cpu().numpy()[light]
+    many = case.index["w_sizes"] > 1
+    # fp32: 20 units of 2^-24 in the exponent (of 2), twice, and the softmax's roundings.  fp16: half of its last place, and
+    # half of a weight's unit of 2^-36 beside every query's dout of at most 2000
+    bound = 4e-6 * ref[2][light] + (0 if dtype == torch.float32 else
+                                    2.0 ** -11 * ref[2][light] + 2000 * 2.0 ** -37 * case.index["w_sizes"][:, None, None])
+    assert (np.abs(dv - ref[2][light]) <= bound)[many].all()
+
+
+@pytest.mark.parametrize("dtype,tables", [(torch.float32, torch.float32), (torch.float16, torch.float16), (torch.float16, torch.float32)])
+def test_backward_sums_by_row_keep_their_bits(oracle_lib, hip_lib, dtype, tables):
+    """The value table's gradient under near-uniform weights: sums of either sign of weights times dout, whose error is the
+    weights' own.  Of a pair: an exponential to two units of 2^-24 (in its argument, and its result) and one each of the
+    logit's sum, the sum of the weights, its reciprocal and the product with it, of random sign; and the sums' own roundings,
+    which the terms' sizes bound.  (Weights in units of 2^-25 left 8e-7 of the result.)"""
+    case = _case(oracle_lib, 7, "XYZ_RGB_NORM", 4, torch.float16)
+    for x in (case.q, case.tq, case.tk):
+        x *= np.float32(2.0 ** -6)
+    to_half_and_back(case)
+    dout = np.random.default_rng(3).standard_normal(case.q.shape).astype(np.float16).astype(np.float32)
+    got = _backward(case, dtype, tables, dout)[5].double().cpu().numpy()
+    ref = np.asarray(oracle_lib.attn_bwd(*case.oracle_args(), dout)[5])
+    assert np.linalg.norm(got - ref) <= 6 * 2.0 ** -24 * np.linalg.norm(ref)
