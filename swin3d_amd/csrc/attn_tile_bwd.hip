@@ -32,16 +32,23 @@ namespace tile {
 namespace {
 
 // dL and P in the gradients kernel.
-//  * Summed by table row they are integers in cells of 32 bits: P in units of 2^-29 (a query's weights sum to 1 but for
-//    rounding, also of fp16 tables in a forward whose backward has fp32 ones; there is room for 8), dL in units of 2^(e-30),
+//  * Summed by table row they are integers in cells of 32 bits: P in units of 2^-28 (a query's weights sum to 1 but for
+//    rounding, also of fp16 tables in a forward whose backward has fp32 ones; there is room for 16), dL in units of 2^(e-30),
 //    2^e the least power above the sum of |dL| of its query (by key: of its key) in the tile.  A cell keeps what fp32 would,
 //    and no order of additions shows.
 //  * They enter the products over 2^-kLiftP and 2^(e-kLift), the cells and the pairs' own alike: beside fp16 operands as two
-//    fp16 numbers, 23 bits down to 2^-3 and units of 2^-24 below, that is 2^-36 of P and 2^-39 of the sum of |dL|.
-constexpr float kFixWeight = 536870912.0f;
+//    fp16 numbers, 23 bits down to 2^-3 and units of 2^-24 below, that is 2^-35 of P and 2^-39 of the sum of |dL|.
+//
+// What is not finite stays in its window, though the products take all columns of a unit and all rows of a table, zeros
+// among them: features and table entries that are not finite go into their operands as zeros.  Their pairs' dL is NaN (a
+// query's, for q and dout; a key's, for k), with dout their P as well, and so dq, dk and dv are what the sums over a
+// window's pairs would be, but for channels beside the one that is not finite.  In the integers such a pair counts for
+// nothing; the table rows it belongs to are marked and their gradients stored as NaN.  A P beyond 8 says that the
+// statistics are not the forward's, and is treated alike.
+constexpr float kFixWeight = 268435456.0f, kMostWeight = 8.0f;
 constexpr int kFixGrad = 30;
 template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // (fp32 features may be as large as fp32 is)
-template <typename TF> constexpr float kLiftP = sizeof(TF) == 2 ? 4096.0f : 1.0f;
+template <typename TF> constexpr float kLiftP = sizeof(TF) == 2 ? 2048.0f : 1.0f;
 template <typename TF> constexpr float kWeightCell = kLiftP<TF> / kFixWeight;
 template <typename TF> constexpr float kGradCell = (sizeof(TF) == 2 ? 32768.0f : 1.0f) / 1073741824.0f;
 constexpr int kLiftFeature = 15;              // exponent of the tile's largest q or k in the table gradients
@@ -118,7 +125,10 @@ __global__ __launch_bounds__(kListThreads) void tile_setup_kernel(BwdTileArgs b)
         if (threadIdx.x == 0) top_s = 0;
         __syncthreads();
         float top = 0.0f;
-        for (int t = threadIdx.x; t < a.total_rows * D; t += kListThreads) top = fmaxf(top, fabsf(table[static_cast<int64_t>(t / D) * HD + t % D]));
+        for (int t = threadIdx.x; t < a.total_rows * D; t += kListThreads) {
+            const float x = table[static_cast<int64_t>(t / D) * HD + t % D];
+            top = fmaxf(top, finite(x) ? fabsf(x) : 0.0f);
+        }
         atomicMax(&top_s, __float_as_int(top));
         __syncthreads();
         scale = power2(min(100, 14 - exponent_of(__int_as_float(top_s))));
@@ -137,6 +147,7 @@ __global__ __launch_bounds__(kListThreads) void tile_setup_kernel(BwdTileArgs b)
             const int r = kind < 3 ? row0 + lane % 32 : row0 + 2 * (lane / 16) + (e & 1) + 8 * (e >> 1);
             const int c = kind < 3 ? lane / 32 * 8 + e : lane % 16;
             v[e] = table[static_cast<int64_t>(first + min(r, rows - 1)) * HD + c];
+            if (kind >= 3 && !finite(to_float(v[e]))) v[e] = static_cast<T>(0.0f);
         }
     }
     Table x;
@@ -325,7 +336,8 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
             for (int s = 0; s < kSteps; ++s) {
                 if (s < my_steps) {
                     const float p = __expf(logit[s] - own_max) * own_inv;
-                    *to = make_float2(p * (dp[s] - own_delta), p);
+                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq)
+                    *to = make_float2(finite(logit[s]) ? p * (dp[s] - own_delta) : __int_as_float(0x7fc00000), p);
                 }
                 to += reach * n_w;
             }
@@ -343,8 +355,9 @@ template <typename TF, int ND> struct GradLayout {
     static constexpr uint32_t kTile = kCols * kStride * 4;                       // dL, [key][query]
     static constexpr uint32_t kFeature = D * kStride * sizeof(TF);               // q, dout, k: [channel][column]
     static constexpr uint32_t kCoords = ND * kCols * 4;
-    static constexpr uint32_t kMeta = 2 * kCols * 4 + 16;                        // exponents of queries and keys; maxima
-    static constexpr uint32_t kBytes = kCells + kTile + 3 * kFeature + 2 * kCoords + kMeta;
+    static constexpr uint32_t kMeta = 2 * kCols * 4 + 32;                        // exponents of queries and keys; maxima, a flag
+    static constexpr uint32_t kMarks = 6 * 8 + kSt * 16;                         // features and table rows that are not finite
+    static constexpr uint32_t kBytes = kCells + kTile + 3 * kFeature + 2 * kCoords + kMeta + kMarks;
 };
 
 template <typename T, typename TF, int ND>
@@ -365,6 +378,9 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
     const uint32_t cells = lds_base(smem), tile = cells + L::kCells, feats = tile + L::kTile;
     const uint32_t coords_i = feats + 3 * L::kFeature, coords_j = coords_i + L::kCoords;
     const uint32_t exp_i = coords_j + L::kCoords, exp_j = exp_i + kCols * 4, exp_top = exp_j + kCols * 4;
+    const uint32_t not_finite = exp_top + 16;                        // the tile has a pair that is not finite
+    const uint32_t bad_columns = exp_top + 32;                       // per wavefront that loads features: 64 bits
+    const uint32_t bad_rows = bad_columns + 6 * 8;                   // per stage: rows of such a dL, of such a P, 64 bits each
     const uint32_t feat_q = feats, feat_d = feats + L::kFeature, feat_k = feats + 2 * L::kFeature;
 
     const bool low = wave < 4;               // wavefronts 0..3 and 4..7 share the products differently
@@ -406,11 +422,16 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                     load_row<8>(from + static_cast<uint64_t>(static_cast<uint32_t>(rows[c])) * static_cast<uint32_t>(HD), v);
                     const bool there = static_cast<int>(c) < (which == 2 ? keys_n : cols);
                     TF *to = reinterpret_cast<TF *>(reinterpret_cast<char *>(smem) + (feats - cells) + which * L::kFeature) + c8 * 8 * kStride + c;
+                    bool bad = false;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        to[e * kStride] = static_cast<TF>(there ? v[e] : 0.0f);
-                        top = fmaxf(top, there ? fabsf(v[e]) : 0.0f);
+                        bad = bad || !finite(v[e]);
+                        const float x = there && finite(v[e]) ? v[e] : 0.0f;
+                        to[e * kStride] = static_cast<TF>(x);
+                        top = fmaxf(top, fabsf(x));
                     }
+                    const uint64_t columns = __ballot(bad && there);
+                    if (c < 2) lds_store_u32(bad_columns + wave * 8 + c * 4, static_cast<uint32_t>(columns >> (32 * c)));
                 } else {
                     const float *from = b.coords + static_cast<int64_t>(wave == 6 ? u : other) * (ND * kCols);
                     const uint32_t to = (wave == 6 ? coords_i : coords_j) + c * 4;
@@ -438,11 +459,28 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             }
             lds_zero<kCols * kStride>(tile, tid);
             lds_zero<kCols * kStride>(cells, tid);
-            if (tid < 4) lds_store_u32(exp_top + tid * 4, static_cast<uint32_t>(-100));
+            if (tid < 5) lds_store_u32(exp_top + tid * 4, tid < 4 ? static_cast<uint32_t>(-100) : 0u);
             lds_barrier();
             // tile and cells [key][query]; the largest exponent of a q or k
             if (wave < 6 && which != 1) lds_max(exp_top + (which == 0 ? 8 : 12), exponent_of(top));
             {
+                uint64_t bad[3];           // queries by q, by dout; keys
+#pragma unroll
+                for (int f = 0; f < 3; ++f) {
+                    const u32x4_t m = *(lds_u32x4 *)(bad_columns + f * 16);
+                    bad[f] = static_cast<uint64_t>(m[1] | m[3]) << 32 | (m[0] | m[2]);
+                }
+                bool any = false;
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) {
+                    if (s < my_steps) {
+                        const bool by_dout = (bad[1] >> own & 1) != 0 || !(weight[s] <= kMostWeight);
+                        if (by_dout || ((bad[0] >> own | bad[2] >> (key0 + first + s * reach)) & 1) != 0) grad[s] = __int_as_float(0x7fc00000);
+                        if (by_dout) weight[s] = __int_as_float(0x7fc00000);
+                        any = any || !finite(grad[s]);
+                    }
+                }
+                if (any) lds_store_u32(not_finite, 1u);
                 const uint32_t at = ((key0 + first) * kStride + own) * 4, step = reach * (kStride * 4);
 #pragma unroll
                 for (int s = 0; s < kSteps; ++s) {
@@ -477,7 +515,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                         for (int e = 0; e < 8; ++e) v[ks][e] = lds_load(tile + (term_at * kStride + column) * 4 + (ks * 32 + e) * kStride * 4);
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) all += fabsf(v[ks][e]);
+                    for (int e = 0; e < 8; ++e) all += finite(v[ks][e]) ? fabsf(v[ks][e]) : 0.0f;
                 }
                 all += __shfl_xor(all, 16);
                 all += __shfl_xor(all, 32);
@@ -537,6 +575,32 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
             uint32_t other_at[kSteps];           // coordinates of the pairs' other side
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) other_at[s] = coords_j + (key0 + min(first + s * reach, per_query - 1)) * 4;
+            const bool marks = __builtin_amdgcn_readfirstlane(lds_load_u32(not_finite)) != 0;
+            if (marks) {
+                if (tid < L::kSt * 4) lds_store_u32(bad_rows + tid * 4, 0u);
+                lds_barrier();
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) {
+                    if (s >= my_steps || finite(grad[s])) continue;
+#pragma unroll 1
+                    for (int axis = 0; axis < ND; ++axis) {
+                        const int rows = axis_rows<ND>(a, axis), st = axis < 3 ? axis : 3 + (axis - 3) / 2;
+                        const int r = crse_row(lds_load(coords_i + (axis * kCols + own) * 4), lds_load(other_at[s] + axis * kCols * 4),
+                                               static_cast<float>(rows / 2), crse_upper(rows));
+                        const uint32_t at = bad_rows + st * 16 + (axis < 3 ? r >> 5 : (axis - 3) & 1) * 4;
+                        lds_or(at, 1u << (r & 31));
+                        if (!finite(weight[s])) lds_or(at + 8, 1u << (r & 31));
+                    }
+                }
+                // (read behind the next barrier)
+            }
+            // four rows of a table gradient, marked ones as NaN
+            auto marked = [&](int st, int of_weight, float4 g) {
+                if (!marks) return g;
+                const uint32_t m = lds_load_u32(bad_rows + st * 16 + of_weight * 8 + (quarter >> 1) * 4) >> ((quarter & 1) * 16 + group16 * 4);
+                const float nan = __int_as_float(0x7fc00000);
+                return make_float4(m & 1 ? nan : g.x, m & 2 ? nan : g.y, m & 4 ? nan : g.z, m & 8 ? nan : g.w);
+            };
             // rows of half ks of stage st in use
             auto half_used = [&](int st, int ks) { return st < 3 ? ks * 32 < axis_rows<ND>(a, st) : S::first(st) + ks < ND; };
             // rows of this wavefront's quarter of stage st
@@ -603,10 +667,11 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                             x.load_lds(feat_d + channel_at + ks * 32 * sizeof(TF));
                             gv = mfma16(c, x, gv);
                         }
-                        slot_at[st * kStageSlot] = make_float4(fmaf(gq[0], grad_i, old_q.x), fmaf(gq[1], grad_i, old_q.y),
-                                                               fmaf(gq[2], grad_i, old_q.z), fmaf(gq[3], grad_i, old_q.w));
-                        slot_at[2 * kKind / 4 + st * kStageSlot] = make_float4(fmaf(gv[0], 1.0f / kLiftP<TF>, old_v.x), fmaf(gv[1], 1.0f / kLiftP<TF>, old_v.y),
-                                                                             fmaf(gv[2], 1.0f / kLiftP<TF>, old_v.z), fmaf(gv[3], 1.0f / kLiftP<TF>, old_v.w));
+                        slot_at[st * kStageSlot] = marked(st, 0, make_float4(fmaf(gq[0], grad_i, old_q.x), fmaf(gq[1], grad_i, old_q.y),
+                                                                             fmaf(gq[2], grad_i, old_q.z), fmaf(gq[3], grad_i, old_q.w)));
+                        constexpr float back = 1.0f / kLiftP<TF>;
+                        slot_at[2 * kKind / 4 + st * kStageSlot] = marked(st, 1, make_float4(fmaf(gv[0], back, old_v.x), fmaf(gv[1], back, old_v.y),
+                                                                                             fmaf(gv[2], back, old_v.z), fmaf(gv[3], back, old_v.w)));
                     }
                 } else if (quarter * 16 < cols) {
 #pragma unroll
@@ -686,8 +751,8 @@ __global__ __launch_bounds__(kThreads, 4) void tile_gradients_kernel(BwdTileArgs
                             x.load_lds(feat_k + channel_at + ks * 32 * sizeof(TF));
                             gk = mfma16(c, x, gk);
                         }
-                        slot_at[kKind / 4 + st * kStageSlot] = make_float4(fmaf(gk[0], grad_j, old_k.x), fmaf(gk[1], grad_j, old_k.y),
-                                                                           fmaf(gk[2], grad_j, old_k.z), fmaf(gk[3], grad_j, old_k.w));
+                        slot_at[kKind / 4 + st * kStageSlot] = marked(st, 0, make_float4(fmaf(gk[0], grad_j, old_k.x), fmaf(gk[1], grad_j, old_k.y),
+                                                                                         fmaf(gk[2], grad_j, old_k.z), fmaf(gk[3], grad_j, old_k.w)));
                     }
                 } else if (quarter * 16 < keys_n) {
 #pragma unroll
