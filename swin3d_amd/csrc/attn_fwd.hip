@@ -228,7 +228,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_plan(
     a.w2n = w2n;
     a.workspace = plan;
     // both lists where the shape may use either: the plan's caller may keep the table sizes on the device
-    if (D == 16 && attn_tile_shape(N, W, H, dtype == S3D_DTYPE_F32)) {
+    if (D == 16 && attn_tile_shape(N, W, H, nd, dtype == S3D_DTYPE_F32)) {
         if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
     }
     return launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream), kAttnBuildList);

@@ -59,7 +59,7 @@ int launch_attn_sweep(const AttnArgs &a, int dtype, hipStream_t stream, int what
 // products on the matrix pipe.  `list` is its unit list, attn_tile_list_bytes of device memory.
 // With sizes_dev the host cannot tell whether every axis fits: it launches the tile kernel and the sweep kernel, and each
 // works or returns by what it reads.
-bool attn_tile_shape(int64_t N, int64_t W, int H, bool fp32);
+bool attn_tile_shape(int64_t N, int64_t W, int H, int nd, bool fp32);
 bool attn_tile_applies(const AttnArgs &a, int dtype);
 size_t attn_tile_list_bytes(int H, int64_t N, int64_t W);
 int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);

@@ -491,29 +491,31 @@ int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, i
 }  // namespace tile
 
 // Where the tile kernel serves a forward (head_dim 16).  It leaves every tile's products, sums and histograms in LDS and
-// crosses some thirty barriers for them, which costs about what 64 x 64 pairs cost, so it needs windows of some size; on
-// these it spends 580 clocks of a CU on 64 pairs and a head where the sweep kernel spends 420 in fp16 and 690 in fp32.
-// But a window is spread over its queries' tiles and a tile's pairs over 512 threads, where the sweep gives a query at
-// most eight lanes: a launch that does not fill the chip ends when its longest unit ends, and that is a quarter as long.
-// Measured, sweep / tile kernel, by N^2 / W * H: fp16 76.7 / 44.7 us at 1.6 M, 108.6 / 87.2 at 3.5 M, 200 / 197 at 9.6 M,
-// 324 / 362 at 19 M; fp32 82 / 58 at 1.6 M, 330 / 282 at 9.6 M, 842 / 817 at 32 M, 1235 / 1254 at 46 M.
+// crosses some thirty barriers for them, which costs about what 64 x 64 pairs cost, so it needs windows of some size.  But a
+// window is spread over its queries' tiles and a tile's pairs over 512 threads, where the sweep gives a query at most eight
+// lanes: a launch that does not fill the chip ends when its longest unit ends, and that is a quarter as long.  Measured on
+// windows of 60 to 95 voxels, tile over sweep kernel, by N^2 / W * H:
+//   fp16, 9 axes: 0.55 at 2.0 M, 0.79 and 0.84 at 3.2 M, 1.01 to 1.12 at 4.1 to 5.5 M, 1.10 to 1.29 at 9 to 35 M
+//   fp16, 6 axes: 0.59 at 2.0 M, 0.84 and 0.87 at 3.2 M, 1.02 to 1.15 at 4.1 to 5.5 M, 1.16 to 1.41 beyond
+//   fp32, 9 axes: 0.67 at 2.0 M, 0.94 to 1.02 at 4 to 11 M (1.05 once), 0.93 and 1.01 at 16 M, 1.03 to 1.09 at 26 to 35 M
+//   fp32, 6 axes: 0.67 at 2.0 M, 0.86 to 0.94 at 4 to 26 M, 0.93 and 0.97 at 35 and 29 M
 constexpr int kTileMeanWindow = 40;
-constexpr double kTilePairsHalf = 8e6, kTilePairsFloat = 35e6;
+constexpr double kTilePairsHalf = 4e6, kTilePairsFloat = 35e6, kTilePairsFloatNormals = 12e6;
 
-bool attn_tile_shape(int64_t N, int64_t W, int H, bool fp32)
+bool attn_tile_shape(int64_t N, int64_t W, int H, int nd, bool fp32)
 {
-    return W > 0 && N >= kTileMeanWindow * W &&
-           static_cast<double>(N) * N / W * H <= (fp32 ? kTilePairsFloat : kTilePairsHalf);
+    const double most = !fp32 ? kTilePairsHalf : nd < 9 ? kTilePairsFloat : kTilePairsFloatNormals;
+    return W > 0 && N >= kTileMeanWindow * W && static_cast<double>(N) * N / W * H <= most;
 }
 
 size_t attn_tile_list_bytes(int H, int64_t N, int64_t W)
 {
-    return attn_tile_shape(N, W, H, true) ? tile::list_bytes(N, W) : 0;
+    return attn_tile_shape(N, W, H, 3, true) ? tile::list_bytes(N, W) : 0;      // (whatever type and axes the call has)
 }
 
 bool attn_tile_applies(const AttnArgs &a, int dtype)
 {
-    if (a.D != tile::D || !attn_tile_shape(a.N, a.W, a.H, dtype == S3D_DTYPE_F32)) return false;
+    if (a.D != tile::D || !attn_tile_shape(a.N, a.W, a.H, a.nd, dtype == S3D_DTYPE_F32)) return false;
     return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
 }
 
