@@ -1,4 +1,11 @@
-// Sparse-voxel windowed self-attention with cRSE tables (gfx950): the tile kernel of the forward.
+// Sparse-voxel windowed self-attention with cRSE tables (gfx950): the tile kernel of the forward, head_dim 16.
+//
+// A workgroup takes 64 queries by 64 keys of a head.  The products of its queries and keys with all rows of an axis table
+// come from the matrix pipe and stay in LDS, where a pair picks its two words instead of gathering two rows of 32 or 64
+// bytes; the value tables enter through histograms of the weights over their rows, one column per query.  811 voxels, 24
+// heads, fp16: 92 us (sweep) -> 47 us a call; 49,682 voxels, 6 heads, 6 axes, fp32: 413 -> 398.  No unit is busy (VALU 27 and
+// 53 % of the time, LDS addressed 25 and 33 %, matrix pipe 2 and 11 %): a tile goes through some thirty phases with a
+// barrier each, and a wavefront waits for half of its time.
 #include "attn_tile.h"
 
 namespace s3d {

@@ -19,10 +19,12 @@
 //
 // Why tiles: the pair sweeps this form replaces run at two wavefronts per SIMD (192 VGPRs) and wait for a gathered table
 // row of 64 bytes per pair, axis and table.  Here a pair's term is a word of LDS.  One form for every window size: a unit
-// packs windows of up to 64 voxels side by side.  Measured, 9 axes, windows of about 100 voxels, 6 heads, 36,000 voxels, fp32
-// tables beside fp16 features (forward and backward of a training step): 1853 us -> 939 us; of these the gradients
-// kernel 510, records 178, setup, columns and finish 34.  What bounds both large kernels is the LDS: per pair and axis
-// three reads (records) or two reads and two atomic additions (gradients).
+// packs windows of up to 64 voxels side by side.  Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables
+// beside fp16 features (forward and backward of a training step): 1860 us -> 947 us; of these the gradients kernel 540,
+// records 188, setup, columns and finish 35.  No unit is busy: in the gradients kernel the VALU issues 39 % of the time, the
+// LDS is addressed for 35 % (two fifths of it bank conflicts), the matrix pipe works for 4 %, and a wavefront waits for
+// 52 % of its time - for the barriers of some 25 phases a tile, at four wavefronts per SIMD, and for 2 GB that a call
+// moves, most of it the slots and registers that did not fit; in the records kernel 36, 31, 5 and 47 %.
 #include "attn_tile.h"
 
 #include <type_traits>
@@ -920,8 +922,8 @@ size_t operand_bytes(int H, int nd)
 
 // Every shape whose tables fit a stage: of windows of 1 to 300 voxels in sets of 300 to 60,000, with 3 and 9 axes and all
 // three types, the pair sweeps were faster in none (fp16: tiles take 0.14 to 0.53 of their time; fp32: 0.17 to 0.95, the
-// most at 4 to 20 voxels a window and three axes).  At head_dim 8, where the sweeps' rows are half as long and a pair's
-// cost on a tile is the same, the two meet at 20 voxels a window.
+// most at 4 to 20 voxels a window and three axes).  At head_dim 8 there is no tile form: half of the 16 terms of a product
+// would be empty while a pair's cost on a tile is the same, and the sweeps' rows are half as long.
 bool attn_tile_bwd_applies(const int32_t *rows, int nd, int D, int64_t pairs)
 {
     return D == 16 && pairs > 0 && pairs < (int64_t(1) << 31) && rows_fit_tiles(rows, nd);
