@@ -155,7 +155,8 @@ int s3d_attn_plan(const int32_t *table_sizes, int32_t nd, int64_t table_len, con
  * call: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  The work list lives
  * in a device array of 8 MiB that is part of the library's code object, one copy per GPU, held until the process
  * ends.  The call fails with S3D_ERR_WORKSPACE when s3d_attn_fwd_workspace_bytes(H, N, W) exceeds 8 MiB (about
- * 2 N + 24 W bytes + 0.3 MB: e.g. one million voxels in up to 200 000 windows fit).  No call allocates or frees.
+ * 2 N + 24 W bytes + 0.3 MB, and N / 2 + 8 W where a call may run on tiles: e.g. one million voxels in up to 200 000
+ * windows fit).  No call allocates or frees.
  * The first call on a device looks up the array's address there (hipGetSymbolAddress) and the first call of a
  * shape (dtype, head_dim, axes, heads per wavefront) raises that kernel's dynamic-LDS limit (hipFuncSetAttribute):
  * neither belongs into a stream capture, so make ONE eager call per device and shape before capturing; the calls
@@ -190,7 +191,9 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  *   pairs          M = sum of w_sizes^2, the pairs of the window set (counts[1] of s3d_window_index; the length
  *                  of the reference's index arrays), or 0.  With M the call runs two pair sweeps on the forward's
  *                  kind of work list (dq; dk and dv), which leave dL and P of every (pair, head) in the workspace
- *                  - 12 * H * pairs bytes -, and two table-gradient sweeps that read them.  With 0 it runs two fused
+ *                  - 12 * H * pairs bytes -, and two table-gradient sweeps that read them; at head_dim 16 with tables
+ *                  of at most 64 rows on a position axis and 32 on a signal axis it runs on tiles of 64 queries by 64
+ *                  keys instead, all six gradients from matrix products.  With 0 it runs two fused
  *                  sweeps that recompute the logits for the table gradients and need no such store (about a third
  *                  more time).  A value below M cannot hold the records of every window: the rows of dq, dk, dv
  *                  that belong to the windows beyond it and all three table gradients then come out as NaN.
@@ -212,6 +215,10 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  * left in a slot of the workspace and summed per head, slots in order, by a reduction kernel: which units a
  * wavefront draws varies from call to call, so these sums are regrouped and agree between calls to fp32 rounding
  * (about 1e-6 of the largest element), not bit for bit.
+ *
+ * On tiles, what is not finite in q, k, v, dout or a table makes NaN of the gradients that it belongs to as a sum over
+ * pairs - those of its window, and of the table rows of its pairs - and of no others, but for the other channels of a
+ * voxel or table row with such a dout; so does a statistic that is not the forward's, where it makes a weight above 8.
  */
 size_t s3d_attn_bwd_workspace_bytes(int32_t H, int32_t D, int32_t nd, int64_t table_len, int64_t N, int64_t W,
                                     int64_t pairs);

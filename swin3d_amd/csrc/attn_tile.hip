@@ -501,11 +501,12 @@ int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, i
 // crosses some thirty barriers for them, which costs about what 64 x 64 pairs cost, so it needs windows of some size.  But a
 // window is spread over its queries' tiles and a tile's pairs over 512 threads, where the sweep gives a query at most eight
 // lanes: a launch that does not fill the chip ends when its longest unit ends, and that is a quarter as long.  Measured on
-// windows of 60 to 95 voxels, tile over sweep kernel, by N^2 / W * H:
-//   fp16, 9 axes: 0.55 at 2.0 M, 0.79 and 0.84 at 3.2 M, 1.01 to 1.12 at 4.1 to 5.5 M, 1.10 to 1.29 at 9 to 35 M
-//   fp16, 6 axes: 0.59 at 2.0 M, 0.84 and 0.87 at 3.2 M, 1.02 to 1.15 at 4.1 to 5.5 M, 1.16 to 1.41 beyond
-//   fp32, 9 axes: 0.67 at 2.0 M, 0.94 to 1.02 at 4 to 11 M (1.05 once), 0.93 and 1.01 at 16 M, 1.03 to 1.09 at 26 to 35 M
-//   fp32, 6 axes: 0.67 at 2.0 M, 0.86 to 0.94 at 4 to 26 M, 0.93 and 0.97 at 35 and 29 M
+// windows of 55 to 110 voxels and 6 to 40 heads, tile over sweep kernel, by N^2 / W * H (what the sweep makes of a small
+// launch jumps with its cut into units, which is most of the spread):
+//   fp16, 9 axes: 0.55 to 0.83 at 2 M, 0.79 to 0.90 at 3 to 4 M, 0.92 to 1.12 at 4 to 6 M, 1.02 in the mean, 0.93 to 1.29 beyond
+//   fp16, 6 axes: 0.59 to 0.72 at 2 M, 0.84 to 0.96 at 3 to 4 M, 0.92 to 1.18 at 4 to 6 M, 1.03 in the mean, 1.03 to 1.41 beyond
+//   fp32, 9 axes: 0.67 at 2 M, 0.94 to 1.05 at 4 to 12 M, 0.99 in the mean, 0.91 to 1.09 beyond, 1.01 in the mean
+//   fp32, 6 axes: 0.67 at 2 M, 0.83 to 0.94 at 4 to 26 M, 0.93 and 0.97 at 35 and 29 M
 constexpr int kTileMeanWindow = 40;
 constexpr double kTilePairsHalf = 4e6, kTilePairsFloat = 35e6, kTilePairsFloatNormals = 12e6;
 

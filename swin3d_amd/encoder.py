@@ -1,7 +1,8 @@
 """Swin3D encoder on the swin3d_amd operators, without MinkowskiEngine (inference path).
 
-The sparse voxel set is a pair of tensors (`SparseVoxels`); dense math (Linear, GELU, the 27-offset stem
-convolution as one GEMM) goes to hipBLASLt through torch.  Window attention runs through
+The sparse voxel set is a pair of tensors (`SparseVoxels`).  Under fp16 autocast the dense layers of inference run on
+the library's kernels, those of a training pass forward through torch (hipBLASLt) and backward on the library's; the
+27-offset stem convolution is one GEMM of torch's.  Window attention runs through
 `SelfAttnAIOFunction`, the window index through `build_window_indices` / `window_signals`, neighbour
 gathering through `KNN` / `knn_max_pool`.  On the GPU the coordinate work runs on the library's kernels too
 (coarse cells and their representatives from the window sort, the stem's neighbour rows by binary search in
