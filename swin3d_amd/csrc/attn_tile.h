@@ -39,10 +39,14 @@ __host__ __device__ constexpr int permuted_row(int row) { return ((row % 8) / 2)
 // A unit is what a workgroup takes on at a time for one head: up to 64 queries of one window, or all voxels of the
 // several small windows of one size that fit 64 columns.  Windows of more than 64 voxels are cut into equal tiles.
 struct UnitList {
-    const int32_t *total;      // [0]: units
+    const int32_t *total;      // [0]: units, [1]: strips
     const int4 *units;         // (first entry, voxels per window, windows, 0) or (entry, voxels, tile, tiles)
     const int2 *entries;       // windows by size: first sorted position, pairs (n^2) of the windows before it
+    const int4 *strips;        // or null; (entry, voxels per window, first column, columns), see Strip
 };
+// A strip is up to 16 voxels of windows of one size: the voxels of its windows (of at most 64 voxels) in the order of the
+// entries, from column `first` of window `entry` on; of a larger window, 16 of its voxels.
+constexpr int kStrip = 16;
 // A unit, decoded: the tile's queries are `cols` voxels; with more than one tile the workgroup goes through the tiles
 // of the window's keys.
 struct Unit {
@@ -72,6 +76,9 @@ inline size_t list_bytes(int64_t N, int64_t W)
 {
     return 256 + list_round(sizeof(int4) * list_max_units(N)) + list_round(sizeof(int2) * static_cast<size_t>(W > 0 ? W : 1));
 }
+// a strip is full, but for the last one of each window size up to 64 and of each larger window
+inline size_t list_max_strips(int64_t N) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(N > 0 ? N : 0) / (kCols + 1) + kCols + 1; }
+inline size_t strips_bytes(int64_t N) { return list_round(sizeof(int4) * list_max_strips(N)); }
 inline UnitList list_at(void *p, int64_t N, int64_t W)
 {
     char *base = static_cast<char *>(p);
@@ -79,6 +86,7 @@ inline UnitList list_at(void *p, int64_t N, int64_t W)
     l.total = reinterpret_cast<const int32_t *>(base);
     l.units = reinterpret_cast<const int4 *>(base + 256);
     l.entries = reinterpret_cast<const int2 *>(base + 256 + list_round(sizeof(int4) * list_max_units(N)));
+    l.strips = nullptr;
     return l;
 }
 int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, int64_t W, hipStream_t stream);
@@ -87,49 +95,61 @@ constexpr int kListThreads = 1024;
 constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 32 and more tiles, then 64 .. 1 voxels
 
 __device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
+__device__ __forceinline__ int strips_of(int n) { return (n + kStrip - 1) / kStrip; }
 __device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
 
 // Unit list: windows in bins of equal size, largest first (a counting sort in LDS), and the pairs of the windows before
 // each.  Inside a bin the windows keep their order: where a window lies in its unit decides in which order the matrix pipe
 // adds its products, and a result is to be the same bits on every call.
 __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
-                                           int32_t *__restrict__ total, int4 *__restrict__ units, int2 *__restrict__ entries)
+                                           int32_t *__restrict__ total, int4 *__restrict__ units, int2 *__restrict__ entries,
+                                           int4 *__restrict__ strips)
 {
     __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
     constexpr int kWavesOfList = kListThreads / 64;
     __shared__ int wave_pairs[kWavesOfList], of_wave[kWavesOfList][kListBins];
+    __shared__ int big_strips[kListBins], strip_at[kListBins], strips_of_wave[kWavesOfList][kBigBins];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t < kListBins) windows[t] = big_units[t] = 0;
+    if (t < kListBins) windows[t] = big_units[t] = big_strips[t] = 0;
     __syncthreads();
     for (int w = t; w < W; w += kListThreads) {
         const int n = w_sizes[w];
         if (n <= 0) continue;
         const int b = list_bin(n);
         atomicAdd(&windows[b], 1);
-        if (n > kCols) atomicAdd(&big_units[b], tiles_of(n));
+        if (n > kCols) {
+            atomicAdd(&big_units[b], tiles_of(n));
+            atomicAdd(&big_strips[b], strips_of(n));
+        }
     }
     __syncthreads();
     if (wave == 0) {
-        // exclusive sums of windows and units over the bins, 64 at a time
-        int e_run = 0, u_run = 0;
+        // exclusive sums of windows, units and strips over the bins, 64 at a time
+        int e_run = 0, u_run = 0, s_run = 0;
         for (int b0 = 0; b0 < kListBins; b0 += 64) {
             const int b = b0 + lane;
             const int count = b < kListBins ? windows[b] : 0;
             const int per = b < kBigBins ? 1 : kCols / max(1, kCols - (b - kBigBins));
             const int mine = b >= kListBins ? 0 : b < kBigBins ? big_units[b] : (count + per - 1) / per;
-            int e = count, u = mine;
+            const int own_strips = b >= kListBins ? 0 : b < kBigBins ? big_strips[b] : strips_of(count * (kCols - (b - kBigBins)));
+            int e = count, u = mine, s = own_strips;
             for (int off = 1; off < 64; off <<= 1) {
-                const int ue = __shfl_up(e, off), uu = __shfl_up(u, off);
-                if (lane >= off) { e += ue; u += uu; }
+                const int ue = __shfl_up(e, off), uu = __shfl_up(u, off), us = __shfl_up(s, off);
+                if (lane >= off) { e += ue; u += uu; s += us; }
             }
             if (b < kListBins) {
+                strip_at[b] = s_run + s - own_strips;
                 entry_at[b] = entry_first[b] = e_run + e - count;
                 unit_at[b] = u_run + u - mine;
             }
             e_run += __shfl(e, 63);
             u_run += __shfl(u, 63);
+            s_run += __shfl(s, 63);
         }
-        if (lane == 0) total[0] = u_run;
+        if (lane == 0) {
+            total[0] = u_run;
+            if (strips) total[1] = s_run;
+        }
     }
     __syncthreads();
     int before = 0;                    // pairs of the windows that earlier rounds placed
@@ -144,15 +164,25 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
         }
         if (lane == 63) wave_pairs[wave] = incl;
         for (int i = t; i < kWavesOfList * kListBins; i += kListThreads) of_wave[0][i] = 0;
+        if (t < kWavesOfList * kBigBins) strips_of_wave[0][t] = 0;
         __syncthreads();
         // a window's place among those of its bin: in its wavefront, then behind the wavefronts before
         const int b = n > 0 ? list_bin(n) : -1;
-        int rank = 0;
+        // (of a bin of larger windows, also the strips of the windows before: all but up to three fewer than four a tile)
+        const int fewer = n > kCols ? 4 * tiles_of(n) - strips_of(n) : 0;
+        int rank = 0, strips_before = 0;
         for (unsigned long long left = __ballot(b >= 0); left;) {
             const int bin = __builtin_amdgcn_readlane(b, __ffsll(static_cast<long long>(left)) - 1);
             const unsigned long long same = __ballot(b == bin);
-            if (b == bin) rank = __popcll(same & ((1ull << lane) - 1));
+            const unsigned long long below = same & ((1ull << lane) - 1);
+            if (b == bin) rank = __popcll(below);
             if (lane == 0) of_wave[wave][bin] = __popcll(same);
+            if (bin < kBigBins) {
+                const unsigned long long one = __ballot((fewer & 1) != 0), two = __ballot((fewer & 2) != 0);
+                const int most = 4 * (32 - bin);       // (not in bin 0, whose windows differ in their tiles)
+                if (b == bin) strips_before = most * rank - __popcll(below & one) - 2 * __popcll(below & two);
+                if (lane == 0) strips_of_wave[wave][bin] = most * __popcll(same) - __popcll(same & one) - 2 * __popcll(same & two);
+            }
             left &= ~same;
         }
         int pairs = before + incl - own, all = 0;
@@ -173,6 +203,16 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
                 run += count[v];
             }
             entry_at[t] = run;
+        } else if (t >= 128 && t < 128 + kBigBins) {
+            const int bin = t - 128;
+            int run = strip_at[bin];
+#pragma unroll
+            for (int v = 0; v < kWavesOfList; ++v) {
+                const int own_count = strips_of_wave[v][bin];
+                strips_of_wave[v][bin] = run;
+                run += own_count;
+            }
+            if (bin > 0) strip_at[bin] = run;
         }
         __syncthreads();
         if (b >= 0) {
@@ -183,9 +223,19 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
                 // (the windows of the first bin differ in their tiles)
                 const int u = b > 0 ? unit_at[b] + in_bin * tiles : atomicAdd(&unit_at[b], tiles);
                 for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
+                if (strips) {
+                    const int count = strips_of(n), first = b > 0 ? strips_of_wave[wave][b] + strips_before : atomicAdd(&strip_at[b], count);
+                    for (int q = 0; q < count; ++q) strips[first + q] = make_int4(e, n, q * kStrip, min(kStrip, n - q * kStrip));
+                }
             } else {
                 const int per = kCols / n;
                 if (in_bin % per == 0) units[unit_at[b] + in_bin / per] = make_int4(e, n, min(per, windows[b] - in_bin), 0);
+                if (strips) {
+                    // the strips whose first column is this window's
+                    const int begin = in_bin * n, end = begin + n, columns = windows[b] * n;
+                    for (int q = strips_of(begin); q * kStrip < end; ++q)
+                        strips[strip_at[b] + q] = make_int4(e, n, q * kStrip - begin, min(kStrip, columns - q * kStrip));
+                }
             }
         }
         __syncthreads();
@@ -211,23 +261,6 @@ __device__ __forceinline__ void lds_store2(uint32_t addr, float a, float b)
 {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     *(__attribute__((address_space(3))) f32x2 *)(addr) = f32x2{a, b};
-}
-__device__ __forceinline__ void lds_load8(uint32_t addr, float *v)
-{
-#pragma unroll
-    for (int c = 0; c < 8; c += 4) {
-        const f32x4_t q = *(lds_float4_t *)(addr + 4 * c);
-        v[c] = q[0]; v[c + 1] = q[1]; v[c + 2] = q[2]; v[c + 3] = q[3];
-    }
-}
-// eight 64-bit cells: low and high words
-__device__ __forceinline__ void lds_load_cells(uint32_t addr, uint32_t *lo, int *hi)
-{
-#pragma unroll
-    for (int c = 0; c < 8; c += 2) {
-        const u32x4_t q = *(lds_u32x4 *)(addr + 8 * c);
-        lo[c] = q[0]; hi[c] = static_cast<int>(q[1]); lo[c + 1] = q[2]; hi[c + 1] = static_cast<int>(q[3]);
-    }
 }
 // cell += hi 2^32 + lo
 __device__ __forceinline__ void lds_add64(uint32_t addr, uint32_t lo, int hi)
@@ -498,26 +531,6 @@ __device__ __forceinline__ f32x16 mfma32(const Operand<__half> &a, const Pair16 
 {
     c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.lo, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.hi, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4_t mfma16(const Pair16 &a, const Cells<__half> &b, f32x4_t c)
-{
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo, b.hi, c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.lo, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.hi, c, 0, 0, 0);
-}
-
-// ... with the cells as A (their columns are the terms) and exact values as B
-template <typename T> struct CellsA : Cells<T> {};
-__device__ __forceinline__ f32x4_t mfma16(const CellsA<__half> &a, const Operand<__half> &b, f32x4_t c)
-{
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.lo, b.x, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.hi, b.x, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4_t mfma16(const CellsA<float> &a, const Operand<float> &b, f32x4_t c)
-{
-    Cells<float> x;
-    x.x = b;
-    return mfma16(a.x, x, c);
 }
 
 }  // namespace tile

@@ -15,7 +15,7 @@ namespace {
 __global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int32_t *w_sizes, const int32_t *w2n, int W, int32_t *total,
                                                                  int4 *units, int2 *entries)
 {
-    build_list(w_sizes, w2n, W, total, units, entries);
+    build_list(w_sizes, w2n, W, total, units, entries, nullptr);
 }
 
 struct FwdArgs {
