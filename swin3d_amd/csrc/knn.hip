@@ -11,11 +11,7 @@
 //
 // Distance arithmetic: d = src - query per axis, ((dx*dx) + (dy*dy)) + (dz*dz),
 // every operation individually rounded to fp32 (no fused multiply-add).
-#include "s3d_common.h"
-
-#include <cstring>
-
-#include <rocprim/rocprim.hpp>
+#include "attn_kernels.h"
 
 namespace s3d {
 namespace {
@@ -30,30 +26,22 @@ struct KnnPlan {
     float origin[3];
     float cell, inv_cell, slack;
     int dim[3];
-    int cells_per_batch;
+    int pitch;            // dim[0] + 1: an x-row of cells has one more in memory, whose start is the row's end
+    int cells_per_batch;  // in memory: pitch dim[1] dim[2]
     int src_end;  // sources at or beyond this row belong to no batch segment
 };
 
 struct Layout {
-    size_t plan, partials, counts, starts, src_place, sorted, temp, temp_bytes, total;
+    size_t plan, partials, counts, starts, src_place, sorted, total;
     int64_t cells_cap;
 };
 
 int64_t cells_cap_for(int64_t Ns)
 {
     int64_t cap = 4 * Ns;
-    if (cap < 4096) cap = 4096;
+    if (cap < 2 * kMaxBatch) cap = 2 * kMaxBatch;      // (a batch segment takes two at least: one cell and the row's end)
     if (cap > (1LL << 24)) cap = 1LL << 24;
     return cap;
-}
-
-size_t scan_temp_bytes(int64_t n)
-{
-    size_t bytes = 0;
-    int32_t *p = nullptr;
-    (void)rocprim::exclusive_scan(nullptr, bytes, p, p, 0, static_cast<size_t>(n),
-                                  rocprim::plus<int32_t>(), hipStream_t(0));
-    return bytes;
 }
 
 Layout make_layout(int64_t Ns)
@@ -61,7 +49,7 @@ Layout make_layout(int64_t Ns)
     Layout L{};
     L.cells_cap = cells_cap_for(Ns);
     const size_t ns = static_cast<size_t>(Ns > 0 ? Ns : 1);
-    const size_t cells = static_cast<size_t>(L.cells_cap) + 1;
+    const size_t cells = static_cast<size_t>(L.cells_cap);
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
@@ -69,13 +57,11 @@ Layout make_layout(int64_t Ns)
         return at;
     };
     L.plan = take(sizeof(KnnPlan));
-    L.partials = take(sizeof(int32_t) * 6 * kBboxBlocks);
+    L.partials = take(sizeof(int32_t) * (6 * kBboxBlocks + 1));      // ... and how many sources have a place
     L.counts = take(cells * sizeof(int32_t));
     L.starts = take(cells * sizeof(int32_t));
     L.src_place = take(ns * sizeof(int2));
     L.sorted = take(ns * sizeof(float4));
-    L.temp_bytes = scan_temp_bytes(static_cast<int64_t>(cells));
-    L.temp = take(L.temp_bytes);
     L.total = off;
     return L;
 }
@@ -100,6 +86,7 @@ __global__ __launch_bounds__(kThreads) void knn_bbox_kernel(const float *__restr
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < cells;
          i += static_cast<int64_t>(gridDim.x) * kThreads)
         counts[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) partials[6 * kBboxBlocks] = 0;
     int lo[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff};
     int hi[3] = {static_cast<int>(0x80000000u), static_cast<int>(0x80000000u),
                  static_cast<int>(0x80000000u)};
@@ -136,33 +123,36 @@ __global__ __launch_bounds__(kThreads) void knn_bbox_kernel(const float *__restr
     }
 }
 
-// One thread: turn the bounding box (plan->lo / hi) into grid parameters that fit `cells_cap`.
+// One wavefront: turn the bounding box (plan->lo / hi) into grid parameters that fit `cells_cap`.  Every workgroup makes the
+// same of it.
 __device__ void make_plan(KnnPlan *plan, const int32_t *__restrict__ src_offset, int B, int64_t Ns, int K,
                           float cell_hint, int64_t cells_cap)
 {
+    const int lane = threadIdx.x & 63;
     int src_end = src_offset[B - 1];
     if (src_end > Ns) src_end = static_cast<int>(Ns);
     if (src_end < 0) src_end = 0;
-    plan->src_end = src_end;
     if (src_end == 0) {  // no candidate anywhere: the query kernel pads every slot
-        for (int a = 0; a < 3; ++a) {
-            plan->origin[a] = 0.0f;
-            plan->dim[a] = 1;
+        if (lane == 0) {
+            for (int a = 0; a < 3; ++a) {
+                plan->origin[a] = 0.0f;
+                plan->dim[a] = 1;
+            }
+            plan->cell = plan->inv_cell = 1.0f;
+            plan->slack = 0.0f;
+            plan->pitch = plan->cells_per_batch = 2;
+            plan->src_end = 0;
         }
-        plan->cell = plan->inv_cell = 1.0f;
-        plan->slack = 0.0f;
-        plan->cells_per_batch = 1;
         return;
     }
     float ext[3], max_abs = 0.0f;
     for (int a = 0; a < 3; ++a) {
         const float lo = ordered_to_float(plan->lo[a]);
         const float hi = ordered_to_float(plan->hi[a]);
-        plan->origin[a] = lo;
         ext[a] = fmaxf(hi - lo, 0.0f);
         max_abs = fmaxf(max_abs, fmaxf(fabsf(lo), fabsf(hi)));
     }
-    const int64_t per_batch_cap = cells_cap / B;  // B <= kMaxBatch <= cells_cap
+    const int64_t per_batch_cap = cells_cap / B;  // B <= kMaxBatch <= cells_cap / 2
     float cell = cell_hint;
     if (!(cell > 0.0f)) {
         // no hint: about K / 32 sources per cell if the sources filled their box (scans of surfaces fill a small part
@@ -175,37 +165,50 @@ __device__ void make_plan(KnnPlan *plan, const int32_t *__restrict__ src_offset,
         cell = fmaxf(cell, cbrtf(vol / static_cast<float>(per_batch_cap > 0 ? per_batch_cap : 1)));
     }
     if (!(cell > 1e-20f)) cell = 1.0f;
+    // the first that fits of a ladder of cell edges (forty steps of 3 %, then of 25 %), a lane each: 64 at a time
     int dim[3];
-    for (int iter = 0; iter < 400; ++iter) {
+    bool fits = false;
+    for (int first = 0; first < 448 && !fits; first += 64) {
+        const int step = first + lane;
+        const float edge = cell * exp2f(static_cast<float>(min(step, 40)) * 0.04264434f + static_cast<float>(max(step - 40, 0)) * 0.32192809f);
         double total = 1.0;
+        int d[3];
         for (int a = 0; a < 3; ++a) {
-            const float cells_f = floorf(ext[a] / cell) + 1.0f;
-            dim[a] = cells_f < 2.0e9f ? static_cast<int>(cells_f) : 2000000000;
-            total *= static_cast<double>(dim[a]);
+            const float cells_f = floorf(ext[a] / edge) + 1.0f;
+            d[a] = cells_f < 2.0e9f ? static_cast<int>(cells_f) : 2000000000;
+            total *= static_cast<double>(d[a]) + (a == 0 ? 1.0 : 0.0);
         }
-        if (total <= static_cast<double>(per_batch_cap)) break;
-        cell *= iter < 40 ? 1.03f : 1.25f;
-    }
-    {
-        double total = static_cast<double>(dim[0]) * dim[1] * dim[2];
-        if (total > static_cast<double>(per_batch_cap)) {  // degenerate input: single cell
-            dim[0] = dim[1] = dim[2] = 1;
-            cell = fmaxf(fmaxf(ext[0], ext[1]), ext[2]) * 2.0f + 1.0f;
+        const unsigned long long good = __ballot(total <= static_cast<double>(per_batch_cap));
+        if (good) {
+            const int which = __ffsll(static_cast<long long>(good)) - 1;
+            for (int a = 0; a < 3; ++a) dim[a] = __shfl(d[a], which);
+            cell = __shfl(edge, which);
+            fits = true;
         }
     }
+    if (!fits) {  // degenerate input: single cell
+        dim[0] = dim[1] = dim[2] = 1;
+        cell = fmaxf(fmaxf(ext[0], ext[1]), ext[2]) * 2.0f + 1.0f;
+    }
+    if (lane != 0) return;
+    plan->src_end = src_end;
     plan->cell = cell;
     plan->inv_cell = 1.0f / cell;
     // sources within `slack` of a cell face may sit in either neighbour cell
     plan->slack = 1e-3f * cell + 8e-6f * max_abs;
-    for (int a = 0; a < 3; ++a) plan->dim[a] = dim[a];
-    plan->cells_per_batch = dim[0] * dim[1] * dim[2];
+    for (int a = 0; a < 3; ++a) {
+        plan->origin[a] = ordered_to_float(plan->lo[a]);
+        plan->dim[a] = dim[a];
+    }
+    plan->pitch = dim[0] + 1;
+    plan->cells_per_batch = (dim[0] + 1) * dim[1] * dim[2];
 }
 
 // the plan of a call without sources (the query kernel pads every slot)
 __global__ void knn_plan_kernel(KnnPlan *plan, const int32_t *__restrict__ src_offset, int B,
                                 int64_t Ns, int K, float cell_hint, int64_t cells_cap)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    if (threadIdx.x >= 64 || blockIdx.x != 0) return;
     make_plan(plan, src_offset, B, Ns, K, cell_hint, cells_cap);
 }
 
@@ -224,6 +227,39 @@ __device__ __forceinline__ int find_batch(const int32_t *__restrict__ offset, in
     return b;  // == B: beyond the last segment
 }
 
+__device__ __forceinline__ int cell_of(const KnnPlan &plan, const float *p, int b)
+{
+    int c[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        c[a] = cell_coord(p[a], plan.origin[a], plan.inv_cell);
+        c[a] = min(max(c[a], 0), plan.dim[a] - 1);
+    }
+    return b * plan.cells_per_batch + (c[2] * plan.dim[1] + c[1]) * plan.pitch + c[0];
+}
+
+// reduce a box of order-preserving integers (lower corner, upper corner) over the workgroup into `box`
+template <int kWaves> __device__ __forceinline__ void reduce_box(int *v, int (*part)[6], int *box)
+{
+#pragma unroll
+    for (int a = 0; a < 6; ++a)
+        for (int off = 32; off > 0; off >>= 1) {
+            const int o = __shfl_down(v[a], off);
+            v[a] = a < 3 ? min(v[a], o) : max(v[a], o);
+        }
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int a = 0; a < 6; ++a) part[threadIdx.x >> 6][a] = v[a];
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        int r = part[0][threadIdx.x];
+        for (int w = 1; w < kWaves; ++w)
+            r = threadIdx.x < 3 ? min(r, part[w][threadIdx.x]) : max(r, part[w][threadIdx.x]);
+        box[threadIdx.x] = r;
+    }
+    __syncthreads();
+}
+
 // Every workgroup first reduces the partial boxes and derives the grid from them (the same arithmetic in every
 // workgroup; workgroup 0 leaves the plan for the kernels that follow), then its sources take their places: a
 // source's cell and its slot there, drawn from the cell's counter.  Neighbouring lanes that fall into the same
@@ -236,6 +272,11 @@ __global__ __launch_bounds__(kThreads) void knn_count_kernel(
 {
     __shared__ KnnPlan plan;
     __shared__ int part[kThreads / 64][6];
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    float own[3] = {0.0f, 0.0f, 0.0f};
+    if (i < Ns)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) own[a] = src[i * 3 + a];
     {
         int v[6];
 #pragma unroll
@@ -243,42 +284,18 @@ __global__ __launch_bounds__(kThreads) void knn_count_kernel(
         for (int t = threadIdx.x; t < boxes; t += kThreads)
 #pragma unroll
             for (int a = 0; a < 6; ++a) v[a] = a < 3 ? min(v[a], partials[t * 6 + a]) : max(v[a], partials[t * 6 + a]);
-#pragma unroll
-        for (int a = 0; a < 6; ++a)
-            for (int off = 32; off > 0; off >>= 1) {
-                const int o = __shfl_down(v[a], off);
-                v[a] = a < 3 ? min(v[a], o) : max(v[a], o);
-            }
-        if ((threadIdx.x & 63) == 0)
-#pragma unroll
-            for (int a = 0; a < 6; ++a) part[threadIdx.x >> 6][a] = v[a];
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int a = 0; a < 6; ++a) {
-                int r = part[0][a];
-                for (int w = 1; w < kThreads / 64; ++w) r = a < 3 ? min(r, part[w][a]) : max(r, part[w][a]);
-                if (a < 3) plan.lo[a] = r; else plan.hi[a - 3] = r;
-            }
+        reduce_box<kThreads / 64>(v, part, plan.lo);      // (lo and hi lie side by side)
+        if (threadIdx.x < 64) {
             make_plan(&plan, src_offset, B, Ns, K, cell_hint, cells_cap);
-            if (blockIdx.x == 0) *plan_out = plan;
+            if (blockIdx.x == 0 && threadIdx.x == 0) *plan_out = plan;
         }
         __syncthreads();
     }
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     const int lane = threadIdx.x & 63;
     int cell = -2;                       // beyond the array
     if (i < Ns) {
         const int b = find_batch(src_offset, B, i);
-        cell = -1;                       // in no batch segment
-        if (b < B) {
-            int c[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                c[a] = cell_coord(src[i * 3 + a], plan.origin[a], plan.inv_cell);
-                c[a] = min(max(c[a], 0), plan.dim[a] - 1);
-            }
-            cell = b * plan.cells_per_batch + (c[2] * plan.dim[1] + c[1]) * plan.dim[0] + c[0];
-        }
+        cell = b < B ? cell_of(plan, own, b) : -1;      // (-1: in no batch segment)
     }
     // runs of equal cells along the lanes: the first lane of a run draws the run's slots
     const int before = __shfl_up(cell, 1);
@@ -292,6 +309,174 @@ __global__ __launch_bounds__(kThreads) void knn_count_kernel(
     if (head && cell >= 0) base = atomicAdd(&counts[cell], next - lane);
     base = __shfl(base, my_head);
     if (i < Ns) src_place[i] = make_int2(cell, base + (lane - my_head));
+}
+
+// inclusive sum over the lanes of a wavefront, by DPP moves
+__device__ __forceinline__ int wave_scan(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);      // row_shr 1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);      // row_bcast15 into rows 1, 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);      // row_bcast31 into rows 2, 3
+    return x;
+}
+
+// Where every cell's sources start.  The sources of an x-row of cells lie one after the other (a query reads runs of cells),
+// the rows in any order: a workgroup takes whole rows, adds their counts up and draws the room for them with one atomic.
+// (One launch and no state to prepare, where a scan over all cells took two: 10.5 -> 6 us for 199,327 sources.)
+constexpr int kStartThreads = 1024, kStartCells = 4 * kStartThreads;
+__global__ __launch_bounds__(kStartThreads) void knn_starts_kernel(const KnnPlan *__restrict__ plan_ptr, int B,
+                                                                   const int32_t *__restrict__ counts, int32_t *__restrict__ starts,
+                                                                   int32_t *__restrict__ placed)
+{
+    __shared__ int wave_sum[kStartThreads / 64];
+    __shared__ int base_s;
+    const int pitch = plan_ptr->pitch;
+    const int64_t rows = static_cast<int64_t>(B) * (plan_ptr->cells_per_batch / pitch);
+    const int64_t rows_here = max(1, kStartCells / pitch);
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * rows_here;
+    if (first >= rows) return;
+    const int64_t cells0 = first * pitch, cells1 = min(first + rows_here, rows) * pitch;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // sum of a thread's four neighbouring cells before it, in the piece from `at` on, and the piece's sum
+    int v[4];
+    auto piece = [&](int64_t at, int &all) {
+        const int64_t mine = at + 4 * static_cast<int>(threadIdx.x);
+        int own = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = mine + e < cells1 ? counts[mine + e] : 0;
+            own += v[e];
+        }
+        const int incl = wave_scan(own);
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        int before = incl - own;
+        all = 0;
+#pragma unroll
+        for (int w = 0; w < kStartThreads / 64; ++w) {
+            before += w < wave ? wave_sum[w] : 0;
+            all += wave_sum[w];
+        }
+        __syncthreads();
+        return before;
+    };
+    auto write = [&](int64_t at, int run) {
+        const int64_t mine = at + 4 * static_cast<int>(threadIdx.x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (mine + e < cells1) starts[mine + e] = run;
+            run += v[e];
+        }
+    };
+    int all = 0, before = piece(cells0, all), total = all;
+    // (a row of more cells than the workgroup takes at a time: twice through it)
+    for (int64_t at = cells0 + kStartCells; at < cells1; at += kStartCells) {
+        int more;
+        piece(at, more);
+        total += more;
+    }
+    if (threadIdx.x == 0) base_s = total > 0 ? atomicAdd(placed, total) : 0;
+    __syncthreads();
+    int base = base_s;
+    if (cells1 - cells0 <= kStartCells) {
+        write(cells0, base + before);
+        return;
+    }
+    for (int64_t at = cells0; at < cells1; at += kStartCells) {
+        before = piece(at, all);
+        write(at, base + before);
+        base += all;
+    }
+}
+
+// The whole grid of up to kSmallSources sources by one workgroup, with the counters in LDS: box, plan, places, starts and
+// sorted sources in one launch of 12 us instead of four that take 16 (2,951 sources).  Whole calls, one workgroup and several
+// kernels: 1,500 sources 23.4 and 29.7 us, 3,000 27.6 and 32.7, 5,000 29.6 and 30.1, 8,100 36.1 and 32.5.
+constexpr int kSmallThreads = 1024, kSmallEach = 4, kSmallSources = kSmallThreads * kSmallEach;
+constexpr size_t small_lds(int64_t cells_cap) { return sizeof(int32_t) * static_cast<size_t>(cells_cap); }
+__global__ __launch_bounds__(kSmallThreads) void knn_small_grid_kernel(
+    const float *__restrict__ src, int Ns, const int32_t *__restrict__ src_offset, int B, int K, float cell_hint, int cells_cap,
+    KnnPlan *__restrict__ plan_out, int32_t *__restrict__ starts, float4 *__restrict__ sorted)
+{
+    extern __shared__ int counts[];
+    __shared__ KnnPlan plan;
+    __shared__ int part[kSmallThreads / 64][6], wave_sum[kSmallThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float p[kSmallEach][3];
+    int v[6];
+#pragma unroll
+    for (int a = 0; a < 6; ++a) v[a] = a < 3 ? 0x7fffffff : static_cast<int>(0x80000000u);
+#pragma unroll
+    for (int k = 0; k < kSmallEach; ++k) {
+        const int i = k * kSmallThreads + static_cast<int>(threadIdx.x);
+        if (k * kSmallThreads >= Ns) break;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            p[k][a] = i < Ns ? src[i * 3 + a] : 0.0f;
+            const int o = float_to_ordered(p[k][a]);
+            v[a] = i < Ns ? min(v[a], o) : v[a];
+            v[3 + a] = i < Ns ? max(v[3 + a], o) : v[3 + a];
+        }
+    }
+    reduce_box<kSmallThreads / 64>(v, part, plan.lo);
+    if (wave == 0) {
+        make_plan(&plan, src_offset, B, Ns, K, cell_hint, cells_cap);
+        if (lane == 0) *plan_out = plan;
+    }
+    __syncthreads();
+    const int cells = B * plan.cells_per_batch;
+    for (int c = threadIdx.x; c < cells; c += kSmallThreads) counts[c] = 0;
+    __syncthreads();
+    int cell[kSmallEach], slot[kSmallEach];
+#pragma unroll
+    for (int k = 0; k < kSmallEach; ++k) {
+        const int i = k * kSmallThreads + static_cast<int>(threadIdx.x);
+        if (k * kSmallThreads >= Ns) break;
+        const int b = i < Ns ? find_batch(src_offset, B, i) : B;
+        cell[k] = b < B ? cell_of(plan, p[k], b) : -1;
+        slot[k] = cell[k] >= 0 ? atomicAdd(&counts[cell[k]], 1) : 0;
+    }
+    __syncthreads();
+    // exclusive sum over the cells, a share of them per wavefront, four neighbours a lane
+    const int share = ((cells + 16 * 256 - 1) / (16 * 256)) * 256;
+    const int c0 = wave * share, c1 = min(c0 + share, cells);
+    int sum = 0;
+    for (int c = c0 + lane; c < c1; c += 64) sum += counts[c];
+    sum = wave_scan(sum);
+    if (lane == 63) wave_sum[wave] = sum;
+    __syncthreads();
+    int run = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallThreads / 64; ++w) run += w < wave ? wave_sum[w] : 0;
+    for (int c = c0; c < c1; c += 256) {
+        int own[4], all = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            own[e] = c + 4 * lane + e < c1 ? counts[c + 4 * lane + e] : 0;
+            all += own[e];
+        }
+        const int incl = wave_scan(all);
+        int at = run + incl - all;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (c + 4 * lane + e < c1) {
+                counts[c + 4 * lane + e] = at;
+                starts[c + 4 * lane + e] = at;
+            }
+            at += own[e];
+        }
+        run += __builtin_amdgcn_readlane(incl, 63);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSmallEach; ++k) {
+        const int i = k * kSmallThreads + static_cast<int>(threadIdx.x);
+        if (k * kSmallThreads >= Ns) break;
+        if (cell[k] >= 0) sorted[counts[cell[k]] + slot[k]] = make_float4(p[k][0], p[k][1], p[k][2], __int_as_float(i));
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void knn_scatter_kernel(
@@ -366,12 +551,16 @@ template <int SIZE> __device__ __forceinline__ void order(uint64_t &x, int t)
 // One query per group of G lanes (G = 4, 8, 16 or 64 >= K).  The group keeps its G best candidates as one sorted list, a
 // candidate per lane: a word of (squared distance, source row), whose order is the result's.  The sources of a run of
 // cells are read G at a time (the next ones while these are worked on), sorted across the lanes and merged: every step
-// is a DPP move and a compare on all lanes, no candidate waits for another.  (Inserting them one by one, with the list
-// shifted through LDS, took 73 us instead of 43 us at K = 16, 199,327 sources, a query for every cell of two voxels; what
-// is left are the chains of loads from the query to its cells' ranges to their sources.)
+// is a DPP move and a compare on all lanes, no candidate waits for another.  At K = 16, 199,327 sources, a query for every
+// cell of two voxels: 34 us, and 43 us with each run of cells read by itself, most of a group's lanes idle in its last step;
+// 73 us with candidates inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
 //
 // A walk starts with the cube of 3 x 3 x 3 cells: the query's own cell alone never proves its K best.
-template <int G>
+// Groups of sixteen for up to four neighbours, too, where there are few queries: a group then looks up the nine rows of cells
+// in one step.  K = 3, 12,170 and 37,140 sources: 50,000 queries 43 us with groups of four, 32 of sixteen; 150,000 52 and 46;
+// 600,000 94 and 131.
+constexpr int64_t kFewQueries = 200000;
+template <int G, int KMAX>
 __global__ __launch_bounds__(kThreads) void knn_query_kernel(
     int K, const float *__restrict__ qry, int64_t Nq, const int32_t *__restrict__ query_offset,
     int B, const KnnPlan *__restrict__ plan_ptr, const int32_t *__restrict__ starts,
@@ -401,33 +590,41 @@ __global__ __launch_bounds__(kThreads) void knn_query_kernel(
         r_last = max(r_last, r_first);
         const int32_t *cell_base = starts + static_cast<int64_t>(b) * plan.cells_per_batch;
         auto scan_rows = [&](int begin, int end) {
-            // every lane's range of sources: the ranges one after the other, G sources at a time
-            unsigned long long todo = __ballot(end > begin);
-            todo = (todo >> group_shift) & (G == 64 ? ~0ULL : ((1ULL << G) - 1));
-            int s = 0, stop = 0;
-            auto advance = [&]() {
-                s += G;
-                if (s < stop) return true;
-                if (!todo) return false;
-                const int k = __ffsll(static_cast<long long>(todo)) - 1;
-                todo &= todo - 1;
-                s = __shfl(begin, k, G);
-                stop = __shfl(end, k, G);
-                return true;
+            // every lane's range of sources: the ranges one after the other, G sources at a time, whatever ranges they
+            // belong to (a wall across the rows leaves some seven sources to each of nine ranges)
+            const int len = max(end - begin, 0);
+            int upto = len;
+            if constexpr (G == 16) {
+                upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, true);      // row_shr
+                upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, true);
+                upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, true);
+                upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, true);
+            } else {
+#pragma unroll
+                for (int off = 1; off < G; off <<= 1) {
+                    const int up = __shfl_up(upto, off, G);
+                    upto += t >= off ? up : 0;
+                }
+            }
+            const int total = __shfl(upto, G - 1, G), ahead = begin - (upto - len);
+            if (total == 0) return;
+            auto source = [&](int at) {
+                at = min(at, total - 1);
+                int k = 0;                         // ranges that end at or before it
+#pragma unroll
+                for (int half = G / 2; half > 0; half >>= 1) k += __shfl(upto, k + half - 1, G) <= at ? half : 0;
+                return sorted[at + __shfl(ahead, k, G)];
             };
-            bool more = advance();
-            float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (more) p = sorted[min(s + t, stop - 1)];
-            while (more) {
+            float4 p = source(t);
+            for (int s = 0; s < total; s += G) {
                 const float4 c = p;
-                const bool have = s + t < stop;
-                more = advance();
-                if (more) p = sorted[min(s + t, stop - 1)];
+                const bool have = s + t < total;
+                if (s + G < total) p = source(s + G + t);
                 uint64_t found = (static_cast<uint64_t>(__float_as_uint(dist2_unfused(c.x, c.y, c.z, qx, qy, qz))) << 32) |
                                  __float_as_uint(c.w);
                 found = have ? found : kNone;
-                // (a group of sixteen skips sources that are all behind its list)
-                if (G == 16 && !__any(found < dpp<0x15f>(best))) continue;
+                // (a group of sixteen skips sources that are all behind the last that can count)
+                if (G == 16 && !__any(found < dpp<0x150 + KMAX - 1>(best))) continue;
                 order<G>(found, t);
                 found = lane_xor<G - 1>(found);
                 best = found < best ? found : best;
@@ -450,7 +647,7 @@ __global__ __launch_bounds__(kThreads) void knn_query_kernel(
                 if (u < n_rows) {
                     const int dz = u / ny, z = z0 + dz, y = y0 + u - dz * ny;
                     const bool face = r == r_first || z == qc[2] - r || z == qc[2] + r || y == qc[1] - r || y == qc[1] + r;
-                    const int32_t *row = cell_base + (z * plan.dim[1] + y) * plan.dim[0];
+                    const int32_t *row = cell_base + (z * plan.dim[1] + y) * plan.pitch;
                     if (face) {
                         const int x0 = max(xl, 0), x1 = min(xh, plan.dim[0] - 1);
                         if (x0 <= x1) {
@@ -535,37 +732,43 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_kernel(const int32_t
         for (int i = 0; i < kAhead; ++i) weight[i] = 1.0f / (sqrtf(weight[i]) + 1e-8f);
         each(row, weight);
     };
-    float norm = 0.0f;
-    for (int i0 = 0; i0 < K; i0 += kAhead)
-        neighbours(i0, [&](const int *row, const float *weight) {
-#pragma unroll
-            for (int i = 0; i < kAhead; ++i) norm += row[i] >= 0 ? weight[i] : 0.0f;
-        });
-    float acc[VEC];
+    float norm = 0.0f, acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
-    for (int i0 = 0; i0 < K; i0 += kAhead)
-        neighbours(i0, [&](const int *row, const float *weight) {
-            T v[kAhead][VEC];
+    auto sum_weights = [&](const int *row, const float *weight) {
 #pragma unroll
-            for (int i = 0; i < kAhead; ++i) {
-                const T *from = feat + static_cast<int64_t>(max(row[i], 0)) * C + c0;
-                if (row[i] < 0) continue;
-                if constexpr (VEC == 4) {
-                    if constexpr (sizeof(T) == 4) *reinterpret_cast<float4 *>(v[i]) = *reinterpret_cast<const float4 *>(from);
-                    else *reinterpret_cast<uint2 *>(v[i]) = *reinterpret_cast<const uint2 *>(from);
-                } else {
-                    v[i][0] = *from;
-                }
+        for (int i = 0; i < kAhead; ++i) norm += row[i] >= 0 ? weight[i] : 0.0f;
+    };
+    auto add_features = [&](const int *row, const float *weight, auto weights_known) {
+        T v[kAhead][VEC];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const T *from = feat + static_cast<int64_t>(max(row[i], 0)) * C + c0;
+            if (row[i] < 0) continue;
+            if constexpr (VEC == 4) {
+                if constexpr (sizeof(T) == 4) *reinterpret_cast<float4 *>(v[i]) = *reinterpret_cast<const float4 *>(from);
+                else *reinterpret_cast<uint2 *>(v[i]) = *reinterpret_cast<const uint2 *>(from);
+            } else {
+                v[i][0] = *from;
             }
+        }
+        weights_known();
 #pragma unroll
-            for (int i = 0; i < kAhead; ++i) {
-                if (row[i] < 0) continue;
-                const float w = weight[i] / norm;
+        for (int i = 0; i < kAhead; ++i) {
+            if (row[i] < 0) continue;
+            const float w = weight[i] / norm;
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) acc[e] += w * static_cast<float>(v[i][e]);
-            }
-        });
+            for (int e = 0; e < VEC; ++e) acc[e] += w * static_cast<float>(v[i][e]);
+        }
+    };
+    if (K <= kAhead) {
+        // (the features on their way while the weights are added up: 9.5 -> 7 us at 12,421 x 192 fp32, K = 3)
+        neighbours(0, [&](const int *row, const float *weight) { add_features(row, weight, [&] { sum_weights(row, weight); }); });
+    } else {
+        for (int i0 = 0; i0 < K; i0 += kAhead) neighbours(i0, sum_weights);
+        for (int i0 = 0; i0 < K; i0 += kAhead)
+            neighbours(i0, [&](const int *row, const float *weight) { add_features(row, weight, [] {}); });
+    }
     T o[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) o[e] = static_cast<T>(acc[e]);
@@ -709,31 +912,37 @@ int knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int
     int2 *src_place = reinterpret_cast<int2 *>(base + L.src_place);
     int32_t *partials = reinterpret_cast<int32_t *>(base + L.partials);
     float4 *sorted = reinterpret_cast<float4 *>(base + L.sorted);
-    void *temp = base + L.temp;
-    size_t temp_bytes = L.temp_bytes;
-    const int64_t cells = L.cells_cap + 1;
+    const int64_t cells = L.cells_cap;
 
-    if (Ns > 0) {
-        // bounding box + zeroed counters, places (grid derived in every workgroup), scan, scatter
+    if (Ns > kSmallSources) {
+        // bounding box + zeroed counters, places (grid derived in every workgroup), starts, scatter
         const dim3 sgrid(static_cast<unsigned>(ceil_div(Ns, kThreads)));
         hipLaunchKernelGGL(knn_bbox_kernel, dim3(kBboxBlocks), dim3(kThreads), 0, s, src_xyz, Ns, partials, counts, cells);
-        S3D_HIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(knn_count_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, Ns, src_offset, B, partials,
                            kBboxBlocks, K, cell_size, L.cells_cap, plan, counts, src_place);
-        S3D_HIP_CHECK(hipGetLastError());
-        S3D_HIP_CHECK(rocprim::exclusive_scan(temp, temp_bytes, counts, starts, 0,
-                                              static_cast<size_t>(cells), rocprim::plus<int32_t>(), s));
+        // (workgroups: a share of whole rows is at least half of kStartCells, or a single row)
+        hipLaunchKernelGGL(knn_starts_kernel, dim3(static_cast<unsigned>(2 * cells / kStartCells + 1)), dim3(kStartThreads), 0, s, plan, B,
+                           counts, starts, partials + 6 * kBboxBlocks);
         hipLaunchKernelGGL(knn_scatter_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, Ns, src_place, starts, sorted);
+        S3D_HIP_CHECK(hipGetLastError());
+    } else if (Ns > 0) {
+        const size_t lds = small_lds(cells);
+        if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(knn_small_grid_kernel), small_lds(cells_cap_for(kSmallSources)))) return rc;
+        hipLaunchKernelGGL(knn_small_grid_kernel, dim3(1), dim3(kSmallThreads), lds, s, src_xyz, static_cast<int>(Ns), src_offset, B, K,
+                           cell_size, static_cast<int>(cells), plan, starts, sorted);
         S3D_HIP_CHECK(hipGetLastError());
     } else {
         hipLaunchKernelGGL(knn_plan_kernel, dim3(1), dim3(64), 0, s, plan, src_offset, B, Ns, K,
                            cell_size, L.cells_cap);
         S3D_HIP_CHECK(hipGetLastError());
     }
-    // lanes per query: the smallest group that holds the K entries, one per lane
-    const int G = K <= 4 ? 4 : K <= 8 ? 8 : K <= 16 ? 16 : 64;
+    // lanes per query: the smallest group that holds the K entries, one per lane; sixteen where groups of four would not
+    // fill the chip
+    const bool few = Nq <= kFewQueries;
+    const int G = K <= 4 && !few ? 4 : K <= 8 && !few ? 8 : K <= 16 ? 16 : 64;
     const dim3 qgrid(static_cast<unsigned>(ceil_div(Nq * G, kThreads)));
-    auto query = G == 4 ? knn_query_kernel<4> : G == 8 ? knn_query_kernel<8> : G == 16 ? knn_query_kernel<16> : knn_query_kernel<64>;
+    auto query = G == 4 ? knn_query_kernel<4, 4> : G == 8 ? knn_query_kernel<8, 8> : G == 64 ? knn_query_kernel<64, 64>
+                 : K <= 4 ? knn_query_kernel<16, 4> : K <= 8 ? knn_query_kernel<16, 8> : knn_query_kernel<16, 16>;
     hipLaunchKernelGGL(query, qgrid, dim3(kThreads), 0, s, K, query_xyz, Nq, query_offset, B, plan, starts, sorted, ret_idx,
                        ret_dist, squared);
     S3D_HIP_CHECK(hipGetLastError());
