@@ -284,6 +284,13 @@ typedef struct {
 size_t s3d_window_indices_workspace_bytes(int64_t N, int32_t num_sets);
 int s3d_window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets,
                        void *workspace, size_t workspace_bytes, void *stream);
+/*
+ * The same, and the calling thread waits for the counts, which also go to host_counts: pinned HOST int64 [num_sets][4]
+ * (hipHostMalloc).  It waits for the launches that lead to them and not for those behind them, which put the voxels in
+ * order.  Not for graph capture.
+ */
+int s3d_window_indices_counted(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets,
+                               int32_t num_sets, int64_t *host_counts, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * Representative voxel of every cell of a window sort: the member whose signal row is nearest (Euclidean, fp32) to

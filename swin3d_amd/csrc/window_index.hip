@@ -12,6 +12,8 @@
 
 #include <cstring>
 
+#include <type_traits>
+
 #include <rocprim/rocprim.hpp>
 
 namespace s3d {
@@ -161,14 +163,19 @@ __global__ __launch_bounds__(kThreads) void segment_size_kernel(const int32_t *_
 // ---- grid path: the same index without a sort of all voxels ----------------------------------------------
 // When the windows of a scene fit a dense lattice of at most cells_cap cells (they do for room-sized scenes: the
 // lattice is the bounding box of the window coordinates), a window is a lattice cell and the index is a counting
-// sort: every voxel draws a slot in its cell, a scan over the cells gives every non-empty cell its rank (= window
+// sort: every voxel draws a slot in its cell, a sum over the cells before it gives every non-empty cell its rank (= window
 // number, ascending (batch, wx, wy, wz) because the cell number is) and its first position, the voxels are placed
 // there, and each window's few voxels are put in (local id, row) order by one wavefront.  Six launches of a few
 // microseconds instead of a block sort and eight merge passes.
 //
 // Up to kMaxSets window sets of the same voxels are built together (blockIdx.y = set): what bounds a set alone is the
-// launches, each with too little work for the card (199,327 voxels, two sets: 46 us of kernels instead of 73).  The lattices come from one bounding box of the coordinates (a
-// window coordinate does not decrease with its voxel's), and one scan runs over the cells of all sets.
+// launches, each with too little work for the card (199,327 voxels, two sets: 46 us of kernels instead of 73).  The lattices
+// come from one bounding box of the coordinates (a window coordinate does not decrease with its voxel's).
+//
+// The windows, their pairs and the largest are known when the cells have been added up, and the host, which sizes what
+// follows by them, waits for that and not for the placing behind it.  (The sums run over the cells that the lattice has, a
+// fifth to a half of those it may have, in two launches; a library's scan over all of them took two as well, 14 us against 6
+// at 199,327 voxels.)
 constexpr int kGridBoxes = 128;          // workgroups of the bounding-box pass
 constexpr int kSlotBits = 20;            // a voxel's slot in its cell, below its local id in one word
 constexpr int kBadRange = 1, kNoGrid = 2;   // counts[3]: coordinates out of range / lattice too large for the grid path
@@ -192,36 +199,26 @@ struct GridPlan {
 };
 
 struct GridLayout {
-    size_t plan, partials, cells, scan, place, keys, temp, temp_bytes, total;
+    size_t plan, partials, cells, sums, scan, place, keys, total;
     int64_t cells_cap;
 };
 
 int64_t grid_cells_cap(int64_t N)
 {
-    int64_t cap = 2 * N;    // the scan over the cells is the longest of the five launches: no more cells than pay
+    int64_t cap = 2 * N;    // (no more cells than pay)
     if (cap < 4096) cap = 4096;
     if (cap > (1LL << 24)) cap = 1LL << 24;
     return cap;
 }
 
-// (non-empty << 32 | voxels) of a cell: one scan yields a cell's window number and its first position
-struct CellWord {
-    __host__ __device__ uint64_t operator()(int32_t count) const
-    {
-        return (count > 0 ? (1ULL << 32) : 0ULL) | static_cast<uint32_t>(count);
-    }
+// cells of a workgroup of the two launches that add them up, and what is left of them there
+constexpr int kSumThreads = 1024, kSumCells = 4 * kSumThreads;
+struct CellSum {
+    uint64_t before;       // (non-empty << 32 | voxels)
+    int64_t squares;
+    int32_t largest, unused;
 };
-typedef rocprim::transform_iterator<const int32_t *, CellWord, uint64_t> CellWordIterator;
-
-size_t grid_scan_temp_bytes(int64_t n)
-{
-    size_t bytes = 0;
-    const int32_t *p = nullptr;
-    uint64_t *o = nullptr;
-    (void)rocprim::exclusive_scan(nullptr, bytes, CellWordIterator(p, CellWord()), o, uint64_t(0), static_cast<size_t>(n),
-                                  rocprim::plus<uint64_t>(), hipStream_t(0));
-    return bytes;
-}
+__host__ __device__ __forceinline__ uint64_t cell_word(int32_t count) { return (count > 0 ? (1ULL << 32) : 0ULL) | static_cast<uint32_t>(count); }
 
 // plans, cells, scan, place and keys: one of each per set, one behind the other
 GridLayout make_grid_layout(int64_t N, int sets)
@@ -238,11 +235,10 @@ GridLayout make_grid_layout(int64_t N, int sets)
     L.plan = take(sizeof(GridPlan) * sets);
     L.partials = take(sizeof(int32_t) * 8 * kGridBoxes);
     L.cells = take(cells * sizeof(int32_t));
+    L.sums = take(sizeof(CellSum) * sets * static_cast<size_t>(ceil_div(L.cells_cap, kSumCells)));
     L.scan = take(cells * sizeof(uint64_t));
     L.place = take(n * sizeof(int2));
     L.keys = take(n * sizeof(uint64_t));
-    L.temp_bytes = grid_scan_temp_bytes(static_cast<int64_t>(cells));
-    L.temp = take(L.temp_bytes);
     L.total = off;
     return L;
 }
@@ -385,6 +381,137 @@ __global__ __launch_bounds__(kThreads) void grid_count_kernel(
     }
 }
 
+// sum over the lanes before this one, by DPP moves, and over all lanes in the last
+__device__ __forceinline__ uint64_t wave_scan(uint64_t x)
+{
+    auto add = [](uint64_t v, auto ctrl, auto rows) {
+        const int lo = static_cast<int>(v), hi = static_cast<int>(v >> 32);
+        const uint32_t l = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, lo, decltype(ctrl)::value, decltype(rows)::value, 0xf, true));
+        const uint32_t h = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, hi, decltype(ctrl)::value, decltype(rows)::value, 0xf, true));
+        return v + ((static_cast<uint64_t>(h) << 32) | l);
+    };
+    x = add(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});      // row_shr 1, 2, 4, 8
+    x = add(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    x = add(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    x = add(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    x = add(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});      // row_bcast15 into rows 1, 3
+    return add(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});   // row_bcast31 into rows 2, 3
+}
+
+__device__ __forceinline__ int64_t cells_of(const GridPlan &plan)
+{
+    return static_cast<int64_t>(plan.dim[0]) * plan.dim[1] * plan.dim[2] * plan.dim[3];
+}
+
+// what a workgroup's cells add up to
+__global__ __launch_bounds__(kSumThreads) void grid_sums_kernel(GridSets sets, const GridPlan *__restrict__ plan,
+                                                                const int32_t *__restrict__ cells, int64_t cells_cap,
+                                                                CellSum *__restrict__ sums)
+{
+    const int set = blockIdx.y;
+    if (!plan[set].ok || (sets.set[set].counts[3] & kNoGrid)) return;
+    const int64_t total = cells_of(plan[set]), first = static_cast<int64_t>(blockIdx.x) * kSumCells;
+    if (first >= total) return;
+    cells += set * (cells_cap + 1);
+    uint64_t sum = 0;
+    int64_t squares = 0;
+    int largest = 0;
+#pragma unroll
+    for (int e = 0; e < kSumCells / kSumThreads; ++e) {
+        const int64_t c = first + e * kSumThreads + threadIdx.x;
+        const int n = c < total ? cells[c] : 0;
+        sum += cell_word(n);
+        squares += static_cast<int64_t>(n) * n;
+        largest = max(largest, n);
+    }
+    sum = wave_scan(sum);
+    squares = static_cast<int64_t>(wave_scan(static_cast<uint64_t>(squares)));
+    for (int off = 32; off > 0; off >>= 1) largest = max(largest, __shfl_xor(largest, off));
+    __shared__ CellSum part[kSumThreads / 64];
+    if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = CellSum{sum, squares, largest, 0};
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    CellSum all = part[0];
+    for (int w = 1; w < kSumThreads / 64; ++w) {
+        all.before += part[w].before;
+        all.squares += part[w].squares;
+        all.largest = max(all.largest, part[w].largest);
+    }
+    sums[set * gridDim.x + blockIdx.x] = all;
+}
+
+// Every cell's window number and first position: what the workgroups before this one add up to and a scan of its own cells.
+// The first workgroup of a set leaves the totals and the status word, also where the host reads them (or null).
+__global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets, const GridPlan *__restrict__ plan,
+                                                                  const int32_t *__restrict__ cells, int64_t cells_cap,
+                                                                  const CellSum *__restrict__ sums, uint64_t *__restrict__ scan,
+                                                                  int64_t *host_counts)
+{
+    const int set = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int64_t *counts = sets.set[set].counts;
+    const int64_t status = counts[3];
+    const bool good = plan[set].ok && !(status & kNoGrid);
+    const int64_t total = good ? cells_of(plan[set]) : 0, first = static_cast<int64_t>(blockIdx.x) * kSumCells;
+    sums += set * gridDim.x;
+    __shared__ CellSum part[kSumThreads / 64];
+    __shared__ uint64_t wave_sum[kSumThreads / 64];
+    if (blockIdx.x == 0) {
+        const int groups = static_cast<int>((total + kSumCells - 1) / kSumCells);
+        CellSum all{0, 0, 0, 0};
+        for (int g = threadIdx.x; g < groups; g += kSumThreads) {
+            all.before += sums[g].before;
+            all.squares += sums[g].squares;
+            all.largest = max(all.largest, sums[g].largest);
+        }
+        all.before = wave_scan(all.before);
+        all.squares = static_cast<int64_t>(wave_scan(static_cast<uint64_t>(all.squares)));
+        for (int off = 32; off > 0; off >>= 1) all.largest = max(all.largest, __shfl_xor(all.largest, off));
+        if (lane == 63) part[wave] = all;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < kSumThreads / 64; ++w) {
+                part[0].before += part[w].before;
+                part[0].squares += part[w].squares;
+                part[0].largest = max(part[0].largest, part[w].largest);
+            }
+            const int64_t totals[4] = {static_cast<int64_t>(part[0].before >> 32), part[0].squares, part[0].largest, status};
+            for (int k = 0; k < 3 && good; ++k) counts[k] = totals[k];
+            if (host_counts)
+                for (int k = 0; k < 4; ++k) host_counts[4 * set + k] = totals[k];
+        }
+        __syncthreads();
+    }
+    if (first >= total) return;
+    cells += set * (cells_cap + 1);
+    scan += set * (cells_cap + 1);
+    uint64_t before = 0;
+    for (int g = threadIdx.x; g < static_cast<int>(blockIdx.x); g += kSumThreads) before += sums[g].before;
+    before = wave_scan(before);
+    if (lane == 63) part[wave].before = before;
+    // four neighbouring cells a thread
+    int n[4];
+    uint64_t own = 0;
+    const int64_t mine = first + 4 * static_cast<int>(threadIdx.x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        n[e] = mine + e < total ? cells[mine + e] : 0;
+        own += cell_word(n[e]);
+    }
+    const uint64_t upto = wave_scan(own);
+    if (lane == 63) wave_sum[wave] = upto;
+    __syncthreads();
+    uint64_t run = upto - own;
+#pragma unroll
+    for (int w = 0; w < kSumThreads / 64; ++w) run += part[w].before + (w < wave ? wave_sum[w] : 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (mine + e <= total) scan[mine + e] = run;
+        run += cell_word(n[e]);
+    }
+    // (the end of the last cell, where that is a workgroup's last)
+    if (threadIdx.x == kSumThreads - 1 && mine + 4 == total) scan[total] = run;
+}
+
 // every voxel to its window's segment (slot order); the voxel in slot 0 also records the window
 __global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__restrict__ place, int64_t N, GridSets sets,
                                                               const GridPlan *__restrict__ plan,
@@ -392,30 +519,26 @@ __global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__rest
                                                               uint64_t *__restrict__ keys)
 {
     const int set = blockIdx.y;
-    int64_t *counts = sets.set[set].counts;
     int32_t *w2n = sets.set[set].w2n, *w_sizes = sets.set[set].w_sizes;
-    if (!plan[set].ok || (counts[3] & kNoGrid)) return;
+    if (!plan[set].ok || (sets.set[set].counts[3] & kNoGrid)) return;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >= N) return;
     scan += set * (cells_cap + 1);
     place += set * N;
     keys += set * N;
-    const uint64_t before = scan[0];       // windows and voxels of the sets before this one
-    if (i == 0) counts[0] = static_cast<int64_t>((scan[cells_cap] - before) >> 32);   // non-empty cells = windows
-    if (i >= N) return;
     const int2 p = place[i];
-    const uint64_t here = scan[p.x] - before;
+    const uint64_t here = scan[p.x];
     const int start = static_cast<int>(here & 0xffffffffu), slot = p.y & ((1 << kSlotBits) - 1);
     keys[start + slot] = (static_cast<uint64_t>(p.y >> kSlotBits) << 32) | static_cast<uint32_t>(i);
     if (slot == 0) {
         const int rank = static_cast<int>(here >> 32);
         w2n[rank] = start;
-        w_sizes[rank] = static_cast<int>((scan[p.x + 1] - before) & 0xffffffffu) - start;
+        w_sizes[rank] = static_cast<int>(scan[p.x + 1] & 0xffffffffu) - start;
     }
 }
 
 // One wavefront per window at a time: the window's voxels in (local id, row) order.  The rank of an element is
 // the number of smaller ones, counted against every element of the window (a few dozen to a few hundred voxels).
-// Also the totals: sum of squared sizes and the largest size, one pair of atomics per workgroup.
 __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__restrict__ plan,
                                                               const uint64_t *__restrict__ keys, int64_t N, GridSets sets)
 {
@@ -426,7 +549,6 @@ __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__
     if (!plan[set].ok || (counts[3] & kNoGrid)) return;
     keys += set * N;
     constexpr int kOrderStage = 512;                       // keys of a window staged in LDS at a time, per wavefront
-    constexpr int kTotalGroups = 32;
     __shared__ uint64_t stage_all[kThreads / 64][kOrderStage];
     uint64_t *stage = stage_all[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
@@ -474,29 +596,6 @@ __global__ __launch_bounds__(kThreads) void grid_order_kernel(const GridPlan *__
                 n2n[start + rank] = static_cast<int32_t>(mine & 0xffffffffu);
                 w_w_id[start + rank] = static_cast<int32_t>(mine >> 32);
             }
-        }
-    }
-    // the totals (sum of squared sizes, largest size): the first kTotalGroups workgroups share the windows, one pair
-    // of atomics each
-    if (blockIdx.x >= kTotalGroups) return;
-    long long squares = 0, largest = 0;
-    for (int w = static_cast<int>(blockIdx.x) * kThreads + threadIdx.x; w < W; w += kTotalGroups * kThreads) {
-        const long long n = w_sizes[w];
-        squares += n * n;
-        largest = max(largest, n);
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        squares += __shfl_down(squares, off);
-        largest = max(largest, __shfl_down(largest, off));
-    }
-    __shared__ long long part[kThreads / 64][2];
-    if (lane == 0) { part[threadIdx.x >> 6][0] = squares; part[threadIdx.x >> 6][1] = largest; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int wv = 1; wv < kThreads / 64; ++wv) { squares += part[wv][0]; largest = max(largest, part[wv][1]); }
-        if (largest > 0) {
-            atomicAdd(reinterpret_cast<unsigned long long *>(counts + 1), static_cast<unsigned long long>(squares));
-            atomicMax(reinterpret_cast<unsigned long long *>(counts + 2), static_cast<unsigned long long>(largest));
         }
     }
 }
@@ -743,11 +842,13 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_window_indices_work
     return num_sets < 1 || num_sets > s3d::kMaxSets ? 0 : s3d::make_grid_layout(N, num_sets).total;
 }
 
-extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
-    const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *jobs, int32_t num_sets, void *workspace,
-    size_t workspace_bytes, void *stream)
+namespace s3d {
+namespace {
+
+// counted: recorded behind the launch that leaves the counts in host_counts (or null, as that)
+int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *jobs, int32_t num_sets,
+                   int64_t *host_counts, hipEvent_t counted, void *workspace, size_t workspace_bytes, void *stream)
 {
-    using namespace s3d;
     if (N < 0 || N > 0x7fffffffLL || num_sets < 1 || num_sets > kMaxSets || N * num_sets > 0xffffffffLL)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_window_indices: N=%lld voxels, %d sets (1..%d)", (long long)N, num_sets, kMaxSets);
     if (!jobs) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: sets is null");
@@ -767,6 +868,8 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
     if (N == 0) {
         for (int i = 0; i < num_sets; ++i) hipLaunchKernelGGL(init_counts_kernel, dim3(1), dim3(64), 0, s, sets.set[i].counts);
         S3D_HIP_CHECK(hipGetLastError());
+        for (int i = 0; host_counts && i < 4 * num_sets; ++i) host_counts[i] = 0;
+        if (counted) S3D_HIP_CHECK(hipEventRecord(counted, s));
         return S3D_OK;
     }
     if (!coords || !workspace) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: null device pointer");
@@ -782,7 +885,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
     uint64_t *scan = reinterpret_cast<uint64_t *>(base + L.scan);
     int2 *place = reinterpret_cast<int2 *>(base + L.place);
     uint64_t *keys = reinterpret_cast<uint64_t *>(base + L.keys);
-    size_t temp_bytes = L.temp_bytes;
+    CellSum *sums = reinterpret_cast<CellSum *>(base + L.sums);
     const int64_t num_cells = (L.cells_cap + 1) * num_sets;
     const unsigned per_set = static_cast<unsigned>(num_sets);
     const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)), per_set);
@@ -791,8 +894,11 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
     hipLaunchKernelGGL(grid_count_kernel, grid, dim3(kThreads), 0, s, coords, N, stride, sets, partials, L.cells_cap, plan,
                        cells, place);
     S3D_HIP_CHECK(hipGetLastError());
-    S3D_HIP_CHECK(rocprim::exclusive_scan(base + L.temp, temp_bytes, CellWordIterator(cells, CellWord()), scan, uint64_t(0),
-                                          static_cast<size_t>(num_cells), rocprim::plus<uint64_t>(), s));
+    const dim3 sum_grid(static_cast<unsigned>(ceil_div(L.cells_cap, kSumCells)), per_set);
+    hipLaunchKernelGGL(grid_sums_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums);
+    hipLaunchKernelGGL(grid_starts_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums, scan, host_counts);
+    S3D_HIP_CHECK(hipGetLastError());
+    if (counted) S3D_HIP_CHECK(hipEventRecord(counted, s));
     hipLaunchKernelGGL(grid_place_kernel, grid, dim3(kThreads), 0, s, place, N, sets, plan, scan, L.cells_cap, keys);
     S3D_HIP_CHECK(hipGetLastError());
     // about one window per wavefront if the windows hold 16 voxels on average, more in turn otherwise
@@ -802,6 +908,32 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
                        N, sets);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
+}
+
+}  // namespace
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
+    const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets, void *workspace,
+    size_t workspace_bytes, void *stream)
+{
+    return s3d::window_indices(coords, N, stride, sets, num_sets, nullptr, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_window_indices_counted(
+    const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets, int64_t *host_counts,
+    void *workspace, size_t workspace_bytes, void *stream)
+{
+    using namespace s3d;
+    if (!host_counts) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices_counted: host_counts is null");
+    hipEvent_t counted = nullptr;
+    S3D_HIP_CHECK(hipEventCreateWithFlags(&counted, hipEventDisableTiming));
+    int rc = window_indices(coords, N, stride, sets, num_sets, host_counts, counted, workspace, workspace_bytes, stream);
+    // (also after an error behind the launches: host_counts is the caller's again when this returns)
+    const hipError_t waited = hipEventSynchronize(counted);
+    if (rc == S3D_OK && waited != hipSuccess) rc = hip_fail(waited, "hipEventSynchronize");
+    (void)hipEventDestroy(counted);
+    return rc;
 }
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_window_index_grid_workspace_bytes(int64_t N)

@@ -71,8 +71,13 @@ def build_window_indices(coords, stride, window_size, shifts):
             job.window, job.shift = int(window), int(shift)
         ws_bytes = lib.s3d_window_indices_workspace_bytes(n, len(some))
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        status = lib.s3d_window_indices(coords.data_ptr(), n, int(stride), jobs, len(some), workspace.data_ptr(), ws_bytes,
-                                        _lib.stream(dev))
+        if first + len(some) < len(sets):
+            status = lib.s3d_window_indices(coords.data_ptr(), n, int(stride), jobs, len(some), workspace.data_ptr(), ws_bytes,
+                                            _lib.stream(dev))
+        else:
+            # (the last ones: the counts of all are there when this returns)
+            status = lib.s3d_window_indices_counted(coords.data_ptr(), n, int(stride), jobs, len(some), host.data_ptr(),
+                                                    workspace.data_ptr(), ws_bytes, _lib.stream(dev))
         _lib.check(status, "s3d_window_indices")
         rows = out[:, :n].unbind(0)
         return [rows[4 * i:4 * i + 4] for i in range(len(some))]
@@ -91,11 +96,13 @@ def build_window_indices(coords, stride, window_size, shifts):
         # the counting sort over the window lattice first; a set whose lattice is too large for it (bit 1 of its
         # status word) is built again by the sort of all voxels, at the price of a second wait
         if USE_GRID_PATH:
+            host = torch.empty((min(len(sets), GRID_SETS), 4), dtype=torch.int64, device="cpu", pin_memory=True)
             for first in range(0, len(sets), GRID_SETS):
                 outputs += enqueue_grid(first, sets[first:first + GRID_SETS])
+            host_counts = host.tolist() if 0 < len(sets) <= GRID_SETS else counts.tolist()
         else:
             outputs = [enqueue(i, window, shift) for i, (window, shift) in enumerate(sets)]
-        host_counts = counts.tolist()
+            host_counts = counts.tolist()
         redo = [i for i, c in enumerate(host_counts) if c[3] & 2]
         if redo:
             for i in redo:
