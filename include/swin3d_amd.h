@@ -229,6 +229,24 @@ int s3d_attn_bwd(const void *q, const void *k, const void *v, const void *table_
                  void *dk, void *dv, float *dtable_q, float *dtable_k, float *dtable_v, int64_t N,
                  int32_t H, int32_t D, int64_t W, int64_t pairs, int32_t dtype, void *workspace,
                  size_t workspace_bytes, void *stream);
+/*
+ * The same with rows of q, k, v `qkv_row_stride` and of dq, dk, dv `grad_row_stride` elements apart (multiples of 8, at
+ * least H*D, base addresses 16-byte aligned): slices of a projection's [N, 3 H D] output and of its gradient, in place.
+ * Other than H*D they need pairs > 0 and a shape that the forms with a pair store take (head_dim 8 or 16).
+ */
+int s3d_attn_bwd_strided(const void *q, const void *k, const void *v, const void *table_q, const void *table_k,
+                         const void *table_v, const int32_t *table_sizes, int32_t nd, int64_t table_len,
+                         const int32_t *w_sizes, const int32_t *w2n, const int32_t *n2n, const float *n_coords,
+                         const void *out, const float *out_max, const float *out_sum, const void *dout, void *dq,
+                         void *dk, void *dv, float *dtable_q, float *dtable_k, float *dtable_v, int64_t N,
+                         int32_t H, int32_t D, int64_t W, int64_t pairs, int64_t qkv_row_stride, int64_t grad_row_stride,
+                         int32_t dtype, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * Up to 16 arrays from fp32 to fp16 (round to nearest even, as a cast of the framework's), in one launch.
+ * from, to, counts: HOST arrays of device addresses and element counts.
+ */
+int s3d_cast_half(const float *const *from, void *const *to, const int64_t *counts, int32_t num, void *stream);
 
 /*
  * Window sort + segment offsets.

@@ -56,8 +56,12 @@ SIGNATURES = {
     # q k v tq tk tv sizes | nd len | w_sizes w2n n2n coords out max sum dout dq dk dv dtq dtk dtv | N H D W pairs dtype | ws bytes stream
     "s3d_attn_bwd": (ctypes.c_int, [_vp] * 7 + [_i32, _i64] + [_vp] * 14 +
                      [_i64, _i32, _i32, _i64, _i64, _i32, _vp, ctypes.c_size_t, _vp]),
+    # ... pairs, row strides of q, k, v and of dq, dk, dv, dtype ...
+    "s3d_attn_bwd_strided": (ctypes.c_int, [_vp] * 7 + [_i32, _i64] + [_vp] * 14 +
+                             [_i64, _i32, _i32, _i64, _i64, _i64, _i64, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_window_index_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_window_index": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),
+    "s3d_cast_half": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp]),
     "s3d_window_index_grid_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_window_index_grid": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),
     "s3d_window_indices_workspace_bytes": (ctypes.c_size_t, [_i64, _i32]),
@@ -118,6 +122,23 @@ def on(device):
 def stream(device):
     """The current stream of `device` as the library takes it."""
     return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def cast_half(tensors):
+    """fp32 CUDA tensors (of one device) in fp16, flat copies in one launch: [tensor of the same shape, contiguous]."""
+    done = []
+    for first in range(0, len(tensors), 16):
+        some = [t.contiguous() for t in tensors[first:first + 16]]
+        out = [torch.empty(t.shape, dtype=torch.float16, device=t.device) for t in some]
+        num = len(some)
+        sources, targets, counts = (ctypes.c_void_p * num)(), (ctypes.c_void_p * num)(), (ctypes.c_int64 * num)()
+        for i, (t, o) in enumerate(zip(some, out)):
+            sources[i], targets[i], counts[i] = t.data_ptr(), o.data_ptr(), t.numel()
+        with on(some[0].device):
+            status = lib().s3d_cast_half(sources, targets, counts, num, stream(some[0].device))
+        check(status, "s3d_cast_half")
+        done += out
+    return done
 
 
 def check(status, what):

@@ -48,6 +48,7 @@ struct BwdArgs {
     const float *out_max, *out_sum;
     const int32_t *w_sizes, *w2n, *n2n;
     const float *n_coords;
+    int64_t qkv_stride;  // elements between rows of q, k, v: H D but in the pair form
     void *dq, *dk, *dv;
     float *dtq, *dtk, *dtv;
     float *delta;     // [N,H] dout_i . o_i
@@ -637,6 +638,7 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
     // the streamed row of the first rank-1 update (k_j, q_i or, for the dTv half, dout_i) and of the second (KIND 1)
     const T *gx = static_cast<const T *>(KIND == 0 ? a.k : KIND == 3 ? a.dout : a.q);
     const T *gy = static_cast<const T *>(a.dout);
+    const int64_t stride_x = KIND == 3 ? HD : a.qkv_stride;
 
     // The rank-1 updates as 4x4x1 MFMAs wherever the VALU form would not fit the registers: the accumulators may
     // then live in accumulation registers.  Measured at head_dim 8 (us, VALU / MFMA form): fp16 with five 64-row
@@ -720,7 +722,7 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
         };
         auto fetch = [&](int it, int st_row, StepIn &in) {
             const int st = min(it * ng + grp, n_w - 1);
-            in.x.load(gx + static_cast<int64_t>(st_row) * HD + h * D);
+            in.x.load(gx + static_cast<int64_t>(st_row) * stride_x + h * D);
             if constexpr (kAccB) in.y.load(gy + static_cast<int64_t>(st_row) * HD + h * D);
 #pragma unroll
             for (int n = 0; n < ND; ++n) in.c[n] = a.n_coords[static_cast<int64_t>(s0 + st) * ND + n];
@@ -1312,15 +1314,17 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_attn_bwd_workspace_
     return need;
 }
 
-extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
+namespace s3d {
+namespace {
+
+int attn_bwd(
     const void *q, const void *k, const void *v, const void *table_q, const void *table_k,
     const void *table_v, const int32_t *table_sizes, int32_t nd, int64_t table_len,
     const int32_t *w_sizes, const int32_t *w2n, const int32_t *n2n, const float *n_coords, const void *out,
     const float *out_max, const float *out_sum, const void *dout, void *dq, void *dk, void *dv,
     float *dtable_q, float *dtable_k, float *dtable_v, int64_t N, int32_t H, int32_t D, int64_t W,
-    int64_t pairs, int32_t dtype, void *workspace, size_t workspace_bytes, void *stream)
+    int64_t pairs, int64_t qkv_stride, int64_t grad_stride, int32_t dtype, void *workspace, size_t workspace_bytes, void *stream)
 {
-    using namespace s3d;
     if (N < 0 || W < 0 || H < 1 || D < 1 || nd < 1 || table_len < 1 || pairs < 0)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_attn_bwd: bad sizes N=%lld W=%lld H=%d D=%d nd=%d table_len=%lld pairs=%lld",
                     (long long)N, (long long)W, H, D, nd, (long long)table_len, (long long)pairs);
@@ -1335,6 +1339,17 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
     if (dtype == S3D_DTYPE_F32_F16_ROWS && pairs == 0 && !general)
         return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: fp32 arithmetic on fp16 rows (dtype 2) needs the pair count; "
                     "without it pass fp32 copies of the rows with dtype 0");
+    const int64_t dense = static_cast<int64_t>(H) * D;
+    if (qkv_stride == 0) qkv_stride = dense;
+    if (grad_stride == 0) grad_stride = dense;
+    if (qkv_stride != dense || grad_stride != dense) {
+        if (pairs == 0 || general)
+            return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: rows %lld and %lld elements apart need the pair count and a shape of the pair form",
+                        (long long)qkv_stride, (long long)grad_stride);
+        if (qkv_stride < dense || grad_stride < dense || qkv_stride % 8 || grad_stride % 8 || qkv_stride > 0x7fffffffLL || grad_stride > 0x7fffffffLL)
+            return fail(S3D_ERR_BAD_SHAPE, "s3d_attn_bwd: rows %lld and %lld elements apart (multiples of 8, at least H*D = %lld)",
+                        (long long)qkv_stride, (long long)grad_stride, (long long)dense);
+    }
     if (!table_sizes) return fail(S3D_ERR_NULL_POINTER, "s3d_attn_bwd: table_sizes (host) is null");
     BwdArgs a{};
     a.H = H;
@@ -1343,6 +1358,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
     a.N = N;
     a.W = W;
     a.table_len = table_len;
+    a.qkv_stride = qkv_stride;
     if (int rc = fill_bwd_axes(a, table_sizes, nd, table_len)) return rc;
     if (!dtable_q || !dtable_k || !dtable_v)
         return fail(S3D_ERR_NULL_POINTER, "s3d_attn_bwd: null table-gradient pointer");
@@ -1406,7 +1422,8 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
         a.pd = pd;
         a.dl_t = dl_t;
         pr.f.q = q; pr.f.k = k; pr.f.v = v;
-        pr.f.row_stride = static_cast<int64_t>(H) * D;
+        pr.f.row_stride = qkv_stride;
+        pr.grad_stride = grad_stride;
         pr.f.table_q = table_q; pr.f.table_k = table_k; pr.f.table_v = table_v;
         pr.f.w_sizes = w_sizes; pr.f.w2n = w2n; pr.f.n2n = n2n;
         pr.f.n_coords = n_coords;
@@ -1437,4 +1454,38 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
     S3D_BWD_CASE(16, 3) S3D_BWD_CASE(16, 6) S3D_BWD_CASE(16, 9)
 #undef S3D_BWD_CASE
     return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: D=%d nd=%d", D, nd);
+}
+
+}  // namespace
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd(
+    const void *q, const void *k, const void *v, const void *table_q, const void *table_k,
+    const void *table_v, const int32_t *table_sizes, int32_t nd, int64_t table_len,
+    const int32_t *w_sizes, const int32_t *w2n, const int32_t *n2n, const float *n_coords, const void *out,
+    const float *out_max, const float *out_sum, const void *dout, void *dq, void *dk, void *dv,
+    float *dtable_q, float *dtable_k, float *dtable_v, int64_t N, int32_t H, int32_t D, int64_t W,
+    int64_t pairs, int32_t dtype, void *workspace, size_t workspace_bytes, void *stream)
+{
+    return s3d::attn_bwd(q, k, v, table_q, table_k, table_v, table_sizes, nd, table_len, w_sizes, w2n, n2n, n_coords, out, out_max,
+                         out_sum, dout, dq, dk, dv, dtable_q, dtable_k, dtable_v, N, H, D, W, pairs, 0, 0, dtype, workspace,
+                         workspace_bytes, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_attn_bwd_strided(
+    const void *q, const void *k, const void *v, const void *table_q, const void *table_k,
+    const void *table_v, const int32_t *table_sizes, int32_t nd, int64_t table_len,
+    const int32_t *w_sizes, const int32_t *w2n, const int32_t *n2n, const float *n_coords, const void *out,
+    const float *out_max, const float *out_sum, const void *dout, void *dq, void *dk, void *dv,
+    float *dtable_q, float *dtable_k, float *dtable_v, int64_t N, int32_t H, int32_t D, int64_t W,
+    int64_t pairs, int64_t qkv_row_stride, int64_t grad_row_stride, int32_t dtype, void *workspace, size_t workspace_bytes,
+    void *stream)
+{
+    using namespace s3d;
+    if (qkv_row_stride < 1 || grad_row_stride < 1)
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_attn_bwd_strided: rows %lld and %lld elements apart", (long long)qkv_row_stride,
+                    (long long)grad_row_stride);
+    return attn_bwd(q, k, v, table_q, table_k, table_v, table_sizes, nd, table_len, w_sizes, w2n, n2n, n_coords, out, out_max, out_sum,
+                    dout, dq, dk, dv, dtable_q, dtable_k, dtable_v, N, H, D, W, pairs, qkv_row_stride, grad_row_stride, dtype,
+                    workspace, workspace_bytes, stream);
 }

@@ -74,7 +74,8 @@ struct BwdPairArgs {
     AttnArgs f;                  // shape, q, k, v, tables, index arrays (n2n required), rows[] / base[], workspace
     const void *dout;            // [N,H,D]
     const float *stat_max, *stat_sum, *delta;   // [N,H]: the forward's statistics, dout_i . o_i
-    void *dq, *dk, *dv;          // [N,H,D]
+    void *dq, *dk, *dv;          // [N,H,D], rows `grad_stride` elements apart (q, k, v: f.row_stride)
+    int64_t grad_stride;
     const int64_t *pos_base;     // [N]: at a window's first sorted position, the pairs of the windows before it
     float2 *pd;                  // [H][pairs]: (dL, P) at base + i n + j  (i, j: query, key position inside the window)
     float *dl_t;                 // [H][pairs]: dL at base + j n + i

@@ -35,6 +35,7 @@ struct StripArgs {
     const float *scales;        // [head][Tq, Tk, Tv]: what a product with the table's operand is multiplied by
     float *slots;               // [workgroup][kind][tile][lane][4]: table gradients as the products leave them
     void *dq, *dk, *dv;
+    uint32_t grad_stride;       // elements between rows of dq, dk, dv (of q, k, v: f.row_stride)
     float *dtq, *dtk, *dtv;
     float half_rows[kMaxAxes], upper[kMaxAxes];    // what crse_row takes (made here, they would take two vector registers an axis)
 };

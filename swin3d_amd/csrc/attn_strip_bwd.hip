@@ -240,6 +240,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int H = a.H, HD = H * D;
+    const uint32_t stride = static_cast<uint32_t>(a.row_stride);       // of q, k, v
     const int h = static_cast<int>(blockIdx.x) % H;
     const int group = static_cast<int>(blockIdx.x) / H, groups = static_cast<int>(gridDim.x) / H;
     const int strips = b.list.total[1];
@@ -307,7 +308,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     auto pair_step = [&](int4 column, int n) { return column.w < 0 ? 0 : kByKey ? 1 : n; };
     auto fetch = [&](int n) {
         if (wave < kKinds)
-            ahead.x.load((wave == 0 ? gx : gd) + (static_cast<uint64_t>(static_cast<uint32_t>(ahead.column.y)) * static_cast<uint32_t>(HD) + 4 * g4));
+            ahead.x.load((wave == 0 ? gx : gd) + (static_cast<uint64_t>(static_cast<uint32_t>(ahead.column.y)) *
+                                                  (wave == 0 ? stride : static_cast<uint32_t>(HD)) + 4 * g4));
         const int first = pair_at(ahead.column, n), step = pair_step(ahead.column, n);
 #pragma unroll
         for (int s = 0; s < kKept; ++s) ahead.kept[s] = records[first + min(reach0 + s * kStripReach, n - 1) * step];
@@ -384,9 +386,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         // what the products of the pairs themselves start with, while the histograms are filled
         Raw4<TF> y, z;
         auto fetch_keys = [&](int row) {
-            const uint64_t at = static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(HD) + 4 * g4;
-            y.load(gy + at);
-            if constexpr (kByKey) z.load(gd + at);
+            y.load(gy + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * stride + 4 * g4));
+            if constexpr (kByKey) z.load(gd + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(HD) + 4 * g4));
         };
         fetch_keys(key_row);
 
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = static_cast<float>(sums[e]) * (which > 0 ? 1.0f / kLiftP<TF> : 1.0f);
-            if (there) store4(static_cast<TF *>(which > 0 ? b.dv : kByKey ? b.dk : b.dq) + static_cast<int64_t>(own_row) * HD + h * D + g4 * 4, o);
+            if (there) store4(static_cast<TF *>(which > 0 ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * D + g4 * 4, o);
         }
     }
     // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]

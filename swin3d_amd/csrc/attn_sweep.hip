@@ -848,13 +848,13 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
         float ci[ND], res_x[HP][D], res_y[kKeyOwned ? HP : 1][D];
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
-            const int64_t at_row = static_cast<int64_t>(own_row) * HD + (h + hh) * D;
+            const int64_t at_row = static_cast<int64_t>(own_row) * a.row_stride + (h + hh) * D;
             if constexpr (kKeyOwned) {
                 own_x[hh].load(gk + at_row);
                 if constexpr (!kRead) own_y[hh].load(gv + at_row);
             } else {
                 own_x[hh].load(gq + at_row);
-                own_y[hh].load(ggo + at_row);
+                own_y[hh].load(ggo + static_cast<int64_t>(own_row) * HD + (h + hh) * D);
                 own_m[hh] = b.stat_max[static_cast<int64_t>(own_row) * H + h + hh];
                 own_inv[hh] = 1.0f / b.stat_sum[static_cast<int64_t>(own_row) * H + h + hh];
                 own_delta[hh] = b.delta[static_cast<int64_t>(own_row) * H + h + hh];
@@ -882,14 +882,15 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
             float st_m[HP], st_inv[HP], st_delta[HP];
 #pragma unroll
             for (int hh = 0; hh < HP; ++hh) {
-                const int64_t at_row = static_cast<int64_t>(st_row) * HD + (h + hh) * D;
+                const int64_t at_row = static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D;
+                const int64_t at_grad = static_cast<int64_t>(st_row) * HD + (h + hh) * D;
                 if constexpr (kRead) {
                     st_x[hh].load(gq + at_row);
-                    st_y[hh].load(ggo + at_row);
+                    st_y[hh].load(ggo + at_grad);
                     st_m[hh] = st_inv[hh] = st_delta[hh] = 0.0f;
                 } else if constexpr (kKeyOwned) {
                     st_x[hh].load(gq + at_row);
-                    st_y[hh].load(ggo + at_row);
+                    st_y[hh].load(ggo + at_grad);
                     st_m[hh] = b.stat_max[static_cast<int64_t>(st_row) * H + h + hh];
                     st_inv[hh] = b.stat_sum[static_cast<int64_t>(st_row) * H + h + hh];
                     st_delta[hh] = b.delta[static_cast<int64_t>(st_row) * H + h + hh];
@@ -992,7 +993,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
                         for (int c = 0; c < D; ++c) res_y[hh][c] = __int_as_float(0x7fc00000);
                     }
                 }
-                const int64_t at_row = static_cast<int64_t>(own_row) * HD + (h + hh) * D;
+                const int64_t at_row = static_cast<int64_t>(own_row) * b.grad_stride + (h + hh) * D;
                 if constexpr (kKeyOwned) {
                     store_row<D>(static_cast<TF *>(b.dk) + at_row, res_x[hh]);
                     store_row<D>(static_cast<TF *>(b.dv) + at_row, res_y[hh]);

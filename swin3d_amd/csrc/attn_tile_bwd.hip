@@ -145,6 +145,7 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int H = a.H, HD = H * D;
+    const uint64_t stride = static_cast<uint32_t>(a.row_stride);      // of q, k, v
     const int h = static_cast<int>(blockIdx.x) % H;
     const int group = static_cast<int>(blockIdx.x) / H, groups = static_cast<int>(gridDim.x) / H;
     const int total_units = b.list.total[0];
@@ -194,12 +195,12 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
             Operand<TF> feat, grad, x_k, x_v;
             {
                 const uint64_t row = static_cast<uint32_t>(b.rows[(wave < 4 ? u : other) * kCols + tile_c * 32 + m32]);
-                feat.load((wave < 4 ? gq : gk) + row * HD + channel);
+                feat.load((wave < 4 ? gq : gk) + row * stride + channel);
                 if (wave < 4) {
                     const uint64_t key_row = static_cast<uint32_t>(b.rows[other * kCols + tile_r * 32 + m32]);
                     grad.load(gd + row * HD + channel);
-                    x_k.load(gk + key_row * HD + channel);
-                    x_v.load(gv + key_row * HD + channel);
+                    x_k.load(gk + key_row * stride + channel);
+                    x_v.load(gv + key_row * stride + channel);
                 }
             }
             float x[ND];
@@ -405,6 +406,7 @@ int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, floa
     g.scales = b.scales;
     g.slots = slots;
     g.dq = p.dq; g.dk = p.dk; g.dv = p.dv;
+    g.grad_stride = static_cast<uint32_t>(p.grad_stride);
     g.dtq = dtq; g.dtk = dtk; g.dtv = dtv;
     return tile::launch_strip_gradients(g, dtype, stream);
 }

@@ -303,8 +303,15 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
     store above BWD_PAIR_STORE_MAX_BYTES, selects the fused sweeps, which need no such store and take about a
     third longer.  head_dim 32 and tables of more than BWD_MAX_ROWS_PER_AXIS rows per axis on average run in the
     library's general form (atomic adds, as the reference works): correct, some fifty times slower per pair."""
+    return _attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w_sizes, w2n, n2n, n_coords, out, out_max, out_sum,
+                               dout, pairs, False)
+
+
+def _attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w_sizes, w2n, n2n, n_coords, out, out_max, out_sum, dout,
+                        pairs, strided):
+    """window_attention_backward; strided: q, k, v may be views with rows apart, as the forward takes them."""
     w_sizes_in = w_sizes
-    _require_cuda("query", q)
+    _require_cuda("query", q, strided_rows=strided)
     dev = q.device
     if q.dim() != 3:
         raise ValueError(f"query must be [N,H,D], got {tuple(q.shape)}")
@@ -312,7 +319,7 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
     if q.dtype not in _DTYPE_CODE:
         raise TypeError(f"unsupported feature dtype {q.dtype} (float16 or float32)")
     for name, t in (("key", k), ("value", v), ("out", out), ("dout", dout)):
-        _require_cuda(name, t, dev)
+        _require_cuda(name, t, dev, strided_rows=strided and name in ("key", "value"))
         if t.shape != q.shape or t.dtype != q.dtype:
             raise ValueError(f"{name} must match query: {tuple(t.shape)} {t.dtype}")
     if d not in BWD_HEAD_DIMS:
@@ -357,21 +364,29 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
         # the fused sweeps take one dtype: fp32 copies of the features, the gradients rounded afterwards
         q, k, v, out, dout = (t.float() for t in (q, k, v, out, dout))
         code = _lib.S3D_DTYPE_F32
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
+    dq, dk, dv = (torch.empty((n, h, d), dtype=q.dtype, device=dev) for _ in range(3))
     dtq, dtk, dtv = (torch.empty(table_len, dtype=torch.float32, device=dev) for _ in range(3))
     lib = _lib.lib()
-    tensors = [t.contiguous() for t in (q, k, v, table_q, table_k, table_v)]
+    # the forms with a pair store read q, k, v in place when they share one row stride
+    row_stride = h * d
+    if pairs > 0 and not general:
+        strides = [_row_stride(t) for t in (q, k, v)]
+        if None not in strides and strides[0] == strides[1] == strides[2]:
+            row_stride = strides[0]
+    if row_stride == h * d:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    tensors = [q, k, v] + [t.contiguous() for t in (table_q, table_k, table_v)]
     out, dout, out_max, out_sum, n_coords = (t.contiguous() for t in (out, dout, out_max, out_sum, n_coords))
     with _lib.on(dev):
         ws_bytes = lib.s3d_attn_bwd_workspace_bytes(h, d, nd, table_len, n, w_sizes.numel(), pairs)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         stream = _lib.stream(dev)
-        status = lib.s3d_attn_bwd(
+        status = lib.s3d_attn_bwd_strided(
             *(t.data_ptr() for t in tensors), c_sizes, nd, table_len, w_sizes.data_ptr(), w2n.data_ptr(),
             None if n2n is None else n2n.data_ptr(), n_coords.data_ptr(), out.data_ptr(), out_max.data_ptr(),
             out_sum.data_ptr(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dtq.data_ptr(), dtk.data_ptr(),
-            dtv.data_ptr(), n, h, d, w_sizes.numel(), pairs, code, workspace.data_ptr(), ws_bytes,
-            stream)
+            dtv.data_ptr(), n, h, d, w_sizes.numel(), pairs, row_stride, h * d, code, workspace.data_ptr(),
+            ws_bytes, stream)
     _lib.check(status, "s3d_attn_bwd")
     if mixed and code == _lib.S3D_DTYPE_F32:
         dq, dk, dv = dq.half(), dk.half(), dv.half()
@@ -383,6 +398,14 @@ def _compute_dtype(precision):
     if torch.is_autocast_enabled() and precision != PrecisionMode.HALF_NONE:
         return torch.get_autocast_dtype("cuda")
     return torch.float32
+
+
+def _tables_as(tables, dtype):
+    """The tables in `dtype`, contiguous; fp32 ones in fp16 by one launch."""
+    if dtype == torch.float16 and all(t.dtype == torch.float32 and t.is_cuda and t.device == tables[0].device and t.numel() > 0
+                                      for t in tables):
+        return _lib.cast_half(tables)
+    return [t.to(dtype).contiguous() for t in tables]
 
 
 class SelfAttnAIOFunction(Function):
@@ -407,7 +430,7 @@ class SelfAttnAIOFunction(Function):
         if None in strides:
             feats = [t.contiguous() if s is None else t for t, s in zip(feats, strides)]
             strides = [_row_stride(t) for t in feats]
-        tables = [t.to(c_dtype).contiguous() for t in raw[3:]]
+        tables = _tables_as(raw[3:], c_dtype)
         n_coords = n_coords.to(torch.float32).contiguous()
         needs_grad = any(ctx.needs_input_grad[:6])
         if needs_grad:
@@ -430,7 +453,8 @@ class SelfAttnAIOFunction(Function):
         # the window set's pair count, for the backward's pair store: on the tensor when the window index of this
         # package built it, else read from w_sizes once (and kept on it)
         ctx.pairs = _pairs_of(w_sizes, w_sizes) if BWD_PAIR_STORE else 0
-        ctx.save_for_backward(out, omax, osum, *raw, w_sizes, w2n, n2n, n_coords)
+        # (tables as the forward took them: a backward in the same type needs no casts of its own)
+        ctx.save_for_backward(out, omax, osum, *raw, w_sizes, w2n, n2n, n_coords, *tables)
         return out
 
     @staticmethod
@@ -438,9 +462,10 @@ class SelfAttnAIOFunction(Function):
         """Compute dtype as in the reference (attn_coff.py:206-215): the gradient's dtype for HALF_ALL,
         fp32 otherwise; the statistics saved by the forward are reused either way."""
         (dout,) = grad_outputs
-        out, omax, osum = ctx.saved_tensors[:3]
-        raw = ctx.saved_tensors[3:9]
-        w_sizes, w2n, n2n, n_coords = ctx.saved_tensors[9:]
+        saved = ctx.saved_tensors
+        out, omax, osum = saved[:3]
+        raw, tables = saved[3:9], saved[13:]
+        w_sizes, w2n, n2n, n_coords = saved[9:13]
         c_dtype = dout.dtype if ctx.precision == PrecisionMode.HALF_ALL else torch.float32
         if c_dtype not in _DTYPE_CODE:
             raise NotImplementedError(f"compute dtype {c_dtype} is not supported (float16 / float32)")
@@ -450,11 +475,12 @@ class SelfAttnAIOFunction(Function):
         if c_dtype == torch.float32 and dout.dtype == torch.float16 and out.dtype == torch.float16 \
                 and all(t.dtype == torch.float16 for t in raw[:3]):
             f_dtype = torch.float16
-        feats = [t.to(f_dtype).contiguous() for t in raw[:3]]
-        tables = [t.to(c_dtype).contiguous() for t in raw[3:]]
-        grads = window_attention_backward(*feats, *tables, ctx.table_sizes, w_sizes, w2n, n2n, n_coords,
-                                          out.to(f_dtype), omax, osum, dout.to(f_dtype).contiguous(),
-                                          pairs=ctx.pairs)
+        feats = [t.to(f_dtype) for t in raw[:3]]
+        feats = [t.contiguous() if _row_stride(t) is None else t for t in feats]
+        if any(t.dtype != c_dtype for t in tables):
+            tables = _tables_as(raw[3:], c_dtype)
+        grads = _attention_backward(*feats, *tables, ctx.table_sizes, w_sizes, w2n, n2n, n_coords, out.to(f_dtype), omax, osum,
+                                    dout.to(f_dtype).contiguous(), ctx.pairs, True)
         grads = [g.to(t.dtype).reshape(t.shape) if need else None
                  for g, t, need in zip(grads, raw, ctx.needs_input_grad[:6])]
         return (*grads, None, None, None, None, None, None)
