@@ -339,6 +339,30 @@ int s3d_cell_representatives(const int32_t *n2n, const int32_t *w2n, const int32
  */
 int s3d_key_neighbours(const int64_t *sorted_keys, const int64_t *order, int64_t N, const int64_t *deltas, int32_t M,
                        int64_t *out, void *stream);
+/*
+ * The 27 neighbours (x first, then y, z; the voxel itself among them) of every voxel on a lattice of `stride`, from keys
+ * as s3d_pack_keys makes them (ascending: sorted_keys, order as for s3d_key_neighbours): out [N][27], N where there is none.
+ */
+int s3d_lattice_neighbours(const int64_t *sorted_keys, const int64_t *order, int64_t N, int32_t field, int32_t stride,
+                           int64_t *out, void *stream);
+/* key of every voxel (batch, x, y, z): ascending in this order for coordinates of less than 2^(field - 1) either side */
+int s3d_pack_keys(const int32_t *coords, int64_t N, int32_t field, int64_t *out, void *stream);
+/* out int32 [B]: how many of the N ascending batch ids (`stride` apart) are at most b */
+int s3d_segment_ends(const int32_t *batch, int64_t stride, int64_t N, int32_t B, int32_t *out, void *stream);
+/*
+ * The next coarser level from a sort of the voxels into its cells: what s3d_cell_representatives gives (pick), the cells'
+ * coordinates (int32 [W][4], rounded down to multiples of `step`) and the picked rows' signals (fp32 [W][num_signals]).
+ */
+int s3d_pool_cells(const int32_t *n2n, const int32_t *w2n, const int32_t *w_sizes, int64_t W, const int32_t *coords,
+                   int32_t step, const float *signals, int64_t signals_stride, int32_t num_signals, int64_t *pick,
+                   int32_t *out_coords, float *out_signals, void *stream);
+/*
+ * s3d_window_signals from a level's voxels and signals (batch, x, y, z in voxel units, num_signals others): the position
+ * inside a voxel is (signal - coordinate) times the reciprocal of the stride.
+ */
+int s3d_level_signals(const int32_t *w_w_id, const int32_t *n2n, const int32_t *coords, int32_t stride, const float *signals,
+                      int64_t signals_stride, int32_t num_signals, int32_t window, float xyz_scale, float other_scale,
+                      float *out, int64_t N, void *stream);
 
 /*
  * Signal matrix of the attention op in window-sorted order (the `n_coords` argument of s3d_attn_fwd), one pass.
@@ -385,6 +409,10 @@ int s3d_knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz,
             float *ret_dist2, float cell_size, void *workspace, size_t workspace_bytes,
             void *stream);
 /* The same with Euclidean distances (the square roots, sqrt(S3D_KNN_PAD_DIST2) for padded slots) in ret_dist. */
+/* ... with rows of three coordinates src_stride and query_stride floats apart (columns of a wider matrix), in place. */
+int s3d_knn_strided(int32_t K, const float *src_xyz, int64_t src_stride, int64_t Ns, const float *query_xyz,
+                    int64_t query_stride, int64_t Nq, const int32_t *src_offset, const int32_t *query_offset, int32_t B,
+                    int32_t *ret_idx, float *ret_dist2, float cell_size, void *workspace, size_t workspace_bytes, void *stream);
 int s3d_knn_distances(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int64_t Nq,
                       const int32_t *src_offset, const int32_t *query_offset, int32_t B, int32_t *ret_idx,
                       float *ret_dist, float cell_size, void *workspace, size_t workspace_bytes, void *stream);

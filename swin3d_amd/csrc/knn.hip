@@ -79,7 +79,7 @@ __device__ __forceinline__ float ordered_to_float(int i)
 
 // Bounding box of the sources, one partial box per workgroup (no atomics, nothing to initialise), and the cell
 // counters set to zero: a small grid-stride grid.
-__global__ __launch_bounds__(kThreads) void knn_bbox_kernel(const float *__restrict__ src, int64_t Ns,
+__global__ __launch_bounds__(kThreads) void knn_bbox_kernel(const float *__restrict__ src, int64_t stride, int64_t Ns,
                                                             int32_t *__restrict__ partials,
                                                             int32_t *__restrict__ counts, int64_t cells)
 {
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void knn_bbox_kernel(const float *__restr
          i += static_cast<int64_t>(gridDim.x) * kThreads) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const int o = float_to_ordered(src[i * 3 + a]);
+            const int o = float_to_ordered(src[i * stride + a]);
             lo[a] = min(lo[a], o);
             hi[a] = max(hi[a], o);
         }
@@ -265,7 +265,7 @@ template <int kWaves> __device__ __forceinline__ void reduce_box(int *v, int (*p
 // source's cell and its slot there, drawn from the cell's counter.  Neighbouring lanes that fall into the same
 // cell (sources usually arrive in lattice order) draw one run of slots with one atomic.
 __global__ __launch_bounds__(kThreads) void knn_count_kernel(
-    const float *__restrict__ src, int64_t Ns, const int32_t *__restrict__ src_offset, int B,
+    const float *__restrict__ src, int64_t stride, int64_t Ns, const int32_t *__restrict__ src_offset, int B,
     const int32_t *__restrict__ partials, int boxes, int K, float cell_hint, int64_t cells_cap,
     KnnPlan *__restrict__ plan_out,
     int32_t *__restrict__ counts, int2 *__restrict__ src_place)
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kThreads) void knn_count_kernel(
     float own[3] = {0.0f, 0.0f, 0.0f};
     if (i < Ns)
 #pragma unroll
-        for (int a = 0; a < 3; ++a) own[a] = src[i * 3 + a];
+        for (int a = 0; a < 3; ++a) own[a] = src[i * stride + a];
     {
         int v[6];
 #pragma unroll
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kStartThreads) void knn_starts_kernel(const KnnPlan
 constexpr int kSmallThreads = 1024, kSmallEach = 4, kSmallSources = kSmallThreads * kSmallEach;
 constexpr size_t small_lds(int64_t cells_cap) { return sizeof(int32_t) * static_cast<size_t>(cells_cap); }
 __global__ __launch_bounds__(kSmallThreads) void knn_small_grid_kernel(
-    const float *__restrict__ src, int Ns, const int32_t *__restrict__ src_offset, int B, int K, float cell_hint, int cells_cap,
+    const float *__restrict__ src, int64_t stride, int Ns, const int32_t *__restrict__ src_offset, int B, int K, float cell_hint, int cells_cap,
     KnnPlan *__restrict__ plan_out, int32_t *__restrict__ starts, float4 *__restrict__ sorted)
 {
     extern __shared__ int counts[];
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(kSmallThreads) void knn_small_grid_kernel(
         if (k * kSmallThreads >= Ns) break;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            p[k][a] = i < Ns ? src[i * 3 + a] : 0.0f;
+            p[k][a] = i < Ns ? src[i * stride + a] : 0.0f;
             const int o = float_to_ordered(p[k][a]);
             v[a] = i < Ns ? min(v[a], o) : v[a];
             v[3 + a] = i < Ns ? max(v[3 + a], o) : v[3 + a];
@@ -480,14 +480,14 @@ __global__ __launch_bounds__(kSmallThreads) void knn_small_grid_kernel(
 }
 
 __global__ __launch_bounds__(kThreads) void knn_scatter_kernel(
-    const float *__restrict__ src, int64_t Ns, const int2 *__restrict__ src_place,
+    const float *__restrict__ src, int64_t stride, int64_t Ns, const int2 *__restrict__ src_place,
     const int32_t *__restrict__ starts, float4 *__restrict__ sorted)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= Ns) return;
     const int2 place = src_place[i];
     if (place.x < 0) return;
-    sorted[starts[place.x] + place.y] = make_float4(src[i * 3], src[i * 3 + 1], src[i * 3 + 2],
+    sorted[starts[place.x] + place.y] = make_float4(src[i * stride], src[i * stride + 1], src[i * stride + 2],
                                                     __int_as_float(static_cast<int>(i)));
 }
 
@@ -562,7 +562,7 @@ template <int SIZE> __device__ __forceinline__ void order(uint64_t &x, int t)
 constexpr int64_t kFewQueries = 200000;
 template <int G, int KMAX>
 __global__ __launch_bounds__(kThreads) void knn_query_kernel(
-    int K, const float *__restrict__ qry, int64_t Nq, const int32_t *__restrict__ query_offset,
+    int K, const float *__restrict__ qry, int64_t stride, int64_t Nq, const int32_t *__restrict__ query_offset,
     int B, const KnnPlan *__restrict__ plan_ptr, const int32_t *__restrict__ starts,
     const float4 *__restrict__ sorted, int32_t *__restrict__ ret_idx, float *__restrict__ ret_dist, bool squared)
 {
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(kThreads) void knn_query_kernel(
     uint64_t best = kNone;
     const int b = find_batch(query_offset, B, g);
     if (b < B && plan.src_end > 0) {
-        const float qx = qry[g * 3], qy = qry[g * 3 + 1], qz = qry[g * 3 + 2];
+        const float qx = qry[g * stride], qy = qry[g * stride + 1], qz = qry[g * stride + 2];
         const float qp[3] = {qx, qy, qz};
         int qc[3], r_first = 1, r_last = 0;
 #pragma unroll
@@ -887,12 +887,15 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_knn_workspace_bytes
 namespace s3d {
 namespace {
 
-int knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int64_t Nq, const int32_t *src_offset,
+int knn(int32_t K, const float *src_xyz, int64_t src_stride, int64_t Ns, const float *query_xyz, int64_t query_stride, int64_t Nq,
+        const int32_t *src_offset,
         const int32_t *query_offset, int32_t B, int32_t *ret_idx, float *ret_dist, bool squared, float cell_size,
         void *workspace, size_t workspace_bytes, void *stream)
 {
     if (K < 1 || K > S3D_KNN_KMAX)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_knn: K=%d outside 1..%d", K, S3D_KNN_KMAX);
+    if (src_stride < 3 || query_stride < 3)
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_knn: rows %lld and %lld floats apart", (long long)src_stride, (long long)query_stride);
     if (Ns < 0 || Nq < 0 || Ns > 0x7fffffffLL || Nq > 0x3fffffffLL || B < 1 || B > kMaxBatch)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_knn: Ns=%lld Nq=%lld B=%d out of range", (long long)Ns,
                     (long long)Nq, B);
@@ -917,18 +920,18 @@ int knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int
     if (Ns > kSmallSources) {
         // bounding box + zeroed counters, places (grid derived in every workgroup), starts, scatter
         const dim3 sgrid(static_cast<unsigned>(ceil_div(Ns, kThreads)));
-        hipLaunchKernelGGL(knn_bbox_kernel, dim3(kBboxBlocks), dim3(kThreads), 0, s, src_xyz, Ns, partials, counts, cells);
-        hipLaunchKernelGGL(knn_count_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, Ns, src_offset, B, partials,
+        hipLaunchKernelGGL(knn_bbox_kernel, dim3(kBboxBlocks), dim3(kThreads), 0, s, src_xyz, src_stride, Ns, partials, counts, cells);
+        hipLaunchKernelGGL(knn_count_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, src_stride, Ns, src_offset, B, partials,
                            kBboxBlocks, K, cell_size, L.cells_cap, plan, counts, src_place);
         // (workgroups: a share of whole rows is at least half of kStartCells, or a single row)
         hipLaunchKernelGGL(knn_starts_kernel, dim3(static_cast<unsigned>(2 * cells / kStartCells + 1)), dim3(kStartThreads), 0, s, plan, B,
                            counts, starts, partials + 6 * kBboxBlocks);
-        hipLaunchKernelGGL(knn_scatter_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, Ns, src_place, starts, sorted);
+        hipLaunchKernelGGL(knn_scatter_kernel, sgrid, dim3(kThreads), 0, s, src_xyz, src_stride, Ns, src_place, starts, sorted);
         S3D_HIP_CHECK(hipGetLastError());
     } else if (Ns > 0) {
         const size_t lds = small_lds(cells);
         if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(knn_small_grid_kernel), small_lds(cells_cap_for(kSmallSources)))) return rc;
-        hipLaunchKernelGGL(knn_small_grid_kernel, dim3(1), dim3(kSmallThreads), lds, s, src_xyz, static_cast<int>(Ns), src_offset, B, K,
+        hipLaunchKernelGGL(knn_small_grid_kernel, dim3(1), dim3(kSmallThreads), lds, s, src_xyz, src_stride, static_cast<int>(Ns), src_offset, B, K,
                            cell_size, static_cast<int>(cells), plan, starts, sorted);
         S3D_HIP_CHECK(hipGetLastError());
     } else {
@@ -943,7 +946,7 @@ int knn(int32_t K, const float *src_xyz, int64_t Ns, const float *query_xyz, int
     const dim3 qgrid(static_cast<unsigned>(ceil_div(Nq * G, kThreads)));
     auto query = G == 4 ? knn_query_kernel<4, 4> : G == 8 ? knn_query_kernel<8, 8> : G == 64 ? knn_query_kernel<64, 64>
                  : K <= 4 ? knn_query_kernel<16, 4> : K <= 8 ? knn_query_kernel<16, 8> : knn_query_kernel<16, 16>;
-    hipLaunchKernelGGL(query, qgrid, dim3(kThreads), 0, s, K, query_xyz, Nq, query_offset, B, plan, starts, sorted, ret_idx,
+    hipLaunchKernelGGL(query, qgrid, dim3(kThreads), 0, s, K, query_xyz, query_stride, Nq, query_offset, B, plan, starts, sorted, ret_idx,
                        ret_dist, squared);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -957,8 +960,17 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn(
     const int32_t *query_offset, int32_t B, int32_t *ret_idx, float *ret_dist2, float cell_size, void *workspace,
     size_t workspace_bytes, void *stream)
 {
-    return s3d::knn(K, src_xyz, Ns, query_xyz, Nq, src_offset, query_offset, B, ret_idx, ret_dist2, true, cell_size, workspace,
+    return s3d::knn(K, src_xyz, 3, Ns, query_xyz, 3, Nq, src_offset, query_offset, B, ret_idx, ret_dist2, true, cell_size, workspace,
                     workspace_bytes, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_knn_strided(
+    int32_t K, const float *src_xyz, int64_t src_stride, int64_t Ns, const float *query_xyz, int64_t query_stride, int64_t Nq,
+    const int32_t *src_offset, const int32_t *query_offset, int32_t B, int32_t *ret_idx, float *ret_dist2, float cell_size,
+    void *workspace, size_t workspace_bytes, void *stream)
+{
+    return s3d::knn(K, src_xyz, src_stride, Ns, query_xyz, query_stride, Nq, src_offset, query_offset, B, ret_idx, ret_dist2, true,
+                    cell_size, workspace, workspace_bytes, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_knn_distances(
@@ -966,7 +978,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn_distances(
     const int32_t *query_offset, int32_t B, int32_t *ret_idx, float *ret_dist, float cell_size, void *workspace,
     size_t workspace_bytes, void *stream)
 {
-    return s3d::knn(K, src_xyz, Ns, query_xyz, Nq, src_offset, query_offset, B, ret_idx, ret_dist, false, cell_size, workspace,
+    return s3d::knn(K, src_xyz, 3, Ns, query_xyz, 3, Nq, src_offset, query_offset, B, ret_idx, ret_dist, false, cell_size, workspace,
                     workspace_bytes, stream);
 }
 

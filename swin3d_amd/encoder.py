@@ -26,7 +26,7 @@ anything in the reference; here pooled voxels are sorted by (batch, x, y, z) and
 the lower row.  Stochastic depth is inference-time identity.
 """
 from dataclasses import dataclass
-from functools import partial
+from functools import lru_cache, partial
 
 import torch
 import torch.nn as nn
@@ -67,6 +67,19 @@ def pack_coords(coords):
     return key
 
 
+def _plain_coords(coords):
+    """Voxel coordinates that the geometry kernels read by address."""
+    return (coords.is_cuda and data_only(coords) and coords.dtype == torch.int32 and coords.dim() == 2 and coords.shape[1] == 4
+            and coords.is_contiguous() and coords.data_ptr() % 16 == 0)
+
+
+def _plain_signals(signals):
+    """... and signal rows."""
+    return (signals.is_cuda and data_only(signals) and signals.dtype == torch.float32 and signals.dim() == 2
+            and signals.shape[1] >= 4 and signals.stride(1) == 1 and signals.stride(0) >= signals.shape[1]
+            and not signals.requires_grad)
+
+
 def lookup_rows(sorted_keys, order, query_keys):
     """row of every query key in the voxel set described by (sorted_keys, order); -1 if absent."""
     pos = torch.searchsorted(sorted_keys, query_keys).clamp_(max=sorted_keys.numel() - 1)
@@ -80,6 +93,17 @@ def conv3x3x3_neighbours(coords, stride):
     neighbour's key is the voxel's key plus a constant per offset; taken in sorted key order the 27 query lists are
     sorted themselves, which keeps the binary searches local."""
     n = coords.shape[0]
+    if _plain_coords(coords) and n > 0:
+        dev = coords.device
+        keys = torch.empty(n, dtype=torch.long, device=dev)
+        out = torch.empty((n, 27), dtype=torch.long, device=dev)
+        with _lib.on(dev):
+            lib, stream = _lib.lib(), _lib.stream(dev)
+            _lib.check(lib.s3d_pack_keys(coords.data_ptr(), n, _FIELD, keys.data_ptr(), stream), "s3d_pack_keys")
+            sorted_keys, order = torch.sort(keys)
+            status = lib.s3d_lattice_neighbours(sorted_keys.data_ptr(), order.data_ptr(), n, _FIELD, int(stride), out.data_ptr(), stream)
+        _lib.check(status, "s3d_lattice_neighbours")
+        return out
     sorted_keys, order = torch.sort(pack_coords(coords))
     deltas = torch.tensor([((dx << _FIELD) + dy << _FIELD) + dz for dx in (-1, 0, 1) for dy in (-1, 0, 1)
                            for dz in (-1, 0, 1)], dtype=torch.long, device=coords.device) * stride
@@ -177,6 +201,43 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
     return coarse, pick_cell_representatives(signals, cell_of_row, coarse.shape[0])
 
 
+def _pool_level(coords, step, signals, index):
+    """(coarse coordinates, signals of the representatives) of the cells of `index`: what pool_and_pick and signals[pick]
+    give, in one kernel; None where it does not take them."""
+    if not (_plain_coords(coords) and _plain_signals(signals) and signals.shape[1] <= 16):
+        return None
+    dev, num, cols = coords.device, index.num_windows, signals.shape[1]
+    coarse = torch.empty((num, 4), dtype=torch.int32, device=dev)
+    coarse_signals = torch.empty((num, cols), dtype=torch.float32, device=dev)
+    pick = torch.empty(num, dtype=torch.long, device=dev)
+    with _lib.on(dev):
+        status = _lib.lib().s3d_pool_cells(index.n2n.data_ptr(), index.w2n.data_ptr(), index.w_sizes.data_ptr(), num, coords.data_ptr(),
+                                           step, signals.data_ptr(), signals.stride(0), cols, pick.data_ptr(), coarse.data_ptr(),
+                                           coarse_signals.data_ptr(), _lib.stream(dev))
+    _lib.check(status, "s3d_pool_cells")
+    return coarse, coarse_signals
+
+
+def _level_signals(index, coords, stride, signals, num_signals, quant):
+    """The scaled signals of a window set from a level's voxels and signals, in one kernel (window_signals of
+    _local_and_extra); None where it does not take them."""
+    if not (_plain_coords(coords) and _plain_signals(signals) and 0 <= num_signals <= min(29, signals.shape[1] - 4)):
+        return None
+    n, dev = coords.shape[0], coords.device
+    out = torch.empty((n, 3 + num_signals), dtype=torch.float32, device=dev)
+    with _lib.on(dev):
+        status = _lib.lib().s3d_level_signals(index.w_w_id.data_ptr(), index.n2n.data_ptr(), coords.data_ptr(), int(stride),
+                                              signals.data_ptr(), signals.stride(0), num_signals, index.window_size, float(quant),
+                                              float(2 * quant), out.data_ptr(), n, _lib.stream(dev))
+    _lib.check(status, "s3d_level_signals")
+    return out
+
+
+def _local_and_extra(coords, stride, signals):
+    """(position of every point inside its voxel, its other signals)"""
+    return (signals[:, 1:4].float() - coords[:, 1:].float()) / stride, signals[:, 4:].float()
+
+
 def pick_cell_representatives(signals, cell_of_row, num_cells):
     """For every coarse cell the fine row whose signal vector (all columns of the coordinate
     features) is nearest to the cell mean; ties go to the lower row."""
@@ -197,6 +258,14 @@ def segment_offsets(batch_column, num_batches=None):
     """cumulative END row of every batch element, int32 (what the KNN op takes).  With `num_batches` given the
     host does not wait for the device (batch ids are ascending: the end of batch b is a binary search)."""
     if num_batches is not None:
+        if batch_column.is_cuda and data_only(batch_column) and batch_column.dtype == torch.int32 and batch_column.dim() == 1 \
+                and batch_column.stride(0) >= 1 and num_batches > 0:
+            out = torch.empty(num_batches, dtype=torch.int32, device=batch_column.device)
+            with _lib.on(batch_column.device):
+                status = _lib.lib().s3d_segment_ends(batch_column.data_ptr(), batch_column.stride(0), batch_column.shape[0], num_batches,
+                                                     out.data_ptr(), _lib.stream(batch_column.device))
+            _lib.check(status, "s3d_segment_ends")
+            return out
         ids = torch.arange(num_batches, dtype=batch_column.dtype, device=batch_column.device)
         return torch.searchsorted(batch_column.contiguous(), ids, right=True).to(torch.int32)
     counts = torch.bincount(batch_column.long())
@@ -341,6 +410,12 @@ class GridKNNDownsample(nn.Module):
         """The part that depends on coordinates and signals only: (coarse coordinates, coarse signals, the K
         nearest fine rows of every coarse voxel).  cell_index: the window index at window = stride factor, when
         the caller built it along with its own."""
+        pooled = None if cell_index is None else _pool_level(coords, stride * self.factor, signals, cell_index)
+        if pooled is not None:
+            coarse, coarse_signals = pooled
+            idx, _ = knn_query(self.k, signals[:, 1:4], coarse_signals[:, 1:4], segment_offsets(coords[:, 0], num_batches),
+                               segment_offsets(coarse[:, 0], num_batches), KNN.cell_size, strided=True)
+            return coarse, coarse_signals, idx
         coarse, pick = pool_and_pick(coords, stride, self.factor, signals, cell_index)
         coarse_signals = signals[pick]
         src_xyz = signals[:, 1:4].contiguous().float()
@@ -542,8 +617,7 @@ class Stage(nn.Module):
         window sort's n2n applied to coordinates, signals and features alike).  The row map of the regular set is
         then the identity and is handed to the attention op as None: its kernels read and write the rows in place,
         without the indirection."""
-        local = (signals[:, 1:4].float() - coords[:, 1:].float()) / stride
-        extra = signals[:, 4:].float()
+        local_and_extra = lru_cache(maxsize=1)(partial(_local_and_extra, coords, stride, signals))
         # both window sets (one, for a single block) are enqueued before the host waits for their window counts
         shifts = list((0, self.window_size // 2)[:max(1, min(2, len(self.blocks)))])
         pooled = self.downsample is not None and coords.is_cuda and 1 <= self.downsample.factor <= 10
@@ -555,12 +629,15 @@ class Stage(nn.Module):
             # the quantiser scaling of the signals is the same for every block of the stage: once per index set,
             # fused with the gather into window order
             attn = self.blocks[0].attn
-            args = [StageArguments(index, index.n2n if i > 0 or not rows_in_window_order else None,      # (None: no row map)
-                                   window_signals(index, local, extra, crse_num_axes(attn.cRSE) - 3, attn.quant_size,
-                                                  2 * attn.quant_size), partial(window_signals, index, local, extra))
-                    for i, index in enumerate(indices)]
+            others, args = crse_num_axes(attn.cRSE) - 3, []
+            for i, index in enumerate(indices):
+                scaled = _level_signals(index, coords, stride, signals, others, attn.quant_size)
+                if scaled is None:
+                    scaled = window_signals(index, *local_and_extra(), others, attn.quant_size, 2 * attn.quant_size)
+                args.append(StageArguments(index, index.n2n if i > 0 or not rows_in_window_order else None,      # (None: no row map)
+                                           scaled, lambda index=index: window_signals(index, *local_and_extra())))
         else:
-            args = [index_arguments(index, local, extra) for index in indices]
+            args = [index_arguments(index, *local_and_extra()) for index in indices]
             if rows_in_window_order and args:
                 args[0] = args[0][:5] + (None,) + args[0][6:]      # (.., w2n, n2n, w2m, ..): no row map
         down = (self.downsample.plan(coords, stride, signals, num_batches, cell_index)
@@ -773,11 +850,15 @@ class Upsample(nn.Module):
         stage plan of the finer level's voxel set with the same window size (the encoder's, whose regular window
         set is the one this level's attention block needs), so that the index is not built a second time.
         num_batches: batch elements of both, where the caller knows it: the host then waits for nothing."""
-        xyz = signals[:, 1:4].detach().contiguous().float()
-        support_xyz = signals_up[:, 1:4].detach().contiguous().float()
-        feats = self._norm_linear(self.linear1, voxels_up.feats) + knn_linear_interpolation(
-            xyz, support_xyz, self._norm_linear(self.linear2, voxels.feats).float(),
-            segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches), K=self.up_k)
+        skip, coarse = self._norm_linear(self.linear1, voxels_up.feats), self._norm_linear(self.linear2, voxels.feats).float()
+        ends, ends_up = segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches)
+        if _plain_signals(signals) and _plain_signals(signals_up):
+            idx, dist2 = knn_query(self.up_k, signals[:, 1:4], signals_up[:, 1:4], ends, ends_up, KNN.cell_size, strided=True)
+            feats = skip + KNNInterpolate.apply(idx, dist2, coarse.contiguous())
+        else:
+            xyz = signals[:, 1:4].detach().contiguous().float()
+            support_xyz = signals_up[:, 1:4].detach().contiguous().float()
+            feats = skip + knn_linear_interpolation(xyz, support_xyz, coarse, ends, ends_up, K=self.up_k)
         voxels_up = voxels_up.with_feats(feats.float())
         if self.attn:
             if plan_up is not None:

@@ -12,16 +12,16 @@ from ... import _lib
 from ...swin_blocks import data_only
 
 
-def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0, squared=True):
+def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0, squared=True, strided=False):
     """-> (idx int32 [Nq,K], SQUARED distances fp32 [Nq,K], or the distances with squared=False).  cell_size <= 0: chosen
-    from the data."""
+    from the data.  strided: the coordinates may be columns of a wider matrix (with squared distances)."""
     K = int(K)
     if not 1 <= K <= _lib.KNN_KMAX:
         raise ValueError(f"K must be in 1..{_lib.KNN_KMAX}, got {K}")
     for name, t in (("src_xyz", src_xyz), ("query_xyz", query_xyz)):
         if not t.is_cuda:
             raise RuntimeError(f"{name} must be a CUDA (HIP) tensor")
-        if not t.is_contiguous():
+        if not (t.is_contiguous() or (strided and squared and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= 3)):
             raise RuntimeError(f"{name} must be contiguous")
         if t.dtype != torch.float32 or t.dim() != 2 or t.shape[1] != 3:
             raise ValueError(f"{name} must be float32 [n,3], got {t.dtype} {tuple(t.shape)}")
@@ -47,7 +47,12 @@ def knn_query(K, src_xyz, query_xyz, src_offset, query_offset, cell_size=0.0, sq
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         stream = _lib.stream(dev)
         fn = lib.s3d_knn if squared else lib.s3d_knn_distances
-        status = fn(K, src_xyz.data_ptr(), ns, query_xyz.data_ptr(), nq,
+        if not (src_xyz.is_contiguous() and query_xyz.is_contiguous()):
+            status = lib.s3d_knn_strided(K, src_xyz.data_ptr(), src_xyz.stride(0) if ns > 1 else 3, ns, query_xyz.data_ptr(),
+                                         query_xyz.stride(0) if nq > 1 else 3, nq, src_offset.data_ptr(), query_offset.data_ptr(), b,
+                                         idx.data_ptr(), dist2.data_ptr(), float(cell_size), workspace.data_ptr(), ws_bytes, stream)
+        else:
+            status = fn(K, src_xyz.data_ptr(), ns, query_xyz.data_ptr(), nq,
                     src_offset.data_ptr(), query_offset.data_ptr(), b, idx.data_ptr(),
                     dist2.data_ptr(), float(cell_size), workspace.data_ptr(), ws_bytes,
                     stream)

@@ -1,0 +1,65 @@
+"""A level's geometry in one kernel a step against the tensor statements, to the bit."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import random_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _level(seed, n, stride, columns, extent=(24, 24, 12), batches=2):
+    rng = np.random.default_rng(seed)
+    coords = torch.from_numpy(random_scene(rng, n, extent=extent, batches=batches, stride=stride)).cuda()
+    coords = coords[torch.argsort(coords[:, 0], stable=True)].contiguous()
+    n = coords.shape[0]
+    signals = torch.from_numpy(rng.uniform(-1, 1, (n, columns)).astype(np.float32)).cuda()
+    signals[:, 0] = coords[:, 0].float()
+    signals[:, 1:4] = coords[:, 1:].float() + stride * torch.rand((n, 3), device="cuda")
+    return coords, signals
+
+
+@pytest.mark.parametrize("n,stride,columns,factor", [(1, 1, 4, 2), (5000, 2, 10, 2), (3000, 1, 7, 3), (4000, 3, 16, 4), (2000, 1, 10, 5)])
+def test_pooled_level(hip_lib, n, stride, columns, factor):
+    from swin3d_amd import encoder
+    from swin3d_amd.window_index import build_window_indices
+    coords, signals = _level(n, n, stride, columns)
+    signals[:: 7] = signals[0].clone()                             # ties
+    index = build_window_indices(coords, stride, factor, (0,))[0]
+    wide = torch.cat([signals, signals], 1)[:, :columns]   # rows apart
+    coarse, coarse_signals = encoder._pool_level(coords, stride * factor, wide, index)
+    want, pick = encoder.pool_and_pick(coords, stride, factor, signals, index)
+    assert torch.equal(coarse, want) and torch.equal(coarse_signals, signals[pick])
+
+
+@pytest.mark.parametrize("n,stride,window,others", [(1, 1, 5, 0), (5000, 2, 5, 6), (3000, 3, 7, 3)])
+def test_level_signals(hip_lib, n, stride, window, others):
+    from swin3d_amd import encoder
+    from swin3d_amd.window_index import build_window_indices, window_signals
+    coords, signals = _level(n + window, n, stride, 10)
+    for index in build_window_indices(coords, stride, window, (0, window // 2)):
+        got = encoder._level_signals(index, coords, stride, signals, others, 4)
+        want = window_signals(index, *encoder._local_and_extra(coords, stride, signals), others, 4, 8)
+        assert torch.equal(got, want)
+    assert encoder._level_signals(index, coords, stride, signals, 7, 4) is None                     # more than there are
+    assert encoder._level_signals(index, coords, stride, signals.requires_grad_(), others, 4) is None
+
+
+@pytest.mark.parametrize("n", [1, 2, 1000])
+def test_segments_keys_and_rows_apart(hip_lib, n):
+    from swin3d_amd import encoder
+    from swin3d_amd.sparse_dl.knn.knn import knn_query
+    coords, signals = _level(n, n, 2, 10, batches=3)
+    n = coords.shape[0]
+    host = coords.cpu()
+    for batches in (1, 3, 5, 700):
+        assert torch.equal(encoder.segment_offsets(coords[:, 0], batches).cpu(), encoder.segment_offsets(host[:, 0], batches))
+    shifted = coords - torch.tensor([0, 40, 0, 7], dtype=torch.int32, device="cuda") * 2
+    assert torch.equal(encoder.conv3x3x3_neighbours(shifted, 2).cpu(), encoder.conv3x3x3_neighbours(shifted.cpu(), 2))
+    ends = encoder.segment_offsets(coords[:, 0], 3)
+    apart = knn_query(3, signals[:, 1:4], signals[:, 1:4], ends, ends, strided=True)
+    dense = knn_query(3, signals[:, 1:4].contiguous(), signals[:, 1:4].contiguous(), ends, ends)
+    assert torch.equal(apart[0], dense[0]) and torch.equal(apart[1], dense[1])
+    if n > 1:
+        with pytest.raises(RuntimeError, match="contiguous"):
+            knn_query(3, signals[:, 1:4], signals[:, 1:4], ends, ends)
