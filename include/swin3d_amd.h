@@ -249,6 +249,25 @@ int s3d_attn_bwd_strided(const void *q, const void *k, const void *v, const void
 int s3d_cast_half(const float *const *from, void *const *to, const int64_t *counts, int32_t num, void *stream);
 
 /*
+ * Up to 24 fp32 arrays [rows, cols] to fp16, as they are and / or transposed, the first scaled_rows rows times `scale` (in
+ * fp32, then rounded), and / or as they are to fp32; in one launch.
+ *   from    HOST array of device addresses
+ *   copies  HOST array
+ *   half    device, fp16, 16-byte aligned: what `to` and `transposed` are offsets into, in elements (-1: not wanted)
+ *   same    device, fp32, 16-byte aligned: what `same` is an offset into (-1: not wanted)
+ * A transposed array has rows and cols that are multiples of 8, and it and its offsets are 16-byte aligned.
+ */
+typedef struct {
+    int64_t rows, cols, scaled_rows, to, transposed, same;
+    float scale;
+} s3d_half_copy;
+
+int s3d_half_copies(const float *const *from, const s3d_half_copy *copies, int32_t num, void *half, float *same, void *stream);
+
+/* out = x + residual (fp16, widened first); count a multiple of 4, all 16-byte aligned; out may be x. */
+int s3d_add_half(const float *x, const void *residual, float *out, int64_t count, void *stream);
+
+/*
  * Window sort + segment offsets.
  *
  * Replaces BasicLayer.get_map_pair / get_window_mapping
@@ -543,6 +562,43 @@ size_t s3d_swin_blocks_workspace_bytes(int64_t N, int32_t C, int32_t hidden);
 int s3d_swin_blocks(const float *x, float *x_out, void *pending, int64_t N, int32_t H, int32_t D, int32_t hidden,
                     const int32_t *table_sizes, int32_t nd, int64_t table_len, const s3d_window_set *sets, int32_t num_sets,
                     const s3d_swin_block *blocks, int32_t num_blocks, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * The gradients of a Swin block behind its first LayerNorm, in training in fp16 with parameters in fp32:
+ *   sum = x + proj(attention(qkv(normed1)));  normed2 = LayerNorm(sum);
+ *   hidden_in = fc1(normed2);  hidden_out = GELU(hidden_in);  pending = fc2(hidden_out)
+ * with dsum [N,C] fp32 and dpending [N,C] fp16 the gradients of sum and pending, C = H*D.
+ *   saved     HOST: what the forward left.  Weights transposed, in fp16 ([in,out]; the q columns of qkv times q_scale)
+ *   grads     HOST: where the gradients go; null for those that are not wanted, but for norm2 and normed1
+ *   dtype     S3D_DTYPE_F16, or S3D_DTYPE_F32_F16_ROWS with tables in fp32, as for s3d_attn_bwd
+ *   pairs     at least 1; head_dim, tables and windows as the forms of s3d_attn_bwd with a pair store take them
+ * N at least 1, C and hidden multiples of 16, C at most 1024; all device pointers 16-byte aligned.
+ */
+typedef struct {
+    const void *normed1, *qkv, *attended;                    /* fp16 [N,C], [N,3C], [N,C] */
+    const float *out_max, *out_sum, *sum;                    /* [N,H], [N,H], [N,C] */
+    const void *normed2, *hidden_in, *hidden_out;            /* fp16 [N,C], [N,hidden], [N,hidden] */
+    const void *qkv_weight_t, *proj_weight_t, *fc1_weight_t, *fc2_weight_t;
+    const void *table_q, *table_k, *table_v;
+    const float *norm2_weight;
+    const int32_t *w_sizes, *w2n, *n2n;                      /* n2n may be null */
+    const float *n_coords;
+    float norm2_eps;
+} s3d_block_saved;
+
+typedef struct {
+    float *x;                                                /* [N,C] */
+    void *normed1;                                           /* fp16 [N,C] */
+    float *norm2_weight, *norm2_bias;
+    float *qkv_weight, *qkv_bias, *proj_weight, *proj_bias, *fc1_weight, *fc1_bias, *fc2_weight, *fc2_bias;
+    float *table_q, *table_k, *table_v;
+} s3d_block_gradients;
+
+size_t s3d_swin_block_grad_workspace_bytes(int64_t N, int32_t H, int32_t D, int32_t hidden, int32_t nd, int64_t table_len, int64_t W,
+                                           int64_t pairs);
+int s3d_swin_block_grad(const s3d_block_saved *saved, const s3d_block_gradients *grads, const float *dsum, const void *dpending, int64_t N,
+                        int32_t H, int32_t D, int32_t hidden, const int32_t *table_sizes, int32_t nd, int64_t table_len, int64_t W,
+                        int64_t pairs, float q_scale, int32_t dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus
 }

@@ -41,6 +41,21 @@ class SwinBlock(ctypes.Structure):
                                    "fc2_weight", "fc2_bias")] + [("norm1_eps", ctypes.c_float), ("norm2_eps", ctypes.c_float)]
 
 
+class HalfCopy(ctypes.Structure):
+    _fields_ = [(n, _i64) for n in ("rows", "cols", "scaled_rows", "to", "transposed", "same")] + [("scale", ctypes.c_float)]
+
+
+class BlockSaved(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("normed1", "qkv", "attended", "out_max", "out_sum", "sum", "normed2", "hidden_in", "hidden_out",
+                                   "qkv_weight_t", "proj_weight_t", "fc1_weight_t", "fc2_weight_t", "table_q", "table_k", "table_v",
+                                   "norm2_weight", "w_sizes", "w2n", "n2n", "n_coords")] + [("norm2_eps", ctypes.c_float)]
+
+
+class BlockGradients(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("x", "normed1", "norm2_weight", "norm2_bias", "qkv_weight", "qkv_bias", "proj_weight", "proj_bias",
+                                   "fc1_weight", "fc1_bias", "fc2_weight", "fc2_bias", "table_q", "table_k", "table_v")]
+
+
 # name -> (restype, argtypes); mirrors include/swin3d_amd.h
 SIGNATURES = {
     "s3d_version": (ctypes.c_int, []),
@@ -68,6 +83,12 @@ SIGNATURES = {
     "s3d_level_signals": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp, _i64, _i32, _i32, ctypes.c_float, ctypes.c_float, _vp, _i64, _vp]),
     "s3d_knn_strided": (ctypes.c_int, [_i32, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i32, _vp, _vp, ctypes.c_float, _vp,
                                        ctypes.c_size_t, _vp]),
+    "s3d_half_copies": (ctypes.c_int, [_vp, _vp, _i32, _vp, _vp, _vp]),
+    "s3d_add_half": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp]),
+    "s3d_swin_block_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i64, _i64, _i64]),
+    # saved grads dsum dpending | N H D hidden | sizes nd len | W pairs scale dtype | ws bytes stream
+    "s3d_swin_block_grad": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp, _i32, _i64, _i64, _i64, ctypes.c_float, _i32, _vp,
+                                           ctypes.c_size_t, _vp]),
     "s3d_cast_half": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp]),
     "s3d_window_index_grid_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_window_index_grid": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),

@@ -11,8 +11,26 @@ struct LinearArgs {
     int64_t M;
     int32_t N, K;
     bool gelu;
+    const void *gelu_at = nullptr;   // [M,N] fp16: the rows, rounded, are gradients behind a GELU of these, and y those before it
 };
 
 int launch_linear(const LinearArgs &a, hipStream_t stream);
+
+// A layer's weight and bias gradients (linear_grad.hip): dw = dy^T x, db = the column sums of dy; the first `scaled` rows of
+// the weight (and numbers of the bias) are parameters times `scale`
+struct LinearGrad {
+    const void *dy, *x;   // [M,N], [M,K] fp16
+    void *dw, *db;        // [N,K], [N]; one of them may be null
+    int64_t M;
+    int32_t N, K, scaled;
+    float scale;
+};
+
+constexpr int kMostLinearGrads = 4;
+size_t linear_grads_bytes(const LinearGrad *grads, int num);
+int launch_linear_grad_parts(const LinearGrad &g, float *parts, hipStream_t stream);
+// the sums of the parts of `num` layers in one launch; parts: where linear_grads_bytes has them, one layer behind the other
+int launch_linear_grad_sums(const LinearGrad *grads, int num, float *parts, int32_t grad_dtype, hipStream_t stream);
+size_t linear_grad_part_count(const LinearGrad &g);
 
 }  // namespace s3d

@@ -42,6 +42,15 @@ __device__ __forceinline__ float gelu(float x)
     return 0.5f * fmaf(-c, __builtin_amdgcn_exp2f(p * c), x + u);
 }
 
+// The derivative of x Phi(x): Phi(x) + x phi(x), in fp32
+__device__ __forceinline__ float gelu_slope(float x)
+{
+    const float phi = 0.3989422804f * __builtin_amdgcn_exp2f(-0.7213475204f * x * x);
+    return fmaf(x, phi, 0.5f * (1.0f + erff(0.7071067812f * x)));
+}
+
+enum class Behind { kNothing, kGelu, kGeluGrad };
+
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
 
@@ -56,10 +65,10 @@ template <int WM, int WN, int TM, int TN> struct Tile {
     static constexpr int kLoads = (kM + kN) * kPieces / kThreads;     // pieces per thread and chunk
 };
 
-template <typename L, bool GELU>
+template <typename L, Behind kBehind>
 __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
                                                              const _Float16 *__restrict__ bias, _Float16 *__restrict__ y,
-                                                             int M, int N, int K, int tiles_n, int tiles)
+                                                             const _Float16 *__restrict__ gelu_at, int M, int N, int K, int tiles_n, int tiles)
 {
     constexpr int TM = L::kTM, TN = L::kTN;
     __shared__ __align__(16) char smem[L::kLds];
@@ -138,7 +147,7 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float v = acc[i][j][4 * g + e] + static_cast<float>(b[e]);
-                    o[e] = static_cast<_Float16>(GELU ? gelu(v) : v);
+                    o[e] = static_cast<_Float16>(kBehind == Behind::kGelu ? gelu(v) : v);
                 }
                 *reinterpret_cast<half4 *>(out + (wave_m + i * 32 + r32) * L::kPitch + n) = o;
             }
@@ -148,8 +157,16 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
 #pragma unroll
     for (int t = tid; t < L::kM * kRowPieces; t += kThreads) {
         const int r = t / kRowPieces, n = t % kRowPieces * 8;
-        if (m0 + r < M && n0 + n < N)
-            *reinterpret_cast<uint4 *>(y + static_cast<int64_t>(m0 + r) * N + n0 + n) = *reinterpret_cast<const uint4 *>(out + r * L::kPitch + n);
+        if (m0 + r < M && n0 + n < N) {
+            const int64_t to = static_cast<int64_t>(m0 + r) * N + n0 + n;
+            half8 piece = *reinterpret_cast<const half8 *>(out + r * L::kPitch + n);
+            if constexpr (kBehind == Behind::kGeluGrad) {
+                const half8 at = *reinterpret_cast<const half8 *>(gelu_at + to);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) piece[e] = static_cast<_Float16>(static_cast<float>(piece[e]) * gelu_slope(static_cast<float>(at[e])));
+            }
+            *reinterpret_cast<half8 *>(y + to) = piece;
+        }
     }
 }
 
@@ -160,9 +177,10 @@ int launch(const LinearArgs &a, hipStream_t stream)
     const int64_t tiles = ceil_div(a.M, L::kM) * tiles_n;
     if (tiles > (1 << 30)) return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M = %lld rows", (long long)a.M);
     const dim3 grid(static_cast<unsigned>(ceil_div(tiles, 8) * 8));
-    auto kernel = a.gelu ? linear_kernel<L, true> : linear_kernel<L, false>;
+    auto kernel = a.gelu_at ? linear_kernel<L, Behind::kGeluGrad> : a.gelu ? linear_kernel<L, Behind::kGelu> : linear_kernel<L, Behind::kNothing>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, static_cast<const _Float16 *>(a.x), static_cast<const _Float16 *>(a.w),
-                       static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<int>(a.M), a.N, a.K, tiles_n,
+                       static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<const _Float16 *>(a.gelu_at),
+                       static_cast<int>(a.M), a.N, a.K, tiles_n,
                        static_cast<int>(tiles));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -183,7 +201,7 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     auto padded = [&](int width) { return (a.N + width - 1) / width * width; };
     auto enough = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width) >= 512; };
     const int least = padded(64);
-    if (padded(192) == least && enough(192) && (!a.gelu || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
+    if (padded(192) == least && enough(192) && (!(a.gelu || a.gelu_at) || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
     if (padded(128) == least && enough(128)) return launch<Tile<2, 2, 2, 2>>(a, stream);
     return launch<Tile<2, 2, 2, 1>>(a, stream);
 }

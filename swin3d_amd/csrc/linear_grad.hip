@@ -15,7 +15,7 @@
 // Both kernels with their launches, against dY^T X and the column sums as two library calls: 199,327 rows, 192 x 48, 30 us
 // (3.2 TB/s of operands) against 499; 48 x 48, 19 against 191; 12,421 rows, 768 x 192, 24 against 100; 811 rows, 384 x 384,
 // 14 (the host's share of the call) against 28.
-#include "s3d_common.h"
+#include "linear.h"
 
 namespace s3d {
 namespace {
@@ -133,24 +133,50 @@ __global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
     }
 }
 
-// The sum of the parts: 64 numbers a workgroup, its four wavefronts share the parts.
+struct GradSums {
+    const float *parts[kMostLinearGrads];
+    void *dw[kMostLinearGrads], *db[kMostLinearGrads];
+    int64_t products[kMostLinearGrads];
+    int n[kMostLinearGrads], k[kMostLinearGrads], splits[kMostLinearGrads], scaled[kMostLinearGrads];
+    int first[kMostLinearGrads];      // the first workgroup of each
+    float scale[kMostLinearGrads];
+};
+
+// The sum of the parts: 64 numbers a workgroup, its four wavefronts share the parts.  Several layers share a launch: the sums
+// of a Swin block's four are 5 us each by themselves, for some 20 MB of parts.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(const float *__restrict__ parts, int splits, int64_t products,
-                                                                   int64_t total, T *__restrict__ dw, T *__restrict__ db)
+__global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(GradSums a)
 {
     __shared__ float shared[kThreads];
+    int at = 0;
+#pragma unroll
+    for (int i = 1; i < kMostLinearGrads; ++i) at = static_cast<int>(blockIdx.x) >= a.first[i] ? i : at;
+    const float *parts = a.parts[0];
+    T *dw = static_cast<T *>(a.dw[0]), *db = static_cast<T *>(a.db[0]);
+    int64_t products = a.products[0];
+    int n = a.n[0], k = a.k[0], splits = a.splits[0], scaled = a.scaled[0], first = a.first[0];
+    float scale = a.scale[0];
+#pragma unroll
+    for (int i = 1; i < kMostLinearGrads; ++i) {
+        if (at != i) continue;
+        parts = a.parts[i]; dw = static_cast<T *>(a.dw[i]); db = static_cast<T *>(a.db[i]); products = a.products[i];
+        n = a.n[i]; k = a.k[i]; splits = a.splits[i]; scaled = a.scaled[i]; first = a.first[i]; scale = a.scale[i];
+    }
+    const int64_t total = products + n;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * 64 + lane, at = min(e, total - 1);
+    const int64_t e = (static_cast<int64_t>(blockIdx.x) - first) * 64 + lane, from = min(e, total - 1);
     float sum = 0.0f;
 #pragma unroll 8
-    for (int s = wave; s < splits; s += 4) sum += parts[s * total + at];
+    for (int s = wave; s < splits; s += 4) sum += parts[s * total + from];
     shared[threadIdx.x] = sum;
     __syncthreads();
     if (wave > 0 || e >= total) return;
     sum = (shared[lane] + shared[lane + 64]) + (shared[lane + 128] + shared[lane + 192]);
     if (e < products) {
+        if (e < static_cast<int64_t>(scaled) * k) sum *= scale;
         if (dw) dw[e] = static_cast<T>(sum);
     } else if (db) {
+        if (e - products < scaled) sum *= scale;
         db[e - products] = static_cast<T>(sum);
     }
 }
@@ -178,6 +204,58 @@ Split split_of(int64_t M, int N, int K)
 bool fits(int64_t M, int32_t N, int32_t K) { return M > 0 && M <= 0x7fffffff && N >= 8 && N % 8 == 0 && K >= 8 && K % 8 == 0 && N <= 16384 && K <= 16384; }
 
 }  // namespace
+
+size_t linear_grad_part_count(const LinearGrad &g) { return static_cast<size_t>(split_of(g.M, g.N, g.K).count) * (static_cast<size_t>(g.N) * g.K + g.N); }
+
+size_t linear_grads_bytes(const LinearGrad *grads, int num)
+{
+    size_t count = 0;
+    for (int i = 0; i < num; ++i) count += linear_grad_part_count(grads[i]);
+    return count * sizeof(float);
+}
+
+int launch_linear_grad_parts(const LinearGrad &g, float *parts, hipStream_t stream)
+{
+    if (!fits(g.M, g.N, g.K))
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_linear_grad: M=%lld N=%d K=%d (N and K multiples of 8, at most 16384)", (long long)g.M, g.N, g.K);
+    const Split split = split_of(g.M, g.N, g.K);
+    const GradArgs args{static_cast<const _Float16 *>(g.dy), static_cast<const _Float16 *>(g.x), parts, g.M, split.rows, g.N, g.K, split.tiles_k};
+    auto kernel = split.un == 3 ? (split.uk == 3 ? linear_grad_kernel<3, 3> : linear_grad_kernel<3, 2>)
+                                : (split.uk == 3 ? linear_grad_kernel<2, 3> : linear_grad_kernel<2, 2>);
+    hipLaunchKernelGGL(kernel, dim3(split.tiles, split.count), dim3(kThreads), 0, stream, args);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+int launch_linear_grad_sums(const LinearGrad *grads, int num, float *parts, int32_t grad_dtype, hipStream_t stream)
+{
+    GradSums a{};
+    int64_t blocks = 0;
+    for (int i = 0; i < kMostLinearGrads; ++i) {
+        a.first[i] = 0x7fffffff;
+        if (i >= num) continue;
+        const LinearGrad &g = grads[i];
+        a.parts[i] = parts;
+        a.dw[i] = g.dw;
+        a.db[i] = g.db;
+        a.products[i] = static_cast<int64_t>(g.N) * g.K;
+        a.n[i] = g.N;
+        a.k[i] = g.K;
+        a.splits[i] = split_of(g.M, g.N, g.K).count;
+        a.scaled[i] = g.scaled;
+        a.scale[i] = g.scale;
+        a.first[i] = static_cast<int>(blocks);
+        blocks += ceil_div(a.products[i] + g.N, 64);      // (at most 2^22 + 256 a layer)
+        parts += linear_grad_part_count(g);
+    }
+    if (grad_dtype == S3D_DTYPE_F32)
+        hipLaunchKernelGGL(linear_grad_sum_kernel<float>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL(linear_grad_sum_kernel<_Float16>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, a);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
 }  // namespace s3d
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_linear_grad_workspace_bytes(int64_t M, int32_t N, int32_t K)
@@ -201,21 +279,8 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
     if (!workspace || workspace_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_linear_grad: workspace %zu B < required %zu B", workspace ? workspace_bytes : size_t(0), need);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const Split split = split_of(M, N, K);
-    const GradArgs args{static_cast<const _Float16 *>(dy), static_cast<const _Float16 *>(x), static_cast<float *>(workspace), M,
-                        split.rows, N, K, split.tiles_k};
-    auto kernel = split.un == 3 ? (split.uk == 3 ? linear_grad_kernel<3, 3> : linear_grad_kernel<3, 2>)
-                                : (split.uk == 3 ? linear_grad_kernel<2, 3> : linear_grad_kernel<2, 2>);
-    hipLaunchKernelGGL(kernel, dim3(split.tiles, split.count), dim3(kThreads), 0, s, args);
-    S3D_HIP_CHECK(hipGetLastError());
-    const int64_t products = static_cast<int64_t>(N) * K, total = products + N;
-    const dim3 sums(static_cast<unsigned>(ceil_div(total, 64)));
-    if (grad_dtype == S3D_DTYPE_F32)
-        hipLaunchKernelGGL(linear_grad_sum_kernel<float>, sums, dim3(kThreads), 0, s, args.parts, split.count, products, total,
-                           static_cast<float *>(dw), static_cast<float *>(db));
-    else
-        hipLaunchKernelGGL(linear_grad_sum_kernel<_Float16>, sums, dim3(kThreads), 0, s, args.parts, split.count, products, total,
-                           static_cast<_Float16 *>(dw), static_cast<_Float16 *>(db));
-    S3D_HIP_CHECK(hipGetLastError());
-    return S3D_OK;
+    const LinearGrad g{dy, x, dw, db, M, N, K, 0, 1.0f};
+    float *parts = static_cast<float *>(workspace);
+    if (int rc = launch_linear_grad_parts(g, parts, s)) return rc;
+    return launch_linear_grad_sums(&g, 1, parts, grad_dtype, s);
 }

@@ -39,6 +39,7 @@ from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .sparse_dl.knn import KNN, KNNInterpolate, KNNMaxPool, knn_max_pool, knn_query
 from .swin_blocks import data_only, linear_rows, plain, swin_blocks
+from .swin_train import trained_branches
 from .window_index import build_window_indices, get_index01, index_arguments, window_signals
 
 
@@ -550,6 +551,10 @@ class SwinBlock(nn.Module):
         done = trained_add_norm(feats, pending, self.norm1)
         if done is None:
             return None
+        whole = trained_branches(self, (SwinBlock, WindowAttention, Mlp), *done, attn_args)
+        if whole is not None:
+            _cache_epoch()      # (a forward that a change of parameters may follow)
+            return whole
         feats, branch = done[0], self.attn(done[1], attn_args)
         done = trained_add_norm(feats, branch, self.norm2)
         if done is None:

@@ -1,0 +1,241 @@
+"""A Swin block behind its first LayerNorm in training under fp16 autocast, as one node of autograd:
+
+    sum = x + proj(attention(qkv(normed)));  pending = fc2(GELU(fc1(LayerNorm(sum))))
+
+Layer by layer that is a dozen nodes, some thirty copies and casts of parameters and fifty dispatches of the backward, which
+on scans of up to 100,000 voxels take the host longer than the kernels take the device.  Here the parameters are cast,
+scaled and transposed by one launch (s3d_half_copies), and the backward is one call of the library (s3d_swin_block_grad).
+
+The forward's products and norm are torch's to the bit, as in linear_grad.py, for the reason given there."""
+import ctypes
+import functools
+import itertools
+
+import torch
+import torch.nn.functional as F
+from torch.autograd.function import Function
+
+from . import _lib
+from .fused_norm import _AddNorm, add_half
+from .linear_grad import _Linear
+from .sparse_dl.attn import attn_coff
+from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
+from .swin_blocks import _applicable, _parts, data_only, followed
+
+_PRECISION = (PrecisionMode.HALF_NONE, PrecisionMode.HALF_FORWARD, PrecisionMode.HALF_ALL)
+_KINDS = ("query", "key", "value")
+_GROUPS = ("xyz", "rgb", "norm")
+
+
+class _Layout:
+    """Where the fp16 copies of a block's parameters lie in one buffer, by the shapes alone: per array (rows, columns) of
+    `shapes`, in the order of _parameters.  Every copy of a layer starts on a multiple of 512 bytes, as an allocation of
+    its own would: the library behind torch's products picks kernels by alignment."""
+
+    def __init__(self, shapes, num_tables, scaled_rows, scale, same_tables):
+        layers = len(shapes) - num_tables
+        self.copies = (_lib.HalfCopy * len(shapes))()
+        self.shapes, self.to, self.transposed = shapes, [], []
+        at = same = 0
+        for i, (copy, (rows, cols)) in enumerate(zip(self.copies, shapes)):
+            table = i >= layers
+            # (a kind's tables lie one behind the other, as the attention reads them)
+            at += 0 if table and (i - layers) % (num_tables // 3) else -at % 256
+            across = not table and cols > 1
+            copy.rows, copy.cols, copy.to = rows, cols, at
+            at += rows * cols
+            if across:
+                at += -at % 256
+            copy.transposed = at if across else -1
+            at += rows * cols if across else 0
+            copy.scaled_rows, copy.scale = (scaled_rows, scale) if rows == 3 * scaled_rows and i < 2 else (0, 1.0)
+            copy.same = same if table and same_tables else -1
+            same += rows * cols if table and same_tables else 0
+            self.to.append(copy.to)
+            self.transposed.append(copy.transposed)
+        self.half_count, self.same_count = at, same
+
+
+_layout = functools.lru_cache(maxsize=64)(_Layout)
+
+
+class _Call:
+    """What a block's pass needs besides tensors that have gradients."""
+    __slots__ = ("heads", "dim", "hidden", "sizes", "table_len", "index", "mode", "eps", "scale", "pairs")
+
+
+def _parameters(parts, groups):
+    """[qkv weight, bias, proj .., fc1 .., fc2 .., query tables, key tables, value tables] of a block; biases may be None."""
+    _, _, attn, qkv, proj, _, _, fc1, _, fc2 = parts
+    tables = attn._parameters
+    return [p for layer in (qkv, proj, fc1, fc2) for p in (layer.weight, layer.bias)] + [
+        tables.get(f"{kind}_{name}_table") for kind in _KINDS for name in _GROUPS[:groups]]
+
+
+def trained_branches(block, kinds, x, normed, attn_args):
+    """(sum, pending) of `block` (of the types `kinds`) for rows x and their first norm `normed`, which trained_add_norm
+    made; None where the layers have to be called one by one."""
+    n, channels = x.shape
+    parts = _parts(block, kinds)
+    if parts is None or len(attn_args) < 9 or normed.dtype != torch.float16 or not _applicable([parts], channels) or followed() \
+            or type(parts[2].scale) is not float:
+        return None
+    _, _, attn, _, _, norm2, _, fc1, _, _ = parts
+    sizes, heads, dim, dev = list(attn.table_sizes), attn.num_heads, attn.head_dim, x.device
+    nd, table_len = len(sizes), sum(sizes)
+    params = _parameters(parts, nd // 3)
+    for t in (norm2.weight, norm2.bias, *params):
+        if t is not None and not (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.device == dev
+                                  and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            return None
+    tables = params[8:]
+    w_sizes, w2n, n2n, coords = attn_args[3], attn_args[4], attn_args[5], attn_args[8]
+    per_kind = nd // 3
+    if nd not in (3, 6, 9) or heads * dim != channels or dim == 32 or table_len > attn_coff.BWD_MAX_ROWS_PER_AXIS * nd * channels \
+            or any(t is None for t in tables) or any(t.numel() != sum(sizes[3 * (i % per_kind):3 * (i % per_kind) + 3]) for i, t in enumerate(tables)) \
+            or not (data_only(coords) and coords.dtype == torch.float32 and coords.shape == (n, nd) and coords.is_contiguous()
+                    and coords.device == dev) \
+            or any(not (data_only(t) and t.device == dev and t.dtype in (torch.int32, torch.int64)) for t in (w_sizes, w2n)) \
+            or not (n2n is None or data_only(n2n) and n2n.device == dev and n2n.dtype in (torch.int32, torch.int64)):
+        return None
+    # (a pass that leaves nothing for the attention's backward runs other kernels)
+    if not (normed.requires_grad or any(t.requires_grad for t in itertools.chain(params[:2], tables) if t is not None)):
+        return None
+    pairs = attn_coff._pairs_of(w_sizes, w_sizes) if attn_coff.BWD_PAIR_STORE else 0
+    if pairs == 0 or 12 * pairs * heads > attn_coff.BWD_PAIR_STORE_MAX_BYTES:
+        return None
+    call = _Call()
+    call.heads, call.dim, call.hidden, call.sizes, call.table_len = heads, dim, fc1.out_features, sizes, table_len
+    call.index, call.mode, call.eps, call.scale, call.pairs = (w_sizes, w2n, n2n, coords), attn.fp16_mode, norm2.eps, attn.scale, pairs
+    return _Branches.apply(call, x, normed, norm2.weight, norm2.bias, *params)
+
+
+def _by_parts(call, index, x, normed, norm_weight, norm_bias, params):
+    """The same through the nodes of the single layers, for gradients of gradients."""
+    qkv_weight, qkv_bias, proj_weight, proj_bias, fc1_weight, fc1_bias, fc2_weight, fc2_bias, *tables = params
+    channels = call.heads * call.dim
+    w_sizes, w2n, n2n, coords = index
+    scale = torch.ones(3 * channels, device=x.device)
+    scale[:channels] = call.scale
+    qkv = _Linear.apply(normed, qkv_weight * scale.unsqueeze(1), None if qkv_bias is None else qkv_bias * scale)
+    groups = len(tables) // 3
+    kinds = [torch.cat([t.reshape(-1) for t in tables[i:i + groups]]) for i in range(0, 3 * groups, groups)]
+    out = SelfAttnAIOFunction.apply(
+        *qkv.view(-1, 3, call.heads, call.dim).unbind(1), *kinds, call.sizes, [None, w_sizes, None, w2n, n2n, coords], PosEmb.SEPARATE,
+        TableDims.D0, IndexMode.INDIRECT, _PRECISION[call.mode])
+    branch = _Linear.apply(out.reshape(-1, channels), proj_weight, proj_bias)
+    norm = torch.nn.LayerNorm(channels, call.eps, elementwise_affine=False, device="meta")      # (shape and eps)
+    summed, normed2 = _AddNorm.apply(x, branch, norm_weight, norm_bias, norm)
+    return summed, _Linear.apply(F.gelu(_Linear.apply(normed2, fc1_weight, fc1_bias)), fc2_weight, fc2_bias)
+
+
+class _Branches(Function):
+    @staticmethod
+    def forward(ctx, call, x, normed, norm_weight, norm_bias, *params):
+        ctx.set_materialize_grads(False)
+        n, channels = x.shape
+        heads, dim, dev = call.heads, call.dim, x.device
+        given = [p for p in params if p is not None]
+        num_tables = len(params) - 8
+        # (the backward of mode 1 reads the tables in fp32)
+        layout = _layout(tuple((p.shape[0], p.shape[1]) if p.dim() == 2 else (p.numel(), 1) for p in given), num_tables, channels,
+                         call.scale, call.mode == 1)
+        half = torch.empty(layout.half_count, dtype=torch.float16, device=dev)
+        same = torch.empty(layout.same_count, dtype=torch.float32, device=dev) if layout.same_count else None
+        lib = _lib.lib()
+        with _lib.on(dev):
+            status = lib.s3d_half_copies((ctypes.c_void_p * len(given))(*[p.data_ptr() for p in given]), layout.copies, len(given),
+                                         half.data_ptr(), None if same is None else same.data_ptr(), _lib.stream(dev))
+        _lib.check(status, "s3d_half_copies")
+        places = iter(zip(layout.shapes, layout.to))
+        copies = []
+        for p in params[:8]:
+            if p is None:
+                copies.append(None)
+                continue
+            (rows, cols), at = next(places)
+            copies.append(half.as_strided((rows, cols), (cols, 1), at) if p.dim() == 2 else half.as_strided((rows,), (1,), at))
+        starts = layout.to[-num_tables::num_tables // 3]
+        tables = [half.as_strided((call.table_len,), (1,), at) for at in starts]
+        qkv = F.linear(normed, copies[0], copies[1])
+        row = channels
+        q, k, v = (qkv.as_strided((n, heads, dim), (3 * row, dim, 1), i * row) for i in range(3))
+        (w_sizes, w2n, n2n, coords), call.index = call.index, None
+        out, omax, osum = attn_coff._attention(q, k, v, [3 * row] * 3, *tables, call.sizes, w_sizes, w2n, n2n, coords, True)
+        branch = F.linear(out.view(n, channels), copies[2], copies[3])
+        summed = add_half(x, branch)
+        normed2 = F.layer_norm(summed, (channels,), norm_weight, norm_bias, call.eps).to(torch.float16)
+        hidden_in = F.linear(normed2, copies[4], copies[5])
+        hidden_out = F.gelu(hidden_in)
+        pending = F.linear(hidden_out, copies[6], copies[7])
+        ctx.call, ctx.layout = call, layout
+        ctx.save_for_backward(x, normed, norm_weight, norm_bias, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same,
+                              w_sizes, w2n, n2n, coords, *params)
+        return summed, pending
+
+    @staticmethod
+    def backward(ctx, dsum, dpending):
+        call, layout, needs = ctx.call, ctx.layout, ctx.needs_input_grad
+        (x, normed, norm_weight, norm_bias, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same, w_sizes, w2n, n2n,
+         coords, *params) = ctx.saved_tensors
+        if torch.is_grad_enabled() or dsum is None or dpending is None or not (data_only(dsum) and data_only(dpending)) \
+                or dsum.dtype != torch.float32 or dpending.dtype != torch.float16:
+            return _Branches._replayed(ctx, (dsum, dpending), (x, normed, norm_weight, norm_bias, *params), (w_sizes, w2n, n2n, coords))
+        n, channels = x.shape
+        heads, dim, dev, nd = call.heads, call.dim, x.device, len(call.sizes)
+        dsum, dpending = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+                          for t in (dsum, dpending))
+        w_sizes, w2n = attn_coff._as_int32("w_sizes", w_sizes, dev), attn_coff._as_int32("w2n_indices", w2n, dev)
+        n2n = None if n2n is None else attn_coff._as_int32("n2n_indices", n2n, dev)
+        saved, grads = _lib.BlockSaved(), _lib.BlockGradients()
+        saved.normed1, saved.qkv, saved.attended = normed.data_ptr(), qkv.data_ptr(), out.data_ptr()
+        saved.out_max, saved.out_sum, saved.sum = omax.data_ptr(), osum.data_ptr(), summed.data_ptr()
+        saved.normed2, saved.hidden_in, saved.hidden_out = normed2.data_ptr(), hidden_in.data_ptr(), hidden_out.data_ptr()
+        base = half.data_ptr()
+        saved.qkv_weight_t, saved.proj_weight_t, saved.fc1_weight_t, saved.fc2_weight_t = (base + 2 * at for at in layout.transposed if at >= 0)
+        num_tables = len(params) - 8
+        if same is None:
+            saved.table_q, saved.table_k, saved.table_v = (base + 2 * at for at in layout.to[-num_tables::num_tables // 3])
+        else:
+            saved.table_q, saved.table_k, saved.table_v = (same.data_ptr() + 4 * i * call.table_len for i in range(3))
+        saved.norm2_weight, saved.norm2_eps = norm_weight.data_ptr(), call.eps
+        saved.w_sizes, saved.w2n, saved.n2n = w_sizes.data_ptr(), w2n.data_ptr(), None if n2n is None else n2n.data_ptr()
+        saved.n_coords = coords.data_ptr()
+        dx, dnormed = torch.empty_like(x), torch.empty_like(normed)
+        dnorm = [torch.empty_like(norm_weight), torch.empty_like(norm_bias)]
+        dparams = [torch.empty_like(p) if need else None for p, need in zip(params[:8], needs[5:13])]
+        dtables = [torch.empty(call.table_len, dtype=torch.float32, device=dev) for _ in range(3)]
+        grads.x, grads.normed1, grads.norm2_weight, grads.norm2_bias = (t.data_ptr() for t in (dx, dnormed, *dnorm))
+        (grads.qkv_weight, grads.qkv_bias, grads.proj_weight, grads.proj_bias, grads.fc1_weight, grads.fc1_bias, grads.fc2_weight,
+         grads.fc2_bias) = (None if t is None else t.data_ptr() for t in dparams)
+        grads.table_q, grads.table_k, grads.table_v = (t.data_ptr() for t in dtables)
+        lib = _lib.lib()
+        with _lib.on(dev):
+            ws_bytes = lib.s3d_swin_block_grad_workspace_bytes(n, heads, dim, call.hidden, nd, call.table_len, w_sizes.numel(), call.pairs)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            status = lib.s3d_swin_block_grad(
+                ctypes.byref(saved), ctypes.byref(grads), dsum.data_ptr(), dpending.data_ptr(), n, heads, dim, call.hidden,
+                (ctypes.c_int32 * nd)(*call.sizes), nd, call.table_len, w_sizes.numel(), call.pairs, call.scale,
+                _lib.S3D_DTYPE_F16 if same is None else _lib.S3D_DTYPE_F32_F16_ROWS, workspace.data_ptr(), ws_bytes, _lib.stream(dev))
+        _lib.check(status, "s3d_swin_block_grad")
+        groups = num_tables // 3
+        pieces = [piece for t in dtables for piece in t.split([p.numel() for p in params[8:8 + groups]])]
+        given = [dx, dnormed, *dnorm, *dparams, *(piece.view(p.shape) for piece, p in zip(pieces, params[8:]))]
+        return (None, *(g if need else None for g, need in zip(given, needs[1:])))
+
+    @staticmethod
+    def _replayed(ctx, grads, inputs, index):
+        """A graph of the gradients is wanted, or something follows them, or one is absent: the pass again through the
+        single layers, whose backward knows these cases."""
+        needs = ctx.needs_input_grad[1:]
+        graph = torch.is_grad_enabled()
+        with torch.enable_grad(), torch.autocast("cuda", dtype=torch.float16):
+            if not graph:
+                inputs = [None if t is None else t.detach().requires_grad_(need) for t, need in zip(inputs, needs)]
+            outs = _by_parts(ctx.call, index, *inputs[:4], inputs[4:])
+        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]
+        wanted = [t for t, need in zip(inputs, needs) if need]
+        if not pairs:
+            return (None,) * (1 + len(needs))
+        got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=graph, allow_unused=True))
+        return (None, *(next(got) if need else None for need in needs))

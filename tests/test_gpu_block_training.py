@@ -1,0 +1,149 @@
+"""A block in training as one node of autograd, against the nodes of its layers; the fp16 copies of its parameters."""
+import ctypes
+
+import pytest
+import torch
+
+from swin3d_amd import encoder, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,scaled,offset", [(1, 1, 0, 0), (37, 3, 11, 1), (4097, 1, 5, 0), (8, 8, 0, None), (72, 136, 24, None),
+                                                     (144, 48, 48, None), (64, 64, 64, None), (1152, 384, 384, None)])
+def test_half_copies(hip_lib, rows, cols, scaled, offset):
+    from swin3d_amd import _lib
+    dev = torch.device("cuda", 0)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    # beside an array of another kind, so that the workgroups have to be told apart
+    other = torch.randn(5000, device=dev, generator=gen)
+    data = torch.randn(rows * cols + 8, device=dev, generator=gen)
+    data[0], data[-9:-8] = 7e4, float("nan")
+    x = data[offset or 0:][:rows * cols].view(rows, cols)
+    scale = 0.3535533905932738
+    turned = offset is None
+    half = torch.zeros(5000 + 2 * (rows * cols + 8), dtype=torch.float16, device=dev)
+    same = torch.zeros(rows * cols + 8, device=dev)
+    second = 5000 + -(-rows * cols // 8) * 8
+    copies = (_lib.HalfCopy * 2)((5000, 1, 0, 0, -1, -1, 1.0), (rows, cols, scaled, 5000, second if turned else -1, 0, scale))
+    status = _lib.lib().s3d_half_copies((ctypes.c_void_p * 2)(other.data_ptr(), x.data_ptr()), copies, 2, half.data_ptr(), same.data_ptr(),
+                                        _lib.stream(dev))
+    _lib.check(status, "s3d_half_copies")
+    bits = lambda t: t.contiguous().view(-1).view(torch.int16)
+    factor = torch.ones(rows, 1, device=dev)
+    factor[:scaled] = scale
+    want = (x * factor).half()
+    assert torch.equal(bits(half[:5000]), bits(other.half()))
+    assert torch.equal(bits(half[5000:5000 + rows * cols]), bits(want))
+    assert torch.equal(same[:rows * cols].view(torch.int32), x.reshape(-1).view(torch.int32)) and not same[rows * cols:].any()
+    if turned:
+        assert torch.equal(bits(half[second:second + rows * cols]), bits(want.t()))
+
+
+def _stage(voxels, channels, heads, window, mode, axes, seed, extent=(3.0, 3.0, 2.0)):
+    dev = torch.device("cuda", 0)
+    scene = synth.make_room(extent, 4, voxels, seed=seed)
+    coords = torch.from_numpy(scene.coords).to(dev)
+    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)[:, :4 + (3 if axes == "XYZ_RGB" else 6)]
+    torch.manual_seed(seed)
+    stage = encoder.Stage(channels, 2, heads, window, 4, downsample=False, cRSE=axes, fp16_mode=mode).to(dev)
+    for name, p in stage.named_parameters():
+        if "table" in name or "bias" in name:
+            torch.nn.init.normal_(p, std=0.1)
+    feats = torch.randn(coords.shape[0], channels, device=dev)
+    return stage, feats, (lambda f: stage(encoder.SparseVoxels(coords, f, 1), signals)[0].feats)
+
+
+def _pass(stage, feats, run, wanted, seed=1, **how):
+    grad = torch.randn(feats.shape, device=feats.device, generator=torch.Generator(device="cuda").manual_seed(seed))
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = run(feats)
+    return out.detach(), torch.autograd.grad(out, wanted, grad, **how)
+
+
+def _nodes(t):
+    seen, todo, names = set(), [t.grad_fn], []
+    while todo:
+        node = todo.pop()
+        if node is None or node in seen:
+            continue
+        seen.add(node)
+        names.append(node.name())
+        todo += [n for n, _ in node.next_functions]
+    return names
+
+
+@pytest.mark.parametrize("voxels,channels,heads,window,mode,axes", [
+    (5000, 48, 6, 5, 2, "XYZ_RGB_NORM"), (5001, 48, 6, 5, 1, "XYZ_RGB"), (3001, 96, 6, 7, 1, "XYZ_RGB_NORM"), (3000, 96, 6, 7, 2, "XYZ_RGB"),
+    (331, 384, 24, 7, 1, "XYZ_RGB_NORM"), (7, 16, 1, 5, 2, "XYZ_RGB_NORM"), (20011, 32, 4, 5, 2, "XYZ_RGB_NORM")])
+@pytest.mark.parametrize("without", ["nothing", "biases", "some gradients"])
+def test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads, window, mode, axes, without):
+    stage, feats, run = _stage(voxels, channels, heads, window, mode, axes, seed=voxels)
+    if without == "biases":
+        for block in stage.blocks:
+            block.attn.qkv.bias = block.mlp.fc1.bias = None
+    feats.requires_grad_(without != "some gradients")
+    if without == "some gradients":
+        for name, p in stage.named_parameters():
+            p.requires_grad_(not any(part in name for part in ("blocks.0.attn.proj.weight", "norm2.bias", "key_xyz_table", "fc2", "blocks.1.attn.qkv")))
+    wanted = [t for t in (feats, *stage.parameters()) if t.requires_grad]
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert sum("Branches" in name for name in _nodes(run(feats))) == 2
+    out, got = _pass(stage, feats, run, wanted)
+    monkeypatch.setattr(encoder, "trained_branches", lambda *_: None)
+    ref, want = _pass(stage, feats, run, wanted)
+    assert torch.equal(out, ref)
+    # the same kernels, but for GELU's derivative (fp32, some ulps, which turn single roundings to fp16 of the hidden
+    # layer's gradient: 2^-11 of an element each) and the order of the tables' fp32 sums; two blocks
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and g.shape == w.shape
+        assert (g - w).double().norm() <= 2 ** -11 * w.double().norm() + 1e-12
+
+
+def test_gradients_of_gradients_and_absent_ones(hip_lib, monkeypatch):
+    stage, feats, run = _stage(900, 48, 3, 5, 2, "XYZ_RGB_NORM", seed=3)
+    feats.requires_grad_()
+    wanted = [feats, *stage.parameters()]
+    _, plain = _pass(stage, feats, run, wanted)
+    _, graph = _pass(stage, feats, run, wanted, create_graph=True)
+    for g, w in zip(graph, plain):
+        assert (g.detach() - w).norm() <= 2e-3 * w.norm()      # torch's products of fp16 numbers for the library's
+    assert graph[0].requires_grad
+    # the sum alone, without the MLP's branch: its parameters get no gradient
+    block = stage.blocks[0]
+    results = []
+    for whole in (True, False):
+        if not whole:
+            monkeypatch.setattr(encoder, "trained_branches", lambda *_: None)
+        seen = []
+        monkeypatch.setattr(block, "forward_trained", lambda *a, f=type(block).forward_trained: seen.append(f(block, *a)) or seen[-1])
+        with torch.autocast("cuda", dtype=torch.float16):
+            run(feats)
+        summed = seen[0][0]
+        results.append(torch.autograd.grad(summed, wanted, torch.ones_like(summed), allow_unused=True))
+        monkeypatch.delattr(block, "forward_trained")
+    assert any(g is None for g in results[0])
+    for g, w in zip(*results):
+        assert (g is None) == (w is None) and (g is None or (g - w).norm() <= 2e-3 * w.norm() + 1e-12)
+
+
+def test_what_steps_aside(hip_lib):
+    """A layer of another kind, a hook, parameters in fp16 and a frozen block take the layers one by one."""
+    def nodes(stage, run, feats):
+        with torch.autocast("cuda", dtype=torch.float16):
+            return sum("Branches" in name for name in _nodes(run(feats)))
+
+    stage, feats, run = _stage(500, 48, 3, 5, 2, "XYZ_RGB", seed=4)
+    assert nodes(stage, run, feats) == 2
+    handle = stage.blocks[0].mlp.fc1.register_forward_hook(lambda *_: None)
+    assert nodes(stage, run, feats) == 1
+    handle.remove()
+    stage.blocks[1].mlp.act = torch.nn.ReLU()
+    assert nodes(stage, run, feats) == 1
+    stage.blocks[0].attn.fp16_mode = 0
+    assert nodes(stage, run, feats) == 0
+    stage.blocks[0].attn.fp16_mode = 1
+    assert nodes(stage, run, feats) == 1
+    for p in stage.blocks[0].parameters():
+        p.requires_grad_(False)
+    assert nodes(stage, run, feats) == 0
