@@ -16,9 +16,10 @@
 // is half of the banks or a quarter of them, and additions of lanes that hold 16 columns meet in none that costs (5.1 and
 // 6.7 clocks a wavefront, 4.7 and 6.7 without any conflict; rows of 72 cells: 6.1 and 8.1).  Eight wavefronts and 128
 // registers, two workgroups a CU: with four wavefronts and 168 registers, three workgroups, the table gradients and tables of
-// a wavefront did not fit beside the rest, and 300 MB a call went to memory and back for it.
-// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 153 us, by key 131
-// (one kernel on 64 x 64 tiles: 523).  VALU 44 and 57 % of the time, LDS addressed 20 %, matrix pipe 11 %; a wavefront waits
+// a wavefront did not fit beside the rest, and 300 MB a call went to memory and back for it.  Registers are what is scarce:
+// with fourteen of them spilled inside the loop the launch by query took 153 us, with none 138.
+// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 138 us, by key 133
+// (one kernel on 64 x 64 tiles: 523).  VALU 48 and 55 % of the time, LDS addressed 20 %, matrix pipe 11 %; a wavefront waits
 // for 55 % of its time, at the barriers and for the pairs and coordinates it reads.
 #include "attn_strip.h"
 
@@ -238,6 +239,13 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     __shared__ float sums_s[kStripWaves][kStrip], grad_s;
     __shared__ __align__(16) Exact4<TF> features_s[kKinds][64];        // q or k, dout of the strip's voxels
     __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s;
+    // Pieces of the table's operands that wait in LDS, as many as leave room for two workgroups a CU (81,864 of 81,920 bytes by
+    // query in fp32).  In registers they would not fit beside the rest, and a spilled operand comes back from memory behind the
+    // pairs of the next strip, which are on their way then: loads return in order.
+    constexpr int kParts = sizeof(Table) / 8, kPieces = kParts * kOwn;
+    constexpr int kShared = kByKey || kPieces < kOwn + 2 ? kPieces : kOwn + 2, kKeptPieces = kPieces - kShared;
+    struct TableParts { u32x2 part[kParts]; };
+    __shared__ u32x2 table_s[kShared][kStripThreads];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int H = a.H, HD = H * D;
     const uint32_t stride = static_cast<uint32_t>(a.row_stride);       // of q, k, v
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
 
     // The table by channel, for dx: rows 4 e + g4 of a tile, whose cells a read of the histogram takes side by side.  Tile
     // 8 i + wave is this wavefront's.
-    Table table[kOwn];
+    u32x2 table[kKeptPieces > 0 ? kKeptPieces : 1];
     {
         const T *from = static_cast<const T *>(kByKey ? a.table_k : a.table_q) + h * D + c16;
 #pragma unroll
@@ -271,8 +279,16 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                     v[e] = finite(x) ? x : 0.0f;
                 }
             }
-            if constexpr (std::is_same<Table, Parts4<__half>>::value) table[i].set(v, 1.0f / scale_table);
-            else table[i].set(v);
+            Table x;
+            if constexpr (std::is_same<Table, Parts4<__half>>::value) x.set(v, 1.0f / scale_table);
+            else x.set(v);
+            const TableParts parts = __builtin_bit_cast(TableParts, x);
+#pragma unroll
+            for (int k = 0; k < kParts; ++k) {
+                const int piece = k * kOwn + i;
+                if (piece < kKeptPieces) table[piece] = parts.part[k];
+                else table_s[piece - kKeptPieces][tid] = parts.part[k];
+            }
         }
     }
     Unit4 unit, identity;                    // for a tile's rows as the histogram is read, for rows in order
@@ -306,10 +322,17 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     // pair with the window's j-th voxel: by query [key][query], by key likewise
     auto pair_at = [&](int4 column, int n) { return column.w < 0 ? 0 : column.w + (kByKey ? (column.x - column.z) * n : column.x - column.z); };
     auto pair_step = [&](int4 column, int n) { return column.w < 0 ? 0 : kByKey ? 1 : n; };
+    // the first of a lane's four channels, in a form that the compiler does not add to the pointers outside of the loop: that
+    // would keep two registers for each
+    auto part4 = [&]() {
+        uint32_t c = 4 * g4;
+        asm volatile("" : "+v"(c));
+        return c;
+    };
     auto fetch = [&](int n) {
         if (wave < kKinds)
             ahead.x.load((wave == 0 ? gx : gd) + (static_cast<uint64_t>(static_cast<uint32_t>(ahead.column.y)) *
-                                                  (wave == 0 ? stride : static_cast<uint32_t>(HD)) + 4 * g4));
+                                                  (wave == 0 ? stride : static_cast<uint32_t>(HD)) + part4()));
         const int first = pair_at(ahead.column, n), step = pair_step(ahead.column, n);
 #pragma unroll
         for (int s = 0; s < kKept; ++s) ahead.kept[s] = records[first + min(reach0 + s * kStripReach, n - 1) * step];
@@ -386,8 +409,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         // what the products of the pairs themselves start with, while the histograms are filled
         Raw4<TF> y, z;
         auto fetch_keys = [&](int row) {
-            y.load(gy + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * stride + 4 * g4));
-            if constexpr (kByKey) z.load(gd + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(HD) + 4 * g4));
+            y.load(gy + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * stride + part4()));
+            if constexpr (kByKey) z.load(gd + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(HD) + part4()));
         };
         fetch_keys(key_row);
 
@@ -537,7 +560,13 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             }
             Cell c;
             c.template set<sizeof(TF) == 2>(l, kGradCell<TF>);       // (the table's operand and the features are the nearest)
-            acc_t = product(table[i], c, acc_t);
+            TableParts parts;
+#pragma unroll
+            for (int k = 0; k < kParts; ++k) {
+                const int piece = k * kOwn + i;
+                parts.part[k] = piece < kKeptPieces ? table[piece < kKeptPieces ? piece : 0] : table_s[piece < kKeptPieces ? 0 : piece - kKeptPieces][tid];
+            }
+            acc_t = product(__builtin_bit_cast(Table, parts), c, acc_t);
             f32x4_t g = product(transposed(c, unit), feature, f32x4_t{});
 #pragma unroll
             for (int e = 0; e < 4; ++e) grads[0][i][e] = fmaf(g[e], grad, grads[0][i][e]);
@@ -579,7 +608,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = static_cast<float>(sums[e]) * (which > 0 ? 1.0f / kLiftP<TF> : 1.0f);
-            if (there) store4(static_cast<TF *>(which > 0 ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * D + g4 * 4, o);
+            if (there) store4(static_cast<TF *>(which > 0 ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * D + part4(), o);
         }
     }
     // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]
