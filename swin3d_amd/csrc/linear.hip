@@ -8,11 +8,14 @@
 // spread over all banks; W goes in as the first operand, so that a lane ends up with four neighbouring outputs of one
 // row, and the tile leaves through LDS as whole rows.
 //
-// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 202 us (178
-// without GELU) against 416 us as product and GELU apart, at 2.4 of the 4.7 TB/s that a copy reaches; 80 -> 240, 125 us against 207.  At the
+// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 173 us against
+// 416 us as product and GELU apart; 80 -> 240, 108 us against 207, at 3.6 of the 4.7 TB/s that a copy reaches.  At the
 // deepest the tiles are few and a tile's chain of chunks is what counts: 811 rows, 384 -> 384, 5 us against 18 through
 // torch, whose launch alone takes the host that long.
+#include "attn_kernels.h"
 #include "linear.h"
+
+#include <type_traits>
 
 namespace s3d {
 namespace {
@@ -60,34 +63,47 @@ template <int WM, int WN, int TM, int TN> struct Tile {
     static constexpr int kWM = WM, kTM = TM, kTN = TN;
     static constexpr int kM = 32 * WM * TM, kN = 32 * WN * TN;
     static constexpr int kStage = (kM + kN) * kChunk * 2;             // bytes of one staged chunk
-    static constexpr int kPitch = kN + 8;                             // of the finished tile
-    static constexpr int kLds = 2 * kStage > kM * kPitch * 2 ? 2 * kStage : kM * kPitch * 2;
+    static constexpr int kPitch = 32 * TN + 8;                        // of 32 finished rows of a wavefront
+    static_assert(kThreads / 64 * 32 * kPitch * 2 <= kStage, "they fit a buffer");
+    static constexpr int kLds = 2 * kStage;
     static constexpr int kLoads = (kM + kN) * kPieces / kThreads;     // pieces per thread and chunk
 };
 
+// A workgroup works on tile after tile: the first chunk of the next one is on its way in registers while the last chunk is
+// multiplied and the finished rows leave, each wavefront's through its own part of the buffer that has just been multiplied (no
+// barrier).  With a workgroup a tile, a tile's first load waited for all that.  us at 600,000 rows, before / so: 80 -> 240
+// 126 / 108, 80 -> 80 52 / 43, 80 -> 320 with GELU 201 / 173 (of which GELU's instructions are 98), 320 -> 80 117 / 105; 199,327
+// rows, 48 -> 144 24 / 18; 9,000 rows, 640 -> 1920 36 / 32; 3,000 rows, where every tile has a workgroup, the same.  Two chunks
+// ahead, as one sequence over the tiles, was 5 % slower at K = 80 and up to 40 % at K above 300 (addresses, and a loop in two
+// halves).
 template <typename L, Behind kBehind>
 __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
                                                              const _Float16 *__restrict__ bias, _Float16 *__restrict__ y,
-                                                             const _Float16 *__restrict__ gelu_at, int M, int N, int K, int tiles_n, int tiles)
+                                                             const _Float16 *__restrict__ gelu_at, int M, int N, int K, int tiles_n,
+                                                             int tiles)
 {
     constexpr int TM = L::kTM, TN = L::kTN;
     __shared__ __align__(16) char smem[L::kLds];
     // workgroups b, b + 8, .. run on one XCD: they get neighbouring tiles, which share rows of X
-    const int share = (tiles + 7) / 8, tile = static_cast<int>(blockIdx.x) % 8 * share + static_cast<int>(blockIdx.x) / 8;
-    if (tile >= tiles) return;
-    const int m0 = tile / tiles_n * L::kM, n0 = tile % tiles_n * L::kN;
+    const int share = (tiles + 7) / 8, begin = static_cast<int>(blockIdx.x) % 8 * share, end = min(begin + share, tiles);
+    const int step = static_cast<int>(gridDim.x) / 8;
+    int tile = begin + static_cast<int>(blockIdx.x) / 8;
+    if (tile >= end) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave % L::kWM * (32 * TM), wave_n = wave / L::kWM * (32 * TN);
     const int r32 = lane & 31, half = lane >> 5;
+    const int whole = (K - 1) / kChunk;      // chunks before the last one
 
     // this thread's pieces of a chunk: row (tid / 8 + 32 i) of [X rows, W rows], piece tid % 8
     const int piece = tid % kPieces, row = tid / kPieces;
     const _Float16 *from[L::kLoads];
+    auto aim = [&](int m0, int n0) {
 #pragma unroll
-    for (int i = 0; i < L::kLoads; ++i) {
-        const int r = row + i * (kThreads / kPieces);
-        from[i] = (r < L::kM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r - L::kM, N - 1)) * K) + piece * 8;
-    }
+        for (int i = 0; i < L::kLoads; ++i) {
+            const int r = row + i * (kThreads / kPieces);
+            from[i] = (r < L::kM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r - L::kM, N - 1)) * K) + piece * 8;
+        }
+    };
     uint4 held[L::kLoads];
     auto fetch = [&](int k0) {
         if (k0 + piece * 8 < K) {
@@ -100,7 +116,7 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
 #pragma unroll
         for (int i = 0; i < L::kLoads; ++i) to[placed(row + i * (kThreads / kPieces), piece)] = held[i];
     };
-    f32x16 acc[TM][TN] = {};
+    f32x16 acc[TM][TN];
     auto multiply = [&](int buffer, int steps) {
         const half8 *at = reinterpret_cast<const half8 *>(smem + buffer * L::kStage);
 #pragma unroll
@@ -119,54 +135,83 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
     };
 #pragma unroll
     for (int i = 0; i < L::kLoads; ++i) held[i] = make_uint4(0, 0, 0, 0);
+    int buffer = 0;
+    aim(tile / tiles_n * L::kM, tile % tiles_n * L::kN);
     fetch(0);
     put(0);
     __syncthreads();
-    const int whole = (K - 1) / kChunk;      // chunks before the last one
-    for (int c = 0; c < whole; ++c) {
-        fetch((c + 1) * kChunk);
-        multiply(c & 1, kChunk / 16);
-        put((c + 1) & 1);
-        __syncthreads();
-    }
-    multiply(whole & 1, (K - whole * kChunk) / 16);
-    __syncthreads();
-
-    // a lane's outputs: row r32 of X, columns 8 g + 4 half .. + 3 of W's 32
-    _Float16 *out = reinterpret_cast<_Float16 *>(smem);
+    for (; tile < end; tile += step) {
+        const int m0 = tile / tiles_n * L::kM, n0 = tile % tiles_n * L::kN;
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int n = wave_n + j * 32 + 8 * g + 4 * half;
-            half4 b = {0, 0, 0, 0};
-            if (bias) b = *reinterpret_cast<const half4 *>(bias + min(n0 + n, N - 4));
+            for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+        for (int c = 0; c < whole; ++c) {
+            fetch((c + 1) * kChunk);
+            multiply(buffer, kChunk / 16);
+            buffer ^= 1;
+            put(buffer);
+            __syncthreads();
+        }
+        // what the end of the tile reads, before the next tile's first chunk: loads return in order
+        half4 b[TN][4];
+        half8 at[TM][2 * TN];
+        constexpr int kRowPieces = TN * 4;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                half4 o;
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = acc[i][j][4 * g + e] + static_cast<float>(b[e]);
-                    o[e] = static_cast<_Float16>(kBehind == Behind::kGelu ? gelu(v) : v);
+            for (int g = 0; g < 4; ++g) {
+                b[j][g] = half4{0, 0, 0, 0};
+                if (bias) b[j][g] = *reinterpret_cast<const half4 *>(bias + min(n0 + wave_n + j * 32 + 8 * g + 4 * half, N - 4));
+            }
+        if constexpr (kBehind == Behind::kGeluGrad) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int t = 0; t < 2 * TN; ++t) {
+                    const int e = t * 64 + lane, r = min(m0 + wave_m + i * 32 + e / kRowPieces, M - 1);
+                    at[i][t] = *reinterpret_cast<const half8 *>(gelu_at + static_cast<int64_t>(r) * N + min(n0 + wave_n + e % kRowPieces * 8, N - 8));
                 }
-                *reinterpret_cast<half4 *>(out + (wave_m + i * 32 + r32) * L::kPitch + n) = o;
+        }
+        const int next = tile + step;
+        if (next < end) {
+            aim(next / tiles_n * L::kM, next % tiles_n * L::kN);
+            fetch(0);
+        }
+        multiply(buffer, (K - whole * kChunk) / 16);
+        __syncthreads();
+        // a lane's outputs: row r32 of X, columns 8 g + 4 half .. + 3 of W's 32.  They become rows in the wavefront's own part of
+        // the buffer that is free now.
+        _Float16 *out = reinterpret_cast<_Float16 *>(smem + buffer * L::kStage) + wave * (32 * L::kPitch);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    half4 o;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = acc[i][j][4 * g + e] + static_cast<float>(b[j][g][e]);
+                        o[e] = static_cast<_Float16>(kBehind == Behind::kGelu ? gelu(v) : v);
+                    }
+                    *reinterpret_cast<half4 *>(out + r32 * L::kPitch + j * 32 + 8 * g + 4 * half) = o;
+                }
+#pragma unroll
+            for (int t = 0; t < 2 * TN; ++t) {
+                const int e = t * 64 + lane, r = e / kRowPieces, n = e % kRowPieces * 8;
+                half8 v = *reinterpret_cast<const half8 *>(out + r * L::kPitch + n);
+                if constexpr (kBehind == Behind::kGeluGrad) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = static_cast<_Float16>(static_cast<float>(v[k]) * gelu_slope(static_cast<float>(at[i][t][k])));
+                }
+                if (m0 + wave_m + i * 32 + r < M && n0 + wave_n + n < N)
+                    *reinterpret_cast<half8 *>(y + static_cast<int64_t>(m0 + wave_m + i * 32 + r) * N + n0 + wave_n + n) = v;
             }
         }
-    __syncthreads();
-    constexpr int kRowPieces = L::kN / 8;
-#pragma unroll
-    for (int t = tid; t < L::kM * kRowPieces; t += kThreads) {
-        const int r = t / kRowPieces, n = t % kRowPieces * 8;
-        if (m0 + r < M && n0 + n < N) {
-            const int64_t to = static_cast<int64_t>(m0 + r) * N + n0 + n;
-            half8 piece = *reinterpret_cast<const half8 *>(out + r * L::kPitch + n);
-            if constexpr (kBehind == Behind::kGeluGrad) {
-                const half8 at = *reinterpret_cast<const half8 *>(gelu_at + to);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) piece[e] = static_cast<_Float16>(static_cast<float>(piece[e]) * gelu_slope(static_cast<float>(at[e])));
-            }
-            *reinterpret_cast<half8 *>(y + to) = piece;
-        }
+        buffer ^= 1;
+        if (next < end) put(buffer);
+        __syncthreads();
     }
 }
 
@@ -176,12 +221,14 @@ int launch(const LinearArgs &a, hipStream_t stream)
     const int tiles_n = (a.N + L::kN - 1) / L::kN;
     const int64_t tiles = ceil_div(a.M, L::kM) * tiles_n;
     if (tiles > (1 << 30)) return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M = %lld rows", (long long)a.M);
-    const dim3 grid(static_cast<unsigned>(ceil_div(tiles, 8) * 8));
     auto kernel = a.gelu_at ? linear_kernel<L, Behind::kGeluGrad> : a.gelu ? linear_kernel<L, Behind::kGelu> : linear_kernel<L, Behind::kNothing>;
+    // as many workgroups as fit the chip (by LDS), or one a tile
+    constexpr int kPerCu = 160 * 1024 / L::kLds < 2 ? 1 : 160 * 1024 / L::kLds < 4 ? 160 * 1024 / L::kLds : 4;
+    const int64_t slots = static_cast<int64_t>(kPerCu) * device_cus();
+    const dim3 grid(static_cast<unsigned>(ceil_div(tiles < slots ? tiles : slots, 8) * 8));
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, static_cast<const _Float16 *>(a.x), static_cast<const _Float16 *>(a.w),
                        static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<const _Float16 *>(a.gelu_at),
-                       static_cast<int>(a.M), a.N, a.K, tiles_n,
-                       static_cast<int>(tiles));
+                       static_cast<int>(a.M), a.N, a.K, tiles_n, static_cast<int>(tiles));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
@@ -195,13 +242,13 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     if (a.M == 0) return S3D_OK;
     if (!a.x || !a.w || !a.y) return fail(S3D_ERR_NULL_POINTER, "s3d_linear: null device pointer");
     // Tiles of 64 x 64 as long as larger ones would leave CUs without work; then 128 rows by the width that pads N least,
-    // the widest of those that still give every CU two tiles.  192 columns take most of a wavefront's registers: with
-    // GELU only where the tile is the whole row.
+    // the widest of those that still give every CU two tiles.  192 columns take all of a wavefront's registers: with GELU only
+    // where the tile is the whole row, with its derivative not at all (63 would spill).
     if (ceil_div(a.M, 64) * ((a.N + 63) / 64) < 1024) return launch<Tile<2, 2, 1, 1>>(a, stream);
     auto padded = [&](int width) { return (a.N + width - 1) / width * width; };
     auto enough = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width) >= 512; };
     const int least = padded(64);
-    if (padded(192) == least && enough(192) && (!(a.gelu || a.gelu_at) || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
+    if (padded(192) == least && enough(192) && !a.gelu_at && (!a.gelu || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
     if (padded(128) == least && enough(128)) return launch<Tile<2, 2, 2, 2>>(a, stream);
     return launch<Tile<2, 2, 2, 1>>(a, stream);
 }

@@ -75,10 +75,12 @@ def _nodes(t):
 
 @pytest.mark.parametrize("voxels,channels,heads,window,mode,axes", [
     (5000, 48, 6, 5, 2, "XYZ_RGB_NORM"), (5001, 48, 6, 5, 1, "XYZ_RGB"), (3001, 96, 6, 7, 1, "XYZ_RGB_NORM"), (3000, 96, 6, 7, 2, "XYZ_RGB"),
-    (331, 384, 24, 7, 1, "XYZ_RGB_NORM"), (7, 16, 1, 5, 2, "XYZ_RGB_NORM"), (20011, 32, 4, 5, 2, "XYZ_RGB_NORM")])
+    (331, 384, 24, 7, 1, "XYZ_RGB_NORM"), (7, 16, 1, 5, 2, "XYZ_RGB_NORM"), (20011, 32, 4, 5, 2, "XYZ_RGB_NORM"),
+    (70001, 48, 6, 5, 2, "XYZ_RGB")])       # dense layers of several tiles a workgroup
 @pytest.mark.parametrize("without", ["nothing", "biases", "some gradients"])
 def test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads, window, mode, axes, without):
-    stage, feats, run = _stage(voxels, channels, heads, window, mode, axes, seed=voxels)
+    stage, feats, run = _stage(voxels, channels, heads, window, mode, axes, voxels, (6.0, 5.0, 2.5) if voxels > 30000 else (3.0, 3.0, 2.0))
+    assert feats.shape[0] > 0.75 * voxels
     if without == "biases":
         for block in stage.blocks:
             block.attn.qkv.bias = block.mlp.fc1.bias = None

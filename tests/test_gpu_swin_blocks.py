@@ -46,6 +46,19 @@ def test_gelu_of_every_number(hip_lib):
     assert bool((got[0] == float("inf")).all()) and bool(got[1:].isnan().all())
 
 
+@pytest.mark.parametrize("m,n,k,gelu", [(300_001, 80, 16, True), (140_000, 240, 80, False), (131_137, 64, 64, True), (99_999, 192, 48, False),
+                                        (70_007, 136, 144, False)])
+def test_linear_of_several_tiles_a_workgroup(hip_lib, m, n, k, gelu):
+    """The same rows in pieces that have a workgroup a tile: the same bits."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, device="cuda", generator=gen).half()
+    w, b = torch.randn(n, k, device="cuda", generator=gen).half(), torch.randn(n, device="cuda", generator=gen).half()
+    for bias in (b, None):
+        whole = linear_rows(x, w, bias, gelu=gelu)
+        for first in range(0, m, 4001):
+            assert torch.equal(whole[first:first + 4001], linear_rows(x[first:first + 4001].clone(), w, bias, gelu=gelu))
+
+
 def test_linear_refuses_what_it_cannot_do(hip_lib):
     x, w = torch.randn(5, 24, device="cuda").half(), torch.randn(8, 24, device="cuda").half()
     assert linear_rows(x, w, None) is None and linear_rows(x.float(), w.float(), None) is None
