@@ -54,9 +54,8 @@ struct BwdArgs {
     float *delta;     // [N,H] dout_i . o_i
     float *tgrad;     // per-wavefront table gradients of a sweep: [wavefront][kind][64 * BLK rows][D]
     int64_t *pos_base;   // [N]: at a window's first sorted position, the pairs (n^2) of the windows before it
-    const float2 *pd;    // [H][pairs]: (dL, P) of the pair sweeps at base + i n + j
-    const float *dl_t;   // [H][pairs]: dL at base + j n + i
-    int64_t pairs;       // capacity of pd and dl_t per head
+    const float2 *pd;    // [H][pairs]: (dL, P) of the pair sweeps at base + j n + i
+    int64_t pairs;       // capacity of pd per head
     int32_t *units;   // H * kQueues work counters (kCounterStride apart), the unit count, (window, chunk) per unit
     int32_t H, D, nd, total_rows;
     int64_t N, W, table_len;
@@ -703,7 +702,8 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
         const int64_t before_u = (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(before >> 32))) << 32) |
                                  static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(before)));
         const bool fits = before_u + static_cast<int64_t>(n_w) * n_w <= a.pairs;
-        const int64_t stored_at = static_cast<int64_t>(h) * a.pairs + before_u + own_in;
+        // (records lie by key and, of a key, by query)
+        const int64_t stored_at = static_cast<int64_t>(h) * a.pairs + before_u + (KEY_OWNED ? static_cast<int64_t>(own_in) * n_w : own_in);
         float own_c[ND];
 #pragma unroll
         for (int n = 0; n < ND; ++n) own_c[n] = a.n_coords[static_cast<int64_t>(s0 + own_in) * ND + n];
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
         };
         // a window beyond the store reads the first record of the head instead (never used: `fits` masks it)
         const int64_t rec_base = fits ? stored_at : static_cast<int64_t>(h) * a.pairs;
-        const int rec_stride = fits ? n_w : 0;
+        const int rec_stride = !fits ? 0 : KEY_OWNED ? 1 : n_w;
         auto fetch_record = [&](int it) {
             const int st = min(it * ng + grp, n_w - 1);
             const int64_t rec_at = rec_base + static_cast<int64_t>(st) * rec_stride;
@@ -737,7 +737,7 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
             if constexpr (KIND == 1) rec = a.pd[rec_at];
             else if constexpr (KIND == 2) rec.x = a.pd[rec_at].x;
             else if constexpr (KIND == 3) rec.x = a.pd[rec_at].y;
-            else rec.x = a.dl_t[rec_at];
+            else rec.x = a.pd[rec_at].x;
             return rec;
         };
         // the next unit's ticket, drawn here: its round trip overlaps the unit's first loads
@@ -1276,11 +1276,9 @@ size_t bwd_tgrad_bytes(int H, int D, int nd)
     return align_up(sizeof(float) * static_cast<size_t>(bwd_grid(H, kTablesPerCu)) * kBwdWaves * 2 * (64 * nd) * D, 256);
 }
 
-// the pair path's part of the workspace: window pair offsets, (dL, P) and transposed dL of every (pair, head), and
-// the pair sweeps' work list
+// the pair path's part of the workspace: window pair offsets, (dL, P) of every (pair, head), and the pair sweeps' work list
 size_t bwd_pos_base_bytes(int64_t N) { return align_up(sizeof(int64_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
-size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(sizeof(float2) * static_cast<size_t>(H) * pairs, 256); }
-size_t bwd_dlt_bytes(int H, int64_t pairs) { return align_up(sizeof(float) * static_cast<size_t>(H) * pairs, 256); }
+size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(sizeof(float2) * (static_cast<size_t>(H) * pairs + kPairSpare), 256); }
 // the last part of every form's workspace: the identity row map that stands in for a null n2n
 size_t bwd_row_map_bytes(int64_t N) { return align_up(sizeof(int32_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
 
@@ -1306,7 +1304,7 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_attn_bwd_workspace_
     size_t need = bwd_units_bytes(W, N, H, pairs) + bwd_delta_bytes(N, H) + bwd_tgrad_bytes(H, D, nd) +
                   bwd_pos_base_bytes(N) + bwd_row_map_bytes(N);
     if (pairs > 0) {
-        need += bwd_pd_bytes(H, pairs) + bwd_dlt_bytes(H, pairs) + align_up(attn_sweep_workspace_bytes(H, W, N), 256);
+        need += bwd_pd_bytes(H, pairs) + align_up(attn_sweep_workspace_bytes(H, W, N), 256);
         // the tile form works in the whole of it (whether it applies depends on the rows of the single axes)
         const size_t tiles = D == 16 ? attn_tile_bwd_bytes(H, nd, N, W, pairs) + bwd_row_map_bytes(N) : 0;
         if (need < tiles) need = tiles;
@@ -1417,10 +1415,7 @@ int attn_bwd(
     if (pairs > 0) {
         float2 *pd = reinterpret_cast<float2 *>(at);
         at += bwd_pd_bytes(H, pairs);
-        float *dl_t = reinterpret_cast<float *>(at);
-        at += bwd_dlt_bytes(H, pairs);
         a.pd = pd;
-        a.dl_t = dl_t;
         pr.f.q = q; pr.f.k = k; pr.f.v = v;
         pr.f.row_stride = qkv_stride;
         pr.grad_stride = grad_stride;
@@ -1435,7 +1430,7 @@ int attn_bwd(
         pr.stat_max = out_max; pr.stat_sum = out_sum; pr.delta = a.delta;
         pr.dq = dq; pr.dk = dk; pr.dv = dv;
         pr.pos_base = a.pos_base;
-        pr.pd = pd; pr.dl_t = dl_t; pr.pairs = pairs;
+        pr.pd = pd; pr.pairs = pairs;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (N > 0 && W > 0 && attn_tile_bwd_applies(a.rows, nd, D, pairs))

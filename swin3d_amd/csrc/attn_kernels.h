@@ -70,6 +70,7 @@ int device_cus();
 
 // The pair sweeps of the backward on the sweep kernel's work list (built here, in b.f.workspace, which needs
 // attn_sweep_workspace_bytes): dq, dk, dv, and dL, P of every (pair, head) for the table-gradient kernels.
+constexpr int kPairSpare = 4;     // records that a lane of the key-owned sweep reads at a time
 struct BwdPairArgs {
     AttnArgs f;                  // shape, q, k, v, tables, index arrays (n2n required), rows[] / base[], workspace
     const void *dout;            // [N,H,D]
@@ -77,9 +78,8 @@ struct BwdPairArgs {
     void *dq, *dk, *dv;          // [N,H,D], rows `grad_stride` elements apart (q, k, v: f.row_stride)
     int64_t grad_stride;
     const int64_t *pos_base;     // [N]: at a window's first sorted position, the pairs of the windows before it
-    float2 *pd;                  // [H][pairs]: (dL, P) at base + i n + j  (i, j: query, key position inside the window)
-    float *dl_t;                 // [H][pairs]: dL at base + j n + i
-    int64_t pairs;               // capacity of pd and dl_t per head; windows beyond it are skipped
+    float2 *pd;                  // [H][pairs], and kPairSpare more: (dL, P) at base + j n + i  (i, j: query, key position inside the window)
+    int64_t pairs;               // capacity of pd per head; windows beyond it are skipped
 };
 int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream);
 

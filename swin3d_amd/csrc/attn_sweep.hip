@@ -727,19 +727,26 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
 //   kKeyOwned = false: lane = query i, streams the keys j:    dq_i += dL (k_j + Tq(i,j))
 //   kKeyOwned = true:  lane = key j, streams the queries i:   dk_j += dL (q_i + Tk(i,j)),  dv_j += P dout_i
 // with P = exp(L - max_i) / sum_i from the forward's saved statistics, dP = dout_i . (v_j + Tv(i,j)) and
-// dL = P (dP - dout_i . o_i).  Every gradient row has one owner and is stored once.  The sweeps also leave dL and
-// P of every (pair, head) for the table-gradient kernels, each in the order its reader wants: the key-owned sweep
-// writes (dL, P) at [head][pairs before the window + i n + j], the query-owned sweep dL at [.. + j n + i] - in both
-// the lanes of a window write consecutive addresses.
+// dL = P (dP - dout_i . o_i).  Every gradient row has one owner and is stored once.  The query-owned sweep leaves (dL, P) of
+// every (pair, head) at [head][pairs before the window + j n + i], where the lanes of a window write consecutive addresses;
+// the key-owned sweep and the table-gradient kernels read them there.
+//
+// The query-owned sweep is bound by VALU issue, the key-owned one by its records' lines.  199,327 voxels in windows of 26,
+// 6 heads of 8, 9 axes, fp16: 338 + 269 us.  When the key-owned sweep made dL and P again (125 of its 280 instructions a pair)
+// and left them in a second order for the table gradients, 326 + 374, with a store of 12 bytes a (pair, head) for 8.
 template <typename T, int D, int HP> __host__ __device__ constexpr int bwd_pair_threads() { return 256; }
+// elements between rows of Tk in the key-owned sweep's LDS (padded as the other's)
+template <typename T, int D, int HP> __host__ __device__ constexpr int key_row_stride()
+{
+    return HP * D + ((HP * D * static_cast<int>(sizeof(T)) / 4) % 8 == 0 ? 16 / static_cast<int>(sizeof(T)) : 0);
+}
 
 // TF is the type the feature rows are stored in (q, k, v, dout and the gradients dq, dk, dv); T the type of the
 // tables and of the arithmetic.  TF = __half with T = float serves an fp16 forward whose backward runs in fp32: the
 // rows are widened as they are loaded and the gradients rounded as they are stored, the arithmetic is that of T = TF
 // = float on widened copies.
-template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned, bool kShared>
-// Wavefronts per SIMD, by register cap.  fp16 at head_dim 8: four (128 registers; -1 to -2 % against the three that
-// the key-owned sweep's 133 registers allow).  fp16 at head_dim 16 and fp32 at head_dim 8: three (168 registers, 3 to
+template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned>
+// Wavefronts per SIMD, by register cap.  fp16 at head_dim 8: four (128 registers).  fp16 at head_dim 16 and fp32 at head_dim 8: three (168 registers, 3 to
 // 20 of them spilled: the backward of the window-7 layer with 6 heads of 16 2.05 -> 1.99 ms, of the headline layer
 // in fp32 2.28 -> 2.05 ms).  fp32 at head_dim 16: two - uncapped it takes 286 registers and runs one wavefront per
 // SIMD (6-head window-7 layer 3.16 ms; capped at 256 with 24 spilled 2.89).
@@ -747,6 +754,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
 {
     const AttnArgs &a = b.f;
     constexpr int kThreads = bwd_pair_threads<T, D, HP>();
+    constexpr int kSlices = kKeyOwned ? 1 : 3;      // the key-owned sweep needs Tk only
     extern __shared__ __align__(16) float smem[];
     __shared__ __align__(16) int group_exit_counter[4];
     int &group_exited = group_exit_counter[0];
@@ -755,7 +763,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
     const int HD = H * D;
     const int hg = a.spread_groups ? blockIdx.x % (H / HP) : (blockIdx.x / kQueues) % (H / HP);
     const int h = hg * HP;
-    constexpr int kRowStride = table_row_stride_heads<T, D, HP>();
+    constexpr int kRowStride = kKeyOwned ? key_row_stride<T, D, HP>() : table_row_stride_heads<T, D, HP>();
     T *tab = reinterpret_cast<T *>(smem);
     {
         const T *gq = static_cast<const T *>(a.table_q);
@@ -767,10 +775,14 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
             const int r = t / (HP * kPieces), hp = t - r * (HP * kPieces);
             const int hh = hp / kPieces, c = (hp - hh * kPieces) * kPerPiece;
             const int64_t g = static_cast<int64_t>(r) * HD + (h + hh) * D + c;
-            T *row = tab + r * kRowStride + hh * 3 * D + c;
-            *reinterpret_cast<uint4 *>(row) = *reinterpret_cast<const uint4 *>(gq + g);
-            *reinterpret_cast<uint4 *>(row + D) = *reinterpret_cast<const uint4 *>(gk + g);
-            *reinterpret_cast<uint4 *>(row + 2 * D) = *reinterpret_cast<const uint4 *>(gv + g);
+            T *row = tab + r * kRowStride + hh * kSlices * D + c;
+            if constexpr (kKeyOwned) {
+                *reinterpret_cast<uint4 *>(row) = *reinterpret_cast<const uint4 *>(gk + g);
+            } else {
+                *reinterpret_cast<uint4 *>(row) = *reinterpret_cast<const uint4 *>(gq + g);
+                *reinterpret_cast<uint4 *>(row + D) = *reinterpret_cast<const uint4 *>(gk + g);
+                *reinterpret_cast<uint4 *>(row + 2 * D) = *reinterpret_cast<const uint4 *>(gv + g);
+            }
         }
     }
     __syncthreads();   // the only workgroup barrier
@@ -786,7 +798,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
     const int total_units = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(ws + ws_total_offset(H))[0]);
     int *counters = static_cast<int *>(a.workspace) + hg * kQueues * kCounterStride;
     constexpr int kRowBytes = kRowStride * static_cast<int>(sizeof(T));
-    constexpr uint32_t kHeadBytes = 3 * D * sizeof(T);
+    constexpr uint32_t kHeadBytes = kSlices * D * sizeof(T);
     const uint32_t tab_addr = __builtin_amdgcn_readfirstlane(lds_address(tab));
     const uint32_t row_bytes = kRowBytes;
     float half_rows[ND], upper[ND];
@@ -797,13 +809,6 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
         upper[n] = crse_upper(a.rows[n]);
         base_off[n] = __builtin_amdgcn_readfirstlane(tab_addr + a.base[n] * kRowBytes);
     }
-    // the one table-row sum that enters the owned gradient as a vector (Tq for dq_i, Tk for dk_j) sits behind the
-    // q-side slice in the query-owned sweep and behind the k-side slice in the key-owned one
-    // kShared: the key-owned sweep reads dL and P from records that the query-owned sweep, which ran before it,
-    // wrote beside its own
-    constexpr bool kRead = kKeyOwned && kShared;
-    constexpr bool kWriteBoth = !kKeyOwned && kShared;
-
     int queue = xcd_id() % kQueues;
     int tried = 0;
     int drawn = 0;
@@ -843,16 +848,13 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
         const int64_t pair_base = b.pos_base[s0];
         const bool fits = pair_base + static_cast<int64_t>(n_w) * n_w <= b.pairs;
 
-        Slice<T, D> own_x[HP], own_y[HP];     // q_i, dout_i  or  k_j, v_j
+        Slice<T, D> own_x[HP], own_y[HP];     // q_i, dout_i
         float own_m[HP], own_inv[HP], own_delta[HP];
         float ci[ND], res_x[HP][D], res_y[kKeyOwned ? HP : 1][D];
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
             const int64_t at_row = static_cast<int64_t>(own_row) * a.row_stride + (h + hh) * D;
-            if constexpr (kKeyOwned) {
-                own_x[hh].load(gk + at_row);
-                if constexpr (!kRead) own_y[hh].load(gv + at_row);
-            } else {
+            if constexpr (!kKeyOwned) {
                 own_x[hh].load(gq + at_row);
                 own_y[hh].load(ggo + static_cast<int64_t>(own_row) * HD + (h + hh) * D);
                 own_m[hh] = b.stat_max[static_cast<int64_t>(own_row) * H + h + hh];
@@ -869,34 +871,68 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
 #pragma unroll
         for (int n = 0; n < ND; ++n) ci[n] = a.n_coords[static_cast<int64_t>(own_pos) * ND + n];
 
-        int row_next = a.n2n[s0 + min(sub, n_w - 1)];
+        // Lanes that share an owned voxel take alternate elements of the stream; of keys, runs of it: a lane's records are then
+        // one after the other.  It reads four of them at a time, four steps ahead: the lanes' records are n_w apart, and a
+        // line fetched for one record would be gone before the next (308 us instead of 269 at the layer below).
+        const int run = (n_w + (1 << gshift) - 1) >> gshift;
+        auto streamed = [&](int it) { return kKeyOwned ? sub * run + it : (it << gshift) + sub; };
+        int row_next = a.n2n[s0 + min(streamed(0), n_w - 1)];
+        constexpr int kRecords = kPairSpare;
+        typedef float f32x4_2 __attribute__((ext_vector_type(4), aligned(8)));
+        float2 rec_now[HP][kRecords], rec_ahead[HP][kRecords];
+        auto records = [&](int it, float2 (&into)[HP][kRecords]) {
+#pragma unroll
+            for (int hh = 0; hh < HP; ++hh) {
+                // (behind the last one of a lane lie others, or what the store has spare: they are not used)
+                const float2 *from = b.pd + static_cast<int64_t>(h + hh) * b.pairs +
+                                     (fits ? pair_base + static_cast<int64_t>(own_in) * n_w + min(streamed(it), n_w - 1) : 0);
+#pragma unroll
+                for (int e = 0; e < kRecords; e += 2) {
+                    const f32x4_2 two = *reinterpret_cast<const f32x4_2 *>(from + e);
+                    into[hh][e] = make_float2(two[0], two[1]);
+                    into[hh][e + 1] = make_float2(two[2], two[3]);
+                }
+            }
+        };
+        if constexpr (kKeyOwned) {
+            records(0, rec_now);
+            records(kRecords, rec_ahead);
+        }
         for (int it = 0; it < max_steps; ++it) {
             if (it + 1 >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
-            const int st = (it << gshift) + sub;
-            const bool valid = st < n_w && own_valid && fits;
+            const int st = streamed(it);
+            const bool valid = st < n_w && (!kKeyOwned || it < run) && own_valid && fits;
             const int st_in = min(st, n_w - 1);
             const int st_pos = s0 + st_in;
             const int st_row = row_next;
-            row_next = a.n2n[s0 + min(st + (1 << gshift), n_w - 1)];
+            row_next = a.n2n[s0 + min(streamed(it + 1), n_w - 1)];
             Slice<T, D> st_x[HP], st_y[HP];   // k_j, v_j  or  q_i, dout_i
-            float st_m[HP], st_inv[HP], st_delta[HP];
 #pragma unroll
             for (int hh = 0; hh < HP; ++hh) {
                 const int64_t at_row = static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D;
                 const int64_t at_grad = static_cast<int64_t>(st_row) * HD + (h + hh) * D;
-                if constexpr (kRead) {
+                if constexpr (kKeyOwned) {
                     st_x[hh].load(gq + at_row);
                     st_y[hh].load(ggo + at_grad);
-                    st_m[hh] = st_inv[hh] = st_delta[hh] = 0.0f;
-                } else if constexpr (kKeyOwned) {
-                    st_x[hh].load(gq + at_row);
-                    st_y[hh].load(ggo + at_grad);
-                    st_m[hh] = b.stat_max[static_cast<int64_t>(st_row) * H + h + hh];
-                    st_inv[hh] = b.stat_sum[static_cast<int64_t>(st_row) * H + h + hh];
-                    st_delta[hh] = b.delta[static_cast<int64_t>(st_row) * H + h + hh];
                 } else {
                     st_x[hh].load(gk + at_row);
                     st_y[hh].load(gv + at_row);
+                }
+            }
+            float2 rec[HP];
+            if constexpr (kKeyOwned) {
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) {
+                    rec[hh] = rec_now[hh][0];
+#pragma unroll
+                    for (int e = 0; e + 1 < kRecords; ++e) rec_now[hh][e] = rec_now[hh][e + 1];
+                }
+                if (it % kRecords == kRecords - 1) {
+#pragma unroll
+                    for (int hh = 0; hh < HP; ++hh)
+#pragma unroll
+                        for (int e = 0; e < kRecords; ++e) rec_now[hh][e] = rec_ahead[hh][e];
+                    records(it + 1 + kRecords, rec_ahead);
                 }
             }
             uint32_t off[ND];
@@ -913,19 +949,11 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
             }
 #pragma unroll
             for (int hh = 0; hh < HP; ++hh) {
-                const Slice<T, D> &qv = kKeyOwned ? st_x[hh] : own_x[hh];
-                const Slice<T, D> &kv = kKeyOwned ? own_x[hh] : st_x[hh];
-                const Slice<T, D> &vv = kKeyOwned ? own_y[hh] : st_y[hh];
-                const Slice<T, D> &gov = kKeyOwned ? st_y[hh] : own_y[hh];
                 const int64_t head_at = static_cast<int64_t>(h + hh) * b.pairs + pair_base;
-                float2 rec = make_float2(0.0f, 0.0f);
-                if constexpr (kRead) {
-                    if (valid) rec = b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in];
-                }
                 float logit = 0.0f, dp = 0.0f;
-                if constexpr (!kRead) {
-                    logit = qv.dot(kv, 0.0f);
-                    dp = gov.dot(vv, 0.0f);
+                if constexpr (!kKeyOwned) {
+                    logit = own_x[hh].dot(st_x[hh], 0.0f);
+                    dp = own_y[hh].dot(st_y[hh], 0.0f);
                 }
                 // sums of three rows of the table that enters the owned gradient as a vector (packed fp16 adds for
                 // fp16 I/O, as the forward adds its value-table rows)
@@ -934,41 +962,35 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
                 Slice<T, D> vec_sum[(ND + kGroup - 1) / kGroup];
 #pragma unroll
                 for (int n = 0; n < ND; ++n) {
-                    Slice<T, D> tq_r, tk_r, tv_r;
-                    tk_r.load_lds(off[n] + hh * kHeadBytes + D * sizeof(T));
-                    if constexpr (!kRead) {
-                        tq_r.load_lds(off[n] + hh * kHeadBytes);
+                    Slice<T, D> vec_r;       // Tk, or Tq
+                    vec_r.load_lds(off[n] + hh * kHeadBytes);
+                    if constexpr (!kKeyOwned) {
+                        Slice<T, D> tk_r, tv_r;
+                        tk_r.load_lds(off[n] + hh * kHeadBytes + D * sizeof(T));
                         tv_r.load_lds(off[n] + hh * kHeadBytes + 2 * D * sizeof(T));
-                        if (Slice<T, D>::kChainLogit) logit = kv.dot(tk_r, qv.dot(tq_r, logit));
-                        else logit += kv.dot(tk_r, qv.dot(tq_r, 0.0f));
-                        if (Slice<T, D>::kChainLogit) dp = gov.dot(tv_r, dp);
-                        else dp += gov.dot(tv_r, 0.0f);
+                        if (Slice<T, D>::kChainLogit) logit = st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, logit));
+                        else logit += st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, 0.0f));
+                        if (Slice<T, D>::kChainLogit) dp = own_y[hh].dot(tv_r, dp);
+                        else dp += own_y[hh].dot(tv_r, 0.0f);
                     }
-                    const Slice<T, D> &vec_r = kKeyOwned ? tk_r : tq_r;
                     if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
                     else vec_sum[n / kGroup].add(vec_r);
                 }
-                const float m_i = kKeyOwned ? st_m[hh] : own_m[hh];
-                const float inv_i = kKeyOwned ? 1.0f / st_inv[hh] : own_inv[hh];
-                const float delta_i = kKeyOwned ? st_delta[hh] : own_delta[hh];
-                const float p = kRead ? rec.y : valid ? __expf(logit - m_i) * inv_i : 0.0f;
-                const float dl = kRead ? rec.x : p * (dp - delta_i);
+                float p, dl;
+                if constexpr (kKeyOwned) {
+                    p = valid ? rec[hh].y : 0.0f;
+                    dl = valid ? rec[hh].x : 0.0f;
+                } else {
+                    p = valid ? __expf(logit - own_m[hh]) * own_inv[hh] : 0.0f;
+                    dl = p * (dp - own_delta[hh]);
+                }
                 // dq_i += dL (k_j + Tq)   or   dk_j += dL (q_i + Tk)
                 st_x[hh].fma_to(res_x[hh], dl);
 #pragma unroll
                 for (int g = 0; g < (ND + kGroup - 1) / kGroup; ++g) vec_sum[g].fma_to(res_x[hh], dl);
                 if constexpr (kKeyOwned) st_y[hh].fma_to(res_y[hh], p);     // dv_j += P dout_i
-                if (valid) {
-                    if constexpr (kRead) {
-                        // nothing to leave: the records are the query-owned sweep's
-                    } else if constexpr (kKeyOwned) {
-                        b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
-                    } else {
-                        b.dl_t[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = dl;
-                        // (dL, P) at [i][j] as well: a lane's records of successive steps are consecutive, the lanes'
-                        // n records apart
-                        if constexpr (kWriteBoth) b.pd[head_at + static_cast<int64_t>(own_in) * n_w + st_in] = make_float2(dl, p);
-                    }
+                if constexpr (!kKeyOwned) {
+                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
                 }
             }
         }
@@ -1109,37 +1131,39 @@ int dispatch_shape(const AttnArgs &a, hipStream_t stream, int what)
 
 namespace {
 
-template <typename T, typename TF, int D, int ND, int HP, bool kShared>
-int launch_bwd_pairs_heads(const BwdPairArgs &b0, hipStream_t stream)
+template <typename T, typename TF, int D, int ND>
+int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
 {
+    // one head per wavefront: with two (fp16, head_dim 8) the pair of sweeps measured 0.3 ms slower at the 6-head layer
+    constexpr int HP = 1;
     const AttnArgs &a = b0.f;
-    const size_t lds = align_up(sizeof(T) * static_cast<size_t>(a.total_rows) * table_row_stride_heads<T, D, HP>(), 16);
-    if (lds > 160 * 1024)
+    // the query-owned sweep keeps a head's slices of the three tables, the key-owned one those of Tk
+    const size_t q_lds = align_up(sizeof(T) * static_cast<size_t>(a.total_rows) * table_row_stride_heads<T, D, HP>(), 16);
+    const size_t k_lds = align_up(sizeof(T) * static_cast<size_t>(a.total_rows) * key_row_stride<T, D, HP>(), 16);
+    if (q_lds > 160 * 1024)
         return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: %d table rows x D=%d need %zu B of LDS (> 160 KiB)",
-                    a.total_rows, D, lds);
-    auto q_sweep = attn_bwd_pairs_kernel<T, TF, D, ND, HP, false, kShared>;
-    auto k_sweep = attn_bwd_pairs_kernel<T, TF, D, ND, HP, true, kShared>;
+                    a.total_rows, D, q_lds);
+    auto q_sweep = attn_bwd_pairs_kernel<T, TF, D, ND, HP, false>;
+    auto k_sweep = attn_bwd_pairs_kernel<T, TF, D, ND, HP, true>;
     constexpr int kThreads = bwd_pair_threads<T, D, HP>();
-    int per_cu = 1;
-    for (auto kernel : {q_sweep, k_sweep}) {
-        if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
-    }
-    {
-        // workgroups per CU: what the registers of the heavier sweep and the tables in LDS allow
-        int fit_q = 0, fit_k = 0;
-        S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit_q, reinterpret_cast<const void *>(q_sweep), kThreads, lds));
-        S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit_k, reinterpret_cast<const void *>(k_sweep), kThreads, lds));
-        per_cu = fit_q < fit_k ? fit_q : fit_k;
-        if (per_cu < 1) per_cu = 1;
-    }
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(q_sweep), q_lds)) return rc;
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k_sweep), k_lds)) return rc;
     const int groups = a.H / HP;
-    const int cus = device_cus();
-    const int slots = per_cu * cus;
-    const int set = kQueues * groups;
-    const int whole = (slots / set) * set;
-    BwdPairArgs b = b0;
-    b.f.spread_groups = 10 * whole < 9 * slots;
-    const int grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
+    // workgroups: as many as registers and the tables in LDS allow, in whole sets as the forward's
+    auto with_grid = [&](BwdPairArgs &b, const void *kernel, size_t lds, int &grid) {
+        int per_cu = 0;
+        S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, lds));
+        if (per_cu < 1) per_cu = 1;
+        const int slots = per_cu * device_cus(), set = kQueues * groups, whole = (slots / set) * set;
+        b.f.spread_groups = 10 * whole < 9 * slots;
+        grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
+        return static_cast<int>(S3D_OK);
+    };
+    BwdPairArgs b = b0, by_key = b0;
+    int grid = 0, key_grid = 0;
+    if (int rc = with_grid(b, reinterpret_cast<const void *>(q_sweep), q_lds, grid)) return rc;
+    if (int rc = with_grid(by_key, reinterpret_cast<const void *>(k_sweep), k_lds, key_grid)) return rc;
+    // (one work list, cut for the query-owned sweep, which takes longer)
     b.f.target_items = grid / groups * (kThreads / 64);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
     const int64_t list_want = (a.W + kListThreads - 1) / kListThreads;
@@ -1147,28 +1171,10 @@ int launch_bwd_pairs_heads(const BwdPairArgs &b0, hipStream_t stream)
     hipLaunchKernelGGL(sweep_count_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
     hipLaunchKernelGGL(sweep_place_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
     S3D_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(q_sweep, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
-    hipLaunchKernelGGL(k_sweep, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
+    hipLaunchKernelGGL(q_sweep, dim3(static_cast<unsigned>(grid)), dim3(kThreads), q_lds, stream, b);
+    hipLaunchKernelGGL(k_sweep, dim3(static_cast<unsigned>(key_grid)), dim3(kThreads), k_lds, stream, by_key);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
-}
-
-template <typename T, typename TF, int D, int ND>
-int launch_bwd_pairs(const BwdPairArgs &b, hipStream_t stream)
-{
-    // one head per wavefront: with two (fp16, head_dim 8) the key-owned sweep needs more than 256 registers and the
-    // pair of sweeps measured 0.3 ms slower at the 6-head layer
-    //
-    // Who computes dL and P for the key-owned sweep.  Either it does, as the query-owned sweep does (the logits, dP,
-    // the exponential: 125 of its 280 instructions per pair and head), or the query-owned sweep, which runs first,
-    // leaves its values at [i][j] as well and the key-owned sweep reads them.  That second copy is written with the
-    // lanes n records apart (a lane's own records of successive steps are consecutive); windows of more than 64
-    // voxels, whose queries have several lanes each on adjacent records, write it in longer runs.  Measured, whole
-    // backward, own values / shared: 1.76 / 1.87 ms on 26-voxel windows (6 heads of 8), 2.24 / 2.12 and 2.33 / 2.25
-    // ms on the window-7 layers of 57 voxels a window (6 heads of 16, 12 of 8).  Shared where the mean window has
-    // more than 32 voxels.
-    if (b.f.N > 32 * b.f.W) return launch_bwd_pairs_heads<T, TF, D, ND, 1, true>(b, stream);
-    return launch_bwd_pairs_heads<T, TF, D, ND, 1, false>(b, stream);
 }
 
 template <typename T, typename TF>
