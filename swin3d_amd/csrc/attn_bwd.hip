@@ -1278,7 +1278,8 @@ size_t bwd_tgrad_bytes(int H, int D, int nd)
 
 // the pair path's part of the workspace: window pair offsets, (dL, P) of every (pair, head), and the pair sweeps' work list
 size_t bwd_pos_base_bytes(int64_t N) { return align_up(sizeof(int64_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
-size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(sizeof(float2) * (static_cast<size_t>(H) * pairs + kPairSpare), 256); }
+// (records take 8 bytes a (pair, head); the size asked for stays 12, which callers may have planned with)
+size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(12 * static_cast<size_t>(H) * pairs + sizeof(float2) * kPairSpare, 256); }
 // the last part of every form's workspace: the identity row map that stands in for a null n2n
 size_t bwd_row_map_bytes(int64_t N) { return align_up(sizeof(int32_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
 
