@@ -851,39 +851,39 @@ __global__ __launch_bounds__(kBwdThreads, (D <= 8 ? (KIND == 1 ? 2 : 3) : (KIND 
     }
 }
 
-// Sums the per-wavefront table gradients of a sweep over the wavefronts of each head.  One wavefront per (kind, flat
-// row, head): its lanes are the D channels of the row times 64 / D shares of the head's slots, which they read 4 D
-// bytes at a time and add up by shuffles at the end.  dst_a / dst_b: the gradient tables of kind 0 / 1 (null = not
-// produced).
+// Sums the per-wavefront table gradients of a sweep over the wavefronts of each head, in 64 bits.  A workgroup takes 64
+// neighbouring words of a head's tables, its four wavefronts share the slots, so that a read is 256 bytes of a slot in a row:
+// the two launches of a call at 6 heads, 312 rows of 8 (63 MB of slots), 18 us; with a wavefront a row, which read 32 bytes of
+// a slot at a time, 51.  dst_a / dst_b: the gradient tables of kind 0 / 1 (null = not produced; blockIdx.y is the kind).
 __global__ __launch_bounds__(256) void bwd_reduce_tables_kernel(BwdArgs a, float *dst_a, float *dst_b, int flat_rows,
                                                                  int groups)
 {
+    __shared__ double shared[4][64];
     const int H = a.H, D = a.D;
-    const int lane = threadIdx.x & 63;
-    const int item = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);   // (kind, row, head)
-    if (item >= 2 * a.total_rows * H) return;
-    const int kind = item / (a.total_rows * H);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int kind = blockIdx.y, h = static_cast<int>(blockIdx.x) % H;
     float *dst = kind == 0 ? dst_a : dst_b;
     if (!dst) return;
-    const int e = item - kind * a.total_rows * H;
-    const int h = e % H, row = e / H;
-    const int c = lane % D, share = lane / D, shares = 64 / D;
+    const int word = static_cast<int>(blockIdx.x) / H * 64 + lane, words = a.total_rows * D;
     const size_t slot_floats = 2 * static_cast<size_t>(flat_rows) * D;
-    const size_t in_slot = (static_cast<size_t>(kind) * flat_rows + row) * D + c;
+    const float *from = a.tgrad + static_cast<size_t>(kind) * flat_rows * D + min(word, words - 1);
     // workgroup b of the sweep serves head (b / kQueues) % H: the head's slots are those of workgroups
     // (set * H + h) * kQueues + x, x < kQueues, four wavefronts each
+    constexpr int kInSet = kQueues * kBwdWaves;
     const int sets = groups / (H * kQueues);
-    const int head_slots = sets * kQueues * kBwdWaves;
-    float sum = 0.0f;
-    for (int x = share; x < head_slots; x += shares) {
-        const int set = x / (kQueues * kBwdWaves), in_set = x - set * (kQueues * kBwdWaves);
-        const size_t slot = (static_cast<size_t>(set) * H + h) * (kQueues * kBwdWaves) + in_set;
-        sum += a.tgrad[slot * slot_floats + in_slot];
+    double sum = 0.0;
+    for (int set = 0; set < sets; ++set) {
+        const float *of_set = from + (static_cast<size_t>(set) * H + h) * kInSet * slot_floats;
+#pragma unroll
+        for (int x = 0; x < kInSet / 4; ++x) sum += of_set[(wave + 4 * x) * slot_floats];
     }
-    for (int other = D; other < 64; other <<= 1) sum += __shfl_xor(sum, other);
+    shared[wave][lane] = sum;
+    __syncthreads();
+    if (wave > 0 || word >= words) return;
+    float all = static_cast<float>((shared[0][lane] + shared[1][lane]) + (shared[2][lane] + shared[3][lane]));
     // the caller's pair count was too small for the window set: windows were skipped, so no sum is valid
-    if (a.pairs > 0 && a.units[units_total_index(H) + 1]) sum = __int_as_float(0x7fc00000);
-    if (share == 0) dst[(static_cast<size_t>(row) * H + h) * D + c] = sum;
+    if (a.pairs > 0 && a.units[units_total_index(H) + 1]) all = __int_as_float(0x7fc00000);
+    dst[(static_cast<size_t>(word / D) * H + h) * D + word % D] = all;
 }
 
 
@@ -1124,9 +1124,8 @@ int launch_sweep_blk(const BwdArgs &a, int grid, hipStream_t stream)
     S3D_HIP_CHECK(hipGetLastError());
     float *dst_a = need_dl ? (KEY_OWNED ? a.dtq : a.dtk) : nullptr;
     float *dst_b = (KEY_OWNED && MODE != 1) ? a.dtv : nullptr;
-    const int items = 2 * a.total_rows * a.H;
-    hipLaunchKernelGGL(bwd_reduce_tables_kernel, dim3(static_cast<unsigned>((items + 3) / 4)), dim3(256), 0, stream,
-                       a, dst_a, dst_b, BLK * 64, grid);
+    hipLaunchKernelGGL(bwd_reduce_tables_kernel, dim3(static_cast<unsigned>((a.total_rows * D + 63) / 64 * a.H), dst_b ? 2 : 1),
+                       dim3(256), 0, stream, a, dst_a, dst_b, BLK * 64, grid);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
@@ -1163,10 +1162,9 @@ int launch_tables_blk(const BwdArgs &a, int grid, hipStream_t stream)
     grid = bwd_grid(a.H, fit < 1 ? 1 : fit > kTablesPerCu ? kTablesPerCu : fit);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kBwdThreads), lds, stream, a);
     S3D_HIP_CHECK(hipGetLastError());
-    const int items = 2 * a.total_rows * a.H;
     float *first = KIND == 0 ? a.dtk : KIND == 3 ? a.dtv : a.dtq;
-    hipLaunchKernelGGL(bwd_reduce_tables_kernel, dim3(static_cast<unsigned>((items + 3) / 4)), dim3(256), 0, stream,
-                       a, first, KIND == 1 ? a.dtv : nullptr, BLK * 64, grid);
+    hipLaunchKernelGGL(bwd_reduce_tables_kernel, dim3(static_cast<unsigned>((a.total_rows * D + 63) / 64 * a.H), KIND == 1 ? 2 : 1),
+                       dim3(256), 0, stream, a, first, KIND == 1 ? a.dtv : nullptr, BLK * 64, grid);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
