@@ -556,10 +556,11 @@ template <int SIZE> __device__ __forceinline__ void order(uint64_t &x, int t)
 // 73 us with candidates inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
 //
 // A walk starts with the cube of 3 x 3 x 3 cells: the query's own cell alone never proves its K best.
-// Groups of sixteen for up to four neighbours, too, where there are few queries: a group then looks up the nine rows of cells
-// in one step.  K = 3, 12,170 and 37,140 sources: 50,000 queries 43 us with groups of four, 32 of sixteen; 150,000 52 and 46;
-// 600,000 94 and 131.
-constexpr int64_t kFewQueries = 200000;
+// Groups of sixteen for up to eight neighbours, too, where there are few queries: a group then looks up the nine rows of cells
+// in one step.  K = 3, groups of four / of sixteen, us a call (with its interpolation for the first): points within their
+// voxels among means of cells, 12,000 queries 41 / 28, 50,000 53 / 40, 100,000 53 / 46, 199,000 65 / 70; centres of voxels among
+// centres of cells, whose first cube always holds what they look for, 59,720 queries 31 / 33, 99,239 32 / 36, 199,185 41 / 55.
+constexpr int64_t kFewQueries = 65536;
 template <int G, int KMAX>
 __global__ __launch_bounds__(kThreads) void knn_query_kernel(
     int K, const float *__restrict__ qry, int64_t stride, int64_t Nq, const int32_t *__restrict__ query_offset,

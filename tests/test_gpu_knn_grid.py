@@ -32,7 +32,7 @@ def test_sizes_and_groups(oracle_lib, hip_lib, ns, K):
 
 
 @pytest.mark.parametrize("ns", [700, 5000])
-@pytest.mark.parametrize("nq", [200000, 200001])    # groups of sixteen, of four
+@pytest.mark.parametrize("nq", [65536, 65537, 200001])    # groups of sixteen, of four
 def test_many_queries(oracle_lib, hip_lib, ns, nq):
     rng = np.random.default_rng(nq)
     _check(oracle_lib, 3, _surface(rng, ns), _surface(rng, nq), [ns], [nq])
