@@ -190,10 +190,11 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  *   dtable_q/k/v   device FP32 [table_len], overwritten; layout of the tables
  *   pairs          M = sum of w_sizes^2, the pairs of the window set (counts[1] of s3d_window_index; the length
  *                  of the reference's index arrays), or 0.  With M the call runs two pair sweeps on the forward's
- *                  kind of work list (dq; dk and dv), which leave dL and P of every (pair, head) in the workspace
- *                  - 12 * H * pairs bytes -, and two table-gradient sweeps that read them; at head_dim 16 with tables
- *                  of at most 64 rows on a position axis and 32 on a signal axis it runs on tiles of 64 queries by 64
- *                  keys instead, all six gradients from matrix products.  With 0 it runs two fused
+ *                  kind of work list (dq, which leaves dL and P of every (pair, head) in the workspace, of which
+ *                  12 * H * pairs bytes are theirs; dk and dv, which reads them), and two table-gradient sweeps that
+ *                  read them too; at head_dim 16 with tables of at most 64 rows on a position axis and 32 on a signal
+ *                  axis tiles of 64 queries by 64 keys leave dL and P, and strips of 16 voxels with all their pairs give
+ *                  all six gradients by matrix products.  With 0 it runs two fused
  *                  sweeps that recompute the logits for the table gradients and need no such store (about a third
  *                  more time).  A value below M cannot hold the records of every window: the rows of dq, dk, dv
  *                  that belong to the windows beyond it and all three table gradients then come out as NaN.
@@ -216,7 +217,7 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  * wavefront draws varies from call to call, so these sums are regrouped and agree between calls to fp32 rounding
  * (about 1e-6 of the largest element), not bit for bit.
  *
- * On tiles, what is not finite in q, k, v, dout or a table makes NaN of the gradients that it belongs to as a sum over
+ * On tiles and strips, what is not finite in q, k, v, dout or a table makes NaN of the gradients that it belongs to as a sum over
  * pairs - those of its window, and of the table rows of its pairs - and of no others, but for the other channels of a
  * voxel or table row with such a dout; so does a statistic that is not the forward's, where it makes a weight above 8.
  */

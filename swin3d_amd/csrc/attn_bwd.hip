@@ -7,10 +7,10 @@
 //   dq_i  += dL (k_j + Tq(i,j))                    dTq[n][row_n(i,j)] += dL q_i
 //   dk_j  += dL (q_i + Tk(i,j))                    dTk[n][row_n(i,j)] += dL k_j
 // The reference adds every term with a global atomic.  Here every output element has ONE owner, and the call has three
-// forms.  With the window set's pair count it runs at head_dim 16 on tiles (attn_tile_bwd.hip: tables of up to 64 rows on
-// a position axis and 32 on a signal axis), otherwise the pair sweeps of attn_sweep.hip (dq; dk and dv; on the
-// forward's packed work list), which leave dL and P of every (pair, head) in the workspace, and the table-gradient
-// kernels below (attn_bwd_tables_kernel), which read them.  Without it, the fused sweeps (attn_bwd_sweep_kernel),
+// forms.  With the window set's pair count it runs at head_dim 16 on tiles and strips (attn_tile_bwd.hip, attn_strip_bwd.hip:
+// tables of up to 64 rows on a position axis and 32 on a signal axis), otherwise the pair sweeps of attn_sweep.hip on the
+// forward's packed work list (dq, which leaves dL and P of every (pair, head) in the workspace; dk and dv) and the
+// table-gradient kernels below (attn_bwd_tables_kernel), which read dL and P.  Without it, the fused sweeps (attn_bwd_sweep_kernel),
 // which recompute the logits and need no store:
 //
 //  * a key-owned sweep gives a lane one key j and streams the window's queries through the wavefront:
