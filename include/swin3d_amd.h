@@ -360,13 +360,19 @@ int s3d_cell_representatives(const int32_t *n2n, const int32_t *w2n, const int32
 int s3d_key_neighbours(const int64_t *sorted_keys, const int64_t *order, int64_t N, const int64_t *deltas, int32_t M,
                        int64_t *out, void *stream);
 /*
- * The 27 neighbours (x first, then y, z; the voxel itself among them) of every voxel on a lattice of `stride`, from keys
- * as s3d_pack_keys makes them (ascending: sorted_keys, order as for s3d_key_neighbours): out [N][27], N where there is none.
+ * The 27 neighbours (x first, then y, z; the voxel itself among them) of every voxel on a lattice of `stride`: out int64 [N][27],
+ * the first row with these coordinates, N where there is none.  coords device int32 [N,4] (batch, x, y, z), 16-byte
+ * aligned, x, y, z of less than 2^(field - 1) either side.  N below 2^30.
  */
-int s3d_lattice_neighbours(const int64_t *sorted_keys, const int64_t *order, int64_t N, int32_t field, int32_t stride,
-                           int64_t *out, void *stream);
-/* key of every voxel (batch, x, y, z): ascending in this order for coordinates of less than 2^(field - 1) either side */
-int s3d_pack_keys(const int32_t *coords, int64_t N, int32_t field, int64_t *out, void *stream);
+size_t s3d_voxel_neighbours_workspace_bytes(int64_t N);
+int s3d_voxel_neighbours(const int32_t *coords, int64_t N, int32_t field, int32_t stride, int64_t *out, void *workspace,
+                         size_t workspace_bytes, void *stream);
+/*
+ * out [M][width]: rows[m] (device int64) of from [n][width], words of 2 (fp16) or 4 (fp32) bytes; row n is a row of zeros,
+ * below zero counts back from behind it, any other index gives a row of NaN.
+ */
+int s3d_gather_rows(const void *from, int64_t n, const int64_t *rows, int64_t M, int32_t width, int32_t word_bytes, void *out,
+                    void *stream);
 /* out int32 [B]: how many of the N ascending batch ids (`stride` apart) are at most b */
 int s3d_segment_ends(const int32_t *batch, int64_t stride, int64_t N, int32_t B, int32_t *out, void *stream);
 /*

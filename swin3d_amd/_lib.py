@@ -76,8 +76,9 @@ SIGNATURES = {
                              [_i64, _i32, _i32, _i64, _i64, _i64, _i64, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_window_index_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_window_index": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [ctypes.c_size_t, _vp]),
-    "s3d_lattice_neighbours": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _vp, _vp]),
-    "s3d_pack_keys": (ctypes.c_int, [_vp, _i64, _i32, _vp, _vp]),
+    "s3d_gather_rows": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _i32, _vp, _vp]),
+    "s3d_voxel_neighbours_workspace_bytes": (ctypes.c_size_t, [_i64]),
+    "s3d_voxel_neighbours": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "s3d_segment_ends": (ctypes.c_int, [_vp, _i64, _i64, _i32, _vp, _vp]),
     "s3d_pool_cells": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _i32, _vp, _i64, _i32, _vp, _vp, _vp, _vp]),
     "s3d_level_signals": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp, _i64, _i32, _i32, ctypes.c_float, ctypes.c_float, _vp, _i64, _vp]),

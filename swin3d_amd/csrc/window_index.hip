@@ -652,16 +652,14 @@ __global__ __launch_bounds__(kThreads) void window_signals_wide_kernel(
 // one thread per (sorted voxel, offset): binary search of key + delta in the sorted keys
 __global__ __launch_bounds__(kThreads) void key_neighbours_kernel(const int64_t *__restrict__ sorted_keys,
                                                                   const int64_t *__restrict__ order, int64_t N,
-                                                                  const int64_t *__restrict__ deltas, int M, int field,
-                                                                  int64_t stride, int64_t *__restrict__ out)
+                                                                  const int64_t *__restrict__ deltas, int M,
+                                                                  int64_t *__restrict__ out)
 {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (t >= N * M) return;
     const int64_t i = t / M;
     const int d = static_cast<int>(t - i * M);
-    // (without a list: the 27 neighbours on a lattice, x first)
-    const int64_t delta = deltas ? deltas[d] : (((static_cast<int64_t>(d / 9 - 1) << field) + (d / 3 % 3 - 1) << field) + (d % 3 - 1)) * stride;
-    const int64_t key = sorted_keys[i] + delta;
+    const int64_t key = sorted_keys[i] + deltas[d];
     int64_t lo = 0, hi = N;   // first position whose key is not below `key`
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
@@ -749,22 +747,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_key_neighbours(const i
         return fail(S3D_ERR_NULL_POINTER, "s3d_key_neighbours: null device pointer");
     const dim3 grid(static_cast<unsigned>(ceil_div(N * M, kThreads)));
     hipLaunchKernelGGL(key_neighbours_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), sorted_keys,
-                       order, N, deltas, M, 0, int64_t(0), out);
-    S3D_HIP_CHECK(hipGetLastError());
-    return S3D_OK;
-}
-
-extern "C" __attribute__((visibility("default"))) int s3d_lattice_neighbours(const int64_t *sorted_keys, const int64_t *order, int64_t N,
-                                                                             int32_t field, int32_t stride, int64_t *out, void *stream)
-{
-    using namespace s3d;
-    if (N < 0 || N * 27 > 0x3fffffffffLL || field < 2 || field > 20 || stride < 1)
-        return fail(S3D_ERR_BAD_SHAPE, "s3d_lattice_neighbours: N=%lld field=%d (2..20 bits) stride=%d", (long long)N, field, stride);
-    if (N == 0) return S3D_OK;
-    if (!sorted_keys || !order || !out) return fail(S3D_ERR_NULL_POINTER, "s3d_lattice_neighbours: null device pointer");
-    hipLaunchKernelGGL(key_neighbours_kernel, dim3(static_cast<unsigned>(ceil_div(N * 27, kThreads))), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), sorted_keys, order, N, static_cast<const int64_t *>(nullptr), 27, field,
-                       static_cast<int64_t>(stride), out);
+                       order, N, deltas, M, out);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

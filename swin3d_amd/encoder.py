@@ -91,19 +91,20 @@ def lookup_rows(sorted_keys, order, query_keys):
 def conv3x3x3_neighbours(coords, stride):
     """[N, 27] long: the row of every voxel's 27 lattice neighbours (offsets ordered x-major), N where the
     neighbour is missing.  Depends on the coordinates only.  A packed key is linear in the coordinates, so a
-    neighbour's key is the voxel's key plus a constant per offset; taken in sorted key order the 27 query lists are
-    sorted themselves, which keeps the binary searches local."""
+    neighbour's key is the voxel's key plus a constant per offset: looked up in a table of the voxels where the kernels take
+    the coordinates by address, else among the sorted keys (taken in their order the 27 query lists are sorted themselves,
+    which keeps the binary searches local)."""
     n = coords.shape[0]
     if _plain_coords(coords) and n > 0:
         dev = coords.device
-        keys = torch.empty(n, dtype=torch.long, device=dev)
         out = torch.empty((n, 27), dtype=torch.long, device=dev)
         with _lib.on(dev):
-            lib, stream = _lib.lib(), _lib.stream(dev)
-            _lib.check(lib.s3d_pack_keys(coords.data_ptr(), n, _FIELD, keys.data_ptr(), stream), "s3d_pack_keys")
-            sorted_keys, order = torch.sort(keys)
-            status = lib.s3d_lattice_neighbours(sorted_keys.data_ptr(), order.data_ptr(), n, _FIELD, int(stride), out.data_ptr(), stream)
-        _lib.check(status, "s3d_lattice_neighbours")
+            lib = _lib.lib()
+            ws_bytes = lib.s3d_voxel_neighbours_workspace_bytes(n)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            status = lib.s3d_voxel_neighbours(coords.data_ptr(), n, _FIELD, int(stride), out.data_ptr(), workspace.data_ptr(), ws_bytes,
+                                              _lib.stream(dev))
+        _lib.check(status, "s3d_voxel_neighbours")
         return out
     sorted_keys, order = torch.sort(pack_coords(coords))
     deltas = torch.tensor([((dx << _FIELD) + dy << _FIELD) + dz for dx in (-1, 0, 1) for dy in (-1, 0, 1)
@@ -123,6 +124,24 @@ def conv3x3x3_neighbours(coords, stride):
     return out
 
 
+def _gather_rows(feats, neighbours):
+    """The stem's 27 rows a voxel side by side, [N, 27 Cin], or None where the kernel does not apply (a row that is no
+    row of `feats` or of the zeros behind them: NaN)."""
+    if not (feats.is_cuda and data_only(feats) and data_only(neighbours) and not (torch.is_grad_enabled() and feats.requires_grad)
+            and feats.dtype in (torch.float16, torch.float32) and feats.dim() == 2 and feats.is_contiguous()
+            and 0 < feats.shape[1] <= 1024 and 0 < feats.numel() < 2 ** 31
+            and neighbours.device == feats.device and neighbours.dtype == torch.long
+            and neighbours.shape == (feats.shape[0], 27) and neighbours.is_contiguous()):
+        return None
+    n, cin = feats.shape
+    out = torch.empty((n, 27 * cin), dtype=feats.dtype, device=feats.device)
+    with _lib.on(feats.device):
+        status = _lib.lib().s3d_gather_rows(feats.data_ptr(), n, neighbours.data_ptr(), n * 27, cin, feats.element_size(), out.data_ptr(),
+                                            _lib.stream(feats.device))
+    _lib.check(status, "s3d_gather_rows")
+    return out
+
+
 def sparse_conv3x3x3(voxels, weight, neighbours=None):
     """Submanifold-style 3x3x3 convolution (outputs on the input voxels; missing neighbours are
     zeros).  weight [27, Cin, Cout], offsets ordered x-major.  One gather + one GEMM."""
@@ -133,8 +152,10 @@ def sparse_conv3x3x3(voxels, weight, neighbours=None):
     if (feats.is_cuda and feats.dtype == torch.float32 and not feats.requires_grad and torch.is_autocast_enabled()
             and torch.get_autocast_dtype("cuda") == torch.float16):
         feats = feats.to(torch.float16)      # as the product takes it: the 27 copies are half as large
-    padded = torch.cat([feats, feats.new_zeros(1, cin)], 0)   # row n = zeros for missing neighbours
-    gathered = padded[neighbours.reshape(-1)].view(n, 27 * cin)
+    gathered = _gather_rows(feats, neighbours)
+    if gathered is None:
+        padded = torch.cat([feats, feats.new_zeros(1, cin)], 0)   # row n = zeros for missing neighbours
+        gathered = padded[neighbours.reshape(-1)].view(n, 27 * cin)
     weight = weight.reshape(27 * cin, -1)
     if torch.is_grad_enabled() and feats.is_cuda and torch.is_autocast_enabled():
         out = trained_linear(gathered, weight.t(), None, any_width=True)

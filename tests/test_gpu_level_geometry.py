@@ -63,3 +63,42 @@ def test_segments_keys_and_rows_apart(hip_lib, n):
     if n > 1:
         with pytest.raises(RuntimeError, match="contiguous"):
             knn_query(3, signals[:, 1:4], signals[:, 1:4], ends, ends)
+
+
+@pytest.mark.parametrize("n,stride", [(1, 1), (7, 1), (8, 2), (9, 3), (4096, 1), (4097, 2), (30011, 1)])
+def test_stem_neighbours_in_any_order_and_twice(hip_lib, n, stride):
+    """Rows in any order, around the sizes where the table doubles, dense and sparse, some coordinates twice: the first
+    row is the one that counts."""
+    from swin3d_amd import encoder
+    side = max(2, round((2 * n) ** (1 / 3)))
+    generator = torch.Generator().manual_seed(n)
+    coords = torch.randint(-side // 2, side // 2 + 1, (n, 4), generator=generator, dtype=torch.int32) * stride
+    coords[:, 0] = torch.randint(0, 3, (n,), generator=generator, dtype=torch.int32)
+    first = {}
+    for row, voxel in enumerate(coords.tolist()):
+        first.setdefault(tuple(voxel), row)
+    offsets = [(x, y, z) for x in (-1, 0, 1) for y in (-1, 0, 1) for z in (-1, 0, 1)]
+    want = torch.tensor([[first.get((b, x + dx * stride, y + dy * stride, z + dz * stride), n) for dx, dy, dz in offsets]
+                         for b, x, y, z in coords.tolist()])
+    assert torch.equal(encoder.conv3x3x3_neighbours(coords.to("cuda"), stride).cpu(), want)
+
+
+@pytest.mark.parametrize("n,width,dtype", [(1, 1, torch.float16), (19, 3, torch.float32), (1896, 9, torch.float16), (1897, 9, torch.float32),
+                                           (500, 6, torch.float16), (60, 257, torch.float16), (7, 1024, torch.float32)])
+def test_stem_rows_side_by_side(hip_lib, n, width, dtype):
+    """The stem's gather: part of a workgroup's rows, whole ones, rows wider than a workgroup; the row of zeros from either end."""
+    from swin3d_amd import encoder
+    generator = torch.Generator().manual_seed(n)
+    feats = torch.randn(n, width, generator=generator).to(dtype)
+    feats[0, 0] = float("inf")
+    rows = torch.randint(-n - 1, n + 1, (n, 27), generator=generator)
+    want = torch.cat([feats, feats.new_zeros(1, width)])[rows.reshape(-1)].view(n, 27 * width)
+    assert torch.equal(encoder._gather_rows(feats.cuda(), rows.cuda()).cpu(), want)
+    feats = feats.cuda()
+    assert encoder._gather_rows(feats.t().contiguous().t(), rows.cuda()) is None or width == 1 or n == 1
+    assert encoder._gather_rows(feats, rows.int().cuda()) is None
+    assert encoder._gather_rows(feats.requires_grad_(), rows.cuda()) is None
+    outside = rows.cuda()
+    outside[0, 0], outside[0, 1] = n + 1, -n - 2       # no such rows
+    got = encoder._gather_rows(feats.detach(), outside).view(n * 27, width)
+    assert got[:2].isnan().all() and torch.equal(got[2:].cpu(), want.view(n * 27, width)[2:])
