@@ -173,10 +173,10 @@ __global__ __launch_bounds__(kThreads) void segment_size_kernel(const int32_t *_
 // come from one bounding box of the coordinates (a window coordinate does not decrease with its voxel's).
 //
 // The windows, their pairs and the largest are known when the cells have been added up, and the host, which sizes what
-// follows by them, waits for that and not for the placing behind it.  (The sums run over the cells that the lattice has, a
-// fifth to a half of those it may have, in two launches; a library's scan over all of them took two as well, 14 us against 6
-// at 199,327 voxels.)
+// follows by them, waits for that and not for the placing behind it.  (The sums run over the cells that the lattice has, not
+// over those it may have, in two launches; a library's scan over 2 N took two as well, 14 us against 6 at 199,327 voxels.)
 constexpr int kGridBoxes = 128;          // workgroups of the bounding-box pass
+constexpr int kGridZeros = 384;          // ... and those beside them that only clear cells (without them two sets 1 to 2 us longer)
 constexpr int kSlotBits = 20;            // a voxel's slot in its cell, below its local id in one word
 constexpr int kBadRange = 1, kNoGrid = 2;   // counts[3]: coordinates out of range / lattice too large for the grid path
 
@@ -205,19 +205,25 @@ struct GridLayout {
 
 int64_t grid_cells_cap(int64_t N)
 {
-    int64_t cap = 2 * N;    // (no more cells than pay)
+    // (Voxels lie on surfaces, so the windows' lattice grows faster than they do: for cells of two voxels a side 1.1 a voxel in a
+    // room of 25,000, 2.0 at 100,000, 4.3 at 450,000.  A set that does not fit is built again by the sort of all voxels after one
+    // more wait of the host: three sets, the third of such cells, at 2 N 178 us for 100,000 voxels, 197 for 199,327 and 335 for
+    // 595,677; at 6 N 69, 77 and 123.  Two sets of windows of five take what they took, 62 us at 199,327: the cells are cleared beside the
+    // box, and those behind the lattice's own are not read.)
+    int64_t cap = 6 * N;
     if (cap < 4096) cap = 4096;
     if (cap > (1LL << 24)) cap = 1LL << 24;
     return cap;
 }
 
-// cells of a workgroup of the two launches that add them up, and what is left of them there
+// cells of a run, which a workgroup of the two launches that add them up takes at a time, and what is left of them there
 constexpr int kSumThreads = 1024, kSumCells = 4 * kSumThreads;
 struct CellSum {
     uint64_t before;       // (non-empty << 32 | voxels)
     int64_t squares;
     int32_t largest, unused;
 };
+__host__ __device__ __forceinline__ int64_t sum_groups(int64_t cells_cap) { return (cells_cap + kSumCells - 1) / kSumCells; }
 __host__ __device__ __forceinline__ uint64_t cell_word(int32_t count) { return (count > 0 ? (1ULL << 32) : 0ULL) | static_cast<uint32_t>(count); }
 
 // plans, cells, scan, place and keys: one of each per set, one behind the other
@@ -235,7 +241,7 @@ GridLayout make_grid_layout(int64_t N, int sets)
     L.plan = take(sizeof(GridPlan) * sets);
     L.partials = take(sizeof(int32_t) * 8 * kGridBoxes);
     L.cells = take(cells * sizeof(int32_t));
-    L.sums = take(sizeof(CellSum) * sets * static_cast<size_t>(ceil_div(L.cells_cap, kSumCells)));
+    L.sums = take(sizeof(CellSum) * sets * static_cast<size_t>(sum_groups(L.cells_cap)));
     L.scan = take(cells * sizeof(uint64_t));
     L.place = take(n * sizeof(int2));
     L.keys = take(n * sizeof(uint64_t));
@@ -270,14 +276,16 @@ __global__ __launch_bounds__(kThreads) void grid_bbox_kernel(const int32_t *__re
 {
     if (blockIdx.x == 0 && threadIdx.x < 4)
         for (int s = 0; s < sets.num; ++s) sets.set[s].counts[threadIdx.x] = 0;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < num_cells;
+    // (four cells at once; the room for them ends on a multiple of that)
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < (num_cells + 3) / 4;
          i += static_cast<int64_t>(gridDim.x) * kThreads)
-        cells[i] = 0;
+        reinterpret_cast<int4 *>(cells)[i] = make_int4(0, 0, 0, 0);
+    if (blockIdx.x >= kGridBoxes) return;
     int lo[4], hi[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) { lo[a] = 0x7fffffff; hi[a] = static_cast<int>(0x80000000u); }
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < N;
-         i += static_cast<int64_t>(gridDim.x) * kThreads) {
+         i += static_cast<int64_t>(kGridBoxes) * kThreads) {
         const int4 c = reinterpret_cast<const int4 *>(coords)[i];
         const int x[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
@@ -410,34 +418,39 @@ __global__ __launch_bounds__(kSumThreads) void grid_sums_kernel(GridSets sets, c
 {
     const int set = blockIdx.y;
     if (!plan[set].ok || (sets.set[set].counts[3] & kNoGrid)) return;
-    const int64_t total = cells_of(plan[set]), first = static_cast<int64_t>(blockIdx.x) * kSumCells;
-    if (first >= total) return;
+    const int64_t total = cells_of(plan[set]);
     cells += set * (cells_cap + 1);
-    uint64_t sum = 0;
-    int64_t squares = 0;
-    int largest = 0;
-#pragma unroll
-    for (int e = 0; e < kSumCells / kSumThreads; ++e) {
-        const int64_t c = first + e * kSumThreads + threadIdx.x;
-        const int n = c < total ? cells[c] : 0;
-        sum += cell_word(n);
-        squares += static_cast<int64_t>(n) * n;
-        largest = max(largest, n);
-    }
-    sum = wave_scan(sum);
-    squares = static_cast<int64_t>(wave_scan(static_cast<uint64_t>(squares)));
-    for (int off = 32; off > 0; off >>= 1) largest = max(largest, __shfl_xor(largest, off));
+    sums += set * sum_groups(cells_cap);
     __shared__ CellSum part[kSumThreads / 64];
-    if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = CellSum{sum, squares, largest, 0};
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    CellSum all = part[0];
-    for (int w = 1; w < kSumThreads / 64; ++w) {
-        all.before += part[w].before;
-        all.squares += part[w].squares;
-        all.largest = max(all.largest, part[w].largest);
+    for (int64_t group = blockIdx.x; group * kSumCells < total; group += gridDim.x) {
+        const int64_t first = group * kSumCells;
+        uint64_t sum = 0;
+        int64_t squares = 0;
+        int largest = 0;
+#pragma unroll
+        for (int e = 0; e < kSumCells / kSumThreads; ++e) {
+            const int64_t c = first + e * kSumThreads + threadIdx.x;
+            const int n = c < total ? cells[c] : 0;
+            sum += cell_word(n);
+            squares += static_cast<int64_t>(n) * n;
+            largest = max(largest, n);
+        }
+        sum = wave_scan(sum);
+        squares = static_cast<int64_t>(wave_scan(static_cast<uint64_t>(squares)));
+        for (int off = 32; off > 0; off >>= 1) largest = max(largest, __shfl_xor(largest, off));
+        if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = CellSum{sum, squares, largest, 0};
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            CellSum all = part[0];
+            for (int w = 1; w < kSumThreads / 64; ++w) {
+                all.before += part[w].before;
+                all.squares += part[w].squares;
+                all.largest = max(all.largest, part[w].largest);
+            }
+            sums[group] = all;
+        }
+        __syncthreads();
     }
-    sums[set * gridDim.x + blockIdx.x] = all;
 }
 
 // Every cell's window number and first position: what the workgroups before this one add up to and a scan of its own cells.
@@ -451,8 +464,8 @@ __global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets,
     int64_t *counts = sets.set[set].counts;
     const int64_t status = counts[3];
     const bool good = plan[set].ok && !(status & kNoGrid);
-    const int64_t total = good ? cells_of(plan[set]) : 0, first = static_cast<int64_t>(blockIdx.x) * kSumCells;
-    sums += set * gridDim.x;
+    const int64_t total = good ? cells_of(plan[set]) : 0;
+    sums += set * sum_groups(cells_cap);
     __shared__ CellSum part[kSumThreads / 64];
     __shared__ uint64_t wave_sum[kSumThreads / 64];
     if (blockIdx.x == 0) {
@@ -481,35 +494,38 @@ __global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets,
         }
         __syncthreads();
     }
-    if (first >= total) return;
     cells += set * (cells_cap + 1);
     scan += set * (cells_cap + 1);
-    uint64_t before = 0;
-    for (int g = threadIdx.x; g < static_cast<int>(blockIdx.x); g += kSumThreads) before += sums[g].before;
-    before = wave_scan(before);
-    if (lane == 63) part[wave].before = before;
-    // four neighbouring cells a thread
-    int n[4];
-    uint64_t own = 0;
-    const int64_t mine = first + 4 * static_cast<int>(threadIdx.x);
+    for (int64_t group = blockIdx.x; group * kSumCells < total; group += gridDim.x) {
+        const int64_t first = group * kSumCells;
+        uint64_t before = 0;
+        for (int g = threadIdx.x; g < static_cast<int>(group); g += kSumThreads) before += sums[g].before;
+        before = wave_scan(before);
+        if (lane == 63) part[wave].before = before;
+        // four neighbouring cells a thread
+        int n[4];
+        uint64_t own = 0;
+        const int64_t mine = first + 4 * static_cast<int>(threadIdx.x);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        n[e] = mine + e < total ? cells[mine + e] : 0;
-        own += cell_word(n[e]);
+        for (int e = 0; e < 4; ++e) {
+            n[e] = mine + e < total ? cells[mine + e] : 0;
+            own += cell_word(n[e]);
+        }
+        const uint64_t upto = wave_scan(own);
+        if (lane == 63) wave_sum[wave] = upto;
+        __syncthreads();
+        uint64_t run = upto - own;
+#pragma unroll
+        for (int w = 0; w < kSumThreads / 64; ++w) run += part[w].before + (w < wave ? wave_sum[w] : 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (mine + e <= total) scan[mine + e] = run;
+            run += cell_word(n[e]);
+        }
+        // (the end of the last cell, where that is a workgroup's last)
+        if (threadIdx.x == kSumThreads - 1 && mine + 4 == total) scan[total] = run;
+        __syncthreads();
     }
-    const uint64_t upto = wave_scan(own);
-    if (lane == 63) wave_sum[wave] = upto;
-    __syncthreads();
-    uint64_t run = upto - own;
-#pragma unroll
-    for (int w = 0; w < kSumThreads / 64; ++w) run += part[w].before + (w < wave ? wave_sum[w] : 0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (mine + e <= total) scan[mine + e] = run;
-        run += cell_word(n[e]);
-    }
-    // (the end of the last cell, where that is a workgroup's last)
-    if (threadIdx.x == kSumThreads - 1 && mine + 4 == total) scan[total] = run;
 }
 
 // every voxel to its window's segment (slot order); the voxel in slot 0 also records the window
@@ -889,12 +905,13 @@ int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_w
     const int64_t num_cells = (L.cells_cap + 1) * num_sets;
     const unsigned per_set = static_cast<unsigned>(num_sets);
     const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)), per_set);
-    hipLaunchKernelGGL(grid_bbox_kernel, dim3(kGridBoxes), dim3(kThreads), 0, s, coords, N, sets, partials, cells, num_cells);
+    hipLaunchKernelGGL(grid_bbox_kernel, dim3(kGridBoxes + kGridZeros), dim3(kThreads), 0, s, coords, N, sets, partials, cells, num_cells);
     S3D_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(grid_count_kernel, grid, dim3(kThreads), 0, s, coords, N, stride, sets, partials, L.cells_cap, plan,
                        cells, place);
     S3D_HIP_CHECK(hipGetLastError());
-    const dim3 sum_grid(static_cast<unsigned>(ceil_div(L.cells_cap, kSumCells)), per_set);
+    // (a third of the runs there may be: most lattices are smaller, and a workgroup takes another run where one is not)
+    const dim3 sum_grid(static_cast<unsigned>(ceil_div(L.cells_cap, 3 * kSumCells)), per_set);
     hipLaunchKernelGGL(grid_sums_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums);
     hipLaunchKernelGGL(grid_starts_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums, scan, host_counts);
     S3D_HIP_CHECK(hipGetLastError());

@@ -176,6 +176,25 @@ def test_lattice_too_large_falls_back_to_the_sort(oracle_lib, hip_lib, index_pat
         assert all(bool((o == -7).all()) for o in outs)
 
 
+@pytest.mark.parametrize("n,depth,fits", [(1000, 30, True), (999, 30, False), (1000, 31, False), (1034, 31, True), (600, 20, True),
+                                          (4100, 120, True), (4100, 124, False), (8192, 245, True)])
+def test_lattices_up_to_the_limit(oracle_lib, hip_lib, n, depth, fits):
+    """Lattices of 10 x 20 x depth windows of one voxel, of exactly 6 N cells, one voxel too few for it and the like, up to three
+    runs of cells a workgroup: the counting sort takes what fits, and the index is the oracle's either way."""
+    rng = np.random.default_rng(n + depth)
+    cells = np.concatenate([[0, 200 * depth - 1], 1 + rng.permutation(200 * depth - 2)[:n - 2]])
+    coords = np.stack([np.zeros(n, np.int64), cells // (20 * depth), cells // depth % 20, cells % depth], 1).astype(np.int32)
+    _compare(oracle_lib, coords, 1, 1, 0)
+    c = torch.from_numpy(coords).cuda()
+    outs = [torch.full((n,), -7, dtype=torch.int32, device="cuda") for _ in range(4)]
+    counts = torch.zeros(4, dtype=torch.int64, device="cuda")
+    ws_bytes = hip_lib.s3d_window_index_grid_workspace_bytes(n)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+    assert hip_lib.s3d_window_index_grid(c.data_ptr(), n, 1, 1, 0, *(o.data_ptr() for o in outs), counts.data_ptr(), ws.data_ptr(),
+                                         ws_bytes, torch.cuda.current_stream().cuda_stream) == 0
+    assert counts.tolist()[3] == (0 if fits else 2) and (fits or all(bool((o == -7).all()) for o in outs))
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 5000])
 def test_several_sets_in_one_call(hip_lib, n):
     """Sets of their own window sizes built together, more than one run of launches takes, one of them (window 1) with a
