@@ -74,11 +74,18 @@ def _plain_coords(coords):
             and coords.is_contiguous() and coords.data_ptr() % 16 == 0)
 
 
-def _plain_signals(signals):
-    """... and signal rows."""
+def _plain_signals(signals, coords):
+    """... and signal rows, one for each of the voxels `coords` and on their device."""
     return (signals.is_cuda and data_only(signals) and signals.dtype == torch.float32 and signals.dim() == 2
+            and signals.device == coords.device and signals.shape[0] == coords.shape[0]
             and signals.shape[1] >= 4 and signals.stride(1) == 1 and signals.stride(0) >= signals.shape[1]
             and not signals.requires_grad)
+
+
+def _check_signals(coords, signals):
+    """A voxel's signals are the row of its own number, which kernels and index operations read without looking."""
+    if signals.device != coords.device or signals.shape[0] < coords.shape[0]:
+        raise ValueError(f"signals {tuple(signals.shape)} on {signals.device} for {coords.shape[0]} voxels on {coords.device}")
 
 
 def lookup_rows(sorted_keys, order, query_keys):
@@ -198,6 +205,7 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
     """(coarse coordinates, representative fine row of every coarse voxel).  On the GPU both come from one window
     sort at window = factor (a coarse cell is a window; `index`, when the caller has built it already) and one
     kernel over the cells; elsewhere from pool_coordinates and pick_cell_representatives."""
+    _check_signals(coords, signals)
     sig = signals.float()
     if coords.is_cuda and 1 <= factor <= 10 and 1 <= sig.shape[1] <= 16:
         if index is None:
@@ -226,7 +234,7 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
 def _pool_level(coords, step, signals, index):
     """(coarse coordinates, signals of the representatives) of the cells of `index`: what pool_and_pick and signals[pick]
     give, in one kernel; None where it does not take them."""
-    if not (_plain_coords(coords) and _plain_signals(signals) and signals.shape[1] <= 16):
+    if not (_plain_coords(coords) and _plain_signals(signals, coords) and signals.shape[1] <= 16):
         return None
     dev, num, cols = coords.device, index.num_windows, signals.shape[1]
     coarse = torch.empty((num, 4), dtype=torch.int32, device=dev)
@@ -243,7 +251,7 @@ def _pool_level(coords, step, signals, index):
 def _level_signals(index, coords, stride, signals, num_signals, quant):
     """The scaled signals of a window set from a level's voxels and signals, in one kernel (window_signals of
     _local_and_extra); None where it does not take them."""
-    if not (_plain_coords(coords) and _plain_signals(signals) and 0 <= num_signals <= min(29, signals.shape[1] - 4)):
+    if not (_plain_coords(coords) and _plain_signals(signals, coords) and 0 <= num_signals <= min(29, signals.shape[1] - 4)):
         return None
     n, dev = coords.shape[0], coords.device
     out = torch.empty((n, 3 + num_signals), dtype=torch.float32, device=dev)
@@ -643,6 +651,7 @@ class Stage(nn.Module):
         window sort's n2n applied to coordinates, signals and features alike).  The row map of the regular set is
         then the identity and is handed to the attention op as None: its kernels read and write the rows in place,
         without the indirection."""
+        _check_signals(coords, signals)
         local_and_extra = lru_cache(maxsize=1)(partial(_local_and_extra, coords, stride, signals))
         # both window sets (one, for a single block) are enqueued before the host waits for their window counts
         shifts = list((0, self.window_size // 2)[:max(1, min(2, len(self.blocks)))])
@@ -738,6 +747,7 @@ def geometry_steps(stem_coords, stride, signals, layers, window_ordered=False, n
     coords = stem_coords
     ordered = False      # the current level's rows are in the order of its regular windows
     if window_ordered:
+        _check_signals(coords, signals)
         order = window_order(coords, stride, layers[0].window_size) if len(layers) else None
         if order is not None:
             coords, signals = coords[order], signals[order]
@@ -878,7 +888,7 @@ class Upsample(nn.Module):
         num_batches: batch elements of both, where the caller knows it: the host then waits for nothing."""
         skip, coarse = self._norm_linear(self.linear1, voxels_up.feats), self._norm_linear(self.linear2, voxels.feats).float()
         ends, ends_up = segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches)
-        if _plain_signals(signals) and _plain_signals(signals_up):
+        if _plain_signals(signals, voxels.coords) and _plain_signals(signals_up, voxels_up.coords):
             idx, dist2 = knn_query(self.up_k, signals[:, 1:4], signals_up[:, 1:4], ends, ends_up, KNN.cell_size, strided=True)
             feats = skip + KNNInterpolate.apply(idx, dist2, coarse.contiguous())
         else:

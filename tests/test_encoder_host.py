@@ -206,3 +206,25 @@ def test_stage_arguments_make_the_unscaled_signals_when_asked():
     assert args[7] == args[-2] == "unscaled" and args[:8] == whole[:8] and tuple(args) == whole and args + (1,) == whole + (1,)
     *_, n_coords, scaled = args
     assert (n_coords, scaled, len(calls)) == ("unscaled", "scaled", 1) and copy.copy(args) == whole
+
+
+def test_signals_that_are_not_the_voxels_own_are_refused(monkeypatch):
+    """Kernels read the signal row of every voxel by address: fewer rows, more of them and rows on another device are not theirs."""
+    from types import SimpleNamespace
+    coords = torch.from_numpy(random_scene(np.random.default_rng(1), 40))
+    signals = torch.cat([coords.float(), torch.rand(40, 3)], 1)
+    stage = encoder.Stage(16, 1, 2, 5, 4, out_channels=16)
+    for wrong in (signals[:39], signals.to("meta")):
+        with pytest.raises(ValueError, match="for 40 voxels"):
+            stage.plan(coords, 1, wrong)
+        with pytest.raises(ValueError, match="for 40 voxels"):
+            encoder.pool_and_pick(coords, 1, 2, wrong)
+    monkeypatch.setattr(encoder, "data_only", lambda _: True)
+
+    def stand_in(rows, device):
+        return SimpleNamespace(is_cuda=True, device=device, dtype=torch.float32, shape=(rows, 7), dim=lambda: 2, stride=(7, 1).__getitem__,
+                               requires_grad=False)
+
+    voxels = SimpleNamespace(device="cuda:0", shape=(40, 4))
+    for rows, device, mine in ((40, "cuda:0", True), (39, "cuda:0", False), (41, "cuda:0", False), (40, "cuda:1", False)):
+        assert encoder._plain_signals(stand_in(rows, device), voxels) is mine

@@ -102,3 +102,19 @@ def test_stem_rows_side_by_side(hip_lib, n, width, dtype):
     outside[0, 0], outside[0, 1] = n + 1, -n - 2       # no such rows
     got = encoder._gather_rows(feats.detach(), outside).view(n * 27, width)
     assert got[:2].isnan().all() and torch.equal(got[2:].cpu(), want.view(n * 27, width)[2:])
+
+
+@pytest.mark.parametrize("rows", [-1, 1])
+def test_rows_that_are_not_the_voxels_own(hip_lib, rows):
+    """Fewer or more signal rows than voxels, and signals on the host: no kernel takes them, and a stage refuses them."""
+    from swin3d_amd import encoder
+    from swin3d_amd.window_index import build_window_indices
+    coords, signals = _level(8, 600, 1, 10)
+    wrong = signals[:rows] if rows < 0 else torch.cat([signals, signals[:rows]])
+    stage = encoder.Stage(48, 2, 6, 5, 4, cRSE="XYZ_RGB_NORM").cuda()
+    index = build_window_indices(coords, 1, 2, (0,))[0]
+    for s in (wrong, signals.cpu()):
+        assert encoder._pool_level(coords, 2, s, index) is None and encoder._level_signals(index, coords, 1, s, 6, 4) is None
+        with pytest.raises((ValueError, RuntimeError)):
+            stage.plan(coords, 1, s)
+    stage.plan(coords, 1, signals)
