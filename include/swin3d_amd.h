@@ -329,6 +329,11 @@ int s3d_window_indices(const int32_t *coords, int64_t N, int32_t stride, const s
  */
 int s3d_window_indices_counted(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets,
                                int32_t num_sets, int64_t *host_counts, void *workspace, size_t workspace_bytes, void *stream);
+/*
+ * The same, but the calling thread waits for all of the stream's work: the sets are finished when this returns.
+ */
+int s3d_window_indices_finished(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets,
+                                int32_t num_sets, int64_t *host_counts, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * Representative voxel of every cell of a window sort: the member whose signal row is nearest (Euclidean, fp32) to

@@ -96,6 +96,7 @@ SIGNATURES = {
     "s3d_window_indices_workspace_bytes": (ctypes.c_size_t, [_i64, _i32]),
     "s3d_window_indices": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_window_indices_counted": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
+    "s3d_window_indices_finished": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "s3d_cell_representatives": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp, _vp]),
     "s3d_key_neighbours": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i32, _vp, _vp]),
     "s3d_window_signals": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _i32, _i32, ctypes.c_float, ctypes.c_float, _vp,

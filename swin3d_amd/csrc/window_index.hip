@@ -172,8 +172,9 @@ __global__ __launch_bounds__(kThreads) void segment_size_kernel(const int32_t *_
 // launches, each with too little work for the card (199,327 voxels, two sets: 46 us of kernels instead of 73).  The lattices
 // come from one bounding box of the coordinates (a window coordinate does not decrease with its voxel's).
 //
-// The windows, their pairs and the largest are known when the cells have been added up, and the host, which sizes what
-// follows by them, waits for that and not for the placing behind it.  (The sums run over the cells that the lattice has, not
+// The windows, their pairs and the largest are known when the cells have been added up, and a host that sizes by them what
+// follows on the same stream waits for that and not for the placing behind it (two sets with their signals at 199,327 voxels: 81 us a
+// pass, 94 where it waits for all, which another stream that reads the sets needs).  (The sums run over the cells that the lattice has, not
 // over those it may have, in two launches; a library's scan over 2 N took two as well, 14 us against 6 at 199,327 voxels.)
 constexpr int kGridBoxes = 128;          // workgroups of the bounding-box pass
 constexpr int kGridZeros = 384;          // ... and those beside them that only clear cells (without them two sets 1 to 2 us longer)
@@ -861,9 +862,9 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_window_indices_work
 namespace s3d {
 namespace {
 
-// counted: recorded behind the launch that leaves the counts in host_counts (or null, as that)
+// counted, finished: recorded behind the launch that leaves the counts in host_counts (or null, as that), and behind the last
 int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *jobs, int32_t num_sets,
-                   int64_t *host_counts, hipEvent_t counted, void *workspace, size_t workspace_bytes, void *stream)
+                   int64_t *host_counts, hipEvent_t counted, hipEvent_t finished, void *workspace, size_t workspace_bytes, void *stream)
 {
     if (N < 0 || N > 0x7fffffffLL || num_sets < 1 || num_sets > kMaxSets || N * num_sets > 0xffffffffLL)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_window_indices: N=%lld voxels, %d sets (1..%d)", (long long)N, num_sets, kMaxSets);
@@ -885,7 +886,8 @@ int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_w
         for (int i = 0; i < num_sets; ++i) hipLaunchKernelGGL(init_counts_kernel, dim3(1), dim3(64), 0, s, sets.set[i].counts);
         S3D_HIP_CHECK(hipGetLastError());
         for (int i = 0; host_counts && i < 4 * num_sets; ++i) host_counts[i] = 0;
-        if (counted) S3D_HIP_CHECK(hipEventRecord(counted, s));
+        for (hipEvent_t e : {counted, finished})
+            if (e) S3D_HIP_CHECK(hipEventRecord(e, s));
         return S3D_OK;
     }
     if (!coords || !workspace) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices: null device pointer");
@@ -924,6 +926,7 @@ int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_w
     hipLaunchKernelGGL(grid_order_kernel, dim3(static_cast<unsigned>(order_blocks), per_set), dim3(kThreads), 0, s, plan, keys,
                        N, sets);
     S3D_HIP_CHECK(hipGetLastError());
+    if (finished) S3D_HIP_CHECK(hipEventRecord(finished, s));
     return S3D_OK;
 }
 
@@ -934,23 +937,45 @@ extern "C" __attribute__((visibility("default"))) int s3d_window_indices(
     const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets, void *workspace,
     size_t workspace_bytes, void *stream)
 {
-    return s3d::window_indices(coords, N, stride, sets, num_sets, nullptr, nullptr, workspace, workspace_bytes, stream);
+    return s3d::window_indices(coords, N, stride, sets, num_sets, nullptr, nullptr, nullptr, workspace, workspace_bytes, stream);
 }
+
+namespace s3d {
+namespace {
+
+// the sets, and the calling thread waits: for the counts, or for all that the call launched
+int waited_window_indices(const char *name, bool all, const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets,
+                          int32_t num_sets, int64_t *host_counts, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!host_counts) return fail(S3D_ERR_NULL_POINTER, "%s: host_counts is null", name);
+    hipEvent_t there = nullptr;
+    S3D_HIP_CHECK(hipEventCreateWithFlags(&there, hipEventDisableTiming));
+    int rc = window_indices(coords, N, stride, sets, num_sets, host_counts, all ? nullptr : there, all ? there : nullptr, workspace,
+                            workspace_bytes, stream);
+    // (after an error between the launches the event may not have been recorded: host_counts is the caller's again all the same)
+    const hipError_t waited = rc == S3D_OK ? hipEventSynchronize(there) : hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    if (rc == S3D_OK && waited != hipSuccess) rc = hip_fail(waited, "hipEventSynchronize");
+    (void)hipEventDestroy(there);
+    return rc;
+}
+
+}  // namespace
+}  // namespace s3d
 
 extern "C" __attribute__((visibility("default"))) int s3d_window_indices_counted(
     const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets, int64_t *host_counts,
     void *workspace, size_t workspace_bytes, void *stream)
 {
-    using namespace s3d;
-    if (!host_counts) return fail(S3D_ERR_NULL_POINTER, "s3d_window_indices_counted: host_counts is null");
-    hipEvent_t counted = nullptr;
-    S3D_HIP_CHECK(hipEventCreateWithFlags(&counted, hipEventDisableTiming));
-    int rc = window_indices(coords, N, stride, sets, num_sets, host_counts, counted, workspace, workspace_bytes, stream);
-    // (also after an error behind the launches: host_counts is the caller's again when this returns)
-    const hipError_t waited = hipEventSynchronize(counted);
-    if (rc == S3D_OK && waited != hipSuccess) rc = hip_fail(waited, "hipEventSynchronize");
-    (void)hipEventDestroy(counted);
-    return rc;
+    return s3d::waited_window_indices("s3d_window_indices_counted", false, coords, N, stride, sets, num_sets, host_counts, workspace,
+                                      workspace_bytes, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_window_indices_finished(
+    const int32_t *coords, int64_t N, int32_t stride, const s3d_window_index_set *sets, int32_t num_sets, int64_t *host_counts,
+    void *workspace, size_t workspace_bytes, void *stream)
+{
+    return s3d::waited_window_indices("s3d_window_indices_finished", true, coords, N, stride, sets, num_sets, host_counts, workspace,
+                                      workspace_bytes, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_window_index_grid_workspace_bytes(int64_t N)

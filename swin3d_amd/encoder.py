@@ -3,7 +3,7 @@
 The sparse voxel set is a pair of tensors (`SparseVoxels`).  Under fp16 autocast the dense layers of inference run on
 the library's kernels, those of a training pass forward through torch (hipBLASLt) and backward on the library's; the
 27-offset stem convolution is one GEMM of torch's.  Window attention runs through
-`SelfAttnAIOFunction`, the window index through `build_window_indices` / `window_signals`, neighbour
+`SelfAttnAIOFunction`, the window index through `window_sets` / `window_signals`, neighbour
 gathering through `KNN` / `knn_max_pool`.  On the GPU the coordinate work runs on the library's kernels too
 (coarse cells and their representatives from the window sort, the stem's neighbour rows by binary search in
 sorted packed keys, the fused add + LayerNorm); the same functions have a tensor statement for host tensors,
@@ -40,7 +40,7 @@ from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttn
 from .sparse_dl.knn import KNN, KNNInterpolate, KNNMaxPool, knn_max_pool, knn_query
 from .swin_blocks import data_only, linear_rows, plain, swin_blocks
 from .swin_train import trained_branches
-from .window_index import build_window_indices, get_index01, index_arguments, window_signals
+from .window_index import get_index01, index_arguments, window_signals, window_sets
 
 
 @dataclass
@@ -179,7 +179,7 @@ def pool_coordinates(coords, stride, factor):
         # on the GPU a coarse cell is a window of `factor` voxels per side: the window sort gives the cells in the
         # same ascending (batch, x, y, z) order, one host wait, a third of the time of unique + scatter
         try:
-            index = build_window_indices(coords, stride, factor, (0,))[0]
+            index = window_sets(coords, stride, factor, (0,))[0]
         except ValueError:          # coordinates outside the window sort's range
             index = None
         if index is not None:
@@ -210,7 +210,7 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
     if coords.is_cuda and 1 <= factor <= 10 and 1 <= sig.shape[1] <= 16:
         if index is None:
             try:
-                index = build_window_indices(coords, stride, factor, (0,))[0]
+                index = window_sets(coords, stride, factor, (0,))[0]
             except ValueError:          # coordinates outside the window sort's range
                 index = None
         if index is not None:
@@ -658,7 +658,7 @@ class Stage(nn.Module):
         pooled = self.downsample is not None and coords.is_cuda and 1 <= self.downsample.factor <= 10
         if pooled:
             shifts.append((self.downsample.factor, 0))      # the downsample's cells: the same host wait
-        indices = build_window_indices(coords, stride, self.window_size, shifts)
+        indices = window_sets(coords, stride, self.window_size, shifts)
         cell_index = indices.pop() if pooled else None
         if len(self.blocks) > 0:
             # the quantiser scaling of the signals is the same for every block of the stage: once per index set,

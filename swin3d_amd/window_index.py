@@ -45,8 +45,14 @@ class WindowIndex:
 def build_window_indices(coords, stride, window_size, shifts):
     """One WindowIndex per entry of `shifts` (voxels: 0, or window_size // 2 for the shifted window set; an entry
     may also be a pair (window size, shift) for a set with a window size of its own) for coords int32 [N,4]
-    (batch,x,y,z) on the GPU.  All index builds are enqueued before the host reads the window counts back, so
-    the call synchronises once however many sets it is given."""
+    (batch,x,y,z) on the GPU.  All index builds are enqueued before the host waits, and what it waits for is the current
+    stream: when the call returns the sets are finished, and other streams and threads may read them."""
+    return window_sets(coords, stride, window_size, shifts, finished=True)
+
+
+def window_sets(coords, stride, window_size, shifts, finished=False):
+    """As build_window_indices for what goes on on the current stream: the host waits for the window counts, while the rows
+    of the sets (n2n, w_w_id, w_sizes, w2n) may still be on their way there."""
     if not coords.is_cuda:
         raise RuntimeError("coords must be a CUDA (HIP) tensor")
     if coords.dim() != 2 or coords.shape[1] != 4:
@@ -76,8 +82,9 @@ def build_window_indices(coords, stride, window_size, shifts):
                                             _lib.stream(dev))
         else:
             # (the last ones: the counts of all are there when this returns)
-            status = lib.s3d_window_indices_counted(coords.data_ptr(), n, int(stride), jobs, len(some), host.data_ptr(),
-                                                    workspace.data_ptr(), ws_bytes, _lib.stream(dev))
+            build = lib.s3d_window_indices_finished if finished else lib.s3d_window_indices_counted
+            status = build(coords.data_ptr(), n, int(stride), jobs, len(some), host.data_ptr(), workspace.data_ptr(), ws_bytes,
+                           _lib.stream(dev))
         _lib.check(status, "s3d_window_indices")
         rows = out[:, :n].unbind(0)
         return [rows[4 * i:4 * i + 4] for i in range(len(some))]
@@ -123,7 +130,7 @@ def build_window_index(coords, stride, window_size, shift=0):
     """coords int32 [N,4] (batch,x,y,z) CUDA tensor -> WindowIndex.
 
     `shift` is in voxels (0, or window_size // 2 for the shifted window set).
-    Synchronises once to read the window count back.
+    Waits for the current stream, as build_window_indices does.
     """
     return build_window_indices(coords, stride, window_size, [shift])[0]
 
