@@ -72,6 +72,16 @@ def _parameters(parts, groups):
         tables.get(f"{kind}_{name}_table") for kind in _KINDS for name in _GROUPS[:groups]]
 
 
+_CHECKED = (2, 4, 6)       # of _parameters: the weights of proj, fc1 and fc2
+
+
+def _unchecked(norm_bias, params):
+    """The parameters that a program may change in place between forward and backward, as it may with the nodes of the
+    single layers: those leave a weight or a norm's input for the backward, but no bias, and of q, k, v's weight and of the
+    tables a product or a copy."""
+    return [norm_bias, *(p for i, p in enumerate(params) if i not in _CHECKED)]
+
+
 def trained_branches(block, kinds, x, normed, attn_args):
     """(sum, pending) of `block` (of the types `kinds`) for rows x and their first norm `normed`, which trained_add_norm
     made; None where the layers have to be called one by one."""
@@ -98,6 +108,9 @@ def trained_branches(block, kinds, x, normed, attn_args):
             or any(not (data_only(t) and t.device == dev and t.dtype in (torch.int32, torch.int64)) for t in (w_sizes, w2n)) \
             or not (n2n is None or data_only(n2n) and n2n.device == dev and n2n.dtype in (torch.int32, torch.int64)):
         return None
+    # (a replay gives a gradient to the tensors themselves, whatever became of them since the forward: they have to be leaves)
+    if any(t is not None and t.grad_fn is not None for t in _unchecked(norm2.bias, params)):
+        return None
     # (a pass that leaves nothing for the attention's backward runs other kernels)
     if not (normed.requires_grad or any(t.requires_grad for t in itertools.chain(params[:2], tables) if t is not None)):
         return None
@@ -110,14 +123,40 @@ def trained_branches(block, kinds, x, normed, attn_args):
     return _Branches.apply(call, x, normed, norm2.weight, norm2.bias, *params)
 
 
-def _by_parts(call, index, x, normed, norm_weight, norm_bias, params):
-    """The same through the nodes of the single layers, for gradients of gradients."""
-    qkv_weight, qkv_bias, proj_weight, proj_bias, fc1_weight, fc1_bias, fc2_weight, fc2_bias, *tables = params
+def _values(layout, params, half, same):
+    """What the forward made of each parameter that may have changed since, None for the others."""
+    copies = iter(zip(layout.copies, layout.to))
+    values = []
+    for i, p in enumerate(params):
+        copy, at = (None, 0) if p is None else next(copies)
+        kept = None if copy is None or i in _CHECKED else same.narrow(0, copy.same, p.numel()) if copy.same >= 0 else half.narrow(0, at, p.numel())
+        values.append(kept)
+    return values
+
+
+class _AsBefore(Function):
+    """`before`, a value of the forward, with the gradient of `now`, from which it was made or is made again."""
+
+    @staticmethod
+    def forward(ctx, now, before):
+        return before.to(now.dtype, copy=True).view(now.shape)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return grad, None
+
+
+def _by_parts(call, index, x, normed, norm_weight, norm_bias, params, before, normed2_before):
+    """The same through the nodes of the single layers, for gradients of gradients.  before: per parameter what the forward
+    made of it, where the parameter itself may have changed since (q, k and v's scaled); normed2_before: as the forward left it."""
     channels = call.heads * call.dim
     w_sizes, w2n, n2n, coords = index
     scale = torch.ones(3 * channels, device=x.device)
     scale[:channels] = call.scale
-    qkv = _Linear.apply(normed, qkv_weight * scale.unsqueeze(1), None if qkv_bias is None else qkv_bias * scale)
+    params = [params[0] * scale.unsqueeze(1), None if params[1] is None else params[1] * scale, *params[2:]]
+    qkv_weight, qkv_bias, proj_weight, proj_bias, fc1_weight, fc1_bias, fc2_weight, fc2_bias, *tables = (
+        p if b is None else _AsBefore.apply(p, b) for p, b in zip(params, before))
+    qkv = _Linear.apply(normed, qkv_weight, qkv_bias)
     groups = len(tables) // 3
     kinds = [torch.cat([t.reshape(-1) for t in tables[i:i + groups]]) for i in range(0, 3 * groups, groups)]
     out = SelfAttnAIOFunction.apply(
@@ -126,6 +165,7 @@ def _by_parts(call, index, x, normed, norm_weight, norm_bias, params):
     branch = _Linear.apply(out.reshape(-1, channels), proj_weight, proj_bias)
     norm = torch.nn.LayerNorm(channels, call.eps, elementwise_affine=False, device="meta")      # (shape and eps)
     summed, normed2 = _AddNorm.apply(x, branch, norm_weight, norm_bias, norm)
+    normed2 = _AsBefore.apply(normed2, normed2_before)
     return summed, _Linear.apply(F.gelu(_Linear.apply(normed2, fc1_weight, fc1_bias)), fc2_weight, fc2_bias)
 
 
@@ -169,18 +209,23 @@ class _Branches(Function):
         hidden_out = F.gelu(hidden_in)
         pending = F.linear(hidden_out, copies[6], copies[7])
         ctx.call, ctx.layout = call, layout
-        ctx.save_for_backward(x, normed, norm_weight, norm_bias, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same,
-                              w_sizes, w2n, n2n, coords, *params)
+        ctx.unchecked = _unchecked(norm_bias, params)     # (leaves: their shapes, and where a replay's gradients go)
+        ctx.save_for_backward(x, normed, norm_weight, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same,
+                              w_sizes, w2n, n2n, coords, *(params[i] for i in _CHECKED))
         return summed, pending
 
     @staticmethod
     def backward(ctx, dsum, dpending):
         call, layout, needs = ctx.call, ctx.layout, ctx.needs_input_grad
-        (x, normed, norm_weight, norm_bias, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same, w_sizes, w2n, n2n,
-         coords, *params) = ctx.saved_tensors
+        (x, normed, norm_weight, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same, w_sizes, w2n, n2n,
+         coords, *checked) = ctx.saved_tensors
+        norm_bias, *params = ctx.unchecked
+        for i, p in zip(_CHECKED, checked):
+            params.insert(i, p)
         if torch.is_grad_enabled() or dsum is None or dpending is None or not (data_only(dsum) and data_only(dpending)) \
                 or dsum.dtype != torch.float32 or dpending.dtype != torch.float16:
-            return _Branches._replayed(ctx, (dsum, dpending), (x, normed, norm_weight, norm_bias, *params), (w_sizes, w2n, n2n, coords))
+            return _Branches._replayed(ctx, (dsum, dpending), (x, normed, norm_weight, norm_bias, *params), (w_sizes, w2n, n2n, coords),
+                                       _values(layout, params, half, same), normed2)
         n, channels = x.shape
         heads, dim, dev, nd = call.heads, call.dim, x.device, len(call.sizes)
         dsum, dpending = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
@@ -224,7 +269,7 @@ class _Branches(Function):
         return (None, *(g if need else None for g, need in zip(given, needs[1:])))
 
     @staticmethod
-    def _replayed(ctx, grads, inputs, index):
+    def _replayed(ctx, grads, inputs, index, before, normed2_before):
         """A graph of the gradients is wanted, or something follows them, or one is absent: the pass again through the
         single layers, whose backward knows these cases."""
         needs = ctx.needs_input_grad[1:]
@@ -232,7 +277,7 @@ class _Branches(Function):
         with torch.enable_grad(), torch.autocast("cuda", dtype=torch.float16):
             if not graph:
                 inputs = [None if t is None else t.detach().requires_grad_(need) for t, need in zip(inputs, needs)]
-            outs = _by_parts(ctx.call, index, *inputs[:4], inputs[4:])
+            outs = _by_parts(ctx.call, index, *inputs[:4], inputs[4:], before, normed2_before)
         pairs = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]
         wanted = [t for t, need in zip(inputs, needs) if need]
         if not pairs:

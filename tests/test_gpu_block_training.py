@@ -149,3 +149,55 @@ def test_what_steps_aside(hip_lib):
     for p in stage.blocks[0].parameters():
         p.requires_grad_(False)
     assert nodes(stage, run, feats) == 0
+
+
+@pytest.mark.parametrize("heads,mode,axes", [(3, 1, "XYZ_RGB_NORM"), (6, 2, "XYZ_RGB")])
+def test_parameters_changed_between_forward_and_backward(hip_lib, monkeypatch, heads, mode, axes):
+    """What the nodes of the layers let a program change in place before the backward, which then goes by the forward's values:
+    every bias behind the first norm, the tables, and q, k, v's weight.  The other weights are refused."""
+    stage, feats, run = _stage(1100, 48, heads, 5, mode, axes, seed=6)
+    feats.requires_grad_()
+    named = dict(stage.named_parameters())
+    wanted = [feats, *named.values()]
+    grad = torch.randn(feats.shape, device=feats.device)
+    changed = [p for name, p in named.items() if "table" in name or "qkv" in name or name.endswith("bias") and "norm1" not in name]
+    kept = [p.detach().clone() for p in changed]
+
+    def gradients(change, **how):
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = run(feats)
+        if change:
+            with torch.no_grad():
+                for p in changed:
+                    p.mul_(-1.5).add_(0.25)
+        first = torch.autograd.grad(out, wanted, grad, **how)
+        second = torch.autograd.grad(first[0].square().sum(), wanted, allow_unused=True) if how else ()
+        with torch.no_grad():
+            for p, before in zip(changed, kept):
+                p.copy_(before)
+        return [*first, *second]
+
+    def close(got, want, share):
+        for g, w in zip(got, want):
+            assert (g is None) == (w is None) and (g is None or (g - w).norm() <= share * w.norm() + 1e-12)
+
+    plain = gradients(False)
+    close(gradients(True), plain, 1e-5)                                        # (the tables' sums are regrouped)
+    whole = gradients(True, create_graph=True)
+    close(whole[:len(plain)], plain, 2e-3)                                     # torch's products of fp16 numbers for the library's
+    with torch.autocast("cuda", dtype=torch.float16):
+        refused = run(feats)
+    with torch.no_grad():
+        stage.blocks[0].mlp.fc2.weight.mul_(1.0)
+    with pytest.raises(RuntimeError, match="inplace"):
+        torch.autograd.grad(refused, wanted, grad)
+    # parameters that something else made go through the layers' nodes, which follow them
+    module, name = stage.blocks[0].mlp.fc1, "bias"
+    made = named["blocks.0.mlp.fc1.bias"] * 1.0
+    monkeypatch.setitem(module._parameters, name, made)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert sum("Branches" in node for node in _nodes(run(feats))) == 1
+    monkeypatch.undo()
+    monkeypatch.setattr(encoder, "trained_branches", lambda *_: None)
+    # (the second gradients: the first ones' difference and a product of the same kind again)
+    close(whole, gradients(True, create_graph=True), 4e-3)
