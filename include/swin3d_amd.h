@@ -344,7 +344,7 @@ int s3d_window_indices_finished(const int32_t *coords, int64_t N, int32_t stride
  *   n2n, w2n, w_sizes  device int32: outputs of s3d_window_index (W = counts[0] cells)
  *   signals            device fp32 rows of `signals_stride` floats, original row order; the first `num_signals`
  *                      columns (1..16) enter the distance
- *   out                device int64 [W]: the chosen row of every cell
+ *   out                device int64 [W]: the chosen row of every cell (2^31 - 1 where NaN leaves no member nearest)
  */
 int s3d_cell_representatives(const int32_t *n2n, const int32_t *w2n, const int32_t *w_sizes, int64_t W,
                              const float *signals, int64_t signals_stride, int32_t num_signals, int64_t *out,
@@ -383,6 +383,8 @@ int s3d_segment_ends(const int32_t *batch, int64_t stride, int64_t N, int32_t B,
 /*
  * The next coarser level from a sort of the voxels into its cells: what s3d_cell_representatives gives (pick), the cells'
  * coordinates (int32 [W][4], rounded down to multiples of `step`) and the picked rows' signals (fp32 [W][num_signals]).
+ * Where NaN among its members' signals leaves a cell without a nearest one, pick is 2^31 - 1 (as there), the batch -1, which
+ * s3d_window_index and its kin report as out of range, and the signals NaN.
  */
 int s3d_pool_cells(const int32_t *n2n, const int32_t *w2n, const int32_t *w_sizes, int64_t W, const int32_t *coords,
                    int32_t step, const float *signals, int64_t signals_stride, int32_t num_signals, int64_t *pick,

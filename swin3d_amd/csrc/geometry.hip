@@ -188,9 +188,10 @@ __global__ __launch_bounds__(kThreads) void pool_cells_kernel(
         pick[w] = best_row;
         const int4 c = coords[n2n[begin]];
         auto down = [&](int x) { return (x >= 0 ? x / step : -((-x + step - 1) / step)) * step; };
-        out_coords[w] = make_int4(c.x, down(c.y), down(c.z), down(c.w));
+        // (no member is nearest where a signal is NaN: a batch that no window index takes says so at the level above, at the
+        // wait which that level has anyway)
+        out_coords[w] = make_int4(best_row == 0x7fffffff ? -1 : c.x, down(c.y), down(c.z), down(c.w));
     }
-    // (no member is nearest where a signal is NaN: the row is then the caller's to trip over, as without this kernel)
     if (t < S) out_signals[w * S + t] = best_row == 0x7fffffff ? __int_as_float(0x7fc00000) : signals[static_cast<int64_t>(best_row) * stride + t];
 }
 

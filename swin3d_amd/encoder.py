@@ -233,7 +233,8 @@ def pool_and_pick(coords, stride, factor, signals, index=None):
 
 def _pool_level(coords, step, signals, index):
     """(coarse coordinates, signals of the representatives) of the cells of `index`: what pool_and_pick and signals[pick]
-    give, in one kernel; None where it does not take them."""
+    give, in one kernel; None where it does not take them.  A cell that none of its points stands for, because of NaN among
+    their signals, has batch -1, which the next window index refuses."""
     if not (_plain_coords(coords) and _plain_signals(signals, coords) and signals.shape[1] <= 16):
         return None
     dev, num, cols = coords.device, index.num_windows, signals.shape[1]
@@ -447,7 +448,13 @@ class GridKNNDownsample(nn.Module):
                                segment_offsets(coarse[:, 0], num_batches), KNN.cell_size, strided=True)
             return coarse, coarse_signals, idx
         coarse, pick = pool_and_pick(coords, stride, self.factor, signals, cell_index)
-        coarse_signals = signals[pick]
+        if coords.is_cuda:
+            # (an index that is no row, of a cell without a representative, would be read all the same: as _pool_level leaves it)
+            nobody = pick >= signals.shape[0]
+            coarse[:, 0].masked_fill_(nobody, -1)
+            coarse_signals = signals[pick.masked_fill(nobody, 0)].masked_fill(nobody.unsqueeze(1), float("nan"))
+        else:
+            coarse_signals = signals[pick]
         src_xyz = signals[:, 1:4].contiguous().float()
         qry_xyz = coarse_signals[:, 1:4].contiguous().float()
         idx, _ = KNN.apply(self.k, src_xyz, qry_xyz, segment_offsets(coords[:, 0], num_batches),
@@ -658,7 +665,13 @@ class Stage(nn.Module):
         pooled = self.downsample is not None and coords.is_cuda and 1 <= self.downsample.factor <= 10
         if pooled:
             shifts.append((self.downsample.factor, 0))      # the downsample's cells: the same host wait
-        indices = window_sets(coords, stride, self.window_size, shifts)
+        try:
+            indices = window_sets(coords, stride, self.window_size, shifts)
+        except ValueError as error:
+            if coords.shape[0] > 0 and int(coords[:, 0].min()) < 0:
+                raise ValueError("voxels of a batch below 0: given so, or pooled from points with NaN among their signals, of which none "
+                                 "stands for the voxel") from error
+            raise
         cell_index = indices.pop() if pooled else None
         if len(self.blocks) > 0:
             # the quantiser scaling of the signals is the same for every block of the stage: once per index set,

@@ -118,3 +118,22 @@ def test_rows_that_are_not_the_voxels_own(hip_lib, rows):
         with pytest.raises((ValueError, RuntimeError)):
             stage.plan(coords, 1, s)
     stage.plan(coords, 1, signals)
+
+
+@pytest.mark.parametrize("how", ["kernel", "tensors"])
+def test_a_cell_that_no_point_stands_for(hip_lib, how):
+    """NaN among the signals of a cell's points: no member is the nearest to their mean.  The next level says so, on the
+    kernel and where tensor operations pool (signals that want a gradient)."""
+    from swin3d_amd import encoder
+    coords, signals = _level(9, 900, 1, 10)
+    stages = [encoder.Stage(48, 1, 6, 5, 4, cRSE="XYZ_RGB_NORM").cuda() for _ in range(2)]
+    signals[17, 5] = float("nan")
+    signals.requires_grad_(how == "tensors")
+    _, (coarse, coarse_signals, _) = stages[0].plan(coords, 1, signals, 2)
+    bad = coarse[:, 0] < 0
+    assert bad.sum() == 1 and coarse_signals[bad].isnan().all() and not coarse_signals[~bad].isnan().any()
+    with pytest.raises(ValueError, match="NaN among their signals"):
+        stages[1].plan(coarse, 2, coarse_signals, 2)
+    net = encoder.Swin3DEncoder([1, 1], [48, 96], [6, 6], [5, 5], 4, num_layers=2, in_channels=6, cRSE="XYZ_RGB_NORM", fp16_mode=2).cuda()
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16), pytest.raises(ValueError, match="NaN among their signals"):
+        net(encoder.SparseVoxels(coords, torch.zeros(900, 6, device="cuda"), 1), signals)
