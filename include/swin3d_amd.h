@@ -190,15 +190,15 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  *   dtable_q/k/v   device FP32 [table_len], overwritten; layout of the tables
  *   pairs          M = sum of w_sizes^2, the pairs of the window set (counts[1] of s3d_window_index; the length
  *                  of the reference's index arrays), or 0.  With M the call runs two pair sweeps on the forward's
- *                  kind of work list (dq, which leaves dL and P of every (pair, head) in the workspace, of which
- *                  12 * H * pairs bytes are theirs; dk and dv, which reads them), and two table-gradient sweeps that
- *                  read them too; at head_dim 16 with tables of at most 64 rows on a position axis and 32 on a signal
+ *                  kind of work list (dq, which leaves dL and P of every (pair, head) in the workspace, 8 * H * pairs
+ *                  bytes; dk and dv, which reads them), and two table-gradient sweeps that read them too; at head_dim 16 with tables of at most 64 rows on a position axis and 32 on a signal
  *                  axis tiles of 64 queries by 64 keys leave dL and P, and strips of 16 voxels with all their pairs give
  *                  all six gradients by matrix products.  With 0 it runs two fused
  *                  sweeps that recompute the logits for the table gradients and need no such store (about a third
  *                  more time).  A value below M cannot hold the records of every window: the rows of dq, dk, dv
  *                  that belong to the windows beyond it and all three table gradients then come out as NaN.
- *   workspace      device scratch of at least s3d_attn_bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs) bytes
+ *   workspace      device scratch of at least s3d_attn_bwd_workspace_least_bytes(H, D, nd, table_len, N, W, pairs) bytes;
+ *                  s3d_attn_bwd_workspace_bytes is never less, and has the 12 bytes a (pair, head) of an earlier store
  *   dtype          S3D_DTYPE_F32, S3D_DTYPE_F16, or S3D_DTYPE_F32_F16_ROWS: the tables fp32, every [N,H,D] tensor
  *                  fp16, the results those of dtype S3D_DTYPE_F32 on fp32 copies of the rows with dq, dk, dv
  *                  rounded to fp16 (the same arithmetic; the two launches may pack the windows differently, which
@@ -223,6 +223,8 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  */
 size_t s3d_attn_bwd_workspace_bytes(int32_t H, int32_t D, int32_t nd, int64_t table_len, int64_t N, int64_t W,
                                     int64_t pairs);
+size_t s3d_attn_bwd_workspace_least_bytes(int32_t H, int32_t D, int32_t nd, int64_t table_len, int64_t N, int64_t W,
+                                          int64_t pairs);
 int s3d_attn_bwd(const void *q, const void *k, const void *v, const void *table_q, const void *table_k,
                  const void *table_v, const int32_t *table_sizes, int32_t nd, int64_t table_len,
                  const int32_t *w_sizes, const int32_t *w2n, const int32_t *n2n, const float *n_coords,

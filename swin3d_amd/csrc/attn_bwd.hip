@@ -1276,8 +1276,10 @@ size_t bwd_tgrad_bytes(int H, int D, int nd)
 
 // the pair path's part of the workspace: window pair offsets, (dL, P) of every (pair, head), and the pair sweeps' work list
 size_t bwd_pos_base_bytes(int64_t N) { return align_up(sizeof(int64_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
-// (records take 8 bytes a (pair, head); the size asked for stays 12, which callers may have planned with)
-size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(12 * static_cast<size_t>(H) * pairs + sizeof(float2) * kPairSpare, 256); }
+size_t bwd_pd_bytes(int H, int64_t pairs) { return align_up(sizeof(float2) * (static_cast<size_t>(H) * pairs + kPairSpare), 256); }
+// (an earlier store held 12 bytes a (pair, head), and callers plan with the size that it gave; it is never less than the above)
+size_t bwd_planned_pd_bytes(int H, int64_t pairs) { return align_up(12 * static_cast<size_t>(H) * pairs, 256); }
+static_assert(sizeof(float2) * (7 + kPairSpare) <= 256 && 12 * 8 >= sizeof(float2) * (8 + kPairSpare), "up to seven records, and from eight on");
 // the last part of every form's workspace: the identity row map that stands in for a null n2n
 size_t bwd_row_map_bytes(int64_t N) { return align_up(sizeof(int32_t) * static_cast<size_t>(N > 0 ? N : 1), 256); }
 
@@ -1285,6 +1287,23 @@ __global__ void bwd_identity_rows_kernel(int32_t *map, int64_t n)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) map[i] = static_cast<int32_t>(i);
+}
+
+size_t bwd_workspace_bytes(int32_t H, int32_t D, int32_t nd, int64_t table_len, int64_t N, int64_t W, int64_t pairs, bool planned)
+{
+    if (H < 1 || D < 1 || nd < 1 || nd > kMaxAxes || table_len < 1 || N < 0 || W < 0 || pairs < 0) return 0;
+    if (bwd_general_form(H, D, nd, table_len))
+        return bwd_units_bytes(W, N, H, 0) + bwd_delta_bytes(N, H) + 2 * bwd_general_acc_bytes(N, H, D) +
+               bwd_row_map_bytes(N);
+    size_t need = bwd_units_bytes(W, N, H, pairs) + bwd_delta_bytes(N, H) + bwd_tgrad_bytes(H, D, nd) +
+                  bwd_pos_base_bytes(N) + bwd_row_map_bytes(N);
+    if (pairs > 0) {
+        need += (planned ? bwd_planned_pd_bytes(H, pairs) : bwd_pd_bytes(H, pairs)) + align_up(attn_sweep_workspace_bytes(H, W, N), 256);
+        // the tile form works in the whole of it (whether it applies depends on the rows of the single axes)
+        const size_t tiles = D == 16 ? attn_tile_bwd_bytes(H, nd, N, W, pairs) + bwd_row_map_bytes(N) : 0;
+        if (need < tiles) need = tiles;
+    }
+    return need;
 }
 
 }  // namespace
@@ -1295,20 +1314,13 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_attn_bwd_workspace_
                                                                                       int64_t N, int64_t W,
                                                                                       int64_t pairs)
 {
-    using namespace s3d;
-    if (H < 1 || D < 1 || nd < 1 || nd > kMaxAxes || table_len < 1 || N < 0 || W < 0 || pairs < 0) return 0;
-    if (bwd_general_form(H, D, nd, table_len))
-        return bwd_units_bytes(W, N, H, 0) + bwd_delta_bytes(N, H) + 2 * bwd_general_acc_bytes(N, H, D) +
-               bwd_row_map_bytes(N);
-    size_t need = bwd_units_bytes(W, N, H, pairs) + bwd_delta_bytes(N, H) + bwd_tgrad_bytes(H, D, nd) +
-                  bwd_pos_base_bytes(N) + bwd_row_map_bytes(N);
-    if (pairs > 0) {
-        need += bwd_pd_bytes(H, pairs) + align_up(attn_sweep_workspace_bytes(H, W, N), 256);
-        // the tile form works in the whole of it (whether it applies depends on the rows of the single axes)
-        const size_t tiles = D == 16 ? attn_tile_bwd_bytes(H, nd, N, W, pairs) + bwd_row_map_bytes(N) : 0;
-        if (need < tiles) need = tiles;
-    }
-    return need;
+    return s3d::bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs, true);
+}
+
+extern "C" __attribute__((visibility("default"))) size_t s3d_attn_bwd_workspace_least_bytes(int32_t H, int32_t D, int32_t nd, int64_t table_len,
+                                                                                            int64_t N, int64_t W, int64_t pairs)
+{
+    return s3d::bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs, false);
 }
 
 namespace s3d {
@@ -1359,7 +1371,7 @@ int attn_bwd(
     if (int rc = fill_bwd_axes(a, table_sizes, nd, table_len)) return rc;
     if (!dtable_q || !dtable_k || !dtable_v)
         return fail(S3D_ERR_NULL_POINTER, "s3d_attn_bwd: null table-gradient pointer");
-    const size_t need = s3d_attn_bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs);
+    const size_t need = bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs, false);
     if (!workspace || workspace_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_attn_bwd: workspace %zu B < required %zu B",
                     workspace ? workspace_bytes : size_t(0), need);

@@ -41,7 +41,7 @@ Places places_of(int64_t N, int32_t C, int32_t hidden, int32_t H, int32_t D, int
     p.parts = p.residual + align_up(row * C, 256);
     const Layers layers = layers_of(N, C, hidden);
     p.rest = p.parts + align_up(linear_grads_bytes(layers.of, kMostLinearGrads), 256);
-    const size_t attention = s3d_attn_bwd_workspace_bytes(H, D, nd, table_len, N, W, pairs), norm = s3d_layernorm_grad_workspace_bytes(N, C);
+    const size_t attention = s3d_attn_bwd_workspace_least_bytes(H, D, nd, table_len, N, W, pairs), norm = s3d_layernorm_grad_workspace_bytes(N, C);
     p.total = p.rest + (attention > norm ? attention : norm);
     return p;
 }

@@ -275,6 +275,11 @@ def _attention(q, k, v, strides, table_q, table_k, table_v, table_sizes, w_sizes
     return out
 
 
+def _pair_store_fits(pairs, heads):
+    """dL and P of every (pair, head), in fp32, are not above BWD_PAIR_STORE_MAX_BYTES."""
+    return 8 * pairs * heads <= BWD_PAIR_STORE_MAX_BYTES
+
+
 def _pairs_of(w_sizes_in, w_sizes):
     """M = sum of w_sizes^2, the pairs of the window set (one host read, kept on the caller's tensor)."""
     if isinstance(w_sizes_in, torch.Tensor):
@@ -298,8 +303,8 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
 
     pairs: M = sum(w_sizes^2) of the window set (the reference's index arrays have this length,
     swin3d_layers.py:96-103); None = read it from w_sizes once and keep it on that tensor.  With it the library
-    runs the pair sweeps, or at head_dim 16 the tile kernels, which keep dL and P of every (pair, head) in the workspace (8
-    bytes; the pair sweeps' workspace has 12); 0, or a
+    runs the pair sweeps, or at head_dim 16 the tile kernels, which keep dL and P of every (pair, head) in the workspace
+    (8 bytes); 0, or a
     store above BWD_PAIR_STORE_MAX_BYTES, selects the fused sweeps, which need no such store and take about a
     third longer.  head_dim 32 and tables of more than BWD_MAX_ROWS_PER_AXIS rows per axis on average run in the
     library's general form (atomic adds, as the reference works): correct, some fifty times slower per pair."""
@@ -357,7 +362,7 @@ def _attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w_sizes
     pairs = int(pairs)
     if pairs < 0:
         raise ValueError(f"pairs = {pairs}")
-    if 12 * pairs * h > BWD_PAIR_STORE_MAX_BYTES:
+    if not _pair_store_fits(pairs, h):
         pairs = 0
     code = _lib.S3D_DTYPE_F32_F16_ROWS if mixed else _DTYPE_CODE[q.dtype]
     if mixed and pairs == 0 and not general:
@@ -378,7 +383,7 @@ def _attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w_sizes
     tensors = [q, k, v] + [t.contiguous() for t in (table_q, table_k, table_v)]
     out, dout, out_max, out_sum, n_coords = (t.contiguous() for t in (out, dout, out_max, out_sum, n_coords))
     with _lib.on(dev):
-        ws_bytes = lib.s3d_attn_bwd_workspace_bytes(h, d, nd, table_len, n, w_sizes.numel(), pairs)
+        ws_bytes = lib.s3d_attn_bwd_workspace_least_bytes(h, d, nd, table_len, n, w_sizes.numel(), pairs)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         stream = _lib.stream(dev)
         status = lib.s3d_attn_bwd_strided(

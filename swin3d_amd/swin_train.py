@@ -115,7 +115,7 @@ def trained_branches(block, kinds, x, normed, attn_args):
     if not (normed.requires_grad or any(t.requires_grad for t in itertools.chain(params[:2], tables) if t is not None)):
         return None
     pairs = attn_coff._pairs_of(w_sizes, w_sizes) if attn_coff.BWD_PAIR_STORE else 0
-    if pairs == 0 or 12 * pairs * heads > attn_coff.BWD_PAIR_STORE_MAX_BYTES:
+    if pairs == 0 or not attn_coff._pair_store_fits(pairs, heads):
         return None
     call = _Call()
     call.heads, call.dim, call.hidden, call.sizes, call.table_len = heads, dim, fc1.out_features, sizes, table_len

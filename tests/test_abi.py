@@ -126,3 +126,25 @@ def test_window_signals_rejects_bad_arguments(hip_lib):
     assert hip_lib.s3d_window_signals(None, None, None, None, 2, 6, 5, f(1), f(1), None, 4, None) < 0      # stride < columns
     assert hip_lib.s3d_window_signals(None, None, None, None, 0, 0, 11, f(1), f(1), None, 4, None) < 0     # window > 10
     assert b"s3d_window_signals" in hip_lib.s3d_last_error_string()
+
+
+def test_backward_workspace_sizes(hip_lib):
+    """The size that callers plan with is the one of the store of 12 bytes a (pair, head), to the byte; the call itself takes 8
+    and some spare records."""
+    from swin3d_amd.crse import crse_table_sizes
+    up = lambda b: -(-b // 256) * 256
+    for heads, dim, n, w, pairs in ((6, 8, 1000, 40, 30000), (1, 8, 1, 1, 1), (1, 8, 3, 3, 3), (7, 8, 2, 2, 1), (8, 8, 1, 1, 1), (64, 8, 4, 1, 16),
+                                    (6, 8, 199_327, 7_554, 5_670_000), (3, 8, 700, 30, 21_845)):
+        length = sum(crse_table_sizes(5, 4, heads, dim, "XYZ_RGB_NORM"))
+        planned = hip_lib.s3d_attn_bwd_workspace_bytes(heads, dim, 9, length, n, w, pairs)
+        least = hip_lib.s3d_attn_bwd_workspace_least_bytes(heads, dim, 9, length, n, w, pairs)
+        assert planned - up(12 * heads * pairs) == least - up(8 * (heads * pairs + 4)) and least <= planned
+        # (without pairs: no store, no sweep list, and room for as many units less)
+        assert hip_lib.s3d_attn_bwd_workspace_least_bytes(heads, dim, 9, length, n, w, 0) == hip_lib.s3d_attn_bwd_workspace_bytes(heads, dim, 9, length, n, w, 0)
+    assert hip_lib.s3d_attn_bwd_workspace_least_bytes(0, 8, 9, 1, 1, 1, 1) == 0
+
+
+def test_pair_store_limit_counts_what_the_store_holds():
+    from swin3d_amd.sparse_dl.attn import attn_coff
+    most = attn_coff.BWD_PAIR_STORE_MAX_BYTES // 8
+    assert attn_coff._pair_store_fits(most // 6, 6) and attn_coff._pair_store_fits(most, 1) and not attn_coff._pair_store_fits(most // 6 + 1, 6)
