@@ -200,7 +200,7 @@ struct GridPlan {
 };
 
 struct GridLayout {
-    size_t plan, partials, cells, sums, scan, place, keys, total;
+    size_t plan, partials, cells, sums, place, keys, total;
     int64_t cells_cap;
 };
 
@@ -227,12 +227,12 @@ struct CellSum {
 __host__ __device__ __forceinline__ int64_t sum_groups(int64_t cells_cap) { return (cells_cap + kSumCells - 1) / kSumCells; }
 __host__ __device__ __forceinline__ uint64_t cell_word(int32_t count) { return (count > 0 ? (1ULL << 32) : 0ULL) | static_cast<uint32_t>(count); }
 
-// plans, cells, scan, place and keys: one of each per set, one behind the other
+// plans, cells, sums, place and keys: one of each per set, one behind the other
 GridLayout make_grid_layout(int64_t N, int sets)
 {
     GridLayout L{};
     L.cells_cap = grid_cells_cap(N);
-    const size_t n = static_cast<size_t>(N > 0 ? N : 1) * sets, cells = (static_cast<size_t>(L.cells_cap) + 1) * sets;
+    const size_t n = static_cast<size_t>(N > 0 ? N : 1) * sets, cells = static_cast<size_t>(L.cells_cap) * sets;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
@@ -243,7 +243,6 @@ GridLayout make_grid_layout(int64_t N, int sets)
     L.partials = take(sizeof(int32_t) * 8 * kGridBoxes);
     L.cells = take(cells * sizeof(int32_t));
     L.sums = take(sizeof(CellSum) * sets * static_cast<size_t>(sum_groups(L.cells_cap)));
-    L.scan = take(cells * sizeof(uint64_t));
     L.place = take(n * sizeof(int2));
     L.keys = take(n * sizeof(uint64_t));
     L.total = off;
@@ -326,7 +325,7 @@ __global__ __launch_bounds__(kThreads) void grid_count_kernel(
     __shared__ int box[8];
     const int set = blockIdx.y, window = sets.set[set].window, shift = sets.set[set].shift;
     int64_t *counts = sets.set[set].counts;
-    cells += set * (cells_cap + 1);
+    cells += set * cells_cap;
     place += set * N;
     {
         // eight numbers by 32 lanes each
@@ -420,7 +419,7 @@ __global__ __launch_bounds__(kSumThreads) void grid_sums_kernel(GridSets sets, c
     const int set = blockIdx.y;
     if (!plan[set].ok || (sets.set[set].counts[3] & kNoGrid)) return;
     const int64_t total = cells_of(plan[set]);
-    cells += set * (cells_cap + 1);
+    cells += set * cells_cap;
     sums += set * sum_groups(cells_cap);
     __shared__ CellSum part[kSumThreads / 64];
     for (int64_t group = blockIdx.x; group * kSumCells < total; group += gridDim.x) {
@@ -454,12 +453,13 @@ __global__ __launch_bounds__(kSumThreads) void grid_sums_kernel(GridSets sets, c
     }
 }
 
-// Every cell's window number and first position: what the workgroups before this one add up to and a scan of its own cells.
-// The first workgroup of a set leaves the totals and the status word, also where the host reads them (or null).
+// Every cell's first position, in the place of its count, and the windows: what the workgroups before this one add up to and
+// a scan of its own cells.  (With window number and position of every cell in an array of its own a set took 72 bytes a voxel
+// for its cells, not 24, and the placing read two of its words for a window's first voxel.)  The first workgroup of a set leaves
+// the totals and the status word, also where the host reads them (or null).
 __global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets, const GridPlan *__restrict__ plan,
-                                                                  const int32_t *__restrict__ cells, int64_t cells_cap,
-                                                                  const CellSum *__restrict__ sums, uint64_t *__restrict__ scan,
-                                                                  int64_t *host_counts)
+                                                                  int32_t *__restrict__ cells, int64_t cells_cap,
+                                                                  const CellSum *__restrict__ sums, int64_t *host_counts)
 {
     const int set = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int64_t *counts = sets.set[set].counts;
@@ -495,8 +495,8 @@ __global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets,
         }
         __syncthreads();
     }
-    cells += set * (cells_cap + 1);
-    scan += set * (cells_cap + 1);
+    int32_t *w2n = sets.set[set].w2n, *w_sizes = sets.set[set].w_sizes;
+    cells += set * cells_cap;
     for (int64_t group = blockIdx.x; group * kSumCells < total; group += gridDim.x) {
         const int64_t first = group * kSumCells;
         uint64_t before = 0;
@@ -520,38 +520,34 @@ __global__ __launch_bounds__(kSumThreads) void grid_starts_kernel(GridSets sets,
         for (int w = 0; w < kSumThreads / 64; ++w) run += part[w].before + (w < wave ? wave_sum[w] : 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if (mine + e <= total) scan[mine + e] = run;
+            const int start = static_cast<int>(run & 0xffffffffu), rank = static_cast<int>(run >> 32);
+            if (mine + e < total) cells[mine + e] = start;
+            if (n[e] > 0) {
+                w2n[rank] = start;
+                w_sizes[rank] = n[e];
+            }
             run += cell_word(n[e]);
         }
-        // (the end of the last cell, where that is a workgroup's last)
-        if (threadIdx.x == kSumThreads - 1 && mine + 4 == total) scan[total] = run;
         __syncthreads();
     }
 }
 
-// every voxel to its window's segment (slot order); the voxel in slot 0 also records the window
+// every voxel to its window's segment (slot order)
 __global__ __launch_bounds__(kThreads) void grid_place_kernel(const int2 *__restrict__ place, int64_t N, GridSets sets,
                                                               const GridPlan *__restrict__ plan,
-                                                              const uint64_t *__restrict__ scan, int64_t cells_cap,
+                                                              const int32_t *__restrict__ cells, int64_t cells_cap,
                                                               uint64_t *__restrict__ keys)
 {
     const int set = blockIdx.y;
-    int32_t *w2n = sets.set[set].w2n, *w_sizes = sets.set[set].w_sizes;
     if (!plan[set].ok || (sets.set[set].counts[3] & kNoGrid)) return;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= N) return;
-    scan += set * (cells_cap + 1);
+    cells += set * cells_cap;
     place += set * N;
     keys += set * N;
     const int2 p = place[i];
-    const uint64_t here = scan[p.x];
-    const int start = static_cast<int>(here & 0xffffffffu), slot = p.y & ((1 << kSlotBits) - 1);
-    keys[start + slot] = (static_cast<uint64_t>(p.y >> kSlotBits) << 32) | static_cast<uint32_t>(i);
-    if (slot == 0) {
-        const int rank = static_cast<int>(here >> 32);
-        w2n[rank] = start;
-        w_sizes[rank] = static_cast<int>(scan[p.x + 1] & 0xffffffffu) - start;
-    }
+    const int slot = p.y & ((1 << kSlotBits) - 1);
+    keys[cells[p.x] + slot] = (static_cast<uint64_t>(p.y >> kSlotBits) << 32) | static_cast<uint32_t>(i);
 }
 
 // One wavefront per window at a time: the window's voxels in (local id, row) order.  The rank of an element is
@@ -900,11 +896,10 @@ int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_w
     GridPlan *plan = reinterpret_cast<GridPlan *>(base + L.plan);
     int32_t *partials = reinterpret_cast<int32_t *>(base + L.partials);
     int32_t *cells = reinterpret_cast<int32_t *>(base + L.cells);
-    uint64_t *scan = reinterpret_cast<uint64_t *>(base + L.scan);
     int2 *place = reinterpret_cast<int2 *>(base + L.place);
     uint64_t *keys = reinterpret_cast<uint64_t *>(base + L.keys);
     CellSum *sums = reinterpret_cast<CellSum *>(base + L.sums);
-    const int64_t num_cells = (L.cells_cap + 1) * num_sets;
+    const int64_t num_cells = L.cells_cap * num_sets;
     const unsigned per_set = static_cast<unsigned>(num_sets);
     const dim3 grid(static_cast<unsigned>(ceil_div(N, kThreads)), per_set);
     hipLaunchKernelGGL(grid_bbox_kernel, dim3(kGridBoxes + kGridZeros), dim3(kThreads), 0, s, coords, N, sets, partials, cells, num_cells);
@@ -915,10 +910,10 @@ int window_indices(const int32_t *coords, int64_t N, int32_t stride, const s3d_w
     // (a third of the runs there may be: most lattices are smaller, and a workgroup takes another run where one is not)
     const dim3 sum_grid(static_cast<unsigned>(ceil_div(L.cells_cap, 3 * kSumCells)), per_set);
     hipLaunchKernelGGL(grid_sums_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums);
-    hipLaunchKernelGGL(grid_starts_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums, scan, host_counts);
+    hipLaunchKernelGGL(grid_starts_kernel, sum_grid, dim3(kSumThreads), 0, s, sets, plan, cells, L.cells_cap, sums, host_counts);
     S3D_HIP_CHECK(hipGetLastError());
     if (counted) S3D_HIP_CHECK(hipEventRecord(counted, s));
-    hipLaunchKernelGGL(grid_place_kernel, grid, dim3(kThreads), 0, s, place, N, sets, plan, scan, L.cells_cap, keys);
+    hipLaunchKernelGGL(grid_place_kernel, grid, dim3(kThreads), 0, s, place, N, sets, plan, cells, L.cells_cap, keys);
     S3D_HIP_CHECK(hipGetLastError());
     // about one window per wavefront if the windows hold 16 voxels on average, more in turn otherwise
     int64_t order_blocks = ceil_div(N, 64);

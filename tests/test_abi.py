@@ -148,3 +148,12 @@ def test_pair_store_limit_counts_what_the_store_holds():
     from swin3d_amd.sparse_dl.attn import attn_coff
     most = attn_coff.BWD_PAIR_STORE_MAX_BYTES // 8
     assert attn_coff._pair_store_fits(most // 6, 6) and attn_coff._pair_store_fits(most, 1) and not attn_coff._pair_store_fits(most // 6 + 1, 6)
+
+
+def test_window_index_workspace_is_what_the_sort_needs(hip_lib):
+    """A set's cells (six a voxel, one word each), the voxels' places and their keys."""
+    for n in (20_000, 199_327, 595_677):
+        for sets in (1, 2, 3):
+            need = hip_lib.s3d_window_indices_workspace_bytes(n, sets)
+            assert 40 * n * sets <= need <= (40 * n + 24 * (6 * n // 4096 + 1)) * sets + 8192     # (sums of 4096 cells; the box)
+        assert hip_lib.s3d_window_index_grid_workspace_bytes(n) == hip_lib.s3d_window_indices_workspace_bytes(n, 1)
