@@ -5,8 +5,8 @@ the library's kernels, those of a training pass forward through torch (hipBLASLt
 27-offset stem convolution is one GEMM of torch's.  Window attention runs through
 `SelfAttnAIOFunction`, the window index through `window_sets` / `window_signals`, neighbour
 gathering through `KNN` / `knn_max_pool`.  On the GPU the coordinate work runs on the library's kernels too
-(coarse cells and their representatives from the window sort, the stem's neighbour rows by binary search in
-sorted packed keys, the fused add + LayerNorm); the same functions have a tensor statement for host tensors,
+(coarse cells and their representatives from the window sort, the stem's neighbour rows from a table of the
+voxels, the fused add + LayerNorm); the same functions have a tensor statement for host tensors,
 against which the kernels are tested.  The geometry of all stages is computed first (`plan_stages`): it
 needs no features and is the only place where the host waits for the device.
 
@@ -86,13 +86,6 @@ def _check_signals(coords, signals):
     """A voxel's signals are the row of its own number, which kernels and index operations read without looking."""
     if signals.device != coords.device or signals.shape[0] < coords.shape[0]:
         raise ValueError(f"signals {tuple(signals.shape)} on {signals.device} for {coords.shape[0]} voxels on {coords.device}")
-
-
-def lookup_rows(sorted_keys, order, query_keys):
-    """row of every query key in the voxel set described by (sorted_keys, order); -1 if absent."""
-    pos = torch.searchsorted(sorted_keys, query_keys).clamp_(max=sorted_keys.numel() - 1)
-    hit = sorted_keys[pos] == query_keys
-    return torch.where(hit, order[pos], torch.full_like(pos, -1))
 
 
 def conv3x3x3_neighbours(coords, stride):
