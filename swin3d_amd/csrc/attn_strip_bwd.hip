@@ -19,8 +19,8 @@
 // a wavefront did not fit beside the rest, and 300 MB a call went to memory and back for it.  Registers are what is scarce:
 // with fourteen of them spilled inside the loop the launch by query took 153 us, with none 138.
 // Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 138 us, by key 133
-// (one kernel on 64 x 64 tiles: 523).  VALU 48 and 55 % of the time, LDS addressed 20 %, matrix pipe 11 %; a wavefront waits
-// for 55 % of its time, at the barriers and for the pairs and coordinates it reads.
+// (one kernel on 64 x 64 tiles: 523).  VALU 58 and 56 % of the time, LDS addressed 28 and 24 %, matrix pipe 14 and 12 %; a
+// wavefront waits for half of its time, at the barriers and for the pairs and coordinates it reads.
 #include "attn_strip.h"
 
 #include <cmath>

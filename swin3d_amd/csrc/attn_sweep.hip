@@ -746,10 +746,15 @@ template <typename T, int D, int HP> __host__ __device__ constexpr int key_row_s
 // rows are widened as they are loaded and the gradients rounded as they are stored, the arithmetic is that of T = TF
 // = float on widened copies.
 template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned>
-// Wavefronts per SIMD, by register cap.  fp16 at head_dim 8: four (128 registers).  fp16 at head_dim 16 and fp32 at head_dim 8: three (168 registers, 3 to
-// 20 of them spilled: the backward of the window-7 layer with 6 heads of 16 2.05 -> 1.99 ms, of the headline layer
-// in fp32 2.28 -> 2.05 ms).  fp32 at head_dim 16: two - uncapped it takes 286 registers and runs one wavefront per
-// SIMD (6-head window-7 layer 3.16 ms; capped at 256 with 24 spilled 2.89).
+// Wavefronts per SIMD, by register cap: fp16 four at head_dim 8, three at 16; fp32 three and two.  The key-owned sweep stays
+// below all of them (113 to 167 registers); of the query-owned one nine axes spill 9 (fp16, 16), 1 (fp32, 8), 21 and, beside
+// fp16 rows, 13 (fp32, 16).  us of the query-owned and the key-owned sweep with one wavefront more, as it is, one less:
+//   head_dim 8, 199,327 voxels in windows of 26, 6 heads: fp16 495 + 383, 336 + 270, 332 + 266 (the cap binds neither);
+//     fp32 1440 + 372, 431 + 366, 574 + 370; beside fp16 rows 1203 + 303, 426 + 303, 551 + 302
+//   head_dim 16, 49,682 voxels, windows of ten a side, whose tables are too long for strips: fp16 2123 + 939, 939 + 589,
+//     953 + 587; fp32 14266 + 1066, 3564 + 1038, 2526 + 1014; beside fp16 rows 12006 + 738, 2864 + 715, 2538 + 714
+// (in the last two LDS holds one workgroup a CU, with tables of 432 rows; it holds two below 394, with six axes too, which spill
+// nothing).
 __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (D == 8 ? 4 : 3) : (D == 8 ? 3 : 2))) void attn_bwd_pairs_kernel(BwdPairArgs b)
 {
     const AttnArgs &a = b.f;

@@ -9,8 +9,8 @@
 // Why tiles: the pair sweeps this form replaces run at two wavefronts per SIMD (192 VGPRs) and wait for a gathered table
 // row of 64 bytes per pair, axis and table.  Here a pair's term is a word of LDS.  One form for every window size: a unit
 // packs windows of up to 64 voxels side by side.  12,421 voxels in windows of 72, 9 axes, 12 heads, fp32 tables beside fp16
-// features: 183 us; the VALU issues 36 % of the time, the LDS is addressed for 31 %, the matrix pipe works for 5 %, and a
-// wavefront waits for 47 % of its time, most of it at barriers.
+// features: 182 us; the VALU issues 40 % of the time, the LDS is addressed for 33 %, the matrix pipe works for 6 %, and a
+// wavefront waits for 48 % of its time, most of it at barriers.
 #include "attn_strip.h"
 
 #include <algorithm>

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kThreads) void segment_size_kernel(const int32_t *_
 //
 // The windows, their pairs and the largest are known when the cells have been added up, and a host that sizes by them what
 // follows on the same stream waits for that and not for the placing behind it (two sets with their signals at 199,327 voxels: 81 us a
-// pass, 94 where it waits for all, which another stream that reads the sets needs).  (The sums run over the cells that the lattice has, not
+// pass, 96 where it waits for all, which another stream that reads the sets needs).  (The sums run over the cells that the lattice has, not
 // over those it may have, in two launches; a library's scan over 2 N took two as well, 14 us against 6 at 199,327 voxels.)
 constexpr int kGridBoxes = 128;          // workgroups of the bounding-box pass
 constexpr int kGridZeros = 384;          // ... and those beside them that only clear cells (without them two sets 1 to 2 us longer)
