@@ -7,8 +7,8 @@
 //   dq_i  += dL (k_j + Tq(i,j))                    dTq[n][row_n(i,j)] += dL q_i
 //   dk_j  += dL (q_i + Tk(i,j))                    dTk[n][row_n(i,j)] += dL k_j
 // The reference adds every term with a global atomic.  Here every output element has ONE owner, and the call has three
-// forms.  With the window set's pair count it runs at head_dim 16 on tiles and strips (attn_tile_bwd.hip, attn_strip_bwd.hip:
-// tables of up to 64 rows on a position axis and 32 on a signal axis), otherwise the pair sweeps of attn_sweep.hip on the
+// forms.  With the window set's pair count it runs on strips (tables of up to 64 rows on a position axis and 32 on a signal
+// axis; attn_strip_bwd.hip, at head_dim 16 behind attn_tile_bwd.hip, at 8 behind a sweep), otherwise the pair sweeps of attn_sweep.hip on the
 // forward's packed work list (dq, which leaves dL and P of every (pair, head) in the workspace; dk and dv) and the
 // table-gradient kernels below (attn_bwd_tables_kernel), which read dL and P.  Without it, the fused sweeps (attn_bwd_sweep_kernel),
 // which recompute the logits and need no store:
@@ -1438,6 +1438,7 @@ int attn_bwd(
         pr.f.N = N; pr.f.W = W;
         for (int n = 0; n < kMaxAxes; ++n) { pr.f.rows[n] = a.rows[n]; pr.f.base[n] = a.base[n]; }
         pr.dout = dout;
+        pr.out = out;
         pr.stat_max = out_max; pr.stat_sum = out_sum; pr.delta = a.delta;
         pr.dq = dq; pr.dk = dk; pr.dv = dv;
         pr.pos_base = a.pos_base;
@@ -1446,6 +1447,12 @@ int attn_bwd(
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (N > 0 && W > 0 && attn_tile_bwd_applies(a.rows, nd, D, pairs))
         return launch_attn_tile_bwd(pr, out, dtable_q, dtable_k, dtable_v, workspace, dtype, s);
+    // (beside the records the strips take the room of the table-gradient kernels' slots; the row map stays where it is)
+    if (N > 0 && W > 0 && pairs > 0) {
+        char *room = reinterpret_cast<char *>(a.tgrad);
+        if (attn_strip8_applies(a.rows, nd, D, dtype, N, W, H, pairs, bwd_tgrad_bytes(H, D, nd)))
+            return launch_attn_strip8(pr, dtable_q, dtable_k, dtable_v, room, dtype, s);
+    }
     if (N == 0 || W == 0) {
         // nothing to differentiate: the table gradients are zero
         a.N = 0;

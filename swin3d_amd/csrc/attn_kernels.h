@@ -73,7 +73,7 @@ int device_cus();
 constexpr int kPairSpare = 4;     // records that a lane of the key-owned sweep reads at a time
 struct BwdPairArgs {
     AttnArgs f;                  // shape, q, k, v, tables, index arrays (n2n required), rows[] / base[], workspace
-    const void *dout;            // [N,H,D]
+    const void *dout, *out;      // [N,H,D]
     const float *stat_max, *stat_sum, *delta;   // [N,H]: the forward's statistics, dout_i . o_i
     void *dq, *dk, *dv;          // [N,H,D], rows `grad_stride` elements apart (q, k, v: f.row_stride)
     int64_t grad_stride;
@@ -82,6 +82,8 @@ struct BwdPairArgs {
     int64_t pairs;               // capacity of pd per head; windows beyond it are skipped
 };
 int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream);
+// dL and P alone (head_dim 8), with dout_i . o_i made from b.out in place of b.delta
+int launch_attn_bwd_records(const BwdPairArgs &b, int dtype, hipStream_t stream);
 
 // The backward on tiles (attn_tile_bwd.hip): head_dim 16, tables that fit a stage, the pair count known.  Of the
 // arguments it takes the shape, inputs and dq, dk, dv; its own workspace holds records, slots, unit and strip list.
@@ -89,5 +91,11 @@ bool attn_tile_bwd_applies(const int32_t *rows, int nd, int D, int64_t pairs);
 size_t attn_tile_bwd_bytes(int H, int nd, int64_t N, int64_t W, int64_t pairs);
 int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, float *dtk, float *dtv, void *workspace, int dtype,
                          hipStream_t stream);
+
+// The backward at head_dim 8 on strips (attn_strip_bwd.hip): records by launch_attn_bwd_records, everything that is a sum over
+// pairs from those.  `room`: attn_strip8_bytes of device memory beside what the pair sweeps have.
+bool attn_strip8_applies(const int32_t *rows, int nd, int D, int dtype, int64_t N, int64_t W, int H, int64_t pairs, size_t room);
+size_t attn_strip8_bytes(int H, int nd, int64_t N, int64_t W);
+int launch_attn_strip8(const BwdPairArgs &p, float *dtq, float *dtk, float *dtv, void *room, int dtype, hipStream_t stream);
 
 }  // namespace s3d

@@ -9,18 +9,21 @@
 //     dx[column][c] += sum_rows H[row][column] T[row][c]      (dq from Tq, dk from Tk)
 // and the pairs themselves, read as matrix operands, the rest of dq, dk and dv.  A voxel's pairs are all in its strip, so dq,
 // dk and dv are stored once; table gradients stay in the registers of the wavefronts that make them for all strips of a
-// workgroup, which works on one head, and meet in a reduction over the workgroups.
+// workgroup, which works on one head, and meet in a reduction over the workgroups.  At head_dim 8 the pairs come from a sweep
+// (attn_sweep.hip, launch_attn_bwd_records), and q (or k) and dout share the sixteen channels of the products.
 //
 // Why strips of 16: the histograms of all axes fit LDS side by side (384 rows of 16 columns: 48 KB with P, 24 KB without), so
-// a strip passes three barriers, where tiles of 64 x 64 pairs, an axis or two at a time, passed some fifty; a row of 16 cells
+// a strip passes two barriers, where tiles of 64 x 64 pairs, an axis or two at a time, passed some fifty; a row of 16 cells
 // is half of the banks or a quarter of them, and additions of lanes that hold 16 columns meet in none that costs (5.1 and
 // 6.7 clocks a wavefront, 4.7 and 6.7 without any conflict; rows of 72 cells: 6.1 and 8.1).  Eight wavefronts and 128
 // registers, two workgroups a CU: with four wavefronts and 168 registers, three workgroups, the table gradients and tables of
 // a wavefront did not fit beside the rest, and 300 MB a call went to memory and back for it.  Registers are what is scarce:
 // with fourteen of them spilled inside the loop the launch by query took 153 us, with none 138.
-// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 138 us, by key 133
-// (one kernel on 64 x 64 tiles: 523).  VALU 58 and 56 % of the time, LDS addressed 28 and 24 %, matrix pipe 14 and 12 %; a
-// wavefront waits for half of its time, at the barriers and for the pairs and coordinates it reads.
+// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 128 us, by key 125
+// (one kernel on 64 x 64 tiles: 523; with a third barrier before the histograms and coordinates asked for behind it, 138 and
+// 133).  head_dim 8, 199,327 voxels in windows of 26, 6 heads, fp16: 572 and 511 us, where the sweeps' own sums and the kernels
+// of the table gradients took 1510.  What bounds them is VALU issue, 71 to 79 % of the time: at head_dim 8 some 300 to 350
+// instructions a wavefront and strip, a third of them the histograms' conversion into operands, 45 the nine rows of a pair.
 #include "attn_strip.h"
 
 #include <cmath>
@@ -88,15 +91,47 @@ __device__ __forceinline__ f16x4 to_half4(float a, float b, float c, float d)
     const f16x2 x = __builtin_convertvector(f32x2{a, b}, f16x2), y = __builtin_convertvector(f32x2{c, d}, f16x2);
     return __builtin_shufflevector(x, y, 0, 1, 2, 3);
 }
+// two numbers times a power of two as fp16 numbers, and what that leaves of them likewise (v_fma_mixlo_f16 and its like, one
+// instruction a number in place of one and a half, take twice the time)
+__device__ __forceinline__ uint32_t scaled_half2(float x, float y, float scale)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x * scale, y * scale}), f16x2));
+}
+__device__ __forceinline__ uint32_t scaled_rest2(float x, float y, float scale, uint32_t h)
+{
+    const f16x2 t = __builtin_bit_cast(f16x2, h);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{__builtin_fmaf(x, scale, -static_cast<float>(t[0])),
+                                                                       __builtin_fmaf(y, scale, -static_cast<float>(t[1]))}), f16x2));
+}
+// a choice among the four numbers of an operand; of a number in both halves of a word
+struct OneOfFour {
+    u32x2 mask;
+    __device__ __forceinline__ explicit OneOfFour(int at)
+    {
+        const uint32_t half = (at & 1) ? 0xffff0000u : 0xffffu;
+        mask = {(at >> 1) == 0 ? half : 0u, (at >> 1) == 1 ? half : 0u};
+    }
+    __device__ __forceinline__ u32x2 of(uint32_t x) const { return {x & mask[0], x & mask[1]}; }
+};
 template <> struct Parts4<__half> {
     f16x4 hi, lo;
     template <bool kNearest = true> __device__ __forceinline__ void set(const float *v, float scale)
     {
-        hi = to_half4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
-        float r[4];
+        u32x2 h, l;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(v[e], scale, -static_cast<float>(hi[e]));
-        lo = to_half4(r[0], r[1], r[2], r[3]);
+        for (int e = 0; e < 2; ++e) {
+            h[e] = scaled_half2(v[2 * e], v[2 * e + 1], scale);
+            l[e] = scaled_rest2(v[2 * e], v[2 * e + 1], scale, h[e]);
+        }
+        hi = __builtin_bit_cast(f16x4, h);
+        lo = __builtin_bit_cast(f16x4, l);
+    }
+    // the number `at` (0..3) of the four, the others zero
+    __device__ __forceinline__ void set_one(float v, float scale, const OneOfFour &at)
+    {
+        const uint32_t h = scaled_half2(v, v, scale), l = scaled_rest2(v, v, scale, h);
+        hi = __builtin_bit_cast(f16x4, at.of(h));
+        lo = __builtin_bit_cast(f16x4, at.of(l));
     }
 };
 template <> struct Parts4<float> {
@@ -128,6 +163,16 @@ template <> struct Parts4<float> {
         }
 #pragma unroll
         for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(s16x4, out[k]);
+    }
+    __device__ __forceinline__ void set_one(float v, float scale, const OneOfFour &at)
+    {
+        float x = v * scale;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, x}), bf16x2));
+            s[k] = __builtin_bit_cast(s16x4, at.of(b));
+            if (k < 2) x -= __uint_as_float(b << 16);
+        }
     }
 };
 template <> struct Exact4<float> : Parts4<float> {
@@ -196,6 +241,15 @@ template <> struct Raw4<float> {
         return mfma4(y.s[0], identity, mfma4(y.s[1], identity, mfma4(y.s[2], identity, f32x4_t{})));
     }
 };
+// sum over the four lanes of a column (lane % 16)
+__device__ __forceinline__ float sum_columns(float x)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 template <typename T, typename TF> struct StripTable { using type = Exact4<TF>; };
 template <> struct StripTable<float, __half> { using type = Parts4<__half>; };
 
@@ -224,7 +278,9 @@ template <typename V> __device__ __forceinline__ V max16(V v)
     return step(v, std::integral_constant<int, 0x140>{});  // row_mirror
 }
 
-template <typename T, typename TF, int ND, bool kByKey>
+// C channels a head: 16, or 8 (packed): q or k and dout then share the sixteen channels of an operand, dTq and dTv the sixteen
+// columns of a product, and dk and dv its rows.
+template <typename T, typename TF, int ND, bool kByKey, int C>
 __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(StripArgs b)
 {
     using Table = typename StripTable<T, TF>::type;
@@ -232,22 +288,28 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     using Unit4 = typename std::conditional<sizeof(TF) == 2, f16x4, s16x4>::type;
     constexpr int kCellBytes = kByKey ? 4 : 8, kRowBytes = kStrip * kCellBytes;
     constexpr int kKinds = kByKey ? 1 : 2, kOwn = kOwnTiles<ND>;
+    constexpr bool kPacked = C == 8;
+    constexpr int kSets = kPacked ? 1 : kKinds;        // of features, and of table gradients
+    constexpr int kParts = kByKey && !kPacked ? 2 : 1; // of dx: dk and dv
+    // Windows whose keys are one step's in a form of their own: most are at the level of eight channels.  (At sixteen few are,
+    // and the second form costs the other one registers.)
+    auto one_step = [](int n) { return kPacked && n <= kStripReach; };
     const AttnArgs &a = b.f;
     // cells [row][column]: dL, by query behind P; then parts of dx (by key: and dv), one a wavefront
     __shared__ __align__(16) uint32_t cells_s[kTiles<ND> * 16 * kStrip * kKinds];
-    __shared__ __align__(16) float part_s[(kByKey ? 2 : 1) * kStripWaves * 256];
+    __shared__ __align__(16) float part_s[kParts * kStripWaves * 256];
     __shared__ float sums_s[kStripWaves][kStrip], grad_s;
-    __shared__ __align__(16) Exact4<TF> features_s[kKinds][64];        // q or k, dout of the strip's voxels
+    __shared__ __align__(16) Exact4<TF> features_s[kSets][64];        // q or k, dout of the strip's voxels
     __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s;
     // Pieces of the table's operands that wait in LDS, as many as leave room for two workgroups a CU (81,864 of 81,920 bytes by
     // query in fp32).  In registers they would not fit beside the rest, and a spilled operand comes back from memory behind the
     // pairs of the next strip, which are on their way then: loads return in order.
-    constexpr int kParts = sizeof(Table) / 8, kPieces = kParts * kOwn;
+    constexpr int kTableParts = sizeof(Table) / 8, kPieces = kTableParts * kOwn;
     constexpr int kShared = kByKey || kPieces < kOwn + 2 ? kPieces : kOwn + 2, kKeptPieces = kPieces - kShared;
-    struct TableParts { u32x2 part[kParts]; };
+    struct TableParts { u32x2 part[kTableParts]; };
     __shared__ u32x2 table_s[kShared][kStripThreads];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int H = a.H, HD = H * D;
+    const int H = a.H, HD = H * C;
     const uint32_t stride = static_cast<uint32_t>(a.row_stride);       // of q, k, v
     const int h = static_cast<int>(blockIdx.x) % H;
     const int group = static_cast<int>(blockIdx.x) / H, groups = static_cast<int>(gridDim.x) / H;
@@ -257,8 +319,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     const int c16 = lane & 15, g4 = lane >> 4, reach0 = tid >> 4;
     const float nan = __int_as_float(0x7fc00000);
 
-    const TF *gx = static_cast<const TF *>(kByKey ? a.k : a.q) + h * D, *gy = static_cast<const TF *>(kByKey ? a.q : a.k) + h * D;
-    const TF *gd = static_cast<const TF *>(b.dout) + h * D;
+    const TF *gx = static_cast<const TF *>(kByKey ? a.k : a.q) + h * C, *gy = static_cast<const TF *>(kByKey ? a.q : a.k) + h * C;
+    const TF *gd = static_cast<const TF *>(b.dout) + h * C;
     const float2 *records = b.records + static_cast<int64_t>(h) * b.pairs;
     const float scale_table = b.scales[h * 3 + (kByKey ? 1 : 0)];    // what a product with the table is multiplied by
 
@@ -266,7 +328,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     // 8 i + wave is this wavefront's.
     u32x2 table[kKeptPieces > 0 ? kKeptPieces : 1];
     {
-        const T *from = static_cast<const T *>(kByKey ? a.table_k : a.table_q) + h * D + c16;
+        const T *from = static_cast<const T *>(kByKey ? a.table_k : a.table_q) + h * C + c16 % C;
 #pragma unroll
         for (int i = 0; i < kOwn; ++i) {
             const int tile = i * kStripWaves + wave, axis = tile_axis(tile);
@@ -276,7 +338,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                 for (int e = 0; e < 4; ++e) {
                     const int r = min(tile_row0(tile) + 4 * e + g4, axis_rows<ND>(a, axis) - 1);
                     const float x = to_float(from[static_cast<int64_t>(axis_base<ND>(a, axis) + r) * HD]);
-                    v[e] = finite(x) ? x : 0.0f;
+                    v[e] = finite(x) && c16 < C ? x : 0.0f;
                 }
             }
             Table x;
@@ -284,7 +346,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             else x.set(v);
             const TableParts parts = __builtin_bit_cast(TableParts, x);
 #pragma unroll
-            for (int k = 0; k < kParts; ++k) {
+            for (int k = 0; k < kTableParts; ++k) {
                 const int piece = k * kOwn + i;
                 if (piece < kKeptPieces) table[piece] = parts.part[k];
                 else table_s[piece - kKeptPieces][tid] = parts.part[k];
@@ -302,9 +364,9 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             identity[e] = static_cast<short>(4 * g4 + e == c16 ? 0x3f80 : 0);
         }
     }
-    f32x4_t grads[kKinds][kOwn];
+    f32x4_t grads[kSets][kOwn];
 #pragma unroll
-    for (int kind = 0; kind < kKinds; ++kind)
+    for (int kind = 0; kind < kSets; ++kind)
 #pragma unroll
         for (int i = 0; i < kOwn; ++i) grads[kind][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     for (int t = tid; t < kTiles<ND> * 16 * kStrip * kKinds / 4; t += kStripThreads) reinterpret_cast<uint4 *>(cells_s)[t] = make_uint4(0, 0, 0, 0);
@@ -316,7 +378,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     // the strip before goes through its products.
     struct Ahead {
         int4 column;
-        Raw4<TF> x;                          // (first wavefront: q or k; second one, by query: dout)
+        Raw4<TF> x;                          // (first wavefront: q or k; second one, by query: dout; packed the first both)
         float2 kept[kKept];
     } ahead;
     // pair with the window's j-th voxel: by query [key][query], by key likewise
@@ -325,98 +387,129 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     // the first of a lane's four channels, in a form that the compiler does not add to the pointers outside of the loop: that
     // would keep two registers for each
     auto part4 = [&]() {
-        uint32_t c = 4 * g4;
+        uint32_t c = 4 * g4 % C;
         asm volatile("" : "+v"(c));
         return c;
     };
-    auto fetch = [&](int n) {
-        if (wave < kKinds)
-            ahead.x.load((wave == 0 ? gx : gd) + (static_cast<uint64_t>(static_cast<uint32_t>(ahead.column.y)) *
-                                                  (wave == 0 ? stride : static_cast<uint32_t>(HD)) + part4()));
-        const int first = pair_at(ahead.column, n), step = pair_step(ahead.column, n);
-#pragma unroll
-        for (int s = 0; s < kKept; ++s) ahead.kept[s] = records[first + min(reach0 + s * kStripReach, n - 1) * step];
+    // four channels of a row of x or, `other`, of dout
+    auto load4 = [&](Raw4<TF> &r, const TF *x, int row, bool other) {
+        r.load((other ? gd : x) + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * (other ? static_cast<uint32_t>(HD) : stride) + part4()));
     };
-    int4 strip = b.list.strips[group];
-    ahead.column = b.columns[group * kStrip + c16];
-    fetch(__builtin_amdgcn_readfirstlane(strip.y));
-
-    for (int u = group; u < strips; u += groups) {
-        const int n = __builtin_amdgcn_readfirstlane(strip.y);
-        const int col0 = __builtin_amdgcn_readfirstlane(strip.z), cols = __builtin_amdgcn_readfirstlane(strip.w);
-        // window of a column or key (these are below 2^12; of a larger window it is the only one)
-        const float inv_n = n > kCols ? 0.0f : 1.0f / static_cast<float>(n);
-        auto window_of = [&](int x) { return static_cast<int>((static_cast<float>(x) + 0.5f) * inv_n); };
-        // this lane's column
-        const int4 column = ahead.column;
-        const int own_window = window_of(col0 + min(c16, cols - 1));
+    auto fetch = [&](int n) {
+        if (wave < kSets) load4(ahead.x, gx, ahead.column.y, kPacked ? !kByKey && g4 >= 2 : wave > 0);
+        const int first = pair_at(ahead.column, n), step = pair_step(ahead.column, n);
+        ahead.kept[0] = records[first + min(reach0, n - 1) * step];
+        if (!one_step(n)) {
+#pragma unroll
+            for (int s = 1; s < kKept; ++s) ahead.kept[s] = records[first + min(reach0 + s * kStripReach, n - 1) * step];
+        }
+    };
+    // dL and P of a column's pair with a voxel
+    auto settle = [&](float2 r, bool fits, bool pair) {
+        if (!fits || !(r.y <= kMostWeight)) r = make_float2(nan, nan);
+        return pair ? r : make_float2(0.0f, 0.0f);
+    };
+    // A strip is opened while the one before waits for its last barrier: its pairs come to rest, their sum of |dL| goes to the
+    // others, and what else its threads read is asked for.
+    int n, col0, cols, key_row;
+    int4 column;
+    float2 kept[kKept];
+    float own[ND], other[2][ND];
+    // (the key of c16 / 4 and, of a window with more than a step's, the term c16 % 4)
+    const int key = wave * (64 / kStrip) + (c16 >> 2), term = key + (c16 & 3) * kStripReach;
+    // window of a column or key, of the strip's (these are below 2^12; of a larger window it is the only one)
+    auto window_of = [](int n, int x) {
+        const float inv = __builtin_amdgcn_rcpf(static_cast<float>(n));      // (an error of 2^-22 does not reach a whole number: n is at most 64)
+        return static_cast<int>((static_cast<float>(x) + 0.5f) * (n > kCols ? 0.0f : inv));
+    };
+    auto last_window = [&](int n, int col0, int cols) { return __builtin_amdgcn_readfirstlane(window_of(n, col0 + cols - 1)); };
+    auto open = [&](int u, int4 strip) {
+        n = __builtin_amdgcn_readfirstlane(strip.y);
+        col0 = __builtin_amdgcn_readfirstlane(strip.z);
+        cols = __builtin_amdgcn_readfirstlane(strip.w);
+        column = ahead.column;
         const bool there = c16 < cols, fits = column.w >= 0;
         incomplete = incomplete || !fits;
         const int pair0 = pair_at(column, n), step = pair_step(column, n);
-        const int windows = __builtin_amdgcn_readfirstlane(window_of(col0 + cols - 1) + 1);
-        const int own_row = column.y;
-        // row of key c16 of a step's sixteen: those of the wavefront's pairs, in the order of the operands' terms (the columns
-        // of the windows' voxels are side by side)
-        const int32_t *rows = b.column_rows + (u * kStrip - col0);
-        const int term = wave * (64 / kStrip) + (c16 >> 2) + (c16 & 3) * kStripReach;
-        int key_row = rows[min(term, n - 1)];
-        // the next strip
-        const int u_next = min(u + groups, strips - 1);
-        strip = b.list.strips[u_next];
-        ahead.column = b.columns[u_next * kStrip + c16];
-
-        // dL and P of this column's pair with a voxel
-        auto settle = [&](float2 r, bool pair) {
-            if (!fits || !(r.y <= kMostWeight)) r = make_float2(nan, nan);
-            return pair ? r : make_float2(0.0f, 0.0f);
-        };
-        float2 kept[kKept];
         float sum = 0.0f, weights = 0.0f;
-#pragma unroll
-        for (int s = 0; s < kKept; ++s) {
+        auto keep = [&](int s) {
             const bool pair = there & (reach0 + s * kStripReach < n);
             kept[s] = make_float2(pair ? ahead.kept[s].x : 0.0f, pair ? ahead.kept[s].y : 0.0f);
             sum += fabsf(kept[s].x);
             weights += kept[s].y;
+        };
+        keep(0);
+        if (!one_step(n)) {
+#pragma unroll
+            for (int s = 1; s < kKept; ++s) keep(s);
         }
         if (__any(!fits | !finite(sum) | !(weights <= kMostWeight))) {
             sum = 0.0f;
 #pragma unroll
             for (int s = 0; s < kKept; ++s) {
-                kept[s] = settle(kept[s], there & (reach0 + s * kStripReach < n));
+                if (s > 0 && one_step(n)) break;
+                kept[s] = settle(kept[s], fits, there & (reach0 + s * kStripReach < n));
                 sum += finite(kept[s].x) ? fabsf(kept[s].x) : 0.0f;
             }
         }
         for (int j0 = kKept * kStripReach; j0 < n; j0 += kStripReach) {
             const int j = j0 + reach0;
-            const float2 r = settle(records[pair0 + min(j, n - 1) * step], there & (j < n));
+            const float2 r = settle(records[pair0 + min(j, n - 1) * step], fits, there & (j < n));
             sum += finite(r.x) ? fabsf(r.x) : 0.0f;
         }
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
+        sum = sum_columns(sum);
         if (lane < kStrip) sums_s[wave][c16] = sum;
-        lds_barrier();
-        sum = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kStripWaves; ++w) sum += sums_s[w][c16];
-        const int exponent = exponent_of(sum);
-
-        float own[ND], other[2][ND];
+        // row of key c16 of a step's sixteen: those of the wavefront's pairs, in the order of the operands' terms (the columns
+        // of the windows' voxels are side by side)
+        key_row = b.column_rows[u * kStrip - col0 + (!one_step(n) ? min(term, n - 1) : min(c16 & 3, last_window(n, col0, cols)) * n + min(key, n - 1))];
         load_coords<ND>(a.n_coords + static_cast<int64_t>(column.x) * ND, own);
         const float *coords = a.n_coords + static_cast<int64_t>(column.z) * ND;
+        load_coords<ND>(coords + min(reach0, n - 1) * ND, other[0]);
+        if (!one_step(n)) load_coords<ND>(coords + min(reach0 + kStripReach, n - 1) * ND, other[1]);
+    };
+    int4 strip = b.list.strips[group];
+    ahead.column = b.columns[group * kStrip + c16];
+    fetch(__builtin_amdgcn_readfirstlane(strip.y));
+    open(group, strip);
+    lds_barrier();
+
+    for (int u = group; u < strips; u += groups) {
+        // this lane's column
+        const int own_window = window_of(n, col0 + min(c16, cols - 1));
+        const bool there = c16 < cols, fits = column.w >= 0;
+        const int pair0 = pair_at(column, n), step = pair_step(column, n);
+        const int windows = last_window(n, col0, cols) + 1;
+        const int own_row = column.y;
+        const int32_t *rows = b.column_rows + (u * kStrip - col0);
+        const float *coords = a.n_coords + static_cast<int64_t>(column.z) * ND;
+        // the next strip
+        const int u_next = min(u + groups, strips - 1);
+        strip = b.list.strips[u_next];
+        ahead.column = b.columns[u_next * kStrip + c16];
+
+        float sum = 0.0f;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) load_coords<ND>(coords + min(reach0 + s * kStripReach, n - 1) * ND, other[s]);
+        for (int w = 0; w < kStripWaves; w += 4) sum += sums_s[w + g4][c16];
+        sum = sum_columns(sum);
+        const int exponent = exponent_of(sum);
         // what the products of the pairs themselves start with, while the histograms are filled
         Raw4<TF> y, z;
         auto fetch_keys = [&](int row) {
-            y.load(gy + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * stride + part4()));
-            if constexpr (kByKey) z.load(gd + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(HD) + part4()));
+            load4(y, gy, row, kPacked && kByKey && g4 >= 2);
+            if constexpr (kByKey && !kPacked) load4(z, gd, row, true);
         };
         fetch_keys(key_row);
 
         // ---- histograms
         const int up = kFixGrad - exponent;
         const uint32_t own_at = cells + c16 * kCellBytes;
+        // (in a form to which the compiler adds an axis' first row as the instruction's offset: it would keep nine sums otherwise)
+        auto cell_of = [](uint32_t row, uint32_t at) {
+            uint32_t r;
+            asm("v_lshl_add_u32 %0, %1, %2, %3" : "=v"(r) : "v"(row), "n"(kByKey ? 6 : 7), "v"(at));
+            return r;
+        };
+        static_assert(kRowBytes == (kByKey ? 64 : 128), "a shift");
         bool bad = false;
         auto add = [&](float2 r, const float *its) {
             const bool good = finite(r.x);
@@ -427,9 +520,9 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             for (int axis = 0; axis < ND; ++axis) {
                 const uint32_t row = static_cast<uint32_t>(kByKey ? crse_row(its[axis], own[axis], b.half_rows[axis], b.upper[axis])
                                                                   : crse_row(own[axis], its[axis], b.half_rows[axis], b.upper[axis]));
-                const uint32_t at = row * kRowBytes + own_at + axis_row0(axis) * kRowBytes;
-                if constexpr (kByKey) lds_add(at, static_cast<uint32_t>(fix_l));
-                else lds_add64(at, fix_p, fix_l);
+                const uint32_t at = cell_of(row, own_at), first = axis_row0(axis) * kRowBytes;
+                if constexpr (kByKey) lds_add(at + first, static_cast<uint32_t>(fix_l));
+                else lds_add64(at + first, fix_p, fix_l);
             }
         };
         add(kept[0], other[0]);
@@ -442,7 +535,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             for (int j0 = kKept * kStripReach; j0 < n; j0 += kStripReach) {
                 const int j = j0 + reach0;
                 load_coords<ND>(coords + min(j, n - 1) * ND, other[0]);
-                add(settle(records[pair0 + min(j, n - 1) * step], there & (j < n)), other[0]);
+                add(settle(records[pair0 + min(j, n - 1) * step], fits, there & (j < n)), other[0]);
             }
         }
         if (__any(bad)) {
@@ -450,7 +543,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             marked_s = 1;
 #pragma unroll 1
             for (int j = reach0; j < n; j += kStripReach) {
-                const float2 r = settle(records[pair0 + j * step], there);
+                const float2 r = settle(records[pair0 + j * step], fits, there);
                 if (finite(r.x)) continue;
 #pragma unroll 1
                 for (int axis = 0; axis < ND; ++axis) {
@@ -469,60 +562,84 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};           // over 2^(exponent - kLift): [channel][column]
         f32x4_t acc_v = {0.0f, 0.0f, 0.0f, 0.0f};
         const float scale = power2(kLift<TF> - exponent);
-        for (int w = 0; w < windows; ++w) {
+        // a step's features, [voxel][channel]; what is not finite as zeros
+        auto voxels_of = [&](Exact4<TF> &f, Exact4<TF> &fz) {
+            f32x4_t ys = y.voxels(identity), zs{};
+            if constexpr (kByKey && !kPacked) zs = z.voxels(identity);
+            if (__any(!finite(fabsf(ys[0]) + fabsf(ys[1]) + fabsf(ys[2]) + fabsf(ys[3]) + fabsf(zs[0]) + fabsf(zs[1]) + fabsf(zs[2]) + fabsf(zs[3])))) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    ys[e] = finite(ys[e]) ? ys[e] : 0.0f;
+                    zs[e] = finite(zs[e]) ? zs[e] : 0.0f;
+                }
+            }
+            const float yv[4] = {ys[0], ys[1], ys[2], ys[3]}, zv[4] = {zs[0], zs[1], zs[2], zs[3]};
+            f.set(yv);
+            if constexpr (kByKey && !kPacked) fz.set(zv);
+            else fz = f;
+        };
+        // windows of a step: a term of the four is the key's of its window, a column's pair in that of its own
+        for (int w0 = 0; one_step(n) && w0 < windows; w0 += 4) {
+            if (w0 > 0) fetch_keys(rows[min(w0 + (c16 & 3), windows - 1) * n + min(key, n - 1)]);
+            Exact4<TF> f, fz;
+            voxels_of(f, fz);
+            const OneOfFour window(own_window - w0);
+            Cell c;
+            c.set_one(kept[0].x, scale, window);
+            acc = product(f, c, acc);
+            if constexpr (kByKey) {
+                c.set_one(kept[0].y, kLiftP<TF>, window);
+                acc_v = product(fz, c, acc_v);
+            }
+        }
+        for (int w = 0; !one_step(n) && w < windows; ++w) {
             for (int j0 = 0; j0 < n; j0 += kKept * kStripReach) {
                 if (w + j0 > 0) fetch_keys(rows[w * n + min(j0 + term, n - 1)]);
-                f32x4_t ys = y.voxels(identity), zs = kByKey ? z.voxels(identity) : f32x4_t{};
-                if (__any(!finite(fabsf(ys[0]) + fabsf(ys[1]) + fabsf(ys[2]) + fabsf(ys[3]) + fabsf(zs[0]) + fabsf(zs[1]) + fabsf(zs[2]) + fabsf(zs[3])))) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        ys[e] = finite(ys[e]) ? ys[e] : 0.0f;
-                        zs[e] = finite(zs[e]) ? zs[e] : 0.0f;
-                    }
-                }
                 float l[4], p[4];
-                const float yv[4] = {ys[0], ys[1], ys[2], ys[3]}, zv[4] = {zs[0], zs[1], zs[2], zs[3]};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float2 r = kept[e];
                     if (j0 > 0) {
                         const int j = j0 + reach0 + e * kStripReach;
-                        r = settle(records[pair0 + min(j, n - 1) * step], there & (j < n));
+                        r = settle(records[pair0 + min(j, n - 1) * step], fits, there & (j < n));
                     }
                     l[e] = own_window == w ? r.x : 0.0f;
                     p[e] = own_window == w ? r.y : 0.0f;
                 }
-                Exact4<TF> f;
+                Exact4<TF> f, fz;
                 Cell c;
-                f.set(yv);
+                voxels_of(f, fz);
                 c.set(l, scale);
                 acc = product(f, c, acc);
                 if constexpr (kByKey) {
-                    f.set(zv);
                     c.set(p, kLiftP<TF>);
-                    acc_v = product(f, c, acc_v);
+                    acc_v = product(fz, c, acc_v);
                 }
             }
         }
 
         // features for the table gradients: q or k over the strip's largest exponent of a column, the largest value below 2^15,
         // as far as can be from where fp16 numbers lose bits
-        if (wave < kKinds) {
+        if (wave < kSets) {
             f32x4_t x = ahead.x.voxels(identity);
             if (__any(!finite(fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]) + fabsf(x[3])))) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x[e] = finite(x[e]) ? x[e] : 0.0f;
             }
             float v[4] = {x[0], x[1], x[2], x[3]};
+            const bool lifted = c16 < C || kByKey;         // (dout is not)
             if (wave == 0) {
                 const int top = __builtin_amdgcn_readfirstlane(max16(there ? exponent : -100));
-                const float most16 = max16(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+                const float most16 = max16(lifted ? fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))) : 0.0f);
                 float most = 0.0f;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) most = fmaxf(most, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(most16), 16 * g)));
                 const int lift = kLiftFeature - exponent_of(most);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = ldexpf(x[e], __shfl(exponent, 4 * g4 + e) - top + lift);
+                for (int e = 0; e < 4; ++e) {
+                    const int up = __shfl(exponent, 4 * g4 + e) - top + lift;
+                    v[e] = ldexpf(x[e], lifted ? up : 0);
+                }
                 grad_s = power2(top - lift - kLift<TF>);
             }
             Exact4<TF> f;
@@ -532,25 +649,39 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         fetch(__builtin_amdgcn_readfirstlane(strip.y));
         lds_barrier();
 
-        const Exact4<TF> feature = features_s[0][lane], feature_d = features_s[kKinds - 1][lane];
-        const float grad = grad_s;
+        Exact4<TF> feature = features_s[0][lane], feature_d = features_s[kSets - 1][lane];
+        const float grad = kPacked && !kByKey && c16 >= C ? 1.0f / kLiftP<TF> : grad_s;
+        if constexpr (kPacked && !kByKey) {
+            // the columns of dTq, and of dTv
+            if (c16 < C) feature_d = Exact4<TF>{};
+            else feature = Exact4<TF>{};
+        }
         // ---- matrix products of the histograms, which are cleared for the next strip (a tile without rows holds zeros)
         f32x4_t acc_t = {0.0f, 0.0f, 0.0f, 0.0f};         // ... the table's part, over scale_table as well
         const bool marked = __builtin_amdgcn_readfirstlane(marked_s) != 0;
         const uint32_t cell_at = cells + (wave * 16 + g4) * kRowBytes + c16 * kCellBytes;
 #pragma unroll
         for (int i = 0; i < kOwn; ++i) {
-            float l[4], p[4];
+            uint32_t cell_l[4], cell_p[4], any = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const uint32_t at = cell_at + (i * kStripWaves * 16 + e * 4) * kRowBytes;
                 if constexpr (kByKey) {
-                    l[e] = static_cast<float>(static_cast<int>(lds_load_u32(at)));
+                    cell_l[e] = lds_load_u32(at);
+                    cell_p[e] = 0;
                 } else {
                     const float2 v = lds_load2(at);
-                    p[e] = static_cast<float>(__float_as_uint(v.x));
-                    l[e] = static_cast<float>(__float_as_int(v.y));
+                    cell_p[e] = __float_as_uint(v.x);
+                    cell_l[e] = __float_as_uint(v.y);
                 }
+                any |= cell_l[e] | cell_p[e];
+            }
+            if (!__any(any != 0)) continue;
+            float l[4], p[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                l[e] = static_cast<float>(static_cast<int>(cell_l[e]));
+                p[e] = static_cast<float>(cell_p[e]);
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -562,45 +693,57 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             c.template set<sizeof(TF) == 2>(l, kGradCell<TF>);       // (the table's operand and the features are the nearest)
             TableParts parts;
 #pragma unroll
-            for (int k = 0; k < kParts; ++k) {
+            for (int k = 0; k < kTableParts; ++k) {
                 const int piece = k * kOwn + i;
                 parts.part[k] = piece < kKeptPieces ? table[piece < kKeptPieces ? piece : 0] : table_s[piece < kKeptPieces ? 0 : piece - kKeptPieces][tid];
             }
             acc_t = product(__builtin_bit_cast(Table, parts), c, acc_t);
             f32x4_t g = product(transposed(c, unit), feature, f32x4_t{});
+            if constexpr (!kByKey && kPacked) {
+                c.template set<sizeof(TF) == 2>(p, kWeightCell<TF>);
+                g = product(transposed(c, unit), feature_d, g);
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) grads[0][i][e] = fmaf(g[e], grad, grads[0][i][e]);
-            if constexpr (!kByKey) {
+            if constexpr (!kByKey && !kPacked) {
                 c.template set<sizeof(TF) == 2>(p, kWeightCell<TF>);
                 g = product(transposed(c, unit), feature_d, f32x4_t{});
 #pragma unroll
-                for (int e = 0; e < 4; ++e) grads[kKinds - 1][i][e] = fmaf(g[e], 1.0f / kLiftP<TF>, grads[kKinds - 1][i][e]);
+                for (int e = 0; e < 4; ++e) grads[kSets - 1][i][e] = fmaf(g[e], 1.0f / kLiftP<TF>, grads[kSets - 1][i][e]);
             }
         }
         if (marked) {
 #pragma unroll
             for (int i = 0; i < kOwn; ++i)
 #pragma unroll
-                for (int kind = 0; kind < kKinds; ++kind)
+                for (int set = 0; set < kSets; ++set) {
+                    const int kind = kPacked && !kByKey ? c16 / C : set;
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (marks_s[kind * kTiles<ND> + i * kStripWaves + wave] >> (4 * g4 + e) & 1) grads[kind][i][e] = nan;
+                        if (marks_s[kind * kTiles<ND> + i * kStripWaves + wave] >> (4 * g4 + e) & 1) grads[set][i][e] = nan;
+                }
         }
         // ---- dx and dv: the wavefronts' parts, added up by the last two
         const float back = power2(exponent - kLift<TF>);
         f32x4_t dx;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dx[e] = fmaf(acc_t[e], scale_table, acc[e]) * back;
+        for (int e = 0; e < 4; ++e) {
+            dx[e] = fmaf(acc_t[e], scale_table, acc[e]) * back;
+            if constexpr (kPacked && kByKey) dx[e] = g4 < 2 ? dx[e] : acc_v[e] * (1.0f / kLiftP<TF>);
+        }
         *reinterpret_cast<f32x4_t *>(&part_s[(wave * 64 + lane) * 4]) = dx;
-        if constexpr (kByKey) *reinterpret_cast<f32x4_t *>(&part_s[((kStripWaves + wave) * 64 + lane) * 4]) = acc_v;
+        if constexpr (kParts > 1) *reinterpret_cast<f32x4_t *>(&part_s[((kStripWaves + wave) * 64 + lane) * 4]) = acc_v;
+        __builtin_amdgcn_sched_barrier(0);
+        open(u_next, strip);
+        __builtin_amdgcn_sched_barrier(0);
         lds_barrier();
         const int which = kStripWaves - 1 - wave;
-        if (which < (kByKey ? 2 : 1)) {
+        if (which < kParts) {
             // (eight parts in fp32 would add to an fp32 result's error what its own rounding is)
             using Sum = typename std::conditional<sizeof(TF) == 4, double, float>::type;
             Sum sums[4] = {0, 0, 0, 0};
             float o[4];
-#pragma unroll
+#pragma unroll 2
             for (int w = 0; w < kStripWaves; ++w) {
                 const f32x4_t v = *reinterpret_cast<const f32x4_t *>(&part_s[((which * kStripWaves + w) * 64 + lane) * 4]);
 #pragma unroll
@@ -608,14 +751,16 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = static_cast<float>(sums[e]) * (which > 0 ? 1.0f / kLiftP<TF> : 1.0f);
-            if (there) store4(static_cast<TF *>(which > 0 ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * D + part4(), o);
+            const bool dv = kPacked ? kByKey && g4 >= 2 : which > 0;
+            if (there && (!kPacked || kByKey || g4 < 2))
+                store4(static_cast<TF *>(dv ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * C + part4(), o);
         }
     }
     // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]
     const bool none = __syncthreads_or(incomplete);
-    float *slot = b.slots + static_cast<int64_t>(blockIdx.x) * (kKinds * kTiles<ND> * 256);
+    float *slot = b.slots + static_cast<int64_t>(blockIdx.x) * (kSets * kTiles<ND> * 256);
 #pragma unroll
-    for (int kind = 0; kind < kKinds; ++kind) {
+    for (int kind = 0; kind < kSets; ++kind) {
 #pragma unroll
         for (int i = 0; i < kOwn; ++i) {
             const int tile = i * kStripWaves + wave;
@@ -627,26 +772,28 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
 }
 
 // The workgroups' table gradients, added up in the workgroups' order: a thread per word of a head's slot.
-template <int ND>
+template <int ND, int C>
 __global__ __launch_bounds__(256) void strip_finish_kernel(StripArgs by_query, StripArgs by_key, int groups)
 {
     const AttnArgs &a = by_query.f;
-    constexpr int kWords = kTiles<ND> * 256;
-    const int HD = a.H * D, t = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
-    const int word = t % kWords, kind = t / kWords % 3, h = t / kWords / 3;          // dTq, dTv, dTk
+    constexpr int kWords = kTiles<ND> * 256, kSets = C == 8 ? 1 : 2;
+    const int HD = a.H * C, t = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+    const int word = t % kWords, set = t / kWords % (kSets + 1), h = t / kWords / (kSets + 1);       // by query, then by key
     if (h >= a.H) return;
     const int e = word % 4, lane = word / 4 % 64, tile = word / 256;
     const int axis = tile_axis(tile), r = tile_row0(tile) + 4 * (lane / 16) + e;
     if (axis >= ND || r >= axis_rows<ND>(a, axis)) return;
-    const int strips = by_query.list.total[1], kinds = kind < 2 ? 2 : 1;
+    const int kind = set == kSets ? 2 : C == 8 ? lane % 16 / C : set;                              // dTq, dTv, dTk
+    if (kind == 2 && lane % 16 >= C) return;
+    const int strips = by_query.list.total[1], sets = set < kSets ? kSets : 1;
     const int used = min(groups, strips);
-    const float *from = (kind < 2 ? by_query.slots + kind * kWords : by_key.slots) + static_cast<int64_t>(h) * (kinds * kWords) + word;
-    const int64_t step = static_cast<int64_t>(a.H) * (kinds * kWords);
+    const float *from = (set < kSets ? by_query.slots + set * kWords : by_key.slots) + static_cast<int64_t>(h) * (sets * kWords) + word;
+    const int64_t step = static_cast<int64_t>(a.H) * (sets * kWords);
     // (in 64 bits: a strip at a time, the parts have been rounded four times as often as by tiles of 64)
     double sum = 0.0;
 #pragma unroll 8
     for (int g = 0; g < used; ++g) sum += from[g * step];
-    (kind == 0 ? by_query.dtq : kind == 1 ? by_query.dtv : by_query.dtk)[static_cast<int64_t>(axis_base<ND>(a, axis) + r) * HD + h * D + lane % 16] = static_cast<float>(sum);
+    (kind == 0 ? by_query.dtq : kind == 1 ? by_query.dtv : by_query.dtk)[static_cast<int64_t>(axis_base<ND>(a, axis) + r) * HD + h * C + lane % C] = static_cast<float>(sum);
 }
 
 // workgroups per head: two per CU
@@ -655,12 +802,12 @@ int strip_groups(int H)
     const int most = 2 * device_cus();
     return most >= H ? most / H : 1;
 }
-size_t slot_bytes(int H, int nd, bool by_key)
+size_t slot_bytes(int H, int nd, int sets)
 {
-    return align_up(sizeof(float) * 256 * static_cast<size_t>(strip_groups(H)) * H * tiles_of_axes(nd) * (by_key ? 1 : 2), 256);
+    return align_up(sizeof(float) * 256 * static_cast<size_t>(strip_groups(H)) * H * tiles_of_axes(nd) * sets, 256);
 }
 
-template <typename T, typename TF, int ND>
+template <typename T, typename TF, int ND, int C>
 int launch_strips(const StripArgs &b0, hipStream_t stream)
 {
     StripArgs b = b0;
@@ -668,32 +815,144 @@ int launch_strips(const StripArgs &b0, hipStream_t stream)
         b.half_rows[n] = static_cast<float>(b.f.rows[n] / 2);
         b.upper[n] = std::nextafterf(static_cast<float>(b.f.rows[n]), 0.0f);
     }
+    constexpr int kSets = C == 8 ? 1 : 2;
     StripArgs by_key = b;
-    by_key.slots = b.slots + slot_bytes(b.f.H, ND, false) / sizeof(float);
+    by_key.slots = b.slots + slot_bytes(b.f.H, ND, kSets) / sizeof(float);
     const int H = b.f.H, groups = strip_groups(H);
-    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, false>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, b);
-    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, true>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, by_key);
-    const int64_t words = static_cast<int64_t>(3) * kTiles<ND> * 256 * H;
-    hipLaunchKernelGGL(strip_finish_kernel<ND>, dim3(static_cast<unsigned>(ceil_div(words, 256))), dim3(256), 0, stream, b, by_key, groups);
+    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, false, C>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, b);
+    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, true, C>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, by_key);
+    const int64_t words = static_cast<int64_t>(kSets + 1) * kTiles<ND> * 256 * H;
+    hipLaunchKernelGGL((strip_finish_kernel<ND, C>), dim3(static_cast<unsigned>(ceil_div(words, 256))), dim3(256), 0, stream, b, by_key, groups);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
 
+// ---- head_dim 8: what the strips need beside the records of the pair sweep --------------------------------------------
+struct StripSetup {
+    StripArgs b;
+    int64_t *pos_base;          // [N]: at a window's first sorted position, the pairs of the windows before it
+};
+
+// The strip list (workgroup 0) and, for fp32 tables beside fp16 features, the scale of a head's operands of Tq and Tk.
+template <bool kScales>
+__global__ __launch_bounds__(kListThreads) void strip_setup_kernel(StripArgs b)
+{
+    const AttnArgs &a = b.f;
+    if (blockIdx.x == 0) {
+        build_list(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(b.list.total), nullptr,
+                   const_cast<int2 *>(b.list.entries), const_cast<int4 *>(b.list.strips));
+        return;
+    }
+    const int job = static_cast<int>(blockIdx.x) - 1, kind = job % 2, h = job / 2;
+    float scale = 1.0f;
+    if constexpr (kScales) {
+        const float *table = static_cast<const float *>(kind == 0 ? a.table_q : a.table_k) + h * a.D;
+        __shared__ int top_s;
+        if (threadIdx.x == 0) top_s = 0;
+        __syncthreads();
+        float top = 0.0f;
+        for (int t = threadIdx.x; t < a.total_rows * a.D; t += kListThreads) {
+            const float x = table[static_cast<int64_t>(t / a.D) * (a.H * a.D) + t % a.D];
+            top = fmaxf(top, finite(x) ? fabsf(x) : 0.0f);
+        }
+        atomicMax(&top_s, __float_as_int(top));
+        __syncthreads();
+        scale = power2(min(100, 14 - exponent_of(__int_as_float(top_s))));
+    }
+    if (threadIdx.x == 0) const_cast<float *>(b.scales)[h * 3 + kind] = 1.0f / scale;
+}
+
+__global__ __launch_bounds__(256) void strip_columns_kernel(StripSetup s)
+{
+    const StripArgs &b = s.b;
+    const int t = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x), u = t / kStrip, c = t % kStrip;
+    if (u >= b.list.total[1]) return;
+    const int4 strip = b.list.strips[u];
+    const int col = strip.z + min(c, strip.w - 1), n = strip.y;
+    const int2 entry = b.list.entries[strip.x + col / n];
+    const int pos = entry.x + col % n, row = b.f.n2n ? b.f.n2n[pos] : pos;
+    const bool fits = static_cast<int64_t>(entry.y) + static_cast<int64_t>(n) * n <= b.pairs;
+    const_cast<int4 *>(b.columns)[t] = make_int4(pos, row, entry.x, fits ? entry.y : -1);
+    const_cast<int32_t *>(b.column_rows)[t] = row;
+    if (pos == entry.x) s.pos_base[pos] = entry.y;
+}
+
 }  // namespace
 
-size_t strip_slots_bytes(int H, int nd) { return slot_bytes(H, nd, false) + slot_bytes(H, nd, true); }
+size_t strip_slots_bytes(int H, int nd) { return slot_bytes(H, nd, 2) + slot_bytes(H, nd, 1); }
 
 int launch_strip_gradients(const StripArgs &b, int dtype, hipStream_t stream)
 {
-#define S3D_CASE(NN)                                                                                           \
-    if (b.f.nd == NN)                                                                                          \
-        return dtype == S3D_DTYPE_F32   ? launch_strips<float, float, NN>(b, stream)                           \
-               : dtype == S3D_DTYPE_F16 ? launch_strips<__half, __half, NN>(b, stream)                         \
-                                        : launch_strips<float, __half, NN>(b, stream);
-    S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
+#define S3D_CASE(NN, CC)                                                                                       \
+    if (b.f.nd == NN && b.f.D == CC)                                                                           \
+        return dtype == S3D_DTYPE_F32   ? launch_strips<float, float, NN, CC>(b, stream)                       \
+               : dtype == S3D_DTYPE_F16 ? launch_strips<__half, __half, NN, CC>(b, stream)                     \
+                                        : launch_strips<float, __half, NN, CC>(b, stream);
+    S3D_CASE(3, 16) S3D_CASE(6, 16) S3D_CASE(9, 16)
+    S3D_CASE(3, 8) S3D_CASE(6, 8) S3D_CASE(9, 8)
 #undef S3D_CASE
     return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: %d axes in the strip form", b.f.nd);
 }
 
 }  // namespace tile
+
+// Where the strips serve a backward at head_dim 8; elsewhere the pair sweeps with the table-gradient kernels, whose cost follows
+// the pairs and table rows where a strip's follows its voxels.  Strips over those, forward left out:
+//   fp16 features, 9 axes: 0.60 to 0.89 (windows of 2 to 60 voxels, 60,000 to 250,000 voxels of 6 heads), 6 axes 0.61 to 0.94;
+//     3 axes 0.61 to 0.98 at 60,000, 1.07 at 250,000 in windows of 26
+//   fp32 (three parts a number, twice the products): windows of 60 0.71 to 0.75; of 26, on scans with 6 axes, forward included,
+//     0.83 at 20,000 voxels, 0.91 at 40,000, 0.98 at 60,000, 1.01 to 1.05 beyond, with 9 axes 0.77 at 20,000, 0.95 to 0.99 at
+//     360,000 to 2,000,000 (voxel, head); with random signals, whose histograms have no empty rows, 1.02 to 1.08 at 360,000 and
+//     1.13 to 1.23 at 1,500,000
+constexpr int64_t kStripMeanWindow = 40, kStripVoxelHeads = 600000, kStripVoxelHeadsFloat = 250000;
+
+bool attn_strip8_applies(const int32_t *rows, int nd, int D, int dtype, int64_t N, int64_t W, int H, int64_t pairs, size_t room)
+{
+    if (D != 8 || pairs <= 0 || pairs >= (int64_t(1) << 31) || !rows_fit_tiles(rows, nd) || attn_strip8_bytes(H, nd, N, W) > room) return false;
+    if (N >= kStripMeanWindow * W) return true;
+    return dtype == S3D_DTYPE_F32 ? N * H <= kStripVoxelHeadsFloat : nd > 3 || N * H <= kStripVoxelHeads;
+}
+
+// slots | list | strips | columns | their rows (64 more) | scales
+size_t attn_strip8_bytes(int H, int nd, int64_t N, int64_t W)
+{
+    return tile::slot_bytes(H, nd, 1) * 2 + tile::list_bytes(N, W) + tile::strips_bytes(N) + tile::strip_columns_bytes(N) +
+           align_up(sizeof(float) * 3 * static_cast<size_t>(H), 256);
+}
+
+int launch_attn_strip8(const BwdPairArgs &p, float *dtq, float *dtk, float *dtv, void *room, int dtype, hipStream_t stream)
+{
+    using namespace tile;
+    const AttnArgs &a = p.f;
+    StripSetup s{};
+    StripArgs &g = s.b;
+    g.f = a;
+    char *at = static_cast<char *>(room);
+    g.slots = reinterpret_cast<float *>(at);
+    at += slot_bytes(a.H, a.nd, 1) * 2;
+    g.list = list_at(at, a.N, a.W);
+    at += list_bytes(a.N, a.W);
+    g.list.strips = reinterpret_cast<const int4 *>(at);
+    at += strips_bytes(a.N);
+    g.columns = reinterpret_cast<const int4 *>(at);
+    g.column_rows = reinterpret_cast<const int32_t *>(g.columns + kStrip * list_max_strips(a.N));
+    at += strip_columns_bytes(a.N);
+    g.scales = reinterpret_cast<const float *>(at);
+    g.dout = p.dout;
+    g.records = p.pd;
+    g.pairs = p.pairs;
+    g.dq = p.dq; g.dk = p.dk; g.dv = p.dv;
+    g.grad_stride = static_cast<uint32_t>(p.grad_stride);
+    g.dtq = dtq; g.dtk = dtk; g.dtv = dtv;
+    s.pos_base = const_cast<int64_t *>(p.pos_base);
+    const dim3 jobs(static_cast<unsigned>(1 + 2 * a.H));
+    if (dtype == S3D_DTYPE_F32_F16_ROWS) hipLaunchKernelGGL(strip_setup_kernel<true>, jobs, dim3(kListThreads), 0, stream, g);
+    else hipLaunchKernelGGL(strip_setup_kernel<false>, jobs, dim3(kListThreads), 0, stream, g);
+    const int64_t columns = static_cast<int64_t>(list_max_strips(a.N)) * kStrip;
+    hipLaunchKernelGGL(strip_columns_kernel, dim3(static_cast<unsigned>(ceil_div(columns, 256))), dim3(256), 0, stream, s);
+    S3D_HIP_CHECK(hipGetLastError());
+    if (int rc = launch_attn_bwd_records(p, dtype, stream)) return rc;
+    return launch_strip_gradients(g, dtype, stream);
+}
+
 }  // namespace s3d

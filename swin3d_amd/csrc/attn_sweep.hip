@@ -735,6 +735,8 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
 // 6 heads of 8, 9 axes, fp16: 338 + 269 us.  When the key-owned sweep made dL and P again (125 of its 280 instructions a pair)
 // and left them in a second order for the table gradients, 326 + 374, with a store of 12 bytes a (pair, head) for 8.
 template <typename T, int D, int HP> __host__ __device__ constexpr int bwd_pair_threads() { return 256; }
+// wavefronts per SIMD of the sweep that leaves records only
+template <typename T, int HP> __host__ __device__ constexpr int record_waves() { return sizeof(T) == 2 ? (HP == 1 ? 4 : 3) : (HP == 1 ? 3 : 2); }
 // elements between rows of Tk in the key-owned sweep's LDS (padded as the other's)
 template <typename T, int D, int HP> __host__ __device__ constexpr int key_row_stride()
 {
@@ -745,7 +747,7 @@ template <typename T, int D, int HP> __host__ __device__ constexpr int key_row_s
 // tables and of the arithmetic.  TF = __half with T = float serves an fp16 forward whose backward runs in fp32: the
 // rows are widened as they are loaded and the gradients rounded as they are stored, the arithmetic is that of T = TF
 // = float on widened copies.
-template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned>
+template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned, bool kOnlyRecords = false>
 // Wavefronts per SIMD, by register cap: fp16 four at head_dim 8, three at 16; fp32 three and two.  The key-owned sweep stays
 // below all of them (113 to 167 registers); of the query-owned one nine axes spill 9 (fp16, 16), 1 (fp32, 8), 21 and, beside
 // fp16 rows, 13 (fp32, 16).  us of the query-owned and the key-owned sweep with one wavefront more, as it is, one less:
@@ -755,7 +757,7 @@ template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned>
 //     953 + 587; fp32 14266 + 1066, 3564 + 1038, 2526 + 1014; beside fp16 rows 12006 + 738, 2864 + 715, 2538 + 714
 // (in the last two LDS holds one workgroup a CU, with tables of 432 rows; it holds two below 394, with six axes too, which spill
 // nothing).
-__global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (D == 8 ? 4 : 3) : (D == 8 ? 3 : 2))) void attn_bwd_pairs_kernel(BwdPairArgs b)
+__global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? record_waves<T, HP>() : sizeof(T) == 2 ? (D == 8 ? 4 : 3) : (D == 8 ? 3 : 2))) void attn_bwd_pairs_kernel(BwdPairArgs b)
 {
     const AttnArgs &a = b.f;
     constexpr int kThreads = bwd_pair_threads<T, D, HP>();
@@ -854,7 +856,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
         const bool fits = pair_base + static_cast<int64_t>(n_w) * n_w <= b.pairs;
 
         Slice<T, D> own_x[HP], own_y[HP];     // q_i, dout_i
-        float own_m[HP], own_inv[HP], own_delta[HP];
+        float own_m[HP], own_inv[HP], own_delta[HP], own_bad[HP];
         float ci[ND], res_x[HP][D], res_y[kKeyOwned ? HP : 1][D];
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
@@ -864,7 +866,20 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
                 own_y[hh].load(ggo + static_cast<int64_t>(own_row) * HD + (h + hh) * D);
                 own_m[hh] = b.stat_max[static_cast<int64_t>(own_row) * H + h + hh];
                 own_inv[hh] = 1.0f / b.stat_sum[static_cast<int64_t>(own_row) * H + h + hh];
-                own_delta[hh] = b.delta[static_cast<int64_t>(own_row) * H + h + hh];
+                if constexpr (!kOnlyRecords) {
+                    own_delta[hh] = b.delta[static_cast<int64_t>(own_row) * H + h + hh];
+                } else {
+                    float x[D], y[D];
+                    const int64_t at_out = static_cast<int64_t>(own_row) * HD + (h + hh) * D;
+                    load_row<D>(ggo + at_out, x);
+                    load_row<D>(static_cast<const TF *>(b.out) + at_out, y);
+                    own_delta[hh] = own_bad[hh] = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < D; ++c) {
+                        own_delta[hh] += x[c] * y[c];
+                        own_bad[hh] = fabsf(x[c]) < INFINITY ? own_bad[hh] : __int_as_float(0x7fc00000);
+                    }
+                }
             }
 #pragma unroll
             for (int c = 0; c < D; ++c) res_x[hh][c] = 0.0f;
@@ -978,8 +993,18 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
                         if (Slice<T, D>::kChainLogit) dp = own_y[hh].dot(tv_r, dp);
                         else dp += own_y[hh].dot(tv_r, 0.0f);
                     }
-                    if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
-                    else vec_sum[n / kGroup].add(vec_r);
+                    if constexpr (!kOnlyRecords) {
+                        if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
+                        else vec_sum[n / kGroup].add(vec_r);
+                    }
+                }
+                if constexpr (kOnlyRecords) {
+                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq; a query
+                    // whose dout is not finite has no weights: the products that follow take its dout as zeros)
+                    const float p = __expf(logit - own_m[hh]) * own_inv[hh];
+                    const float dl = fabsf(logit) < INFINITY ? p * (dp - own_delta[hh]) : __int_as_float(0x7fc00000);
+                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p + own_bad[hh]);
+                    continue;
                 }
                 float p, dl;
                 if constexpr (kKeyOwned) {
@@ -999,6 +1024,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (sizeof(T) == 2 ? (
                 }
             }
         }
+        if constexpr (kOnlyRecords) continue;
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
             // lanes that share an owned voxel saw alternate elements of the stream
@@ -1182,6 +1208,46 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
     return S3D_OK;
 }
 
+template <typename T, typename TF, int ND, int HP>
+int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
+{
+    constexpr int D = 8;
+    const AttnArgs &a = b0.f;
+    const size_t lds = align_up(sizeof(T) * static_cast<size_t>(a.total_rows) * table_row_stride_heads<T, D, HP>(), 16);
+    auto kernel = attn_bwd_pairs_kernel<T, TF, D, ND, HP, false, true>;
+    constexpr int kThreads = bwd_pair_threads<T, D, HP>();
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
+    int per_cu = 0;
+    S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kernel), kThreads, lds));
+    if (per_cu < 1) per_cu = 1;
+    const int groups = a.H / HP, slots = per_cu * device_cus(), set = kQueues * groups, whole = (slots / set) * set;
+    BwdPairArgs b = b0;
+    b.f.spread_groups = 10 * whole < 9 * slots;
+    const int grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
+    b.f.target_items = grid / groups * (kThreads / 64);
+    b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
+    const int64_t list_want = (a.W + kListThreads - 1) / kListThreads;
+    const dim3 list_grid(static_cast<unsigned>(list_want < 1 ? 1 : (list_want > kListGroups ? kListGroups : list_want)));
+    hipLaunchKernelGGL(sweep_count_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
+    hipLaunchKernelGGL(sweep_place_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+// Records alone, for the strips of attn_strip_bwd.hip (head_dim 8).  Bound by VALU issue, 65 % of the time, 322 instructions a
+// step of two heads.  199,327 voxels in windows of 26, 6 heads, 9 axes: fp16 288 us with pairs of heads, 378 with three heads
+// (38 registers spilled), 347 the query-owned sweep with its dq.  fp32 with 9 axes: 463 with one head, 489 with two (two
+// wavefronts a SIMD); with 6 axes 372 and 339.
+template <typename T, typename TF, int ND>
+int dispatch_bwd_records(const BwdPairArgs &b, hipStream_t stream)
+{
+    if constexpr (sizeof(TF) == 2 || ND < 9) {
+        if (b.f.H % 2 == 0) return launch_bwd_records<T, TF, ND, 2>(b, stream);
+    }
+    return launch_bwd_records<T, TF, ND, 1>(b, stream);
+}
+
 template <typename T, typename TF>
 int dispatch_bwd_pairs(const BwdPairArgs &b, hipStream_t stream)
 {
@@ -1203,6 +1269,18 @@ int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream)
     case S3D_DTYPE_F32_F16_ROWS: return dispatch_bwd_pairs<float, __half>(b, stream);
     default: return fail(S3D_ERR_BAD_DTYPE, "s3d_attn_bwd: dtype %d (0 = fp32, 1 = fp16, 2 = fp32 on fp16 rows)", dtype);
     }
+}
+
+int launch_attn_bwd_records(const BwdPairArgs &b, int dtype, hipStream_t stream)
+{
+#define S3D_CASE(NN)                                                                                       \
+    if (b.f.D == 8 && b.f.nd == NN)                                                                        \
+        return dtype == S3D_DTYPE_F32   ? dispatch_bwd_records<float, float, NN>(b, stream)                \
+               : dtype == S3D_DTYPE_F16 ? dispatch_bwd_records<__half, __half, NN>(b, stream)              \
+                                        : dispatch_bwd_records<float, __half, NN>(b, stream);
+    S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
+#undef S3D_CASE
+    return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: head_dim %d, %d axes in the records sweep", b.f.D, b.f.nd);
 }
 
 size_t attn_sweep_workspace_bytes(int H, int64_t W, int64_t N)

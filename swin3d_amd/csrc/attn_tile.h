@@ -79,6 +79,8 @@ inline size_t list_bytes(int64_t N, int64_t W)
 // a strip is full, but for the last one of each window size up to 64 and of each larger window
 inline size_t list_max_strips(int64_t N) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(N > 0 ? N : 0) / (kCols + 1) + kCols + 1; }
 inline size_t strips_bytes(int64_t N) { return list_round(sizeof(int4) * list_max_strips(N)); }
+// a strip's voxels: see StripArgs
+inline size_t strip_columns_bytes(int64_t N) { return align_up(kStrip * list_max_strips(N) * (sizeof(int4) + sizeof(int32_t)) + 256, 256); }
 inline UnitList list_at(void *p, int64_t N, int64_t W)
 {
     char *base = static_cast<char *>(p);
@@ -107,7 +109,8 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
 {
     __shared__ int windows[kListBins], big_units[kListBins], entry_at[kListBins], unit_at[kListBins], entry_first[kListBins];
     constexpr int kWavesOfList = kListThreads / 64;
-    __shared__ int wave_pairs[kWavesOfList], of_wave[kWavesOfList][kListBins];
+    __shared__ long long wave_pairs[kWavesOfList];
+    __shared__ int of_wave[kWavesOfList][kListBins];
     __shared__ int big_strips[kListBins], strip_at[kListBins], strips_of_wave[kWavesOfList][kBigBins];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (t < kListBins) windows[t] = big_units[t] = big_strips[t] = 0;
@@ -152,14 +155,14 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
         }
     }
     __syncthreads();
-    int before = 0;                    // pairs of the windows that earlier rounds placed
+    long long before = 0;              // pairs of the windows that earlier rounds placed
     for (int w0 = 0; w0 < W; w0 += kListThreads) {
         const int w = w0 + t;
         const int n = w < W ? w_sizes[w] : 0;
-        int incl = n > 0 ? n * n : 0;
-        const int own = incl;
+        long long incl = n > 0 ? static_cast<long long>(n) * n : 0;
+        const long long own = incl;
         for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off);
+            const long long up = __shfl_up(incl, off);
             if (lane >= off) incl += up;
         }
         if (lane == 63) wave_pairs[wave] = incl;
@@ -185,7 +188,7 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
             }
             left &= ~same;
         }
-        int pairs = before + incl - own, all = 0;
+        long long pairs = before + incl - own, all = 0;
 #pragma unroll
         for (int v = 0; v < kWavesOfList; ++v) {
             pairs += v < wave ? wave_pairs[v] : 0;
@@ -217,19 +220,21 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
         __syncthreads();
         if (b >= 0) {
             const int e = of_wave[wave][b] + rank, in_bin = e - entry_first[b];
-            entries[e] = make_int2(w2n[w], pairs);
+            // (a window that begins beyond 2^31 pairs does not fit any store of this form)
+            entries[e] = make_int2(w2n[w], static_cast<int>(pairs < 0x7fffffffll ? pairs : 0x7fffffffll));
             if (n > kCols) {
                 const int tiles = tiles_of(n);
                 // (the windows of the first bin differ in their tiles)
                 const int u = b > 0 ? unit_at[b] + in_bin * tiles : atomicAdd(&unit_at[b], tiles);
-                for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
+                if (units)
+                    for (int q = 0; q < tiles; ++q) units[u + q] = make_int4(e, n, q, tiles);
                 if (strips) {
                     const int count = strips_of(n), first = b > 0 ? strips_of_wave[wave][b] + strips_before : atomicAdd(&strip_at[b], count);
                     for (int q = 0; q < count; ++q) strips[first + q] = make_int4(e, n, q * kStrip, min(kStrip, n - q * kStrip));
                 }
             } else {
                 const int per = kCols / n;
-                if (in_bin % per == 0) units[unit_at[b] + in_bin / per] = make_int4(e, n, min(per, windows[b] - in_bin), 0);
+                if (units && in_bin % per == 0) units[unit_at[b] + in_bin / per] = make_int4(e, n, min(per, windows[b] - in_bin), 0);
                 if (strips) {
                     // the strips whose first column is this window's
                     const int begin = in_bin * n, end = begin + n, columns = windows[b] * n;

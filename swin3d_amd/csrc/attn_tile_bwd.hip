@@ -330,8 +330,6 @@ int launch_records(const BwdTileArgs &b0, hipStream_t stream)
 // row, first pair and coordinates of the units' columns
 size_t columns_bytes(int64_t N, int nd) { return align_up(sizeof(int32_t) * list_max_units(N) * kCols * (2 + static_cast<size_t>(nd)), 256); }
 
-size_t strip_columns_bytes(int64_t N) { return align_up(kStrip * list_max_strips(N) * (sizeof(int4) + sizeof(int32_t)) + 256, 256); }
-
 // tables as operands, at most 48 bytes a lane, and their scales
 size_t operand_bytes(int H, int nd)
 {

@@ -73,7 +73,7 @@ def test_forward_weights_keep_their_bits(oracle_lib, hip_lib, dtype, ws, fill):
     assert (np.abs(got - want[:, None, None]) <= bound[:, None, None])[some].all()
 
 
-def _windows_case(oracle_lib, sizes, cRSE, heads, seed, ws=7):
+def _windows_case(oracle_lib, sizes, cRSE, heads, seed, ws=7, dim=16):
     """Windows of the given numbers of voxels, in rows of a random order."""
     from conftest import random_scene
     from helpers import AttnCase, n_coords_from_scene
@@ -88,9 +88,9 @@ def _windows_case(oracle_lib, sizes, cRSE, heads, seed, ws=7):
     sig = rng.uniform(-1, 1, (n, crse.crse_num_axes(cRSE) - 3)).astype(np.float32)
     index, n_coords = n_coords_from_scene(oracle_lib, coords, frac, sig, 1, ws, 4, cRSE)
     assert sorted(index["w_sizes"]) == sorted(sizes)
-    table_sizes = crse.crse_table_sizes(ws, 4, heads, 16, cRSE)
-    q, k, v, tables = synth.layer_inputs(n, heads * 16, heads, int(sum(table_sizes)), seed=seed, recipe="sharp")
-    return AttnCase(coords, 1, ws, 4, heads, 16, cRSE, index, n_coords, q, k, 0.4 * v, (0.3 * tables[0], 0.3 * tables[1], 0.2 * tables[2]),
+    table_sizes = crse.crse_table_sizes(ws, 4, heads, dim, cRSE)
+    q, k, v, tables = synth.layer_inputs(n, heads * dim, heads, int(sum(table_sizes)), seed=seed, recipe="sharp")
+    return AttnCase(coords, 1, ws, 4, heads, dim, cRSE, index, n_coords, q, k, 0.4 * v, (0.3 * tables[0], 0.3 * tables[1], 0.2 * tables[2]),
                     table_sizes)
 
 
