@@ -95,8 +95,8 @@ const char *s3d_last_error_string(void);
  *                  and / or S3D_ATTN_SIZES_ON_DEVICE (see table_sizes)
  *   workspace      device scratch of at least s3d_attn_fwd_workspace_bytes(H, N, W) bytes: the work list of the
  *                  launch (work-queue counters, one record per unit of 8 to 64 queries and one per window, the
- *                  list builder's notes), about 2 N + 24 W bytes + 0.3 MB whatever the window sizes, and where a call
- *                  of this shape may run on tiles their unit list, about N / 2 + 8 W bytes
+ *                  list builder's notes, which give way to the strip list), about 2 N + 24 W bytes + 0.3 MB whatever
+ *                  the window sizes, and where a call of this shape may run on tiles their unit list, about N / 2 + 8 W bytes
  *   w2n must be ascending (the exclusive prefix sum of w_sizes, as the reference builds it:
  *   Swin3D/modules/swin3d_layers.py:100-103).
  *   D in {8,16,32}, nd in {3,6,9}, H >= 1 (the reference takes head_dim up to 32: self_attn_aio_fwd.cu:486).
@@ -111,12 +111,12 @@ const char *s3d_last_error_string(void);
  * fp16: inputs, tables and output are fp16; products accumulate in fp32, exp in fp32.  Every call gives the same bits
  * for the same inputs (no atomics on data but integer ones, work list in window order).
  *
- * Two kernels.  The sweep serves every shape: persistent workgroups that keep their heads' table slices in LDS, a lane
+ * Three kernels.  The sweep serves every shape: persistent workgroups that keep their heads' table slices in LDS, a lane
  * per query streaming its window's keys (VALU; packed fp16 dot products for fp16 I/O; there the value-table rows of a
  * pair are added three at a time in fp16 before they enter the fp32 sums - the reference's half path adds all of them
  * and the value in half2, Swin3D/src/attn/self_attn_aio_fwd.cu:147).  At head_dim 16 in launches that do not fill the
- * chip, mean window of at least 40 voxels, without out_max and out_sum, it is the tile kernel: 64 queries by 64 keys of a
- * head, the tables on the matrix pipe, no sum in fp16.  A NaN or an infinity in q, k, v or a table reaches the queries of
+ * chip, without out_max and out_sum, it is a kernel with the tables on the matrix pipe and no sum in fp16: in fp16 on strips
+ * of 16 queries, in fp32, with a mean window of at least 40 voxels, on tiles of 64 queries by 64 keys.  A NaN or an infinity in q, k, v or a table reaches the queries of
  * its own window, or of the pairs that use the table row, and no others.
  */
 #define S3D_ATTN_PLANNED 4   /* `workspace` holds a plan written by s3d_attn_plan: see there */
@@ -138,7 +138,7 @@ int s3d_attn_fwd(const void *q, const void *k, const void *v, const void *table_
  * units of 64 lanes.  s3d_attn_fwd builds it on every call (two small kernels); a caller that keeps a window set
  * for several calls builds it once with s3d_attn_plan and passes the plan buffer as `workspace` together with
  * the flag S3D_ATTN_PLANNED, for calls with the same w_sizes, w2n, N, W, H, D, dtype and table_sizes.  Such a call
- * runs the sweep kernel or the tile kernel and nothing else (with table sizes on the device both are launched, and one
+ * runs the sweep, strip or tile kernel and nothing else (with table sizes on the device the sweep and the other, and one
  * of them returns); the plan has both lists where the shape may use either.  It holds the sweep's work counters, which a
  * launch leaves at zero again: a plan serves one call at a time (calls in stream order; not two streams at once).
  *   plan           device buffer of at least s3d_attn_plan_bytes(H, N, W) bytes (= s3d_attn_fwd_workspace_bytes)

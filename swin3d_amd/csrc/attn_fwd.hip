@@ -59,8 +59,9 @@ int launch_fwd(const AttnArgs &a, int dtype, hipStream_t stream, int what)
     // A call that leaves softmax statistics is a training step's, and stays on the sweep: the two kernels differ by fp16
     // roundings of the features (2.7e-4, neither further from exact), and on scans of 20,000 voxels that gives another
     // sample of the 2 to 5 % by which fp16 activations move the gradients of an encoder (2 % between the two).
-    if (a.out_max || a.out_sum || !attn_tile_applies(a, dtype)) return launch_attn_sweep(a, dtype, stream, what);
-    if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), stream, what)) return rc;
+    const bool strips = attn_strip_applies(a, dtype);
+    if (a.out_max || a.out_sum || !(strips || attn_tile_applies(a, dtype))) return launch_attn_sweep(a, dtype, stream, what);
+    if (int rc = strips ? launch_attn_strip(a, stream, what) : launch_attn_tile(a, tile_list_of(a), stream, what)) return rc;
     if (!a.sizes_dev) return S3D_OK;
     AttnArgs b = a;
     b.leave_to_tiles = 1;
@@ -228,10 +229,12 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_plan(
     a.w2n = w2n;
     a.workspace = plan;
     // both lists where the shape may use either: the plan's caller may keep the table sizes on the device
-    if (D == 16 && attn_tile_shape(N, W, H, nd, dtype == S3D_DTYPE_F32)) {
-        if (int rc = launch_attn_tile(a, dtype, tile_list_of(a), static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
+    if (D == 16 && dtype == S3D_DTYPE_F32 && attn_tile_shape(N, W, H, nd)) {
+        if (int rc = launch_attn_tile(a, tile_list_of(a), static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
     }
-    return launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream), kAttnBuildList);
+    if (int rc = launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
+    if (D == 16 && dtype == S3D_DTYPE_F16 && attn_strip_shape(N, W, H)) return launch_attn_strip(a, static_cast<hipStream_t>(stream), kAttnBuildList);
+    return S3D_OK;
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_attn_fwd_noalloc(

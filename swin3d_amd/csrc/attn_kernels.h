@@ -20,7 +20,7 @@ struct AttnArgs {
     void *workspace;                       // the work list: queue counters, unit and window records
     int32_t block_shift;                   // the step target, a lane streams about 2^block_shift keys
     int32_t target_items;                  // wavefronts that serve one head group (sizes the finer units at the list's end)
-    int32_t leave_to_tiles;                // sizes_dev: the tile kernel was launched too and serves sizes that fit it
+    int32_t leave_to_tiles;                // sizes_dev: the tile or strip kernel was launched too and serves sizes that fit it
     int32_t spread_groups;                 // head groups take the workgroups in turn (else in runs of eight)
     int32_t H, D, nd, total_rows;
     int64_t N, W;
@@ -28,7 +28,7 @@ struct AttnArgs {
     int32_t base[kMaxAxes];                // first row of each axis table in the flat table
 };
 
-// Table rows of an axis that the tile kernel takes: of a position axis, of a colour or normal axis.
+// Table rows of an axis that the tile and strip kernels take: of a position axis, of a colour or normal axis.
 constexpr int kTileRows = 64, kTileSignalRows = 32;
 template <typename Rows> __host__ __device__ inline bool rows_fit_tiles(const Rows &rows, int nd)
 {
@@ -50,19 +50,29 @@ __device__ __forceinline__ int device_rows(const AttnArgs &a, int n, int nd, int
 // which streams that window's keys; VALU math (packed fp16 dot products for fp16 I/O), any dtype, windows of any
 // size.  Needs a.workspace (work queues, sorted window list, unit list).
 size_t attn_sweep_workspace_bytes(int H, int64_t W, int64_t N);
+// The part of it that holds notes of the list builder, and its size.
+constexpr size_t kSweepNotesBytes = size_t(320) << 10;
+void *attn_sweep_notes(const AttnArgs &a);
 // what: kAttnBuildList (the two list kernels: needs w_sizes, w2n and the shape only), kAttnSweep (the sweep on a
 // work list that is already in a.workspace; the launch leaves it ready for the next one), or both.
 constexpr int kAttnBuildList = 1, kAttnSweep = 2;
 int launch_attn_sweep(const AttnArgs &a, int dtype, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
 
-// The tile kernel (attn_tile.hip): a workgroup works off tiles of up to 64 queries by 64 keys of a head, the table
+// The tile kernel (attn_tile.hip), fp32: a workgroup works off tiles of up to 64 queries by 64 keys of a head, the table
 // products on the matrix pipe.  `list` is its unit list, attn_tile_list_bytes of device memory.
 // With sizes_dev the host cannot tell whether every axis fits: it launches the tile kernel and the sweep kernel, and each
 // works or returns by what it reads.
-bool attn_tile_shape(int64_t N, int64_t W, int H, int nd, bool fp32);
+bool attn_tile_shape(int64_t N, int64_t W, int H, int nd);
 bool attn_tile_applies(const AttnArgs &a, int dtype);
 size_t attn_tile_list_bytes(int H, int64_t N, int64_t W);
-int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
+int launch_attn_tile(const AttnArgs &a, void *list, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
+
+// The strip kernel (attn_strip_fwd.hip), fp16: a workgroup works off strips of up to 16 queries of a window and a head, the
+// table products on the matrix pipe.  Its strip list lies where the sweep's list builder has its notes, which nothing reads once
+// that list is there: a plan with both builds the sweep's first.  With sizes_dev as above.
+bool attn_strip_shape(int64_t N, int64_t W, int H);
+bool attn_strip_applies(const AttnArgs &a, int dtype);
+int launch_attn_strip(const AttnArgs &a, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);
 
 // host side: a kernel's dynamic-LDS limit (see there), compute units of the current device
 int allow_dynamic_lds(const void *kernel, size_t bytes);

@@ -1,5 +1,5 @@
-// Interface between the backward's records kernel (attn_tile_bwd.hip) and the kernels that sum over pairs
-// (attn_strip_bwd.hip).
+// Pieces shared by the kernels on strips of 16 voxels (attn_strip_fwd.hip, attn_strip_bwd.hip), and the interface between the
+// backward's records kernel (attn_tile_bwd.hip) and the kernels that sum over pairs.
 #pragma once
 
 #include "attn_tile.h"
@@ -21,6 +21,211 @@ template <int ND> __device__ __forceinline__ int axis_base(const AttnArgs &a, in
 #pragma unroll
     for (int n = 1; n < ND; ++n) r = axis == n ? a.base[n] : r;
     return r;
+}
+
+constexpr int kStripThreads = 512, kStripWaves = kStripThreads / 64;
+
+// 16-row tiles of the histograms: four to a position axis, two to a colour or normal axis, up to as many for each wavefront
+// (with a branch around the last one, six axes took 60 registers more)
+constexpr int tiles_of_axes(int nd) { return (12 + 2 * (nd - 3) + kStripWaves - 1) / kStripWaves * kStripWaves; }
+template <int ND> constexpr int kTiles = tiles_of_axes(ND);
+template <int ND> constexpr int kOwnTiles = kTiles<ND> / kStripWaves;
+__host__ __device__ constexpr int axis_row0(int axis) { return axis < 3 ? axis * 64 : 192 + (axis - 3) * 32; }
+__host__ __device__ constexpr int tile_axis(int tile) { return tile < 12 ? tile / 4 : 3 + (tile - 12) / 2; }
+__host__ __device__ constexpr int tile_row0(int tile) { return (tile < 12 ? tile % 4 : tile % 2) * 16; }
+
+// ---- matrix operands of 16 terms: lane % 16 is the row of A or the column of B, terms 4 (lane / 16) + 0..3 ----------------
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int32_t i32x4_1 __attribute__((ext_vector_type(4), aligned(4)));
+
+// numbers that are exact in the features' type
+template <typename TF> struct Exact4;
+// fp32 numbers: two fp16 numbers each beside fp16 features (of the numbers times a scale), three bf16 numbers beside fp32
+template <typename TF> struct Parts4;
+template <> struct Exact4<__half> {
+    f16x4 x;
+    __device__ __forceinline__ void set(const float *v)
+    {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = static_cast<_Float16>(v[e]);
+    }
+};
+__device__ __forceinline__ f16x4 to_half4(float a, float b, float c, float d)
+{
+    const f16x2 x = __builtin_convertvector(f32x2{a, b}, f16x2), y = __builtin_convertvector(f32x2{c, d}, f16x2);
+    return __builtin_shufflevector(x, y, 0, 1, 2, 3);
+}
+// two numbers times a power of two as fp16 numbers, and what that leaves of them likewise (v_fma_mixlo_f16 and its like, one
+// instruction a number in place of one and a half, take twice the time)
+__device__ __forceinline__ uint32_t scaled_half2(float x, float y, float scale)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x * scale, y * scale}), f16x2));
+}
+__device__ __forceinline__ uint32_t scaled_rest2(float x, float y, float scale, uint32_t h)
+{
+    const f16x2 t = __builtin_bit_cast(f16x2, h);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{__builtin_fmaf(x, scale, -static_cast<float>(t[0])),
+                                                                       __builtin_fmaf(y, scale, -static_cast<float>(t[1]))}), f16x2));
+}
+// a choice among the four numbers of an operand; of a number in both halves of a word
+struct OneOfFour {
+    u32x2 mask;
+    __device__ __forceinline__ explicit OneOfFour(int at)
+    {
+        const uint32_t half = (at & 1) ? 0xffff0000u : 0xffffu;
+        mask = {(at >> 1) == 0 ? half : 0u, (at >> 1) == 1 ? half : 0u};
+    }
+    __device__ __forceinline__ u32x2 of(uint32_t x) const { return {x & mask[0], x & mask[1]}; }
+};
+template <> struct Parts4<__half> {
+    f16x4 hi, lo;
+    template <bool kNearest = true> __device__ __forceinline__ void set(const float *v, float scale)
+    {
+        u32x2 h, l;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            h[e] = scaled_half2(v[2 * e], v[2 * e + 1], scale);
+            l[e] = scaled_rest2(v[2 * e], v[2 * e + 1], scale, h[e]);
+        }
+        hi = __builtin_bit_cast(f16x4, h);
+        lo = __builtin_bit_cast(f16x4, l);
+    }
+    // the number `at` (0..3) of the four, the others zero
+    __device__ __forceinline__ void set_one(float v, float scale, const OneOfFour &at)
+    {
+        const uint32_t h = scaled_half2(v, v, scale), l = scaled_rest2(v, v, scale, h);
+        hi = __builtin_bit_cast(f16x4, at.of(h));
+        lo = __builtin_bit_cast(f16x4, at.of(l));
+    }
+};
+template <> struct Parts4<float> {
+    s16x4 s[3];
+    template <bool kNearest = true> __device__ __forceinline__ void set(const float *v, float scale)
+    {
+        u32x2 out[3];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            f32x2 x = {v[2 * e] * scale, v[2 * e + 1] * scale};
+            if constexpr (kNearest) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    out[k][e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
+                    if (k < 2) x -= f32x2{__uint_as_float(out[k][e] << 16), __uint_as_float(out[k][e] & 0xffff0000u)};
+                }
+            } else {
+                uint32_t b[3][2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    b[0][u] = __float_as_uint(x[u]) & 0xffff0000u;
+                    const float r = x[u] - __uint_as_float(b[0][u]);
+                    b[1][u] = __float_as_uint(r) & 0xffff0000u;
+                    b[2][u] = __float_as_uint(r - __uint_as_float(b[1][u]));
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k) out[k][e] = __builtin_amdgcn_perm(b[k][1], b[k][0], 0x07060302u);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(s16x4, out[k]);
+    }
+    __device__ __forceinline__ void set_one(float v, float scale, const OneOfFour &at)
+    {
+        float x = v * scale;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, x}), bf16x2));
+            s[k] = __builtin_bit_cast(s16x4, at.of(b));
+            if (k < 2) x -= __uint_as_float(b << 16);
+        }
+    }
+};
+template <> struct Exact4<float> : Parts4<float> {
+    __device__ __forceinline__ void set(const float *v) { Parts4<float>::set<true>(v, 1.0f); }
+};
+
+__device__ __forceinline__ f32x4_t mfma4(f16x4 a, f16x4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4_t mfma4(s16x4 a, s16x4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4_t product(const Exact4<__half> &a, const Parts4<__half> &b, f32x4_t c) { return mfma4(a.x, b.hi, mfma4(a.x, b.lo, c)); }
+__device__ __forceinline__ f32x4_t product(const Parts4<__half> &a, const Exact4<__half> &b, f32x4_t c) { return mfma4(a.hi, b.x, mfma4(a.lo, b.x, c)); }
+__device__ __forceinline__ f32x4_t product(const Parts4<__half> &a, const Parts4<__half> &b, f32x4_t c)
+{
+    return mfma4(a.hi, b.hi, mfma4(a.hi, b.lo, mfma4(a.lo, b.hi, c)));
+}
+// (the six partial products meet before they join the sum, which is then rounded once a product)
+__device__ __forceinline__ f32x4_t product(const Parts4<float> &a, const Parts4<float> &b, f32x4_t c)
+{
+    f32x4_t p = mfma4(a.s[2], b.s[0], f32x4_t{});
+    p = mfma4(a.s[1], b.s[1], p);
+    p = mfma4(a.s[0], b.s[2], p);
+    p = mfma4(a.s[1], b.s[0], p);
+    p = mfma4(a.s[0], b.s[1], p);
+    p = mfma4(a.s[0], b.s[0], p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] += p[e];
+    return c;
+}
+// the 16 x 16 matrix whose transpose x is, as an operand: multiplied by a permutation matrix `unit`, which is exact
+__device__ __forceinline__ Parts4<__half> transposed(const Parts4<__half> &x, f16x4 unit)
+{
+    Parts4<__half> r;
+    const f32x4_t hi = mfma4(x.hi, unit, f32x4_t{}), lo = mfma4(x.lo, unit, f32x4_t{});
+    r.hi = to_half4(hi[0], hi[1], hi[2], hi[3]);
+    r.lo = to_half4(lo[0], lo[1], lo[2], lo[3]);
+    return r;
+}
+__device__ __forceinline__ Parts4<float> transposed(const Parts4<float> &x, s16x4 unit)
+{
+    Parts4<float> r;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const f32x4_t v = mfma4(x.s[k], unit, f32x4_t{});
+        u32x2 out;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) out[e] = __builtin_amdgcn_perm(__float_as_uint(v[2 * e + 1]), __float_as_uint(v[2 * e]), 0x07060302u);
+        r.s[k] = __builtin_bit_cast(s16x4, out);
+    }
+    return r;
+}
+// Four channels of a voxel as loaded.  A lane that wants one channel of four voxels instead, as the products do, gets it from
+// a product with the identity, which is exact (and all of a voxel's channels are NaN then where one is not finite).
+template <typename TF> struct Raw4;
+template <> struct Raw4<__half> {
+    f16x4 x;
+    __device__ __forceinline__ void load(const __half *p) { x = *reinterpret_cast<const f16x4 *>(p); }
+    __device__ __forceinline__ f32x4_t voxels(f16x4 identity) const { return mfma4(x, identity, f32x4_t{}); }
+};
+template <> struct Raw4<float> {
+    f32x4_t x;
+    __device__ __forceinline__ void load(const float *p) { x = *reinterpret_cast<const f32x4_t *>(p); }
+    __device__ __forceinline__ f32x4_t voxels(s16x4 identity) const
+    {
+        Parts4<float> y;
+        const float v[4] = {x[0], x[1], x[2], x[3]};
+        y.set<false>(v, 1.0f);
+        return mfma4(y.s[0], identity, mfma4(y.s[1], identity, mfma4(y.s[2], identity, f32x4_t{})));
+    }
+};
+// sum over the four lanes of a column (lane % 16)
+__device__ __forceinline__ float sum_columns(float x)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// coordinates of a voxel (rows of 3, 6 or 9 floats: aligned to a float)
+template <int ND> __device__ __forceinline__ void load_coords(const float *p, float *c)
+{
+    typedef float f32x3_1 __attribute__((ext_vector_type(3), aligned(4)));
+#pragma unroll
+    for (int n = 0; n < ND; n += 3) {
+        const f32x3_1 x = *reinterpret_cast<const f32x3_1 *>(p + n);
+        c[n] = x[0]; c[n + 1] = x[1]; c[n + 2] = x[2];
+    }
 }
 
 struct StripArgs {

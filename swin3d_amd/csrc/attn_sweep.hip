@@ -1289,6 +1289,12 @@ size_t attn_sweep_workspace_bytes(int H, int64_t W, int64_t N)
     return ws_end_offset(H, W, N);
 }
 
+void *attn_sweep_notes(const AttnArgs &a)
+{
+    static_assert(sizeof(unsigned long long) * kListGroups * (kListThreads / 64 + 1) * kBins == kSweepNotesBytes, "the bins");
+    return static_cast<char *>(a.workspace) + ws_bins_offset(a.H, a.W, a.N);
+}
+
 int launch_attn_sweep(const AttnArgs &a, int dtype, hipStream_t stream, int what)
 {
     switch (dtype) {

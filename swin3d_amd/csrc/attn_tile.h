@@ -376,11 +376,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct Operand;
 template <> struct Operand<__half> {
     f16x8 x;
-    struct Raw { uint4 v; };             // as loaded, before any conversion
-    static __device__ __forceinline__ Raw fetch(const __half *p) { return {*reinterpret_cast<const uint4 *>(p)}; }
-    __device__ __forceinline__ void set(const Raw &r) { x = __builtin_bit_cast(f16x8, r.v); }
     __device__ __forceinline__ void load(const __half *p) { x = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4 *>(p)); }
-    __device__ __forceinline__ void load_lds(uint32_t addr) { x = __builtin_bit_cast(f16x8, *(lds_u32x4 *)(addr)); }
     __device__ __forceinline__ void set_values(const __half *v)
     {
 #pragma unroll
@@ -389,7 +385,7 @@ template <> struct Operand<__half> {
 };
 template <> struct Operand<float> {
     bf16x8 s[3];
-    struct Raw { float4 v[2]; };
+    struct Raw { float4 v[2]; };         // as loaded, before any conversion
     static __device__ __forceinline__ Raw fetch(const float *p)
     {
         return {{reinterpret_cast<const float4 *>(p)[0], reinterpret_cast<const float4 *>(p)[1]}};
@@ -495,11 +491,6 @@ template <> struct Cells<float> {
         if constexpr (kNearest) x.split(y); else x.cut(y);
     }
 };
-__device__ __forceinline__ f32x4_t mfma16(const Operand<__half> &a, const Cells<__half> &b, f32x4_t c)
-{
-    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.x, b.lo, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.x, b.hi, c, 0, 0, 0);
-}
 // (the six partial products meet before they join the sum, which is then rounded once a product: the forward's error against
 // 64 bits on 3000 voxels of near-uniform weights is 1.0e-7 so, 2.4e-7 one after the other, 1.9e-7 in the sweep)
 __device__ __forceinline__ f32x4_t mfma16(const Operand<float> &a, const Cells<float> &b, f32x4_t c)
@@ -536,6 +527,70 @@ __device__ __forceinline__ f32x16 mfma32(const Operand<__half> &a, const Pair16 
 {
     c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.lo, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.x, b.hi, c, 0, 0, 0);
+}
+
+// ---- the forward's last resort: a query pair by pair, where something in its window is not finite
+template <typename T, int ND, typename Rows, typename First>
+__device__ __forceinline__ void exact_query(const AttnArgs &a, int h, int64_t row, int pos0, int n_w, int sub, const float *own, Rows rows_n, First first_row)
+{
+    // eight neighbouring lanes a query, which take every eighth key
+    const int HD = a.H * D;
+    const T *gq = static_cast<const T *>(a.q) + h * D, *gk = static_cast<const T *>(a.k) + h * D, *gv = static_cast<const T *>(a.v) + h * D;
+    const T *table_q = static_cast<const T *>(a.table_q) + h * D, *table_k = static_cast<const T *>(a.table_k) + h * D;
+    const T *table_v = static_cast<const T *>(a.table_v) + h * D;
+    float q[D], acc[D], m = -INFINITY, l = 0.0f;
+    load_row<D>(gq + row * a.row_stride, q);
+#pragma unroll
+    for (int c = 0; c < D; ++c) acc[c] = 0.0f;
+    for (int j = sub; j < n_w; j += 8) {
+        const int pos = pos0 + j;
+        const int64_t key = a.n2n ? a.n2n[pos] : pos;
+        float k[D], x[D], logit = 0.0f;
+        int at[ND];
+        load_row<D>(gk + key * a.row_stride, k);
+#pragma unroll
+        for (int c = 0; c < D; ++c) logit = fmaf(q[c], k[c], logit);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+            const float cj = a.n_coords[static_cast<int64_t>(pos) * ND + n];
+            at[n] = (first_row(n) + crse_row(own[n], cj, static_cast<float>(rows_n(n) / 2), crse_upper(rows_n(n)))) * HD;
+            float part = 0.0f;
+            load_row<D>(table_q + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) part = fmaf(q[c], x[c], part);
+            load_row<D>(table_k + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) part = fmaf(k[c], x[c], part);
+            logit += part;
+        }
+        const float top = fmaxf(m, logit);
+        const float scale = m == -INFINITY ? 0.0f : __expf(m - top), p = logit == -INFINITY ? 0.0f : __expf(logit - top);
+        m = top;
+        l = fmaf(l, scale, p);
+        load_row<D>(gv + key * a.row_stride, x);
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c] * scale);
+#pragma unroll
+        for (int n = 0; n < ND; ++n) {
+            load_row<D>(table_v + at[n], x);
+#pragma unroll
+            for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c]);
+        }
+    }
+#pragma unroll
+    for (int other = 1; other < 8; other <<= 1) {
+        const float m_o = __shfl_xor(m, other), l_o = __shfl_xor(l, other), top = fmaxf(m, m_o);
+        const float w = m == -INFINITY ? 0.0f : __expf(m - top), w_o = m_o == -INFINITY ? 0.0f : __expf(m_o - top);
+        l = l * w + l_o * w_o;
+#pragma unroll
+        for (int c = 0; c < D; ++c) acc[c] = acc[c] * w + __shfl_xor(acc[c], other) * w_o;
+        m = top;
+    }
+    if (sub > 0) return;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int c = 0; c < D; ++c) acc[c] *= inv;
+    store_row<D>(static_cast<T *>(a.out) + row * HD + h * D, acc);
 }
 
 }  // namespace tile

@@ -1,11 +1,11 @@
-// Sparse-voxel windowed self-attention with cRSE tables (gfx950): the tile kernel of the forward, head_dim 16.
+// Sparse-voxel windowed self-attention with cRSE tables (gfx950): the tile kernel of the forward, fp32, head_dim 16.
 //
 // A workgroup takes 64 queries by 64 keys of a head.  The products of its queries and keys with all rows of an axis table
 // come from the matrix pipe and stay in LDS, where a pair picks its two words instead of gathering two rows of 32 or 64
-// bytes; the value tables enter through histograms of the weights over their rows, one column per query.  811 voxels, 24
-// heads, fp16: 92 us (sweep) -> 47 us a call; 49,682 voxels, 6 heads, 6 axes, fp32: 413 -> 398.  No unit is busy (VALU 27 and
-// 53 % of the time, LDS addressed 25 and 33 %, matrix pipe 2 and 11 %): a tile goes through some thirty phases with a
-// barrier each, and a wavefront waits for half of its time.
+// bytes; the value tables enter through histograms of the weights over their rows, one column per query.  49,682 voxels, 6
+// heads, 6 axes: 413 us (sweep) -> 398.  No unit is busy (VALU 53 % of the time, LDS addressed 33 %, matrix pipe 11 %): a tile
+// goes through some thirty phases with a barrier each, and a wavefront waits for half of its time.  fp16 runs on strips
+// (attn_strip_fwd.hip), which in fp32, with operands of three parts, took 1.6 to 2.5 times as long as tiles.
 #include "attn_tile.h"
 
 namespace s3d {
@@ -28,15 +28,14 @@ struct FwdArgs {
 //  * summed by table row: 32-bit integers in units of 2^(e-31), below 2^-31 of the sum of all weights, so that a cell keeps
 //    what fp32 would whatever else falls into it, and no order of additions shows;
 //  * beside a value: as they are, in fp32.
-// They enter the matrix products over 2^(e - kLift): beside fp16 operands as two fp16 numbers, 23 bits from 2^15 down to
-// 2^-3 and units of 2^-24 below, which is 2^-39 of the sum; beside fp32 in full.
+// They enter the matrix products over 2^e, in full.
 constexpr float kSumFix = 33554432.0f;               // 2^25: the high word of a sum, at most 64 weights
 constexpr float kSumLow = 1.0f / 4294967296.0f;
 constexpr int kCellBits = 31;
-template <typename T> constexpr int kLift = sizeof(T) == 2 ? 15 : 0;      // (fp32 values may be as large as fp32 is)
-template <typename T> constexpr float kCellScale = sizeof(T) == 2 ? 1.0f / 65536.0f : 1.0f / 2147483648.0f;   // 2^(kLift - kCellBits)
+constexpr float kCellScale = 1.0f / 2147483648.0f;   // 2^-kCellBits
 
-template <typename T, int ND> struct FwdLayout {
+using T = float;
+template <int ND> struct FwdLayout {
     static constexpr int kSt = Stages<ND>::kCount;
     static constexpr uint32_t kSums = kCols * kStride * 4;                       // a [row][column] array of fp32 or u32
     static constexpr uint32_t kKeys = kCols * kKeyStride * 4;                    // keys: coordinates and table products
@@ -53,73 +52,11 @@ template <typename T, int ND> struct FwdLayout {
 // that is not finite.  A marked query's result is stored as NaN, and a workgroup that has marked any goes through its units
 // once more and does over, pair by pair, what is NaN.  (Done over inside the loop over units, it took the tiles 3 us of 45,
 // in registers.)
-template <typename T, int ND, typename Rows, typename First>
-__device__ __forceinline__ void exact_query(const AttnArgs &a, int h, int64_t row, int pos0, int n_w, int sub, const float *own, Rows rows_n, First first_row)
-{
-    // eight neighbouring lanes a query, which take every eighth key
-    const int HD = a.H * D;
-    const T *gq = static_cast<const T *>(a.q) + h * D, *gk = static_cast<const T *>(a.k) + h * D, *gv = static_cast<const T *>(a.v) + h * D;
-    const T *table_q = static_cast<const T *>(a.table_q) + h * D, *table_k = static_cast<const T *>(a.table_k) + h * D;
-    const T *table_v = static_cast<const T *>(a.table_v) + h * D;
-    float q[D], acc[D], m = -INFINITY, l = 0.0f;
-    load_row<D>(gq + row * a.row_stride, q);
-#pragma unroll
-    for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-    for (int j = sub; j < n_w; j += 8) {
-        const int pos = pos0 + j;
-        const int64_t key = a.n2n ? a.n2n[pos] : pos;
-        float k[D], x[D], logit = 0.0f;
-        int at[ND];
-        load_row<D>(gk + key * a.row_stride, k);
-#pragma unroll
-        for (int c = 0; c < D; ++c) logit = fmaf(q[c], k[c], logit);
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-            const float cj = a.n_coords[static_cast<int64_t>(pos) * ND + n];
-            at[n] = (first_row(n) + crse_row(own[n], cj, static_cast<float>(rows_n(n) / 2), crse_upper(rows_n(n)))) * HD;
-            float part = 0.0f;
-            load_row<D>(table_q + at[n], x);
-#pragma unroll
-            for (int c = 0; c < D; ++c) part = fmaf(q[c], x[c], part);
-            load_row<D>(table_k + at[n], x);
-#pragma unroll
-            for (int c = 0; c < D; ++c) part = fmaf(k[c], x[c], part);
-            logit += part;
-        }
-        const float top = fmaxf(m, logit);
-        const float scale = m == -INFINITY ? 0.0f : __expf(m - top), p = logit == -INFINITY ? 0.0f : __expf(logit - top);
-        m = top;
-        l = fmaf(l, scale, p);
-        load_row<D>(gv + key * a.row_stride, x);
-#pragma unroll
-        for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c] * scale);
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-            load_row<D>(table_v + at[n], x);
-#pragma unroll
-            for (int c = 0; c < D; ++c) acc[c] = fmaf(p, x[c], acc[c]);
-        }
-    }
-#pragma unroll
-    for (int other = 1; other < 8; other <<= 1) {
-        const float m_o = __shfl_xor(m, other), l_o = __shfl_xor(l, other), top = fmaxf(m, m_o);
-        const float w = m == -INFINITY ? 0.0f : __expf(m - top), w_o = m_o == -INFINITY ? 0.0f : __expf(m_o - top);
-        l = l * w + l_o * w_o;
-#pragma unroll
-        for (int c = 0; c < D; ++c) acc[c] = acc[c] * w + __shfl_xor(acc[c], other) * w_o;
-        m = top;
-    }
-    if (sub > 0) return;
-    const float inv = 1.0f / l;
-#pragma unroll
-    for (int c = 0; c < D; ++c) acc[c] *= inv;
-    store_row<D>(static_cast<T *>(a.out) + row * HD + h * D, acc);
-}
 
-template <typename T, int ND, bool kDeviceSizes>
+template <int ND, bool kDeviceSizes>
 __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
 {
-    using L = FwdLayout<T, ND>;
+    using L = FwdLayout<ND>;
     using S = Stages<ND>;
     const AttnArgs &a = f.a;
     extern __shared__ __align__(16) float smem[];
@@ -383,7 +320,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
             f32x4_t tile_acc = {0.0f, 0.0f, 0.0f, 0.0f};
             const uint32_t cell_at = ((out_half * 32 + 2 * group16) * kStride + out_tile * 16 + n16) * 4;
             const float l_tile = sum_of(out_tile * 16 + n16);
-            const int exponent = exponent_of(l_tile) - kLift<T>;
+            const int exponent = exponent_of(l_tile);
             auto read_out = [&](uint32_t cells, uint32_t operand, bool table) {
                 if (out_tile * 16 >= cols) return;
                 float v[8];
@@ -393,7 +330,7 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
                     v[e] = table ? static_cast<float>(lds_load_u32(at)) : lds_load(at);
                 }
                 Cells<T> b;
-                b.template set<false>(v, table ? kCellScale<T> : power2(-exponent));      // (to the nearest: 3 % of a call, no smaller error)
+                b.template set<false>(v, table ? kCellScale : power2(-exponent));      // (to the nearest: 3 % of a call, no smaller error)
                 Operand<T> t;
                 t.load_lds(operand + (n16 * kStride + out_half * 32 + group16 * 8) * sizeof(T));
                 tile_acc = mfma16(t, b, tile_acc);
@@ -467,15 +404,15 @@ __global__ __launch_bounds__(kThreads, 4) void attn_fwd_tile_kernel(FwdArgs f)
     }
 }
 
-template <typename T, int ND, bool kDeviceSizes>
+template <int ND, bool kDeviceSizes>
 int launch_fwd(const AttnArgs &a, const UnitList &list, hipStream_t stream)
 {
-    using L = FwdLayout<T, ND>;
+    using L = FwdLayout<ND>;
     FwdArgs f;
     f.a = a;
     f.list = list;
     constexpr uint32_t lds = L::kBytes;
-    auto kernel = attn_fwd_tile_kernel<T, ND, kDeviceSizes>;
+    auto kernel = attn_fwd_tile_kernel<ND, kDeviceSizes>;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
     const int per_cu = lds <= 80 * 1024 ? 2 : 1;
     const int slots = per_cu * device_cus();
@@ -497,50 +434,46 @@ int launch_list(const UnitList &l, const int32_t *w_sizes, const int32_t *w2n, i
 
 }  // namespace tile
 
-// Where the tile kernel serves a forward (head_dim 16).  It leaves every tile's products, sums and histograms in LDS and
+// Where the tile kernel serves a forward (fp32, head_dim 16).  It leaves every tile's products, sums and histograms in LDS and
 // crosses some thirty barriers for them, which costs about what 64 x 64 pairs cost, so it needs windows of some size.  But a
 // window is spread over its queries' tiles and a tile's pairs over 512 threads, where the sweep gives a query at most eight
 // lanes: a launch that does not fill the chip ends when its longest unit ends, and that is a quarter as long.  Measured on
 // windows of 55 to 110 voxels and 6 to 40 heads, tile over sweep kernel, by N^2 / W * H (what the sweep makes of a small
 // launch jumps with its cut into units, which is most of the spread):
-//   fp16, 9 axes: 0.55 to 0.83 at 2 M, 0.79 to 0.90 at 3 to 4 M, 0.92 to 1.12 at 4 to 6 M, 1.02 in the mean, 0.93 to 1.29 beyond
-//   fp16, 6 axes: 0.59 to 0.72 at 2 M, 0.84 to 0.96 at 3 to 4 M, 0.92 to 1.18 at 4 to 6 M, 1.03 in the mean, 1.03 to 1.41 beyond
-//   fp32, 9 axes: 0.67 at 2 M, 0.94 to 1.05 at 4 to 12 M, 0.99 in the mean, 0.91 to 1.09 beyond, 1.01 in the mean
-//   fp32, 6 axes: 0.67 at 2 M, 0.83 to 0.94 at 4 to 26 M, 0.93 and 0.97 at 35 and 29 M
+//   9 axes: 0.67 at 2 M, 0.94 to 1.05 at 4 to 12 M, 0.99 in the mean, 0.91 to 1.09 beyond, 1.01 in the mean
+//   6 axes: 0.67 at 2 M, 0.83 to 0.94 at 4 to 26 M, 0.93 and 0.97 at 35 and 29 M
 constexpr int kTileMeanWindow = 40;
-constexpr double kTilePairsHalf = 4e6, kTilePairsFloat = 35e6, kTilePairsFloatNormals = 12e6;
+constexpr double kTilePairsFloat = 35e6, kTilePairsFloatNormals = 12e6;
 
-bool attn_tile_shape(int64_t N, int64_t W, int H, int nd, bool fp32)
+bool attn_tile_shape(int64_t N, int64_t W, int H, int nd)
 {
-    const double most = !fp32 ? kTilePairsHalf : nd < 9 ? kTilePairsFloat : kTilePairsFloatNormals;
+    const double most = nd < 9 ? kTilePairsFloat : kTilePairsFloatNormals;
     return W > 0 && N >= kTileMeanWindow * W && static_cast<double>(N) * N / W * H <= most;
 }
 
 size_t attn_tile_list_bytes(int H, int64_t N, int64_t W)
 {
-    return attn_tile_shape(N, W, H, 3, true) ? tile::list_bytes(N, W) : 0;      // (whatever type and axes the call has)
+    return attn_tile_shape(N, W, H, 3) ? tile::list_bytes(N, W) : 0;      // (whatever type and axes the call has)
 }
 
 bool attn_tile_applies(const AttnArgs &a, int dtype)
 {
-    if (a.D != tile::D || !attn_tile_shape(a.N, a.W, a.H, a.nd, dtype == S3D_DTYPE_F32)) return false;
+    if (dtype != S3D_DTYPE_F32 || a.D != tile::D || !attn_tile_shape(a.N, a.W, a.H, a.nd)) return false;
     return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
 }
 
-int launch_attn_tile(const AttnArgs &a, int dtype, void *list, hipStream_t stream, int what)
+int launch_attn_tile(const AttnArgs &a, void *list, hipStream_t stream, int what)
 {
     const tile::UnitList l = tile::list_at(list, a.N, a.W);
     if (what & kAttnBuildList) {
         if (int rc = tile::launch_list(l, a.w_sizes, a.w2n, a.W, stream)) return rc;
     }
     if (!(what & kAttnSweep)) return S3D_OK;
-#define S3D_CASE(TT, CODE, NN)                                                            \
-    if (dtype == CODE && a.D == tile::D && a.nd == NN)                                    \
-        return a.sizes_dev ? tile::launch_fwd<TT, NN, true>(a, l, stream) : tile::launch_fwd<TT, NN, false>(a, l, stream);
-    S3D_CASE(__half, S3D_DTYPE_F16, 3) S3D_CASE(__half, S3D_DTYPE_F16, 6) S3D_CASE(__half, S3D_DTYPE_F16, 9)
-    S3D_CASE(float, S3D_DTYPE_F32, 3) S3D_CASE(float, S3D_DTYPE_F32, 6) S3D_CASE(float, S3D_DTYPE_F32, 9)
+#define S3D_CASE(NN) \
+    if (a.nd == NN) return a.sizes_dev ? tile::launch_fwd<NN, true>(a, l, stream) : tile::launch_fwd<NN, false>(a, l, stream);
+    S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
 #undef S3D_CASE
-    return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_fwd: head_dim %d, %d axes in the tile form", a.D, a.nd);
+    return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_fwd: %d axes in the tile form", a.nd);
 }
 
 }  // namespace s3d

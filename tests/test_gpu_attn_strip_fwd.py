@@ -1,0 +1,41 @@
+"""The strip kernel of the window attention forward (fp16, head_dim 16, launches of few strips) against the float64 oracle, at
+the edges of its strips of 16 queries and blocks of 64 keys, and on either side of its dispatch."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import to_half_and_back
+from test_gpu_attn_tile import _windows_case
+
+pytestmark = pytest.mark.gpu
+
+# a strip, two, a full block of keys, two blocks, three and six of them
+EDGES = [1, 2, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 96, 127, 128, 129, 200, 343]
+SMALL = [3, 5, 8, 13, 1, 21]
+
+
+@pytest.mark.parametrize("cRSE,heads,sizes", [
+    ("XYZ_RGB_NORM", 3, EDGES), ("XYZ_RGB", 2, EDGES), ("XYZ", 1, EDGES),
+    ("XYZ_RGB_NORM", 24, [98]), ("XYZ_RGB_NORM", 1, [1]),
+    ("XYZ", 2, SMALL * 10),                    # a mean window below the rule's
+    ("XYZ", 40, [64] * 25),                    # 5000 strips at most: more than one a workgroup
+    ("XYZ", 40, [64] * 40),                    # beyond the rule: the sweep's
+])
+def test_strips_of_every_size(oracle_lib, hip_lib, cRSE, heads, sizes):
+    from gpu_helpers import assert_attn_close, run_attention
+    case = to_half_and_back(_windows_case(oracle_lib, sizes, cRSE, heads, seed=len(sizes)))
+    got = run_attention(case, torch.float16)
+    assert_attn_close(got, oracle_lib.attn_fwd(*case.oracle_args()), torch.float16)
+    assert np.array_equal(run_attention(case, torch.float16), got)
+    assert np.array_equal(run_attention(case, torch.float16, device_sizes=True), got)
+
+
+def test_error_is_no_larger_than_the_sweeps(oracle_lib, hip_lib):
+    """What is left of a result in fp16 is its own rounding, half of 2^-10 to 2^-11 of it uniformly: 2^-11 / sqrt(3) = 2.8e-4
+    at the most; sums in fp16, as the sweep's of three value rows, would add as much."""
+    from gpu_helpers import run_attention
+    case = to_half_and_back(_windows_case(oracle_lib, [49] * 6 + [91] * 3, "XYZ_RGB_NORM", 2, seed=4))
+    ref = np.asarray(oracle_lib.attn_fwd(*case.oracle_args()))
+    strips, sweep = (run_attention(case, torch.float16), run_attention(case, torch.float16, return_stats=True)[0])
+    error = [np.linalg.norm(x - ref) / np.linalg.norm(ref) for x in (strips, sweep)]
+    assert error[0] <= 2.0 ** -11 / 3 ** 0.5 and error[0] <= error[1]
