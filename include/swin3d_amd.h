@@ -495,6 +495,17 @@ int s3d_knn_interpolate(const int32_t *idx, const float *dist2, int32_t K, int64
                         int64_t Ns, int32_t C, int32_t dtype, void *out, void *stream);
 
 /*
+ * The same for fp16 features, in fp32 and added to a row of features beside it: out = skip + interpolation, src_feat device
+ * [Ns,C] and skip device [Nq,C] fp16, out device [Nq,C] fp32, dense and 16-byte aligned, C a multiple of 4 (an upsample's sum:
+ * Swin3D/modules/swin3d_layers.py:358-366).  Its gradients: dout fp32, to dsrc_feat fp32 [Ns,C], which holds zeros before (by
+ * atomic additions, in any order), and dskip fp16 [Nq,C]; either may be null.
+ */
+int s3d_knn_interpolate_add(const int32_t *idx, const float *dist2, int32_t K, int64_t Nq, const void *src_feat,
+                            int64_t Ns, int32_t C, const void *skip, float *out, void *stream);
+int s3d_knn_interpolate_grad(const int32_t *idx, const float *dist2, int32_t K, int64_t Nq, const float *dout, int64_t Ns,
+                             int32_t C, float *dsrc_feat, void *dskip, void *stream);
+
+/*
  * Residual add fused with LayerNorm, for the Swin block on either side of the attention operator.
  *
  * The reference block (Swin3D/modules/swin3d_layers.py:617-623) computes

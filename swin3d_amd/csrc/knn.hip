@@ -13,6 +13,8 @@
 // every operation individually rounded to fp32 (no fused multiply-add).
 #include "attn_kernels.h"
 
+#include <type_traits>
+
 namespace s3d {
 namespace {
 
@@ -707,12 +709,16 @@ inline dim3 xcd_grid(int64_t items) { return dim3(static_cast<unsigned>(ceil_div
 // (Swin3D/modules/swin3d_layers.py:53-73): weight_i = 1 / (sqrt(dist2_i) + 1e-8), normalised over the K
 // neighbours, out = sum_i weight_i * src_feat[idx_i].  One thread per (query, group of VEC channels);
 // padded neighbour slots (index -1) carry no weight.  fp32 accumulation, one rounding to the output type.
-template <typename T, int VEC>
+// kSkip: the result is fp32, added to a row of fp16 features (the projected skip features of an upsample), where the framework
+// took a launch to widen src_feat and a sum of two types at a tenth of what memory gives: 25,013 x 96 48 us for the sum alone.
+template <typename T, int VEC, bool kSkip>
 __global__ __launch_bounds__(kThreads) void knn_interpolate_kernel(const int32_t *__restrict__ idx,
                                                                    const float *__restrict__ dist2, int K,
                                                                    int64_t Nq, const T *__restrict__ feat, int C,
-                                                                   T *__restrict__ out)
+                                                                   const _Float16 *__restrict__ skip,
+                                                                   typename std::conditional<kSkip, float, T>::type *__restrict__ out)
 {
+    using Out = typename std::conditional<kSkip, float, T>::type;
     const int groups = C / VEC;
     const int64_t t = share_of_xcd(Nq * groups);
     if (t >= Nq * groups) return;
@@ -770,16 +776,54 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_kernel(const int32_t
         for (int i0 = 0; i0 < K; i0 += kAhead)
             neighbours(i0, [&](const int *row, const float *weight) { add_features(row, weight, [] {}); });
     }
-    T o[VEC];
+    Out o[VEC];
+    if constexpr (kSkip) {
+        static_assert(VEC == 4, "rows of fours");
+        _Float16 beside[VEC];
+        *reinterpret_cast<uint2 *>(beside) = *reinterpret_cast<const uint2 *>(skip + qi * C + c0);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) o[e] = static_cast<T>(acc[e]);
+        for (int e = 0; e < VEC; ++e) acc[e] += static_cast<float>(beside[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o[e] = static_cast<Out>(acc[e]);
     if constexpr (VEC == 4) {
-        if constexpr (sizeof(T) == 4)
+        if constexpr (sizeof(Out) == 4)
             *reinterpret_cast<float4 *>(out + qi * C + c0) = *reinterpret_cast<const float4 *>(o);
         else
             *reinterpret_cast<uint2 *>(out + qi * C + c0) = *reinterpret_cast<const uint2 *>(o);
     } else {
         out[qi * C + c0] = o[0];
+    }
+}
+
+// The gradient of that for src_feat, added to dsrc (zeros before), and of the rows beside it: dout in fp16.  A thread has four
+// channels of a query, a quarter of a row apart, so that the lanes' additions lie side by side.
+constexpr int kGradChannels = 4;
+__global__ __launch_bounds__(kThreads) void knn_interpolate_grad_kernel(const int32_t *__restrict__ idx, const float *__restrict__ dist2, int K,
+                                                                        int64_t Nq, const float *__restrict__ dout, int C,
+                                                                        float *__restrict__ dsrc, _Float16 *__restrict__ dskip)
+{
+    const int quarter = C / kGradChannels;
+    const int64_t t = share_of_xcd(Nq * quarter);
+    if (t >= Nq * quarter) return;
+    const int64_t qi = t / quarter;
+    const int c = static_cast<int>(t - qi * quarter);
+    float g[kGradChannels];
+#pragma unroll
+    for (int e = 0; e < kGradChannels; ++e) g[e] = dout[qi * C + c + e * quarter];
+    if (dskip) {
+#pragma unroll
+        for (int e = 0; e < kGradChannels; ++e) dskip[qi * C + c + e * quarter] = static_cast<_Float16>(g[e]);
+    }
+    if (!dsrc) return;
+    float norm = 0.0f;
+    for (int i = 0; i < K; ++i) norm += idx[qi * K + i] >= 0 ? 1.0f / (sqrtf(dist2[qi * K + i]) + 1e-8f) : 0.0f;
+    for (int i = 0; i < K; ++i) {
+        const int64_t row = idx[qi * K + i];
+        if (row < 0) continue;
+        const float w = 1.0f / (sqrtf(dist2[qi * K + i]) + 1e-8f) / norm;
+#pragma unroll
+        for (int e = 0; e < kGradChannels; ++e) unsafeAtomicAdd(dsrc + row * C + c + e * quarter, g[e] * w);
     }
 }
 
@@ -791,10 +835,10 @@ int launch_interpolate(const int32_t *idx, const float *dist2, int K, int64_t Nq
     T *o = static_cast<T *>(out);
     if (C % 4 == 0) {
         const int64_t threads = Nq * (C / 4);
-        hipLaunchKernelGGL((knn_interpolate_kernel<T, 4>), xcd_grid(threads), dim3(kThreads), 0, s, idx, dist2, K, Nq, f, C, o);
+        hipLaunchKernelGGL((knn_interpolate_kernel<T, 4, false>), xcd_grid(threads), dim3(kThreads), 0, s, idx, dist2, K, Nq, f, C, nullptr, o);
     } else {
         const int64_t threads = Nq * C;
-        hipLaunchKernelGGL((knn_interpolate_kernel<T, 1>), xcd_grid(threads), dim3(kThreads), 0, s, idx, dist2, K, Nq, f, C, o);
+        hipLaunchKernelGGL((knn_interpolate_kernel<T, 1, false>), xcd_grid(threads), dim3(kThreads), 0, s, idx, dist2, K, Nq, f, C, nullptr, o);
     }
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -1000,4 +1044,47 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn_interpolate(
     hipStream_t s = static_cast<hipStream_t>(stream);
     return dtype == S3D_DTYPE_F16 ? launch_interpolate<_Float16>(idx, dist2, K, Nq, src_feat, C, out, s)
                                   : launch_interpolate<float>(idx, dist2, K, Nq, src_feat, C, out, s);
+}
+
+namespace s3d {
+namespace {
+
+int check_interpolation(const char *who, const void *idx, const void *dist2, int32_t K, int64_t Nq, int64_t Ns, int32_t C)
+{
+    if (K < 1 || K > S3D_KNN_KMAX) return fail(S3D_ERR_BAD_SHAPE, "%s: K=%d outside 1..%d", who, K, S3D_KNN_KMAX);
+    if (Nq < 0 || Ns < 1 || C < 4 || C % 4 || Nq * static_cast<int64_t>(C) > 0x3fffffffffLL)
+        return fail(S3D_ERR_BAD_SHAPE, "%s: Nq=%lld Ns=%lld C=%d (a multiple of 4) out of range", who, (long long)Nq, (long long)Ns, C);
+    if (Nq > 0 && (!idx || !dist2)) return fail(S3D_ERR_NULL_POINTER, "%s: null device pointer", who);
+    return S3D_OK;
+}
+
+}  // namespace
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_knn_interpolate_add(
+    const int32_t *idx, const float *dist2, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C,
+    const void *skip, float *out, void *stream)
+{
+    using namespace s3d;
+    if (int rc = check_interpolation("s3d_knn_interpolate_add", idx, dist2, K, Nq, Ns, C)) return rc;
+    if (Nq == 0) return S3D_OK;
+    if (!src_feat || !skip || !out) return fail(S3D_ERR_NULL_POINTER, "s3d_knn_interpolate_add: null device pointer");
+    hipLaunchKernelGGL((knn_interpolate_kernel<_Float16, 4, true>), xcd_grid(Nq * (C / 4)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                       idx, dist2, K, Nq, static_cast<const _Float16 *>(src_feat), C, static_cast<const _Float16 *>(skip), out);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_knn_interpolate_grad(
+    const int32_t *idx, const float *dist2, int32_t K, int64_t Nq, const float *dout, int64_t Ns, int32_t C, float *dsrc_feat,
+    void *dskip, void *stream)
+{
+    using namespace s3d;
+    if (int rc = check_interpolation("s3d_knn_interpolate_grad", idx, dist2, K, Nq, Ns, C)) return rc;
+    if (Nq == 0 || (!dsrc_feat && !dskip)) return S3D_OK;
+    if (!dout) return fail(S3D_ERR_NULL_POINTER, "s3d_knn_interpolate_grad: null device pointer");
+    hipLaunchKernelGGL(knn_interpolate_grad_kernel, xcd_grid(Nq * (C / kGradChannels)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                       idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
 }

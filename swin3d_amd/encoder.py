@@ -37,7 +37,7 @@ from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
 from .fused_norm import add_layernorm, trained_add_norm
 from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
-from .sparse_dl.knn import KNN, KNNInterpolate, KNNMaxPool, knn_max_pool, knn_query
+from .sparse_dl.knn import KNN, KNNInterpolate, KNNInterpolateAdd, KNNMaxPool, interpolate_add_applies, knn_max_pool, knn_query
 from .swin_blocks import data_only, linear_rows, plain, swin_blocks
 from .swin_train import trained_branches
 from .window_index import get_index01, index_arguments, window_signals, window_sets
@@ -892,15 +892,18 @@ class Upsample(nn.Module):
         stage plan of the finer level's voxel set with the same window size (the encoder's, whose regular window
         set is the one this level's attention block needs), so that the index is not built a second time.
         num_batches: batch elements of both, where the caller knows it: the host then waits for nothing."""
-        skip, coarse = self._norm_linear(self.linear1, voxels_up.feats), self._norm_linear(self.linear2, voxels.feats).float()
+        skip, coarse = self._norm_linear(self.linear1, voxels_up.feats), self._norm_linear(self.linear2, voxels.feats)
         ends, ends_up = segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches)
         if _plain_signals(signals, voxels.coords) and _plain_signals(signals_up, voxels_up.coords):
             idx, dist2 = knn_query(self.up_k, signals[:, 1:4], signals_up[:, 1:4], ends, ends_up, KNN.cell_size, strided=True)
-            feats = skip + KNNInterpolate.apply(idx, dist2, coarse.contiguous())
+            if interpolate_add_applies(idx, dist2, coarse, skip):
+                feats = KNNInterpolateAdd.apply(idx, dist2, coarse, skip)
+            else:
+                feats = skip + KNNInterpolate.apply(idx, dist2, coarse.float().contiguous())
         else:
             xyz = signals[:, 1:4].detach().contiguous().float()
             support_xyz = signals_up[:, 1:4].detach().contiguous().float()
-            feats = skip + knn_linear_interpolation(xyz, support_xyz, coarse, ends, ends_up, K=self.up_k)
+            feats = skip + knn_linear_interpolation(xyz, support_xyz, coarse.float(), ends, ends_up, K=self.up_k)
         voxels_up = voxels_up.with_feats(feats.float())
         if self.attn:
             if plan_up is not None:

@@ -155,9 +155,30 @@ class KNNMaxPool(Function):
         return None, grad
 
 
+def _interpolate_grads(idx, dist2, grad_out, num_src, need_src, need_skip):
+    """Gradients of the interpolation (fp32) and of fp16 features beside it for grad_out in fp32, by one launch behind a fill."""
+    grad_out = grad_out.contiguous()
+    nq, c = grad_out.shape
+    grad_src = torch.zeros((num_src, c), dtype=torch.float32, device=grad_out.device) if need_src else None
+    grad_skip = torch.empty((nq, c), dtype=torch.float16, device=grad_out.device) if need_skip else None
+    with _lib.on(grad_out.device):
+        status = _lib.lib().s3d_knn_interpolate_grad(idx.data_ptr(), dist2.data_ptr(), idx.shape[1], nq, grad_out.data_ptr(), num_src, c,
+                                                     None if grad_src is None else grad_src.data_ptr(),
+                                                     None if grad_skip is None else grad_skip.data_ptr(), _lib.stream(grad_out.device))
+    _lib.check(status, "s3d_knn_interpolate_grad")
+    return grad_src, grad_skip
+
+
+def _native_grads(idx, dist2, grad_out, num_src):
+    """The library's kernel has these gradients: no graph of them is wanted, nothing follows them, and it takes the types."""
+    return (not torch.is_grad_enabled() and data_only(grad_out) and grad_out.is_cuda and grad_out.dtype == torch.float32
+            and grad_out.shape[1] % 4 == 0 and grad_out.shape[1] > 0 and num_src > 0
+            and idx.is_contiguous() and dist2.is_contiguous() and idx.dtype == torch.int32)
+
+
 class KNNInterpolate(Function):
     """Differentiable (w.r.t. the features) inverse-distance interpolation; the forward is the fused
-    HIP kernel, the backward scatters the weighted output gradient back with torch's index_add_."""
+    HIP kernel, the backward adds the weighted output gradient to the sources' rows."""
 
     @staticmethod
     def forward(ctx, idx, dist2, src_feat):
@@ -168,6 +189,8 @@ class KNNInterpolate(Function):
     @staticmethod
     def backward(ctx, grad_out):
         idx, dist2 = ctx.saved_tensors
+        if _native_grads(idx, dist2, grad_out, ctx.num_src):
+            return None, None, _interpolate_grads(idx, dist2, grad_out, ctx.num_src, True, False)[0]
         valid = idx >= 0
         weight = torch.where(valid, 1.0 / (torch.sqrt(dist2) + 1e-8), torch.zeros_like(dist2))
         weight = weight / weight.sum(dim=1, keepdim=True).clamp_min(1e-30)
@@ -176,3 +199,39 @@ class KNNInterpolate(Function):
         for i in range(idx.shape[1]):
             grad_src.index_add_(0, rows[:, i], grad_out.float() * weight[:, i:i + 1])
         return None, None, grad_src.to(grad_out.dtype)
+
+
+class KNNInterpolateAdd(Function):
+    """skip + KNNInterpolate of the features, both fp16, in fp32: an upsample's sum in one kernel.  The caller has checked
+    interpolate_add_applies."""
+
+    @staticmethod
+    def forward(ctx, idx, dist2, src_feat, skip):
+        ctx.save_for_backward(idx, dist2)
+        ctx.num_src = src_feat.shape[0]
+        (nq, k), c = idx.shape, src_feat.shape[1]
+        out = torch.empty((nq, c), dtype=torch.float32, device=src_feat.device)
+        with _lib.on(src_feat.device):
+            status = _lib.lib().s3d_knn_interpolate_add(idx.data_ptr(), dist2.data_ptr(), k, nq, src_feat.data_ptr(), src_feat.shape[0], c,
+                                                        skip.data_ptr(), out.data_ptr(), _lib.stream(src_feat.device))
+        _lib.check(status, "s3d_knn_interpolate_add")
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        idx, dist2 = ctx.saved_tensors
+        _, _, need_src, need_skip = ctx.needs_input_grad
+        if _native_grads(idx, dist2, grad_out, ctx.num_src):
+            grad_src, grad_skip = _interpolate_grads(idx, dist2, grad_out, ctx.num_src, need_src, need_skip)
+            return None, None, None if grad_src is None else grad_src.half(), grad_skip
+        grad_src = KNNInterpolate.backward(ctx, grad_out)[2].half() if need_src else None
+        return None, None, grad_src, grad_out.half() if need_skip else None
+
+
+def interpolate_add_applies(idx, dist2, src_feat, skip):
+    """KNNInterpolateAdd can stand in for skip + KNNInterpolate of src_feat.float()."""
+    return (all(data_only(t) and t.is_cuda and t.device == idx.device and t.is_contiguous() for t in (idx, dist2, src_feat, skip))
+            and src_feat.dtype == skip.dtype == torch.float16 and idx.dtype == torch.int32 and dist2.dtype == torch.float32
+            and src_feat.dim() == skip.dim() == 2 and idx.dim() == 2 and skip.shape == (idx.shape[0], src_feat.shape[1])
+            and src_feat.shape[0] > 0 and src_feat.shape[1] > 0 and src_feat.shape[1] % 4 == 0
+            and src_feat.data_ptr() % 16 == 0 and skip.data_ptr() % 16 == 0)

@@ -1,0 +1,47 @@
+"""The upsample's sum of skip features and interpolated ones (fp16 in, fp32 out) in one kernel, and its gradients, against the
+two steps it replaces."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _neighbours(nq, ns, k, seed):
+    """A list with an empty place or two where there is a second batch element of fewer sources than k."""
+    import swin3d_amd
+    rng = np.random.default_rng(seed)
+    t = lambda *shape: torch.from_numpy((rng.random(shape) * 6).astype(np.float32)).cuda()
+    few = min(2, ns - 1)
+    ends = lambda n, last: torch.tensor([n - last, n], dtype=torch.int32).cuda()
+    idx, dist2 = swin3d_amd.knn_query(k, t(ns, 3), t(nq, 3), ends(ns, few), ends(nq, min(5, nq - 1)))
+    return idx, dist2
+
+
+@pytest.mark.parametrize("nq,ns,channels,k", [(1, 3, 4, 3), (700, 300, 48, 3), (700, 300, 36, 3), (1023, 257, 192, 3), (65, 40, 8, 1), (300, 90, 20, 7)])
+def test_sum_and_gradients(hip_lib, nq, ns, channels, k):
+    import swin3d_amd
+    from swin3d_amd.sparse_dl.knn import KNNInterpolateAdd, interpolate_add_applies
+    idx, dist2 = _neighbours(nq, ns, k, channels)
+    gen = torch.Generator("cuda").manual_seed(nq)
+    feat, skip = (torch.randn((n, channels), device="cuda", generator=gen).half().requires_grad_() for n in (ns, nq))
+    dout = torch.randn((nq, channels), device="cuda", generator=gen)
+    assert interpolate_add_applies(idx, dist2, feat, skip) and not interpolate_add_applies(idx, dist2, feat[:, :3], skip[:, :3])
+    out = KNNInterpolateAdd.apply(idx, dist2, feat, skip)
+    assert torch.equal(out, skip + swin3d_amd.KNNInterpolate.apply(idx, dist2, feat.float()))
+    got = torch.autograd.grad(out, (feat, skip), dout)
+    assert torch.equal(got[1], dout.half())
+    weight = torch.where(idx >= 0, 1 / (dist2.double().sqrt() + 1e-8), 0.0)
+    weight = weight / weight.sum(1, keepdim=True)
+    ref, size = (torch.zeros((ns, channels), dtype=torch.float64, device="cuda") for _ in range(2))
+    for i in range(k):
+        rows, share = idx[:, i].clamp(min=0).long(), weight[:, i:i + 1]
+        ref.index_add_(0, rows, dout.double() * share)
+        size.index_add_(0, rows, (dout.double() * share).abs())
+    # a share of dout is rounded some ten times, and a sum of n of them up to n times: 2^-24 each of the terms' sizes; the result
+    # to fp16
+    most = int(torch.bincount(idx[idx >= 0].long()).max())
+    assert bool(((got[0].double() - ref).abs() <= 2.0 ** -11 * ref.abs() + (10 + most) * 2.0 ** -24 * size + 2.0 ** -25).all())
+    # with a graph of the gradients: by operations that have one
+    (again,) = torch.autograd.grad(KNNInterpolateAdd.apply(idx, dist2, feat, skip), feat, dout.requires_grad_(), create_graph=True)
+    assert again.requires_grad and bool(((again.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + (10 + most) * 2.0 ** -24 * size + 2.0 ** -25).all())
