@@ -22,57 +22,9 @@ namespace s3d {
 namespace tile {
 namespace {
 
-// ---- strip list -------------------------------------------------------------------------------------------------------
-// A window of n voxels is ceil(n / 16) strips of equal size.  A strip: first sorted position of the window, n, and which of
-// the window's strips it is, in 22, 22 and 20 bits.
-constexpr int kPosBits = 22;
-struct StripList {
-    const int32_t *total;
-    const uint64_t *strips;
-};
-inline size_t strip_list_most(int64_t N, int64_t W) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(W > 0 ? W : 0); }
-
-// The strips of the largest windows first: bins of one size, by a counting sort in LDS.  (A strip's result does not depend on
-// its place, so the order inside a bin may be any.)
-constexpr int kSizeBins = 256;
-__global__ __launch_bounds__(kListThreads) void strip_list_kernel(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
-                                                                  int32_t *__restrict__ total, uint64_t *__restrict__ strips)
+__global__ __launch_bounds__(kListThreads) void strip_list_kernel(const int32_t *w_sizes, const int32_t *w2n, int W, int32_t *total, uint64_t *strips)
 {
-    __shared__ int at[kSizeBins];
-    const int t = threadIdx.x;
-    auto bin = [](int n) { return kSizeBins - min(n, kSizeBins); };
-    if (t < kSizeBins) at[t] = 0;
-    __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n > 0) atomicAdd(&at[bin(n)], strips_of(n));
-    }
-    __syncthreads();
-    if (t < 64) {
-        int own[kSizeBins / 64], sum = 0;
-#pragma unroll
-        for (int e = 0; e < kSizeBins / 64; ++e) sum += own[e] = at[t * (kSizeBins / 64) + e];
-        int incl = sum;
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off);
-            if (t >= off) incl += up;
-        }
-        int run = incl - sum;
-#pragma unroll
-        for (int e = 0; e < kSizeBins / 64; ++e) {
-            at[t * (kSizeBins / 64) + e] = run;
-            run += own[e];
-        }
-        if (t == 63) total[0] = incl;
-    }
-    __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n <= 0) continue;
-        const int count = strips_of(n), first = atomicAdd(&at[bin(n)], count);
-        const uint64_t window = static_cast<uint64_t>(static_cast<uint32_t>(w2n[w])) | static_cast<uint64_t>(n) << kPosBits;
-        for (int q = 0; q < count; ++q) strips[first + q] = window | static_cast<uint64_t>(q) << (2 * kPosBits);
-    }
+    build_strip_list<kListThreads>(w_sizes, w2n, W, total, strips);
 }
 
 struct FwdArgs {
@@ -484,12 +436,17 @@ bool attn_strip_applies(const AttnArgs &a, int dtype)
     return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
 }
 
+tile::StripList attn_strip_list(const AttnArgs &a)
+{
+    char *at = static_cast<char *>(attn_sweep_notes(a)) + kSweepNotesKept;
+    static_assert(kSweepNotesKept + 256 + sizeof(uint64_t) * kStripsMost <= kSweepNotesBytes, "the list fits");
+    return {reinterpret_cast<const int32_t *>(at), reinterpret_cast<const uint64_t *>(at + 256)};
+}
+
 int launch_attn_strip(const AttnArgs &a, hipStream_t stream, int what)
 {
     using namespace tile;
-    char *notes = static_cast<char *>(attn_sweep_notes(a));
-    static_assert(256 + sizeof(uint64_t) * kStripsMost <= kSweepNotesBytes, "the list fits");
-    const StripList l{reinterpret_cast<const int32_t *>(notes), reinterpret_cast<const uint64_t *>(notes + 256)};
+    const StripList l = attn_strip_list(a);
     if (what & kAttnBuildList) {
         hipLaunchKernelGGL(strip_list_kernel, dim3(1), dim3(kListThreads), 0, stream, a.w_sizes, a.w2n, static_cast<int>(a.W),
                            const_cast<int32_t *>(l.total), const_cast<uint64_t *>(l.strips));

@@ -170,12 +170,12 @@ __host__ __device__ inline UnitPlan plan_units(int total_slots, int waves)
 // the wavefront keeps in registers (lane b % 64 holds bin b), and the wavefront leaves its bin totals.  No
 // atomics: the list, and with it the cut of the queries into units and so every bit of the result, is the same
 // on every run.
-__global__ __launch_bounds__(kListThreads) void sweep_count_kernel(AttnArgs a)
+__device__ __forceinline__ void count_windows(const AttnArgs &a, int group, int groups)
 {
     constexpr int kWaves = kListThreads / 64;
     const int lane = threadIdx.x & 63;
-    const int table = static_cast<int>(blockIdx.x) * kWaves + static_cast<int>(threadIdx.x >> 6);
-    const int tables = static_cast<int>(gridDim.x) * kWaves;
+    const int table = group * kWaves + static_cast<int>(threadIdx.x >> 6);
+    const int tables = groups * kWaves;
     char *ws = static_cast<char *>(a.workspace);
     int2 *place = reinterpret_cast<int2 *>(ws + ws_place_offset(a.H, a.W, a.N));
     unsigned long long *group_bins = reinterpret_cast<unsigned long long *>(ws + ws_bins_offset(a.H, a.W, a.N));
@@ -238,14 +238,15 @@ __global__ __launch_bounds__(kListThreads) void sweep_count_kernel(AttnArgs a)
     unsigned long long sum = 0;
 #pragma unroll
     for (int v = 0; v < kWaves; ++v) sum += wave_bins[v][threadIdx.x];
-    sum_bins[static_cast<size_t>(blockIdx.x) * kBins + threadIdx.x] = sum;
+    sum_bins[static_cast<size_t>(group) * kBins + threadIdx.x] = sum;
 }
+__global__ __launch_bounds__(kListThreads) void sweep_count_kernel(AttnArgs a) { count_windows(a, blockIdx.x, gridDim.x); }
 
 // sweep_place_kernel (same grid): bins in order, wavefronts in order inside a bin.  Writes one entry (first
 // query of its class, voxels, first sorted position, class) per window in sorted order, one record per unit
 // (the entry that holds its first query, lanes per query as a shift, first query, queries), the totals, and
 // the queue counters at zero.
-__global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
+__device__ __forceinline__ void place_windows(const AttnArgs &a, int group, int groups)
 {
     constexpr int kWaves = kListThreads / 64;
     __shared__ int bin_entry[kWaves][kBins], bin_slot[kWaves][kBins];
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
     const int2 *place = reinterpret_cast<const int2 *>(ws + ws_place_offset(a.H, a.W, a.N));
     const unsigned long long *group_bins =
         reinterpret_cast<const unsigned long long *>(ws + ws_bins_offset(a.H, a.W, a.N));
-    const int tables = static_cast<int>(gridDim.x) * kWaves, first_table = static_cast<int>(blockIdx.x) * kWaves;
+    const int tables = groups * kWaves, first_table = group * kWaves;
     const unsigned long long *sum_bins = group_bins + static_cast<size_t>(kListGroups) * kWaves * kBins;
     // thread t holds bin t: the launch's total, and what the workgroups before this one put there; an exclusive
     // scan over the threads gives the bins their places (entries over all bins, queries restarting per class)
@@ -268,10 +269,10 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         unsigned long long all = 0, before = 0;
 #pragma unroll 8
-        for (int g = 0; g < static_cast<int>(gridDim.x); ++g) {
+        for (int g = 0; g < groups; ++g) {
             const unsigned long long v = sum_bins[static_cast<size_t>(g) * kBins + threadIdx.x];
             all += v;
-            before += g < static_cast<int>(blockIdx.x) ? v : 0;
+            before += g < group ? v : 0;
         }
         const int cnt = static_cast<int>(all >> 32), slots = static_cast<int>(all & 0xffffffffu);
         int incl_c = cnt, incl_s = slots;
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
             }
         }
     }
-    if (blockIdx.x == 0) {
+    if (group == 0) {
         // a wavefront reads 64 entries from a unit's first one: pad the list with entries no query belongs to
         if (threadIdx.x < kChunk) entries[total_entries + threadIdx.x] = make_int4(0x7fffffff, 1, 0, -1);
         if (threadIdx.x == 0) {
@@ -348,6 +349,35 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a)
         if (threadIdx.x < kQueues) total[(1 + threadIdx.x) * kCounterStride] = 0;
         for (int t = threadIdx.x; t < a.H * kQueues; t += kListThreads) counters[t * kCounterStride] = 0;
     }
+}
+__global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a) { place_windows(a, blockIdx.x, gridDim.x); }
+
+// Few windows, of which every wavefront has one round: both steps by one workgroup, and the strip list, where it is asked for, by
+// another beside it.  A plan for strips of 2 windows 10.1 us (three launches) -> 5.8, of 84 windows 14.4 -> 8.9; at 340 windows, two
+// rounds, one launch takes 17.2 and two 11.6.
+__global__ __launch_bounds__(kListThreads) void sweep_list_kernel(AttnArgs a)
+{
+    if (blockIdx.x == 1) {
+        tile::build_strip_list<kListThreads>(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(a.also_strips.total),
+                                             const_cast<uint64_t *>(a.also_strips.strips));
+        return;
+    }
+    count_windows(a, 0, 1);
+    __threadfence();
+    __syncthreads();
+    place_windows(a, 0, 1);
+}
+
+void launch_work_list(const AttnArgs &a, hipStream_t stream)
+{
+    if (a.W <= kFewWindows) {
+        hipLaunchKernelGGL(sweep_list_kernel, dim3(a.also_strips.total ? 2 : 1), dim3(kListThreads), 0, stream, a);
+        return;
+    }
+    const int64_t want = ceil_div(a.W, kListThreads);
+    const dim3 grid(static_cast<unsigned>(want > kListGroups ? kListGroups : want));
+    hipLaunchKernelGGL(sweep_count_kernel, grid, dim3(kListThreads), 0, stream, a);
+    hipLaunchKernelGGL(sweep_place_kernel, grid, dim3(kListThreads), 0, stream, a);
 }
 
 // Workgroup shapes.  A workgroup holds its heads' table slices once, so what fits a CU is set by registers and LDS:
@@ -1103,11 +1133,8 @@ int launch_sweep_heads(const AttnArgs &a, hipStream_t stream, int what)
     constexpr int kThreads = group_threads<T, D, HP>();
     b.target_items = grid / groups * (kThreads / 64);   // wavefronts that serve one head group
     b.block_shift = target_shift_for(a.N, a.W, b.target_items);
-    const int64_t list_want = (a.W + kListThreads - 1) / kListThreads;
-    const dim3 list_grid(static_cast<unsigned>(list_want < 1 ? 1 : (list_want > kListGroups ? kListGroups : list_want)));
     if (what & 1) {
-        hipLaunchKernelGGL(sweep_count_kernel, list_grid, dim3(kListThreads), 0, stream, b);
-        hipLaunchKernelGGL(sweep_place_kernel, list_grid, dim3(kListThreads), 0, stream, b);
+        launch_work_list(b, stream);
         S3D_HIP_CHECK(hipGetLastError());
     }
     if (what & 2) {
@@ -1197,10 +1224,7 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
     // (one work list, cut for the query-owned sweep, which takes longer)
     b.f.target_items = grid / groups * (kThreads / 64);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
-    const int64_t list_want = (a.W + kListThreads - 1) / kListThreads;
-    const dim3 list_grid(static_cast<unsigned>(list_want < 1 ? 1 : (list_want > kListGroups ? kListGroups : list_want)));
-    hipLaunchKernelGGL(sweep_count_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
-    hipLaunchKernelGGL(sweep_place_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
+    launch_work_list(b.f, stream);
     S3D_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(q_sweep, dim3(static_cast<unsigned>(grid)), dim3(kThreads), q_lds, stream, b);
     hipLaunchKernelGGL(k_sweep, dim3(static_cast<unsigned>(key_grid)), dim3(kThreads), k_lds, stream, by_key);
@@ -1226,10 +1250,7 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
     const int grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
     b.f.target_items = grid / groups * (kThreads / 64);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
-    const int64_t list_want = (a.W + kListThreads - 1) / kListThreads;
-    const dim3 list_grid(static_cast<unsigned>(list_want < 1 ? 1 : (list_want > kListGroups ? kListGroups : list_want)));
-    hipLaunchKernelGGL(sweep_count_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
-    hipLaunchKernelGGL(sweep_place_kernel, list_grid, dim3(kListThreads), 0, stream, b.f);
+    launch_work_list(b.f, stream);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -1292,6 +1313,8 @@ size_t attn_sweep_workspace_bytes(int H, int64_t W, int64_t N)
 void *attn_sweep_notes(const AttnArgs &a)
 {
     static_assert(sizeof(unsigned long long) * kListGroups * (kListThreads / 64 + 1) * kBins == kSweepNotesBytes, "the bins");
+    // (one workgroup: its wavefronts' bins in front, and its own behind all that 32 would have)
+    static_assert(sizeof(unsigned long long) * (kListThreads / 64) * kBins <= kSweepNotesKept, "the bins of one workgroup");
     return static_cast<char *>(a.workspace) + ws_bins_offset(a.H, a.W, a.N);
 }
 

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "attn_kernels.h"
+#include "attn_strip_list.h"
 #include "sweep_common.h"
 
 namespace s3d {
@@ -46,7 +47,6 @@ struct UnitList {
 };
 // A strip is up to 16 voxels of windows of one size: the voxels of its windows (of at most 64 voxels) in the order of the
 // entries, from column `first` of window `entry` on; of a larger window, 16 of its voxels.
-constexpr int kStrip = 16;
 // A unit, decoded: the tile's queries are `cols` voxels; with more than one tile the workgroup goes through the tiles
 // of the window's keys.
 struct Unit {
@@ -97,7 +97,6 @@ constexpr int kListThreads = 1024;
 constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 32 and more tiles, then 64 .. 1 voxels
 
 __device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
-__device__ __forceinline__ int strips_of(int n) { return (n + kStrip - 1) / kStrip; }
 __device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
 
 // Unit list: windows in bins of equal size, largest first (a counting sort in LDS), and the pairs of the windows before

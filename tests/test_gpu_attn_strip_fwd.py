@@ -20,12 +20,14 @@ SMALL = [3, 5, 8, 13, 1, 21]
     ("XYZ", 2, SMALL * 10),                    # a mean window below the rule's
     ("XYZ", 40, [64] * 25),                    # 5000 strips at most: more than one a workgroup
     ("XYZ", 40, [64] * 40),                    # beyond the rule: the sweep's
+    ("XYZ", 1, [5, 9] * 128), ("XYZ", 1, [5, 9] * 128 + [7]),      # windows whose lists one launch makes, and one more
 ])
 def test_strips_of_every_size(oracle_lib, hip_lib, cRSE, heads, sizes):
     from gpu_helpers import assert_attn_close, run_attention
     case = to_half_and_back(_windows_case(oracle_lib, sizes, cRSE, heads, seed=len(sizes)))
-    got = run_attention(case, torch.float16)
-    assert_attn_close(got, oracle_lib.attn_fwd(*case.oracle_args()), torch.float16)
+    got, ref = run_attention(case, torch.float16), oracle_lib.attn_fwd(*case.oracle_args())
+    assert_attn_close(got, ref, torch.float16)
+    assert_attn_close(run_attention(case, torch.float16, return_stats=True)[0], ref, torch.float16)      # (the sweep's, on a plan like it)
     assert np.array_equal(run_attention(case, torch.float16), got)
     assert np.array_equal(run_attention(case, torch.float16, device_sizes=True), got)
 
