@@ -8,7 +8,7 @@
 //   dk_j  += dL (q_i + Tk(i,j))                    dTk[n][row_n(i,j)] += dL k_j
 // The reference adds every term with a global atomic.  Here every output element has ONE owner, and the call has three
 // forms.  With the window set's pair count it runs on strips (tables of up to 64 rows on a position axis and 32 on a signal
-// axis; attn_strip_bwd.hip, at head_dim 16 behind attn_tile_bwd.hip, at 8 behind a sweep), otherwise the pair sweeps of attn_sweep.hip on the
+// axis; attn_strip_bwd.hip, at head_dim 16 behind attn_strip_records.hip or attn_tile_bwd.hip, at 8 behind a sweep), otherwise the pair sweeps of attn_sweep.hip on the
 // forward's packed work list (dq, which leaves dL and P of every (pair, head) in the workspace; dk and dv) and the
 // table-gradient kernels below (attn_bwd_tables_kernel), which read dL and P.  Without it, the fused sweeps (attn_bwd_sweep_kernel),
 // which recompute the logits and need no store:

@@ -100,7 +100,7 @@ int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream);
 // dL and P alone (head_dim 8), with dout_i . o_i made from b.out in place of b.delta
 int launch_attn_bwd_records(const BwdPairArgs &b, int dtype, hipStream_t stream);
 
-// The backward on tiles (attn_tile_bwd.hip): head_dim 16, tables that fit a stage, the pair count known.  Of the
+// The backward on tiles or strips (attn_tile_bwd.hip, attn_strip_records.hip): head_dim 16, tables that fit a stage, the pair count known.  Of the
 // arguments it takes the shape, inputs and dq, dk, dv; its own workspace holds records, slots, unit and strip list.
 bool attn_tile_bwd_applies(const int32_t *rows, int nd, int D, int64_t pairs);
 size_t attn_tile_bwd_bytes(int H, int nd, int64_t N, int64_t W, int64_t pairs);

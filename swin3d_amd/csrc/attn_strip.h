@@ -1,5 +1,5 @@
-// Pieces shared by the kernels on strips of 16 voxels (attn_strip_fwd.hip, attn_strip_bwd.hip), and the interface between the
-// backward's records kernel (attn_tile_bwd.hip) and the kernels that sum over pairs.
+// Pieces shared by the kernels on strips of 16 voxels (attn_strip_fwd.hip, attn_strip_records.hip, attn_strip_bwd.hip), and the
+// interfaces between the backward's kernels at head_dim 16.
 #pragma once
 
 #include "attn_tile.h"
@@ -148,6 +148,7 @@ template <> struct Exact4<float> : Parts4<float> {
 
 __device__ __forceinline__ f32x4_t mfma4(f16x4 a, f16x4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4_t mfma4(s16x4 a, s16x4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4_t product(const Exact4<__half> &a, const Exact4<__half> &b, f32x4_t c) { return mfma4(a.x, b.x, c); }
 __device__ __forceinline__ f32x4_t product(const Exact4<__half> &a, const Parts4<__half> &b, f32x4_t c) { return mfma4(a.x, b.hi, mfma4(a.x, b.lo, c)); }
 __device__ __forceinline__ f32x4_t product(const Parts4<__half> &a, const Exact4<__half> &b, f32x4_t c) { return mfma4(a.hi, b.x, mfma4(a.lo, b.x, c)); }
 __device__ __forceinline__ f32x4_t product(const Parts4<__half> &a, const Parts4<__half> &b, f32x4_t c)
@@ -228,6 +229,114 @@ template <int ND> __device__ __forceinline__ void load_coords(const float *p, fl
     }
 }
 
+// a table as operands beside features of type TF
+template <typename T, typename TF> struct StripTable { using type = Exact4<TF>; };
+template <> struct StripTable<float, __half> { using type = Parts4<__half>; };
+
+// ---- strips of single windows -----------------------------------------------------------------------------------------
+// A window of n voxels is ceil(n / 16) strips of equal size.  A strip: first sorted position of the window, n, which of the
+// window's strips it is, and the pairs (n^2) of the windows before it.
+struct WindowStrips {
+    const int32_t *total;
+    const int4 *strips;
+};
+inline size_t window_strips_most(int64_t N, int64_t W) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(W > 0 ? W : 0); }
+
+// By one workgroup: the strips of the largest windows first, bins of one size by a counting sort in LDS.  (A strip's result
+// does not depend on its place, so the order inside a bin may be any.)
+__device__ __forceinline__ void build_window_strips(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
+                                                    int32_t *__restrict__ total, int4 *__restrict__ strips)
+{
+    __shared__ int at[kSizeBins];
+    __shared__ long long wave_pairs[kListThreads / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    auto bin = [](int n) { return kSizeBins - min(n, kSizeBins); };
+    if (t < kSizeBins) at[t] = 0;
+    __syncthreads();
+    for (int w = t; w < W; w += kListThreads) {
+        const int n = w_sizes[w];
+        if (n > 0) atomicAdd(&at[bin(n)], strips_of(n));
+    }
+    __syncthreads();
+    if (t < 64) {
+        int own[kSizeBins / 64], sum = 0;
+#pragma unroll
+        for (int e = 0; e < kSizeBins / 64; ++e) sum += own[e] = at[t * (kSizeBins / 64) + e];
+        int incl = sum;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off);
+            if (t >= off) incl += up;
+        }
+        int run = incl - sum;
+#pragma unroll
+        for (int e = 0; e < kSizeBins / 64; ++e) {
+            at[t * (kSizeBins / 64) + e] = run;
+            run += own[e];
+        }
+        if (t == 63) total[0] = incl;
+    }
+    __syncthreads();
+    long long before = 0;              // pairs of the windows of earlier rounds
+    for (int w0 = 0; w0 < W; w0 += kListThreads) {
+        const int w = w0 + t, n = w < W ? max(w_sizes[w], 0) : 0;
+        const long long own = static_cast<long long>(n) * n;
+        long long pairs = own;
+        for (int off = 1; off < 64; off <<= 1) {
+            const long long up = __shfl_up(pairs, off);
+            if (lane >= off) pairs += up;
+        }
+        if (lane == 63) wave_pairs[wave] = pairs;
+        __syncthreads();
+        pairs += before - own;
+        for (int v = 0; v < kListThreads / 64; ++v) {
+            pairs += v < wave ? wave_pairs[v] : 0;
+            before += wave_pairs[v];
+        }
+        if (n > 0) {
+            const int count = strips_of(n), first = atomicAdd(&at[bin(n)], count), pos = w2n[w];
+            // (a window that begins beyond 2^31 pairs does not fit any store)
+            for (int q = 0; q < count; ++q) strips[first + q] = make_int4(pos, n, q, static_cast<int>(pairs < 0x7fffffffll ? pairs : 0x7fffffffll));
+        }
+        __syncthreads();
+    }
+}
+
+// A strip with a block of at most kKeyBlock of its window's keys: what a workgroup works off at a time.
+template <int kKeyBlock> struct StripItem {
+    int pos0, n, first, cols, blocks, block, first_key, keys_n, pairs;
+    __device__ __forceinline__ void set_block(int which)
+    {
+        const int size = (n + blocks - 1) / blocks;
+        block = which;
+        first_key = block * size;
+        keys_n = min(size, n - first_key);
+    }
+    __device__ __forceinline__ void set(int4 s)
+    {
+        pos0 = __builtin_amdgcn_readfirstlane(s.x);
+        n = __builtin_amdgcn_readfirstlane(s.y);
+        pairs = __builtin_amdgcn_readfirstlane(s.w);
+        const int count = strips_of(n), size = (n + count - 1) / count;
+        first = __builtin_amdgcn_readfirstlane(s.z) * size;
+        cols = min(size, n - first);
+        blocks = (n + kKeyBlock - 1) / kKeyBlock;
+        set_block(0);
+    }
+};
+// lane `which` of each sixteen
+__device__ __forceinline__ float of_sixteen(float value, int which)
+{
+    const int x = __float_as_int(value);
+    // (row_newbcast; the lane is part of the instruction)
+    switch (which) {
+#define S3D_LANE(N) case N: return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x150 + N, 0xf, 0xf, true));
+        S3D_LANE(0) S3D_LANE(1) S3D_LANE(2) S3D_LANE(3) S3D_LANE(4) S3D_LANE(5) S3D_LANE(6) S3D_LANE(7)
+#undef S3D_LANE
+    }
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x158, 0xf, 0xf, true));
+}
+typedef __attribute__((address_space(3))) f32x4_t lds_f32x4;
+
 struct StripArgs {
     AttnArgs f;                 // shape, q, k, tables, index arrays, rows[] / base[]
     UnitList list;              // entries and strips
@@ -244,6 +353,27 @@ struct StripArgs {
     float *dtq, *dtk, *dtv;
     float half_rows[kMaxAxes], upper[kMaxAxes];    // what crse_row takes (made here, they would take two vector registers an axis)
 };
+// The kernels that leave dL and P of every pair, at head_dim 16: on tiles (attn_tile_bwd.hip, fp32 and small windows) or strips
+// (attn_strip_records.hip, fp16 features).
+struct RecordsCall {
+    AttnArgs f;                 // shape, q, k, v, tables, index arrays, rows[] / base[]
+    UnitList list;              // entries and strips of the kernels that sum over pairs (and the units)
+    const void *dout, *out;
+    const float *stat_max, *stat_sum;
+    float2 *records;            // [H][pairs]: (dL, P)
+    int64_t pairs;              // capacity of records per head; windows beyond it are skipped
+    int4 *strip_columns;        // see StripArgs
+    int32_t *strip_rows;
+    void *operands;             // the tables as matrix operands, and
+    float *scales;              // [head][Tq, Tk, Tv] what a product with them is multiplied by
+};
+__device__ __forceinline__ bool window_fits(int before, int n, int64_t pairs)
+{
+    return static_cast<int64_t>(before) + static_cast<int64_t>(n) * n <= pairs;
+}
+size_t strip_records_bytes(int H, int nd, int64_t N, int64_t W);
+int launch_strip_records(const RecordsCall &c, void *room, int dtype, hipStream_t stream);
+
 size_t strip_slots_bytes(int H, int nd);
 int launch_strip_gradients(const StripArgs &b, int dtype, hipStream_t stream);
 

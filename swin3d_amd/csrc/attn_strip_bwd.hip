@@ -1,5 +1,5 @@
 // Attention backward at head_dim 16: what is a sum over pairs, from dL and P of every (pair, head) (gfx950).  The mathematics
-// is in attn_bwd.hip, the kernel that leaves the pairs in attn_tile_bwd.hip.
+// is in attn_bwd.hip, the kernels that leave the pairs in attn_strip_records.hip and attn_tile_bwd.hip.
 //
 // A workgroup takes a strip of up to 16 voxels of windows of one size and all their pairs: as queries (dq, dTq, dTv) in one
 // launch, as keys (dk, dv, dTk) in another.  It adds up the pairs' dL (and P) by table row into histograms over the rows of
@@ -56,9 +56,6 @@ constexpr int kLiftFeature = 15;              // exponent of the strip's largest
 
 constexpr int kStripReach = kStripThreads / kStrip;        // pairs of a voxel that a step of the workgroup takes
 constexpr int kKept = 4;                                   // pairs that a thread keeps from the sum of |dL| on: an operand's terms
-
-template <typename T, typename TF> struct StripTable { using type = Exact4<TF>; };
-template <> struct StripTable<float, __half> { using type = Parts4<__half>; };
 
 // largest of a 16-lane group
 template <typename V> __device__ __forceinline__ V max16(V v)

@@ -55,26 +55,12 @@ constexpr int kStageRows = kStripWaves * 16;       // table rows of a stage: a t
 // words between the products of one voxel and the next: 16-byte stores of 16 voxels meet in no bank
 constexpr int kProductStride = kStageRows + 4;
 
-typedef __attribute__((address_space(3))) f32x4_t lds_f32x4;
 __device__ __forceinline__ float max_columns(float x)
 {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ f32x4_t product(const Exact4<__half> &a, const Exact4<__half> &b, f32x4_t c) { return mfma4(a.x, b.x, c); }
-
-// lane `which` of each sixteen
-__device__ __forceinline__ int of_sixteen(int x, int which)
-{
-    // (row_newbcast; the lane is part of the instruction)
-    switch (which) {
-#define S3D_LANE(N) case N: return __builtin_amdgcn_update_dpp(0, x, 0x150 + N, 0xf, 0xf, true);
-        S3D_LANE(0) S3D_LANE(1) S3D_LANE(2) S3D_LANE(3) S3D_LANE(4) S3D_LANE(5) S3D_LANE(6) S3D_LANE(7)
-#undef S3D_LANE
-    }
-    return __builtin_amdgcn_update_dpp(0, x, 0x158, 0xf, 0xf, true);
 }
 
 template <int ND, bool kDeviceSizes>
@@ -282,7 +268,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
 #pragma unroll
                 for (int axis = 0; axis < ND; ++axis) {
                     if (axis_row0(axis) / kStageRows != st) continue;
-                    const float its = __int_as_float(of_sixteen(__float_as_int(other[s]), axis));
+                    const float its = of_sixteen(other[s], axis);
                     const uint32_t r = static_cast<uint32_t>(crse_row(own[axis], its, half_rows(axis), upper(axis)));
                     const int first = axis_row0(axis) % kStageRows;
                     row_at[s][axis] = r * (kStrip * 4) + c16 * 4;

@@ -1,16 +1,16 @@
-// Attention backward at head_dim 16 (gfx950): dL and P of every pair, on tiles of up to 64 queries by 64 keys of a head.  The
-// mathematics is in attn_bwd.hip, what is a sum over pairs in attn_strip_bwd.hip.
+// Attention backward at head_dim 16 (gfx950): dL and P of every pair, on tiles of up to 64 queries by 64 keys of a head, in fp32
+// and of small windows; other fp16 features run on strips (attn_strip_records.hip).  The mathematics is in attn_bwd.hip, what is a
+// sum over pairs in attn_strip_bwd.hip.
 //
 // tile_records_kernel, on the forward's unit list, makes the logits again and dP = dout_i . (v_j + Tv(i,j)) as the forward's
 // tile kernel makes its logits: the products of the tile's queries (q with Tq, dout with Tv) and keys (k with Tk) with all
 // rows of an axis come from the matrix pipe and stay in LDS, where every pair picks its three.  It leaves dL and P of every
 // (pair, head): 8 bytes at [head][pairs before the window + j n + i].
 //
-// Why tiles: the pair sweeps this form replaces run at two wavefronts per SIMD (192 VGPRs) and wait for a gathered table
-// row of 64 bytes per pair, axis and table.  Here a pair's term is a word of LDS.  One form for every window size: a unit
-// packs windows of up to 64 voxels side by side.  12,421 voxels in windows of 72, 9 axes, 12 heads, fp32 tables beside fp16
-// features: 182 us; the VALU issues 40 % of the time, the LDS is addressed for 33 %, the matrix pipe works for 6 %, and a
-// wavefront waits for 48 % of its time, most of it at barriers.
+// Why tiles: one form for every window size, since a unit packs windows of up to 64 voxels side by side; and an operand of three
+// bf16 numbers makes a product six instructions, which tiles of 32 by 32 take at twice the rate of the strips' 16 by 16.  fp32 on
+// strips, layers of 6,000 to 49,682 voxels: 1.03 to 1.07 times as long, forward included, with 64 keys at a time, 1.1 to 1.3 with 96
+// (registers).
 #include "attn_strip.h"
 
 #include <algorithm>
@@ -25,27 +25,12 @@ namespace {
 template <typename T, typename TF> struct TableOperand { using type = Operand<T>; };
 template <> struct TableOperand<float, __half> { using type = Pair16; };
 
-struct BwdTileArgs {
-    AttnArgs f;                 // shape, q, k, v (dense), tables, index arrays, rows[] / base[]
-    UnitList list;
-    const void *dout, *out;
-    const float *stat_max, *stat_sum;
-    float2 *records;            // [H][pairs]: (dL, P)
-    int64_t pairs;              // capacity of records per head; windows beyond it are skipped
+struct BwdTileArgs : RecordsCall {
     int32_t *rows, *first_pair; // [unit][column]: the units' voxels, their rows and, of the pairs of their windows, the one
                                 // with the window's first key (-1: beyond the records); see tile_columns_kernel
     float *coords;              // [unit][axis][column]
-    int4 *strip_columns;        // see StripArgs
-    int32_t *strip_rows;
-    void *operands;             // the tables as matrix operands, and
-    float *scales;              // [head][3] what a product with them is multiplied by: see tile_setup_kernel
     int32_t groups;             // workgroups per head
 };
-
-__device__ __forceinline__ bool window_fits(const int2 entry, int n, int64_t pairs)
-{
-    return static_cast<int64_t>(entry.y) + static_cast<int64_t>(n) * n <= pairs;
-}
 
 // ---- setup ------------------------------------------------------------------------------------------------------------
 // The unit list (workgroup 0) and, a workgroup for each head and table, the tables as the lanes' matrix operands:
@@ -110,7 +95,7 @@ __global__ __launch_bounds__(256) void tile_columns_kernel(BwdTileArgs b)
         const int col = strip.z + min(c % kStrip, strip.w - 1);
         const int2 entry = b.list.entries[strip.x + col / strip.y];
         const int pos = entry.x + col % strip.y, row = a.n2n ? a.n2n[pos] : pos;
-        b.strip_columns[s * kStrip + c % kStrip] = make_int4(pos, row, entry.x, window_fits(entry, strip.y, b.pairs) ? entry.y : -1);
+        b.strip_columns[s * kStrip + c % kStrip] = make_int4(pos, row, entry.x, window_fits(entry.y, strip.y, b.pairs) ? entry.y : -1);
         b.strip_rows[s * kStrip + c % kStrip] = row;
     }
     if (u >= b.list.total[0]) return;
@@ -119,7 +104,7 @@ __global__ __launch_bounds__(256) void tile_columns_kernel(BwdTileArgs b)
     const int2 entry = unit.entry_of(b.list, cc);
     const int in = unit.inside(unit.tile, cc), pos = entry.x + in;
     b.rows[u * kCols + c] = a.n2n ? a.n2n[pos] : pos;
-    b.first_pair[u * kCols + c] = window_fits(entry, unit.n_w, b.pairs) ? entry.y + in : -1;
+    b.first_pair[u * kCols + c] = window_fits(entry.y, unit.n_w, b.pairs) ? entry.y + in : -1;
 #pragma unroll
     for (int n = 0; n < ND; ++n)
         b.coords[(static_cast<int64_t>(u) * ND + n) * kCols + c] = a.n_coords[static_cast<int64_t>(pos) * ND + n];
@@ -139,6 +124,8 @@ template <int ND> struct RecordsLayout {
 template <typename T, typename TF, int ND>
 __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b)
 {
+    using Table = typename TableOperand<T, TF>::type;
+    constexpr bool kScaled = std::is_same<Table, Pair16>::value;
     using L = RecordsLayout<ND>;
     using S = Stages<ND>;
     const AttnArgs &a = b.f;
@@ -153,9 +140,8 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
     const uint32_t queries = lds_base(smem), keys = queries + L::kQueries, coords = keys + L::kKeys;
     const TF *gq = static_cast<const TF *>(a.q), *gk = static_cast<const TF *>(a.k), *gv = static_cast<const TF *>(a.v);
     const TF *gd = static_cast<const TF *>(b.dout), *go = static_cast<const TF *>(b.out);
-    using Table = typename TableOperand<T, TF>::type;
     const Table *operands = static_cast<const Table *>(b.operands) + static_cast<int64_t>(h) * (3 * S::kCount * 128);
-    const float scale_q = b.scales[h * 3], scale_k = b.scales[h * 3 + 1], scale_v = b.scales[h * 3 + 2];
+    const float scale_q = kScaled ? b.scales[h * 3] : 1.0f, scale_k = kScaled ? b.scales[h * 3 + 1] : 1.0f, scale_v = kScaled ? b.scales[h * 3 + 2] : 1.0f;
     const int tile_c = wave & 1, tile_r = (wave >> 1) & 1;
 
     for (int u = group; u < total_units; u += groups) {
@@ -276,8 +262,9 @@ __global__ __launch_bounds__(kThreads, 4) void tile_records_kernel(BwdTileArgs b
                         const uint32_t r = static_cast<uint32_t>(crse_row(ci, cj, half_rows, upper));
                         const float2 x = lds_load2(__umul24(r, kStride * 8) + own_at);
                         const float k = lds_load(r * 4 + key_at[s] + (kCoordWords + p * 32) * 4);
-                        logit[s] += fmaf(k, scale_k, x.x * scale_q);      // (the long sum is rounded once an axis)
-                        dp[s] = fmaf(x.y, scale_v, dp[s]);
+                        // (the long sum is rounded once an axis)
+                        logit[s] += kScaled ? fmaf(k, scale_k, x.x * scale_q) : k + x.x;
+                        dp[s] = kScaled ? fmaf(x.y, scale_v, dp[s]) : dp[s] + x.y;
                     });
                 }
             };
@@ -330,12 +317,9 @@ int launch_records(const BwdTileArgs &b0, hipStream_t stream)
 // row, first pair and coordinates of the units' columns
 size_t columns_bytes(int64_t N, int nd) { return align_up(sizeof(int32_t) * list_max_units(N) * kCols * (2 + static_cast<size_t>(nd)), 256); }
 
-// tables as operands, at most 48 bytes a lane, and their scales
-size_t operand_bytes(int H, int nd)
-{
-    return align_up(sizeof(Operand<float>) * static_cast<size_t>(H) * 3 * (3 + (nd - 3 + 1) / 2) * 128, 256) +
-           align_up(sizeof(float) * 3 * static_cast<size_t>(H), 256);
-}
+// tables as operands
+size_t operand_bytes(int H, int nd) { return align_up(sizeof(Operand<float>) * static_cast<size_t>(H) * 3 * (3 + (nd - 3 + 1) / 2) * 128, 256); }
+size_t scales_bytes(int H) { return align_up(sizeof(float) * 3 * static_cast<size_t>(H), 256); }
 
 }  // namespace
 }  // namespace tile
@@ -349,11 +333,17 @@ bool attn_tile_bwd_applies(const int32_t *rows, int nd, int D, int64_t pairs)
     return D == 16 && pairs > 0 && pairs < (int64_t(1) << 31) && rows_fit_tiles(rows, nd);
 }
 
+// Where strips leave the records: fp16 features, windows of some size (a strip is of one window).  Strips over tiles, forward
+// included, layers of 60,000 to 100,000 voxels: 1.26 to 1.32 with windows of 4, 0.99 to 1.04 of 10, 0.91 to 0.95 of 17, 0.92 to 0.96
+// of 26 to 72; fp32 see above.
+constexpr int64_t kStripRecordsMeanWindow = 14;
+
+// records | slots | lists | strips and their columns | scales | what the kernel that leaves the records has
 size_t attn_tile_bwd_bytes(int H, int nd, int64_t N, int64_t W, int64_t pairs)
 {
-    return align_up(sizeof(float2) * static_cast<size_t>(H) * pairs, 256) + tile::strip_slots_bytes(H, nd) +
-           tile::operand_bytes(H, nd) + tile::columns_bytes(N, nd) + tile::list_bytes(N, W) + tile::strips_bytes(N) +
-           tile::strip_columns_bytes(N);
+    return align_up(sizeof(float2) * static_cast<size_t>(H) * pairs, 256) + tile::strip_slots_bytes(H, nd) + tile::list_bytes(N, W) +
+           tile::strips_bytes(N) + tile::strip_columns_bytes(N) + tile::scales_bytes(H) +
+           std::max(tile::operand_bytes(H, nd) + tile::columns_bytes(N, nd), tile::strip_records_bytes(H, nd, N, W));
 }
 
 int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, float *dtk, float *dtv, void *workspace, int dtype,
@@ -367,31 +357,37 @@ int launch_attn_tile_bwd(const BwdPairArgs &p, const void *out, float *dtq, floa
     at += align_up(sizeof(float2) * static_cast<size_t>(H) * p.pairs, 256);
     float *slots = reinterpret_cast<float *>(at);
     at += tile::strip_slots_bytes(H, nd);
-    b.operands = at;
-    at += tile::operand_bytes(H, nd);
-    b.scales = reinterpret_cast<float *>(at - align_up(sizeof(float) * 3 * static_cast<size_t>(H), 256));
-    const size_t columns = tile::list_max_units(p.f.N) * tile::kCols;
-    b.rows = reinterpret_cast<int32_t *>(at);
-    b.first_pair = b.rows + columns;
-    b.coords = reinterpret_cast<float *>(b.first_pair + columns);
-    at += tile::columns_bytes(p.f.N, nd);
     b.list = tile::list_at(at, p.f.N, p.f.W);
-    b.list.strips = reinterpret_cast<const int4 *>(at + tile::list_bytes(p.f.N, p.f.W));
-    b.strip_columns = reinterpret_cast<int4 *>(at + tile::list_bytes(p.f.N, p.f.W) + tile::strips_bytes(p.f.N));
+    at += tile::list_bytes(p.f.N, p.f.W);
+    b.list.strips = reinterpret_cast<const int4 *>(at);
+    at += tile::strips_bytes(p.f.N);
+    b.strip_columns = reinterpret_cast<int4 *>(at);
     b.strip_rows = reinterpret_cast<int32_t *>(b.strip_columns + tile::kStrip * tile::list_max_strips(p.f.N));
+    at += tile::strip_columns_bytes(p.f.N);
+    b.scales = reinterpret_cast<float *>(at);
+    at += tile::scales_bytes(H);
     b.dout = p.dout;
     b.out = out;
     b.stat_max = p.stat_max;
     b.stat_sum = p.stat_sum;
     b.pairs = p.pairs;
     int rc = fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: %d axes in the tile form", nd);
+    if (dtype == S3D_DTYPE_F32 || p.f.N < kStripRecordsMeanWindow * p.f.W) {
+        b.operands = at;
+        const size_t columns = tile::list_max_units(p.f.N) * tile::kCols;
+        b.rows = reinterpret_cast<int32_t *>(at + tile::operand_bytes(H, nd));
+        b.first_pair = b.rows + columns;
+        b.coords = reinterpret_cast<float *>(b.first_pair + columns);
 #define S3D_CASE(NN)                                                                                           \
     if (nd == NN)                                                                                              \
         rc = dtype == S3D_DTYPE_F32   ? tile::launch_records<float, float, NN>(b, stream)                      \
              : dtype == S3D_DTYPE_F16 ? tile::launch_records<__half, __half, NN>(b, stream)                    \
                                       : tile::launch_records<float, __half, NN>(b, stream);
-    S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
+        S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
 #undef S3D_CASE
+    } else {
+        rc = tile::launch_strip_records(b, at, dtype, stream);
+    }
     if (rc) return rc;
     tile::StripArgs g{};
     g.f = p.f;
