@@ -24,13 +24,16 @@ struct LinearGrad {
     int64_t M;
     int32_t N, K, scaled;
     float scale;
+    const float *parts = nullptr;   // where launch_linear_grad_parts has put them, and how many
+    int32_t splits = 0;
 };
 
 constexpr int kMostLinearGrads = 4;
+// room for the parts of `num` layers, however they are grouped
 size_t linear_grads_bytes(const LinearGrad *grads, int num);
-int launch_linear_grad_parts(const LinearGrad &g, float *parts, hipStream_t stream);
-// the sums of the parts of `num` layers in one launch; parts: where linear_grads_bytes has them, one layer behind the other
-int launch_linear_grad_sums(const LinearGrad *grads, int num, float *parts, int32_t grad_dtype, hipStream_t stream);
-size_t linear_grad_part_count(const LinearGrad &g);
+// the parts of `num` layers of as many rows, to *parts and on, which is moved behind them
+int launch_linear_grad_parts(LinearGrad *grads, int num, float **parts, hipStream_t stream);
+// the sums of the parts of `num` layers in one launch
+int launch_linear_grad_sums(const LinearGrad *grads, int num, int32_t grad_dtype, hipStream_t stream);
 
 }  // namespace s3d

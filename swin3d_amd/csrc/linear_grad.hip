@@ -34,18 +34,34 @@ __device__ __forceinline__ int placed(int c, int p) { return c * kOctets + (p ^ 
 struct GradArgs {
     const _Float16 *dy, *x;   // [M,N], [M,K]
     float *parts;             // [splits][N K + N]
-    int64_t M, rows;          // rows of a split: a multiple of kRows
+    int64_t M, rows, chain;   // rows of a split, and of a chain of additions in it: multiples of kRows
     int N, K, tiles_k;
 };
 
-// 2 x 2 wavefronts of UN x UK products of 16 x 16: a tile of 32 UN columns of dY by 32 UK columns of X
-template <int UN, int UK>
-__global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
+// Layers of as many rows and the same tiles share a launch
+struct GradGroup {
+    GradArgs of[kMostLinearGrads];
+    int first[kMostLinearGrads];      // the first tile of each
+};
+
+// 2 x 2 wavefronts of UN x UK products of 16 x 16: a tile of 32 UN columns of dY by 32 UK columns of X.  kChains: the sum over
+// the rows is one of chains, as long as the parts of the layer by itself (one chain for twice the rows has 1.2 to 1.4 times the
+// error against 64 bits).
+template <int UN, int UK, bool kChains>
+__global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradGroup group)
 {
+    GradArgs a = group.of[0];
+    int first = 0;
+#pragma unroll
+    for (int i = 1; i < kMostLinearGrads; ++i) {
+        if (static_cast<int>(blockIdx.x) < group.first[i]) continue;
+        a = group.of[i];
+        first = group.first[i];
+    }
     constexpr int kN = 32 * UN, kK = 32 * UK;
     static_assert(kN + kK <= kThreads, "a thread turns one block of a chunk");
     __shared__ uint4 staged[2][(kN + kK) * kOctets];
-    const int n0 = static_cast<int>(blockIdx.x) / a.tiles_k * kN, k0 = static_cast<int>(blockIdx.x) % a.tiles_k * kK;
+    const int tile = static_cast<int>(blockIdx.x) - first, n0 = tile / a.tiles_k * kN, k0 = tile % a.tiles_k * kK;
     const int64_t begin = static_cast<int64_t>(blockIdx.y) * a.rows, end = min(begin + a.rows, a.M);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_n = wave % 2 * (16 * UN), wave_k = wave / 2 * (16 * UK);
@@ -82,7 +98,19 @@ __global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
             to[placed(column + 2 * w + 1, octet)] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
         }
     };
-    f32x4 acc[UN][UK] = {}, sums[UN] = {};
+    f32x4 acc[UN][UK] = {}, sums[UN] = {}, total[UN][UK] = {}, total_sums[UN] = {};
+    auto end_chain = [&]() {
+#pragma unroll
+        for (int i = 0; i < UN; ++i) {
+#pragma unroll
+            for (int j = 0; j < UK; ++j) {
+                total[i][j] += acc[i][j];
+                acc[i][j] = f32x4{};
+            }
+            total_sums[i] += sums[i];
+            sums[i] = f32x4{};
+        }
+    };
     const bool sum_dy = k0 == 0 && wave_k == 0;
     half8 ones;
 #pragma unroll
@@ -112,13 +140,19 @@ __global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
     put(staged[0]);
     __syncthreads();
     int buffer = 0;
+    int64_t next_chain = begin + a.chain;
     for (int64_t row = begin; row < end; row += kRows, buffer ^= 1) {
+        if (kChains && row == next_chain) {
+            end_chain();
+            next_chain += a.chain;
+        }
         const bool more = row + kRows < end;      // (the same for the whole workgroup)
         if (more) fetch(row + kRows);
         multiply(staged[buffer]);
         if (more) put(staged[buffer ^ 1]);
         __syncthreads();
     }
+    if (kChains) end_chain();
     float *part = a.parts + static_cast<int64_t>(blockIdx.y) * (static_cast<int64_t>(a.N) * a.K + a.N);
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
@@ -127,9 +161,9 @@ __global__ __launch_bounds__(kThreads, 2) void linear_grad_kernel(GradArgs a)
 #pragma unroll
         for (int j = 0; j < UK; ++j) {
             const int k = k0 + wave_k + 16 * j + 4 * quarter;
-            if (k < a.K) *reinterpret_cast<f32x4 *>(part + static_cast<int64_t>(n) * a.K + k) = acc[i][j];
+            if (k < a.K) *reinterpret_cast<f32x4 *>(part + static_cast<int64_t>(n) * a.K + k) = kChains ? total[i][j] : acc[i][j];
         }
-        if (sum_dy && quarter == 0) part[static_cast<int64_t>(a.N) * a.K + n] = sums[i][0];
+        if (sum_dy && quarter == 0) part[static_cast<int64_t>(a.N) * a.K + n] = kChains ? total_sums[i][0] : sums[i][0];
     }
 }
 
@@ -142,12 +176,26 @@ struct GradSums {
     float scale[kMostLinearGrads];
 };
 
-// The sum of the parts: 64 numbers a workgroup, its four wavefronts share the parts.  Several layers share a launch: the sums
+// Four results to where they fit in one piece, which a gradient inside a larger buffer may not
+template <typename T> __device__ __forceinline__ void store_four(T *to, const f32x4 &v)
+{
+    typedef T four __attribute__((ext_vector_type(4)));
+    if (reinterpret_cast<uintptr_t>(to) % sizeof(four) == 0) {
+        *reinterpret_cast<four *>(to) = four{static_cast<T>(v[0]), static_cast<T>(v[1]), static_cast<T>(v[2]), static_cast<T>(v[3])};
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) to[i] = static_cast<T>(v[i]);
+    }
+}
+
+// The sum of the parts: 256 numbers a workgroup, its four wavefronts share the parts.  Several layers share a launch: the sums
 // of a Swin block's four are 5 us each by themselves, for some 20 MB of parts.
+// With 16-byte loads, where they were 4 bytes, and half the parts (launch_linear_grad_parts), us a block: 96 channels, 50,000 rows, 15 / 10; 192,
+// 12,400, 16 / 8; 384, 3,000, 21 / 9; 384, 811, 17.5 / 7.5 (35 MB).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(GradSums a)
 {
-    __shared__ float shared[kThreads];
+    __shared__ f32x4 shared[kThreads];
     int at = 0;
 #pragma unroll
     for (int i = 1; i < kMostLinearGrads; ++i) at = static_cast<int>(blockIdx.x) >= a.first[i] ? i : at;
@@ -164,70 +212,140 @@ __global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(GradSums a)
     }
     const int64_t total = products + n;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t e = (static_cast<int64_t>(blockIdx.x) - first) * 64 + lane, from = min(e, total - 1);
-    float sum = 0.0f;
+    // (N and K are multiples of 8: four numbers are of one row, and of the weight or of the bias)
+    const int64_t e = (static_cast<int64_t>(blockIdx.x) - first) * 256 + 4 * lane, from = min(e, total - 4);
+    f32x4 sum = {};
 #pragma unroll 8
-    for (int s = wave; s < splits; s += 4) sum += parts[s * total + from];
+    for (int s = wave; s < splits; s += 4) sum += *reinterpret_cast<const f32x4 *>(parts + s * total + from);
     shared[threadIdx.x] = sum;
     __syncthreads();
     if (wave > 0 || e >= total) return;
     sum = (shared[lane] + shared[lane + 64]) + (shared[lane + 128] + shared[lane + 192]);
     if (e < products) {
         if (e < static_cast<int64_t>(scaled) * k) sum *= scale;
-        if (dw) dw[e] = static_cast<T>(sum);
+        if (dw) store_four(dw + e, sum);
     } else if (db) {
-        if (e - products < scaled) sum *= scale;
-        db[e - products] = static_cast<T>(sum);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (e - products + i < scaled) sum[i] *= scale;
+        store_four(db + (e - products), sum);
     }
 }
 
-struct Split {
-    int un, uk, tiles, tiles_k, count;
-    int64_t rows;
+// Per side the tile of 64 or 96 columns that pads least (96 for equals: fewer reads of the other side).
+struct Tiles {
+    int un, uk, count, along_k;
 };
 
-// Per side the tile of 64 or 96 columns that pads least (96 for equals: fewer reads of the other side), and as many parts
-// of the rows as give every CU two workgroups, but none of fewer than 256 rows: a part is written and read in fp32, which
-// for a tile of 96 x 96 is as much traffic as 192 rows of its operands.
-Split split_of(int64_t M, int N, int K)
+Tiles tiles_of(int N, int K)
 {
     auto units = [](int width) { return (width + 95) / 96 * 96 <= (width + 63) / 64 * 64 ? 3 : 2; };
-    Split s{units(N), units(K), 0, 0, 0, 0};
-    s.tiles_k = (K + 32 * s.uk - 1) / (32 * s.uk);
-    s.tiles = (N + 32 * s.un - 1) / (32 * s.un) * s.tiles_k;
-    const int64_t most = ceil_div(M, 256), wanted = ceil_div(512, s.tiles);
-    s.rows = ceil_div(ceil_div(M, most < wanted ? most : wanted), kRows) * kRows;
-    s.count = static_cast<int>(ceil_div(M, s.rows));
-    return s;
+    Tiles t{units(N), units(K), 0, 0};
+    t.along_k = (K + 32 * t.uk - 1) / (32 * t.uk);
+    t.count = (N + 32 * t.un - 1) / (32 * t.un) * t.along_k;
+    return t;
+}
+
+// As many parts of the rows as give every CU two workgroups, but none of fewer than 256 rows: a part is written and read in
+// fp32, which for a tile of 96 x 96 is as much traffic as 192 rows of its operands.  More tiles never make more parts.
+struct Split {
+    int64_t rows;
+    int count;
+};
+
+Split split_of(int64_t M, int tiles)
+{
+    const int64_t most = ceil_div(M, 256), wanted = ceil_div(512, tiles);
+    const int64_t rows = ceil_div(ceil_div(M, most < wanted ? most : wanted), kRows) * kRows;
+    return {rows, static_cast<int>(ceil_div(M, rows))};
 }
 
 bool fits(int64_t M, int32_t N, int32_t K) { return M > 0 && M <= 0x7fffffff && N >= 8 && N % 8 == 0 && K >= 8 && K % 8 == 0 && N <= 16384 && K <= 16384; }
 
 }  // namespace
 
-size_t linear_grad_part_count(const LinearGrad &g) { return static_cast<size_t>(split_of(g.M, g.N, g.K).count) * (static_cast<size_t>(g.N) * g.K + g.N); }
-
 size_t linear_grads_bytes(const LinearGrad *grads, int num)
 {
     size_t count = 0;
-    for (int i = 0; i < num; ++i) count += linear_grad_part_count(grads[i]);
+    for (int i = 0; i < num; ++i)
+        count += static_cast<size_t>(split_of(grads[i].M, tiles_of(grads[i].N, grads[i].K).count).count) *
+                 (static_cast<size_t>(grads[i].N) * grads[i].K + grads[i].N);
     return count * sizeof(float);
 }
 
-int launch_linear_grad_parts(const LinearGrad &g, float *parts, hipStream_t stream)
+namespace {
+
+template <int UN, int UK> int launch_group(const GradGroup &group, int tiles, int splits, bool chains, hipStream_t stream)
 {
-    if (!fits(g.M, g.N, g.K))
-        return fail(S3D_ERR_BAD_SHAPE, "s3d_linear_grad: M=%lld N=%d K=%d (N and K multiples of 8, at most 16384)", (long long)g.M, g.N, g.K);
-    const Split split = split_of(g.M, g.N, g.K);
-    const GradArgs args{static_cast<const _Float16 *>(g.dy), static_cast<const _Float16 *>(g.x), parts, g.M, split.rows, g.N, g.K, split.tiles_k};
-    auto kernel = split.un == 3 ? (split.uk == 3 ? linear_grad_kernel<3, 3> : linear_grad_kernel<3, 2>)
-                                : (split.uk == 3 ? linear_grad_kernel<2, 3> : linear_grad_kernel<2, 2>);
-    hipLaunchKernelGGL(kernel, dim3(split.tiles, split.count), dim3(kThreads), 0, stream, args);
+    if (chains)
+        hipLaunchKernelGGL((linear_grad_kernel<UN, UK, true>), dim3(tiles, splits), dim3(kThreads), 0, stream, group);
+    else
+        hipLaunchKernelGGL((linear_grad_kernel<UN, UK, false>), dim3(tiles, splits), dim3(kThreads), 0, stream, group);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
 
-int launch_linear_grad_sums(const LinearGrad *grads, int num, float *parts, int32_t grad_dtype, hipStream_t stream)
+// the layers of `which` (bits), whose tiles are the same, in one launch
+int launch_some(LinearGrad *grads, int num, unsigned which, float **parts, hipStream_t stream)
+{
+    int tiles = 0, at = 0;
+    for (int i = 0; i < num; ++i)
+        if (which >> i & 1) tiles += tiles_of(grads[i].N, grads[i].K).count;
+    const Split split = split_of(grads[0].M, tiles);
+    GradGroup group{};
+    Tiles t{};
+    bool chains = false;
+    for (int i = 0, first = 0; i < num; ++i) {
+        if (!(which >> i & 1)) continue;
+        LinearGrad &g = grads[i];
+        t = tiles_of(g.N, g.K);
+        const int64_t chain = split_of(g.M, t.count).rows;
+        chains = chains || chain < split.rows;
+        group.of[at] = {static_cast<const _Float16 *>(g.dy), static_cast<const _Float16 *>(g.x), *parts, g.M, split.rows, chain, g.N, g.K, t.along_k};
+        group.first[at++] = first;
+        first += t.count;
+        g.parts = *parts;
+        g.splits = split.count;
+        *parts += static_cast<size_t>(split.count) * (static_cast<size_t>(g.N) * g.K + g.N);
+    }
+    for (; at < kMostLinearGrads; ++at) group.first[at] = 0x7fffffff;
+    return t.un == 3 ? (t.uk == 3 ? launch_group<3, 3>(group, tiles, split.count, chains, stream) : launch_group<3, 2>(group, tiles, split.count, chains, stream))
+                     : (t.uk == 3 ? launch_group<2, 3>(group, tiles, split.count, chains, stream) : launch_group<2, 2>(group, tiles, split.count, chains, stream));
+}
+
+}  // namespace
+
+// Layers with the same tiles share a launch as long as that leaves each a part: two have half the parts each, and one beginning
+// and one end.  (Beyond, they have one part or two by themselves, and the registers of chains cost a workgroup a CU: 640 -> 2560
+// and back, 2,300 rows, together 1.3 times as slow.)  The four layers of a Swin block, us for the parts, alone / in pairs: 96
+// channels, 50,000 rows, 62 / 50; 192, 12,400, 59 / 47; 384, 3,000, 51 / 39; 384, 811, 34 / 21.
+int launch_linear_grad_parts(LinearGrad *grads, int num, float **parts, hipStream_t stream)
+{
+    unsigned left = 0;
+    for (int i = 0; i < num; ++i) {
+        if (!fits(grads[i].M, grads[i].N, grads[i].K) || grads[i].M != grads[0].M)
+            return fail(S3D_ERR_BAD_SHAPE, "s3d_linear_grad: M=%lld N=%d K=%d (N and K multiples of 8, at most 16384)", (long long)grads[i].M,
+                        grads[i].N, grads[i].K);
+        left |= 1u << i;
+    }
+    for (int i = 0; i < num; ++i) {
+        if (!(left >> i & 1)) continue;
+        const Tiles t = tiles_of(grads[i].N, grads[i].K);
+        unsigned which = 1u << i;
+        int tiles = t.count;
+        for (int j = i + 1; j < num; ++j) {
+            const Tiles other = tiles_of(grads[j].N, grads[j].K);
+            if (other.un != t.un || other.uk != t.uk || tiles + other.count > 512) continue;
+            which |= 1u << j;
+            tiles += other.count;
+        }
+        left &= ~which;
+        if (int rc = launch_some(grads, num, which, parts, stream)) return rc;
+    }
+    return S3D_OK;
+}
+
+int launch_linear_grad_sums(const LinearGrad *grads, int num, int32_t grad_dtype, hipStream_t stream)
 {
     GradSums a{};
     int64_t blocks = 0;
@@ -235,18 +353,17 @@ int launch_linear_grad_sums(const LinearGrad *grads, int num, float *parts, int3
         a.first[i] = 0x7fffffff;
         if (i >= num) continue;
         const LinearGrad &g = grads[i];
-        a.parts[i] = parts;
+        a.parts[i] = g.parts;
         a.dw[i] = g.dw;
         a.db[i] = g.db;
         a.products[i] = static_cast<int64_t>(g.N) * g.K;
         a.n[i] = g.N;
         a.k[i] = g.K;
-        a.splits[i] = split_of(g.M, g.N, g.K).count;
+        a.splits[i] = g.splits;
         a.scaled[i] = g.scaled;
         a.scale[i] = g.scale;
         a.first[i] = static_cast<int>(blocks);
-        blocks += ceil_div(a.products[i] + g.N, 64);      // (at most 2^22 + 256 a layer)
-        parts += linear_grad_part_count(g);
+        blocks += ceil_div(a.products[i] + g.N, 256);      // (at most 2^20 + 64 a layer)
     }
     if (grad_dtype == S3D_DTYPE_F32)
         hipLaunchKernelGGL(linear_grad_sum_kernel<float>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, a);
@@ -262,7 +379,8 @@ extern "C" __attribute__((visibility("default"))) size_t s3d_linear_grad_workspa
 {
     using namespace s3d;
     if (!fits(M, N, K)) return 0;
-    return static_cast<size_t>(split_of(M, N, K).count) * (static_cast<size_t>(N) * K + N) * sizeof(float);
+    const LinearGrad g{nullptr, nullptr, nullptr, nullptr, M, N, K, 0, 1.0f};
+    return linear_grads_bytes(&g, 1);
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
@@ -279,8 +397,8 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
     if (!workspace || workspace_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_linear_grad: workspace %zu B < required %zu B", workspace ? workspace_bytes : size_t(0), need);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const LinearGrad g{dy, x, dw, db, M, N, K, 0, 1.0f};
+    LinearGrad g{dy, x, dw, db, M, N, K, 0, 1.0f};
     float *parts = static_cast<float *>(workspace);
-    if (int rc = launch_linear_grad_parts(g, parts, s)) return rc;
-    return launch_linear_grad_sums(&g, 1, parts, grad_dtype, s);
+    if (int rc = launch_linear_grad_parts(&g, 1, &parts, s)) return rc;
+    return launch_linear_grad_sums(&g, 1, grad_dtype, s);
 }

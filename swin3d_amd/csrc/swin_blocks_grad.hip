@@ -5,8 +5,8 @@
 // some twenty nodes and fifty dispatches (0.57 ms a block, 15 ms of Swin3D-S's pass), while its kernels take a third of that
 // at 10,000 voxels.  Here the launches follow each other with nothing in between.  And there are fewer of them: the
 // derivative of GELU is taken where fc2's gradient leaves its tile (a launch and two passes over the hidden layer less),
-// dq, dk, dv are written where the projection's gradient reads them (no stacking copy), and the parts of the four
-// layers' weight gradients are summed by one launch.
+// dq, dk, dv are written where the projection's gradient reads them (no stacking copy), the parts of two
+// layers' weight gradients come from one launch where their tiles are the same, and those of all four are summed by one.
 #include "linear.h"
 
 namespace s3d {
@@ -90,31 +90,33 @@ extern "C" __attribute__((visibility("default"))) int s3d_swin_block_grad(
     float *parts = reinterpret_cast<float *>(base + p.parts);
     const size_t rest_bytes = p.total - p.rest, row = static_cast<size_t>(C) * 2;
     LinearGrad wanted[kMostLinearGrads];
-    int num = 0;
-    float *next = parts;
-    // the parts of a layer's weight and bias gradients, where they are wanted
+    int num = 0, launched = 0;
+    // the parts of a layer's weight and bias gradients, where they are wanted: with those of the layer behind it, in one launch
     auto layer = [&](const void *dy, const void *x, float *dw, float *db, int32_t n, int32_t k, int32_t scaled, float scale) {
-        if (!dw && !db) return static_cast<int>(S3D_OK);
-        wanted[num] = LinearGrad{dy, x, dw, db, N, n, k, scaled, scale};
-        const int rc = launch_linear_grad_parts(wanted[num], next, s);
-        next += linear_grad_part_count(wanted[num++]);
+        if (dw || db) wanted[num++] = LinearGrad{dy, x, dw, db, N, n, k, scaled, scale};
+    };
+    auto launch_parts = [&]() {
+        const int rc = launch_linear_grad_parts(wanted + launched, num - launched, &parts, s);
+        launched = num;
         return rc;
     };
-    if (int rc = layer(dpending, b.hidden_out, g.fc2_weight, g.fc2_bias, C, hidden, 0, 1.0f)) return rc;
+    layer(dpending, b.hidden_out, g.fc2_weight, g.fc2_bias, C, hidden, 0, 1.0f);
     if (int rc = launch_linear({dpending, b.fc2_weight_t, nullptr, wide, N, hidden, C, false, b.hidden_in}, s)) return rc;
-    if (int rc = layer(wide, b.normed2, g.fc1_weight, g.fc1_bias, hidden, C, 0, 1.0f)) return rc;
+    layer(wide, b.normed2, g.fc1_weight, g.fc1_bias, hidden, C, 0, 1.0f);
+    if (int rc = launch_parts()) return rc;
     if (int rc = launch_linear({wide, b.fc1_weight_t, nullptr, normed, N, C, hidden, false}, s)) return rc;
     if (int rc = s3d_layernorm_grad(b.sum, dsum, normed, b.norm2_weight, b.norm2_eps, g.x, residual, g.norm2_weight, g.norm2_bias, N, C,
                                     rest, rest_bytes, stream))
         return rc;
-    if (int rc = layer(residual, b.attended, g.proj_weight, g.proj_bias, C, C, 0, 1.0f)) return rc;
+    layer(residual, b.attended, g.proj_weight, g.proj_bias, C, C, 0, 1.0f);
     if (int rc = launch_linear({residual, b.proj_weight_t, nullptr, normed, N, C, C, false}, s)) return rc;
     const char *qkv = static_cast<const char *>(b.qkv);
     if (int rc = s3d_attn_bwd_strided(qkv, qkv + row, qkv + 2 * row, b.table_q, b.table_k, b.table_v, table_sizes, nd, table_len, b.w_sizes,
                                       b.w2n, b.n2n, b.n_coords, b.attended, b.out_max, b.out_sum, normed, wide, wide + row, wide + 2 * row,
                                       g.table_q, g.table_k, g.table_v, N, H, D, W, pairs, 3 * C, 3 * C, dtype, rest, rest_bytes, stream))
         return rc;
-    if (int rc = layer(wide, b.normed1, g.qkv_weight, g.qkv_bias, 3 * C, C, C, q_scale)) return rc;
+    layer(wide, b.normed1, g.qkv_weight, g.qkv_bias, 3 * C, C, C, q_scale);
+    if (int rc = launch_parts()) return rc;
     if (int rc = launch_linear({wide, b.qkv_weight_t, nullptr, g.normed1, N, C, 3 * C, false}, s)) return rc;
-    return num > 0 ? launch_linear_grad_sums(wanted, num, parts, S3D_DTYPE_F32, s) : S3D_OK;
+    return num > 0 ? launch_linear_grad_sums(wanted, num, S3D_DTYPE_F32, s) : S3D_OK;
 }

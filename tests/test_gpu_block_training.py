@@ -102,6 +102,13 @@ def test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads,
         assert (g - w).double().norm() <= 2 ** -11 * w.double().norm() + 1e-12
 
 
+@pytest.mark.parametrize("voxels,channels,heads,mode,without", [
+    (12_011, 192, 12, 1, "nothing"), (3000, 384, 24, 1, "some gradients"),      # pairs of fewer parts, in chains; pairs and single ones
+    (2999, 640, 40, 1, "nothing"), (4000, 144, 9, 2, "biases")])                # too many tiles for pairs; only some have the same tiles
+def test_layers_that_share_a_launch(hip_lib, monkeypatch, voxels, channels, heads, mode, without):
+    test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads, 5, mode, "XYZ_RGB_NORM", without)
+
+
 def test_gradients_of_gradients_and_absent_ones(hip_lib, monkeypatch):
     stage, feats, run = _stage(900, 48, 3, 5, 2, "XYZ_RGB_NORM", seed=3)
     feats.requires_grad_()

@@ -33,6 +33,23 @@ def test_weight_gradients(hip_lib, m, n, k, dtype):
     assert torch.equal(_weight_gradients(dy, x, True, False, dtype)[0], dw)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 8, 16), (700, 48, 72), (3100, 384, 96)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_gradients_inside_a_larger_buffer(hip_lib, m, n, k, dtype):
+    """Wherever they lie the same bits, and nothing around them is written."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    dy, x = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, n), (m, k)))
+    dw, db = _weight_gradients(dy, x, True, True, dtype)
+    ws = torch.empty(hip_lib.s3d_linear_grad_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    for offset in (0, 1, 2, 3):
+        buffer = torch.full((n * k + n + 8,), -50000.0, dtype=dtype, device="cuda")
+        inside = buffer[offset:offset + n * k], buffer[offset + n * k + 1:offset + n * k + 1 + n]
+        assert hip_lib.s3d_linear_grad(dy.data_ptr(), x.data_ptr(), inside[0].data_ptr(), inside[1].data_ptr(), 0 if dtype == torch.float32 else 1,
+                                       m, n, k, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(inside[0].view(n, k), dw) and torch.equal(inside[1], db)
+        assert int((buffer == buffer[-1]).sum()) == 8
+
+
 def test_weight_gradients_show_what_is_not_finite(hip_lib):
     dy, x = torch.ones(300, 48, device="cuda").half(), torch.ones(300, 64, device="cuda").half()
     dy[123, 5], x[7, 9] = float("inf"), float("nan")
