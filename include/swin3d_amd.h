@@ -191,9 +191,11 @@ int s3d_attn_fwd_noalloc(const void *q, const void *k, const void *v, const void
  *   pairs          M = sum of w_sizes^2, the pairs of the window set (counts[1] of s3d_window_index; the length
  *                  of the reference's index arrays), or 0.  With M the call runs two pair sweeps on the forward's
  *                  kind of work list (dq, which leaves dL and P of every (pair, head) in the workspace, 8 * H * pairs
- *                  bytes; dk and dv, which reads them), and two table-gradient sweeps that read them too; at head_dim 16 with tables of at most 64 rows on a position axis and 32 on a signal
- *                  axis tiles of 64 queries by 64 keys leave dL and P, and strips of 16 voxels with all their pairs give
- *                  all six gradients by matrix products.  With 0 it runs two fused
+ *                  bytes; dk and dv, which reads them), and two table-gradient sweeps that read them too; with tables of at
+ *                  most 64 rows on a position axis and 32 on a signal axis strips of 16 voxels with all their pairs give
+ *                  all six gradients by matrix products instead: at head_dim 16, where strips leave dL and P too (tiles of
+ *                  64 queries by 64 keys in fp32 and where the mean window has fewer than 14 voxels), and at head_dim 8,
+ *                  where the first pair sweep does, but for the largest launches in fp32 and with three axes.  With 0 it runs two fused
  *                  sweeps that recompute the logits for the table gradients and need no such store (about a third
  *                  more time).  A value below M cannot hold the records of every window: the rows of dq, dk, dv
  *                  that belong to the windows beyond it and all three table gradients then come out as NaN.

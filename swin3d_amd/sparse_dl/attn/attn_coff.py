@@ -303,8 +303,8 @@ def window_attention_backward(q, k, v, table_q, table_k, table_v, table_sizes, w
 
     pairs: M = sum(w_sizes^2) of the window set (the reference's index arrays have this length,
     swin3d_layers.py:96-103); None = read it from w_sizes once and keep it on that tensor.  With it the library
-    runs the pair sweeps, or at head_dim 16 the tile kernels, which keep dL and P of every (pair, head) in the workspace
-    (8 bytes); 0, or a
+    runs the strip kernels, or the pair sweeps where those do not apply, which keep dL and P of every (pair, head) in the
+    workspace (8 bytes); 0, or a
     store above BWD_PAIR_STORE_MAX_BYTES, selects the fused sweeps, which need no such store and take about a
     third longer.  head_dim 32 and tables of more than BWD_MAX_ROWS_PER_AXIS rows per axis on average run in the
     library's general form (atomic adds, as the reference works): correct, some fifty times slower per pair."""
