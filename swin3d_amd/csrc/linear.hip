@@ -10,8 +10,8 @@
 //
 // At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 173 us against
 // 416 us as product and GELU apart; 80 -> 240, 108 us against 207, at 3.6 of the 4.7 TB/s that a copy reaches.  At the
-// deepest the tiles are few and a tile's chain of chunks is what counts: 811 rows, 384 -> 384, 5 us against 18 through
-// torch, whose launch alone takes the host that long.
+// deepest the tiles are few and a tile's chain of chunks is what counts (linear_thin_kernel): 390 rows, 384 -> 384, 3.4 us against 18
+// through torch, whose launch alone takes the host that long.
 #include "attn_kernels.h"
 #include "linear.h"
 
@@ -21,6 +21,7 @@ namespace s3d {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -56,6 +57,13 @@ enum class Behind { kNothing, kGelu, kGeluGrad };
 
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
+
+// between what a wavefront's lanes write to its LDS and what other lanes of it read (it serves a wavefront in order)
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // WM x WN wavefronts of TM x TN products of 32 x 32
 template <int WM, int WN, int TM, int TN> struct Tile {
@@ -233,6 +241,107 @@ int launch(const LinearArgs &a, hipStream_t stream)
     return S3D_OK;
 }
 
+// A tile of 32 x 32 whose chunks are shared by eight wavefronts, wavefront s taking chunks s, s + 8, .. through an LDS buffer of its
+// own (no barrier), two chunks ahead in registers.  The sums meet in LDS.
+//
+// Where tiles of 64 x 64 leave most CUs idle, a launch takes as long as one tile's chain of chunks, 720 clocks each: LDS reads and
+// writes of 48 KB, a barrier, a memory round trip in front of it.  (Four groups of wavefronts on that tile's chunks were 14 % faster
+// at K = 1536: the LDS traffic is the same.)  Here four times as many CUs have a quarter of it each, and a wavefront all its
+// loads under way.  us, tiles of 64 x 64 / so: 390 rows, 1536 -> 384, 10.0 / 5.2; 384 -> 384, 4.5 / 3.4; 390, 2560 -> 640, 22.0 / 9.9;
+// 100, 384 -> 1536 with GELU 4.9 / 3.8; 1,563, 192 -> 192, 3.7 / 3.6.
+constexpr int kShares = 8;
+
+template <Behind kBehind>
+__global__ __launch_bounds__(64 * kShares) void linear_thin_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
+                                                                   const _Float16 *__restrict__ bias, _Float16 *__restrict__ y, int M, int N,
+                                                                   int K, int tiles_n, int tiles)
+{
+    constexpr int kOwn = 2 * 32 * kChunk * 2, kPitch = 32 + 4;
+    static_assert(32 * kPitch * 4 <= kOwn, "a wavefront's sums fit its buffer");
+    __shared__ __align__(16) char smem[kShares * kOwn];
+    // workgroups b, b + 8, .. run on one XCD: they get neighbouring tiles, which share rows of X
+    const int share = (tiles + 7) / 8, tile = static_cast<int>(blockIdx.x) % 8 * share + static_cast<int>(blockIdx.x) / 8;
+    if (tile >= tiles) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, half = lane >> 5;
+    const int m0 = tile / tiles_n * 32, n0 = tile % tiles_n * 32, chunks = (K + kChunk - 1) / kChunk;
+    char *own = smem + wave * kOwn;
+
+    const int piece = lane % kPieces, row = lane / kPieces;      // rows row + 8 i: of X, then of W
+    const _Float16 *from[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = row + 8 * (i % 4);
+        from[i] = (i < 4 ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r, N - 1)) * K) + piece * 8;
+    }
+    f32x16 acc = {};
+    auto fetch = [&](uint4 (&held)[8], int chunk) {
+        if (chunk * kChunk + piece * 8 < K) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) held[i] = *reinterpret_cast<const uint4 *>(from[i] + chunk * kChunk);
+        }
+    };
+    auto multiply = [&](uint4 (&held)[8], int chunk) {
+        uint4 *to = reinterpret_cast<uint4 *>(own);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) to[placed(row + 8 * i, piece)] = held[i];
+        fetch(held, chunk + 2 * kShares);
+        wave_fence();
+        const half8 *at = reinterpret_cast<const half8 *>(own);
+        const int steps = min(K - chunk * kChunk, kChunk) / 16;
+#pragma unroll
+        for (int s = 0; s < kChunk / 16; ++s) {
+            if (s >= steps) break;
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(at[placed(32 + r32, 2 * s + half)], at[placed(r32, 2 * s + half)], acc, 0, 0, 0);
+        }
+        wave_fence();
+    };
+    uint4 first[8], second[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) first[i] = second[i] = make_uint4(0, 0, 0, 0);
+    fetch(first, wave);
+    fetch(second, wave + kShares);
+    const int n = n0 + threadIdx.x % 16 * 2;
+    half2 b = {0, 0};
+    if (bias) b = *reinterpret_cast<const half2 *>(bias + min(n, N - 2));
+    for (int chunk = wave; chunk < chunks; chunk += 2 * kShares) {
+        multiply(first, chunk);
+        if (chunk + kShares < chunks) multiply(second, chunk + kShares);
+    }
+    float *sums = reinterpret_cast<float *>(own);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4 *>(sums + r32 * kPitch + 8 * g + 4 * half) = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+    __syncthreads();
+#pragma unroll
+    for (int r = threadIdx.x / 16; r < 32; r += 4 * kShares) {
+        float v[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < kShares; ++i) {
+            const float2 part = *reinterpret_cast<const float2 *>(smem + i * kOwn + (r * kPitch + threadIdx.x % 16 * 2) * 4);
+            v[0] += part.x;
+            v[1] += part.y;
+        }
+        half2 o;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float z = v[e] + static_cast<float>(b[e]);
+            o[e] = static_cast<_Float16>(kBehind == Behind::kGelu ? gelu(z) : z);
+        }
+        if (m0 + r < M && n < N) *reinterpret_cast<half2 *>(y + static_cast<int64_t>(m0 + r) * N + n) = o;
+    }
+}
+
+int launch_thin(const LinearArgs &a, hipStream_t stream)
+{
+    const int tiles_n = (a.N + 31) / 32, tiles = static_cast<int>(ceil_div(a.M, 32)) * tiles_n;
+    auto kernel = a.gelu ? linear_thin_kernel<Behind::kGelu> : linear_thin_kernel<Behind::kNothing>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ceil_div(tiles, 8) * 8)), dim3(64 * kShares), 0, stream, static_cast<const _Float16 *>(a.x),
+                       static_cast<const _Float16 *>(a.w), static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<int>(a.M), a.N,
+                       a.K, tiles_n, tiles);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
 }  // namespace
 
 int launch_linear(const LinearArgs &a, hipStream_t stream)
@@ -241,6 +350,12 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
         return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M=%lld N=%d K=%d (N a multiple of 8, K of 16)", (long long)a.M, a.N, a.K);
     if (a.M == 0) return S3D_OK;
     if (!a.x || !a.w || !a.y) return fail(S3D_ERR_NULL_POINTER, "s3d_linear: null device pointer");
+    // Tiles of 32 x 32 with K shared as long as each has a CU, or half of one with enough chunks to share, or long chains.  us, 64 x 64 /
+    // so, by tiles of 32 x 32: up to 260, all K, 0.45 to 0.97 of the time; 282 at K = 96 3.3 / 3.6, 441 3.4 / 3.6; 294 to 490 at K = 192 to
+    // 640 0.86 to 1.00; 520 at K = 320 4.8 / 5.8, at 640 5.9 / 6.2, at 2560 23.0 / 13.9; 588 at K = 1536 10.4 / 10.0; 980 at 2560 23.7 / 19.4,
+    // at 640 6.3 / 8.0; 1880 at 2560 27.0 / 35.4.
+    const int64_t thin = ceil_div(a.M, 32) * ((a.N + 31) / 32);
+    if (!a.gelu_at && (thin <= 256 || (thin <= 512 && a.K >= 192) || (thin <= 1024 && a.K >= 2048))) return launch_thin(a, stream);
     // Tiles of 64 x 64 as long as larger ones would leave CUs without work; then 128 rows by the width that pads N least,
     // the widest of those that still give every CU two tiles.  192 columns take all of a wavefront's registers: with GELU only
     // where the tile is the whole row, with its derivative not at all (63 would spill).

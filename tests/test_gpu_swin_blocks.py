@@ -29,6 +29,17 @@ def test_linear(hip_lib, m, n, k, gelu):
         assert bool(((got - want).abs() <= 6e-4 * want.abs() + 2e-6 * float(want.abs().max()) + 6e-7).all())
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 16), (31, 40, 80), (33, 8, 256), (390, 384, 1536),      # tiles of 32 x 32 whose K eight wavefronts share, remainders on every side
+    (256, 1024, 96), (257, 1024, 192), (512, 1024, 192), (513, 1024, 192),      # around 256 and 512 tiles
+    (1024, 1024, 2048), (1025, 1024, 2048), (700, 640, 2560),      # long chains, up to 1024 tiles
+    (100, 136, 528), (64, 96, 1040), (45, 72, 2064),               # a last chunk of 16, chunks that not every wavefront has
+])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_of_few_rows(hip_lib, m, n, k, gelu):
+    test_linear(hip_lib, m, n, k, gelu)
+
+
 def test_gelu_of_every_number(hip_lib):
     """All finite fp16 numbers through the identity: half a place of rounding, and the approximation, which is fp32's own
     rounding and below 2^-25 where the result is too small for fp16."""
