@@ -70,7 +70,8 @@ class _Kept:
 
 def _descriptions(parts, half_copy):
     """The blocks as the library takes them, and the tensors they point to.  half_copy: (layer) -> its (weight, bias) in
-    fp16."""
+    fp16, for parameters that are not copied by one launch."""
+    from .swin_train import packed_copies      # (which reads this module)
     kept, blocks = [], (_lib.SwinBlock * len(parts))()
 
     def at(t):
@@ -79,14 +80,21 @@ def _descriptions(parts, half_copy):
         kept.append(t)
         return t.data_ptr()
 
-    for b, (_, norm1, attn, _, proj, norm2, _, fc1, _, fc2) in zip(blocks, parts):
-        weight, bias, tables = attn._prepared()
-        b.qkv_weight, b.qkv_bias = at(weight.contiguous()), at(bias)
-        b.table_q, b.table_k, b.table_v = (at(t) for t in tables)
-        for name, layer in (("proj", proj), ("fc1", fc1), ("fc2", fc2)):
-            w, bias = half_copy(layer)
-            setattr(b, name + "_weight", at(w.contiguous()))
-            setattr(b, name + "_bias", at(bias))
+    for b, block in zip(blocks, parts):
+        _, norm1, attn, _, proj, norm2, _, fc1, _, fc2 = block
+        packed = packed_copies(block)
+        if packed is not None:
+            kept.append(packed[0])
+            (b.qkv_weight, b.qkv_bias, b.proj_weight, b.proj_bias, b.fc1_weight, b.fc1_bias, b.fc2_weight, b.fc2_bias,
+             b.table_q, b.table_k, b.table_v) = packed[1]
+        else:
+            weight, bias, tables = attn._prepared()
+            b.qkv_weight, b.qkv_bias = at(weight.contiguous()), at(bias)
+            b.table_q, b.table_k, b.table_v = (at(t) for t in tables)
+            for name, layer in (("proj", proj), ("fc1", fc1), ("fc2", fc2)):
+                w, bias = half_copy(layer)
+                setattr(b, name + "_weight", at(w.contiguous()))
+                setattr(b, name + "_bias", at(bias))
         for name, norm in (("norm1", norm1), ("norm2", norm2)):
             setattr(b, name + "_weight", at(norm.weight.detach().float().contiguous()))
             setattr(b, name + "_bias", at(norm.bias.detach().float().contiguous()))

@@ -30,9 +30,10 @@ _GROUPS = ("xyz", "rgb", "norm")
 class _Layout:
     """Where the fp16 copies of a block's parameters lie in one buffer, by the shapes alone: per array (rows, columns) of
     `shapes`, in the order of _parameters.  Every copy of a layer starts on a multiple of 512 bytes, as an allocation of
-    its own would: the library behind torch's products picks kernels by alignment."""
+    its own would: the library behind torch's products picks kernels by alignment.  turned: with transposed copies of the
+    weights, which a backward reads."""
 
-    def __init__(self, shapes, num_tables, scaled_rows, scale, same_tables):
+    def __init__(self, shapes, num_tables, scaled_rows, scale, same_tables, turned=True):
         layers = len(shapes) - num_tables
         self.copies = (_lib.HalfCopy * len(shapes))()
         self.shapes, self.to, self.transposed = shapes, [], []
@@ -41,7 +42,7 @@ class _Layout:
             table = i >= layers
             # (a kind's tables lie one behind the other, as the attention reads them)
             at += 0 if table and (i - layers) % (num_tables // 3) else -at % 256
-            across = not table and cols > 1
+            across = turned and not table and cols > 1
             copy.rows, copy.cols, copy.to = rows, cols, at
             at += rows * cols
             if across:
@@ -57,6 +58,33 @@ class _Layout:
 
 
 _layout = functools.lru_cache(maxsize=64)(_Layout)
+
+
+def _shapes(params):
+    return tuple((p.shape[0], p.shape[1]) if p.dim() == 2 else (p.numel(), 1) for p in params)
+
+
+def packed_copies(parts):
+    """What inference reads of a block's parameters, in fp16 and with the scale of q in, by one launch: the buffer that has
+    them and [address or None of qkv weight, bias, proj .., fc1 .., fc2 .., query, key, value tables] in it; None where they
+    are not plain fp32 arrays.  `parts` has passed _applicable."""
+    attn = parts[2]
+    groups = len(attn.table_sizes) // 3
+    params = _parameters(parts, groups)
+    dev = params[0].device
+    if type(attn.scale) is not float or not params[0].is_cuda or followed() or any(t is None for t in params[8:]) \
+            or any(t is not None and not (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_contiguous()) for t in params):
+        return None
+    given = [p for p in params if p is not None]
+    layout = _layout(_shapes(given), 3 * groups, attn.dim, attn.scale, False, False)
+    half = torch.empty(layout.half_count, dtype=torch.float16, device=dev)
+    with _lib.on(dev):
+        status = _lib.lib().s3d_half_copies((ctypes.c_void_p * len(given))(*[p.data_ptr() for p in given]), layout.copies, len(given),
+                                            half.data_ptr(), None, _lib.stream(dev))
+    _lib.check(status, "s3d_half_copies")
+    base, places = half.data_ptr(), iter(layout.to)
+    layers = [None if p is None else base + 2 * next(places) for p in params[:8]]
+    return half, layers + [base + 2 * at for at in layout.to[-3 * groups::groups]]
 
 
 class _Call:
@@ -178,8 +206,7 @@ class _Branches(Function):
         given = [p for p in params if p is not None]
         num_tables = len(params) - 8
         # (the backward of mode 1 reads the tables in fp32)
-        layout = _layout(tuple((p.shape[0], p.shape[1]) if p.dim() == 2 else (p.numel(), 1) for p in given), num_tables, channels,
-                         call.scale, call.mode == 1)
+        layout = _layout(_shapes(given), num_tables, channels, call.scale, call.mode == 1)
         half = torch.empty(layout.half_count, dtype=torch.float16, device=dev)
         same = torch.empty(layout.same_count, dtype=torch.float32, device=dev) if layout.same_count else None
         lib = _lib.lib()

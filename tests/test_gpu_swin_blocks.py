@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from swin3d_amd import _lib, encoder, synth
+from swin3d_amd import _lib, encoder, swin_train, synth
 from swin3d_amd.swin_blocks import linear_rows
 
 pytestmark = pytest.mark.gpu
@@ -131,3 +131,36 @@ def test_a_precision_set_after_a_call_is_followed(hip_lib):
     del stage._s3d_blocks
     assert torch.equal(got, run())
     assert stage._s3d_blocks.described is None
+
+
+@pytest.mark.parametrize("axes,biases,shifted", [("XYZ_RGB_NORM", True, False), ("XYZ_RGB", False, True), ("XYZ", True, True)])
+def test_parameters_in_one_launch_are_the_layers_copies(hip_lib, monkeypatch, axes, biases, shifted):
+    """The bits of the copies that the layers make one by one; shifted: parameters at odd places of a larger buffer."""
+    dev = torch.device("cuda")
+    scene = synth.make_room((3.0, 3.0, 2.0), 4, 3000, seed=5)
+    coords = torch.from_numpy(scene.coords).to(dev)
+    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)[:, :4 + {"XYZ": 0, "XYZ_RGB": 3}.get(axes, 6)].contiguous()
+    torch.manual_seed(1)
+    stage = encoder.Stage(48, 2, 6, 5, 4, downsample=False, cRSE=axes, fp16_mode=2).to(dev).eval()
+    for name, p in stage.named_parameters():
+        torch.nn.init.normal_(p, std=0.1)
+        if shifted:
+            p.data = torch.cat([p.data.new_zeros(1), p.data.reshape(-1)])[1:].view(p.shape)
+    if not biases:
+        for block in stage.blocks:
+            block.attn.qkv.bias = block.mlp.fc2.bias = None
+    feats, made = torch.randn(coords.shape[0], 48, device=dev), []
+    real = swin_train.packed_copies
+    monkeypatch.setattr(swin_train, "packed_copies", lambda parts: made.append(real(parts)) or made[-1])
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            return stage(encoder.SparseVoxels(coords, feats, 1), signals)[0].feats
+
+    got = run()
+    assert len(made) == 2 and all(m is not None for m in made)
+    run()
+    assert len(made) == 2
+    encoder.drop_inference_copies(stage)
+    monkeypatch.setattr(swin_train, "packed_copies", lambda parts: None)
+    assert torch.equal(run(), got)
