@@ -30,6 +30,12 @@ def test_add_layernorm_matches_torch(hip_lib, channels, res_dtype, out_dtype):
     assert (y.float() - want).abs().max().item() <= tol
 
 
+@pytest.mark.parametrize("channels", [4, 64, 68, 128, 132, 256, 260, 512, 516, 768])      # around the rows' lanes and fours a lane
+@pytest.mark.parametrize("res_dtype", [None, torch.float16, torch.float32])
+def test_add_layernorm_at_the_edges_of_its_rows(hip_lib, channels, res_dtype):
+    test_add_layernorm_matches_torch(hip_lib, channels, res_dtype, torch.float32)
+
+
 def test_inplace_and_empty(hip_lib):
     from swin3d_amd.fused_norm import add_layernorm
     dev = torch.device("cuda")
