@@ -19,10 +19,28 @@ namespace {
 constexpr int kLnThreads = 256;
 constexpr int kMaxChunks = 4;   // float4 chunks per lane: rows of up to 4 * 4 * 64 = 1024 channels
 
+template <int kControl> __device__ __forceinline__ float moved(float v)
+{
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), kControl, 0xf, 0xf, true));
+}
+// The sum over G lanes in all of them, pairs first: within rows of sixteen lanes by moves of the VALU (neighbours, pairs, then the
+// mirror images of eight and of sixteen, whose quads and eights hold the sums already), where a shuffle goes through LDS.  The same sums in the same pairs.  us with
+// shuffles / so: LayerNorm of 390 rows of 384 2.9 / 2.7, of 600 of 640 3.5 / 3.1, of 50,000 of 96 10.7 / 10.6; its gradients, with the
+// sums below in sixteen shares / so, 811 rows of 384 9.8 / 8.1, 3,000 11.2 / 9.5, 50,000 of 96 20.1 / 19.5, 199,327 of 48 30.1 / 28.2.
 template <int G> __device__ __forceinline__ float group_sum(float v)
 {
-#pragma unroll
-    for (int off = 1; off < G; off <<= 1) v += __shfl_xor(v, off, G);
+    v += moved<0xb1>(v);
+    v += moved<0x4e>(v);
+    v += moved<0x141>(v);
+    v += moved<0x140>(v);
+    if (G >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    if (G >= 64) {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
     return v;
 }
 
@@ -30,8 +48,8 @@ template <int G> __device__ __forceinline__ float group_sum(float v)
 //
 // What bounds it: memory for many rows, for few the trips to it, of which there was one for each four and one more for gamma and
 // beta behind the sums.  Now all loads of a row are under way together (lanes without a four read the last one).  us, fp16 residual and
-// result, before / so: 390 rows of 384, 3.3 / 2.9; 600 of 640, 3.8 / 3.5; 50,000 of 96, 11.5 / 10.7; 600,000 of 80, 111 / 107; no residual,
-// 37,000 of 320, 18.5 / 14.5.
+// result, before / so: 390 rows of 384, 3.3 / 2.9 (2.7 with group_sum as it is); 600 of 640, 3.8 / 3.5 (3.1); 50,000 of 96, 11.5 / 10.7;
+// 600,000 of 80, 111 / 107; no residual, 37,000 of 320, 18.5 / 14.5.
 template <int G, int FOURS, int RES, bool OUT16>
 __global__ __launch_bounds__(kLnThreads) void add_layernorm_kernel(const float *x, const void *residual, const float *__restrict__ gamma,
                                                                    const float *__restrict__ beta, float eps, float *x_out, void *y,
@@ -264,21 +282,25 @@ template <int G, int CH> __global__ __launch_bounds__(kLnThreads) void layernorm
     }
 }
 
-// The sum of the parts: 16 numbers a workgroup, sixteen shares of the parts each.
-__global__ __launch_bounds__(kLnThreads) void layernorm_grad_sum_kernel(const float *__restrict__ parts, int count, int C,
-                                                                        float *__restrict__ dgamma, float *__restrict__ dbeta)
+// The sum of the parts: 16 numbers a workgroup, 64 shares of the parts each (sixteen were a chain of eight trips to memory).
+constexpr int kSumThreads = 1024;
+
+__global__ __launch_bounds__(kSumThreads) void layernorm_grad_sum_kernel(const float *__restrict__ parts, int count, int C,
+                                                                         float *__restrict__ dgamma, float *__restrict__ dbeta)
 {
-    __shared__ float shared[kLnThreads];
+    constexpr int kShares = kSumThreads / 16;
+    __shared__ float shared[kSumThreads];
     const int e = threadIdx.x & 15, share = threadIdx.x >> 4, c = static_cast<int>(blockIdx.x) * 16 + e, at = min(c, 2 * C - 1);
     float sum = 0.0f;
 #pragma unroll 8
-    for (int p = share; p < count; p += 16) sum += parts[static_cast<int64_t>(p) * 2 * C + at];
+    for (int p = share; p < count; p += kShares) sum += parts[static_cast<int64_t>(p) * 2 * C + at];
     shared[threadIdx.x] = sum;
-    __syncthreads();
-    if (share > 0 || c >= 2 * C) return;
-    sum = 0.0f;
 #pragma unroll
-    for (int s = 0; s < 16; ++s) sum += shared[16 * s + e];
+    for (int half = kShares / 2; half > 0; half /= 2) {
+        __syncthreads();
+        if (share < half) shared[threadIdx.x] = sum += shared[threadIdx.x + 16 * half];
+    }
+    if (share > 0 || c >= 2 * C) return;
     (c < C ? dgamma[c] : dbeta[c - C]) = sum;
 }
 
@@ -321,7 +343,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_layernorm_grad(
                   : C <= 512 ? layernorm_grad_kernel<64, 2> : layernorm_grad_kernel<64, 4>;
     hipLaunchKernelGGL(kernel, dim3(parts), dim3(kLnThreads), 0, s, args);
     S3D_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(layernorm_grad_sum_kernel, dim3(static_cast<unsigned>(ceil_div(2 * C, 16))), dim3(kLnThreads), 0, s,
+    hipLaunchKernelGGL(layernorm_grad_sum_kernel, dim3(static_cast<unsigned>(ceil_div(2 * C, 16))), dim3(kSumThreads), 0, s,
                        args.parts, parts, C, dgamma, dbeta);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
