@@ -384,6 +384,9 @@ int s3d_gather_rows(const void *from, int64_t n, const int64_t *rows, int64_t M,
                     void *stream);
 /* out int32 [B]: how many of the N ascending batch ids (`stride` apart) are at most b */
 int s3d_segment_ends(const int32_t *batch, int64_t stride, int64_t N, int32_t B, int32_t *out, void *stream);
+/* the same for two columns, out int32 [2][B]: sources and queries of s3d_knn */
+int s3d_segment_ends_of_two(const int32_t *first, int64_t first_stride, int64_t first_N, const int32_t *second, int64_t second_stride,
+                            int64_t second_N, int32_t B, int32_t *out, void *stream);
 /*
  * The next coarser level from a sort of the voxels into its cells: what s3d_cell_representatives gives (pick), the cells'
  * coordinates (int32 [W][4], rounded down to multiples of `step`) and the picked rows' signals (fp32 [W][num_signals]).

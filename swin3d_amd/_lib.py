@@ -81,6 +81,7 @@ SIGNATURES = {
     "s3d_voxel_neighbours_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "s3d_voxel_neighbours": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "s3d_segment_ends": (ctypes.c_int, [_vp, _i64, _i64, _i32, _vp, _vp]),
+    "s3d_segment_ends_of_two": (ctypes.c_int, [_vp, _i64, _i64, _vp, _i64, _i64, _i32, _vp, _vp]),
     "s3d_pool_cells": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _i32, _vp, _i64, _i32, _vp, _vp, _vp, _vp]),
     "s3d_level_signals": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp, _i64, _i32, _i32, ctypes.c_float, ctypes.c_float, _vp, _i64, _vp]),
     "s3d_knn_strided": (ctypes.c_int, [_i32, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i32, _vp, _vp, ctypes.c_float, _vp,

@@ -278,12 +278,28 @@ def pick_cell_representatives(signals, cell_of_row, num_cells):
     return pick
 
 
+def _searchable(batch_column):
+    return batch_column.is_cuda and data_only(batch_column) and batch_column.dtype == torch.int32 and batch_column.dim() == 1 \
+        and batch_column.stride(0) >= 1
+
+
+def segment_offsets_of_two(first, second, num_batches=None):
+    """segment_offsets of two batch columns, by one launch where the library takes both."""
+    if num_batches is None or num_batches < 1 or not (_searchable(first) and _searchable(second)) or first.device != second.device:
+        return segment_offsets(first, num_batches), segment_offsets(second, num_batches)
+    out = torch.empty((2, num_batches), dtype=torch.int32, device=first.device)
+    with _lib.on(first.device):
+        status = _lib.lib().s3d_segment_ends_of_two(first.data_ptr(), first.stride(0), first.shape[0], second.data_ptr(), second.stride(0),
+                                                    second.shape[0], num_batches, out.data_ptr(), _lib.stream(first.device))
+    _lib.check(status, "s3d_segment_ends_of_two")
+    return out[0], out[1]
+
+
 def segment_offsets(batch_column, num_batches=None):
     """cumulative END row of every batch element, int32 (what the KNN op takes).  With `num_batches` given the
     host does not wait for the device (batch ids are ascending: the end of batch b is a binary search)."""
     if num_batches is not None:
-        if batch_column.is_cuda and data_only(batch_column) and batch_column.dtype == torch.int32 and batch_column.dim() == 1 \
-                and batch_column.stride(0) >= 1 and num_batches > 0:
+        if _searchable(batch_column) and num_batches > 0:
             out = torch.empty(num_batches, dtype=torch.int32, device=batch_column.device)
             with _lib.on(batch_column.device):
                 status = _lib.lib().s3d_segment_ends(batch_column.data_ptr(), batch_column.stride(0), batch_column.shape[0], num_batches,
@@ -437,8 +453,8 @@ class GridKNNDownsample(nn.Module):
         pooled = None if cell_index is None else _pool_level(coords, stride * self.factor, signals, cell_index)
         if pooled is not None:
             coarse, coarse_signals = pooled
-            idx, _ = knn_query(self.k, signals[:, 1:4], coarse_signals[:, 1:4], segment_offsets(coords[:, 0], num_batches),
-                               segment_offsets(coarse[:, 0], num_batches), KNN.cell_size, strided=True)
+            idx, _ = knn_query(self.k, signals[:, 1:4], coarse_signals[:, 1:4],
+                               *segment_offsets_of_two(coords[:, 0], coarse[:, 0], num_batches), KNN.cell_size, strided=True)
             return coarse, coarse_signals, idx
         coarse, pick = pool_and_pick(coords, stride, self.factor, signals, cell_index)
         if coords.is_cuda:
@@ -450,8 +466,7 @@ class GridKNNDownsample(nn.Module):
             coarse_signals = signals[pick]
         src_xyz = signals[:, 1:4].contiguous().float()
         qry_xyz = coarse_signals[:, 1:4].contiguous().float()
-        idx, _ = KNN.apply(self.k, src_xyz, qry_xyz, segment_offsets(coords[:, 0], num_batches),
-                           segment_offsets(coarse[:, 0], num_batches))
+        idx, _ = KNN.apply(self.k, src_xyz, qry_xyz, *segment_offsets_of_two(coords[:, 0], coarse[:, 0], num_batches))
         return coarse, coarse_signals, idx
 
     def forward(self, voxels, signals, plan=None, pending=None):
@@ -893,7 +908,7 @@ class Upsample(nn.Module):
         set is the one this level's attention block needs), so that the index is not built a second time.
         num_batches: batch elements of both, where the caller knows it: the host then waits for nothing."""
         skip, coarse = self._norm_linear(self.linear1, voxels_up.feats), self._norm_linear(self.linear2, voxels.feats)
-        ends, ends_up = segment_offsets(voxels.coords[:, 0], num_batches), segment_offsets(voxels_up.coords[:, 0], num_batches)
+        ends, ends_up = segment_offsets_of_two(voxels.coords[:, 0], voxels_up.coords[:, 0], num_batches)
         if _plain_signals(signals, voxels.coords) and _plain_signals(signals_up, voxels_up.coords):
             idx, dist2 = knn_query(self.up_k, signals[:, 1:4], signals_up[:, 1:4], ends, ends_up, KNN.cell_size, strided=True)
             if interpolate_add_applies(idx, dist2, coarse, skip):

@@ -65,6 +65,20 @@ def test_segments_keys_and_rows_apart(hip_lib, n):
             knn_query(3, signals[:, 1:4], signals[:, 1:4], ends, ends)
 
 
+@pytest.mark.parametrize("sizes", [(1, 1), (63, 64), (65, 129), (4096, 4097), (30011, 262_145), (0, 7)])
+@pytest.mark.parametrize("batches", [1, 2, 5, 300])
+def test_ends_of_two_columns(hip_lib, sizes, batches):
+    """Around the sizes where the search takes another step, elements without rows among them, columns of wider rows."""
+    from swin3d_amd import encoder
+    gen = torch.Generator().manual_seed(sizes[1] + batches)
+    columns = [torch.randint(0, max(1, batches - 1), (n, 1 + i), generator=gen, dtype=torch.int32).sort(0)[0].cuda() for i, n in enumerate(sizes)]
+    columns = [c[:, -1] for c in columns]
+    got = encoder.segment_offsets_of_two(*columns, batches)
+    for column, ends in zip(columns, got):
+        want = torch.searchsorted(column.cpu().contiguous(), torch.arange(batches, dtype=torch.int32), right=True)
+        assert ends.dtype == torch.int32 and torch.equal(ends.cpu().long(), want) and torch.equal(encoder.segment_offsets(column, batches), ends)
+
+
 @pytest.mark.parametrize("n,stride", [(1, 1), (7, 1), (8, 2), (9, 3), (4096, 1), (4097, 2), (30011, 1)])
 def test_stem_neighbours_in_any_order_and_twice(hip_lib, n, stride):
     """Rows in any order, around the sizes where the table doubles, dense and sparse, some coordinates twice: the first
