@@ -796,24 +796,26 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_kernel(const int32_t
     }
 }
 
-// The gradient of that for src_feat, added to dsrc (zeros before), and of the rows beside it: dout in fp16.  A thread has four
-// channels of a query, a quarter of a row apart, so that the lanes' additions lie side by side.
-constexpr int kGradChannels = 4;
+// The gradient of that for src_feat, added to dsrc (zeros before), and of the rows beside it: dout in fp16.  A thread has CH channels
+// of a query, a CH-th of a row apart, so that the lanes' additions lie side by side.  What bounds it is the pieces of lines that a
+// wavefront's additions fall into: a whole row of up to 128 channels in lanes next to each other, half a row beyond.  us by CH = 4 / 2 / 1:
+// 199,866 queries of 48 channels 205 / 131 / 124, 50,651 of 96 70 / 60 / 57, 12,652 of 192 33 / 28 / 31, 3,116 of 384 16 / 17 / 18.
+template <int CH>
 __global__ __launch_bounds__(kThreads) void knn_interpolate_grad_kernel(const int32_t *__restrict__ idx, const float *__restrict__ dist2, int K,
                                                                         int64_t Nq, const float *__restrict__ dout, int C,
                                                                         float *__restrict__ dsrc, _Float16 *__restrict__ dskip)
 {
-    const int quarter = C / kGradChannels;
-    const int64_t t = share_of_xcd(Nq * quarter);
-    if (t >= Nq * quarter) return;
-    const int64_t qi = t / quarter;
-    const int c = static_cast<int>(t - qi * quarter);
-    float g[kGradChannels];
+    const int part = C / CH;
+    const int64_t t = share_of_xcd(Nq * part);
+    if (t >= Nq * part) return;
+    const int64_t qi = t / part;
+    const int c = static_cast<int>(t - qi * part);
+    float g[CH];
 #pragma unroll
-    for (int e = 0; e < kGradChannels; ++e) g[e] = dout[qi * C + c + e * quarter];
+    for (int e = 0; e < CH; ++e) g[e] = dout[qi * C + c + e * part];
     if (dskip) {
 #pragma unroll
-        for (int e = 0; e < kGradChannels; ++e) dskip[qi * C + c + e * quarter] = static_cast<_Float16>(g[e]);
+        for (int e = 0; e < CH; ++e) dskip[qi * C + c + e * part] = static_cast<_Float16>(g[e]);
     }
     if (!dsrc) return;
     float norm = 0.0f;
@@ -823,7 +825,7 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_grad_kernel(const in
         if (row < 0) continue;
         const float w = 1.0f / (sqrtf(dist2[qi * K + i]) + 1e-8f) / norm;
 #pragma unroll
-        for (int e = 0; e < kGradChannels; ++e) unsafeAtomicAdd(dsrc + row * C + c + e * quarter, g[e] * w);
+        for (int e = 0; e < CH; ++e) unsafeAtomicAdd(dsrc + row * C + c + e * part, g[e] * w);
     }
 }
 
@@ -1083,8 +1085,12 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn_interpolate_grad(
     if (int rc = check_interpolation("s3d_knn_interpolate_grad", idx, dist2, K, Nq, Ns, C)) return rc;
     if (Nq == 0 || (!dsrc_feat && !dskip)) return S3D_OK;
     if (!dout) return fail(S3D_ERR_NULL_POINTER, "s3d_knn_interpolate_grad: null device pointer");
-    hipLaunchKernelGGL(knn_interpolate_grad_kernel, xcd_grid(Nq * (C / kGradChannels)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                       idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
+    if (C <= 128)
+        hipLaunchKernelGGL(knn_interpolate_grad_kernel<1>, xcd_grid(Nq * C), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                           idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
+    else
+        hipLaunchKernelGGL(knn_interpolate_grad_kernel<2>, xcd_grid(Nq * (C / 2)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                           idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
