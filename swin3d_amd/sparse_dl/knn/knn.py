@@ -170,8 +170,9 @@ def _interpolate_grads(idx, dist2, grad_out, num_src, need_src, need_skip):
 
 
 def _native_grads(idx, dist2, grad_out, num_src):
-    """The library's kernel has these gradients: no graph of them is wanted, nothing follows them, and it takes the types."""
-    return (not torch.is_grad_enabled() and data_only(grad_out) and grad_out.is_cuda and grad_out.dtype == torch.float32
+    """The library's kernel has these gradients: no graph of them is wanted, nothing follows them, it takes the types, and any
+    order of the additions will do (torch's index_add has a fixed one for programs that ask for it)."""
+    return (not torch.is_grad_enabled() and not torch.are_deterministic_algorithms_enabled() and data_only(grad_out) and grad_out.is_cuda and grad_out.dtype == torch.float32
             and grad_out.shape[1] % 4 == 0 and grad_out.shape[1] > 0 and num_src > 0
             and idx.is_contiguous() and dist2.is_contiguous() and idx.dtype == torch.int32)
 

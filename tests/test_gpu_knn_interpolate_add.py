@@ -50,3 +50,36 @@ def test_sum_and_gradients(hip_lib, nq, ns, channels, k):
 @pytest.mark.parametrize("channels", [124, 128, 132, 136])      # a whole row in lanes side by side, half a row
 def test_gradients_where_the_rows_are_halved(hip_lib, channels):
     test_sum_and_gradients(hip_lib, 515, 130, channels, 3)
+
+
+@pytest.mark.parametrize("add", [False, True])
+def test_gradients_in_a_fixed_order_where_a_program_asks_for_it(hip_lib, add):
+    """Under torch.use_deterministic_algorithms the gradient is that of index_add, the same bits on every call: here with some
+    500 terms a sum of sizes apart, whose order shows."""
+    import swin3d_amd
+    from swin3d_amd.sparse_dl.knn import KNNInterpolateAdd
+    nq, ns, channels, k = 20_000, 128, 64, 3
+    idx, dist2 = _neighbours(nq, ns, k, 5)
+    gen = torch.Generator("cuda").manual_seed(6)
+    feat, skip = (torch.randn((n, channels), device="cuda", generator=gen).half().requires_grad_() for n in (ns, nq))
+    wide = feat.detach().float().requires_grad_()
+    dout = torch.randn((nq, channels), device="cuda", generator=gen) * 2.0 ** torch.randint(-12, 12, (nq, 1), device="cuda", generator=gen)
+
+    def grads():
+        if add:
+            return torch.autograd.grad(KNNInterpolateAdd.apply(idx, dist2, feat, skip), (feat, skip), dout)
+        return torch.autograd.grad(swin3d_amd.KNNInterpolate.apply(idx, dist2, wide), (wide,), dout)
+
+    rows = idx.clamp(min=0).long()
+    weight = torch.where(idx >= 0, 1.0 / (torch.sqrt(dist2) + 1e-8), torch.zeros_like(dist2))
+    weight = weight / weight.sum(dim=1, keepdim=True).clamp_min(1e-30)
+    torch.use_deterministic_algorithms(True)
+    try:
+        want = torch.zeros((ns, channels), device="cuda")
+        for i in range(k):
+            want.index_add_(0, rows[:, i], dout * weight[:, i:i + 1])
+        for _ in range(8):
+            got = grads()
+            assert torch.equal(got[0], want.half() if add else want)
+    finally:
+        torch.use_deterministic_algorithms(False)
