@@ -820,6 +820,7 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_grad_kernel(const in
     if (!dsrc) return;
     float norm = 0.0f;
     for (int i = 0; i < K; ++i) norm += idx[qi * K + i] >= 0 ? 1.0f / (sqrtf(dist2[qi * K + i]) + 1e-8f) : 0.0f;
+    norm = norm < 1e-30f ? 1e-30f : norm;      // (neighbours at an infinite distance have no share)
     for (int i = 0; i < K; ++i) {
         const int64_t row = idx[qi * K + i];
         if (row < 0) continue;

@@ -83,3 +83,18 @@ def test_gradients_in_a_fixed_order_where_a_program_asks_for_it(hip_lib, add):
             assert torch.equal(got[0], want.half() if add else want)
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+def test_gradients_of_neighbours_beyond_any_distance(hip_lib):
+    """Infinite distances have no share, also where a query has no other neighbours; NaN makes NaN."""
+    import swin3d_amd
+    idx = torch.tensor([[0, 1, 2], [1, 2, 3], [2, 3, 4], [4, 5, -1], [-1, -1, -1], [6, 7, 5]], dtype=torch.int32, device="cuda")
+    dist2 = torch.rand((6, 3), device="cuda") + 0.5
+    dist2[1, 0], dist2[2], dist2[3, :2], dist2[5, 1] = float("inf"), float("inf"), float("inf"), float("nan")
+    feat = torch.randn((8, 8), device="cuda").requires_grad_()
+    dout = torch.randn((6, 8), device="cuda")
+    (got,) = torch.autograd.grad(swin3d_amd.KNNInterpolate.apply(idx, dist2, feat), feat, dout)
+    (want,) = torch.autograd.grad(swin3d_amd.KNNInterpolate.apply(idx, dist2, feat), feat, dout.requires_grad_(), create_graph=True)
+    assert torch.equal(got.isnan(), want.isnan()) and int(got.isnan().any(1).sum()) == 3      # the sources of the last query
+    assert bool(((got - want).abs() <= 2.0 ** -20 * (1 + want.abs()))[~want.isnan()].all())
+    assert not got[4].any()
