@@ -355,11 +355,11 @@ __global__ __launch_bounds__(kListThreads) void sweep_place_kernel(AttnArgs a) {
 // Few windows, of which every wavefront has one round: both steps by one workgroup, and the strip list, where it is asked for, by
 // another beside it.  A plan for strips of 2 windows 10.1 us (three launches) -> 5.8, of 84 windows 14.4 -> 8.9; at 340 windows, two
 // rounds, one launch takes 17.2 and two 11.6.
-__global__ __launch_bounds__(kListThreads) void sweep_list_kernel(AttnArgs a)
+__global__ __launch_bounds__(kListThreads) void sweep_list_kernel(AttnArgs a, tile::StripList also)
 {
     if (blockIdx.x == 1) {
-        tile::build_strip_list<kListThreads>(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(a.also_strips.total),
-                                             const_cast<uint64_t *>(a.also_strips.strips));
+        tile::build_strip_list<kListThreads>(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(also.total),
+                                             const_cast<uint64_t *>(also.strips));
         return;
     }
     count_windows(a, 0, 1);
@@ -368,10 +368,11 @@ __global__ __launch_bounds__(kListThreads) void sweep_list_kernel(AttnArgs a)
     place_windows(a, 0, 1);
 }
 
-void launch_work_list(const AttnArgs &a, hipStream_t stream)
+void launch_work_list(const AttnArgs &a, hipStream_t stream, bool strips_too = false)
 {
     if (a.W <= kFewWindows) {
-        hipLaunchKernelGGL(sweep_list_kernel, dim3(a.also_strips.total ? 2 : 1), dim3(kListThreads), 0, stream, a);
+        hipLaunchKernelGGL(sweep_list_kernel, dim3(strips_too ? 2 : 1), dim3(kListThreads), 0, stream, a,
+                           strips_too ? attn_strip_list(a) : tile::StripList{});
         return;
     }
     const int64_t want = ceil_div(a.W, kListThreads);
@@ -1133,11 +1134,11 @@ int launch_sweep_heads(const AttnArgs &a, hipStream_t stream, int what)
     constexpr int kThreads = group_threads<T, D, HP>();
     b.target_items = grid / groups * (kThreads / 64);   // wavefronts that serve one head group
     b.block_shift = target_shift_for(a.N, a.W, b.target_items);
-    if (what & 1) {
-        launch_work_list(b, stream);
+    if (what & kAttnBuildList) {
+        launch_work_list(b, stream, what & kAttnStripList);
         S3D_HIP_CHECK(hipGetLastError());
     }
-    if (what & 2) {
+    if (what & kAttnSweep) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
         S3D_HIP_CHECK(hipGetLastError());
     }
