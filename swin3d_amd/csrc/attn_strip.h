@@ -209,7 +209,14 @@ template <> struct Raw4<float> {
         return mfma4(y.s[0], identity, mfma4(y.s[1], identity, mfma4(y.s[2], identity, f32x4_t{})));
     }
 };
-// sum over the four lanes of a column (lane % 16)
+// largest, and sum, over the four lanes of a column (lane % 16)
+__device__ __forceinline__ float max_columns(float x)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 __device__ __forceinline__ float sum_columns(float x)
 {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);

@@ -38,8 +38,11 @@ namespace {
 //    rounding, also of fp16 tables in a forward whose backward has fp32 ones; there is room for 16), dL in units of 2^(e-30),
 //    2^e the least power above the sum of |dL| of its query (by key: of its key).  A cell keeps what fp32 would, and no order
 //    of additions shows.
-//  * They enter the products over 2^-kLiftP and 2^(e-kLift), the cells and the pairs' own alike: beside fp16 operands as two
-//    fp16 numbers, 23 bits down to 2^-3 and units of 2^-24 below, that is 2^-35 of P and 2^-39 of the sum of |dL|.
+//  * They enter the products over 2^-kLiftP and 2^(e-kLift), beside fp16 operands as two fp16 numbers, 23 bits down to 2^-3 and
+//    units of 2^-24 below: 2^-35 of P, and 2^-39 of the sum of |dL|, in the cells and for the pairs themselves.  The pairs' own P
+//    by key, whose sum is nowhere near 1 where no query gives the key much weight, are over a unit that follows the largest P
+//    that the wavefront holds of the key: 2^-39 of that.  (Over 2^-kLiftP, dv of a key whose weights are 2^-26 had ten bits.
+//    0.6 % of a backward of 199,327 voxels at head_dim 8, 0.2 % of one of 12,421 at 16.)
 //
 // What is not finite stays in its window, though the products take all columns of a strip and all rows of a table, zeros
 // among them: features and table entries that are not finite go into their operands as zeros.  The records kernel has left
@@ -52,6 +55,14 @@ template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // 
 template <typename TF> constexpr float kLiftP = sizeof(TF) == 2 ? 2048.0f : 1.0f;
 template <typename TF> constexpr float kWeightCell = kLiftP<TF> / kFixWeight;
 template <typename TF> constexpr float kGradCell = (sizeof(TF) == 2 ? 32768.0f : 1.0f) / 1073741824.0f;
+// What P enters a product over, by the largest there is: a power of two, by which the largest P is below 2^kLift; and its inverse.
+template <typename TF> __device__ __forceinline__ float weight_unit(float most)
+{
+    if (kLift<TF> == 0) return 1.0f;
+    constexpr uint32_t kLeast = 47u << 23, kUp = static_cast<uint32_t>(kLift<TF> - 1) << 23;      // 2^-80
+    return __uint_as_float(max(__float_as_uint(most) & 0x7f800000u, kLeast) - kUp);
+}
+__device__ __forceinline__ float inverse_power2(float x) { return __uint_as_float(0x7f000000u - __float_as_uint(x)); }
 constexpr int kLiftFeature = 15;              // exponent of the strip's largest q or k in the table gradients
 
 constexpr int kStripReach = kStripThreads / kStrip;        // pairs of a voxel that a step of the workgroup takes
@@ -355,6 +366,10 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};           // over 2^(exponent - kLift): [channel][column]
         f32x4_t acc_v = {0.0f, 0.0f, 0.0f, 0.0f};
         const float scale = power2(kLift<TF> - exponent);
+        // by key: P over unit_p, and so acc_v
+        auto unit_of = [](float most) { return kLift<TF> > 0 ? weight_unit<TF>(max_columns(most)) : 1.0f; };
+        float unit_p = 1.0f;
+        if constexpr (kByKey) unit_p = unit_of(one_step(n) ? kept[0].y : fmaxf(fmaxf(kept[0].y, kept[1].y), fmaxf(kept[2].y, kept[3].y)));
         // a step's features, [voxel][channel]; what is not finite as zeros
         auto voxels_of = [&](Exact4<TF> &f, Exact4<TF> &fz) {
             f32x4_t ys = y.voxels(identity), zs{};
@@ -381,7 +396,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             c.set_one(kept[0].x, scale, window);
             acc = product(f, c, acc);
             if constexpr (kByKey) {
-                c.set_one(kept[0].y, kLiftP<TF>, window);
+                c.set_one(kept[0].y, inverse_power2(unit_p), window);
                 acc_v = product(fz, c, acc_v);
             }
         }
@@ -405,7 +420,14 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                 c.set(l, scale);
                 acc = product(f, c, acc);
                 if constexpr (kByKey) {
-                    c.set(p, kLiftP<TF>);
+                    if (kLift<TF> > 0 && j0 > 0) {
+                        const float most = fmaxf(unit_p, unit_of(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]))));
+                        const float less = unit_p * inverse_power2(most);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc_v[e] *= less;
+                        unit_p = most;
+                    }
+                    c.set(p, inverse_power2(unit_p));
                     acc_v = product(fz, c, acc_v);
                 }
             }
@@ -522,7 +544,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             dx[e] = fmaf(acc_t[e], scale_table, acc[e]) * back;
-            if constexpr (kPacked && kByKey) dx[e] = g4 < 2 ? dx[e] : acc_v[e] * (1.0f / kLiftP<TF>);
+            if constexpr (kByKey) acc_v[e] *= unit_p;
+            if constexpr (kPacked && kByKey) dx[e] = g4 < 2 ? dx[e] : acc_v[e];
         }
         *reinterpret_cast<f32x4_t *>(&part_s[(wave * 64 + lane) * 4]) = dx;
         if constexpr (kParts > 1) *reinterpret_cast<f32x4_t *>(&part_s[((kStripWaves + wave) * 64 + lane) * 4]) = acc_v;
@@ -543,7 +566,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                 for (int e = 0; e < 4; ++e) sums[e] += v[e];
             }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = static_cast<float>(sums[e]) * (which > 0 ? 1.0f / kLiftP<TF> : 1.0f);
+            for (int e = 0; e < 4; ++e) o[e] = static_cast<float>(sums[e]);
             const bool dv = kPacked ? kByKey && g4 >= 2 : which > 0;
             if (there && (!kPacked || kByKey || g4 < 2))
                 store4(static_cast<TF *>(dv ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * C + part4(), o);

@@ -55,14 +55,6 @@ constexpr int kStageRows = kStripWaves * 16;       // table rows of a stage: a t
 // words between the products of one voxel and the next: 16-byte stores of 16 voxels meet in no bank
 constexpr int kProductStride = kStageRows + 4;
 
-__device__ __forceinline__ float max_columns(float x)
-{
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 template <int ND, bool kDeviceSizes>
 __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArgs f)
 {

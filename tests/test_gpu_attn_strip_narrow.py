@@ -91,3 +91,25 @@ def test_sums_by_row_keep_their_bits(oracle_lib, hip_lib, dtype, tables):
     got = _backward(case, dtype, tables, dout)[5].double().cpu().numpy()
     ref = np.asarray(oracle_lib.attn_bwd(*case.oracle_args(), dout)[5])
     assert np.linalg.norm(got - ref) <= 6 * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype,tables", TYPES)
+@pytest.mark.parametrize("dim", [8, 16])
+def test_keys_of_little_weight_keep_their_bits(oracle_lib, hip_lib, dtype, tables, dim):
+    """dv of keys whose weights are e^-7 to e^-22 in every query, under a gradient as large as a loss scale makes it.  A weight's
+    relative error is that of its logit, up to 22 in some twenty roundings of 2^-24, and of an exponential: 2^-14 of the terms'
+    sizes; the result is rounded to its type."""
+    case = _windows_case(oracle_lib, SIZES, "XYZ_RGB", 2, seed=37, dim=dim)
+    rng = np.random.default_rng(38)
+    for x in (case.q, case.k, case.tq, case.tk):
+        x *= np.float32(2.0 ** -3)
+    light = rng.random(case.N) < 0.4
+    case.q[:, :, 0] = 1
+    case.k[light, :, 0] = -rng.uniform(7, 22, (int(light.sum()), 1))
+    to_half_and_back(case)
+    dout = (8192 * rng.standard_normal(case.q.shape)).astype(np.float16).astype(np.float32)
+    forward = []
+    got = _backward(case, dtype, tables, dout, forward=forward)[2].double().cpu()
+    ref, size = (_pairwise_backward(case, *forward, x)[2] for x in (dout, np.abs(dout)))
+    bound = 2.0 ** -14 * size + (2.0 ** -11 * ref.abs() + 2.0 ** -25 if dtype == torch.float16 else 0)
+    assert bool(((got.view_as(ref) - ref).abs() <= bound).all())
