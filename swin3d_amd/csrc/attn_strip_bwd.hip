@@ -45,10 +45,13 @@ namespace {
 //    0.6 % of a backward of 199,327 voxels at head_dim 8, 0.2 % of one of 12,421 at 16.)
 //
 // What is not finite stays in its window, though the products take all columns of a strip and all rows of a table, zeros
-// among them: features and table entries that are not finite go into their operands as zeros.  The records kernel has left
-// their pairs' dL as NaN or infinity, with dout their P as NaN as well, and so dq, dk and dv are what the sums over a window's
-// pairs would be, but for channels beside the one that is not finite.  In the integers such a pair counts for nothing; the table rows it belongs to are marked and their gradients stored as NaN.  A P
-// beyond 8 says that the statistics are not the forward's, and is treated alike.
+// among them: features and table entries that are not finite go into their operands as zeros, with all channels of their
+// voxel.  The records kernel has left their pairs' dL as NaN or infinity, and so dq and dk are what the sums over a window's pairs
+// would be, but for channels beside the one that is not finite.  In the integers such a pair counts for nothing; the table rows
+// it belongs to are marked and their gradients stored as NaN.  A P beyond 8 says that the statistics are not the forward's, and
+// is treated alike.  A dout that is not finite leaves P alone.  At head_dim 16 the records kernel makes NaN of it all the same,
+// and so of all channels of dv and dTv; at 8 a workgroup that has met a dL that is not finite goes through its strips once
+// more and adds up, pair by pair, dv of the windows with such a dout and what its voxel gives dTv.
 constexpr float kFixWeight = 268435456.0f, kMostWeight = 8.0f;
 constexpr int kFixGrad = 30;
 template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // (fp32 features may be as large as fp32 is)
@@ -80,6 +83,103 @@ template <typename V> __device__ __forceinline__ V max16(V v)
     v = step(v, std::integral_constant<int, 0x4E>{});      // quad_perm [2,3,0,1]
     v = step(v, std::integral_constant<int, 0x141>{});     // row_half_mirror
     return step(v, std::integral_constant<int, 0x140>{});  // row_mirror
+}
+
+// What the products of head_dim 8 leave out, by a workgroup that has met a dL that is not finite: P dout of the voxels whose dout is
+// not finite in some channel, pair by pair.  By key dv of their windows is added up again; by query what they give dTv joins the
+// workgroup's slot.  (It takes its arguments from where the launch put them: what is kept for it through the loop over strips comes
+// back from memory there, 1 % of a call in fp32.)
+template <typename TF, int ND, bool kByKey>
+__device__ __forceinline__ void add_left_out(float *shared)
+{
+    constexpr int C = 8;
+    const void *at_args = (const void *)__builtin_amdgcn_kernarg_segment_ptr();
+    int tid = threadIdx.x, block = blockIdx.x;
+    asm volatile("" : "+s"(at_args), "+v"(tid), "+s"(block));
+    const StripArgs &b = *static_cast<const StripArgs *>(at_args);
+    const AttnArgs &a = b.f;
+    const int H = a.H, HD = H * C, h = block % H, group = block / H, groups = static_cast<int>(gridDim.x) / H, strips = b.list.total[1];
+    const int c16 = tid & 15, channel = tid >> 4 & 7, part = tid >> 7;
+    const TF *gd = static_cast<const TF *>(b.dout) + h * C;
+    const float2 *records = b.records + static_cast<int64_t>(h) * b.pairs;
+    auto row_of = [&](int pos) { return static_cast<int64_t>(a.n2n ? a.n2n[pos] : pos) * HD; };
+    auto any_bad = [&](const TF *dout) {
+        float x[C];
+        load_row<C>(dout, x);
+        bool bad = false;
+#pragma unroll
+        for (int c = 0; c < C; ++c) bad = bad || !finite(x[c]);
+        return bad;
+    };
+    __threadfence();      // (what is stored may be stored again, by other lanes)
+    __syncthreads();
+    if constexpr (kByKey) {
+        // a thread for a column, a channel and every fourth query
+        for (int u = group; u < strips; u += groups) {
+            const int4 strip = b.list.strips[u], column = b.columns[u * kStrip + c16];
+            const int n = strip.y;
+            const bool there = c16 < strip.w && column.w >= 0;
+            const float2 *from = records + (there ? column.w + (column.x - column.z) * n : 0);
+            float sum = 0.0f;
+            bool bad = false;
+            for (int i = part; there && i < n; i += 4) {
+                const TF *dout = gd + row_of(column.z + i);
+                bad = bad || any_bad(dout);
+                sum = fmaf(from[i].y, to_float(dout[channel]), sum);
+            }
+            shared[tid] = sum;
+            shared[kStripThreads + tid] = bad ? 1.0f : 0.0f;
+            __syncthreads();
+            bad = false;
+            sum = 0.0f;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                sum += shared[(tid & 127) + 128 * p];
+                bad = bad || shared[kStripThreads + (tid & 127) + 128 * p] > 0.0f;
+            }
+            TF *to = static_cast<TF *>(b.dv) + static_cast<uint64_t>(static_cast<uint32_t>(column.y)) * b.grad_stride + h * C + channel;
+            if (there && bad && part == 0) {
+                if constexpr (sizeof(TF) == 2) *to = __float2half_rn(sum);
+                else *to = sum;
+            }
+            __syncthreads();
+        }
+    } else {
+        // Table rows times channels, four times, in the place of the cells, which are zeros; a thread for an axis, a channel and
+        // every fourth column, which has its words to itself.
+        constexpr int kWords = kTiles<ND> * 16 * C;
+        static_assert(4 * kWords == kTiles<ND> * 16 * kStrip * 2, "the cells, of P and dL");
+        const int axis = tid >> 3 & 15, c = tid & 7;
+        for (int u = group; u < strips; u += groups) {
+            const int4 strip = b.list.strips[u];
+            const int n = strip.y;
+            for (int at = part; axis < ND && at < strip.w; at += 4) {
+                const int4 column = b.columns[u * kStrip + at];
+                const TF *dout = gd + row_of(column.x);
+                if (column.w < 0 || !any_bad(dout)) continue;
+                const int rows_n = axis_rows<ND>(a, axis);
+                const float x = to_float(dout[c]), half_rows = static_cast<float>(rows_n / 2), upper = crse_upper(rows_n);
+                const float mine = a.n_coords[static_cast<int64_t>(column.x) * ND + axis];
+                const float2 *from = records + column.w + column.x - column.z;
+#pragma unroll 4
+                for (int j = 0; j < n; ++j) {
+                    const int r = crse_row(mine, a.n_coords[static_cast<int64_t>(column.z + j) * ND + axis], half_rows, upper);
+                    float *to = shared + part * kWords + (axis_row0(axis) + r) * C + c;
+                    *to = fmaf(from[static_cast<int64_t>(j) * n].y, x, *to);
+                }
+            }
+        }
+        __syncthreads();
+        if (c16 < C) return;       // (the columns of dTq)
+        float *slot = b.slots + static_cast<int64_t>(block) * (kTiles<ND> * 256);
+        for (int tile = tid >> 6; tile < kTiles<ND>; tile += kStripWaves) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float *from = shared + (tile * 16 + 4 * (tid >> 4 & 3) + e) * C + c16 - C;
+                slot[tile * 256 + (tid & 63) * 4 + e] += (from[0] + from[kWords]) + (from[2 * kWords] + from[3 * kWords]);
+            }
+        }
+    }
 }
 
 // C channels a head: 16, or 8 (packed): q or k and dout then share the sixteen channels of an operand, dTq and dTv the sixteen
@@ -572,8 +672,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                 store4(static_cast<TF *>(dv ? b.dv : kByKey ? b.dk : b.dq) + static_cast<uint64_t>(static_cast<uint32_t>(own_row)) * b.grad_stride + h * C + part4(), o);
         }
     }
-    // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]
     const bool none = __syncthreads_or(incomplete);
+    // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]
     float *slot = b.slots + static_cast<int64_t>(blockIdx.x) * (kSets * kTiles<ND> * 256);
 #pragma unroll
     for (int kind = 0; kind < kSets; ++kind) {
@@ -584,6 +684,9 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             if (none) g = f32x4_t{nan, nan, nan, nan};
             *reinterpret_cast<f32x4_t *>(slot + (kind * kTiles<ND> + tile) * 256 + lane * 4) = g;
         }
+    }
+    if constexpr (kPacked) {
+        if (__builtin_amdgcn_readfirstlane(marked_s) != 0) add_left_out<TF, ND, kByKey>(kByKey ? part_s : reinterpret_cast<float *>(cells_s));
     }
 }
 

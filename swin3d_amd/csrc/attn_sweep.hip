@@ -887,7 +887,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
         const bool fits = pair_base + static_cast<int64_t>(n_w) * n_w <= b.pairs;
 
         Slice<T, D> own_x[HP], own_y[HP];     // q_i, dout_i
-        float own_m[HP], own_inv[HP], own_delta[HP], own_bad[HP];
+        float own_m[HP], own_inv[HP], own_delta[HP];
         float ci[ND], res_x[HP][D], res_y[kKeyOwned ? HP : 1][D];
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
@@ -904,12 +904,9 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
                     const int64_t at_out = static_cast<int64_t>(own_row) * HD + (h + hh) * D;
                     load_row<D>(ggo + at_out, x);
                     load_row<D>(static_cast<const TF *>(b.out) + at_out, y);
-                    own_delta[hh] = own_bad[hh] = 0.0f;
+                    own_delta[hh] = 0.0f;
 #pragma unroll
-                    for (int c = 0; c < D; ++c) {
-                        own_delta[hh] += x[c] * y[c];
-                        own_bad[hh] = fabsf(x[c]) < INFINITY ? own_bad[hh] : __int_as_float(0x7fc00000);
-                    }
+                    for (int c = 0; c < D; ++c) own_delta[hh] += x[c] * y[c];
                 }
             }
 #pragma unroll
@@ -1030,11 +1027,10 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
                     }
                 }
                 if constexpr (kOnlyRecords) {
-                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq; a query
-                    // whose dout is not finite has no weights: the products that follow take its dout as zeros)
+                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq)
                     const float p = __expf(logit - own_m[hh]) * own_inv[hh];
                     const float dl = fabsf(logit) < INFINITY ? p * (dp - own_delta[hh]) : __int_as_float(0x7fc00000);
-                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p + own_bad[hh]);
+                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
                     continue;
                 }
                 float p, dl;

@@ -113,3 +113,36 @@ def test_keys_of_little_weight_keep_their_bits(oracle_lib, hip_lib, dtype, table
     ref, size = (_pairwise_backward(case, *forward, x)[2] for x in (dout, np.abs(dout)))
     bound = 2.0 ** -14 * size + (2.0 ** -11 * ref.abs() + 2.0 ** -25 if dtype == torch.float16 else 0)
     assert bool(((got.view_as(ref) - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype,tables", TYPES)
+@pytest.mark.parametrize("cRSE,value", [("XYZ_RGB_NORM", np.inf), ("XYZ_RGB", np.nan), ("XYZ", -np.inf)])
+def test_a_channel_of_dout_that_is_not_finite_stays_one(oracle_lib, hip_lib, dtype, tables, cRSE, value):
+    """A dout with a channel that is not finite spoils that channel of dv in its window, and of dTv in the rows of its pairs: the
+    others are the sums over pairs that they are without it."""
+    case = to_half_and_back(_windows_case(oracle_lib, SIZES, cRSE, 3, seed=39, dim=8))
+    dout = _dout(case, 40)
+    clean = _backward(case, dtype, tables, dout)
+    touched = np.zeros((case.N, 3), bool)
+    for i, size in enumerate((1, 3, 7, 26, 32, 65, 160, 257)):
+        w = int(np.flatnonzero(case.index["w_sizes"] == size)[0])
+        rows = case.index["n2n"][case.index["w2n"][w]:case.index["w2n"][w] + size]
+        touched[rows, i % 3] = True
+        dout[rows[size // 2], i % 3, i % 2 + 3] = value
+    forward = []
+    got = _backward(case, dtype, tables, dout, forward=forward)
+    ref = _pairwise_backward(case, *forward, dout)
+    dv, want = got[2].double().cpu(), ref[2]
+    assert torch.equal(dv.isnan(), want.isnan()) and torch.equal(dv.isinf(), want.isinf())
+    there = torch.isfinite(want)
+    rel = 2e-5 if dtype == torch.float32 else 3e-3         # as elsewhere in the tests of this operator
+    assert float((dv - want)[there].abs().max()) <= rel * float(want[there].abs().max())
+    rest = torch.as_tensor(~touched)
+    assert torch.equal(dv[rest], clean[2].double().cpu()[rest])
+    dtv, want = got[5].double().cpu().view_as(ref[5]), ref[5]
+    assert torch.equal(~torch.isfinite(dtv), ~torch.isfinite(want)) and not torch.isfinite(dtv[..., 3:5]).all() \
+        and bool(torch.isfinite(dtv[..., [0, 1, 2, 5, 6, 7]]).all())
+    there = torch.isfinite(want)
+    assert float((dtv - want)[there].abs().max()) <= rel * float(want[there].abs().max())
+    again = _backward(case, dtype, tables, dout)
+    assert all(torch.equal(x.nan_to_num(1.0, 2.0, 3.0), y.nan_to_num(1.0, 2.0, 3.0)) for x, y in zip(got, again))
