@@ -50,8 +50,9 @@ namespace {
 // would be, but for channels beside the one that is not finite.  In the integers such a pair counts for nothing; the table rows
 // it belongs to are marked and their gradients stored as NaN.  A P beyond 8 says that the statistics are not the forward's, and
 // is treated alike.  A dout that is not finite leaves P alone.  At head_dim 16 the records kernel makes NaN of it all the same,
-// and so of all channels of dv and dTv; at 8 a workgroup that has met a dL that is not finite goes through its strips once
-// more and adds up, pair by pair, dv of the windows with such a dout and what its voxel gives dTv.
+// and so of all channels of dv and dTv; at 8 it does where no channel of dout is finite; elsewhere a workgroup goes
+// through its strips with such a dL once more and adds up, pair by pair, dv of the windows and what the voxel gives dTv.  (Every dout
+// infinite, 199,327 voxels x 6, fp16: 4.6 ms where the call takes 1.5, 10.4 pair by pair.)
 constexpr float kFixWeight = 268435456.0f, kMostWeight = 8.0f;
 constexpr int kFixGrad = 30;
 template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // (fp32 features may be as large as fp32 is)
@@ -85,12 +86,13 @@ template <typename V> __device__ __forceinline__ V max16(V v)
     return step(v, std::integral_constant<int, 0x140>{});  // row_mirror
 }
 
-// What the products of head_dim 8 leave out, by a workgroup that has met a dL that is not finite: P dout of the voxels whose dout is
+// What the products of head_dim 8 leave out, in the strips that have a dL that is not finite beside a P that is: P dout of the voxels whose dout is
 // not finite in some channel, pair by pair.  By key dv of their windows is added up again; by query what they give dTv joins the
 // workgroup's slot.  (It takes its arguments from where the launch put them: what is kept for it through the loop over strips comes
 // back from memory there, 1 % of a call in fp32.)
+constexpr int kMetWords = 64;                              // a bit for each of a workgroup's strips (modulo 2048)
 template <typename TF, int ND, bool kByKey>
-__device__ __forceinline__ void add_left_out(float *shared)
+__device__ __forceinline__ void add_left_out(float *shared, const uint32_t *strips_met)
 {
     constexpr int C = 8;
     const void *at_args = (const void *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -102,6 +104,10 @@ __device__ __forceinline__ void add_left_out(float *shared)
     const int c16 = tid & 15, channel = tid >> 4 & 7, part = tid >> 7;
     const TF *gd = static_cast<const TF *>(b.dout) + h * C;
     const float2 *records = b.records + static_cast<int64_t>(h) * b.pairs;
+    auto met = [&](int u) {
+        const int turn = u / groups;
+        return (__builtin_amdgcn_readfirstlane(strips_met[turn / 32 % kMetWords]) >> (turn & 31) & 1) != 0;
+    };
     auto row_of = [&](int pos) { return static_cast<int64_t>(a.n2n ? a.n2n[pos] : pos) * HD; };
     auto any_bad = [&](const TF *dout) {
         float x[C];
@@ -116,6 +122,7 @@ __device__ __forceinline__ void add_left_out(float *shared)
     if constexpr (kByKey) {
         // a thread for a column, a channel and every fourth query
         for (int u = group; u < strips; u += groups) {
+            if (!met(u)) continue;
             const int4 strip = b.list.strips[u], column = b.columns[u * kStrip + c16];
             const int n = strip.y;
             const bool there = c16 < strip.w && column.w >= 0;
@@ -151,6 +158,7 @@ __device__ __forceinline__ void add_left_out(float *shared)
         static_assert(4 * kWords == kTiles<ND> * 16 * kStrip * 2, "the cells, of P and dL");
         const int axis = tid >> 3 & 15, c = tid & 7;
         for (int u = group; u < strips; u += groups) {
+            if (!met(u)) continue;
             const int4 strip = b.list.strips[u];
             const int n = strip.y;
             for (int at = part; axis < ND && at < strip.w; at += 4) {
@@ -204,7 +212,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     __shared__ __align__(16) float part_s[kParts * kStripWaves * 256];
     __shared__ float sums_s[kStripWaves][kStrip], grad_s;
     __shared__ __align__(16) Exact4<TF> features_s[kSets][64];        // q or k, dout of the strip's voxels
-    __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s;
+    __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s, met_s[kPacked ? kMetWords : 1];
     // Pieces of the table's operands that wait in LDS, as many as leave room for two workgroups a CU (81,864 of 81,920 bytes by
     // query in fp32).  In registers they would not fit beside the rest, and a spilled operand comes back from memory behind the
     // pairs of the next strip, which are on their way then: loads return in order.
@@ -276,6 +284,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     for (int t = tid; t < kTiles<ND> * 16 * kStrip * kKinds / 4; t += kStripThreads) reinterpret_cast<uint4 *>(cells_s)[t] = make_uint4(0, 0, 0, 0);
     if (tid < 2 * kTiles<ND>) marks_s[tid] = 0;
     if (tid == 0) marked_s = 0;
+    if (kPacked && tid < kMetWords) met_s[tid] = 0;
     bool incomplete = false;                 // a window did not fit the records
 
     // A strip's voxels, their features (channels 4 g4 .. of voxel c16) and the first of their pairs.  They are under way while
@@ -449,6 +458,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
             for (int j = reach0; j < n; j += kStripReach) {
                 const float2 r = settle(records[pair0 + j * step], fits, there);
                 if (finite(r.x)) continue;
+                if (kPacked && finite(r.y)) atomicOr(&met_s[u / groups / 32 % kMetWords], 1u << (u / groups & 31));
 #pragma unroll 1
                 for (int axis = 0; axis < ND; ++axis) {
                     const int rows_n = axis_rows<ND>(a, axis);
@@ -686,7 +696,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
         }
     }
     if constexpr (kPacked) {
-        if (__builtin_amdgcn_readfirstlane(marked_s) != 0) add_left_out<TF, ND, kByKey>(kByKey ? part_s : reinterpret_cast<float *>(cells_s));
+        if (__builtin_amdgcn_readfirstlane(marked_s) != 0) add_left_out<TF, ND, kByKey>(kByKey ? part_s : reinterpret_cast<float *>(cells_s), met_s);
     }
 }
 

@@ -887,7 +887,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
         const bool fits = pair_base + static_cast<int64_t>(n_w) * n_w <= b.pairs;
 
         Slice<T, D> own_x[HP], own_y[HP];     // q_i, dout_i
-        float own_m[HP], own_inv[HP], own_delta[HP];
+        float own_m[HP], own_inv[HP], own_delta[HP], own_none[HP];
         float ci[ND], res_x[HP][D], res_y[kKeyOwned ? HP : 1][D];
 #pragma unroll
         for (int hh = 0; hh < HP; ++hh) {
@@ -905,8 +905,13 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
                     load_row<D>(ggo + at_out, x);
                     load_row<D>(static_cast<const TF *>(b.out) + at_out, y);
                     own_delta[hh] = 0.0f;
+                    bool some = false;
 #pragma unroll
-                    for (int c = 0; c < D; ++c) own_delta[hh] += x[c] * y[c];
+                    for (int c = 0; c < D; ++c) {
+                        own_delta[hh] += x[c] * y[c];
+                        some = some || fabsf(x[c]) < INFINITY;
+                    }
+                    own_none[hh] = some ? 0.0f : __int_as_float(0x7fc00000);
                 }
             }
 #pragma unroll
@@ -1027,10 +1032,11 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
                     }
                 }
                 if constexpr (kOnlyRecords) {
-                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq)
+                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq; a query
+                    // whose dout has no finite channel has no weights either: all channels of what they make are NaN)
                     const float p = __expf(logit - own_m[hh]) * own_inv[hh];
                     const float dl = fabsf(logit) < INFINITY ? p * (dp - own_delta[hh]) : __int_as_float(0x7fc00000);
-                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
+                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p + own_none[hh]);
                     continue;
                 }
                 float p, dl;
