@@ -798,8 +798,10 @@ __global__ __launch_bounds__(kThreads) void knn_interpolate_kernel(const int32_t
 
 // The gradient of that for src_feat, added to dsrc (zeros before), and of the rows beside it: dout in fp16.  A thread has CH channels
 // of a query, a CH-th of a row apart, so that the lanes' additions lie side by side.  What bounds it is the pieces of lines that a
-// wavefront's additions fall into: a whole row of up to 128 channels in lanes next to each other, half a row beyond.  us by CH = 4 / 2 / 1:
-// 199,866 queries of 48 channels 205 / 131 / 124, 50,651 of 96 70 / 60 / 57, 12,652 of 192 33 / 28 / 31, 3,116 of 384 16 / 17 / 18.
+// wavefront's additions fall into: a whole row of up to 128 channels in lanes next to each other, half a row beyond, a quarter where
+// that is a wavefront's width.  us by CH = 4 / 2 / 1: 199,866 queries of 48 channels 205 / 131 / 124, 50,651 of 96 70 / 60 / 57; of 160
+// 103 / 80; 12,652 of 192 34 / 28 / 31; of 256 34.2 / 34.7, of 384 49.0 / 49.5, of 640 79.9 / 79.5; 3,116 of 256 11.6 / 11.7, of 320 13.7 /
+// 14.0, of 384 15.4 / 16.2, of 512 19.0 / 19.7, of 640 23.1 / 23.4.
 template <int CH>
 __global__ __launch_bounds__(kThreads) void knn_interpolate_grad_kernel(const int32_t *__restrict__ idx, const float *__restrict__ dist2, int K,
                                                                         int64_t Nq, const float *__restrict__ dout, int C,
@@ -1086,12 +1088,10 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn_interpolate_grad(
     if (int rc = check_interpolation("s3d_knn_interpolate_grad", idx, dist2, K, Nq, Ns, C)) return rc;
     if (Nq == 0 || (!dsrc_feat && !dskip)) return S3D_OK;
     if (!dout) return fail(S3D_ERR_NULL_POINTER, "s3d_knn_interpolate_grad: null device pointer");
-    if (C <= 128)
-        hipLaunchKernelGGL(knn_interpolate_grad_kernel<1>, xcd_grid(Nq * C), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
-    else
-        hipLaunchKernelGGL(knn_interpolate_grad_kernel<2>, xcd_grid(Nq * (C / 2)), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           idx, dist2, K, Nq, dout, C, dsrc_feat, static_cast<_Float16 *>(dskip));
+    const int own = C <= 128 ? 1 : C < 256 ? 2 : 4;
+    auto kernel = own == 1 ? knn_interpolate_grad_kernel<1> : own == 2 ? knn_interpolate_grad_kernel<2> : knn_interpolate_grad_kernel<4>;
+    hipLaunchKernelGGL(kernel, xcd_grid(Nq * (C / own)), dim3(kThreads), 0, static_cast<hipStream_t>(stream), idx, dist2, K, Nq, dout, C,
+                       dsrc_feat, static_cast<_Float16 *>(dskip));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

@@ -47,7 +47,7 @@ def test_sum_and_gradients(hip_lib, nq, ns, channels, k):
     assert again.requires_grad and bool(((again.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + (10 + most) * 2.0 ** -24 * size + 2.0 ** -25).all())
 
 
-@pytest.mark.parametrize("channels", [124, 128, 132, 136])      # a whole row in lanes side by side, half a row
+@pytest.mark.parametrize("channels", [124, 128, 132, 136, 252, 256, 260])      # a whole row in lanes side by side, half a row, a quarter
 def test_gradients_where_the_rows_are_halved(hip_lib, channels):
     test_sum_and_gradients(hip_lib, 515, 130, channels, 3)
 
