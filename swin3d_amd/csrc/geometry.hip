@@ -17,20 +17,22 @@ struct SegmentColumns {
 // query in one launch.  A network on 25,013 voxels: sixteen launches of 3.3 us before, eight of 1.8 now.
 __global__ __launch_bounds__(kThreads) void segment_ends_kernel(SegmentColumns columns, int count, int B, int32_t *__restrict__ out)
 {
-    const int at = static_cast<int>(blockIdx.x) * (kThreads / 64) + static_cast<int>(threadIdx.x) / 64, lane = threadIdx.x & 63;
-    if (at >= count * B) return;
-    const int which = at / B, b = at % B;
-    const int32_t *batch = which ? columns.batch[1] : columns.batch[0];
-    const int64_t stride = which ? columns.stride[1] : columns.stride[0];
-    int64_t lo = 0, hi = which ? columns.N[1] : columns.N[0];
-    while (lo < hi) {      // the end is from lo to hi
-        const int64_t piece = (hi - lo + 63) / 64, probe = min(lo + (lane + 1) * piece, hi) - 1;
-        const int below = __popcll(__ballot(batch[probe * stride] <= b));
-        const int64_t first = lo + below * piece;
-        hi = below == 64 ? hi : min(first + piece, hi) - 1;
-        lo = min(first, hi);
+    const int lane = threadIdx.x & 63, step = static_cast<int>(gridDim.x) * (kThreads / 64);
+    for (int64_t at = static_cast<int>(blockIdx.x) * (kThreads / 64) + static_cast<int>(threadIdx.x) / 64; at < static_cast<int64_t>(count) * B; at += step) {
+        const bool second = at >= B;
+        const int b = static_cast<int>(second ? at - B : at);
+        const int32_t *batch = second ? columns.batch[1] : columns.batch[0];
+        const int64_t stride = second ? columns.stride[1] : columns.stride[0];
+        int64_t lo = 0, hi = second ? columns.N[1] : columns.N[0];
+        while (lo < hi) {      // the end is from lo to hi
+            const int64_t piece = (hi - lo + 63) / 64, probe = min(lo + (lane + 1) * piece, hi) - 1;
+            const int below = __popcll(__ballot(batch[probe * stride] <= b));
+            const int64_t first = lo + below * piece;
+            hi = below == 64 ? hi : min(first + piece, hi) - 1;
+            lo = min(first, hi);
+        }
+        if (lane == 0) out[at] = static_cast<int32_t>(lo);
     }
-    if (lane == 0) out[at] = static_cast<int32_t>(lo);
 }
 
 // The voxels by their packed coordinates: an open table of at least twice as many slots, four neighbours in z side by side.
@@ -236,8 +238,9 @@ __global__ __launch_bounds__(kThreads) void level_signals_kernel(
 
 int launch_segment_ends(const SegmentColumns &columns, int count, int B, int32_t *out, hipStream_t stream)
 {
-    const int64_t wavefronts = static_cast<int64_t>(count) * B;
-    hipLaunchKernelGGL(segment_ends_kernel, dim3(static_cast<unsigned>(ceil_div(wavefronts, kThreads / 64))), dim3(kThreads), 0, stream, columns, count, B, out);
+    // (a launch has at most 2^32 threads, and an end has 64)
+    const int64_t blocks = ceil_div(static_cast<int64_t>(count) * B, kThreads / 64);
+    hipLaunchKernelGGL(segment_ends_kernel, dim3(static_cast<unsigned>(blocks < (1 << 16) ? blocks : 1 << 16)), dim3(kThreads), 0, stream, columns, count, B, out);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }

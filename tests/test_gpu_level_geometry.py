@@ -79,6 +79,17 @@ def test_ends_of_two_columns(hip_lib, sizes, batches):
         assert ends.dtype == torch.int32 and torch.equal(ends.cpu().long(), want) and torch.equal(encoder.segment_offsets(column, batches), ends)
 
 
+def test_ends_of_more_elements_than_a_launch_has_wavefronts(hip_lib):
+    """2^26 wavefronts are as many threads as a launch may have."""
+    from swin3d_amd import encoder
+    count = 2 ** 26 + 12_345
+    column = torch.tensor([0, 0, 3, 70_000, 2 ** 26 + 5], dtype=torch.int32, device="cuda")
+    ends = encoder.segment_offsets(column, count)
+    want = torch.full((count,), 4, dtype=torch.int32, device="cuda")
+    want[:3], want[3:70_000], want[2 ** 26 + 5:] = 2, 3, 5
+    assert torch.equal(ends, want)
+
+
 @pytest.mark.parametrize("n,stride", [(1, 1), (7, 1), (8, 2), (9, 3), (4096, 1), (4097, 2), (30011, 1)])
 def test_stem_neighbours_in_any_order_and_twice(hip_lib, n, stride):
     """Rows in any order, around the sizes where the table doubles, dense and sparse, some coordinates twice: the first
