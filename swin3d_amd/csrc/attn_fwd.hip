@@ -232,7 +232,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_attn_plan(
     if (D == 16 && dtype == S3D_DTYPE_F32 && attn_tile_shape(N, W, H, nd)) {
         if (int rc = launch_attn_tile(a, tile_list_of(a), static_cast<hipStream_t>(stream), kAttnBuildList)) return rc;
     }
-    const bool strips = D == 16 && dtype == S3D_DTYPE_F16 && attn_strip_shape(N, W, H);
+    const bool strips = D == 16 && dtype == S3D_DTYPE_F16 && attn_strip_shape(N, W, H, nd);
     const int what = kAttnBuildList | (strips && W <= kFewWindows ? kAttnStripList : 0);
     if (int rc = launch_attn_sweep(a, dtype, static_cast<hipStream_t>(stream), what)) return rc;
     return strips && W > kFewWindows ? launch_attn_strip(a, static_cast<hipStream_t>(stream), kAttnBuildList) : S3D_OK;

@@ -77,7 +77,7 @@ int launch_attn_tile(const AttnArgs &a, void *list, hipStream_t stream, int what
 // The strip kernel (attn_strip_fwd.hip), fp16: a workgroup works off strips of up to 16 queries of a window and a head, the
 // table products on the matrix pipe.  Its strip list lies where the sweep's list builder has its notes, which nothing reads once
 // that list is there: a plan with both builds the sweep's first, or both in one launch (kAttnStripList).  With sizes_dev as above.
-bool attn_strip_shape(int64_t N, int64_t W, int H);
+bool attn_strip_shape(int64_t N, int64_t W, int H, int nd);
 tile::StripList attn_strip_list(const AttnArgs &a);
 bool attn_strip_applies(const AttnArgs &a, int dtype);
 int launch_attn_strip(const AttnArgs &a, hipStream_t stream, int what = kAttnBuildList | kAttnSweep);

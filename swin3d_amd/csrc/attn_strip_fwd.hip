@@ -397,27 +397,30 @@ int launch_fwd(const AttnArgs &a, const StripList &list, hipStream_t stream)
 // fill the chip ends when its longest unit ends.  Measured, strips over the sweep (or over the kernel on 64 x 64 tiles that
 // served windows of 40 and more up to N^2 / W * H = 4 M), by (N / 16 + W) H, N / 16 + W being the most strips of a head:
 //   windows of 24 to 98 voxels, 9 axes: 0.15 to 0.72 up to 2300 (98 voxels, 24 heads 63 -> 9 us and, in two windows, 26 -> 13;
-//     1000 x 24 100 -> 33), 0.82 to 0.93 with 0.60 at 3000 x 12 up to 5500, 0.67 to 1.02 at 6800 to 8400, 1.1 to 1.24 at 11,000
-//     and beyond; 6 axes: 0.16 to 0.91 up to 5500, 1.10 at 7000 to 7300, 1.15 to 1.31 beyond
+//     1000 x 24 100 -> 33), 0.82 to 0.93 with 0.60 at 3000 x 12 up to 5500; over the sweep alone, 6 to 40 heads, 0.50 to 1.05, 0.91
+//     in the mean, at 6000 to 7200, 0.56 to 1.07, 0.94 in the mean, at 7200 to 8000, 0.69 to 1.14, 0.99 in the mean, at 8000 to 8800,
+//     1.1 to 1.24 at 11,000 and beyond; 6 axes: 0.16 to 0.91 up to 5500, 0.54 to 1.10, 0.95 in the mean, at 6000 to 7200, 0.63 to
+//     1.12, 0.99 in the mean, at 7200 to 8000, 0.78 to 1.23 at 8000 to 8800, 1.15 to 1.31 beyond (the sweep's time jumps with its
+//     cut into units, and the lines lie where strips lose little anywhere)
 //   windows of 5 to 11 voxels: 0.30 to 0.70 up to 2800, 0.70 to 1.15 at 3000 to 3700, 1.10 to 1.68 at 5500 to 7500
-constexpr int64_t kStripsMost = 6000, kStripsMostSmall = 3000, kStripMeanWindowSmall = 24;
+constexpr int64_t kStripsMost = 6000, kStripsMostNormals = 7200, kStripsMostSmall = 3000, kStripMeanWindowSmall = 24;
 
-bool attn_strip_shape(int64_t N, int64_t W, int H)
+bool attn_strip_shape(int64_t N, int64_t W, int H, int nd)
 {
-    return W > 0 && N < (int64_t(1) << tile::kPosBits) &&
-           (N / tile::kStrip + W) * H <= (N < kStripMeanWindowSmall * W ? kStripsMostSmall : kStripsMost);
+    const int64_t most = N < kStripMeanWindowSmall * W ? kStripsMostSmall : nd < 9 ? kStripsMost : kStripsMostNormals;
+    return W > 0 && N < (int64_t(1) << tile::kPosBits) && (N / tile::kStrip + W) * H <= most;
 }
 
 bool attn_strip_applies(const AttnArgs &a, int dtype)
 {
-    if (dtype != S3D_DTYPE_F16 || a.D != tile::D || !attn_strip_shape(a.N, a.W, a.H)) return false;
+    if (dtype != S3D_DTYPE_F16 || a.D != tile::D || !attn_strip_shape(a.N, a.W, a.H, a.nd)) return false;
     return a.sizes_dev || rows_fit_tiles(a.rows, a.nd);
 }
 
 tile::StripList attn_strip_list(const AttnArgs &a)
 {
     char *at = static_cast<char *>(attn_sweep_notes(a)) + kSweepNotesKept;
-    static_assert(kSweepNotesKept + 256 + sizeof(uint64_t) * kStripsMost <= kSweepNotesBytes, "the list fits");
+    static_assert(kSweepNotesKept + 256 + sizeof(uint64_t) * kStripsMostNormals <= kSweepNotesBytes, "the list fits");
     return {reinterpret_cast<const int32_t *>(at), reinterpret_cast<const uint64_t *>(at + 256)};
 }
 

@@ -20,6 +20,7 @@ SMALL = [3, 5, 8, 13, 1, 21]
     ("XYZ", 2, SMALL * 10),                    # a mean window below the rule's
     ("XYZ", 40, [64] * 25),                    # 5000 strips at most: more than one a workgroup
     ("XYZ", 40, [64] * 40),                    # beyond the rule: the sweep's
+    ("XYZ_RGB", 40, [64] * 32), ("XYZ_RGB_NORM", 40, [64] * 32), ("XYZ_RGB_NORM", 40, [64] * 37),      # 6400: with nine axes strips; 7400
     ("XYZ", 1, [5, 9] * 128), ("XYZ", 1, [5, 9] * 128 + [7]),      # windows whose lists one launch makes, and one more
 ])
 def test_strips_of_every_size(oracle_lib, hip_lib, cRSE, heads, sizes):
