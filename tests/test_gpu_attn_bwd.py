@@ -106,8 +106,9 @@ def test_dense_windows_up_to_343_voxels(oracle_lib, hip_lib, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("heads,dim", [(2, 8), (2, 16)])
 def test_window_sizes_at_the_kernel_boundaries(oracle_lib, hip_lib, dtype, heads, dim):
-    """Windows of exactly 1, 16, 31..33, 63..65, 127..129, 192 and 193 voxels: where the sweeps change their lane
-    mapping and start splitting a window into chunks of 64 owned elements."""
+    """Windows of exactly 1, 16, 31..33, 63..65, 127..129, 192 and 193 voxels: where a strip is full, a window's pairs are one
+    step's or a thread's, and a lane of the sweep that leaves the records (head_dim 8) shares its query with others.  (The sweeps
+    with tables that no strip takes: test_gpu_attn_pairs.py.)"""
     from test_gpu_attn import boundary_size_case
     case = boundary_size_case(oracle_lib, heads, dim, seed=71)
     if dtype == torch.float16:
@@ -135,8 +136,8 @@ def test_other_window_and_quant_sizes(oracle_lib, hip_lib, dtype, ws, quant, hea
 @pytest.mark.parametrize("seed", range(24))
 def test_random_shapes(oracle_lib, hip_lib, seed):
     """Randomly drawn shapes: head counts that do and do not divide the grid of workgroups evenly, both
-    head_dims (VALU and MFMA table-gradient updates), 3 / 6 / 9 axes, sparse to dense windows (every size class of
-    the unit list), several batch elements, strides and window shifts; fp32 on even seeds, fp16 on odd ones."""
+    head_dims (strips behind a sweep, behind strips and behind tiles), 3 / 6 / 9 axes, sparse to dense windows (every size class of
+    the lists), several batch elements, strides and window shifts; fp32 on even seeds, fp16 on odd ones."""
     rng = np.random.default_rng(2000 + seed)
     ws = int(rng.choice([3, 5, 7]))
     heads = int(rng.choice([1, 2, 3, 5, 6, 7]))
@@ -413,9 +414,9 @@ def test_headline_size_properties(hip_lib):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_repeated_calls(oracle_lib, hip_lib, dtype):
-    """dq, dk, dv have one owner per element and come out bit-identical on every call.  The table gradients are sums
-    of per-wavefront partial sums, and which units a wavefront draws from the work queues varies between calls: they
-    agree to fp32 rounding (1e-5 of the largest element here; 1e-6 is typical), not bit for bit."""
+    """dq, dk, dv have one owner per element and come out bit-identical on every call.  The table gradients agree to fp32
+    rounding (1e-5 of the largest element), which is what the operator promises: here, on strips, a workgroup's share is fixed; on the
+    sweeps (test_gpu_attn_pairs.py) which units a wavefront draws from the work queues varies between calls."""
     import swin3d_amd
     case = make_attn_case(oracle_lib, seed=77, n=20000, ws=5, quant=4, heads=6, dim=8, extent=(24, 24, 8), recipe="layer")
     dev = torch.device("cuda")
@@ -459,8 +460,8 @@ def test_pair_count_larger_than_needed(oracle_lib, hip_lib):
 
 @pytest.mark.parametrize("heads,dim", [(10, 16), (20, 16), (40, 16), (40, 8)])
 def test_head_counts_of_the_large_model(oracle_lib, hip_lib, heads, dim):
-    """Swin3D-L runs 10, 20 and 40 heads of 16 channels (many head groups: the sweeps' workgroups then take the
-    head groups in turn instead of in whole sets per XCD)."""
+    """Swin3D-L runs 10, 20 and 40 heads of 16 channels: few workgroups a head, and in sweeps (the forward's; at head_dim 8 the one
+    that leaves the records) workgroups that take the head groups in turn instead of in whole sets per XCD."""
     case = make_attn_case(oracle_lib, seed=300 + heads, n=700, ws=7, quant=4, heads=heads, dim=dim, extent=(12, 12, 6),
                           recipe="layer")
     _check(oracle_lib, case, torch.float16, seed=heads)
