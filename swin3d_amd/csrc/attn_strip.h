@@ -352,7 +352,7 @@ struct StripArgs {
     int64_t pairs;              // capacity of records per head; windows beyond it are not there
     const int4 *columns;        // [strip][column]: sorted position, row, window's first position, pairs before it (-1: beyond
                                 // the records)
-    const int32_t *column_rows; // [strip][column], and 64 more that nothing is made of
+    const int32_t *column_rows; // [strip][column]: the rows alone
     const float *scales;        // [head][Tq, Tk, Tv]: what a product with the table's operand is multiplied by
     float *slots;               // [workgroup][kind][tile][lane][4]: table gradients as the products leave them
     void *dq, *dk, *dv;

@@ -842,7 +842,7 @@ bool attn_strip8_applies(const int32_t *rows, int nd, int D, int dtype, int64_t 
     return dtype == S3D_DTYPE_F32 ? N * H <= kStripVoxelHeadsFloat : nd > 3 || N * H <= kStripVoxelHeads;
 }
 
-// slots | list | strips | columns | their rows (64 more) | scales
+// slots | list | strips | columns | their rows | scales
 size_t attn_strip8_bytes(int H, int nd, int64_t N, int64_t W)
 {
     return tile::slot_bytes(H, nd, 1) * 2 + tile::list_bytes(N, W) + tile::strips_bytes(N) + tile::strip_columns_bytes(N) +

@@ -9,8 +9,8 @@
 // No unit bounds it (811 voxels x 24: the VALU issues for 37 % of the time, the LDS is addressed for 27, the address unit works for
 // 26, the matrix pipe for 7): a launch of few strips is a chain of loads (list, row map, features: 9000 clocks to the first
 // product) and then 9000 to 10,000 clocks for each block of keys, of which a wavefront waits for two fifths, at barriers.  811 voxels
-// in windows of 90, 24 heads: 49 us on tiles of 64 x 64 pairs, which passed some thirty barriers where a strip passes nine, 40 here;
-// 390 voxels 33 -> 23, 98 voxels 26 -> 13.  The next strip's loads run ahead: every address that a wavefront's load touches takes a
+// in windows of 90, 24 heads: 49 us on tiles of 64 x 64 pairs, which passed some thirty barriers a tile, 40 here, where a strip passes
+// eight a block of keys and one more, seventeen in all; 390 voxels 33 -> 23, 98 voxels 26 -> 13.  The next strip's loads run ahead: every address that a wavefront's load touches takes a
 // clock of the CU's address unit, and with coordinates by lane and each wavefront's own copies of the keys (22 loads a strip in
 // place of 10) the same launches took 53, 30 and 16.
 #include "attn_strip.h"

@@ -80,7 +80,7 @@ inline size_t list_bytes(int64_t N, int64_t W)
 inline size_t list_max_strips(int64_t N) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(N > 0 ? N : 0) / (kCols + 1) + kCols + 1; }
 inline size_t strips_bytes(int64_t N) { return list_round(sizeof(int4) * list_max_strips(N)); }
 // a strip's voxels: see StripArgs
-inline size_t strip_columns_bytes(int64_t N) { return align_up(kStrip * list_max_strips(N) * (sizeof(int4) + sizeof(int32_t)) + 256, 256); }
+inline size_t strip_columns_bytes(int64_t N) { return align_up(kStrip * list_max_strips(N) * (sizeof(int4) + sizeof(int32_t)), 256); }
 inline UnitList list_at(void *p, int64_t N, int64_t W)
 {
     char *base = static_cast<char *>(p);
