@@ -249,40 +249,14 @@ struct WindowStrips {
 };
 inline size_t window_strips_most(int64_t N, int64_t W) { return static_cast<size_t>(N > 0 ? N : 0) / kStrip + static_cast<size_t>(W > 0 ? W : 0); }
 
-// By one workgroup: the strips of the largest windows first, bins of one size by a counting sort in LDS.  (A strip's result
-// does not depend on its place, so the order inside a bin may be any.)
+// By one workgroup, as the forward's list.
 __device__ __forceinline__ void build_window_strips(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
                                                     int32_t *__restrict__ total, int4 *__restrict__ strips)
 {
     __shared__ int at[kSizeBins];
     __shared__ long long wave_pairs[kListThreads / 64];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    auto bin = [](int n) { return kSizeBins - min(n, kSizeBins); };
-    if (t < kSizeBins) at[t] = 0;
-    __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n > 0) atomicAdd(&at[bin(n)], strips_of(n));
-    }
-    __syncthreads();
-    if (t < 64) {
-        int own[kSizeBins / 64], sum = 0;
-#pragma unroll
-        for (int e = 0; e < kSizeBins / 64; ++e) sum += own[e] = at[t * (kSizeBins / 64) + e];
-        int incl = sum;
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off);
-            if (t >= off) incl += up;
-        }
-        int run = incl - sum;
-#pragma unroll
-        for (int e = 0; e < kSizeBins / 64; ++e) {
-            at[t * (kSizeBins / 64) + e] = run;
-            run += own[e];
-        }
-        if (t == 63) total[0] = incl;
-    }
-    __syncthreads();
+    place_strips<kListThreads>(w_sizes, W, total, at);
     long long before = 0;              // pairs of the windows of earlier rounds
     for (int w0 = 0; w0 < W; w0 += kListThreads) {
         const int w = w0 + t, n = w < W ? max(w_sizes[w], 0) : 0;
@@ -300,7 +274,7 @@ __device__ __forceinline__ void build_window_strips(const int32_t *__restrict__ 
             before += wave_pairs[v];
         }
         if (n > 0) {
-            const int count = strips_of(n), first = atomicAdd(&at[bin(n)], count), pos = w2n[w];
+            const int count = strips_of(n), first = atomicAdd(&at[size_bin(n)], count), pos = w2n[w];
             // (a window that begins beyond 2^31 pairs does not fit any store)
             for (int q = 0; q < count; ++q) strips[first + q] = make_int4(pos, n, q, static_cast<int>(pairs < 0x7fffffffll ? pairs : 0x7fffffffll));
         }

@@ -103,29 +103,15 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
         r.load(x + (static_cast<uint64_t>(static_cast<uint32_t>(row)) * stride + static_cast<uint32_t>(opaque(4 * g4))));
     };
 
-    // A strip with a block of its window's keys: what the workgroup works off at a time.
-    struct Item {
-        int pos0, n, first, cols, blocks, block, first_pos, keys_n;
-        __device__ __forceinline__ void set_block(int which)
-        {
-            const int size = (n + blocks - 1) / blocks;
-            block = which;
-            first_pos = pos0 + block * size;
-            keys_n = min(size, n - block * size);
-        }
-        __device__ __forceinline__ void set(uint64_t s)
-        {
-            const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s >> 32));
-            constexpr uint32_t kMask = (1u << kPosBits) - 1;
-            pos0 = static_cast<int>(lo & kMask);
-            n = static_cast<int>((lo >> kPosBits | hi << (32 - kPosBits)) & kMask);
-            const int count = strips_of(n), size = (n + count - 1) / count;
-            first = static_cast<int>(hi >> (2 * kPosBits - 32)) * size;
-            cols = min(size, n - first);
-            blocks = (n + kKeyBlock - 1) / kKeyBlock;
-            set_block(0);
-        }
-    } item;
+    // A strip with a block of its window's keys is what the workgroup works off at a time.
+    using Item = StripItem<kKeyBlock>;
+    auto set = [](Item &i, uint64_t s) {
+        const uint32_t lo = static_cast<uint32_t>(s), hi = static_cast<uint32_t>(s >> 32);
+        constexpr uint32_t kMask = (1u << kPosBits) - 1;
+        i.set(make_int4(static_cast<int>(lo & kMask), static_cast<int>((lo >> kPosBits | hi << (32 - kPosBits)) & kMask),
+                        static_cast<int>(hi >> (2 * kPosBits - 32)), 0));
+    };
+    Item item;
     // Its rows, then its features and coordinates, are asked for while the item before is worked on.  A lane's pairs are those
     // of query c16 with the keys key0 + kReach s; as rows of a product the wavefront's keys are in the order in which its
     // result has them as these.  A key's coordinates are a number a lane of its sixteen: a broadcast among those is part of the
@@ -136,8 +122,8 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
     const int key0 = wave * (64 / kStrip) + g4;
     auto fetch_rows = [&](const Item &i) {
         rows.own = i.pos0 + i.first + min(c16, i.cols - 1);
-        rows.key = i.first_pos + min(wave * (64 / kStrip) + (c16 >> 2) + (c16 & 3) * kReach, i.keys_n - 1);
-        rows.operand = i.first_pos + min(wave * 16 + c16, i.keys_n - 1);
+        rows.key = i.pos0 + i.first_key + min(wave * (64 / kStrip) + (c16 >> 2) + (c16 & 3) * kReach, i.keys_n - 1);
+        rows.operand = i.pos0 + i.first_key + min(wave * 16 + c16, i.keys_n - 1);
         if (a.n2n) {
             rows.own = a.n2n[rows.own];
             rows.key = a.n2n[rows.key];
@@ -151,9 +137,9 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
         load_coords<ND>(a.n_coords + static_cast<int64_t>(i.pos0 + i.first + min(c16, i.cols - 1)) * ND, own);
 #pragma unroll
         for (int s = 0; s < kKeySteps; ++s)
-            other[s] = a.n_coords[static_cast<int64_t>(i.first_pos + min(key0 + s * kReach, i.keys_n - 1)) * ND + min(c16, ND - 1)];
+            other[s] = a.n_coords[static_cast<int64_t>(i.pos0 + i.first_key + min(key0 + s * kReach, i.keys_n - 1)) * ND + min(c16, ND - 1)];
     };
-    item.set(first_strip);
+    set(item, first_strip);
     fetch_rows(item);
 
     // The tables: tile 8 i + wave is this wavefront's.  Row 4 e + g of the tile is row 4 g + e of an operand: the lanes that
@@ -217,7 +203,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
         const int u_next = ends ? u + groups : u;
         Item next = item;
         if (ends) {
-            next.set(strip_ahead);
+            set(next, strip_ahead);
             strip_ahead = f.list.strips[min(u_next + groups, strips - 1)];
         } else {
             next.set_block(item.block + 1);
@@ -357,7 +343,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void attn_fwd_strip_kernel(FwdArg
     }
     if (!__syncthreads_or(again)) return;
     for (int u = group; u < strips; u += groups) {
-        item.set(f.list.strips[u]);
+        set(item, f.list.strips[u]);
         const int i = tid >> 3;
         if (i >= item.cols) continue;
         const int pos = item.pos0 + item.first + i;

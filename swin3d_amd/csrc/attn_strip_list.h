@@ -21,20 +21,19 @@ inline size_t strip_list_most(int64_t N, int64_t W) { return static_cast<size_t>
 
 #ifdef __HIPCC__
 // By one workgroup: the strips of the largest windows first, bins of one size by a counting sort in LDS.  (A strip's result does
-// not depend on its place, so the order inside a bin may be any.)
+// not depend on its place, so the order inside a bin may be any.)  place_strips leaves the places of the bins in `at`, from which
+// the windows then draw theirs.
 constexpr int kSizeBins = 256;
+__device__ __forceinline__ int size_bin(int n) { return kSizeBins - min(n, kSizeBins); }
 template <int kThreads>
-__device__ __forceinline__ void build_strip_list(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
-                                                 int32_t *__restrict__ total, uint64_t *__restrict__ strips)
+__device__ __forceinline__ void place_strips(const int32_t *__restrict__ w_sizes, int W, int32_t *__restrict__ total, int *at)
 {
-    __shared__ int at[kSizeBins];
     const int t = threadIdx.x;
-    auto bin = [](int n) { return kSizeBins - min(n, kSizeBins); };
     for (int b = t; b < kSizeBins; b += kThreads) at[b] = 0;
     __syncthreads();
     for (int w = t; w < W; w += kThreads) {
         const int n = w_sizes[w];
-        if (n > 0) atomicAdd(&at[bin(n)], strips_of(n));
+        if (n > 0) atomicAdd(&at[size_bin(n)], strips_of(n));
     }
     __syncthreads();
     if (t < 64) {
@@ -55,10 +54,17 @@ __device__ __forceinline__ void build_strip_list(const int32_t *__restrict__ w_s
         if (t == 63) total[0] = incl;
     }
     __syncthreads();
-    for (int w = t; w < W; w += kThreads) {
+}
+template <int kThreads>
+__device__ __forceinline__ void build_strip_list(const int32_t *__restrict__ w_sizes, const int32_t *__restrict__ w2n, int W,
+                                                 int32_t *__restrict__ total, uint64_t *__restrict__ strips)
+{
+    __shared__ int at[kSizeBins];
+    place_strips<kThreads>(w_sizes, W, total, at);
+    for (int w = threadIdx.x; w < W; w += kThreads) {
         const int n = w_sizes[w];
         if (n <= 0) continue;
-        const int count = strips_of(n), first = atomicAdd(&at[bin(n)], count);
+        const int count = strips_of(n), first = atomicAdd(&at[size_bin(n)], count);
         const uint64_t window = static_cast<uint64_t>(static_cast<uint32_t>(w2n[w])) | static_cast<uint64_t>(n) << kPosBits;
         for (int q = 0; q < count; ++q) strips[first + q] = window | static_cast<uint64_t>(q) << (2 * kPosBits);
     }

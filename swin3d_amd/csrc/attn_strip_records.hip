@@ -10,8 +10,8 @@
 // What bounds it: nothing by itself; the VALU issues for 48 % of the time, the address unit works for 53, the LDS for 36, the matrix
 // pipe for 20, and a wavefront waits for 38 %.  12,421 voxels in windows of 72, 9 axes, 12 heads, fp32 tables beside fp16 features:
 // 178 us, where tiles of 64 x 64 pairs took 196 (480,000 clocks, 398,000 here): a window of 72 is two such tiles of 36, whose
-// products are made at 64 x 64.  Layers of 12,421 to 49,682 voxels take 0.92 to 0.97 of what they took, forward included.  With 64
-// keys at a time, and so two blocks a window, 212 us; with the next item's features asked for behind the last stage, 189.
+// products are made at 64 x 64 (by size, against tiles: see the rule).  With 64 keys at a time, and so two blocks a window, 212
+// us; with the next item's features asked for behind the last stage, 189.
 #include "attn_strip.h"
 
 #include <algorithm>

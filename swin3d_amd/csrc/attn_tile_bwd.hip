@@ -334,8 +334,10 @@ bool attn_tile_bwd_applies(const int32_t *rows, int nd, int D, int64_t pairs)
 }
 
 // Where strips leave the records: fp16 features, windows of some size (a strip is of one window).  Strips over tiles, forward
-// included, layers of 60,000 to 100,000 voxels: 1.26 to 1.32 with windows of 4, 0.99 to 1.04 of 10, 0.91 to 0.95 of 17, 0.92 to 0.96
-// of 26 to 72; fp32 see above.
+// included, layers of 60,000 to 100,000 voxels: 1.26 to 1.32 with windows of 4, 0.99 to 1.04 of 10, 0.91 to 0.95 of 17; fp32 see
+// above.  The backward alone, windows of 30 to 98, 6 to 40 heads, by voxels (least, mean, most; fp32 tables | fp16 tables with 9 axes |
+// with 6): 98 to 811 0.78 0.87 0.94 | 0.78 0.87 0.94 | 0.78 0.89 0.97; 1,500 to 3,100 0.83 0.92 0.97 | 0.83 0.92 0.97 | 0.86 0.94 1.00;
+// 4,700 to 6,000 0.90 0.95 0.99 | 0.92 0.96 0.99 | 0.93 0.97 1.00; 9,400 to 75,000 0.94 0.98 1.02 | 0.96 0.99 1.02 | 0.97 1.01 1.04.
 constexpr int64_t kStripRecordsMeanWindow = 14;
 
 // records | slots | lists | strips and their columns | scales | what the kernel that leaves the records has
