@@ -150,7 +150,8 @@ def _plan_for(lib, w_sizes_in, w2n_in, w_sizes, w2n, c_sizes, sizes, nd, table_l
     plans = getattr(w_sizes_in, "_s3d_attn_plans", None)
     if plans is None:
         plans = w_sizes_in._s3d_attn_plans = {}
-    key = (h, d, code, tuple(sizes) if sizes is not None else None, n, stream)
+    # (which lists a plan has follows from the axes too, and how the sweep's is cut from the tables' length)
+    key = (h, d, code, tuple(sizes) if sizes is not None else (nd, table_len), n, stream)
     stamp = (w_sizes_in._version, w2n_in._version, w2n_in.data_ptr())
     kept = plans.get(key)
     if kept is not None and kept[0] == stamp:

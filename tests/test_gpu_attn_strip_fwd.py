@@ -42,3 +42,23 @@ def test_error_is_no_larger_than_the_sweeps(oracle_lib, hip_lib):
     strips, sweep = (run_attention(case, torch.float16), run_attention(case, torch.float16, return_stats=True)[0])
     error = [np.linalg.norm(x - ref) / np.linalg.norm(ref) for x in (strips, sweep)]
     assert error[0] <= 2.0 ** -11 / 3 ** 0.5 and error[0] <= error[1]
+
+
+@pytest.mark.parametrize("dtype,windows", [(torch.float16, 32), (torch.float32, 120)])
+@pytest.mark.parametrize("order", [(6, 9, 3), (9, 6, 9)])
+def test_plans_of_calls_with_more_or_fewer_axes(hip_lib, dtype, windows, order):
+    """One window set, table sizes on the device, between the lines for six axes and for nine: a plan has the lists of its own call."""
+    from swin3d_amd import window_attention_forward
+    gen = torch.Generator("cuda").manual_seed(windows)
+    heads, n = 40, 64 * windows
+    w_sizes = torch.full((windows,), 64, dtype=torch.int32, device="cuda")
+    w2n = (w_sizes.cumsum(0) - w_sizes).int()
+    n2n = torch.randperm(n, device="cuda", generator=gen).int()
+    q, k, v = (torch.randn(n, heads, 16, device="cuda", generator=gen).to(dtype) for _ in range(3))
+    for axes in order:
+        sizes = [20 * heads * 16] * axes
+        tables = [(0.1 * torch.randn(sum(sizes), device="cuda", generator=gen)).to(dtype) for _ in range(3)]
+        coords = 10 * torch.rand(n, axes, device="cuda", generator=gen)
+        got = window_attention_forward(0.25 * q, k, v, *tables, torch.tensor(sizes, dtype=torch.int32, device="cuda"), w_sizes, w2n, n2n, coords)
+        want = window_attention_forward(0.25 * q, k, v, *tables, sizes, w_sizes.clone(), w2n, n2n, coords)
+        assert torch.equal(got, want) and bool(got.isfinite().all()), axes
