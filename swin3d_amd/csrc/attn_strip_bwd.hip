@@ -52,7 +52,7 @@ namespace {
 // is treated alike.  A dout that is not finite leaves P alone.  At head_dim 16 the records kernel makes NaN of it all the same,
 // and so of all channels of dv and dTv; at 8 it does where no channel of dout is finite; elsewhere a workgroup goes
 // through its strips with such a dL once more and adds up, pair by pair, dv of the windows and what the voxel gives dTv.  (Every dout
-// infinite, 199,327 voxels x 6, fp16: 4.6 ms where the call takes 1.5, 10.4 pair by pair.)
+// infinite, 199,327 voxels x 6, fp16: 2.4 ms where the call takes 1.5, 8 more pair by pair.)
 constexpr float kFixWeight = 268435456.0f, kMostWeight = 8.0f;
 constexpr int kFixGrad = 30;
 template <typename TF> constexpr int kLift = sizeof(TF) == 2 ? 15 : 0;       // (fp32 features may be as large as fp32 is)
@@ -459,14 +459,24 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
                 const float2 r = settle(records[pair0 + j * step], fits, there);
                 if (finite(r.x)) continue;
                 if (kPacked && finite(r.y)) atomicOr(&met_s[u / groups / 32 % kMetWords], 1u << (u / groups & 31));
+                const bool weight = !finite(r.y);
+                int begin = 0;
+                if constexpr (ND == 3) asm volatile("" : "+s"(begin));      // (a loop all the same: coordinates kept for it take registers)
 #pragma unroll 1
-                for (int axis = 0; axis < ND; ++axis) {
-                    const int rows_n = axis_rows<ND>(a, axis);
-                    const float half_rows = static_cast<float>(rows_n / 2), upper = crse_upper(rows_n);
-                    const float mine = a.n_coords[static_cast<int64_t>(column.x) * ND + axis], its = coords[j * ND + axis];
-                    const int row = axis_row0(axis) + (kByKey ? crse_row(its, mine, half_rows, upper) : crse_row(mine, its, half_rows, upper));
-                    atomicOr(&marks_s[row >> 4], 1u << (row & 15));
-                    if (!finite(r.y)) atomicOr(&marks_s[kTiles<ND> + (row >> 4)], 1u << (row & 15));
+                for (int first = begin; first < ND; first += 3) {
+                    float mine[3], its[3];
+                    load_coords<3>(a.n_coords + static_cast<int64_t>(column.x) * ND + first, mine);
+                    load_coords<3>(coords + j * ND + first, its);
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        const int axis = first + e, rows_n = axis_rows<ND>(a, axis);
+                        const float half_rows = static_cast<float>(rows_n / 2), upper = crse_upper(rows_n);
+                        const int row = axis_row0(axis) + (kByKey ? crse_row(its[e], mine[e], half_rows, upper) : crse_row(mine[e], its[e], half_rows, upper));
+                        const uint32_t bit = 1u << (row & 15);
+                        // (most have been marked by then)
+                        if (!(marks_s[row >> 4] & bit)) atomicOr(&marks_s[row >> 4], bit);
+                        if (weight && !(marks_s[kTiles<ND> + (row >> 4)] & bit)) atomicOr(&marks_s[kTiles<ND> + (row >> 4)], bit);
+                    }
                 }
             }
         }
