@@ -532,7 +532,15 @@ int s3d_add_layernorm(const float *x, const void *residual, int32_t residual_dty
                       void *stream);
 
 /*
- * The gradients of that call with y in fp16: dx = dsum + the gradient of LayerNorm in fp32, dresidual the same in fp16,
+ * The same for training: sum = x + residual (fp16, widened first) and y = LayerNorm of it in fp16, with the bits that
+ * torch.nn.functional.layer_norm gives in fp32, rounded to the nearest.  residual and sum may be null (then the rows are x
+ * themselves).  All dense and 16-byte aligned, sum apart from x; C a multiple of 4 and at most 1024.
+ */
+int s3d_train_add_layernorm(const float *x, const void *residual, const float *gamma, const float *beta, float eps, float *sum,
+                            void *y, int64_t N, int32_t C, void *stream);
+
+/*
+ * The gradients of either call with y in fp16: dx = dsum + the gradient of LayerNorm in fp32, dresidual the same in fp16,
  * dgamma and dbeta [C] in fp32.  sum device [N,C] is the call's x_out (x without a residual), dsum fp32 [N,C] or null,
  * dy fp16 [N,C]; dx and dresidual may be null; all dense and 16-byte aligned.  The same bits on every call.
  */

@@ -2,7 +2,6 @@
 attention operator (Swin3D/modules/swin3d_layers.py:617-623)."""
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 from torch.autograd.function import Function
 
 from . import _lib
@@ -46,13 +45,18 @@ def add_layernorm(x, residual, norm, out_dtype=torch.float16, inplace=False):
     return summed, y
 
 
-def add_half(x, residual):
-    """x + residual for dense 16-byte aligned fp32 rows and a branch in fp16, widened by itself first, which is exact."""
-    out = torch.empty_like(x)
+def train_add_layernorm(x, residual, weight, bias, eps):
+    """(x + residual, LayerNorm of it in fp16) for dense 16-byte aligned fp32 rows and a branch in fp16 or None, with the bits of
+    torch's operations: a rounding of the mean elsewhere in fp32 moves single fp16 roundings of the rows, and with them the
+    gradients of an encoder on scans of 20,000 voxels by a fiftieth (see linear_grad.py)."""
+    summed = x if residual is None else torch.empty_like(x)
+    y = torch.empty_like(x, dtype=torch.float16)
     with _lib.on(x.device):
-        status = _lib.lib().s3d_add_half(x.data_ptr(), residual.data_ptr(), out.data_ptr(), x.numel(), _lib.stream(x.device))
-    _lib.check(status, "s3d_add_half")
-    return out
+        status = _lib.lib().s3d_train_add_layernorm(x.data_ptr(), None if residual is None else residual.data_ptr(), weight.data_ptr(),
+                                                    bias.data_ptr(), eps, None if residual is None else summed.data_ptr(), y.data_ptr(),
+                                                    x.shape[0], x.shape[1], _lib.stream(x.device))
+    _lib.check(status, "s3d_train_add_layernorm")
+    return summed, y
 
 
 class _AddNorm(Function):
@@ -61,10 +65,7 @@ class _AddNorm(Function):
     @staticmethod
     def forward(ctx, x, residual, weight, bias, norm):
         ctx.set_materialize_grads(False)
-        # torch's own forward: a rounding of the mean elsewhere in fp32 moves single fp16 roundings of the rows, and with
-        # them the gradients of an encoder on scans of 20,000 voxels by a fiftieth (see linear_grad.py)
-        summed = x if residual is None else add_half(x, residual)
-        y = F.layer_norm(summed, norm.normalized_shape, weight, bias, norm.eps).to(torch.float16)
+        summed, y = train_add_layernorm(x, residual, weight, bias, norm.eps)
         ctx.save_for_backward(summed, weight)
         ctx.eps, ctx.residual = norm.eps, residual is not None
         return summed, y

@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.autograd.function import Function
 
 from . import _lib
-from .fused_norm import _AddNorm, add_half
+from .fused_norm import _AddNorm, train_add_layernorm
 from .linear_grad import _Linear
 from .sparse_dl.attn import attn_coff
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
@@ -230,8 +230,7 @@ class _Branches(Function):
         (w_sizes, w2n, n2n, coords), call.index = call.index, None
         out, omax, osum = attn_coff._attention(q, k, v, [3 * row] * 3, *tables, call.sizes, w_sizes, w2n, n2n, coords, True)
         branch = F.linear(out.view(n, channels), copies[2], copies[3])
-        summed = add_half(x, branch)
-        normed2 = F.layer_norm(summed, (channels,), norm_weight, norm_bias, call.eps).to(torch.float16)
+        summed, normed2 = train_add_layernorm(x, branch, norm_weight, norm_bias, call.eps)
         hidden_in = F.linear(normed2, copies[4], copies[5])
         hidden_out = F.gelu(hidden_in)
         pending = F.linear(hidden_out, copies[6], copies[7])

@@ -36,6 +36,26 @@ def test_add_layernorm_at_the_edges_of_its_rows(hip_lib, channels, res_dtype):
     test_add_layernorm_matches_torch(hip_lib, channels, res_dtype, torch.float32)
 
 
+@pytest.mark.parametrize("channels", [4, 48, 64, 68, 96, 128, 132, 192, 256, 260, 384, 512, 516, 640, 768, 772, 1024])
+@pytest.mark.parametrize("residual", [False, True])
+def test_training_norm_has_the_bits_of_torch(hip_lib, channels, residual):
+    """Around the rows' lanes and parts a lane, rows far from zero, constant ones and such as are not finite among them."""
+    from swin3d_amd.fused_norm import train_add_layernorm
+    gen = torch.Generator(device="cuda").manual_seed(channels)
+    x = torch.randn(4099, channels, device="cuda", generator=gen) * torch.logspace(-3, 3, 4099, device="cuda")[:, None]
+    x += 10 * torch.randn(4099, 1, device="cuda", generator=gen)
+    x[5], x[6], x[7, 1], x[8, 2], x[9, 0], x[10], x[11] = 0, 3, float("nan"), float("inf"), float("-inf"), 3e19, x[12] * 1e30
+    branch = torch.randn(4099, channels, device="cuda", generator=gen).half() if residual else None
+    weight, bias = torch.rand(channels, device="cuda", generator=gen) + 0.5, torch.randn(channels, device="cuda", generator=gen)
+    for n in (4099, 1):
+        rows, beside = x[:n].contiguous(), None if branch is None else branch[:n]
+        want = rows if beside is None else rows + beside.float()
+        summed, y = train_add_layernorm(rows, beside, weight, bias, 1e-5)
+        assert torch.equal(summed.view(torch.int32), want.view(torch.int32))
+        norm = torch.nn.functional.layer_norm(want, (channels,), weight, bias, 1e-5).half()
+        assert torch.equal(y.isnan(), norm.isnan()) and torch.equal(y.nan_to_num(7).view(torch.int16), norm.nan_to_num(7).view(torch.int16))
+
+
 def test_inplace_and_empty(hip_lib):
     from swin3d_amd.fused_norm import add_layernorm
     dev = torch.device("cuda")
