@@ -556,6 +556,8 @@ int s3d_layernorm_grad(const float *sum, const float *dsum, const void *dy, cons
  */
 int s3d_linear(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, int32_t gelu,
                void *stream);
+/* The same without GELU, the K products of a number added up one after the other: the bits of a product that is not split. */
+int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, void *stream);
 
 /*
  * The gradients of that layer's weight and bias: dw = dy^T x [N,K] and db = column sums of dy [N], either may be null.

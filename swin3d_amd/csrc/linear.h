@@ -12,6 +12,7 @@ struct LinearArgs {
     int32_t N, K;
     bool gelu;
     const void *gelu_at = nullptr;   // [M,N] fp16: the rows, rounded, are gradients behind a GELU of these, and y those before it
+    bool in_order = false;           // a number's K products are added up one after the other, whatever the tile
 };
 
 int launch_linear(const LinearArgs &a, hipStream_t stream);

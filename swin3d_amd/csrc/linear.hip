@@ -355,7 +355,7 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     // 640 0.86 to 1.00; 520 at K = 320 4.8 / 5.8, at 640 5.9 / 6.2, at 2560 23.0 / 13.9; 588 at K = 1536 10.4 / 10.0; 980 at 2560 23.7 / 19.4,
     // at 640 6.3 / 8.0; 1880 at 2560 27.0 / 35.4.
     const int64_t thin = ceil_div(a.M, 32) * ((a.N + 31) / 32);
-    if (!a.gelu_at && (thin <= 256 || (thin <= 512 && a.K >= 192) || (thin <= 1024 && a.K >= 2048))) return launch_thin(a, stream);
+    if (!a.gelu_at && !a.in_order && (thin <= 256 || (thin <= 512 && a.K >= 192) || (thin <= 1024 && a.K >= 2048))) return launch_thin(a, stream);
     // Tiles of 64 x 64 as long as larger ones would leave CUs without work; then 128 rows by the width that pads N least,
     // the widest of those that still give every CU two tiles.  192 columns take all of a wavefront's registers: with GELU only
     // where the tile is the whole row, with its derivative not at all (63 would spill).
@@ -374,4 +374,10 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear(
     const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, int32_t gelu, void *stream)
 {
     return s3d::launch_linear(s3d::LinearArgs{x, w, bias, y, M, N, K, gelu != 0}, static_cast<hipStream_t>(stream));
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N,
+                                                                          int32_t K, void *stream)
+{
+    return s3d::launch_linear(s3d::LinearArgs{x, w, bias, y, M, N, K, false, nullptr, true}, static_cast<hipStream_t>(stream));
 }

@@ -1,12 +1,12 @@
-"""Dense layers in training under fp16 autocast: torch's product, and its gradients on the library's kernels (s3d_linear
-for the rows, s3d_linear_grad for weight and bias).  Tall rows and small weights are what the networks have, where a product
-that does not split the sum over the rows leaves most of the chip idle.
+"""Dense layers in training under fp16 autocast, on the library's kernels: the forward on s3d_linear_in_order, the gradients on
+s3d_linear (for the rows) and s3d_linear_grad (for weight and bias).  Tall rows and small weights are what the networks have,
+where a product that does not split the sum over the rows leaves most of the chip idle.
 
-The product of the forward is torch's to the bit, as it is outside of this file.  A sum over K in another order is no less
-exact, but it gives another sample of what fp16 activations do to the gradients of a network: on scans of 5,000 to 40,000
-voxels the gradients of Swin3D-S's encoder lie 1 to 5 % from those of an fp32 pass, and s3d_linear in the forward moved them
-by 0.1 to 1.6 % (single elements by up to a seventh of the largest).  With torch's product they are what they were to the
-scatter of two runs, 0.05 to 0.1 %."""
+The product of the forward is torch's to the bit, as it is outside of this file (dense_rows has where).  A sum over K in another
+order is no less exact, but it gives another sample of what fp16 activations do to the gradients of a network: on scans of 5,000
+to 40,000 voxels the gradients of Swin3D-S's encoder lie 1 to 5 % from those of an fp32 pass, and products that share K among
+wavefronts in the forward moved them by 0.1 to 1.6 % (single elements by up to a seventh of the largest).  With torch's bits they
+are what they were to the scatter of two runs, 0.05 to 0.1 %."""
 import torch
 import torch.nn.functional as F
 from torch.autograd.function import Function
@@ -44,6 +44,24 @@ def _weight_gradients(dy, x, want_weight, want_bias, dtype=torch.float32):
     return dw, db
 
 
+# torch's library adds up K in order, too, unless it splits it: for few rows (up to 31 at K from 384 to 768), for long K (1280: up to
+# 800 rows, 1536: 340, 2560: 26,000), and where a launch's last tiles would leave most of the chip idle (from 65,536 rows on).
+# The widths of both networks, 20 to 200,000 rows, 270,000 products: up to K = 768, from 32 rows on and below 65,536 at up to 240
+# channels, all of them have the same bits.  Beyond, 1 to 5 in 100 row counts have 10^-5 to 10^-4 of their numbers a rounding apart,
+# of layers that get narrower up to one in ten: those stay with torch.
+_LEAST_ROWS, _MOST_K, _MANY_ROWS = 64, 768, 65536
+
+
+def dense_rows(x, weight, bias):
+    """F.linear of fp16 operands in a forward that is trained: on the library's kernel where torch's has the same bits.  us, torch /
+    so: 199,327 rows of 48 to 144 53 / 18, to 192 54 / 19; 49,682 of 96 to 288 27 / 12, of 384 to 96 17 / 13; 12,421 of 192 to 576
+    16 / 9, of 768 to 192 10.2 / 10.3; 811 of 384 to 384 5.3 / 4.6."""
+    (n, k), out = weight.shape, None
+    if x.dim() == 2 and x.shape[0] >= _LEAST_ROWS and k <= _MOST_K and (n >= k or x.shape[0] < _MANY_ROWS):
+        out = linear_rows(x, weight, bias, in_order=True)
+    return F.linear(x, weight, bias) if out is None else out
+
+
 class _Linear(Function):
     """F.linear in fp16 of fp16 rows and parameters in fp16 or fp32, whose gradients come in their own type: autocast would
     round them to fp16 on the way."""
@@ -53,7 +71,7 @@ class _Linear(Function):
         half = weight.to(torch.float16)
         ctx.save_for_backward(x, weight, half)
         ctx.bias_dtype = None if bias is None else bias.dtype
-        return F.linear(x, half, None if bias is None else bias.to(torch.float16))
+        return dense_rows(x, half, None if bias is None else bias.to(torch.float16))
 
     @staticmethod
     def backward(ctx, dy):

@@ -124,9 +124,9 @@ def _applicable(parts, channels):
     return True
 
 
-def linear_rows(x, weight, bias, gelu=False):
-    """x @ weight.T + bias (then GELU) of fp16 rows on the library's kernel (s3d_linear); None where it does not take the
-    operands."""
+def linear_rows(x, weight, bias, gelu=False, in_order=False):
+    """x @ weight.T + bias (then GELU) of fp16 rows on the library's kernel (s3d_linear; in_order: without GELU, on
+    s3d_linear_in_order); None where it does not take the operands."""
     if not data_only(x) or x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] \
             or any(t is not None and (t.dtype != torch.float16 or t.device != x.device or not t.is_contiguous()
                                       or t.data_ptr() % 16) for t in (x, weight, bias)) \
@@ -135,9 +135,9 @@ def linear_rows(x, weight, bias, gelu=False):
         return None
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
     with _lib.on(x.device):
-        status = _lib.lib().s3d_linear(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
-                                       x.shape[0], weight.shape[0], x.shape[1], int(gelu),
-                                       _lib.stream(x.device))
+        call, more = (_lib.lib().s3d_linear_in_order, ()) if in_order else (_lib.lib().s3d_linear, (int(gelu),))
+        status = call(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), x.shape[0],
+                      weight.shape[0], x.shape[1], *more, _lib.stream(x.device))
     _lib.check(status, "s3d_linear")
     return out
 

@@ -17,7 +17,7 @@ from torch.autograd.function import Function
 
 from . import _lib
 from .fused_norm import _AddNorm, train_add_layernorm
-from .linear_grad import _Linear
+from .linear_grad import _Linear, dense_rows
 from .sparse_dl.attn import attn_coff
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .swin_blocks import _applicable, _parts, data_only, followed
@@ -224,16 +224,16 @@ class _Branches(Function):
             copies.append(half.as_strided((rows, cols), (cols, 1), at) if p.dim() == 2 else half.as_strided((rows,), (1,), at))
         starts = layout.to[-num_tables::num_tables // 3]
         tables = [half.as_strided((call.table_len,), (1,), at) for at in starts]
-        qkv = F.linear(normed, copies[0], copies[1])
+        qkv = dense_rows(normed, copies[0], copies[1])
         row = channels
         q, k, v = (qkv.as_strided((n, heads, dim), (3 * row, dim, 1), i * row) for i in range(3))
         (w_sizes, w2n, n2n, coords), call.index = call.index, None
         out, omax, osum = attn_coff._attention(q, k, v, [3 * row] * 3, *tables, call.sizes, w_sizes, w2n, n2n, coords, True)
-        branch = F.linear(out.view(n, channels), copies[2], copies[3])
+        branch = dense_rows(out.view(n, channels), copies[2], copies[3])
         summed, normed2 = train_add_layernorm(x, branch, norm_weight, norm_bias, call.eps)
-        hidden_in = F.linear(normed2, copies[4], copies[5])
+        hidden_in = dense_rows(normed2, copies[4], copies[5])
         hidden_out = F.gelu(hidden_in)
-        pending = F.linear(hidden_out, copies[6], copies[7])
+        pending = dense_rows(hidden_out, copies[6], copies[7])
         ctx.call, ctx.layout = call, layout
         ctx.unchecked = _unchecked(norm_bias, params)     # (leaves: their shapes, and where a replay's gradients go)
         ctx.save_for_backward(x, normed, norm_weight, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same,

@@ -5,7 +5,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from swin3d_amd import encoder
-from swin3d_amd.linear_grad import _weight_gradients, trained_linear
+from swin3d_amd.linear_grad import _weight_gradients, dense_rows, trained_linear
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +90,12 @@ def test_layer_keeps_its_hooks_in_training(hip_lib):
     with torch.autocast("cuda", dtype=torch.float16):
         encoder._linear(layer, torch.randn(8, 32, device="cuda", requires_grad=True)).sum().backward()
     assert calls == [1]
+
+
+@pytest.mark.parametrize("m", [63, 64, 811, 1563, 6250, 25013])      # torch's own, few tiles (whose K no wavefronts share), several
+@pytest.mark.parametrize("n,k", [(144, 48), (48, 192), (240, 80), (384, 384), (192, 768), (384, 1536), (13, 48)])
+def test_forward_of_a_layer_in_training_has_the_bits_of_torch(hip_lib, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, weight, bias = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k), (n,)))
+    for b in (bias, None):
+        assert torch.equal(dense_rows(x, weight, b), F.linear(x, weight, b))
