@@ -534,7 +534,7 @@ int s3d_add_layernorm(const float *x, const void *residual, int32_t residual_dty
 /*
  * The same for training: sum = x + residual (fp16, widened first) and y = LayerNorm of it in fp16, with the bits that
  * torch.nn.functional.layer_norm gives in fp32, rounded to the nearest.  residual and sum may be null (then the rows are x
- * themselves).  All dense and 16-byte aligned, sum apart from x; C a multiple of 4 and at most 1024.
+ * themselves).  All dense and 16-byte aligned, sum apart from x, y the residual's place or apart; C a multiple of 4 and at most 1024.
  */
 int s3d_train_add_layernorm(const float *x, const void *residual, const float *gamma, const float *beta, float eps, float *sum,
                             void *y, int64_t N, int32_t C, void *stream);
@@ -556,8 +556,12 @@ int s3d_layernorm_grad(const float *sum, const float *dsum, const void *dy, cons
  */
 int s3d_linear(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, int32_t gelu,
                void *stream);
-/* The same without GELU, the K products of a number added up one after the other: the bits of a product that is not split. */
-int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N, int32_t K, void *stream);
+/*
+ * The same without GELU, the K products of a number added up one after the other: the bits of a product that is not split.
+ * gelu, [M,N] or null: GELU (by erf, in fp32) of the rounded rows y, with the bits that torch's vectorized kernel gives.
+ */
+int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, void *gelu, int64_t M, int32_t N, int32_t K,
+                        void *stream);
 
 /*
  * The gradients of that layer's weight and bias: dw = dy^T x [N,K] and db = column sums of dy [N], either may be null.
@@ -604,6 +608,37 @@ size_t s3d_swin_blocks_workspace_bytes(int64_t N, int32_t C, int32_t hidden);
 int s3d_swin_blocks(const float *x, float *x_out, void *pending, int64_t N, int32_t H, int32_t D, int32_t hidden,
                     const int32_t *table_sizes, int32_t nd, int64_t table_len, const s3d_window_set *sets, int32_t num_sets,
                     const s3d_swin_block *blocks, int32_t num_blocks, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * A Swin block behind its first LayerNorm in training, in fp16 with parameters in fp32:
+ *   qkv = normed1 Wqkv^T + b;  attended = attention(qkv);  sum = x + (attended Wproj^T + b);  normed2 = LayerNorm(sum);
+ *   hidden_in = normed2 Wfc1^T + b;  hidden_out = GELU(hidden_in);  pending = hidden_out Wfc2^T + b
+ * in one host call: s3d_half_copies of the parameters, then products, attention and norm as s3d_linear_in_order, s3d_attn_fwd
+ * and s3d_train_add_layernorm give them.
+ *   params, copies   HOST, as for s3d_half_copies, which fills half and same
+ *   qkv_weight ..    where in half, in elements, the copies of a layer and the tables begin; -1: there is no such bias
+ *   pending          null: the last product is left to the caller
+ *   windows          HOST, as for s3d_swin_blocks
+ * N at least 1, C = H*D and hidden multiples of 16, C at most 1024; all device pointers 16-byte aligned.
+ */
+typedef struct {
+    const float *const *params;
+    const s3d_half_copy *copies;
+    int64_t num_copies;
+    void *half;
+    float *same;                                             /* or null */
+    int64_t qkv_weight, qkv_bias, proj_weight, proj_bias, fc1_weight, fc1_bias, fc2_weight, fc2_bias, table_q, table_k, table_v;
+    const float *norm2_weight, *norm2_bias, *x;              /* fp32 [C], [C], [N,C] */
+    const void *normed1;                                     /* fp16 [N,C] */
+    void *qkv, *attended;                                    /* fp16 [N,3C], [N,C] */
+    float *out_max, *out_sum, *sum;                          /* [N,H], [N,H], [N,C] */
+    void *normed2, *hidden_in, *hidden_out, *pending;        /* fp16 [N,C], [N,hidden], [N,hidden], [N,C] */
+    const s3d_window_set *windows;
+    float norm2_eps;
+} s3d_block_pass;
+
+int s3d_swin_block_train(const s3d_block_pass *pass, int64_t N, int32_t H, int32_t D, int32_t hidden, const int32_t *table_sizes, int32_t nd,
+                         int64_t table_len, void *stream);
 
 /*
  * The gradients of a Swin block behind its first LayerNorm, in training in fp16 with parameters in fp32:

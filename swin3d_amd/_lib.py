@@ -45,6 +45,15 @@ class HalfCopy(ctypes.Structure):
     _fields_ = [(n, _i64) for n in ("rows", "cols", "scaled_rows", "to", "transposed", "same")] + [("scale", ctypes.c_float)]
 
 
+class BlockPass(ctypes.Structure):
+    _fields_ = [("params", ctypes.POINTER(_vp)), ("copies", ctypes.POINTER(HalfCopy)), ("num_copies", _i64), ("half", _vp), ("same", _vp),
+                *((n, _i64) for n in ("qkv_weight", "qkv_bias", "proj_weight", "proj_bias", "fc1_weight", "fc1_bias", "fc2_weight", "fc2_bias",
+                                      "table_q", "table_k", "table_v")),
+                *((n, _vp) for n in ("norm2_weight", "norm2_bias", "x", "normed1", "qkv", "attended", "out_max", "out_sum", "sum", "normed2",
+                                     "hidden_in", "hidden_out", "pending")),
+                ("windows", ctypes.POINTER(WindowSet)), ("norm2_eps", ctypes.c_float)]
+
+
 class BlockSaved(ctypes.Structure):
     _fields_ = [(n, _vp) for n in ("normed1", "qkv", "attended", "out_max", "out_sum", "sum", "normed2", "hidden_in", "hidden_out",
                                    "qkv_weight_t", "proj_weight_t", "fc1_weight_t", "fc2_weight_t", "table_q", "table_k", "table_v",
@@ -90,6 +99,7 @@ SIGNATURES = {
     "s3d_add_half": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp]),
     "s3d_swin_block_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i64, _i64, _i64]),
     # saved grads dsum dpending | N H D hidden | sizes nd len | W pairs scale dtype | ws bytes stream
+    "s3d_swin_block_train": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _i32, _i64, _vp]),
     "s3d_swin_block_grad": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp, _i32, _i64, _i64, _i64, ctypes.c_float, _i32, _vp,
                                            ctypes.c_size_t, _vp]),
     "s3d_cast_half": (ctypes.c_int, [_vp, _vp, _vp, _i32, _vp]),
@@ -119,7 +129,7 @@ SIGNATURES = {
     "s3d_layernorm_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32]),
     "s3d_layernorm_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_float] + [_vp] * 4 + [_i64, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_linear": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp]),
-    "s3d_linear_in_order": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _vp]),
+    "s3d_linear_in_order": (ctypes.c_int, [_vp] * 5 + [_i64, _i32, _i32, _vp]),
     "s3d_linear_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32]),
     "s3d_linear_grad": (ctypes.c_int, [_vp] * 4 + [_i32, _i64, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_swin_blocks_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32]),

@@ -232,9 +232,9 @@ template <int G> __device__ __forceinline__ float of_first(float v)
 }
 
 template <int G, int PARTS, bool kResidual>
-__global__ __launch_bounds__(kLnThreads) void train_layernorm_kernel(const float *__restrict__ x, const __half *__restrict__ residual,
+__global__ __launch_bounds__(kLnThreads) void train_layernorm_kernel(const float *__restrict__ x, const __half *residual,
                                                                      const float *__restrict__ gamma, const float *__restrict__ beta, float eps,
-                                                                     float *__restrict__ sum, __half *__restrict__ y, int64_t N, int C)
+                                                                     float *__restrict__ sum, __half *y, int64_t N, int C)
 {
     const int lane = threadIdx.x % G;
     const int64_t row = (static_cast<int64_t>(blockIdx.x) * kLnThreads + threadIdx.x) / G;

@@ -13,6 +13,7 @@ struct LinearArgs {
     bool gelu;
     const void *gelu_at = nullptr;   // [M,N] fp16: the rows, rounded, are gradients behind a GELU of these, and y those before it
     bool in_order = false;           // a number's K products are added up one after the other, whatever the tile
+    void *gelu_out = nullptr;        // [M,N] fp16: GELU of y's rounded rows, beside them (in_order; without gelu and gelu_at)
 };
 
 int launch_linear(const LinearArgs &a, hipStream_t stream);

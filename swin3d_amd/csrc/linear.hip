@@ -53,7 +53,10 @@ __device__ __forceinline__ float gelu_slope(float x)
     return fmaf(x, phi, 0.5f * (1.0f + erff(0.7071067812f * x)));
 }
 
-enum class Behind { kNothing, kGelu, kGeluGrad };
+// x Phi(x) of a training forward, as torch has it: by the math library's erff, in this order of operations
+__device__ __forceinline__ float gelu_erf(float x) { return (x * 0.5f) * (1.0f + erff(x * 0.70710678f)); }
+
+enum class Behind { kNothing, kGelu, kGeluGrad, kGeluBeside };
 
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
@@ -87,8 +90,8 @@ template <int WM, int WN, int TM, int TN> struct Tile {
 template <typename L, Behind kBehind>
 __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
                                                              const _Float16 *__restrict__ bias, _Float16 *__restrict__ y,
-                                                             const _Float16 *__restrict__ gelu_at, int M, int N, int K, int tiles_n,
-                                                             int tiles)
+                                                             const _Float16 *__restrict__ gelu_at, _Float16 *__restrict__ gelu_out, int M,
+                                                             int N, int K, int tiles_n, int tiles)
 {
     constexpr int TM = L::kTM, TN = L::kTN;
     __shared__ __align__(16) char smem[L::kLds];
@@ -213,8 +216,14 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
 #pragma unroll
                     for (int k = 0; k < 8; ++k) v[k] = static_cast<_Float16>(static_cast<float>(v[k]) * gelu_slope(static_cast<float>(at[i][t][k])));
                 }
-                if (m0 + wave_m + i * 32 + r < M && n0 + wave_n + n < N)
-                    *reinterpret_cast<half8 *>(y + static_cast<int64_t>(m0 + wave_m + i * 32 + r) * N + n0 + wave_n + n) = v;
+                const int64_t to = static_cast<int64_t>(m0 + wave_m + i * 32 + r) * N + n0 + wave_n + n;
+                const bool there = m0 + wave_m + i * 32 + r < M && n0 + wave_n + n < N;
+                if (there) *reinterpret_cast<half8 *>(y + to) = v;
+                if constexpr (kBehind == Behind::kGeluBeside) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = static_cast<_Float16>(gelu_erf(static_cast<float>(v[k])));
+                    if (there) *reinterpret_cast<half8 *>(gelu_out + to) = v;
+                }
             }
         }
         buffer ^= 1;
@@ -230,13 +239,14 @@ int launch(const LinearArgs &a, hipStream_t stream)
     const int64_t tiles = ceil_div(a.M, L::kM) * tiles_n;
     if (tiles > (1 << 30)) return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M = %lld rows", (long long)a.M);
     auto kernel = a.gelu_at ? linear_kernel<L, Behind::kGeluGrad> : a.gelu ? linear_kernel<L, Behind::kGelu> : linear_kernel<L, Behind::kNothing>;
+    if constexpr (L::kTM == 1 && L::kTN == 1) kernel = a.gelu_out ? linear_kernel<L, Behind::kGeluBeside> : kernel;
     // as many workgroups as fit the chip (by LDS), or one a tile
     constexpr int kPerCu = 160 * 1024 / L::kLds < 2 ? 1 : 160 * 1024 / L::kLds < 4 ? 160 * 1024 / L::kLds : 4;
     const int64_t slots = static_cast<int64_t>(kPerCu) * device_cus();
     const dim3 grid(static_cast<unsigned>(ceil_div(tiles < slots ? tiles : slots, 8) * 8));
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, static_cast<const _Float16 *>(a.x), static_cast<const _Float16 *>(a.w),
                        static_cast<const _Float16 *>(a.bias), static_cast<_Float16 *>(a.y), static_cast<const _Float16 *>(a.gelu_at),
-                       static_cast<int>(a.M), a.N, a.K, tiles_n, static_cast<int>(tiles));
+                       static_cast<_Float16 *>(a.gelu_out), static_cast<int>(a.M), a.N, a.K, tiles_n, static_cast<int>(tiles));
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
@@ -359,7 +369,11 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     // Tiles of 64 x 64 as long as larger ones would leave CUs without work; then 128 rows by the width that pads N least,
     // the widest of those that still give every CU two tiles.  192 columns take all of a wavefront's registers: with GELU only
     // where the tile is the whole row, with its derivative not at all (63 would spill).
-    if (ceil_div(a.M, 64) * ((a.N + 63) / 64) < 1024) return launch<Tile<2, 2, 1, 1>>(a, stream);
+    // So, too, with erff's GELU beside the rows, whose fifty instructions a number overlap with other tiles' loads only where
+    // several tiles share a SIMD.  us, torch's GELU behind the layer / larger tiles / so: 199,327 rows of 48 to 192 47.0 / 50.9 / 45.0,
+    // 49,682 of 96 to 384 30.8 / 34.9 / 26.5, 12,421 of 192 to 768 25.8 / 23.3 / 17.1, 3,105 of 384 to 1536 19.9 / 14.9 / 12.6;
+    // 6,250 of 96 11.2 / 7.4.
+    if (a.gelu_out || ceil_div(a.M, 64) * ((a.N + 63) / 64) < 1024) return launch<Tile<2, 2, 1, 1>>(a, stream);
     auto padded = [&](int width) { return (a.N + width - 1) / width * width; };
     auto enough = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width) >= 512; };
     const int least = padded(64);
@@ -376,8 +390,11 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear(
     return s3d::launch_linear(s3d::LinearArgs{x, w, bias, y, M, N, K, gelu != 0}, static_cast<hipStream_t>(stream));
 }
 
-extern "C" __attribute__((visibility("default"))) int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, int64_t M, int32_t N,
-                                                                          int32_t K, void *stream)
+extern "C" __attribute__((visibility("default"))) int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y, void *gelu, int64_t M,
+                                                                          int32_t N, int32_t K, void *stream)
 {
-    return s3d::launch_linear(s3d::LinearArgs{x, w, bias, y, M, N, K, false, nullptr, true}, static_cast<hipStream_t>(stream));
+    s3d::LinearArgs a{x, w, bias, y, M, N, K, false};
+    a.in_order = true;
+    a.gelu_out = gelu;
+    return s3d::launch_linear(a, static_cast<hipStream_t>(stream));
 }

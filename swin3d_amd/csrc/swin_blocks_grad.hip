@@ -1,4 +1,4 @@
-// The gradients of a Swin block behind its first LayerNorm (Swin3D/modules/swin3d_layers.py:563-625) in one call:
+// A Swin block behind its first LayerNorm (Swin3D/modules/swin3d_layers.py:563-625) in training, and its gradients, a call each:
 //   sum = x + proj(attention(qkv(normed)));  pending = fc2(GELU(fc1(LayerNorm(sum))))
 //
 // What bounds a training pass on scans of 10,000 to 100,000 voxels is the host: through autograd a block's backward is
@@ -54,6 +54,41 @@ bool fits(int64_t N, int32_t H, int32_t D, int32_t hidden)
 
 }  // namespace
 }  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_swin_block_train(const s3d_block_pass *pass, int64_t N, int32_t H, int32_t D, int32_t hidden,
+                                                                           const int32_t *table_sizes, int32_t nd, int64_t table_len, void *stream)
+{
+    using namespace s3d;
+    if (!fits(N, H, D, hidden))
+        return fail(S3D_ERR_BAD_SHAPE, "s3d_swin_block_train: N=%lld H=%d D=%d hidden=%d (H D and hidden multiples of 16, H D at most 1024)",
+                    (long long)N, H, D, hidden);
+    if (!pass || !pass->windows || !table_sizes) return fail(S3D_ERR_NULL_POINTER, "s3d_swin_block_train: null pointer");
+    const s3d_block_pass &p = *pass;
+    const s3d_window_set &w = *p.windows;
+    if (!p.half || !p.norm2_weight || !p.norm2_bias || !p.x || !p.normed1 || !p.qkv || !p.attended || !p.out_max || !p.out_sum || !p.sum || !p.normed2 ||
+        !p.hidden_in || !p.hidden_out || p.qkv_weight < 0 || p.proj_weight < 0 || p.fc1_weight < 0 || p.fc2_weight < 0 || p.table_q < 0 ||
+        p.table_k < 0 || p.table_v < 0)
+        return fail(S3D_ERR_NULL_POINTER, "s3d_swin_block_train: null device pointer");
+    if (p.num_copies < 0 || p.num_copies > 0x7fffffff) return fail(S3D_ERR_BAD_SHAPE, "s3d_swin_block_train: %lld copies", (long long)p.num_copies);
+    if (int rc = s3d_half_copies(p.params, p.copies, static_cast<int32_t>(p.num_copies), p.half, p.same, stream)) return rc;
+    const int32_t C = H * D;
+    const size_t row = static_cast<size_t>(C) * 2;
+    auto at = [&](int64_t element) { return element < 0 ? nullptr : static_cast<const char *>(p.half) + 2 * element; };
+    auto dense = [&](const void *x, int64_t weight, int64_t bias, void *y, void *gelu, int32_t n, int32_t k) {
+        return s3d_linear_in_order(x, at(weight), at(bias), y, gelu, N, n, k, stream);
+    };
+    if (int rc = dense(p.normed1, p.qkv_weight, p.qkv_bias, p.qkv, nullptr, 3 * C, C)) return rc;
+    const char *qkv = static_cast<const char *>(p.qkv);
+    if (int rc = s3d_attn_fwd(qkv, qkv + row, qkv + 2 * row, at(p.table_q), at(p.table_k), at(p.table_v), table_sizes, nd, table_len, w.w_sizes,
+                              w.w2n, w.n2n, w.n_coords, p.attended, p.out_max, p.out_sum, N, H, D, w.num_windows, 3 * C, S3D_DTYPE_F16,
+                              w.planned ? S3D_ATTN_PLANNED : 0, w.plan, w.plan_bytes, stream))
+        return rc;
+    // (proj's rows are needed until the norm has added them: in the place of the norm's rows that come after)
+    if (int rc = dense(p.attended, p.proj_weight, p.proj_bias, p.normed2, nullptr, C, C)) return rc;
+    if (int rc = s3d_train_add_layernorm(p.x, p.normed2, p.norm2_weight, p.norm2_bias, p.norm2_eps, p.sum, p.normed2, N, C, stream)) return rc;
+    if (int rc = dense(p.normed2, p.fc1_weight, p.fc1_bias, p.hidden_in, p.hidden_out, hidden, C)) return rc;
+    return p.pending ? dense(p.hidden_out, p.fc2_weight, p.fc2_bias, p.pending, nullptr, C, hidden) : S3D_OK;
+}
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_swin_block_grad_workspace_bytes(
     int64_t N, int32_t H, int32_t D, int32_t hidden, int32_t nd, int64_t table_len, int64_t W, int64_t pairs)

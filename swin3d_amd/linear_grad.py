@@ -52,13 +52,16 @@ def _weight_gradients(dy, x, want_weight, want_bias, dtype=torch.float32):
 _LEAST_ROWS, _MOST_K, _MANY_ROWS = 64, 768, 65536
 
 
+def has_torchs_bits(m, n, k):
+    """A product of m rows of k channels by a weight [n, k] in order is torch's."""
+    return m >= _LEAST_ROWS and k <= _MOST_K and (n >= k or m < _MANY_ROWS)
+
+
 def dense_rows(x, weight, bias):
     """F.linear of fp16 operands in a forward that is trained: on the library's kernel where torch's has the same bits.  us, torch /
     so: 199,327 rows of 48 to 144 53 / 18, to 192 54 / 19; 49,682 of 96 to 288 27 / 12, of 384 to 96 17 / 13; 12,421 of 192 to 576
     16 / 9, of 768 to 192 10.2 / 10.3; 811 of 384 to 384 5.3 / 4.6."""
-    (n, k), out = weight.shape, None
-    if x.dim() == 2 and x.shape[0] >= _LEAST_ROWS and k <= _MOST_K and (n >= k or x.shape[0] < _MANY_ROWS):
-        out = linear_rows(x, weight, bias, in_order=True)
+    out = linear_rows(x, weight, bias, in_order=True) if x.dim() == 2 and has_torchs_bits(x.shape[0], *weight.shape) else None
     return F.linear(x, weight, bias) if out is None else out
 
 

@@ -135,9 +135,10 @@ def linear_rows(x, weight, bias, gelu=False, in_order=False):
         return None
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float16, device=x.device)
     with _lib.on(x.device):
-        call, more = (_lib.lib().s3d_linear_in_order, ()) if in_order else (_lib.lib().s3d_linear, (int(gelu),))
-        status = call(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), x.shape[0],
-                      weight.shape[0], x.shape[1], *more, _lib.stream(x.device))
+        operands = x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr()
+        sizes, stream = (x.shape[0], weight.shape[0], x.shape[1]), _lib.stream(x.device)
+        status = _lib.lib().s3d_linear_in_order(*operands, None, *sizes, stream) if in_order else \
+            _lib.lib().s3d_linear(*operands, *sizes, int(gelu), stream)
     _lib.check(status, "s3d_linear")
     return out
 

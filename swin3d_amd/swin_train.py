@@ -4,7 +4,8 @@
 
 Layer by layer that is a dozen nodes, some thirty copies and casts of parameters and fifty dispatches of the backward, which
 on scans of up to 100,000 voxels take the host longer than the kernels take the device.  Here the parameters are cast,
-scaled and transposed by one launch (s3d_half_copies), and the backward is one call of the library (s3d_swin_block_grad).
+scaled and transposed by one launch (s3d_half_copies), and forward and backward are one call of the library each
+(s3d_swin_block_train, s3d_swin_block_grad).
 
 The forward's products and norm are torch's to the bit, as in linear_grad.py, for the reason given there."""
 import ctypes
@@ -17,7 +18,7 @@ from torch.autograd.function import Function
 
 from . import _lib
 from .fused_norm import _AddNorm, train_add_layernorm
-from .linear_grad import _Linear, dense_rows
+from .linear_grad import _Linear, dense_rows, has_torchs_bits
 from .sparse_dl.attn import attn_coff
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
 from .swin_blocks import _applicable, _parts, data_only, followed
@@ -197,43 +198,110 @@ def _by_parts(call, index, x, normed, norm_weight, norm_bias, params, before, no
     return summed, _Linear.apply(F.gelu(_Linear.apply(normed2, fc1_weight, fc1_bias)), fc2_weight, fc2_bias)
 
 
+def _in_one_call(call, x, normed, norm_weight, norm_bias, given, params, layout, half, same, index):
+    """(qkv, attended, its maxima and sums, sum, normed2, hidden_in, hidden_out, pending) of a block by s3d_swin_block_train, the last
+    product by torch where that has bits of its own; None where one of the others' is torch's too, or where the index has to be
+    looked at first."""
+    (n, channels), dev = x.shape, x.device
+    hidden, heads, dim, nd = call.hidden, call.heads, call.dim, len(call.sizes)
+    w_sizes, w2n, n2n, coords = index
+    if not (has_torchs_bits(n, 3 * channels, channels) and has_torchs_bits(n, channels, channels) and has_torchs_bits(n, hidden, channels)) \
+            or w_sizes.dim() != 1 or w2n.shape != w_sizes.shape or not (n2n is None or n2n.shape == (n,)) \
+            or not (x.is_contiguous() and normed.is_contiguous()) or (x.data_ptr() | normed.data_ptr()) % 16:
+        return None
+    last = has_torchs_bits(n, channels, hidden)
+    qkv, out, normed2, hidden_in, hidden_out = (torch.empty(shape, dtype=torch.float16, device=dev) for shape in (
+        (n, 3 * channels), (n, heads, dim), (n, channels), (n, hidden), (n, hidden)))
+    pending = torch.empty((n, channels), dtype=torch.float16, device=dev) if last else None
+    summed, omax, osum = (torch.empty(shape, dtype=torch.float32, device=dev) for shape in ((n, channels), (n, heads), (n, heads)))
+    c_sizes = (ctypes.c_int32 * nd)(*call.sizes)
+    p, s = _lib.BlockPass(), _lib.WindowSet()
+    lib = _lib.lib()
+    with _lib.on(dev):
+        stream = _lib.stream(dev)
+        w_sizes32, w2n32 = attn_coff._as_int32("w_sizes", w_sizes, dev), attn_coff._as_int32("w2n_indices", w2n, dev)
+        n2n32 = None if n2n is None else attn_coff._as_int32("n2n_indices", n2n, dev)
+        windows = w_sizes32.numel()
+        plan = attn_coff._plan_for(lib, w_sizes, w2n, w_sizes32, w2n32, c_sizes, call.sizes, nd, call.table_len, n, heads, dim,
+                                   _lib.S3D_DTYPE_F16, stream) if attn_coff.REUSE_PLANS else None
+        s.planned = plan is not None
+        if plan is None:
+            plan = torch.empty(lib.s3d_attn_plan_bytes(heads, n, windows), dtype=torch.uint8, device=dev)
+        s.w_sizes, s.w2n, s.n2n, s.n_coords = w_sizes32.data_ptr(), w2n32.data_ptr(), None if n2n is None else n2n32.data_ptr(), coords.data_ptr()
+        s.num_windows, s.plan, s.plan_bytes = windows, plan.data_ptr(), plan.numel()
+        p.params, p.copies, p.num_copies = (ctypes.c_void_p * len(given))(*[t.data_ptr() for t in given]), layout.copies, len(given)
+        p.half, p.same = half.data_ptr(), None if same is None else same.data_ptr()
+        places = iter(layout.to)
+        (p.qkv_weight, p.qkv_bias, p.proj_weight, p.proj_bias, p.fc1_weight, p.fc1_bias, p.fc2_weight, p.fc2_bias) = (
+            -1 if t is None else next(places) for t in params[:8])
+        p.table_q, p.table_k, p.table_v = _table_places(layout, params)
+        p.norm2_weight, p.norm2_bias, p.norm2_eps = norm_weight.data_ptr(), norm_bias.data_ptr(), call.eps
+        p.x, p.normed1, p.qkv, p.attended, p.out_max, p.out_sum = (t.data_ptr() for t in (x, normed, qkv, out, omax, osum))
+        p.sum, p.normed2, p.hidden_in, p.hidden_out = (t.data_ptr() for t in (summed, normed2, hidden_in, hidden_out))
+        p.pending, p.windows = None if pending is None else pending.data_ptr(), ctypes.pointer(s)
+        status = lib.s3d_swin_block_train(ctypes.byref(p), n, heads, dim, hidden, c_sizes, nd, call.table_len, stream)
+    _lib.check(status, "s3d_swin_block_train")
+    if pending is None:
+        pending = F.linear(hidden_out, *_layer_copies(layout, params, half)[6:])
+    return qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, pending
+
+
+def _table_places(layout, params):
+    """Where the query, key and value tables begin in the copies."""
+    num_tables = len(params) - 8
+    return layout.to[-num_tables::num_tables // 3]
+
+
+def _layer_copies(layout, params, half):
+    """The fp16 copies of the layers' weights and biases."""
+    places, copies = iter(zip(layout.shapes, layout.to)), []
+    for p in params[:8]:
+        if p is None:
+            copies.append(None)
+            continue
+        (rows, cols), at = next(places)
+        copies.append(half.as_strided((rows, cols), (cols, 1), at) if p.dim() == 2 else half.as_strided((rows,), (1,), at))
+    return copies
+
+
+def _layer_by_layer(call, x, normed, norm_weight, norm_bias, given, params, layout, half, same, index):
+    """The same by a call for each: where torch splits the sums of one of the products (few rows, or many channels)."""
+    n, channels = x.shape
+    heads, dim, dev = call.heads, call.dim, x.device
+    lib = _lib.lib()
+    with _lib.on(dev):
+        status = lib.s3d_half_copies((ctypes.c_void_p * len(given))(*[p.data_ptr() for p in given]), layout.copies, len(given),
+                                     half.data_ptr(), None if same is None else same.data_ptr(), _lib.stream(dev))
+    _lib.check(status, "s3d_half_copies")
+    copies = _layer_copies(layout, params, half)
+    tables = [half.as_strided((call.table_len,), (1,), at) for at in _table_places(layout, params)]
+    qkv = dense_rows(normed, copies[0], copies[1])
+    row = channels
+    q, k, v = (qkv.as_strided((n, heads, dim), (3 * row, dim, 1), i * row) for i in range(3))
+    out, omax, osum = attn_coff._attention(q, k, v, [3 * row] * 3, *tables, call.sizes, *index, True)
+    branch = dense_rows(out.view(n, channels), copies[2], copies[3])
+    summed, normed2 = train_add_layernorm(x, branch, norm_weight, norm_bias, call.eps)
+    hidden_in = dense_rows(normed2, copies[4], copies[5])
+    hidden_out = F.gelu(hidden_in)
+    return qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, dense_rows(hidden_out, copies[6], copies[7])
+
+
 class _Branches(Function):
     @staticmethod
     def forward(ctx, call, x, normed, norm_weight, norm_bias, *params):
         ctx.set_materialize_grads(False)
-        n, channels = x.shape
-        heads, dim, dev = call.heads, call.dim, x.device
+        channels, dev = x.shape[1], x.device
         given = [p for p in params if p is not None]
-        num_tables = len(params) - 8
         # (the backward of mode 1 reads the tables in fp32)
-        layout = _layout(_shapes(given), num_tables, channels, call.scale, call.mode == 1)
+        layout = _layout(_shapes(given), len(params) - 8, channels, call.scale, call.mode == 1)
         half = torch.empty(layout.half_count, dtype=torch.float16, device=dev)
         same = torch.empty(layout.same_count, dtype=torch.float32, device=dev) if layout.same_count else None
-        lib = _lib.lib()
-        with _lib.on(dev):
-            status = lib.s3d_half_copies((ctypes.c_void_p * len(given))(*[p.data_ptr() for p in given]), layout.copies, len(given),
-                                         half.data_ptr(), None if same is None else same.data_ptr(), _lib.stream(dev))
-        _lib.check(status, "s3d_half_copies")
-        places = iter(zip(layout.shapes, layout.to))
-        copies = []
-        for p in params[:8]:
-            if p is None:
-                copies.append(None)
-                continue
-            (rows, cols), at = next(places)
-            copies.append(half.as_strided((rows, cols), (cols, 1), at) if p.dim() == 2 else half.as_strided((rows,), (1,), at))
-        starts = layout.to[-num_tables::num_tables // 3]
-        tables = [half.as_strided((call.table_len,), (1,), at) for at in starts]
-        qkv = dense_rows(normed, copies[0], copies[1])
-        row = channels
-        q, k, v = (qkv.as_strided((n, heads, dim), (3 * row, dim, 1), i * row) for i in range(3))
         (w_sizes, w2n, n2n, coords), call.index = call.index, None
-        out, omax, osum = attn_coff._attention(q, k, v, [3 * row] * 3, *tables, call.sizes, w_sizes, w2n, n2n, coords, True)
-        branch = dense_rows(out.view(n, channels), copies[2], copies[3])
-        summed, normed2 = train_add_layernorm(x, branch, norm_weight, norm_bias, call.eps)
-        hidden_in = dense_rows(normed2, copies[4], copies[5])
-        hidden_out = F.gelu(hidden_in)
-        pending = dense_rows(hidden_out, copies[6], copies[7])
+        index = (w_sizes, w2n, n2n, coords)
+        made = _in_one_call(call, x, normed, norm_weight, norm_bias, given, params, layout, half, same, index)
+        if made is None:
+            made = _layer_by_layer(call, x, normed, norm_weight, norm_bias, given, params, layout, half, same, index)
+        qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, pending = made
         ctx.call, ctx.layout = call, layout
         ctx.unchecked = _unchecked(norm_bias, params)     # (leaves: their shapes, and where a replay's gradients go)
         ctx.save_for_backward(x, normed, norm_weight, qkv, out, omax, osum, summed, normed2, hidden_in, hidden_out, half, same,
@@ -266,7 +334,7 @@ class _Branches(Function):
         saved.qkv_weight_t, saved.proj_weight_t, saved.fc1_weight_t, saved.fc2_weight_t = (base + 2 * at for at in layout.transposed if at >= 0)
         num_tables = len(params) - 8
         if same is None:
-            saved.table_q, saved.table_k, saved.table_v = (base + 2 * at for at in layout.to[-num_tables::num_tables // 3])
+            saved.table_q, saved.table_k, saved.table_v = (base + 2 * at for at in _table_places(layout, params))
         else:
             saved.table_q, saved.table_k, saved.table_v = (same.data_ptr() + 4 * i * call.table_len for i in range(3))
         saved.norm2_weight, saved.norm2_eps = norm_weight.data_ptr(), call.eps

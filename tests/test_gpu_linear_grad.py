@@ -99,3 +99,35 @@ def test_forward_of_a_layer_in_training_has_the_bits_of_torch(hip_lib, m, n, k):
     x, weight, bias = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k), (n,)))
     for b in (bias, None):
         assert torch.equal(dense_rows(x, weight, b), F.linear(x, weight, b))
+
+
+def _rows_and_gelu(x, weight, bias):
+    from swin3d_amd import _lib
+    y, gelu = (torch.full((x.shape[0], weight.shape[0]), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    status = _lib.lib().s3d_linear_in_order(x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), gelu.data_ptr(),
+                                            x.shape[0], weight.shape[0], x.shape[1], _lib.stream(x.device))
+    _lib.check(status, "s3d_linear_in_order")
+    return y, gelu
+
+
+def _same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7), b.nan_to_num(7))      # (torch has zeros of either sign)
+
+
+def test_gelu_of_a_training_forward_has_the_bits_of_torch(hip_lib):
+    """Of every fp16 number, infinities and NaN among them."""
+    values = torch.arange(-32768, 32768, device="cuda").to(torch.int16).view(torch.float16)
+    x, weight = (torch.zeros(s, dtype=torch.float16, device="cuda") for s in ((65536, 16), (8, 16)))
+    x[:, 0], weight[:, 0] = values, 1
+    y, gelu = _rows_and_gelu(x, weight, None)
+    assert torch.equal(y[:, 3].isnan(), values.isnan()) and torch.equal(y[:, 3].nan_to_num(7), values.nan_to_num(7))
+    assert _same(gelu, F.gelu(y))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 8, 16), (63, 64, 48), (129, 72, 64), (16387, 192, 48), (16385, 384, 96), (70001, 72, 16)])      # each tile, and its edges
+def test_gelu_beside_a_layers_rows(hip_lib, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x, weight, bias = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k), (n,)))
+    y, gelu = _rows_and_gelu(x, weight, bias)
+    from swin3d_amd.swin_blocks import linear_rows
+    assert torch.equal(y, linear_rows(x, weight, bias, in_order=True)) and _same(gelu, F.gelu(y))
