@@ -208,3 +208,28 @@ def test_parameters_changed_between_forward_and_backward(hip_lib, monkeypatch, h
     monkeypatch.setattr(encoder, "trained_branches", lambda *_: None)
     # (the second gradients: the first ones' difference and a product of the same kind again)
     close(whole, gradients(True, create_graph=True), 4e-3)
+
+
+def test_gelus_derivative_at_every_fp16_number(hip_lib):
+    """fc1 gives its bias, fc2 passes one row's gradient on to the whole hidden layer: fc1's bias has the derivative as its gradient."""
+    hidden, values = 16384, torch.arange(-32768, 32768).to(torch.int16).view(torch.float16)
+    stage, feats, run = _stage(100, 16, 1, 5, 2, "XYZ_RGB", 3)
+    block, dev = stage.blocks[-1], feats.device
+    block.mlp = encoder.Mlp(16, hidden).to(dev)
+    torch.nn.init.zeros_(block.mlp.fc1.weight)
+    torch.nn.init.zeros_(block.mlp.fc2.weight)
+    block.mlp.fc2.weight.data[0] = 1
+    grad = torch.zeros_like(feats)
+    grad[7, 0] = 1
+    for first in range(0, 65536, hidden):
+        x = values[first:first + hidden]
+        block.mlp.fc1.bias.data.copy_(x)
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = run(feats)
+        assert any("Branches" in name for name in _nodes(out))
+        got = torch.autograd.grad(out, block.mlp.fc1.bias, grad)[0].double().cpu()
+        finite, x = x.isfinite(), x.double()
+        assert got[~finite].isnan().all()
+        want = 0.5 * (1 + torch.erf(x / 2 ** 0.5)) + x * torch.exp(-x * x / 2) / (2 * torch.pi) ** 0.5
+        # the rounding to fp16, and of fp32 before it
+        assert ((got - want).abs() <= 2 ** -11 * want.abs() + 2 ** -25 + 1.5e-7)[finite].all()
