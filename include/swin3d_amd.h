@@ -564,6 +564,14 @@ int s3d_linear_in_order(const void *x, const void *w, const void *bias, void *y,
                         void *stream);
 
 /*
+ * Both layers of an MLP in one kernel, y = fc2(GELU(fc1(x))), with the bits of two calls of s3d_linear on many rows: x, y device
+ * [M,C], apart; w1 [hidden,C], b1 [hidden] or null, w2 [C,hidden], b2 [C] or null; fp16, dense and 16-byte aligned.  hidden a
+ * multiple of 32 up to 1024, C one of 48, 64, 80, 96, 128, 160 and 192.
+ */
+int s3d_mlp(const void *x, const void *w1, const void *b1, const void *w2, const void *b2, void *y, int64_t M, int32_t C, int32_t hidden,
+            void *stream);
+
+/*
  * The gradients of that layer's weight and bias: dw = dy^T x [N,K] and db = column sums of dy [N], either may be null.
  * dy device [M,N], x device [M,K], fp16, dense and 16-byte aligned; dw, db of grad_dtype (fp32 sums, rounded once for
  * fp16); N and K multiples of 8, M at least 1.  The same bits on every call.

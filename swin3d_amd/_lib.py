@@ -130,6 +130,7 @@ SIGNATURES = {
     "s3d_layernorm_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_float] + [_vp] * 4 + [_i64, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_linear": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp]),
     "s3d_linear_in_order": (ctypes.c_int, [_vp] * 5 + [_i64, _i32, _i32, _vp]),
+    "s3d_mlp": (ctypes.c_int, [_vp] * 6 + [_i64, _i32, _i32, _vp]),
     "s3d_linear_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32]),
     "s3d_linear_grad": (ctypes.c_int, [_vp] * 4 + [_i32, _i64, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "s3d_swin_blocks_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32]),

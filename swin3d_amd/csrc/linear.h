@@ -18,6 +18,17 @@ struct LinearArgs {
 
 int launch_linear(const LinearArgs &a, hipStream_t stream);
 
+// Both layers of an MLP in one kernel (mlp.hip): y = fc2(GELU(fc1(x)))
+struct MlpArgs {
+    const void *x, *w1, *b1, *w2, *b2;   // [M,C], [hidden,C], [hidden] or null, [C,hidden], [C] or null; fp16
+    void *y;                             // [M,C] fp16, apart from x
+    int64_t M;
+    int32_t C, hidden;
+};
+bool mlp_takes(int64_t M, int32_t C, int32_t hidden);
+bool mlp_pays(int64_t M, int32_t C, int32_t hidden);      // ... and is faster than the layers apart
+int launch_mlp(const MlpArgs &a, hipStream_t stream);
+
 // A layer's weight and bias gradients (linear_grad.hip): dw = dy^T x, db = the column sums of dy; the first `scaled` rows of
 // the weight (and numbers of the bias) are parameters times `scale`
 struct LinearGrad {

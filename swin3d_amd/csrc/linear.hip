@@ -13,6 +13,7 @@
 // deepest the tiles are few and a tile's chain of chunks is what counts (linear_thin_kernel): 390 rows, 384 -> 384, 3.4 us against 18
 // through torch, whose launch alone takes the host that long.
 #include "attn_kernels.h"
+#include "dense.h"
 #include "linear.h"
 
 #include <type_traits>
@@ -20,31 +21,9 @@
 namespace s3d {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr int kThreads = 256;
 constexpr int kChunk = 64;        // numbers of K staged at a time
 constexpr int kPieces = kChunk / 8;
-
-// x Phi(x) = (x + |x|) / 2 - |x| Phi(-|x|), with 2 Phi(-u) = 2^p(u): the logarithm of the normal distribution's tail is
-// close to a parabola, and the polynomial of degree 7 with p(0) = 0 that fits it best for |x| Phi(-|x|) over [0, 5.8] (least
-// squares at Chebyshev nodes) is 2.5e-7 off, the rounding of fp32; from 5.8 on the tail is below fp16's smallest number.
-// Fifteen instruction slots where a rational form with an exponential took 22, and small results keep fp16's relative
-// precision.  Infinities and NaN as x Phi(x) has them: the first sum is NaN for -infinity.
-__device__ __forceinline__ float gelu(float x)
-{
-    const float u = fabsf(x), c = fminf(u, 5.8f);
-    float p = fmaf(-7.429386528e-7f, c, 4.341329259e-5f);
-    p = fmaf(p, c, -8.166006301e-4f);
-    p = fmaf(p, c, 8.171264082e-3f);
-    p = fmaf(p, c, -5.347365886e-2f);
-    p = fmaf(p, c, -4.587851465e-1f);
-    p = fmaf(p, c, -1.151172519f);
-    return 0.5f * fmaf(-c, __builtin_amdgcn_exp2f(p * c), x + u);
-}
 
 // The derivative of x Phi(x): Phi(x) + x phi(x), in fp32.  With Phi(-u) = phi(u) M(u), M the ratio of Mills, that is
 // phi(u) (u - M(u)) with the sign of x, and 1 more for x above 0, u = |x|: u - M(u) by the polynomial of degree 12 that fits
@@ -78,13 +57,6 @@ enum class Behind { kNothing, kGelu, kGeluGrad, kGeluBeside };
 
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
-
-// between what a wavefront's lanes write to its LDS and what other lanes of it read (it serves a wavefront in order)
-__device__ __forceinline__ void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // WM x WN wavefronts of TM x TN products of 32 x 32
 template <int WM, int WN, int TM, int TN> struct Tile {

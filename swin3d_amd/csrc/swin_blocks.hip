@@ -2,7 +2,7 @@
 //
 // What bounds them on small scans is the host: through torch a block is some fifteen dispatches (300 us), while its seven
 // kernels take a third of that.  Here the launches follow each other with nothing in between: per block
-//   LayerNorm, qkv, attention, proj, add + LayerNorm, fc1 + GELU, fc2
+//   LayerNorm, qkv, attention, proj, add + LayerNorm, fc1 + GELU, fc2 (the last two as one on many rows)
 // with the residual stream in fp32 and everything else in fp16, as under autocast.
 #include "linear.h"
 
@@ -59,6 +59,10 @@ extern "C" __attribute__((visibility("default"))) int s3d_swin_blocks(
         if (int rc = s3d_add_layernorm(from, pending, S3D_DTYPE_F16, b.norm2_weight, b.norm2_bias, b.norm2_eps, x_out, normed,
                                        S3D_DTYPE_F16, N, C, stream))
             return rc;
+        if (mlp_pays(N, C, hidden)) {
+            if (int rc = launch_mlp({normed, b.fc1_weight, b.fc1_bias, b.fc2_weight, b.fc2_bias, pending, N, C, hidden}, s)) return rc;
+            continue;
+        }
         if (int rc = launch_linear({normed, b.fc1_weight, b.fc1_bias, wide, N, hidden, C, true}, s)) return rc;
         if (int rc = launch_linear({wide, b.fc2_weight, b.fc2_bias, pending, N, C, hidden, false}, s)) return rc;
     }

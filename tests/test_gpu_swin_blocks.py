@@ -70,19 +70,47 @@ def test_linear_of_several_tiles_a_workgroup(hip_lib, m, n, k, gelu):
             assert torch.equal(whole[first:first + 4001], linear_rows(x[first:first + 4001].clone(), w, bias, gelu=gelu))
 
 
+@pytest.mark.parametrize("c", [48, 64, 80, 96, 128, 160, 192])
+@pytest.mark.parametrize("m,hidden", [(1, 32), (127, 64), (129, 96), (16385, None), (40001, None)])      # one stage, two, three, the networks'; edges of 128 rows
+def test_both_layers_of_an_mlp_at_once(hip_lib, c, m, hidden):
+    """The bits of the layers apart."""
+    hidden = hidden or 4 * c
+    gen = torch.Generator(device="cuda").manual_seed(m + c)
+    x, w1, b1, w2, b2 = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, c), (hidden, c), (hidden,), (c, hidden), (c,)))
+    w1, w2 = (w1.float() * c ** -0.5).half(), (w2.float() * hidden ** -0.5).half()
+    x[m // 2, 0], x[m // 3, 1] = float("inf"), float("nan")
+    for bias1, bias2 in ((b1, b2), (None, None)):
+        y = torch.empty(m + 1, c, device="cuda", dtype=torch.float16)
+        y[m] = 7
+        status = _lib.lib().s3d_mlp(x.data_ptr(), w1.data_ptr(), None if bias1 is None else bias1.data_ptr(), w2.data_ptr(),
+                                    None if bias2 is None else bias2.data_ptr(), y.data_ptr(), m, c, hidden, _lib.stream(x.device))
+        _lib.check(status, "s3d_mlp")
+        # (among so many rows that no wavefronts share the sums over K)
+        inner = linear_rows(torch.cat([x, x.new_zeros(40000, c)]), w1, bias1, gelu=True)[:m].contiguous()
+        want = linear_rows(inner, w2, bias2, in_order=True)
+        assert torch.equal(y[:m].isnan(), want.isnan()) and torch.equal(y[:m].nan_to_num(7), want.nan_to_num(7)) and bool((y[m] == 7).all())
+
+
+def test_mlp_refuses_what_it_cannot_do(hip_lib):
+    x = torch.zeros(64, 1024, device="cuda").half()
+    for c, hidden in ((40, 32), (320, 64), (48, 48), (48, 1056)):
+        assert _lib.lib().s3d_mlp(x.data_ptr(), x.data_ptr(), None, x.data_ptr(), None, x.data_ptr(), 1, c, hidden, None) < 0
+
+
 def test_linear_refuses_what_it_cannot_do(hip_lib):
     x, w = torch.randn(5, 24, device="cuda").half(), torch.randn(8, 24, device="cuda").half()
     assert linear_rows(x, w, None) is None and linear_rows(x.float(), w.float(), None) is None
     assert _lib.lib().s3d_linear(x.data_ptr(), w.data_ptr(), None, x.data_ptr(), 5, 8, 24, 0, None) < 0
 
 
-@pytest.mark.parametrize("heads,dim,window,mode", [(6, 8, 5, 2), (5, 16, 7, 1)])
-def test_blocks_in_one_call_equal_single_blocks(hip_lib, heads, dim, window, mode):
+@pytest.mark.parametrize("heads,dim,window,mode,voxels", [(6, 8, 5, 2, 5000), (5, 16, 7, 1, 5000), (6, 8, 5, 1, 21000)])      # (both layers of the MLP at once)
+def test_blocks_in_one_call_equal_single_blocks(hip_lib, heads, dim, window, mode, voxels):
     """Same launches but for the GELU (fused with fc1, which then is not rounded in between) and the products' order of
     summation; hooks and changed parameters are noticed."""
     dev = torch.device("cuda")
-    scene = synth.make_room((3.0, 3.0, 2.0), 4, 5000, seed=5)
+    scene = synth.make_room((3.0, 3.0, 2.0) if voxels < 10000 else (6.0, 5.0, 2.5), 4, voxels, seed=5)
     coords = torch.from_numpy(scene.coords).to(dev)
+    assert (coords.shape[0] >= 16384) == (voxels > 10000)
     signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)
     torch.manual_seed(1)
     stage = encoder.Stage(heads * dim, 3, heads, window, 4, downsample=False, cRSE="XYZ_RGB_NORM", fp16_mode=mode).to(dev).eval()
