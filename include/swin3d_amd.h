@@ -485,6 +485,9 @@ int s3d_knn_distances(int32_t K, const float *src_xyz, int64_t Ns, const float *
  */
 int s3d_knn_max_pool(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C,
                      int32_t dtype, void *out, void *stream);
+/* The same of fp16 rows, the maxima in fp32. */
+int s3d_knn_max_pool_widened(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C, float *out,
+                             void *stream);
 
 /*
  * The gradient of that call for src_feat: every query's dout goes in equal shares to the rows of its list that hold the

@@ -853,11 +853,12 @@ int launch_interpolate(const int32_t *idx, const float *dist2, int K, int64_t Nq
 // Swin3D/modules/swin3d_layers.py:292-312: gather [Nq,K,C], then max over K) without the gathered intermediate.
 // One thread per (query, 16 bytes of channels).  A padded slot (row -1) reads row 0, as the clamped gather of
 // the tensor statement does.  Bound by the gathered rows: with eight of them under way per thread and an XCD's queries next
-// to each other 12.8 us at 199,327 x 96 fp16, K = 16, without 29.3.
-template <typename T, int VEC>
+// to each other 12.8 us at 199,327 x 96 fp16, K = 16, without 29.3.  The next level's rows are fp32: fp16 ones leave widened,
+// 14.9 us where they and a cast took 21.8.
+template <typename T, int VEC, typename Out>
 __global__ __launch_bounds__(kThreads) void knn_max_pool_kernel(const int32_t *__restrict__ idx, int K, int64_t Nq,
                                                                 const T *__restrict__ feat, int C,
-                                                                T *__restrict__ out)
+                                                                Out *__restrict__ out)
 {
     const int groups = C / VEC;
     const int64_t t = share_of_xcd(Nq * groups);
@@ -883,24 +884,30 @@ __global__ __launch_bounds__(kThreads) void knn_max_pool_kernel(const int32_t *_
 #pragma unroll
             for (int e = 0; e < VEC; ++e) best[e] = (i0 + i == 0 || v[i][e] > best[e] || v[i][e] != v[i][e]) ? v[i][e] : best[e];
     }
-    if constexpr (VEC * sizeof(T) == 16)
-        *reinterpret_cast<uint4 *>(out + qi * C + c0) = *reinterpret_cast<const uint4 *>(best);
-    else
-        out[qi * C + c0] = best[0];
+    if constexpr (VEC * sizeof(T) == 16) {
+        constexpr int kPiece = 16 / sizeof(Out);
+        Out o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o[e] = static_cast<Out>(best[e]);
+#pragma unroll
+        for (int e = 0; e < VEC; e += kPiece) *reinterpret_cast<uint4 *>(out + qi * C + c0 + e) = *reinterpret_cast<const uint4 *>(o + e);
+    } else {
+        out[qi * C + c0] = static_cast<Out>(best[0]);
+    }
 }
 
-template <typename T>
+template <typename T, typename Out>
 int launch_max_pool(const int32_t *idx, int K, int64_t Nq, const void *feat, int C, void *out, hipStream_t s)
 {
     const T *f = static_cast<const T *>(feat);
-    T *o = static_cast<T *>(out);
+    Out *o = static_cast<Out *>(out);
     constexpr int kVec = 16 / static_cast<int>(sizeof(T));
     if (C % kVec == 0 && reinterpret_cast<uintptr_t>(feat) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
         const int64_t threads = Nq * (C / kVec);
-        hipLaunchKernelGGL((knn_max_pool_kernel<T, kVec>), xcd_grid(threads), dim3(kThreads), 0, s, idx, K, Nq, f, C, o);
+        hipLaunchKernelGGL((knn_max_pool_kernel<T, kVec, Out>), xcd_grid(threads), dim3(kThreads), 0, s, idx, K, Nq, f, C, o);
     } else {
         const int64_t threads = Nq * C;
-        hipLaunchKernelGGL((knn_max_pool_kernel<T, 1>), xcd_grid(threads), dim3(kThreads), 0, s, idx, K, Nq, f, C, o);
+        hipLaunchKernelGGL((knn_max_pool_kernel<T, 1, Out>), xcd_grid(threads), dim3(kThreads), 0, s, idx, K, Nq, f, C, o);
     }
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -909,11 +916,11 @@ int launch_max_pool(const int32_t *idx, int K, int64_t Nq, const void *feat, int
 }  // namespace
 }  // namespace s3d
 
-extern "C" __attribute__((visibility("default"))) int s3d_knn_max_pool(const int32_t *idx, int32_t K, int64_t Nq,
-                                                                        const void *src_feat, int64_t Ns, int32_t C,
-                                                                        int32_t dtype, void *out, void *stream)
+namespace s3d {
+namespace {
+
+int max_pool(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat, int64_t Ns, int32_t C, int32_t dtype, bool widened, void *out, void *stream)
 {
-    using namespace s3d;
     if (K < 1 || K > S3D_KNN_KMAX) return fail(S3D_ERR_BAD_SHAPE, "s3d_knn_max_pool: K=%d outside 1..%d", K, S3D_KNN_KMAX);
     if (Nq < 0 || Ns < 0 || C < 1 || Nq * static_cast<int64_t>(C) > 0x3fffffffffLL || (Nq > 0 && Ns < 1))
         return fail(S3D_ERR_BAD_SHAPE, "s3d_knn_max_pool: Nq=%lld Ns=%lld C=%d out of range", (long long)Nq, (long long)Ns,
@@ -923,8 +930,25 @@ extern "C" __attribute__((visibility("default"))) int s3d_knn_max_pool(const int
     if (Nq == 0) return S3D_OK;
     if (!idx || !out || !src_feat) return fail(S3D_ERR_NULL_POINTER, "s3d_knn_max_pool: null device pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    return dtype == S3D_DTYPE_F16 ? launch_max_pool<_Float16>(idx, K, Nq, src_feat, C, out, s)
-                                  : launch_max_pool<float>(idx, K, Nq, src_feat, C, out, s);
+    return dtype == S3D_DTYPE_F32 ? launch_max_pool<float, float>(idx, K, Nq, src_feat, C, out, s)
+           : widened              ? launch_max_pool<_Float16, float>(idx, K, Nq, src_feat, C, out, s)
+                                  : launch_max_pool<_Float16, _Float16>(idx, K, Nq, src_feat, C, out, s);
+}
+
+}  // namespace
+}  // namespace s3d
+
+extern "C" __attribute__((visibility("default"))) int s3d_knn_max_pool(const int32_t *idx, int32_t K, int64_t Nq,
+                                                                        const void *src_feat, int64_t Ns, int32_t C,
+                                                                        int32_t dtype, void *out, void *stream)
+{
+    return s3d::max_pool(idx, K, Nq, src_feat, Ns, C, dtype, false, out, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int s3d_knn_max_pool_widened(const int32_t *idx, int32_t K, int64_t Nq, const void *src_feat,
+                                                                                int64_t Ns, int32_t C, float *out, void *stream)
+{
+    return s3d::max_pool(idx, K, Nq, src_feat, Ns, C, S3D_DTYPE_F16, true, out, stream);
 }
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_knn_workspace_bytes(int64_t Ns, int64_t Nq, int32_t B)

@@ -1,8 +1,8 @@
 """Swin3D encoder on the swin3d_amd operators, without MinkowskiEngine (inference path).
 
 The sparse voxel set is a pair of tensors (`SparseVoxels`).  Under fp16 autocast the dense layers of inference run on
-the library's kernels, those of a training pass forward through torch (hipBLASLt) and backward on the library's; the
-27-offset stem convolution is one GEMM of torch's.  Window attention runs through
+the library's kernels; those of a training pass too, but for products to which torch gives bits of their own.  The 27-offset
+stem convolution is one GEMM of torch's.  Window attention runs through
 `SelfAttnAIOFunction`, the window index through `window_sets` / `window_signals`, neighbour
 gathering through `KNN` / `knn_max_pool`.  On the GPU the coordinate work runs on the library's kernels too
 (coarse cells and their representatives from the window sort, the stem's neighbour rows from a table of the
@@ -34,10 +34,11 @@ import torch.nn.functional as F
 
 from . import _lib
 from .crse import crse_num_axes, crse_table_sizes, scale_crse_coords
-from .fused_norm import add_layernorm, trained_add_norm
+from .fused_norm import add_half, add_layernorm, trained_add_norm
 from .linear_grad import trained_linear
 from .sparse_dl.attn.attn_coff import IndexMode, PosEmb, PrecisionMode, SelfAttnAIOFunction, TableDims
-from .sparse_dl.knn import KNN, KNNInterpolate, KNNInterpolateAdd, KNNMaxPool, interpolate_add_applies, knn_max_pool, knn_query
+from .sparse_dl.knn import KNN, KNNInterpolate, KNNInterpolateAdd, KNNMaxPool, interpolate_add_applies, knn_query
+from .sparse_dl.knn.knn import _max_pool
 from .swin_blocks import data_only, linear_rows, plain, swin_blocks
 from .swin_train import trained_branches
 from .window_index import get_index01, index_arguments, window_signals, window_sets
@@ -425,9 +426,10 @@ def _fused_norm_applies(feats):
 
 
 def _plus(feats, branch):
-    """feats + branch for an fp32 stream and a branch in fp16: widened by itself first, which is exact; torch's sum of two
-    types takes 53 us for 49,682 x 96, at a tenth of what either kernel reaches."""
-    return feats + branch.to(feats.dtype)
+    """feats + branch for an fp32 stream and a branch in fp16, widened first, which is exact, in one kernel where it takes them;
+    torch's sum of two types takes 53 us for 49,682 x 96, at a tenth of what either kernel of two reaches."""
+    done = add_half(feats, branch)
+    return feats + branch.to(feats.dtype) if done is None else done
 
 
 def _norm(norm, x):
@@ -484,7 +486,7 @@ class GridKNNDownsample(nn.Module):
             normed = _norm(self.norm, voxels.feats)
         projected = _linear(self.linear, normed)
         if not torch.is_grad_enabled() and projected.is_cuda and projected.dtype in (torch.float16, torch.float32):
-            feats = knn_max_pool(idx, projected)      # one kernel, no [Nq, K, C] intermediate
+            feats = _max_pool(idx, projected, torch.float32)      # one kernel, no [Nq, K, C] intermediate
         elif (projected.is_cuda and projected.dtype in (torch.float16, torch.float32) and data_only(projected)
               and idx.is_cuda and idx.dtype == torch.int32 and idx.numel() > 0 and projected.shape[0] > 0):
             feats = KNNMaxPool.apply(idx, projected)

@@ -59,6 +59,34 @@ def train_add_layernorm(x, residual, weight, bias, eps):
     return summed, y
 
 
+def add_half(x, residual):
+    """x + residual for fp32 rows and a branch in fp16, with their gradients where they are followed; None where the kernel does
+    not take them."""
+    if followed() or not (x.is_cuda and type(x) is type(residual) is torch.Tensor and x.dtype == torch.float32 and residual.dtype == torch.float16
+                          and x.device == residual.device and x.shape == residual.shape and x.is_contiguous() and residual.is_contiguous()
+                          and x.numel() % 4 == 0 and (x.data_ptr() | residual.data_ptr()) % 16 == 0):
+        return None
+    return _AddHalf.apply(x, residual) if torch.is_grad_enabled() and (x.requires_grad or residual.requires_grad) else _added_half(x, residual)
+
+
+def _added_half(x, residual):
+    out = torch.empty_like(x)
+    with _lib.on(x.device):
+        status = _lib.lib().s3d_add_half(x.data_ptr(), residual.data_ptr(), out.data_ptr(), x.numel(), _lib.stream(x.device))
+    _lib.check(status, "s3d_add_half")
+    return out
+
+
+class _AddHalf(Function):
+    @staticmethod
+    def forward(ctx, x, residual):
+        return _added_half(x, residual)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return grad, grad.to(torch.float16) if ctx.needs_input_grad[1] else None
+
+
 class _AddNorm(Function):
     """(x + residual, LayerNorm of it in fp16); x itself in the first place without a residual."""
 

@@ -101,6 +101,11 @@ def knn_max_pool(idx, src_feat):
     knn_query result) -> [Nq,C] in the dtype of src_feat: the gather + max of the KNN downsample
     (Swin3D/modules/swin3d_layers.py:292-312) without the [Nq,K,C] intermediate.  Padded slots (row -1) read
     row 0, as the clamped gather does.  No autograd: KNNMaxPool has it."""
+    return _max_pool(idx, src_feat, src_feat.dtype)
+
+
+def _max_pool(idx, src_feat, dtype):
+    """knn_max_pool in `dtype`: that of src_feat, or float32."""
     if not (idx.is_cuda and src_feat.is_cuda):
         raise RuntimeError("idx and src_feat must be CUDA (HIP) tensors")
     if idx.dtype != torch.int32 or idx.dim() != 2:
@@ -110,11 +115,14 @@ def knn_max_pool(idx, src_feat):
     idx, src_feat = idx.contiguous(), src_feat.contiguous()
     nq, k = idx.shape
     ns, c = src_feat.shape
-    out = torch.empty((nq, c), dtype=src_feat.dtype, device=src_feat.device)
+    out = torch.empty((nq, c), dtype=dtype, device=src_feat.device)
     with _lib.on(src_feat.device):
         stream = _lib.stream(src_feat.device)
-        status = _lib.lib().s3d_knn_max_pool(idx.data_ptr(), k, nq, src_feat.data_ptr(), ns, c,
-                                             _FEAT_DTYPE[src_feat.dtype], out.data_ptr(), stream)
+        if dtype == src_feat.dtype:
+            status = _lib.lib().s3d_knn_max_pool(idx.data_ptr(), k, nq, src_feat.data_ptr(), ns, c,
+                                                 _FEAT_DTYPE[src_feat.dtype], out.data_ptr(), stream)
+        else:
+            status = _lib.lib().s3d_knn_max_pool_widened(idx.data_ptr(), k, nq, src_feat.data_ptr(), ns, c, out.data_ptr(), stream)
     _lib.check(status, "s3d_knn_max_pool")
     return out
 

@@ -123,3 +123,19 @@ def test_stage_with_downsample_fused_path_matches_torch_path(hip_lib):
     for fused, plain in ((fine_f.feats, fine_p.feats.detach()), (down_f.feats, down_p.feats.detach())):
         assert fused.dtype == torch.float32 and fused.shape == plain.shape
         assert (fused - plain).abs().max().item() <= 2e-2 * plain.abs().max().item()
+
+
+@pytest.mark.parametrize("rows,channels", [(1, 4), (301, 48), (70001, 20)])
+def test_sum_with_a_branch_in_fp16(hip_lib, rows, channels):
+    from swin3d_amd.fused_norm import add_half
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x, branch, grad = (torch.randn(rows, channels, device="cuda", generator=gen) for _ in range(3))
+    branch = branch.half()
+    assert torch.equal(add_half(x, branch), x + branch.float())
+    x.requires_grad_(), branch.requires_grad_()
+    got = torch.autograd.grad(add_half(x, branch), (x, branch), grad)
+    want = torch.autograd.grad(x + branch.to(x.dtype), (x, branch), grad)
+    assert all(torch.equal(g, w) and g.dtype == w.dtype for g, w in zip(got, want))
+    assert add_half(x, branch.float()) is None
+    if rows > 1:
+        assert add_half(x.t(), branch.t()) is None and add_half(x[:, :3], branch[:, :3]) is None

@@ -174,3 +174,6 @@ def test_max_pool_over_neighbours_matches_gather_and_max(hip_lib, dtype, channel
     feat = torch.from_numpy(rng.standard_normal((3000, channels)).astype(np.float32)).cuda().to(dtype)
     ref = feat[idx.view(-1).long().clamp(min=0)].view(700, 16, channels).amax(dim=1)
     assert torch.equal(knn_max_pool(idx, feat), ref)
+    if feat.dtype == torch.float16:
+        from swin3d_amd.sparse_dl.knn.knn import _max_pool
+        assert torch.equal(_max_pool(idx, feat, torch.float32), ref.float())
