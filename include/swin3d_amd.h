@@ -584,6 +584,19 @@ int s3d_linear_grad(const void *dy, const void *x, void *dw, void *db, int32_t g
                     void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The stem at inference (Swin3D/modules/mink_layers.py:50-80): the 3x3x3 convolution over a voxel's neighbours, rounded to fp16,
+ * BatchNorm with its running statistics and ReLU in fp32.
+ *   feats        device [N,cin] of `dtype` (fp32 is rounded to fp16), cin at most 16
+ *   neighbours   device int64 [N,27]: rows of feats, N where there is none (zeros)
+ *   weight       device fp32 [27,cin,cout] (rounded to fp16), cout a multiple of 16 up to 96
+ *   mean, var    device fp32 [cout];  gamma, beta likewise, or null;  out device fp32 [N,cout], 16-byte aligned
+ */
+size_t s3d_stem_workspace_bytes(int64_t N, int32_t cout);
+int s3d_stem(const void *feats, int32_t dtype, int64_t N, int32_t cin, const int64_t *neighbours, const float *weight, int32_t cout,
+             const float *mean, const float *var, const float *gamma, const float *beta, float eps, float *out, void *workspace,
+             size_t workspace_bytes, void *stream);
+
+/*
  * The Swin blocks of a stage at inference (Swin3D/modules/swin3d_layers.py:563-625): per block
  *   x = x + proj(attention(qkv(LayerNorm(x))));  x = x + fc2(GELU(fc1(LayerNorm(x))))
  * with the residual stream in fp32 and the branches in fp16, in one host call.  Block i works on window set i % num_sets.

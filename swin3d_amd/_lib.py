@@ -99,6 +99,8 @@ SIGNATURES = {
     "s3d_add_half": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp]),
     "s3d_swin_block_grad_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i64, _i64, _i64]),
     # saved grads dsum dpending | N H D hidden | sizes nd len | W pairs scale dtype | ws bytes stream
+    "s3d_stem_workspace_bytes": (ctypes.c_size_t, [_i64, _i32]),
+    "s3d_stem": (ctypes.c_int, [_vp, _i32, _i64, _i32, _vp, _vp, _i32] + [_vp] * 4 + [ctypes.c_float, _vp, _vp, ctypes.c_size_t, _vp]),
     "s3d_swin_block_train": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _i32, _i64, _vp]),
     "s3d_swin_block_grad": (ctypes.c_int, [_vp] * 4 + [_i64, _i32, _i32, _i32, _vp, _i32, _i64, _i64, _i64, ctypes.c_float, _i32, _vp,
                                            ctypes.c_size_t, _vp]),

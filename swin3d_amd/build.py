@@ -13,7 +13,7 @@ LIB = os.path.join(HERE, "libswin3d_amd.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["api_common.hip", "attn_fwd.hip", "attn_sweep.hip", "attn_tile.hip", "attn_strip_fwd.hip", "attn_tile_bwd.hip", "attn_strip_records.hip", "attn_strip_bwd.hip", "attn_bwd.hip",
-           "window_index.hip", "knn.hip", "geometry.hip", "knn_pool_grad.hip", "layernorm.hip", "cast.hip", "linear.hip", "mlp.hip", "linear_grad.hip", "swin_blocks.hip",
+           "window_index.hip", "knn.hip", "geometry.hip", "knn_pool_grad.hip", "layernorm.hip", "cast.hip", "linear.hip", "mlp.hip", "stem.hip", "linear_grad.hip", "swin_blocks.hip",
            "swin_blocks_grad.hip"]
 
 # packed-fp32 VALU forms are disabled for every device compilation unit

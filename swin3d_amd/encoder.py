@@ -1,8 +1,8 @@
 """Swin3D encoder on the swin3d_amd operators, without MinkowskiEngine (inference path).
 
 The sparse voxel set is a pair of tensors (`SparseVoxels`).  Under fp16 autocast the dense layers of inference run on
-the library's kernels; those of a training pass too, but for products to which torch gives bits of their own.  The 27-offset
-stem convolution is one GEMM of torch's.  Window attention runs through
+the library's kernels, the stem among them; those of a training pass too, but for products to which torch gives bits of
+their own, the 27-offset stem convolution among these.  Window attention runs through
 `SelfAttnAIOFunction`, the window index through `window_sets` / `window_signals`, neighbour
 gathering through `KNN` / `knn_max_pool`.  On the GPU the coordinate work runs on the library's kernels too
 (coarse cells and their representatives from the window sort, the stem's neighbour rows from a table of the
@@ -349,8 +349,43 @@ class StemConv(nn.Module):
         return self.conv_layers[0].kernel
 
     def forward(self, voxels, neighbours=None):
+        done = self._at_once(voxels, neighbours)
+        if done is not None:
+            return voxels.with_feats(done)
         out = sparse_conv3x3x3(voxels, self.weight, neighbours)
         return voxels.with_feats(F.relu(self.conv_layers[1](out.float())))
+
+    def _at_once(self, voxels, neighbours):
+        """Inference under fp16 autocast in one call of the library (s3d_stem); None where that does not stand for the layers."""
+        feats, conv, norm = voxels.feats, *self.conv_layers
+        if torch.is_grad_enabled() or not (feats.is_cuda and torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.float16) \
+                or not (data_only(feats) and plain(self.conv_layers, nn.Sequential) and type(conv) is _ConvKernel and plain(norm, _BatchNorm)):
+            return None
+        bn, weight = norm.bn, conv.kernel
+        if not plain(bn, nn.BatchNorm1d) or bn.training or bn.running_mean is None or bn.running_var is None \
+                or feats.dtype not in (torch.float16, torch.float32) or feats.dim() != 2 or not feats.is_contiguous():
+            return None
+        (n, cin), dev = feats.shape, feats.device
+        cout = weight.shape[-1]
+        neighbours = conv3x3x3_neighbours(voxels.coords, voxels.stride) if neighbours is None else neighbours
+        if not (0 < n < 2 ** 31 - 16 and 0 < cin <= 16 and cout % 16 == 0 and 0 < cout <= 96 and weight.shape == (27, cin, cout)
+                and data_only(neighbours) and neighbours.device == dev and neighbours.dtype == torch.long
+                and neighbours.shape == (n, 27) and neighbours.is_contiguous()):
+            return None
+        params = (weight, bn.running_mean, bn.running_var, bn.weight, bn.bias)
+        if any(p is not None and not (type(p) in (torch.Tensor, nn.Parameter) and p.dtype == torch.float32 and p.device == dev and p.is_contiguous())
+               for p in params) or any(p is not None and p.shape != (cout,) for p in params[1:]):
+            return None
+        out = torch.empty((n, cout), dtype=torch.float32, device=dev)
+        with _lib.on(dev):
+            lib = _lib.lib()
+            ws_bytes = lib.s3d_stem_workspace_bytes(n, cout)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            weight_at, *norm_at = (None if p is None else p.data_ptr() for p in params)
+            status = lib.s3d_stem(feats.data_ptr(), int(feats.dtype == torch.float16), n, cin, neighbours.data_ptr(), weight_at, cout, *norm_at,
+                                  bn.eps, out.data_ptr(), workspace.data_ptr(), ws_bytes, _lib.stream(dev))
+        _lib.check(status, "s3d_stem")
+        return out
 
 
 # Inference-time copies of parameters (autocast-dtype weights, scaled projections, flat tables) are kept on their

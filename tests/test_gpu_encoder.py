@@ -294,3 +294,42 @@ def test_inference_copies_of_parameters_follow_training_updates(hip_lib):
     encoder.drop_inference_copies(layer)
     third = infer()
     assert torch.equal(third, torch.nn.functional.linear(x.half(), layer.weight.half(), layer.bias.half()).float())
+
+
+@pytest.mark.parametrize("n,cin,cout,dtype", [(1, 1, 16, torch.float32), (31, 6, 48, torch.float16), (33, 9, 80, torch.float32),
+                                              (5001, 16, 96, torch.float32), (70001, 9, 48, torch.float32), (150001, 9, 32, torch.float16)])
+@pytest.mark.parametrize("affine", [True, False])
+def test_stem_at_once(hip_lib, n, cin, cout, dtype, affine):
+    """Few voxels, several tiles a wavefront, one to three tiles of channels, rows that are no voxels': against the layers in fp32 of
+    the same fp16 numbers, the convolution rounded to fp16 (half a place; one where fp32 sums differ) before the norm."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    stem = encoder.StemConv(cin, cout).cuda().eval()
+    bn = stem.conv_layers[1].bn
+    bn.running_mean.normal_(generator=gen)
+    bn.running_var.uniform_(0.5, 2.0, generator=gen)
+    if affine:
+        torch.nn.init.normal_(bn.weight, 1.0, 0.3)
+        torch.nn.init.normal_(bn.bias)
+    else:
+        bn.weight = bn.bias = None
+    feats = torch.randn(n, cin, device="cuda", generator=gen).to(dtype)
+    neighbours = torch.randint(0, n + 1, (n, 27), device="cuda", generator=gen)
+    neighbours[n // 2, 3], neighbours[n // 2, 5] = -1, -2
+    calls = []
+    voxels = encoder.SparseVoxels(torch.zeros(n, 4, dtype=torch.int32, device="cuda"), feats, 1)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        got = stem(voxels, neighbours).feats
+        handle = bn.register_forward_hook(lambda *_: calls.append(1))
+        apart = stem(voxels, neighbours).feats
+        handle.remove()
+    assert calls == [1] and got.dtype == torch.float32 and got.shape == (n, cout)
+    padded = torch.cat([feats.half(), feats.new_zeros(1, cin).half()]).float()
+    conv = padded[neighbours.reshape(-1)].view(n, 27 * cin) @ stem.weight.half().float().reshape(27 * cin, cout)
+    scale = (bn.running_var + bn.eps).rsqrt() * (1.0 if bn.weight is None else bn.weight)
+    want = torch.relu((conv - bn.running_mean) * scale + (0.0 if bn.bias is None else bn.bias))
+    room = scale.abs() * (2.0 ** -10 * conv.abs() + 2.0 ** -20 * (27 * cin) ** 0.5) + 1e-5
+    assert ((got - want).abs() <= room).all() and ((apart - want).abs() <= room).all()
+    bad = neighbours.clone()
+    bad[n // 3, 1] = n + 5
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        assert stem(voxels, bad).feats[n // 3].isnan().all()
