@@ -99,6 +99,15 @@ constexpr int kBigBins = 31, kListBins = kBigBins + kCols;   // windows of 2 .. 
 __device__ __forceinline__ int tiles_of(int n) { return (n + kCols - 1) / kCols; }
 __device__ __forceinline__ int list_bin(int n) { return n > kCols ? 32 - min(tiles_of(n), 32) : kBigBins + kCols - n; }
 
+// Barrier of the workgroup for what it shares in LDS.  __syncthreads() also waits for every load from memory that is under
+// way, among them what a stage has asked for ahead of its use, and for every store.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Unit list: windows in bins of equal size, largest first (a counting sort in LDS), and the pairs of the windows before
 // each.  Inside a bin the windows keep their order: where a window lies in its unit decides in which order the matrix pipe
 // adds its products, and a result is to be the same bits on every call.
@@ -110,18 +119,27 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
     constexpr int kWavesOfList = kListThreads / 64;
     __shared__ long long wave_pairs[kWavesOfList];
     __shared__ int of_wave[kWavesOfList][kListBins];
+    __shared__ unsigned long long same_of_wave[kWavesOfList][kListBins];
     __shared__ int big_strips[kListBins], strip_at[kListBins], strips_of_wave[kWavesOfList][kBigBins];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (t < kListBins) windows[t] = big_units[t] = big_strips[t] = 0;
     __syncthreads();
-    for (int w = t; w < W; w += kListThreads) {
-        const int n = w_sizes[w];
-        if (n <= 0) continue;
-        const int b = list_bin(n);
-        atomicAdd(&windows[b], 1);
-        if (n > kCols) {
-            atomicAdd(&big_units[b], tiles_of(n));
-            atomicAdd(&big_strips[b], strips_of(n));
+    // (loads ahead of their use, here and below: the rounds are a chain of trips to memory otherwise)
+    constexpr int kAhead = 8;
+    for (int w0 = t; w0 < W; w0 += kAhead * kListThreads) {
+        int size[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) size[k] = w_sizes[min(w0 + k * kListThreads, W - 1)];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const int n = w0 + k * kListThreads < W ? size[k] : 0;
+            if (n <= 0) continue;
+            const int b = list_bin(n);
+            atomicAdd(&windows[b], 1);
+            if (n > kCols) {
+                atomicAdd(&big_units[b], tiles_of(n));
+                atomicAdd(&big_strips[b], strips_of(n));
+            }
         }
     }
     __syncthreads();
@@ -155,9 +173,12 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
     }
     __syncthreads();
     long long before = 0;              // pairs of the windows that earlier rounds placed
+    int next_n = t < W ? w_sizes[t] : 0, next_pos = t < W ? w2n[t] : 0;
     for (int w0 = 0; w0 < W; w0 += kListThreads) {
-        const int w = w0 + t;
-        const int n = w < W ? w_sizes[w] : 0;
+        const int n = next_n, pos = next_pos;
+        const int ahead = w0 + kListThreads + t;
+        next_n = ahead < W ? w_sizes[ahead] : 0;
+        next_pos = ahead < W ? w2n[ahead] : 0;
         long long incl = n > 0 ? static_cast<long long>(n) * n : 0;
         const long long own = incl;
         for (int off = 1; off < 64; off <<= 1) {
@@ -165,27 +186,32 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
             if (lane >= off) incl += up;
         }
         if (lane == 63) wave_pairs[wave] = incl;
-        for (int i = t; i < kWavesOfList * kListBins; i += kListThreads) of_wave[0][i] = 0;
+        for (int i = t; i < kWavesOfList * kListBins; i += kListThreads) {
+            of_wave[0][i] = 0;
+            same_of_wave[0][i] = 0;
+        }
         if (t < kWavesOfList * kBigBins) strips_of_wave[0][t] = 0;
-        __syncthreads();
-        // a window's place among those of its bin: in its wavefront, then behind the wavefronts before
+        lds_barrier();
+        // A window's place among those of its bin: in its wavefront, by the lanes with windows of the bin, then behind the
+        // wavefronts before.  (A bit for each lane, set in LDS: a vote for every size that a wavefront has took 38 us for 7,600
+        // windows of some thirty sizes, so 30, and 9.5 for 220 windows, so 8.)
         const int b = n > 0 ? list_bin(n) : -1;
         // (of a bin of larger windows, also the strips of the windows before: all but up to three fewer than four a tile)
         const int fewer = n > kCols ? 4 * tiles_of(n) - strips_of(n) : 0;
+        const unsigned long long one = __ballot((fewer & 1) != 0), two = __ballot((fewer & 2) != 0);
+        if (b >= 0) atomicOr(&same_of_wave[wave][b], 1ull << lane);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         int rank = 0, strips_before = 0;
-        for (unsigned long long left = __ballot(b >= 0); left;) {
-            const int bin = __builtin_amdgcn_readlane(b, __ffsll(static_cast<long long>(left)) - 1);
-            const unsigned long long same = __ballot(b == bin);
-            const unsigned long long below = same & ((1ull << lane) - 1);
-            if (b == bin) rank = __popcll(below);
-            if (lane == 0) of_wave[wave][bin] = __popcll(same);
-            if (bin < kBigBins) {
-                const unsigned long long one = __ballot((fewer & 1) != 0), two = __ballot((fewer & 2) != 0);
-                const int most = 4 * (32 - bin);       // (not in bin 0, whose windows differ in their tiles)
-                if (b == bin) strips_before = most * rank - __popcll(below & one) - 2 * __popcll(below & two);
-                if (lane == 0) strips_of_wave[wave][bin] = most * __popcll(same) - __popcll(same & one) - 2 * __popcll(same & two);
+        if (b >= 0) {
+            const unsigned long long same = same_of_wave[wave][b], below = same & ((1ull << lane) - 1);
+            rank = __popcll(below);
+            const int most = 4 * (32 - b);             // (not in bin 0, whose windows differ in their tiles)
+            if (b < kBigBins) strips_before = most * rank - __popcll(below & one) - 2 * __popcll(below & two);
+            if (rank == 0) {
+                of_wave[wave][b] = __popcll(same);
+                if (b < kBigBins) strips_of_wave[wave][b] = most * __popcll(same) - __popcll(same & one) - 2 * __popcll(same & two);
             }
-            left &= ~same;
         }
         long long pairs = before + incl - own, all = 0;
 #pragma unroll
@@ -194,7 +220,7 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
             all += wave_pairs[v];
         }
         before += all;
-        __syncthreads();
+        lds_barrier();
         if (t < kListBins) {
             int count[kWavesOfList], run = entry_at[t];
 #pragma unroll
@@ -216,11 +242,11 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
             }
             if (bin > 0) strip_at[bin] = run;
         }
-        __syncthreads();
+        lds_barrier();
         if (b >= 0) {
             const int e = of_wave[wave][b] + rank, in_bin = e - entry_first[b];
             // (a window that begins beyond 2^31 pairs does not fit any store of this form)
-            entries[e] = make_int2(w2n[w], static_cast<int>(pairs < 0x7fffffffll ? pairs : 0x7fffffffll));
+            entries[e] = make_int2(pos, static_cast<int>(pairs < 0x7fffffffll ? pairs : 0x7fffffffll));
             if (n > kCols) {
                 const int tiles = tiles_of(n);
                 // (the windows of the first bin differ in their tiles)
@@ -242,7 +268,7 @@ __device__ __forceinline__ void build_list(const int32_t *__restrict__ w_sizes, 
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
     }
 }
 
@@ -308,14 +334,6 @@ __device__ __forceinline__ int float_order(float f)
     return i >= 0 ? i : i ^ 0x7fffffff;
 }
 __device__ __forceinline__ float order_float(int i) { return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff); }
-// Barrier of the workgroup for what it shares in LDS.  __syncthreads() also waits for every load from memory that is under
-// way, among them what a stage has asked for ahead of its use.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 // a value that the compiler cannot follow
 __device__ __forceinline__ int opaque(int x)
 {
