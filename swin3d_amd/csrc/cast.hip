@@ -54,9 +54,9 @@ struct HalfCopies {
 __global__ __launch_bounds__(kCastThreads) void half_copies_kernel(HalfCopies a)
 {
     __shared__ _Float16 turned[kSquare * (kSquare + 4)];
-    int at = 0;
-    for (int i = 1; i < a.num; ++i) at = static_cast<int>(blockIdx.x) >= a.first[i] ? i : at;
-    at = __builtin_amdgcn_readfirstlane(at);
+    // (a lane looks at an array's first workgroup: one by one they were a chain of sixteen loads)
+    const int lane = threadIdx.x & 63;
+    const int at = __popcll(__ballot(lane < a.num && static_cast<int>(blockIdx.x) >= a.first[min(lane, kMostCopies - 1)])) - 1;
     const s3d_half_copy &c = a.of[at];
     const float *from = a.from[at];
     const float scale = c.scale;

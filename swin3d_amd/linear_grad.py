@@ -7,6 +7,9 @@ order is no less exact, but it gives another sample of what fp16 activations do 
 to 40,000 voxels the gradients of Swin3D-S's encoder lie 1 to 5 % from those of an fp32 pass, and products that share K among
 wavefronts in the forward moved them by 0.1 to 1.6 % (single elements by up to a seventh of the largest).  With torch's bits they
 are what they were to the scatter of two runs, 0.05 to 0.1 %."""
+import ctypes
+import functools
+
 import torch
 import torch.nn.functional as F
 from torch.autograd.function import Function
@@ -65,26 +68,55 @@ def dense_rows(x, weight, bias):
     return F.linear(x, weight, bias) if out is None else out
 
 
+@functools.lru_cache(maxsize=64)
+def _copies_layout(rows, cols, with_bias, turned):
+    """The copies that _half_copies makes, and where the weight's, its transpose and the bias's begin: on multiples of 512 bytes,
+    as allocations of their own would."""
+    step = rows * cols + -rows * cols % 256
+    at = [0, step if turned else -1, step * (2 if turned else 1)]
+    copies = (_lib.HalfCopy * 2)((rows, cols, 0, 0, at[1], -1, 1.0), (rows, 1, 0, at[2], -1, -1, 1.0))
+    return copies, at, at[2] + (rows if with_bias else 0)
+
+
+def _half_copies(weight, bias, turned):
+    """(weight, its transpose or None, bias or None) in fp16 by one launch, in place of one each; None where they are not plain
+    fp32 arrays of whole pieces."""
+    given = [weight] if bias is None else [weight, bias]
+    rows, cols = weight.shape
+    if not weight.is_cuda or rows % 8 or cols % 8 or any(t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16 for t in given):
+        return None
+    copies, at, count = _copies_layout(rows, cols, bias is not None, turned)
+    half = torch.empty(count, dtype=torch.float16, device=weight.device)
+    with _lib.on(weight.device):
+        status = _lib.lib().s3d_half_copies((ctypes.c_void_p * len(given))(*[t.data_ptr() for t in given]), copies, len(given), half.data_ptr(), None,
+                                            _lib.stream(weight.device))
+    _lib.check(status, "s3d_half_copies")
+    return (half.as_strided((rows, cols), (cols, 1), 0), half.as_strided((cols, rows), (rows, 1), at[1]) if turned else None,
+            None if bias is None else half.as_strided((rows,), (1,), at[2]))
+
+
 class _Linear(Function):
     """F.linear in fp16 of fp16 rows and parameters in fp16 or fp32, whose gradients come in their own type: autocast would
     round them to fp16 on the way."""
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        half = weight.to(torch.float16)
-        ctx.save_for_backward(x, weight, half)
+        copies = _half_copies(weight, bias, ctx.needs_input_grad[0])
+        half, turned, half_bias = copies if copies is not None else (
+            weight.to(torch.float16), None, None if bias is None else bias.to(torch.float16))
+        ctx.save_for_backward(x, weight, half, turned)
         ctx.bias_dtype = None if bias is None else bias.dtype
-        return dense_rows(x, half, None if bias is None else bias.to(torch.float16))
+        return dense_rows(x, half, half_bias)
 
     @staticmethod
     def backward(ctx, dy):
-        x, weight, half = ctx.saved_tensors
+        x, weight, half, turned = ctx.saved_tensors
         need_x, need_weight, need_bias = ctx.needs_input_grad
         dx = grads = None
         if not torch.is_grad_enabled():
             dy = dy.contiguous()
             if need_x:
-                dx = linear_rows(dy, half.t().contiguous(), None)
+                dx = linear_rows(dy, half.t().contiguous() if turned is None else turned, None)
                 dx = dy.mm(half) if dx is None else dx
             if need_weight or need_bias:
                 grads = _weight_gradients(dy, x.contiguous(), need_weight, need_bias, weight.dtype if need_weight else ctx.bias_dtype)
