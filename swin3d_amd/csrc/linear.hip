@@ -3,13 +3,13 @@
 // (rows = voxels), K and N a few dozen to a few thousand.
 //
 // Both operands are contiguous along K, which is how a lane of v_mfma_f32_32x32x16 wants them: eight consecutive numbers
-// of a row.  A workgroup stages 64 numbers of K of its rows of X and W in LDS (the next 64 on their way in registers
+// of a row.  A workgroup stages 64 numbers of K of its rows of X and W in LDS (the next 64 on their way into a second buffer
 // meanwhile) with the 16-byte pieces of a row in an order that depends on the row, so that the lanes' reads of 32 rows
 // spread over all banks; W goes in as the first operand, so that a lane ends up with four neighbouring outputs of one
 // row, and the tile leaves through LDS as whole rows.
 //
-// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 173 us against
-// 416 us as product and GELU apart; 80 -> 240, 108 us against 207, at 3.6 of the 4.7 TB/s that a copy reaches.  At the
+// At the first levels the layers are bound by memory (K and N below 400): 600,000 rows, 80 -> 320 with GELU, 165 us against
+// 416 us as product and GELU apart; 80 -> 240, 96 us against 207, at 4.0 of the 4.7 TB/s that a copy reaches.  At the
 // deepest the tiles are few and a tile's chain of chunks is what counts (linear_thin_kernel): 390 rows, 384 -> 384, 3.4 us against 18
 // through torch, whose launch alone takes the host that long.
 #include "attn_kernels.h"
@@ -58,6 +58,16 @@ enum class Behind { kNothing, kGelu, kGeluGrad, kGeluBeside };
 // The place of 16-byte piece p of row r: sixteen consecutive rows' pieces p lie in 64 different banks.
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
 
+// Sixteen bytes a lane from `from` to the wavefront's 1024 at `to` in LDS.  The compiler knows nothing of them: who reads them
+// has waited for them (loads and stores end in the order of their issue) and met the other wavefronts at a barrier.
+__device__ __forceinline__ void load_to_lds(uint32_t to, const void *from)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory");
+}
+// ... all but the kBehind instructions issued last
+template <int kBehind> __device__ __forceinline__ void loads_done() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory"); }
+__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // WM x WN wavefronts of TM x TN products of 32 x 32
 template <int WM, int WN, int TM, int TN> struct Tile {
     static_assert(WM * WN == kThreads / 64, "four wavefronts");
@@ -70,13 +80,19 @@ template <int WM, int WN, int TM, int TN> struct Tile {
     static constexpr int kLoads = (kM + kN) * kPieces / kThreads;     // pieces per thread and chunk
 };
 
-// A workgroup works on tile after tile: the first chunk of the next one is on its way in registers while the last chunk is
+// A workgroup works on tile after tile: the first chunk of the next one is on its way while the last chunk is
 // multiplied and the finished rows leave, each wavefront's through its own part of the buffer that has just been multiplied (no
-// barrier).  With a workgroup a tile, a tile's first load waited for all that.  us at 600,000 rows, before / so: 80 -> 240
-// 126 / 108, 80 -> 80 52 / 43, 80 -> 320 with GELU 201 / 173 (of which GELU's instructions are 98), 320 -> 80 117 / 105; 199,327
-// rows, 48 -> 144 24 / 18; 9,000 rows, 640 -> 1920 36 / 32; 3,000 rows, where every tile has a workgroup, the same.  Two chunks
-// ahead, as one sequence over the tiles, was 5 % slower at K = 80 and up to 40 % at K above 300 (addresses, and a loop in two
-// halves).
+// barrier); where they all are rows of the result, the wait for that chunk leaves their stores under way.  With a workgroup a tile,
+// a tile's first load waited for all that.
+//
+// Chunks go from memory to LDS without a register between.  Through registers a chunk was held by every thread until it was needed,
+// stored (a quarter of LDS's time and of the instructions), and two barriers met per tile's end.  us, through registers / so: 9,400
+// rows, 2560 -> 640 49.5 / 43.7, 640 -> 1920 33.7 / 30.4; 37,500, 1280 -> 320 51.3 / 45.2, 320 -> 960 38.7 / 34.8; 595,677, 80 -> 240 106 / 96;
+// 12,421, 768 -> 192 11.1 / 9.7; 3,105, 1536 -> 384 13.6 / 11.1; 776 and 390 rows of it 9.8 / 8.3; 199,327, 48 -> 48, bound by its rows, 8.7 / 8.4.
+// The matrix pipe is busy for a third of the time: a chunk of 128 x 128 is 512 clocks of it and 768 of LDS, and each waits for the
+// chunk before.  A third, fourth and fifth buffer, which leave fewer workgroups a CU, were 2 to 15 % slower; operands of the
+// next step read ahead 10 to 20 % (spread over the buffers by sched_barriers); 256 x 128 by eight wavefronts the same, 256 x 256 up
+// to 1.5 times as long where the last round is nearly empty.
 template <typename L, Behind kBehind>
 __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__restrict__ x, const _Float16 *__restrict__ w,
                                                              const _Float16 *__restrict__ bias, _Float16 *__restrict__ y,
@@ -95,27 +111,22 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
     const int r32 = lane & 31, half = lane >> 5;
     const int whole = (K - 1) / kChunk;      // chunks before the last one
 
-    // this thread's pieces of a chunk: row (tid / 8 + 32 i) of [X rows, W rows], piece tid % 8
-    const int piece = tid % kPieces, row = tid / kPieces;
+    // This thread's pieces of a chunk: row (tid / 8 + 32 i) of [X rows, W rows], and of it the piece whose place is lane % 8, as
+    // sixteen bytes a lane go to consecutive places.  Where the last chunk has no such piece the lane loads its first one.
+    const int row = tid / kPieces, piece = (lane ^ (row >> 1)) & (kPieces - 1);
     const _Float16 *from[L::kLoads];
+    const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
     auto aim = [&](int m0, int n0) {
 #pragma unroll
         for (int i = 0; i < L::kLoads; ++i) {
             const int r = row + i * (kThreads / kPieces);
-            from[i] = (r < L::kM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r - L::kM, N - 1)) * K) + piece * 8;
+            from[i] = r < L::kM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K : w + static_cast<int64_t>(min(n0 + r - L::kM, N - 1)) * K;
         }
     };
-    uint4 held[L::kLoads];
-    auto fetch = [&](int k0) {
-        if (k0 + piece * 8 < K) {
+    auto fetch = [&](int buffer, int k0) {
+        const int k = k0 + (k0 + piece * 8 < K ? piece * 8 : 0);
 #pragma unroll
-            for (int i = 0; i < L::kLoads; ++i) held[i] = *reinterpret_cast<const uint4 *>(from[i] + k0);
-        }
-    };
-    auto put = [&](int buffer) {
-        uint4 *to = reinterpret_cast<uint4 *>(smem + buffer * L::kStage);
-#pragma unroll
-        for (int i = 0; i < L::kLoads; ++i) to[placed(row + i * (kThreads / kPieces), piece)] = held[i];
+        for (int i = 0; i < L::kLoads; ++i) load_to_lds(lds + buffer * L::kStage + i * (kThreads * 16) + wave * 1024, from[i] + k);
     };
     f32x16 acc[TM][TN];
     auto multiply = [&](int buffer, int steps) {
@@ -134,26 +145,30 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
                 for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[j], a[i], acc[i][j], 0, 0, 0);
         }
     };
-#pragma unroll
-    for (int i = 0; i < L::kLoads; ++i) held[i] = make_uint4(0, 0, 0, 0);
     int buffer = 0;
+    bool inside = false;      // the tile before left all its rows and columns: as many stores behind the loads under way
     aim(tile / tiles_n * L::kM, tile % tiles_n * L::kN);
-    fetch(0);
-    put(0);
-    __syncthreads();
+    fetch(0, 0);
     for (; tile < end; tile += step) {
         const int m0 = tile / tiles_n * L::kM, n0 = tile % tiles_n * L::kN;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+        // the chunk is there, and nobody reads the other buffer any more
+        auto meet = [&]() {
+            if (inside) loads_done<TM * 2 * TN * (kBehind == Behind::kGeluBeside ? 2 : 1)>();
+            else loads_done<0>();
+            inside = false;
+            workgroup_barrier();
+        };
         for (int c = 0; c < whole; ++c) {
-            fetch((c + 1) * kChunk);
+            meet();
+            fetch(buffer ^ 1, (c + 1) * kChunk);
             multiply(buffer, kChunk / 16);
             buffer ^= 1;
-            put(buffer);
-            __syncthreads();
         }
+        meet();
         // what the end of the tile reads, before the next tile's first chunk: loads return in order
         half4 b[TN][4];
         half8 at[TM][2 * TN];
@@ -177,10 +192,11 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
         const int next = tile + step;
         if (next < end) {
             aim(next / tiles_n * L::kM, next % tiles_n * L::kN);
-            fetch(0);
+            fetch(buffer ^ 1, 0);
         }
         multiply(buffer, (K - whole * kChunk) / 16);
-        __syncthreads();
+        workgroup_barrier();
+        inside = m0 + L::kM <= M && n0 + L::kN <= N;
         // a lane's outputs: row r32 of X, columns 8 g + 4 half .. + 3 of W's 32.  They become rows in the wavefront's own part of
         // the buffer that is free now.
         _Float16 *out = reinterpret_cast<_Float16 *>(smem + buffer * L::kStage) + wave * (32 * L::kPitch);
@@ -207,7 +223,7 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
                     for (int k = 0; k < 8; ++k) v[k] = static_cast<_Float16>(static_cast<float>(v[k]) * gelu_slope(static_cast<float>(at[i][t][k])));
                 }
                 const int64_t to = static_cast<int64_t>(m0 + wave_m + i * 32 + r) * N + n0 + wave_n + n;
-                const bool there = m0 + wave_m + i * 32 + r < M && n0 + wave_n + n < N;
+                const bool there = inside || (m0 + wave_m + i * 32 + r < M && n0 + wave_n + n < N);
                 if (there) *reinterpret_cast<half8 *>(y + to) = v;
                 if constexpr (kBehind == Behind::kGeluBeside) {
 #pragma unroll
@@ -217,8 +233,6 @@ __global__ __launch_bounds__(kThreads, 2) void linear_kernel(const _Float16 *__r
             }
         }
         buffer ^= 1;
-        if (next < end) put(buffer);
-        __syncthreads();
     }
 }
 
@@ -356,23 +370,30 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     // at 640 6.3 / 8.0; 1880 at 2560 27.0 / 35.4.
     const int64_t thin = ceil_div(a.M, 32) * ((a.N + 31) / 32);
     if (!a.gelu_at && !a.in_order && (thin <= 256 || (thin <= 512 && a.K >= 192) || (thin <= 1024 && a.K >= 2048))) return launch_thin(a, stream);
-    // Tiles of 64 x 64 as long as larger ones would leave CUs without work (with GELU's derivative and up to 384 channels until there
-    // are 6144 of them, its instructions being hidden by more wavefronts: 0.87 to 0.98 of the time at 1100 to 1700 and 2300 to 6000
+    // Tiles of 64 x 64 as long as larger ones would leave CUs without work: up to 576 of them, with GELU or its derivative, whose
+    // instructions more wavefronts hide, up to 1024 (768 and 576 to 192, 64 x 64 / 128 x 64, us, by number: 288 6.7 / 7.0, 576 8.8 / 8.5,
+    // 720 9.4 / 9.1, 864 11.8 / 9.6; with GELU 585 9.6 / 10.6).  With GELU's derivative and up to 384 channels until there
+    // are 6144 of them (0.87 to 0.98 of the time at 1100 to 1700 and 2300 to 6000
     // tiles, 62,000 rows of 96 34.0 -> 29.7 us, 12,421 of 192 18.6 -> 15.8; 1.01 to 1.08 at some 1900 and at 3000; 1.02 to 1.12
     // beyond, and 1.12 to 1.22 at 640 channels); then 128 rows by the width that pads N least,
-    // the widest of those that still give every CU two tiles.  192 columns take all of a wavefront's registers: with GELU only
+    // the widest of those that still fill the chip: of 128 columns two are on a CU, so between 384 and 512 they end in one round and
+    // from 640 on the second is full enough (640 -> 640, 128 x 128 / 128 x 64, us, by number: 355 13.2 / 12.8, 385 13.8 / 15.7, 450
+    // 14.7 / 16.8, 515 21.0 / 18.3, 560 20.6 / 19.5; 1536 -> 384: 354 25.7 / 26.1, 450 28.3 / 35.7, 561 41.8 / 38.9, 642 41.6 / 49.7; with
+    // GELU the first is from 448 on).  Over nineteen layers of 96 to 2560 and 96 to 1400 such tiles the choice is 0.8 % behind
+    // the best of the three in the mean.  192 columns take all of a wavefront's registers: with GELU only
     // where the tile is the whole row, with its derivative not at all (63 would spill).
     // So, too, with erff's GELU beside the rows, whose fifty instructions a number overlap with other tiles' loads only where
     // several tiles share a SIMD.  us, torch's GELU behind the layer / larger tiles / so: 199,327 rows of 48 to 192 47.0 / 50.9 / 45.0,
     // 49,682 of 96 to 384 30.8 / 34.9 / 26.5, 12,421 of 192 to 768 25.8 / 23.3 / 17.1, 3,105 of 384 to 1536 19.9 / 14.9 / 12.6;
     // 6,250 of 96 11.2 / 7.4.
     const int64_t small = ceil_div(a.M, 64) * ((a.N + 63) / 64);
-    if (a.gelu_out || small < 1024 || (a.gelu_at && a.K <= 384 && small <= 6144)) return launch<Tile<2, 2, 1, 1>>(a, stream);
+    const bool heavy = a.gelu || a.gelu_at;
+    if (a.gelu_out || small < (heavy ? 1024 : 576) || (a.gelu_at && a.K <= 384 && small <= 6144)) return launch<Tile<2, 2, 1, 1>>(a, stream);
     auto padded = [&](int width) { return (a.N + width - 1) / width * width; };
-    auto enough = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width) >= 512; };
+    auto count = [&](int width) { return ceil_div(a.M, 128) * (padded(width) / width); };
     const int least = padded(64);
-    if (padded(192) == least && enough(192) && !a.gelu_at && (!a.gelu || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
-    if (padded(128) == least && enough(128)) return launch<Tile<2, 2, 2, 2>>(a, stream);
+    if (padded(192) == least && count(192) >= 512 && !a.gelu_at && (!a.gelu || a.N <= 192)) return launch<Tile<2, 2, 2, 3>>(a, stream);
+    if (padded(128) == least && ((count(128) >= (heavy ? 448 : 384) && count(128) <= 512) || count(128) >= 640)) return launch<Tile<2, 2, 2, 2>>(a, stream);
     return launch<Tile<2, 2, 2, 1>>(a, stream);
 }
 

@@ -40,6 +40,13 @@ def test_linear_of_few_rows(hip_lib, m, n, k, gelu):
     test_linear(hip_lib, m, n, k, gelu)
 
 
+@pytest.mark.parametrize("m,n", [(64 * tiles - 59, 64) for tiles in (575, 576, 1023, 1024)] +        # 64 x 64, 128 x 64
+                         [(128 * tiles - 123, 128) for tiles in (383, 384, 447, 448, 512, 513, 639, 640, 1100)])        # ... and 128 x 128
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_where_its_tiles_change(hip_lib, m, n, gelu):
+    test_linear(hip_lib, m, n, 208, gelu)        # (three chunks and a quarter)
+
+
 def test_gelu_of_every_number(hip_lib):
     """All finite fp16 numbers through the identity: half a place of rounding, and the approximation, which is fp32's own
     rounding and below 2^-25 where the result is too small for fp16."""
