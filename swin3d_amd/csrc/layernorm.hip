@@ -10,6 +10,7 @@
 // One group of G lanes per row (G = 16, 32 or 64 by row length), 16-byte loads, two-pass mean / variance in
 // registers (the row stays in registers between the passes), fp32 arithmetic.
 #include "s3d_common.h"
+#include "linear.h"
 
 #include <hip/hip_fp16.h>
 
@@ -319,7 +320,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_train_add_layernorm(co
 // Memory bound: the rows of sum, dsum, dy once in, d (and its fp16 copy) once out.  Mean and deviation are taken again from
 // the row, which is read anyway.  A lane keeps its channels' share of dgamma and dbeta in registers over all the rows that
 // its group draws; the groups of a workgroup add theirs in LDS and leave a part per workgroup, in a fixed order.
-// 199,327 rows of 48: 24 us (153 MB moved, 6.5 TB/s), 12,421 of 192: 12 us and the parts' sum 5; through torch the same
+// 199,327 rows of 48: 24 us (153 MB moved, 6.5 TB/s), 12,421 of 192: 12 us and the parts' sum 4.7 (linear_grad_sum_kernel); through torch the same
 // three gradients took 300 us and 40, with two more passes for the sum with dsum and the fp16 copy.
 namespace s3d {
 namespace {
@@ -427,28 +428,6 @@ template <int G, int CH> __global__ __launch_bounds__(kLnThreads) void layernorm
     }
 }
 
-// The sum of the parts: 16 numbers a workgroup, 64 shares of the parts each (sixteen were a chain of eight trips to memory).
-constexpr int kSumThreads = 1024;
-
-__global__ __launch_bounds__(kSumThreads) void layernorm_grad_sum_kernel(const float *__restrict__ parts, int count, int C,
-                                                                         float *__restrict__ dgamma, float *__restrict__ dbeta)
-{
-    constexpr int kShares = kSumThreads / 16;
-    __shared__ float shared[kSumThreads];
-    const int e = threadIdx.x & 15, share = threadIdx.x >> 4, c = static_cast<int>(blockIdx.x) * 16 + e, at = min(c, 2 * C - 1);
-    float sum = 0.0f;
-#pragma unroll 8
-    for (int p = share; p < count; p += kShares) sum += parts[static_cast<int64_t>(p) * 2 * C + at];
-    shared[threadIdx.x] = sum;
-#pragma unroll
-    for (int half = kShares / 2; half > 0; half /= 2) {
-        __syncthreads();
-        if (share < half) shared[threadIdx.x] = sum += shared[threadIdx.x + 16 * half];
-    }
-    if (share > 0 || c >= 2 * C) return;
-    (c < C ? dgamma[c] : dbeta[c - C]) = sum;
-}
-
 // lanes a row: as few as hold it in two chunks each
 int ln_lanes(int C) { return C <= 128 ? 16 : C <= 256 ? 32 : 64; }
 
@@ -462,11 +441,28 @@ int64_t ln_parts(int64_t N, int C)
 bool ln_fits(int64_t N, int32_t C) { return N >= 1 && C >= 4 && C % 4 == 0 && C <= 4 * kMaxChunks * 64; }
 
 }  // namespace
+
+size_t layernorm_grad_bytes(int64_t N, int32_t C) { return ln_fits(N, C) ? static_cast<size_t>(ln_parts(N, C)) * 2 * C * sizeof(float) : 0; }
+
+int launch_layernorm_grad(const float *sum, const float *dsum, const void *dy, const float *gamma, float eps, float *dx, void *dresidual, NormGrad *norm,
+                          int64_t N, int32_t C, float *parts, hipStream_t stream)
+{
+    const LnGradArgs args{sum, dsum, static_cast<const __half *>(dy), gamma, eps, dx, static_cast<__half *>(dresidual), parts, N, C};
+    norm->parts = parts;
+    norm->count = static_cast<int>(ln_parts(N, C));
+    norm->C = C;
+    auto kernel = C <= 64 ? layernorm_grad_kernel<16, 1> : C <= 128 ? layernorm_grad_kernel<16, 2> : C <= 256 ? layernorm_grad_kernel<32, 2>
+                  : C <= 512 ? layernorm_grad_kernel<64, 2> : layernorm_grad_kernel<64, 4>;
+    hipLaunchKernelGGL(kernel, dim3(norm->count), dim3(kLnThreads), 0, stream, args);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
+}
+
 }  // namespace s3d
 
 extern "C" __attribute__((visibility("default"))) size_t s3d_layernorm_grad_workspace_bytes(int64_t N, int32_t C)
 {
-    return s3d::ln_fits(N, C) ? static_cast<size_t>(s3d::ln_parts(N, C)) * 2 * C * sizeof(float) : 0;
+    return s3d::layernorm_grad_bytes(N, C);
 }
 
 extern "C" __attribute__((visibility("default"))) int s3d_layernorm_grad(
@@ -481,15 +477,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_layernorm_grad(
     if (!workspace || workspace_bytes < need)
         return fail(S3D_ERR_WORKSPACE, "s3d_layernorm_grad: workspace %zu B < required %zu B", workspace ? workspace_bytes : size_t(0), need);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const LnGradArgs args{sum, dsum, static_cast<const __half *>(dy), gamma, eps, dx, static_cast<__half *>(dresidual),
-                          static_cast<float *>(workspace), N, C};
-    const int parts = static_cast<int>(ln_parts(N, C));
-    auto kernel = C <= 64 ? layernorm_grad_kernel<16, 1> : C <= 128 ? layernorm_grad_kernel<16, 2> : C <= 256 ? layernorm_grad_kernel<32, 2>
-                  : C <= 512 ? layernorm_grad_kernel<64, 2> : layernorm_grad_kernel<64, 4>;
-    hipLaunchKernelGGL(kernel, dim3(parts), dim3(kLnThreads), 0, s, args);
-    S3D_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(layernorm_grad_sum_kernel, dim3(static_cast<unsigned>(ceil_div(2 * C, 16))), dim3(kSumThreads), 0, s,
-                       args.parts, parts, C, dgamma, dbeta);
-    S3D_HIP_CHECK(hipGetLastError());
-    return S3D_OK;
+    NormGrad norm{nullptr, dgamma, dbeta};
+    if (int rc = launch_layernorm_grad(sum, dsum, dy, gamma, eps, dx, dresidual, &norm, N, C, static_cast<float *>(workspace), s)) return rc;
+    return launch_linear_grad_sums(nullptr, 0, &norm, S3D_DTYPE_F32, s);
 }

@@ -46,7 +46,18 @@ constexpr int kMostLinearGrads = 4;
 size_t linear_grads_bytes(const LinearGrad *grads, int num);
 // the parts of `num` layers of as many rows, to *parts and on, which is moved behind them
 int launch_linear_grad_parts(LinearGrad *grads, int num, float **parts, hipStream_t stream);
-// the sums of the parts of `num` layers in one launch
-int launch_linear_grad_sums(const LinearGrad *grads, int num, int32_t grad_dtype, hipStream_t stream);
+
+// The gradients of (sum, y) = (x + residual, LayerNorm(x + residual)) (layernorm.hip), those of the norm's parameters in parts
+struct NormGrad {
+    const float *parts;      // [count][2 C]: of the weight, of the bias
+    float *dgamma, *dbeta;
+    int32_t count, C;
+};
+size_t layernorm_grad_bytes(int64_t N, int32_t C);
+int launch_layernorm_grad(const float *sum, const float *dsum, const void *dy, const float *gamma, float eps, float *dx, void *dresidual, NormGrad *norm,
+                          int64_t N, int32_t C, float *parts, hipStream_t stream);
+
+// the sums of the parts of `num` layers and, unless null, of a norm in one launch
+int launch_linear_grad_sums(const LinearGrad *grads, int num, const NormGrad *norm, int32_t grad_dtype, hipStream_t stream);
 
 }  // namespace s3d

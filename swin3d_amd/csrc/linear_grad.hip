@@ -174,6 +174,8 @@ struct GradSums {
     int n[kMostLinearGrads], k[kMostLinearGrads], splits[kMostLinearGrads], scaled[kMostLinearGrads];
     int first[kMostLinearGrads];      // the first workgroup of each
     float scale[kMostLinearGrads];
+    NormGrad norm;
+    int first_norm;
 };
 
 // Four results to where they fit in one piece, which a gradient inside a larger buffer may not
@@ -192,10 +194,30 @@ template <typename T> __device__ __forceinline__ void store_four(T *to, const f3
 // of a Swin block's four are 5 us each by themselves, for some 20 MB of parts.
 // With 16-byte loads, where they were 4 bytes, and half the parts (launch_linear_grad_parts), us a block: 96 channels, 50,000 rows, 15 / 10; 192,
 // 12,400, 16 / 8; 384, 3,000, 21 / 9; 384, 811, 17.5 / 7.5 (35 MB).
+// The parts of a norm, up to 1024 of 2 C numbers, are summed beside them, 16 numbers a workgroup and 64 shares of the parts (sixteen
+// were a chain of eight trips to memory).  In a launch of its own behind every block that was 4.5 us
+// and the gap before it; 24 blocks, 200,000 voxels: the sums 619 us a pass -> 522, the pass 29.5 ms -> 29.2.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void linear_grad_sum_kernel(GradSums a)
 {
     __shared__ f32x4 shared[kThreads];
+    if (static_cast<int>(blockIdx.x) >= a.first_norm) {
+        typedef float four __attribute__((ext_vector_type(4), aligned(4)));      // (the caller's scratch memory, as it is)
+        constexpr int kShares = kThreads / 4;
+        const int share = threadIdx.x / 4, c = (static_cast<int>(blockIdx.x) - a.first_norm) * 16 + threadIdx.x % 4 * 4, width = 2 * a.norm.C;
+        const float *from = a.norm.parts + min(c, width - 4);
+        f32x4 sum = {};
+#pragma unroll 8
+        for (int p = share; p < a.norm.count; p += kShares) sum += *reinterpret_cast<const four *>(from + static_cast<int64_t>(p) * width);
+        shared[threadIdx.x] = sum;
+#pragma unroll
+        for (int half = kShares / 2; half > 0; half /= 2) {
+            __syncthreads();
+            if (share < half) shared[threadIdx.x] = sum += shared[threadIdx.x + 4 * half];
+        }
+        if (share == 0 && c < width) store_four(c < a.norm.C ? a.norm.dgamma + c : a.norm.dbeta + (c - a.norm.C), sum);
+        return;
+    }
     int at = 0;
 #pragma unroll
     for (int i = 1; i < kMostLinearGrads; ++i) at = static_cast<int>(blockIdx.x) >= a.first[i] ? i : at;
@@ -345,7 +367,7 @@ int launch_linear_grad_parts(LinearGrad *grads, int num, float **parts, hipStrea
     return S3D_OK;
 }
 
-int launch_linear_grad_sums(const LinearGrad *grads, int num, int32_t grad_dtype, hipStream_t stream)
+int launch_linear_grad_sums(const LinearGrad *grads, int num, const NormGrad *norm, int32_t grad_dtype, hipStream_t stream)
 {
     GradSums a{};
     int64_t blocks = 0;
@@ -365,6 +387,12 @@ int launch_linear_grad_sums(const LinearGrad *grads, int num, int32_t grad_dtype
         a.first[i] = static_cast<int>(blocks);
         blocks += ceil_div(a.products[i] + g.N, 256);      // (at most 2^20 + 64 a layer)
     }
+    a.first_norm = static_cast<int>(blocks);
+    if (norm) {
+        a.norm = *norm;
+        blocks += ceil_div(2 * norm->C, 16);
+    }
+    if (blocks == 0) return S3D_OK;
     if (grad_dtype == S3D_DTYPE_F32)
         hipLaunchKernelGGL(linear_grad_sum_kernel<float>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream, a);
     else
@@ -400,5 +428,5 @@ extern "C" __attribute__((visibility("default"))) int s3d_linear_grad(
     LinearGrad g{dy, x, dw, db, M, N, K, 0, 1.0f};
     float *parts = static_cast<float *>(workspace);
     if (int rc = launch_linear_grad_parts(&g, 1, &parts, s)) return rc;
-    return launch_linear_grad_sums(&g, 1, grad_dtype, s);
+    return launch_linear_grad_sums(&g, 1, nullptr, grad_dtype, s);
 }

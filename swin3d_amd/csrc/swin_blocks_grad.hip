@@ -6,14 +6,15 @@
 // at 10,000 voxels.  Here the launches follow each other with nothing in between.  And there are fewer of them: the
 // derivative of GELU is taken where fc2's gradient leaves its tile (a launch and two passes over the hidden layer less),
 // dq, dk, dv are written where the projection's gradient reads them (no stacking copy), the parts of two
-// layers' weight gradients come from one launch where their tiles are the same, and those of all four are summed by one.
+// layers' weight gradients come from one launch where their tiles are the same, and those of all four and of the norm are
+// summed by one.
 #include "linear.h"
 
 namespace s3d {
 namespace {
 
 struct Places {
-    size_t wide, normed, residual, parts, rest, total;
+    size_t wide, normed, residual, parts, norm, rest, total;
 };
 
 // the layers in the order of the calls: fc2, fc1, proj, qkv
@@ -30,7 +31,8 @@ Layers layers_of(int64_t N, int32_t C, int32_t hidden)
 }
 
 // wide: the hidden layer's gradient, then that of q, k, v;  normed: that of LayerNorm's rows, then of the attention's
-// result;  residual: that of proj's result;  parts: of the weights' gradients;  rest: the scratch of one call at a time
+// result;  residual: that of proj's result;  parts, norm: of the weights' and of
+// the norm's gradients;  rest: the scratch of one call at a time
 Places places_of(int64_t N, int32_t C, int32_t hidden, int32_t H, int32_t D, int32_t nd, int64_t table_len, int64_t W, int64_t pairs)
 {
     Places p;
@@ -40,9 +42,9 @@ Places places_of(int64_t N, int32_t C, int32_t hidden, int32_t H, int32_t D, int
     p.residual = p.normed + align_up(row * C, 256);
     p.parts = p.residual + align_up(row * C, 256);
     const Layers layers = layers_of(N, C, hidden);
-    p.rest = p.parts + align_up(linear_grads_bytes(layers.of, kMostLinearGrads), 256);
-    const size_t attention = s3d_attn_bwd_workspace_least_bytes(H, D, nd, table_len, N, W, pairs), norm = s3d_layernorm_grad_workspace_bytes(N, C);
-    p.total = p.rest + (attention > norm ? attention : norm);
+    p.norm = p.parts + align_up(linear_grads_bytes(layers.of, kMostLinearGrads), 256);
+    p.rest = p.norm + align_up(layernorm_grad_bytes(N, C), 256);
+    p.total = p.rest + s3d_attn_bwd_workspace_least_bytes(H, D, nd, table_len, N, W, pairs);
     return p;
 }
 
@@ -140,8 +142,9 @@ extern "C" __attribute__((visibility("default"))) int s3d_swin_block_grad(
     layer(wide, b.normed2, g.fc1_weight, g.fc1_bias, hidden, C, 0, 1.0f);
     if (int rc = launch_parts()) return rc;
     if (int rc = launch_linear({wide, b.fc1_weight_t, nullptr, normed, N, C, hidden, false}, s)) return rc;
-    if (int rc = s3d_layernorm_grad(b.sum, dsum, normed, b.norm2_weight, b.norm2_eps, g.x, residual, g.norm2_weight, g.norm2_bias, N, C,
-                                    rest, rest_bytes, stream))
+    NormGrad norm{nullptr, g.norm2_weight, g.norm2_bias};
+    if (int rc = launch_layernorm_grad(b.sum, dsum, normed, b.norm2_weight, b.norm2_eps, g.x, residual, &norm, N, C,
+                                       reinterpret_cast<float *>(base + p.norm), s))
         return rc;
     layer(residual, b.attended, g.proj_weight, g.proj_bias, C, C, 0, 1.0f);
     if (int rc = launch_linear({residual, b.proj_weight_t, nullptr, normed, N, C, C, false}, s)) return rc;
@@ -153,5 +156,5 @@ extern "C" __attribute__((visibility("default"))) int s3d_swin_block_grad(
     layer(wide, b.normed1, g.qkv_weight, g.qkv_bias, 3 * C, C, C, q_scale);
     if (int rc = launch_parts()) return rc;
     if (int rc = launch_linear({wide, b.qkv_weight_t, nullptr, g.normed1, N, C, 3 * C, false}, s)) return rc;
-    return num > 0 ? launch_linear_grad_sums(wanted, num, S3D_DTYPE_F32, s) : S3D_OK;
+    return launch_linear_grad_sums(wanted, num, &norm, S3D_DTYPE_F32, s);
 }
