@@ -328,11 +328,12 @@ struct StripArgs {
                                 // the records)
     const int32_t *column_rows; // [strip][column]: the rows alone
     const float *scales;        // [head][Tq, Tk, Tv]: what a product with the table's operand is multiplied by
-    float *slots;               // [workgroup][kind][tile][lane][4]: table gradients as the products leave them
+    float *slots;               // [workgroup][kind][tile][lane][4]: table gradients as the products leave them, by query
     void *dq, *dk, *dv;
     uint32_t grad_stride;       // elements between rows of dq, dk, dv (of q, k, v: f.row_stride)
     float *dtq, *dtk, *dtv;
     float half_rows[kMaxAxes], upper[kMaxAxes];    // what crse_row takes (made here, they would take two vector registers an axis)
+    float *key_slots;           // ... and by key
 };
 // The kernels that leave dL and P of every pair, at head_dim 16: on tiles (attn_tile_bwd.hip, fp32 and small windows) or strips
 // (attn_strip_records.hip, fp16 features).

@@ -96,11 +96,12 @@ __device__ __forceinline__ void add_left_out(float *shared, const uint32_t *stri
 {
     constexpr int C = 8;
     const void *at_args = (const void *)__builtin_amdgcn_kernarg_segment_ptr();
-    int tid = threadIdx.x, block = blockIdx.x;
+    const int blocks = static_cast<int>(gridDim.x) / 2;
+    int tid = threadIdx.x, block = static_cast<int>(blockIdx.x) - (kByKey ? blocks : 0);
     asm volatile("" : "+s"(at_args), "+v"(tid), "+s"(block));
     const StripArgs &b = *static_cast<const StripArgs *>(at_args);
     const AttnArgs &a = b.f;
-    const int H = a.H, HD = H * C, h = block % H, group = block / H, groups = static_cast<int>(gridDim.x) / H, strips = b.list.total[1];
+    const int H = a.H, HD = H * C, h = block % H, group = block / H, groups = blocks / H, strips = b.list.total[1];
     const int c16 = tid & 15, channel = tid >> 4 & 7, part = tid >> 7;
     const TF *gd = static_cast<const TF *>(b.dout) + h * C;
     const float2 *records = b.records + static_cast<int64_t>(h) * b.pairs;
@@ -192,39 +193,68 @@ __device__ __forceinline__ void add_left_out(float *shared, const uint32_t *stri
 
 // C channels a head: 16, or 8 (packed): q or k and dout then share the sixteen channels of an operand, dTq and dTv the sixteen
 // columns of a product, and dk and dv its rows.
-template <typename T, typename TF, int ND, bool kByKey, int C>
-__global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(StripArgs b)
-{
+template <typename T, typename TF, int ND, bool kByKey, int C> struct StripForm {
     using Table = typename StripTable<T, TF>::type;
+    static constexpr bool kPacked = C == 8;
+    static constexpr int kKinds = kByKey ? 1 : 2, kOwn = kOwnTiles<ND>;
+    static constexpr int kSets = kPacked ? 1 : kKinds;        // of features, and of table gradients
+    static constexpr int kParts = kByKey && !kPacked ? 2 : 1; // of dx: dk and dv
+    // Pieces of the table's operands that wait in LDS, as many as leave room for two workgroups a CU (81,864 of 81,920 bytes by
+    // query in fp32).  In registers they would not fit beside the rest, and a spilled operand comes back from memory behind the
+    // pairs of the next strip, which are on their way then: loads return in order.
+    static constexpr int kTableParts = sizeof(Table) / 8, kPieces = kTableParts * kOwn;
+    static constexpr int kShared = kByKey || kPieces < kOwn + 2 ? kPieces : kOwn + 2, kKeptPieces = kPieces - kShared;
+    using Cells = uint32_t[kTiles<ND> * 16 * kStrip * kKinds];      // [row][column]: dL, by query behind P
+    using Sums = float[kParts * kStripWaves * 256];                 // parts of dx (by key: and dv), one a wavefront
+    using Features = Exact4<TF>[kSets][64];                         // q or k, dout of the strip's voxels
+    using Pieces = u32x2[kShared][kStripThreads];
+    using AbsSums = float[kStripWaves][kStrip];
+    using Marks = uint32_t[2 * kTiles<ND>];
+    using Met = uint32_t[kPacked ? kMetWords : 1];
+    struct Lds {
+        alignas(16) Cells cells;
+        alignas(16) Sums part;
+        alignas(16) Features features;
+        Pieces table;
+        AbsSums sums;
+        float grad;
+        Marks marks;
+        uint32_t marked;
+        Met met;
+    };
+    static_assert(sizeof(Lds) <= 80 * 1024, "two workgroups a CU");
+};
+
+// (The arguments by value: by reference the same code was 2 % slower at eight channels.)
+template <typename T, typename TF, int ND, bool kByKey, int C>
+__device__ __forceinline__ void strip_gradients(StripArgs b, typename StripForm<T, TF, ND, kByKey, C>::Lds &lds, int block, int blocks)
+{
+    using Form = StripForm<T, TF, ND, kByKey, C>;
+    using Table = typename Form::Table;
     using Cell = Parts4<TF>;
     using Unit4 = typename std::conditional<sizeof(TF) == 2, f16x4, s16x4>::type;
     constexpr int kCellBytes = kByKey ? 4 : 8, kRowBytes = kStrip * kCellBytes;
-    constexpr int kKinds = kByKey ? 1 : 2, kOwn = kOwnTiles<ND>;
-    constexpr bool kPacked = C == 8;
-    constexpr int kSets = kPacked ? 1 : kKinds;        // of features, and of table gradients
-    constexpr int kParts = kByKey && !kPacked ? 2 : 1; // of dx: dk and dv
+    constexpr int kKinds = Form::kKinds, kOwn = Form::kOwn, kSets = Form::kSets, kParts = Form::kParts;
+    constexpr int kTableParts = Form::kTableParts, kKeptPieces = Form::kKeptPieces;
+    constexpr bool kPacked = Form::kPacked;
     // Windows whose keys are one step's in a form of their own: most are at the level of eight channels.  (At sixteen few are,
     // and the second form costs the other one registers.)
     auto one_step = [](int n) { return kPacked && n <= kStripReach; };
     const AttnArgs &a = b.f;
-    // cells [row][column]: dL, by query behind P; then parts of dx (by key: and dv), one a wavefront
-    __shared__ __align__(16) uint32_t cells_s[kTiles<ND> * 16 * kStrip * kKinds];
-    __shared__ __align__(16) float part_s[kParts * kStripWaves * 256];
-    __shared__ float sums_s[kStripWaves][kStrip], grad_s;
-    __shared__ __align__(16) Exact4<TF> features_s[kSets][64];        // q or k, dout of the strip's voxels
-    __shared__ uint32_t marks_s[2 * kTiles<ND>], marked_s, met_s[kPacked ? kMetWords : 1];
-    // Pieces of the table's operands that wait in LDS, as many as leave room for two workgroups a CU (81,864 of 81,920 bytes by
-    // query in fp32).  In registers they would not fit beside the rest, and a spilled operand comes back from memory behind the
-    // pairs of the next strip, which are on their way then: loads return in order.
-    constexpr int kTableParts = sizeof(Table) / 8, kPieces = kTableParts * kOwn;
-    constexpr int kShared = kByKey || kPieces < kOwn + 2 ? kPieces : kOwn + 2, kKeptPieces = kPieces - kShared;
+    auto &cells_s = lds.cells;
+    auto &part_s = lds.part;
+    auto &sums_s = lds.sums;
+    auto &grad_s = lds.grad;
+    auto &features_s = lds.features;
+    auto &marks_s = lds.marks;
+    auto &marked_s = lds.marked;
+    auto &met_s = lds.met;
+    auto &table_s = lds.table;
     struct TableParts { u32x2 part[kTableParts]; };
-    __shared__ u32x2 table_s[kShared][kStripThreads];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int H = a.H, HD = H * C;
     const uint32_t stride = static_cast<uint32_t>(a.row_stride);       // of q, k, v
-    const int h = static_cast<int>(blockIdx.x) % H;
-    const int group = static_cast<int>(blockIdx.x) / H, groups = static_cast<int>(gridDim.x) / H;
+    const int h = block % H, group = block / H, groups = blocks / H;
     const int strips = b.list.total[1];
     if (group >= strips) return;       // its slot is not read
     const uint32_t cells = lds_address(cells_s);
@@ -694,7 +724,7 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     }
     const bool none = __syncthreads_or(incomplete);
     // the workgroup's table gradients: [workgroup][kind][tile][lane][4 rows]
-    float *slot = b.slots + static_cast<int64_t>(blockIdx.x) * (kSets * kTiles<ND> * 256);
+    float *slot = (kByKey ? b.key_slots : b.slots) + static_cast<int64_t>(block) * (kSets * kTiles<ND> * 256);
 #pragma unroll
     for (int kind = 0; kind < kSets; ++kind) {
 #pragma unroll
@@ -710,11 +740,25 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     }
 }
 
+// By query, and behind that by key in the places that are free by then: in a launch each the second waits for the longest
+// workgroup of the first.  A call, forward included, us, before / so: 12,421 voxels x 12 of 16 615 / 606, 3,105 x 24 397 / 389, 49,682 x 6 979 /
+// 968, in fp32 972 / 963 and 1413 / 1397; 199,327 x 6 of 8 1548 / 1531, 60,000 with six axes 490 / 480, with three the same.
+template <typename T, typename TF, int ND, int C>
+__global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(StripArgs b)
+{
+    using Query = typename StripForm<T, TF, ND, false, C>::Lds;
+    using Key = typename StripForm<T, TF, ND, true, C>::Lds;
+    __shared__ __align__(16) char lds[sizeof(Query) > sizeof(Key) ? sizeof(Query) : sizeof(Key)];
+    const int blocks = static_cast<int>(gridDim.x) / 2, block = static_cast<int>(blockIdx.x);
+    if (block < blocks) strip_gradients<T, TF, ND, false, C>(b, *reinterpret_cast<Query *>(lds), block, blocks);
+    else strip_gradients<T, TF, ND, true, C>(b, *reinterpret_cast<Key *>(lds), block - blocks, blocks);
+}
+
 // The workgroups' table gradients, added up in the workgroups' order: a thread per word of a head's slot.
 template <int ND, int C>
-__global__ __launch_bounds__(256) void strip_finish_kernel(StripArgs by_query, StripArgs by_key, int groups)
+__global__ __launch_bounds__(256) void strip_finish_kernel(StripArgs b, int groups)
 {
-    const AttnArgs &a = by_query.f;
+    const AttnArgs &a = b.f;
     constexpr int kWords = kTiles<ND> * 256, kSets = C == 8 ? 1 : 2;
     const int HD = a.H * C, t = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
     const int word = t % kWords, set = t / kWords % (kSets + 1), h = t / kWords / (kSets + 1);       // by query, then by key
@@ -724,15 +768,15 @@ __global__ __launch_bounds__(256) void strip_finish_kernel(StripArgs by_query, S
     if (axis >= ND || r >= axis_rows<ND>(a, axis)) return;
     const int kind = set == kSets ? 2 : C == 8 ? lane % 16 / C : set;                              // dTq, dTv, dTk
     if (kind == 2 && lane % 16 >= C) return;
-    const int strips = by_query.list.total[1], sets = set < kSets ? kSets : 1;
+    const int strips = b.list.total[1], sets = set < kSets ? kSets : 1;
     const int used = min(groups, strips);
-    const float *from = (set < kSets ? by_query.slots + set * kWords : by_key.slots) + static_cast<int64_t>(h) * (sets * kWords) + word;
+    const float *from = (set < kSets ? b.slots + set * kWords : b.key_slots) + static_cast<int64_t>(h) * (sets * kWords) + word;
     const int64_t step = static_cast<int64_t>(a.H) * (sets * kWords);
     // (in 64 bits: a strip at a time, the parts have been rounded four times as often as by tiles of 64)
     double sum = 0.0;
 #pragma unroll 8
     for (int g = 0; g < used; ++g) sum += from[g * step];
-    (kind == 0 ? by_query.dtq : kind == 1 ? by_query.dtv : by_query.dtk)[static_cast<int64_t>(axis_base<ND>(a, axis) + r) * HD + h * C + lane % C] = static_cast<float>(sum);
+    (kind == 0 ? b.dtq : kind == 1 ? b.dtv : b.dtk)[static_cast<int64_t>(axis_base<ND>(a, axis) + r) * HD + h * C + lane % C] = static_cast<float>(sum);
 }
 
 // workgroups per head: two per CU
@@ -755,13 +799,11 @@ int launch_strips(const StripArgs &b0, hipStream_t stream)
         b.upper[n] = std::nextafterf(static_cast<float>(b.f.rows[n]), 0.0f);
     }
     constexpr int kSets = C == 8 ? 1 : 2;
-    StripArgs by_key = b;
-    by_key.slots = b.slots + slot_bytes(b.f.H, ND, kSets) / sizeof(float);
+    b.key_slots = b.slots + slot_bytes(b.f.H, ND, kSets) / sizeof(float);
     const int H = b.f.H, groups = strip_groups(H);
-    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, false, C>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, b);
-    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, true, C>), dim3(static_cast<unsigned>(groups * H)), dim3(kStripThreads), 0, stream, by_key);
+    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, C>), dim3(static_cast<unsigned>(2 * groups * H)), dim3(kStripThreads), 0, stream, b);
     const int64_t words = static_cast<int64_t>(kSets + 1) * kTiles<ND> * 256 * H;
-    hipLaunchKernelGGL((strip_finish_kernel<ND, C>), dim3(static_cast<unsigned>(ceil_div(words, 256))), dim3(256), 0, stream, b, by_key, groups);
+    hipLaunchKernelGGL((strip_finish_kernel<ND, C>), dim3(static_cast<unsigned>(ceil_div(words, 256))), dim3(256), 0, stream, b, groups);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
 }
