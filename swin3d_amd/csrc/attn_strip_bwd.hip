@@ -1,8 +1,8 @@
 // Attention backward at head_dim 16: what is a sum over pairs, from dL and P of every (pair, head) (gfx950).  The mathematics
 // is in attn_bwd.hip, the kernels that leave the pairs in attn_strip_records.hip and attn_tile_bwd.hip.
 //
-// A workgroup takes a strip of up to 16 voxels of windows of one size and all their pairs: as queries (dq, dTq, dTv) in one
-// launch, as keys (dk, dv, dTk) in another.  It adds up the pairs' dL (and P) by table row into histograms over the rows of
+// A workgroup takes a strip of up to 16 voxels of windows of one size and all their pairs: as queries (dq, dTq, dTv) in the
+// first half of the launch, as keys (dk, dv, dTk) in the second.  It adds up the pairs' dL (and P) by table row into histograms over the rows of
 // all axes at once, one column per voxel: integers on a fixed-point image, scaled per voxel by its sum of |dL|, so no order
 // of additions shows in a result.  A histogram H then gives, by matrix products,
 //     dT[row][c] += sum_columns H[row][column] x[column][c]   (x = q, dout, k: the three table gradients)
@@ -19,9 +19,9 @@
 // registers, two workgroups a CU: with four wavefronts and 168 registers, three workgroups, the table gradients and tables of
 // a wavefront did not fit beside the rest, and 300 MB a call went to memory and back for it.  Registers are what is scarce:
 // with fourteen of them spilled inside the loop the launch by query took 153 us, with none 138.
-// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 128 us, by key 125
+// Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 128 us, by key 125 in a launch each
 // (one kernel on 64 x 64 tiles: 523; with a third barrier before the histograms and coordinates asked for behind it, 138 and
-// 133).  head_dim 8, 199,327 voxels in windows of 26, 6 heads, fp16: 543 and 502 us, where the sweeps' own sums and the kernels
+// 133).  head_dim 8, 199,327 voxels in windows of 26, 6 heads, fp16: 543 and 502 us (in one launch 990), where the sweeps' own sums and the kernels
 // of the table gradients took 1510.  What bounds them is VALU issue, 70 % of the time: at head_dim 8 some 300 to 350
 // instructions a wavefront and strip, a third of them the histograms' conversion into operands, 45 the nine rows of a pair.
 #include "attn_strip.h"
