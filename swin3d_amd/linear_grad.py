@@ -47,23 +47,25 @@ def _weight_gradients(dy, x, want_weight, want_bias, dtype=torch.float32):
     return dw, db
 
 
-# torch's library adds up K in order, too, unless it splits it: for few rows (up to 31 at K from 384 to 768), for long K (1280: up to
-# 800 rows, 1536: 340, 2560: 26,000), and where a launch's last tiles would leave most of the chip idle (from 65,536 rows on).
-# The widths of both networks, 20 to 200,000 rows, 270,000 products: up to K = 768, from 32 rows on and below 65,536 at up to 240
-# channels, all of them have the same bits.  Beyond, 1 to 5 in 100 row counts have 10^-5 to 10^-4 of their numbers a rounding apart,
-# of layers that get narrower up to one in ten: those stay with torch.
-_LEAST_ROWS, _MOST_K, _MANY_ROWS = 64, 768, 65536
+# torch's library (hipBLASLt, of torch 2.10.0 for ROCm 7.0) adds up K in order, too, unless it splits it: for few rows or columns, for
+# long K, and where a launch's last tiles would leave most of the chip idle.  Where it does not follows from results alone: of 1.28
+# million products of random widths (N 8 to 2560, K 16 to 768) and 64 to 65,535 rows those inside the line are the same to the bit, and
+# so are 126,000 of both networks' widths; outside of it lie 2,500 with N >= 32, none below 22.9 million numbers of a result, and 7,800
+# with N = 8 to 24.  From 65,536 rows on 1 to 12 in 100 row counts have 10^-5 to 2 x 10^-4 of their numbers a rounding apart (K = 48 to
+# N = 144: 67,301 rows), which moved the gradients of Swin3D-S by 0.3 to 0.6 % there; with torch's product 0.01 %, as two runs.
+_LEAST_ROWS, _MANY_ROWS, _LEAST_N, _MOST_K = 64, 65536, 32, 768
+_WIDE, _MOST_NUMBERS = 512, 20_000_000
 
 
 def has_torchs_bits(m, n, k):
     """A product of m rows of k channels by a weight [n, k] in order is torch's."""
-    return m >= _LEAST_ROWS and k <= _MOST_K and (n >= k or m < _MANY_ROWS)
+    return _LEAST_ROWS <= m < _MANY_ROWS and n >= _LEAST_N and k <= _MOST_K and (n < _WIDE or m * n <= _MOST_NUMBERS)
 
 
 def dense_rows(x, weight, bias):
     """F.linear of fp16 operands in a forward that is trained: on the library's kernel where torch's has the same bits.  us, torch /
-    so: 199,327 rows of 48 to 144 53 / 18, to 192 54 / 19; 49,682 of 96 to 288 27 / 12, of 384 to 96 17 / 13; 12,421 of 192 to 576
-    16 / 9, of 768 to 192 10.2 / 10.3; 811 of 384 to 384 5.3 / 4.6."""
+    so: 49,682 rows of 96 to 288 27 / 12, of 384 to 96 17 / 13; 12,421 of 192 to 576 16 / 9, of 768 to 192 10.2 / 10.3; 811 of 384 to
+    384 5.3 / 4.6."""
     out = linear_rows(x, weight, bias, in_order=True) if x.dim() == 2 and has_torchs_bits(x.shape[0], *weight.shape) else None
     return F.linear(x, weight, bias) if out is None else out
 

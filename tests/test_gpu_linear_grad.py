@@ -101,6 +101,21 @@ def test_forward_of_a_layer_in_training_has_the_bits_of_torch(hip_lib, m, n, k):
         assert torch.equal(dense_rows(x, weight, b), F.linear(x, weight, b))
 
 
+@pytest.mark.parametrize("m,n,k,here", [
+    (64, 144, 48, True), (1563, 32, 768, True), (65535, 144, 48, True), (65535, 504, 192, True), (39062, 512, 320, True), (7812, 2560, 640, True),
+    (63, 144, 48, False), (67301, 144, 48, False), (131074, 48, 48, False), (199327, 192, 48, False), (264, 8, 176, False), (2000, 24, 592, False),
+    (52555, 640, 160, False), (21907, 1536, 384, False), (14881, 2560, 640, False), (1563, 384, 1536, False)])
+def test_forward_of_a_layer_in_training_is_here_where_torchs_bits_are(hip_lib, monkeypatch, m, n, k, here):
+    """The ends of the rule, and sizes beyond it, at most of which torch splits the sums."""
+    from swin3d_amd import linear_grad
+    calls = []
+    monkeypatch.setattr(linear_grad, "linear_rows", lambda *a, f=linear_grad.linear_rows, **how: calls.append(f(*a, **how)) or calls[-1])
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, weight, bias = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k), (n,)))
+    assert torch.equal(dense_rows(x, weight, bias), F.linear(x, weight, bias))
+    assert [c is not None for c in calls] == [True] * here
+
+
 def _rows_and_gelu(x, weight, bias):
     from swin3d_amd import _lib
     y, gelu = (torch.full((x.shape[0], weight.shape[0]), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
