@@ -27,27 +27,30 @@ constexpr int kPieces = kChunk / 8;
 
 // The derivative of x Phi(x): Phi(x) + x phi(x), in fp32.  With Phi(-u) = phi(u) M(u), M the ratio of Mills, that is
 // phi(u) (u - M(u)) with the sign of x, and 1 more for x above 0, u = |x|: u - M(u) by the polynomial of degree 12 that fits
-// phi(u) (u - M(u)) best over [0, 5.8], 4e-9 off.  The error over all
-// fp16 numbers is the rounding of fp32, 9.2e-8 at most and 2.45e-8 in the mean of squares (1.47e-7 and 2.45e-8 with erff and the
-// exponential apart), below -3 a relative 1.4e-4 at most (1.7e-3, since 1 + erf cancels there).  Infinities and NaN as the sum of
+// phi(u) (u - M(u)) best over [0, 5.8], 8.7e-9 off at most, up to 5, where phi is still large enough to hold its relative error, and by
+// a line from there on, where u - M(u) is close to one.  Over all fp16 numbers the error is the rounding of fp32, 9.2e-8 at most
+// (1.47e-7 with erff and the exponential apart).  Where the derivative is small and negative it is a relative 1.4e-4 at most from -3 to
+// -5, 1.0e-3 to -8 and 6.5e-3 to -13 (1.7e-3, 3.3e-2 and 2.1e-2, since 1 + erf cancels there; with the polynomial alone 3e-2 at -5.8, and beyond -6.8
+// the other sign).  Infinities and NaN as the sum of
 // the two terms has them: NaN.  A third of the instructions less: 199,327 rows of 48 to 192, us, 52.6 -> 41.5, 49,682 of 96 to 384
 // 33.4 -> 27.0, 12,421 of 192 to 768 24.2 -> 19.0, with their rows alone 18, 15 and 12.
 __device__ __forceinline__ float gelu_slope(float x)
 {
-    const float u = fminf(fabsf(x), 8.0f), phi = __builtin_amdgcn_exp2f(fmaf(u * u, -0.7213475204f, -1.325748064f));
-    float q = fmaf(-1.467262933e-07f, u, 4.019878816e-06f);
-    q = fmaf(q, u, -4.986505519e-05f);
-    q = fmaf(q, u, 3.754729696e-04f);
-    q = fmaf(q, u, -1.954356674e-03f);
-    q = fmaf(q, u, 7.658625022e-03f);
-    q = fmaf(q, u, -2.421350777e-02f);
-    q = fmaf(q, u, 6.534569710e-02f);
-    q = fmaf(q, u, -1.560686380e-01f);
-    q = fmaf(q, u, 3.331732452e-01f);
-    q = fmaf(q, u, -6.266347766e-01f);
-    q = fmaf(q, u, 1.999998808e+00f);
-    q = fmaf(q, u, -1.253314137e+00f);
-    return fmaf(x, 0.0f, fmaf(__builtin_copysignf(phi, x), q, 0.5f + __builtin_copysignf(0.5f, x)));
+    const float u = fabsf(x), c = fminf(u, 5.0f), phi = __builtin_amdgcn_exp2f(fmaf(u * u, -0.7213475204f, -1.325748064f));
+    float q = fmaf(-1.467262933e-07f, c, 4.019878816e-06f);
+    q = fmaf(q, c, -4.986505519e-05f);
+    q = fmaf(q, c, 3.754729696e-04f);
+    q = fmaf(q, c, -1.954356674e-03f);
+    q = fmaf(q, c, 7.658625022e-03f);
+    q = fmaf(q, c, -2.421350777e-02f);
+    q = fmaf(q, c, 6.534569710e-02f);
+    q = fmaf(q, c, -1.560686380e-01f);
+    q = fmaf(q, c, 3.331732452e-01f);
+    q = fmaf(q, c, -6.266347766e-01f);
+    q = fmaf(q, c, 1.999998808e+00f);
+    q = fmaf(q, c, -1.253314137e+00f);
+    q = fmaf(u - c, 1.025f, q);
+    return fmaf(__builtin_copysignf(phi, x), q, 0.5f + __builtin_copysignf(0.5f, x));
 }
 
 // x Phi(x) of a training forward, as torch has it: by the math library's erff, in this order of operations

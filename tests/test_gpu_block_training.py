@@ -233,3 +233,33 @@ def test_gelus_derivative_at_every_fp16_number(hip_lib):
         want = 0.5 * (1 + torch.erf(x / 2 ** 0.5)) + x * torch.exp(-x * x / 2) / (2 * torch.pi) ** 0.5
         # the rounding to fp16, and of fp32 before it
         assert ((got - want).abs() <= 2 ** -11 * want.abs() + 2 ** -25 + 1.5e-7)[finite].all()
+
+
+def test_gelus_derivative_where_it_is_small(hip_lib):
+    """From -3 down, for a gradient of 2^15, as one scaled against underflow has: relative to itself, to the last number whose product is
+    a normal one in fp16, and no product of the other sign behind that."""
+    hidden, dev = 4096, torch.device("cuda")
+    x = torch.arange(-32768, 32768).to(torch.int16).view(torch.float16)
+    x = x[(x <= -3) & (x >= -12)]
+    stage, feats, run = _stage(100, 16, 1, 5, 2, "XYZ_RGB", 3)
+    block = stage.blocks[-1]
+    block.mlp = encoder.Mlp(16, hidden).to(dev)
+    torch.nn.init.zeros_(block.mlp.fc1.weight)
+    torch.nn.init.zeros_(block.mlp.fc2.weight)
+    block.mlp.fc2.weight.data[0] = 1
+    assert len(x) <= hidden
+    block.mlp.fc1.bias.data.copy_(torch.nn.functional.pad(x.float(), (0, hidden - len(x)), value=-4.0))
+    grad = torch.zeros_like(feats)
+    grad[7, 0] = 2.0 ** 15
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = run(feats)
+    assert any("Branches" in name for name in _nodes(out))
+    got = torch.autograd.grad(out, block.mlp.fc1.bias, grad)[0].double().cpu()[:len(x)] * 2.0 ** -15
+    u = -x.double()
+    phi = torch.exp(-u * u / 2) / (2 * torch.pi) ** 0.5
+    want = -phi * (u - (torch.pi / 2) ** 0.5 * torch.special.erfcx(u / 2 ** 0.5))
+    normal = want.abs() * 2.0 ** 15 >= 2.0 ** -14
+    assert (u[normal].max() > 6) and (got <= 0).all()
+    # the approximation's relative error, and the rounding to fp16
+    share = torch.where(u <= 5, 1.4e-4, 1.0e-3) + 2.0 ** -11 * 1.01
+    assert ((got - want).abs() <= share * want.abs())[normal].all()
