@@ -2,7 +2,7 @@
 // is in attn_bwd.hip, the kernels that leave the pairs in attn_strip_records.hip and attn_tile_bwd.hip.
 //
 // A workgroup takes a strip of up to 16 voxels of windows of one size and all their pairs: as queries (dq, dTq, dTv) in the
-// first half of the launch, as keys (dk, dv, dTk) in the second.  It adds up the pairs' dL (and P) by table row into histograms over the rows of
+// first half of the launch, as keys (dk, dv, dTk) in the second (or in a launch each).  It adds up the pairs' dL (and P) by table row into histograms over the rows of
 // all axes at once, one column per voxel: integers on a fixed-point image, scaled per voxel by its sum of |dL|, so no order
 // of additions shows in a result.  A histogram H then gives, by matrix products,
 //     dT[row][c] += sum_columns H[row][column] x[column][c]   (x = q, dout, k: the three table gradients)
@@ -86,6 +86,9 @@ template <typename V> __device__ __forceinline__ V max16(V v)
     return step(v, std::integral_constant<int, 0x140>{});  // row_mirror
 }
 
+// One launch for the sums by query and by key, or one each (strip_gradients_apart_kernel)
+template <typename TF, int C> constexpr bool kOneLaunch = C == 16 || sizeof(TF) == 2;
+
 // What the products of head_dim 8 leave out, in the strips that have a dL that is not finite beside a P that is: P dout of the voxels whose dout is
 // not finite in some channel, pair by pair.  By key dv of their windows is added up again; by query what they give dTv joins the
 // workgroup's slot.  (It takes its arguments from where the launch put them: what is kept for it through the loop over strips comes
@@ -96,8 +99,9 @@ __device__ __forceinline__ void add_left_out(float *shared, const uint32_t *stri
 {
     constexpr int C = 8;
     const void *at_args = (const void *)__builtin_amdgcn_kernarg_segment_ptr();
-    const int blocks = static_cast<int>(gridDim.x) / 2;
-    int tid = threadIdx.x, block = static_cast<int>(blockIdx.x) - (kByKey ? blocks : 0);
+    constexpr bool kHalf = kOneLaunch<TF, C>;
+    const int blocks = static_cast<int>(gridDim.x) / (kHalf ? 2 : 1);
+    int tid = threadIdx.x, block = static_cast<int>(blockIdx.x) - (kByKey && kHalf ? blocks : 0);
     asm volatile("" : "+s"(at_args), "+v"(tid), "+s"(block));
     const StripArgs &b = *static_cast<const StripArgs *>(at_args);
     const AttnArgs &a = b.f;
@@ -225,9 +229,17 @@ template <typename T, typename TF, int ND, bool kByKey, int C> struct StripForm 
     static_assert(sizeof(Lds) <= 80 * 1024, "two workgroups a CU");
 };
 
+// A member of what two forms share in LDS, or (kApart) an array by itself
+template <bool kApart, typename A> using Own = typename std::conditional<kApart, A, char>::type;
+template <bool kApart, typename L, typename A> __device__ __forceinline__ A &in_lds(Own<kApart, A> &own, L *lds, A L::*member)
+{
+    if constexpr (kApart) return own;
+    else return lds->*member;
+}
+
 // (The arguments by value: by reference the same code was 2 % slower at eight channels.)
-template <typename T, typename TF, int ND, bool kByKey, int C>
-__device__ __forceinline__ void strip_gradients(StripArgs b, typename StripForm<T, TF, ND, kByKey, C>::Lds &lds, int block, int blocks)
+template <typename T, typename TF, int ND, bool kByKey, int C, bool kApart>
+__device__ __forceinline__ void strip_gradients(StripArgs b, typename StripForm<T, TF, ND, kByKey, C>::Lds *lds, int block, int blocks)
 {
     using Form = StripForm<T, TF, ND, kByKey, C>;
     using Table = typename Form::Table;
@@ -241,15 +253,24 @@ __device__ __forceinline__ void strip_gradients(StripArgs b, typename StripForm<
     // and the second form costs the other one registers.)
     auto one_step = [](int n) { return kPacked && n <= kStripReach; };
     const AttnArgs &a = b.f;
-    auto &cells_s = lds.cells;
-    auto &part_s = lds.part;
-    auto &sums_s = lds.sums;
-    auto &grad_s = lds.grad;
-    auto &features_s = lds.features;
-    auto &marks_s = lds.marks;
-    auto &marked_s = lds.marked;
-    auto &met_s = lds.met;
-    auto &table_s = lds.table;
+    __shared__ __align__(16) Own<kApart, typename Form::Cells> own_cells;
+    __shared__ __align__(16) Own<kApart, typename Form::Sums> own_part;
+    __shared__ Own<kApart, typename Form::AbsSums> own_sums;
+    __shared__ Own<kApart, float> own_grad;
+    __shared__ __align__(16) Own<kApart, typename Form::Features> own_features;
+    __shared__ Own<kApart, typename Form::Marks> own_marks;
+    __shared__ Own<kApart, uint32_t> own_marked;
+    __shared__ Own<kApart, typename Form::Met> own_met;
+    __shared__ Own<kApart, typename Form::Pieces> own_table;
+    auto &cells_s = in_lds<kApart>(own_cells, lds, &Form::Lds::cells);
+    auto &part_s = in_lds<kApart>(own_part, lds, &Form::Lds::part);
+    auto &sums_s = in_lds<kApart>(own_sums, lds, &Form::Lds::sums);
+    auto &grad_s = in_lds<kApart>(own_grad, lds, &Form::Lds::grad);
+    auto &features_s = in_lds<kApart>(own_features, lds, &Form::Lds::features);
+    auto &marks_s = in_lds<kApart>(own_marks, lds, &Form::Lds::marks);
+    auto &marked_s = in_lds<kApart>(own_marked, lds, &Form::Lds::marked);
+    auto &met_s = in_lds<kApart>(own_met, lds, &Form::Lds::met);
+    auto &table_s = in_lds<kApart>(own_table, lds, &Form::Lds::table);
     struct TableParts { u32x2 part[kTableParts]; };
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int H = a.H, HD = H * C;
@@ -742,7 +763,7 @@ __device__ __forceinline__ void strip_gradients(StripArgs b, typename StripForm<
 
 // By query, and behind that by key in the places that are free by then: in a launch each the second waits for the longest
 // workgroup of the first.  A call, forward included, us, before / so: 12,421 voxels x 12 of 16 615 / 606, 3,105 x 24 397 / 389, 49,682 x 6 979 /
-// 968, in fp32 972 / 963 and 1413 / 1397; 199,327 x 6 of 8 1548 / 1531, 60,000 with six axes 490 / 480, with three the same.
+// 968, in fp32 972 / 963 and 1418 / 1402; 199,327 x 6 of 8 1548 / 1531, 60,000 with six axes 490 / 480, with three the same.
 template <typename T, typename TF, int ND, int C>
 __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(StripArgs b)
 {
@@ -750,8 +771,18 @@ __global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_kernel(Strip
     using Key = typename StripForm<T, TF, ND, true, C>::Lds;
     __shared__ __align__(16) char lds[sizeof(Query) > sizeof(Key) ? sizeof(Query) : sizeof(Key)];
     const int blocks = static_cast<int>(gridDim.x) / 2, block = static_cast<int>(blockIdx.x);
-    if (block < blocks) strip_gradients<T, TF, ND, false, C>(b, *reinterpret_cast<Query *>(lds), block, blocks);
-    else strip_gradients<T, TF, ND, true, C>(b, *reinterpret_cast<Key *>(lds), block - blocks, blocks);
+    if (block < blocks) strip_gradients<T, TF, ND, false, C, false>(b, reinterpret_cast<Query *>(lds), block, blocks);
+    else strip_gradients<T, TF, ND, true, C, false>(b, reinterpret_cast<Key *>(lds), block - blocks, blocks);
+}
+
+// fp32 at head_dim 8 in a launch each, and what is in LDS as arrays by themselves: as parts of one block the compiler takes more
+// registers than there are (spilled with six axes 11 by one kernel, 7 and 1 by two with a block each, 5 and none so).  A call, forward
+// included, us, by one kernel / so: windows of 60, 100,003 voxels x 6 1810 / 1786, with nine axes 2118 / 2091; of 26, 20,000 and 40,000
+// the same.
+template <typename T, typename TF, int ND, bool kByKey, int C>
+__global__ __launch_bounds__(kStripThreads, 4) void strip_gradients_apart_kernel(StripArgs b)
+{
+    strip_gradients<T, TF, ND, kByKey, C, true>(b, nullptr, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
 }
 
 // The workgroups' table gradients, added up in the workgroups' order: a thread per word of a head's slot.
@@ -801,7 +832,13 @@ int launch_strips(const StripArgs &b0, hipStream_t stream)
     constexpr int kSets = C == 8 ? 1 : 2;
     b.key_slots = b.slots + slot_bytes(b.f.H, ND, kSets) / sizeof(float);
     const int H = b.f.H, groups = strip_groups(H);
-    hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, C>), dim3(static_cast<unsigned>(2 * groups * H)), dim3(kStripThreads), 0, stream, b);
+    const unsigned blocks = static_cast<unsigned>(groups * H);
+    if constexpr (kOneLaunch<TF, C>) {
+        hipLaunchKernelGGL((strip_gradients_kernel<T, TF, ND, C>), dim3(2 * blocks), dim3(kStripThreads), 0, stream, b);
+    } else {
+        hipLaunchKernelGGL((strip_gradients_apart_kernel<T, TF, ND, false, C>), dim3(blocks), dim3(kStripThreads), 0, stream, b);
+        hipLaunchKernelGGL((strip_gradients_apart_kernel<T, TF, ND, true, C>), dim3(blocks), dim3(kStripThreads), 0, stream, b);
+    }
     const int64_t words = static_cast<int64_t>(kSets + 1) * kTiles<ND> * 256 * H;
     hipLaunchKernelGGL((strip_finish_kernel<ND, C>), dim3(static_cast<unsigned>(ceil_div(words, 256))), dim3(256), 0, stream, b, groups);
     S3D_HIP_CHECK(hipGetLastError());
