@@ -349,6 +349,7 @@ class StemConv(nn.Module):
         return self.conv_layers[0].kernel
 
     def forward(self, voxels, neighbours=None):
+        neighbours = conv3x3x3_neighbours(voxels.coords, voxels.stride) if neighbours is None else neighbours
         done = self._at_once(voxels, neighbours)
         if done is not None:
             return voxels.with_feats(done)
@@ -367,7 +368,6 @@ class StemConv(nn.Module):
             return None
         (n, cin), dev = feats.shape, feats.device
         cout = weight.shape[-1]
-        neighbours = conv3x3x3_neighbours(voxels.coords, voxels.stride) if neighbours is None else neighbours
         if not (0 < n < 2 ** 31 - 16 and 0 < cin <= 16 and cout % 16 == 0 and 0 < cout <= 96 and weight.shape == (27, cin, cout)
                 and data_only(neighbours) and neighbours.device == dev and neighbours.dtype == torch.long
                 and neighbours.shape == (n, 27) and neighbours.is_contiguous()):

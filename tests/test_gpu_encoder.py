@@ -333,3 +333,19 @@ def test_stem_at_once(hip_lib, n, cin, cout, dtype, affine):
     bad[n // 3, 1] = n + 5
     with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
         assert stem(voxels, bad).feats[n // 3].isnan().all()
+
+
+@pytest.mark.parametrize("cin,cout,at_once", [(9, 48, True), (17, 48, False), (9, 40, False), (9, 112, False)])
+def test_stem_looks_its_neighbours_up_once(hip_lib, monkeypatch, cin, cout, at_once):
+    """A stem called without them, of widths that the kernel takes and of others."""
+    lookups, layers = [], []
+    monkeypatch.setattr(encoder, "conv3x3x3_neighbours", lambda *a, f=encoder.conv3x3x3_neighbours: lookups.append(f(*a)) or lookups[-1])
+    monkeypatch.setattr(encoder, "sparse_conv3x3x3", lambda *a, f=encoder.sparse_conv3x3x3: layers.append(f(*a)) or layers[-1])
+    coords = torch.from_numpy(synth.make_room((3.0, 2.0, 1.0), 2, 3000, seed=1).coords).cuda()
+    stem = encoder.StemConv(cin, cout).cuda().eval()
+    voxels = encoder.SparseVoxels(coords, torch.randn(coords.shape[0], cin, device="cuda"), 1)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        got = stem(voxels).feats
+    assert len(lookups) == 1 and len(layers) == (not at_once)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        assert torch.equal(got, stem(voxels, lookups[0]).feats)
