@@ -62,11 +62,15 @@ enum class Behind { kNothing, kGelu, kGeluGrad, kGeluBeside };
 __device__ __forceinline__ int placed(int r, int p) { return r * kPieces + (p ^ ((r >> 1) & (kPieces - 1))); }
 
 // Sixteen bytes a lane from `from` to the wavefront's 1024 at `to` in LDS.  The compiler knows nothing of them: who reads them
-// has waited for them (loads and stores end in the order of their issue) and met the other wavefronts at a barrier.
+// has waited for them (loads and stores end in the order of their issue) and met the other wavefronts at a barrier.  (m0 is reserved,
+// of which it warns; named, it is a definition of m0, which the compiler's own uses of it have to respect.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_to_lds(uint32_t to, const void *from)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 // ... all but the kBehind instructions issued last
 template <int kBehind> __device__ __forceinline__ void loads_done() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory"); }
 __device__ __forceinline__ void workgroup_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

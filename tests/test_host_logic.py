@@ -1,4 +1,7 @@
 """Host-side mirror of the reference interface (runs without a GPU)."""
+import pathlib
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -103,3 +106,11 @@ def test_synthetic_room_is_deterministic_and_dense():
     assert np.allclose(np.linalg.norm(a.normal, axis=1), 1.0)
     order = np.lexsort((a.coords[:, 3], a.coords[:, 2], a.coords[:, 1]))
     np.testing.assert_array_equal(order, np.arange(a.coords.shape[0]))          # sorted by (x,y,z)
+
+
+def test_inline_assembly_names_the_m0_that_it_writes():
+    """Otherwise the compiler may keep a value of its own in m0 across the statement."""
+    csrc = pathlib.Path(swin3d_amd.__file__).parent / "csrc"
+    writes = [(f.name, text) for f in sorted(csrc.iterdir()) if f.suffix in (".hip", ".h")
+              for text in re.findall(r"\basm\b[^;]*;", f.read_text()) if re.search(r'"[^"]*\bs_\w+ m0,', text)]
+    assert writes and all('"m0"' in text for _, text in writes), writes
