@@ -249,7 +249,8 @@ int launch(const LinearArgs &a, hipStream_t stream)
     const int tiles_n = (a.N + L::kN - 1) / L::kN;
     const int64_t tiles = ceil_div(a.M, L::kM) * tiles_n;
     if (tiles > (1 << 30)) return fail(S3D_ERR_BAD_SHAPE, "s3d_linear: M = %lld rows", (long long)a.M);
-    auto kernel = a.gelu_at ? linear_kernel<L, Behind::kGeluGrad> : a.gelu ? linear_kernel<L, Behind::kGelu> : linear_kernel<L, Behind::kNothing>;
+    auto kernel = a.gelu ? linear_kernel<L, Behind::kGelu> : linear_kernel<L, Behind::kNothing>;
+    if constexpr (L::kTN < 3) kernel = a.gelu_at ? linear_kernel<L, Behind::kGeluGrad> : kernel;
     if constexpr (L::kTM == 1 && L::kTN == 1) kernel = a.gelu_out ? linear_kernel<L, Behind::kGeluBeside> : kernel;
     // as many workgroups as fit the chip (by LDS), or one a tile
     constexpr int kPerCu = 160 * 1024 / L::kLds < 2 ? 1 : 160 * 1024 / L::kLds < 4 ? 160 * 1024 / L::kLds : 4;
@@ -388,7 +389,7 @@ int launch_linear(const LinearArgs &a, hipStream_t stream)
     // 14.7 / 16.8, 515 21.0 / 18.3, 560 20.6 / 19.5; 1536 -> 384: 354 25.7 / 26.1, 450 28.3 / 35.7, 561 41.8 / 38.9, 642 41.6 / 49.7; with
     // GELU the first is from 448 on).  Over nineteen layers of 96 to 2560 and 96 to 1400 such tiles the choice is 0.8 % behind
     // the best of the three in the mean.  192 columns take all of a wavefront's registers: with GELU only
-    // where the tile is the whole row, with its derivative not at all (63 would spill).
+    // where the tile is the whole row, with its derivative not at all (6 would spill).
     // So, too, with erff's GELU beside the rows, whose fifty instructions a number overlap with other tiles' loads only where
     // several tiles share a SIMD.  us, torch's GELU behind the layer / larger tiles / so: 199,327 rows of 48 to 192 47.0 / 50.9 / 45.0,
     // 49,682 of 96 to 384 30.8 / 34.9 / 26.5, 12,421 of 192 to 768 25.8 / 23.3 / 17.1, 3,105 of 384 to 1536 19.9 / 14.9 / 12.6;
