@@ -40,11 +40,11 @@ def test_half_copies(hip_lib, rows, cols, scaled, offset):
         assert torch.equal(bits(half[second:second + rows * cols]), bits(want.t()))
 
 
-def _stage(voxels, channels, heads, window, mode, axes, seed, extent=(3.0, 3.0, 2.0)):
+def _stage(voxels, channels, heads, window, mode, axes, seed, extent=(3.0, 3.0, 2.0), rows=None):
     dev = torch.device("cuda", 0)
     scene = synth.make_room(extent, 4, voxels, seed=seed)
-    coords = torch.from_numpy(scene.coords).to(dev)
-    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)[:, :4 + (3 if axes == "XYZ_RGB" else 6)]
+    coords = torch.from_numpy(scene.coords).to(dev)[:rows]
+    signals = torch.from_numpy(synth.encoder_inputs(scene)[1].copy()).to(dev)[:rows, :4 + (3 if axes == "XYZ_RGB" else 6)]
     torch.manual_seed(seed)
     stage = encoder.Stage(channels, 2, heads, window, 4, downsample=False, cRSE=axes, fp16_mode=mode).to(dev)
     for name, p in stage.named_parameters():
@@ -107,6 +107,30 @@ def test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads,
     (2999, 640, 40, 1, "nothing"), (4000, 144, 9, 2, "biases")])                # too many tiles for pairs; only some have the same tiles
 def test_layers_that_share_a_launch(hip_lib, monkeypatch, voxels, channels, heads, mode, without):
     test_against_the_layers_nodes(hip_lib, monkeypatch, voxels, channels, heads, 5, mode, "XYZ_RGB_NORM", without)
+
+
+@pytest.mark.parametrize("rows,channels,heads,window,mode", [
+    (63, 48, 6, 5, 2), (64, 48, 6, 5, 2), (811, 384, 24, 7, 1), (12_011, 192, 12, 7, 1), (65535, 48, 6, 5, 2),      # ends of the one call
+    (67301, 48, 6, 5, 2)])                                                                                       # torch splits the sums of q, k, v
+def test_forward_has_the_bits_of_torchs_operations(hip_lib, monkeypatch, rows, channels, heads, window, mode):
+    """Products, norms, GELU and sums by torch, with the same attention between."""
+    from swin3d_amd import swin_train
+    stage, feats, run = _stage(rows + 8000, channels, heads, window, mode, "XYZ_RGB", 9, (8.0, 7.0, 3.0), rows)
+    assert feats.shape[0] == rows
+    calls = []
+    monkeypatch.setattr(swin_train, "_in_one_call", lambda *a, f=swin_train._in_one_call: calls.append(f(*a)) or calls[-1])
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = run(feats)
+    assert [c is not None for c in calls] == [64 <= rows < 65536] * 2
+    monkeypatch.setattr(encoder, "trained_branches", lambda *_: None)
+    monkeypatch.setattr(encoder, "trained_linear", lambda *_, **__: None)
+    monkeypatch.setattr(encoder, "trained_add_norm", lambda *_: None)
+    monkeypatch.setattr(encoder, "add_half", lambda *_: None)
+    with torch.autocast("cuda", dtype=torch.float16):
+        ref = run(feats)
+    names = _nodes(ref)
+    assert any("AddmmBackward" in name for name in names) and not any(part in name for name in names for part in ("Branches", "_Linear", "AddNorm", "AddHalf"))
+    assert torch.equal(out, ref)
 
 
 def test_gradients_of_gradients_and_absent_ones(hip_lib, monkeypatch):
