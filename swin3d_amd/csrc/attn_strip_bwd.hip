@@ -22,7 +22,7 @@
 // Measured, 9 axes, 12,421 voxels in windows of 72, 12 heads, fp32 tables beside fp16 features: by query 128 us, by key 125 in a launch each
 // (one kernel on 64 x 64 tiles: 523; with a third barrier before the histograms and coordinates asked for behind it, 138 and
 // 133).  head_dim 8, 199,327 voxels in windows of 26, 6 heads, fp16: 543 and 502 us (in one launch 990), where the sweeps' own sums and the kernels
-// of the table gradients took 1510.  What bounds them is VALU issue, 70 % of the time: at head_dim 8 some 300 to 350
+// of the table gradients took 1510.  What bounds them is VALU issue, 73 % of the time: at head_dim 8 some 300 to 350
 // instructions a wavefront and strip, a third of them the histograms' conversion into operands, 45 the nine rows of a pair.
 #include "attn_strip.h"
 

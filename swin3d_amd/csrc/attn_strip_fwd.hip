@@ -389,6 +389,7 @@ int launch_fwd(const AttnArgs &a, const StripList &list, hipStream_t stream)
 //     1.12, 0.99 in the mean, at 7200 to 8000, 0.78 to 1.23 at 8000 to 8800, 1.15 to 1.31 beyond (the sweep's time jumps with its
 //     cut into units, and the lines lie where strips lose little anywhere)
 //   windows of 5 to 11 voxels: 0.30 to 0.70 up to 2800, 0.70 to 1.15 at 3000 to 3700, 1.10 to 1.68 at 5500 to 7500
+//   windows of 18 to 24: 0.36 to 0.63 at 4000 to 6000, which the line at 24 still leaves to the sweep; nothing is recorded from 12 to 17
 constexpr int64_t kStripsMost = 6000, kStripsMostNormals = 7200, kStripsMostSmall = 3000, kStripMeanWindowSmall = 24;
 
 bool attn_strip_shape(int64_t N, int64_t W, int H, int nd)

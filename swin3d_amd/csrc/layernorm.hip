@@ -172,6 +172,7 @@ extern "C" __attribute__((visibility("default"))) int s3d_add_layernorm(
 // row's mean moves single fp16 roundings and with them the gradients of a network on a small scan.  Its sums are running means and
 // squared deviations (Welford's recurrence, Chan's rule for two parts): 256 threads a row with four neighbouring numbers each, whose
 // parts meet over a wavefront's lanes, the lower halves taking in the upper ones, and then over the wavefronts, two apart first.
+// That this is torch's order (2.10.0 for ROCm 7.0) rests on results alone: the test compares every bit of rows of these widths.
 // Here a lane holds up to four of those threads' parts, 64 apart, so that all of a row's numbers are loaded at once and none is
 // read again, and rows of up to 64 or 128 channels share a wavefront; threads without numbers are parts of no weight.
 // Bound by memory: 199,327 rows of 48 with a residual 18.3 us, 6.3 TB/s, where a sum, torch's norm (185 us: a workgroup a row) and a

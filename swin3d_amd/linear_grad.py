@@ -2,11 +2,11 @@
 s3d_linear (for the rows) and s3d_linear_grad (for weight and bias).  Tall rows and small weights are what the networks have,
 where a product that does not split the sum over the rows leaves most of the chip idle.
 
-The product of the forward is torch's to the bit, as it is outside of this file (dense_rows has where).  A sum over K in another
-order is no less exact, but it gives another sample of what fp16 activations do to the gradients of a network: on scans of 5,000
-to 40,000 voxels the gradients of Swin3D-S's encoder lie 1 to 5 % from those of an fp32 pass, and products that share K among
-wavefronts in the forward moved them by 0.1 to 1.6 % (single elements by up to a seventh of the largest).  With torch's bits they
-are what they were to the scatter of two runs, 0.05 to 0.1 %."""
+The product of the forward is torch's to the bit, as it is outside of this file (has_torchs_bits has where it is made here).  A sum
+over K in another order is no less exact, but it gives another sample of what fp16 activations do to the gradients of a network: on
+scans of 5,000 to 40,000 voxels the gradients of Swin3D-S's encoder lie 1 to 5 % from those of an fp32 pass, and products that share
+K among wavefronts in the forward moved them by 0.1 to 1.6 % (single elements by up to a seventh of the largest).  With torch's bits
+they are what they were to the scatter of two runs, 0.05 to 0.1 %."""
 import ctypes
 import functools
 

@@ -265,7 +265,7 @@ def _layer_copies(layout, params, half):
 
 
 def _layer_by_layer(call, x, normed, norm_weight, norm_bias, given, params, layout, half, same, index):
-    """The same by a call for each: where torch splits the sums of one of the products (few rows, or many channels)."""
+    """The same by a call for each: where torch splits the sums of one of the products (few or very many rows, or many channels)."""
     n, channels = x.shape
     heads, dim, dev = call.heads, call.dim, x.device
     lib = _lib.lib()
