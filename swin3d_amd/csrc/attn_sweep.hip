@@ -425,6 +425,12 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
     constexpr int kKeys = D == 16 && HP == 1 ? 2 : 1;
     // lazy softmax reference (see the loop): -4 % for fp16; fp32 measured no gain (head_dim 8) or a loss (16)
     constexpr bool kLazy = sizeof(T) == 2;
+    // What hides the round trips of two or three heads in fp16.  The table rows of the next axis are read from LDS before the
+    // products of this one's, and the next key with its signals is asked for once its predecessor's logits stand, in its
+    // registers; the compiler's own order waited for every row right behind its read.  The same sums in the same order.  us
+    // without / so, 9 axes: 149,993 voxels x 10 heads of 16 1104 / 1019, 12,421 x 12 192 / 176, 9,400 x 40 470 / 431, 199,327 x 6 of 8
+    // 207 / 200.  Two rows ahead at head_dim 16 spills 30 registers (1469), and eight wavefronts with room for it are slower (1111).
+    constexpr bool kAhead = sizeof(T) == 2 && HP > 1;
     // 16-byte aligned like the table rows behind it, which are read 16 bytes at a time
     extern __shared__ __align__(16) float smem[];
     __shared__ __align__(16) int group_exit_counter[4];   // [0]: wavefronts of this workgroup that have left their loop
@@ -555,49 +561,84 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
 
         // kKeys streamed keys per iteration: their loads and dependent chains interleave, which hides the
         // LDS and cache round trips a single chain would wait out one after the other
-        int row_next[kKeys];
+        int row_next[kKeys], row_now[kKeys];
+        Slice<T, D> kv[kKeys][HP];
+        float cj[kKeys][ND];
 #pragma unroll
         for (int u = 0; u < kKeys; ++u) row_next[u] = kSorted ? 0 : a.n2n[k0 + min((u << gshift) + grp, n_k - 1)];
+        auto row_at = [&](int row) { return static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint64_t>(a.row_stride); };
+        // the keys of an iteration and their signals
+        auto fetch_keys = [&](int it) {
+#pragma unroll
+            for (int u = 0; u < kKeys; ++u) {
+                const int st = ((it + u) << gshift) + grp;
+                const int st_pos = k0 + min(st, n_k - 1);
+                row_now[u] = kSorted ? st_pos : row_next[u];
+                if (!kSorted) row_next[u] = a.n2n[k0 + min(st + (kKeys << gshift), n_k - 1)];
+#pragma unroll
+                for (int n = 0; n < ND; ++n) cj[u][n] = a.n_coords[static_cast<uint64_t>(static_cast<uint32_t>(st_pos)) * ND + n];
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) kv[u][hh].load(gk + (row_at(row_now[u]) + static_cast<uint32_t>((h + hh) * D)));
+            }
+        };
+        if constexpr (kAhead) fetch_keys(0);
         for (int it = 0; it < max_steps; it += kKeys) {
             // the next unit's ticket is drawn during the last iteration: the atomic's round trip overlaps that
             // work, and a unit is not held back (out of reach of idle wavefronts) for longer than one step
             if (it + kKeys >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
-            Slice<T, D> kv[kKeys][HP], v_in[kKeys][HP];
+            Slice<T, D> v_in[kKeys][HP];
             float logit[kKeys][HP];
             uint32_t off[kKeys][ND];
             bool valid[kKeys];
+            auto load_values = [&](int u) {
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) v_in[u][hh].load(gv + (row_at(row_now[u]) + static_cast<uint32_t>((h + hh) * D)));
+            };
+            if constexpr (!kAhead) fetch_keys(it);
 #pragma unroll
             for (int u = 0; u < kKeys; ++u) {
-                const int st = ((it + u) << gshift) + grp;
-                valid[u] = st < n_k;
-                const int st_pos = k0 + min(st, n_k - 1);
-                const int st_row = kSorted ? st_pos : row_next[u];
-                if (!kSorted) row_next[u] = a.n2n[k0 + min(st + (kKeys << gshift), n_k - 1)];
-#pragma unroll
-                for (int hh = 0; hh < HP; ++hh) {
-                    kv[u][hh].load(gk + static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D);
-                    v_in[u][hh].load(gv + static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D);
-                }
-                float cj[ND];
-#pragma unroll
-                for (int n = 0; n < ND; ++n) cj[n] = a.n_coords[static_cast<int64_t>(st_pos) * ND + n];
+                valid[u] = ((it + u) << gshift) + grp < n_k;
+                if constexpr (!kAhead) load_values(u);
 #pragma unroll
                 for (int n = 0; n < ND; ++n)
-                    off[u][n] = mad_u24(static_cast<uint32_t>(crse_row(ci[n], cj[n], half_rows[n], upper[n])), row_bytes, base_off[n]);
+                    off[u][n] = mad_u24(static_cast<uint32_t>(crse_row(ci[n], cj[u][n], half_rows[n], upper[n])), row_bytes, base_off[n]);
             }
+            if constexpr (kAhead) {
+                // rows of the q-side table and of the k-side table in turn, of all heads, the next ones on their way; the values
+                // of the keys are asked for once the registers of the first rows are free
+                constexpr int kItems = 2 * ND, kAskForValues = 4;
+                Slice<T, D> rows[2][HP];
+                auto read = [&](int i) {
 #pragma unroll
-            for (int u = 0; u < kKeys; ++u) {
+                    for (int hh = 0; hh < HP; ++hh) rows[i % 2][hh].load_lds(off[0][i / 2] + hh * kHeadBytes + (i % 2) * D * sizeof(T));
+                };
+                read(0);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int hh = 0; hh < HP; ++hh) logit[u][hh] = qv[hh].dot(kv[u][hh], 0.0f);
+                for (int hh = 0; hh < HP; ++hh) logit[0][hh] = qv[hh].dot(kv[0][hh], 0.0f);
 #pragma unroll
-                for (int n = 0; n < ND; ++n) {
+                for (int i = 0; i < kItems; ++i) {
+                    if (i == kAskForValues) load_values(0);
+                    if (i + 1 < kItems) read(i + 1);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int hh = 0; hh < HP; ++hh) {
-                        Slice<T, D> tq_r, tk_r;
-                        tq_r.load_lds(off[u][n] + hh * kHeadBytes);
-                        tk_r.load_lds(off[u][n] + hh * kHeadBytes + D * sizeof(T));
-                        if (Slice<T, D>::kChainLogit) logit[u][hh] = kv[u][hh].dot(tk_r, qv[hh].dot(tq_r, logit[u][hh]));
-                        else logit[u][hh] += kv[u][hh].dot(tk_r, qv[hh].dot(tq_r, 0.0f));
+                    for (int hh = 0; hh < HP; ++hh) logit[0][hh] = (i % 2 ? kv[0][hh] : qv[hh]).dot(rows[i % 2][hh], logit[0][hh]);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < kKeys; ++u) {
+#pragma unroll
+                    for (int hh = 0; hh < HP; ++hh) logit[u][hh] = qv[hh].dot(kv[u][hh], 0.0f);
+#pragma unroll
+                    for (int n = 0; n < ND; ++n) {
+#pragma unroll
+                        for (int hh = 0; hh < HP; ++hh) {
+                            Slice<T, D> tq_r, tk_r;
+                            tq_r.load_lds(off[u][n] + hh * kHeadBytes);
+                            tk_r.load_lds(off[u][n] + hh * kHeadBytes + D * sizeof(T));
+                            if (Slice<T, D>::kChainLogit) logit[u][hh] = kv[u][hh].dot(tk_r, qv[hh].dot(tq_r, logit[u][hh]));
+                            else logit[u][hh] += kv[u][hh].dot(tk_r, qv[hh].dot(tq_r, 0.0f));
+                        }
                     }
                 }
             }
@@ -636,6 +677,16 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                 // (and the sums are rescaled) only when the lane's logit exceeds it by more than kSlack, which
                 // after the first keys of a unit is rare, so most steps skip the rescaling of l and the D outputs;
                 // weights stay below e^kSlack.  `top` is the true running maximum.
+                // (the value rows, two of them on their way)
+                constexpr int kRows = HP * ND, kOnWay = 2;
+                Slice<T, D> rows[kOnWay + 1];
+                auto read = [&](int r) { rows[r % (kOnWay + 1)].load_lds(off[0][r % ND] + r / ND * kHeadBytes + 2 * D * sizeof(T)); };
+                if constexpr (kAhead) {
+#pragma unroll
+                    for (int r = 0; r < kOnWay; ++r) read(r);
+                    fetch_keys(it + kKeys);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 float hi[HP];
                 bool moved = false;
 #pragma unroll
@@ -679,6 +730,18 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                             // for the same reason not to.  The reference's half path adds all rows and the value in
                             // half2 (self_attn_aio_fwd.cu:147).
                             constexpr int kGroup = 3;
+                            Slice<T, D> sum_of_rows;
+                            if constexpr (kAhead) {
+#pragma unroll
+                                for (int n = 0; n < ND; ++n) {
+                                    const int r = hh * ND + n;
+                                    if (r + kOnWay < kRows) read(r + kOnWay);
+                                    __builtin_amdgcn_sched_barrier(0);
+                                    if (n % kGroup == 0) sum_of_rows = rows[r % (kOnWay + 1)];
+                                    else sum_of_rows.add(rows[r % (kOnWay + 1)]);
+                                    if (n % kGroup == kGroup - 1 || n == ND - 1) sum_of_rows.fma_to(acc[hh], p);
+                                }
+                            } else
 #pragma unroll
                             for (int n0 = 0; n0 < ND; n0 += kGroup) {
                                 Slice<T, D> tv_sum;
