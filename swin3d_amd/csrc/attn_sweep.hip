@@ -381,6 +381,27 @@ void launch_work_list(const AttnArgs &a, hipStream_t stream, bool strips_too = f
     hipLaunchKernelGGL(sweep_place_kernel, grid, dim3(kListThreads), 0, stream, a);
 }
 
+// Which head group a workgroup serves, for its whole life.  Workgroups go to the XCDs in turn: runs of eight consecutive ones serve
+// one head group, as far as whole sets of (XCDs x head groups) go, so that every XCD serves every head group and the rows of a
+// unit reach one L2; the head groups take the workgroups behind those in turn.  (All in turn, an even number of head groups meets
+// only some of the XCDs: 199,327 voxels x 6 heads of 8 200 -> 215 us.  Without the ones behind, sixteen of 256 CUs had no workgroup
+// at 6, 10, 12 and 20 heads of 16: with them 149,993 x 10 1036 -> 1018 us, 49,682 x 6 278 -> 271, 37,485 x 20 664 -> 651.  At 24
+// and 40 heads, all of whose workgroups came in turn, 9,000 x 24 285 -> 266, 9,400 x 40 443 -> 432.)
+__device__ __forceinline__ int head_group(const AttnArgs &a, int groups)
+{
+    const int block = static_cast<int>(blockIdx.x);
+    return block < a.set_groups ? block / kQueues % groups : (block - a.set_groups) % groups;
+}
+// The grid for `slots` workgroups at a time.  The work list is cut for as many wavefronts as whole sets have, or, where those
+// leave more than a tenth of the slots empty, for all.
+int place_groups(AttnArgs &a, int slots, int groups, int threads)
+{
+    const int set = kQueues * groups, all = slots >= groups ? slots / groups * groups : groups;
+    a.set_groups = slots / set * set;
+    a.target_items = (10 * a.set_groups < 9 * slots ? all : a.set_groups) / groups * (threads / 64);
+    return all;
+}
+
 // Workgroup shapes.  A workgroup holds its heads' table slices once, so what fits a CU is set by registers and LDS:
 //   one head per wavefront: four workgroups of four wavefronts per CU at head_dim 8 (one wavefront of each on every
 //     SIMD), three at head_dim 16, two at head_dim 32 (an fp32 query, key, value and output row are 128 registers);
@@ -444,9 +465,7 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
         for (int n = 0; n < ND; ++n) run += rows[n] = device_rows(a, n, ND, run);
         if (rows_fit_tiles(rows, ND)) return;
     }
-    // workgroups go to the XCDs in turn: consecutive runs of eight serve one head group, so every XCD gets every head
-    // (or, with many head groups, the head groups take the workgroups in turn: see the launch)
-    const int hg = a.spread_groups ? blockIdx.x % (H / HP) : (blockIdx.x / kQueues) % (H / HP);
+    const int hg = head_group(a, H / HP);
     const int h = hg * HP;   // first head of the group
     // table slices of the heads in the I/O type, interleaved per row: [head][q-side | k-side | v-side]
     constexpr int kRowStride = table_row_stride_heads<T, D, HP>();
@@ -862,7 +881,7 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
     if (threadIdx.x == 0) group_exited = 0;
     const int H = a.H;
     const int HD = H * D;
-    const int hg = a.spread_groups ? blockIdx.x % (H / HP) : (blockIdx.x / kQueues) % (H / HP);
+    const int hg = head_group(a, H / HP);
     const int h = hg * HP;
     constexpr int kRowStride = kKeyOwned ? key_row_stride<T, D, HP>() : table_row_stride_heads<T, D, HP>();
     T *tab = reinterpret_cast<T *>(smem);
@@ -1182,22 +1201,11 @@ int launch_sweep_heads(const AttnArgs &a, hipStream_t stream, int what)
     auto kernel = attn_fwd_sweep_kernel<T, D, ND, HP, kSorted>;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
     // A workgroup serves one head group for its whole life: as many workgroups per CU as registers and LDS allow.
-    // They come in whole sets of (XCDs x head groups) - runs of eight consecutive workgroups, one per XCD, serve one
-    // head group, so every XCD serves every head group and the rows of a unit reach one L2 - unless whole sets
-    // would leave more than a tenth of the slots empty (many head groups): then the head groups take the workgroups
-    // in turn and every slot is used, at the price of that locality (the kernel is not bound by memory traffic).
     int per_cu = groups_per_cu<T, D, HP>();
     while (per_cu > 1 && per_cu * lds > 160 * 1024) --per_cu;
-    const int groups = a.H / HP;
-    const int cus = device_cus();
-    const int slots = per_cu * cus;
-    const int set = kQueues * groups;
-    const int whole = (slots / set) * set;
     AttnArgs b = a;
-    b.spread_groups = 10 * whole < 9 * slots;
-    const int grid = b.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
     constexpr int kThreads = group_threads<T, D, HP>();
-    b.target_items = grid / groups * (kThreads / 64);   // wavefronts that serve one head group
+    const int grid = place_groups(b, per_cu * device_cus(), a.H / HP, kThreads);
     b.block_shift = target_shift_for(a.N, a.W, b.target_items);
     if (what & kAttnBuildList) {
         launch_work_list(b, stream, what & kAttnStripList);
@@ -1278,9 +1286,7 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
         int per_cu = 0;
         S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, lds));
         if (per_cu < 1) per_cu = 1;
-        const int slots = per_cu * device_cus(), set = kQueues * groups, whole = (slots / set) * set;
-        b.f.spread_groups = 10 * whole < 9 * slots;
-        grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
+        grid = place_groups(b.f, per_cu * device_cus(), groups, kThreads);
         return static_cast<int>(S3D_OK);
     };
     BwdPairArgs b = b0, by_key = b0;
@@ -1288,7 +1294,6 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
     if (int rc = with_grid(b, reinterpret_cast<const void *>(q_sweep), q_lds, grid)) return rc;
     if (int rc = with_grid(by_key, reinterpret_cast<const void *>(k_sweep), k_lds, key_grid)) return rc;
     // (one work list, cut for the query-owned sweep, which takes longer)
-    b.f.target_items = grid / groups * (kThreads / 64);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
     launch_work_list(b.f, stream);
     S3D_HIP_CHECK(hipGetLastError());
@@ -1310,11 +1315,8 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
     int per_cu = 0;
     S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kernel), kThreads, lds));
     if (per_cu < 1) per_cu = 1;
-    const int groups = a.H / HP, slots = per_cu * device_cus(), set = kQueues * groups, whole = (slots / set) * set;
     BwdPairArgs b = b0;
-    b.f.spread_groups = 10 * whole < 9 * slots;
-    const int grid = b.f.spread_groups ? (slots >= groups ? slots / groups * groups : groups) : whole;
-    b.f.target_items = grid / groups * (kThreads / 64);
+    const int grid = place_groups(b.f, per_cu * device_cus(), a.H / HP, kThreads);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
     launch_work_list(b.f, stream);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
