@@ -393,13 +393,14 @@ __device__ __forceinline__ int head_group(const AttnArgs &a, int groups)
     return block < a.set_groups ? block / kQueues % groups : (block - a.set_groups) % groups;
 }
 // The grid for `slots` workgroups at a time.  The work list is cut for as many wavefronts as whole sets have, or, where those
-// leave more than a tenth of the slots empty, for all.
-int place_groups(AttnArgs &a, int slots, int groups, int threads)
+// leave more than a tenth of the slots empty, for all.  (The key-owned sweep of the backward, whose records' lines bound it, stays
+// with whole sets: 370 us, 386 with workgroups behind them, 199,327 voxels x 6 heads of 8 in fp32.)
+int place_groups(AttnArgs &a, int slots, int groups, int threads, bool whole_sets = false)
 {
     const int set = kQueues * groups, all = slots >= groups ? slots / groups * groups : groups;
     a.set_groups = slots / set * set;
     a.target_items = (10 * a.set_groups < 9 * slots ? all : a.set_groups) / groups * (threads / 64);
-    return all;
+    return whole_sets && 10 * a.set_groups >= 9 * slots ? a.set_groups : all;
 }
 
 // Workgroup shapes.  A workgroup holds its heads' table slices once, so what fits a CU is set by registers and LDS:
@@ -848,8 +849,8 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
 // 6 heads of 8, 9 axes, fp16: 338 + 269 us.  When the key-owned sweep made dL and P again (125 of its 280 instructions a pair)
 // and left them in a second order for the table gradients, 326 + 374, with a store of 12 bytes a (pair, head) for 8.
 template <typename T, int D, int HP> __host__ __device__ constexpr int bwd_pair_threads() { return 256; }
-// wavefronts per SIMD of the sweep that leaves records only
-template <typename T, int HP> __host__ __device__ constexpr int record_waves() { return sizeof(T) == 2 ? (HP == 1 ? 4 : 3) : (HP == 1 ? 3 : 2); }
+// The sweep that leaves records only: one workgroup of twelve wavefronts a CU, three per SIMD.
+constexpr int kRecordThreads = 768, kRecordWaves = 3;
 // elements between rows of Tk in the key-owned sweep's LDS (padded as the other's)
 template <typename T, int D, int HP> __host__ __device__ constexpr int key_row_stride()
 {
@@ -870,10 +871,10 @@ template <typename T, typename TF, int D, int ND, int HP, bool kKeyOwned, bool k
 //     953 + 587; fp32 14266 + 1066, 3564 + 1038, 2526 + 1014; beside fp16 rows 12006 + 738, 2864 + 715, 2538 + 714
 // (in the last two LDS holds one workgroup a CU, with tables of 432 rows; it holds two below 394, with six axes too, which spill
 // nothing).
-__global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? record_waves<T, HP>() : sizeof(T) == 2 ? (D == 8 ? 4 : 3) : (D == 8 ? 3 : 2))) void attn_bwd_pairs_kernel(BwdPairArgs b)
+__global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? kRecordWaves : sizeof(T) == 2 ? (D == 8 ? 4 : 3) : (D == 8 ? 3 : 2))) void attn_bwd_pairs_kernel(BwdPairArgs b)
 {
     const AttnArgs &a = b.f;
-    constexpr int kThreads = bwd_pair_threads<T, D, HP>();
+    constexpr int kThreads = kOnlyRecords ? kRecordThreads : bwd_pair_threads<T, D, HP>();
     constexpr int kSlices = kKeyOwned ? 1 : 3;      // the key-owned sweep needs Tk only
     extern __shared__ __align__(16) float smem[];
     __shared__ __align__(16) int group_exit_counter[4];
@@ -1033,6 +1034,78 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
             records(0, rec_now);
             records(kRecords, rec_ahead);
         }
+        if constexpr (kOnlyRecords) {
+            // As in the forward, the next table rows and the next key are on their way; the same sums in the same order.
+            Slice<TF, D> next_k[HP], next_v[HP];
+            float cj[ND];
+            auto fetch = [&](int it) {
+                const int pos = s0 + min(streamed(it), n_w - 1);
+                const uint64_t at_row = static_cast<uint64_t>(static_cast<uint32_t>(row_next)) * static_cast<uint64_t>(a.row_stride);
+                row_next = a.n2n[s0 + min(streamed(it + 1), n_w - 1)];
+#pragma unroll
+                for (int n = 0; n < ND; ++n) cj[n] = a.n_coords[static_cast<uint64_t>(static_cast<uint32_t>(pos)) * ND + n];
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) {
+                    next_k[hh].load(gk + (at_row + static_cast<uint32_t>((h + hh) * D)));
+                    next_v[hh].load(gv + (at_row + static_cast<uint32_t>((h + hh) * D)));
+                }
+            };
+            fetch(0);
+            for (int it = 0; it < max_steps; ++it) {
+                if (it + 1 >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+                const int st = streamed(it);
+                const bool valid = st < n_w && own_valid && fits;
+                uint32_t off[ND];
+#pragma unroll
+                for (int n = 0; n < ND; ++n) off[n] = mad_u24(static_cast<uint32_t>(crse_row(ci[n], cj[n], half_rows[n], upper[n])), row_bytes, base_off[n]);
+                // rows of the three tables in turn, of all heads
+                constexpr int kItems = 3 * ND, kAskAt = 3;
+                Slice<T, D> rows[2][HP], key[HP];
+                auto read = [&](int i) {
+#pragma unroll
+                    for (int hh = 0; hh < HP; ++hh) rows[i % 2][hh].load_lds(off[i / 3] + hh * kHeadBytes + (i % 3) * D * sizeof(T));
+                };
+                read(0);
+                __builtin_amdgcn_sched_barrier(0);
+                float logit[HP], dp[HP], part[HP];
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) {
+                    key[hh].widen(next_k[hh]);
+                    Slice<T, D> value;
+                    value.widen(next_v[hh]);
+                    logit[hh] = own_x[hh].dot(key[hh], 0.0f);
+                    dp[hh] = own_y[hh].dot(value, 0.0f);
+                }
+#pragma unroll
+                for (int i = 0; i < kItems; ++i) {
+                    if (i + 1 < kItems) read(i + 1);
+                    if (i == kAskAt) fetch(it + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int hh = 0; hh < HP; ++hh) {
+                        const Slice<T, D> &row = rows[i % 2][hh];
+                        constexpr bool kChain = Slice<T, D>::kChainLogit;
+                        if (i % 3 == 0) part[hh] = own_x[hh].dot(row, kChain ? logit[hh] : 0.0f);
+                        else if (i % 3 == 1) part[hh] = key[hh].dot(row, part[hh]), logit[hh] = kChain ? part[hh] : logit[hh] + part[hh];
+                        else if (kChain) dp[hh] = own_y[hh].dot(row, dp[hh]);
+                        else dp[hh] += own_y[hh].dot(row, 0.0f);
+                    }
+                }
+                // (or the compiler moves the products below `valid`, away from their rows)
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) asm volatile("" : "+v"(logit[hh]), "+v"(dp[hh]));
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) {
+                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq; a query
+                    // whose dout has no finite channel has no weights either: all channels of what they make are NaN)
+                    const int64_t head_at = static_cast<int64_t>(h + hh) * b.pairs + pair_base;
+                    const float p = __expf(logit[hh] - own_m[hh]) * own_inv[hh];
+                    const float dl = fabsf(logit[hh]) < INFINITY ? p * (dp[hh] - own_delta[hh]) : __int_as_float(0x7fc00000);
+                    if (valid) b.pd[head_at + static_cast<int64_t>(min(st, n_w - 1)) * n_w + own_in] = make_float2(dl, p + own_none[hh]);
+                }
+            }
+            continue;
+        }
         for (int it = 0; it < max_steps; ++it) {
             if (it + 1 >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
             const int st = streamed(it);
@@ -1108,18 +1181,8 @@ __global__ __launch_bounds__((bwd_pair_threads<T, D, HP>()), (kOnlyRecords ? rec
                         if (Slice<T, D>::kChainLogit) dp = own_y[hh].dot(tv_r, dp);
                         else dp += own_y[hh].dot(tv_r, 0.0f);
                     }
-                    if constexpr (!kOnlyRecords) {
-                        if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
-                        else vec_sum[n / kGroup].add(vec_r);
-                    }
-                }
-                if constexpr (kOnlyRecords) {
-                    // (a logit of minus infinity has no weight, but its dL meets an infinite key or table row in dq; a query
-                    // whose dout has no finite channel has no weights either: all channels of what they make are NaN)
-                    const float p = __expf(logit - own_m[hh]) * own_inv[hh];
-                    const float dl = fabsf(logit) < INFINITY ? p * (dp - own_delta[hh]) : __int_as_float(0x7fc00000);
-                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p + own_none[hh]);
-                    continue;
+                    if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
+                    else vec_sum[n / kGroup].add(vec_r);
                 }
                 float p, dl;
                 if constexpr (kKeyOwned) {
@@ -1282,17 +1345,17 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k_sweep), k_lds)) return rc;
     const int groups = a.H / HP;
     // workgroups: as many as registers and the tables in LDS allow, in whole sets as the forward's
-    auto with_grid = [&](BwdPairArgs &b, const void *kernel, size_t lds, int &grid) {
+    auto with_grid = [&](BwdPairArgs &b, const void *kernel, size_t lds, int &grid, bool whole_sets) {
         int per_cu = 0;
         S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, lds));
         if (per_cu < 1) per_cu = 1;
-        grid = place_groups(b.f, per_cu * device_cus(), groups, kThreads);
+        grid = place_groups(b.f, per_cu * device_cus(), groups, kThreads, whole_sets);
         return static_cast<int>(S3D_OK);
     };
     BwdPairArgs b = b0, by_key = b0;
     int grid = 0, key_grid = 0;
-    if (int rc = with_grid(b, reinterpret_cast<const void *>(q_sweep), q_lds, grid)) return rc;
-    if (int rc = with_grid(by_key, reinterpret_cast<const void *>(k_sweep), k_lds, key_grid)) return rc;
+    if (int rc = with_grid(b, reinterpret_cast<const void *>(q_sweep), q_lds, grid, false)) return rc;
+    if (int rc = with_grid(by_key, reinterpret_cast<const void *>(k_sweep), k_lds, key_grid, true)) return rc;
     // (one work list, cut for the query-owned sweep, which takes longer)
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
     launch_work_list(b.f, stream);
@@ -1310,7 +1373,7 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
     const AttnArgs &a = b0.f;
     const size_t lds = align_up(sizeof(T) * static_cast<size_t>(a.total_rows) * table_row_stride_heads<T, D, HP>(), 16);
     auto kernel = attn_bwd_pairs_kernel<T, TF, D, ND, HP, false, true>;
-    constexpr int kThreads = bwd_pair_threads<T, D, HP>();
+    constexpr int kThreads = kRecordThreads;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
     int per_cu = 0;
     S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kernel), kThreads, lds));
@@ -1324,13 +1387,17 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
     return S3D_OK;
 }
 
-// Records alone, for the strips of attn_strip_bwd.hip (head_dim 8).  Bound by VALU issue, 65 % of the time, 322 instructions a
-// step of two heads.  199,327 voxels in windows of 26, 6 heads, 9 axes: fp16 288 us with pairs of heads, 378 with three heads
-// (38 registers spilled), 347 the query-owned sweep with its dq.  fp32 with 9 axes: 463 with one head, 489 with two (two
-// wavefronts a SIMD); with 6 axes 372 and 339.
+// Records alone, for the strips of attn_strip_bwd.hip (head_dim 8).  Bound by VALU issue, some 320 instructions a step of two
+// heads.  A call, forward included, us: 199,327 voxels in windows of 26, 6 heads, 9 axes, fp16 1475 with pairs of heads, 1465 with
+// three (6 axes, 60,001 voxels, 467 and 469.5); beside fp16 rows 1570, fp32 tables.  As one workgroup of 256 for each wavefront of a
+// SIMD 1482 and 1604, of 384 1551 and 1684; before rows and keys were read ahead, 1520 and 1700.  fp32 with 9 axes: 463 us the
+// sweep with one head, 489 with two (then two wavefronts a SIMD); with 6 axes 372 and 339.
 template <typename T, typename TF, int ND>
 int dispatch_bwd_records(const BwdPairArgs &b, hipStream_t stream)
 {
+    if constexpr (sizeof(T) == 2 && ND == 9) {
+        if (b.f.H % 3 == 0) return launch_bwd_records<T, TF, ND, 3>(b, stream);
+    }
     if constexpr (sizeof(TF) == 2 || ND < 9) {
         if (b.f.H % 2 == 0) return launch_bwd_records<T, TF, ND, 2>(b, stream);
     }

@@ -106,6 +106,8 @@ template <int D> struct Slice<float, D> {
             x[c] = v[0]; x[c + 1] = v[1]; x[c + 2] = v[2]; x[c + 3] = v[3];
         }
     }
+    __device__ __forceinline__ void widen(const Slice &o) { *this = o; }
+    __device__ __forceinline__ void widen(const Slice<__half, D> &o);
     __device__ __forceinline__ float dot(const Slice &o, float acc) const
     {
 #pragma unroll
@@ -165,6 +167,7 @@ template <int D> struct Slice<__half, D> {
 #pragma unroll
         for (int c = 0; c < D; c += 8) *reinterpret_cast<u32x4_t *>(&x[c / 2]) = *(lds_uint4_t *)(addr + 2 * c);
     }
+    __device__ __forceinline__ void widen(const Slice &o) { *this = o; }
     __device__ __forceinline__ float dot(const Slice &o, float acc) const
     {
 #pragma unroll
@@ -218,6 +221,12 @@ template <int D> struct Slice<__half, D> {
     // fp16 I/O: the whole logit is one chain of dot-product accumulations
     static constexpr bool kChainLogit = true;
 };
+
+template <int D> __device__ __forceinline__ void Slice<float, D>::widen(const Slice<__half, D> &o)
+{
+#pragma unroll
+    for (int c = 0; c < D; ++c) x[c] = static_cast<float>(o.x[c / 2][c % 2]);
+}
 
 // Row of the axis table hit by a pair; fp32 arithmetic in the reference's operation order (subtract, add
 // half the row count, clamp, truncate).  The reference clamps to [0, rows] and folds the upper edge onto
