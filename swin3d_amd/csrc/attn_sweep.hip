@@ -409,8 +409,8 @@ int place_groups(AttnArgs &a, int slots, int groups, int threads, bool whole_set
 //   fp16, head_dim 8, two heads: four of four (128 registers without spills; the fourth wavefront per SIMD measured
 //     -2 to -3 %); three heads: one workgroup of twelve wavefronts (168 registers, 45 KB of tables: -4 % against
 //     three workgroups of four; sixteen-wavefront workgroups for the one- and two-head instances measured +-2 %);
-//   fp32, head_dim 8, two heads: two workgroups of eight wavefronts (126 registers, 65 KB of tables each: four
-//     wavefronts per SIMD; one workgroup of twelve measured 17 % slower than one head per wavefront, this -4 %);
+//   fp32, head_dim 8, two heads: one workgroup of twelve wavefronts with the rows read ahead (168 registers; 199,327 voxels x 6 327
+//     -> 299 us, 60,001 x 10 with six axes 165 -> 144; two of eight wavefronts, four per SIMD without, two with, 327 and 330);
 //   fp16, head_dim 16, two heads: one workgroup of twelve wavefronts (75 KB of tables, three wavefronts per SIMD; two
 //     workgroups of six measured 25 % slower than one of twelve);
 //   fp32, head_dim 16: one workgroup of twelve wavefronts as well (75 KB of tables, 160 registers: -19 % against two
@@ -419,13 +419,13 @@ template <typename T, int D, int HP> __host__ __device__ constexpr int group_thr
 {
     return sizeof(T) == 4 && D == 32 ? 512
            : HP == 3 ? 768
-           : HP == 2 && sizeof(T) == 4 && D == 8 ? 512
+           : HP == 2 && sizeof(T) == 4 ? 768
            : (HP == 2 || sizeof(T) == 4) && D == 16 ? 768 : 256;
 }
 template <typename T, int D, int HP> __host__ __device__ constexpr int groups_per_cu()
 {
     return sizeof(T) == 4 && D == 32 ? 1
-           : group_threads<T, D, HP>() == 512 ? 2 : group_threads<T, D, HP>() == 768 ? 1
+           : group_threads<T, D, HP>() == 768 ? 1
            : D > 16 ? 2 : D > 8 ? 3 : 4;
 }
 
@@ -442,17 +442,17 @@ template <typename T, int D, int ND, int HP, bool kSorted>
 __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, HP>())) void attn_fwd_sweep_kernel(AttnArgs a)
 {
     constexpr int kThreads = group_threads<T, D, HP>();
-    // streamed keys per loop iteration: at head_dim 16 with one head two interleaved chains hide the LDS round trips;
-    // with two heads the heads are the two chains
-    constexpr int kKeys = D == 16 && HP == 1 ? 2 : 1;
+    // streamed keys per loop iteration: in fp16 at head_dim 16 with one head two interleaved chains hide the LDS round trips
+    constexpr int kKeys = sizeof(T) == 2 && D == 16 && HP == 1 ? 2 : 1;
     // lazy softmax reference (see the loop): -4 % for fp16; fp32 measured no gain (head_dim 8) or a loss (16)
     constexpr bool kLazy = sizeof(T) == 2;
-    // What hides the round trips of two or three heads in fp16.  The table rows of the next axis are read from LDS before the
+    // What hides the round trips where a lane has one key at a time.  The table rows of the next axis are read from LDS before the
     // products of this one's, and the next key with its signals is asked for once its predecessor's logits stand, in its
-    // registers; the compiler's own order waited for every row right behind its read.  The same sums in the same order.  us
-    // without / so, 9 axes: 149,993 voxels x 10 heads of 16 1104 / 1019, 12,421 x 12 192 / 176, 9,400 x 40 470 / 431, 199,327 x 6 of 8
-    // 207 / 200.  Two rows ahead at head_dim 16 spills 30 registers (1469), and eight wavefronts with room for it are slower (1111).
-    constexpr bool kAhead = sizeof(T) == 2 && HP > 1;
+    // registers; the compiler's own order waited for every row right behind its read.  us without / so, 9 axes, fp16: 149,993
+    // voxels x 10 heads of 16 1104 / 1019, 12,421 x 12 192 / 176, 9,400 x 40 470 / 431, 199,327 x 6 of 8 207 / 200; fp32: 120,001 x
+    // 6 of 16 868 / 798, with six axes 60,001 x 12 785 / 746 (two keys at a time before), 199,327 x 6 of 8 327 / 299, 20,001 x 5 83 / 77.
+    // Two rows ahead at head_dim 16 in fp16 spills 30 registers (1469), and eight wavefronts with room for it are slower (1111).
+    constexpr bool kAhead = D <= 16 && kKeys == 1;
     // 16-byte aligned like the table rows behind it, which are read 16 bytes at a time
     extern __shared__ __align__(16) float smem[];
     __shared__ __align__(16) int group_exit_counter[4];   // [0]: wavefronts of this workgroup that have left their loop
@@ -628,6 +628,7 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                 // of the keys are asked for once the registers of the first rows are free
                 constexpr int kItems = 2 * ND, kAskForValues = 4;
                 Slice<T, D> rows[2][HP];
+                float of_axis[HP];
                 auto read = [&](int i) {
 #pragma unroll
                     for (int hh = 0; hh < HP; ++hh) rows[i % 2][hh].load_lds(off[0][i / 2] + hh * kHeadBytes + (i % 2) * D * sizeof(T));
@@ -642,8 +643,19 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                     if (i + 1 < kItems) read(i + 1);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int hh = 0; hh < HP; ++hh) logit[0][hh] = (i % 2 ? kv[0][hh] : qv[hh]).dot(rows[i % 2][hh], logit[0][hh]);
+                    for (int hh = 0; hh < HP; ++hh) {
+                        const Slice<T, D> &mine = i % 2 ? kv[0][hh] : qv[hh];
+                        if constexpr (Slice<T, D>::kChainLogit) {
+                            logit[0][hh] = mine.dot(rows[i % 2][hh], logit[0][hh]);
+                        } else {
+                            of_axis[hh] = mine.dot(rows[i % 2][hh], i % 2 ? of_axis[hh] : 0.0f);
+                            if (i % 2) logit[0][hh] += of_axis[hh];
+                        }
+                    }
                 }
+                // (or the compiler moves the products below `valid`, away from their rows)
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) asm volatile("" : "+v"(logit[0][hh]));
             } else {
 #pragma unroll
                 for (int u = 0; u < kKeys; ++u) {
@@ -661,6 +673,16 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                         }
                     }
                 }
+            }
+            // (the value rows, two of them on their way)
+            constexpr int kRows = HP * ND, kOnWay = 2;
+            Slice<T, D> rows[kOnWay + 1];
+            auto read = [&](int r) { rows[r % (kOnWay + 1)].load_lds(off[0][r % ND] + r / ND * kHeadBytes + 2 * D * sizeof(T)); };
+            if constexpr (kAhead) {
+#pragma unroll
+                for (int r = 0; r < kOnWay; ++r) read(r);
+                fetch_keys(it + kKeys);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if constexpr (!kLazy) {
                 // online softmax: the running maximum moves with every key that raises it
@@ -682,6 +704,15 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                             const float p = __expf(logit[u][hh] - m_new);
                             l[hh] += p;
                             v_in[u][hh].fma_to(acc[hh], p);
+                            if constexpr (kAhead) {
+#pragma unroll
+                                for (int n = 0; n < ND; ++n) {
+                                    const int r = hh * ND + n;
+                                    if (r + kOnWay < kRows) read(r + kOnWay);
+                                    __builtin_amdgcn_sched_barrier(0);
+                                    rows[r % (kOnWay + 1)].fma_to(acc[hh], p);
+                                }
+                            } else
 #pragma unroll
                             for (int n = 0; n < ND; ++n) {
                                 Slice<T, D> tv_r;
@@ -697,16 +728,6 @@ __global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, H
                 // (and the sums are rescaled) only when the lane's logit exceeds it by more than kSlack, which
                 // after the first keys of a unit is rare, so most steps skip the rescaling of l and the D outputs;
                 // weights stay below e^kSlack.  `top` is the true running maximum.
-                // (the value rows, two of them on their way)
-                constexpr int kRows = HP * ND, kOnWay = 2;
-                Slice<T, D> rows[kOnWay + 1];
-                auto read = [&](int r) { rows[r % (kOnWay + 1)].load_lds(off[0][r % ND] + r / ND * kHeadBytes + 2 * D * sizeof(T)); };
-                if constexpr (kAhead) {
-#pragma unroll
-                    for (int r = 0; r < kOnWay; ++r) read(r);
-                    fetch_keys(it + kKeys);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
                 float hi[HP];
                 bool moved = false;
 #pragma unroll
