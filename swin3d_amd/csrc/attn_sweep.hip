@@ -403,31 +403,16 @@ int place_groups(AttnArgs &a, int slots, int groups, int threads, bool whole_set
     return whole_sets && 10 * a.set_groups >= 9 * slots ? a.set_groups : all;
 }
 
-// Workgroup shapes.  A workgroup holds its heads' table slices once, so what fits a CU is set by registers and LDS:
-//   one head per wavefront: four workgroups of four wavefronts per CU at head_dim 8 (one wavefront of each on every
-//     SIMD), three at head_dim 16, two at head_dim 32 (an fp32 query, key, value and output row are 128 registers);
-//   fp16, head_dim 8, two heads: four of four (128 registers without spills; the fourth wavefront per SIMD measured
-//     -2 to -3 %); three heads: one workgroup of twelve wavefronts (168 registers, 45 KB of tables: -4 % against
-//     three workgroups of four; sixteen-wavefront workgroups for the one- and two-head instances measured +-2 %);
-//   fp32, head_dim 8, two heads: one workgroup of twelve wavefronts with the rows read ahead (168 registers; 199,327 voxels x 6 327
-//     -> 299 us, 60,001 x 10 with six axes 165 -> 144; two of eight wavefronts, four per SIMD without, two with, 327 and 330);
-//   fp16, head_dim 16, two heads: one workgroup of twelve wavefronts (75 KB of tables, three wavefronts per SIMD; two
-//     workgroups of six measured 25 % slower than one of twelve);
-//   fp32, head_dim 16: one workgroup of twelve wavefronts as well (75 KB of tables, 160 registers: -19 % against two
-//     workgroups of four, which is all that LDS held); fp32, head_dim 32: one workgroup of eight (125 KB of tables).
-template <typename T, int D, int HP> __host__ __device__ constexpr int group_threads()
-{
-    return sizeof(T) == 4 && D == 32 ? 512
-           : HP == 3 ? 768
-           : HP == 2 && sizeof(T) == 4 ? 768
-           : (HP == 2 || sizeof(T) == 4) && D == 16 ? 768 : 256;
-}
-template <typename T, int D, int HP> __host__ __device__ constexpr int groups_per_cu()
-{
-    return sizeof(T) == 4 && D == 32 ? 1
-           : group_threads<T, D, HP>() == 768 ? 1
-           : D > 16 ? 2 : D > 8 ? 3 : 4;
-}
+// Workgroup shapes.  A workgroup holds its heads' table slices once: up to head_dim 16 one of twelve wavefronts a CU, three per SIMD
+// with 168 registers (fp16 75 KB of tables for two heads of 16, 45 for three of 8; fp32 65 for two heads of 8, 75 for one of 16).
+// With the rows read ahead three wavefronts hide what four hid, and the tables are staged once: against four workgroups of four
+// wavefronts at head_dim 8 with one and two heads, fp16, 9 axes, us 595,677 voxels x 10 heads 918 / 919, 100,003 x 10 213 / 200, 20,003 x 10
+// 87 / 72, 2,003 x 10 76 / 50, 100,003 x 5 138 / 123, fp32 20,001 x 5 77 / 54; two of eight, three or four per SIMD, 978 and 939 at
+// 595,677; two of eight for pairs of heads in fp32 330 for 299 (199,327 x 6).  Two of six at head_dim 16 25 % slower than one of twelve.
+// head_dim 32 (an fp32 query, key, value and output row are 128 registers): two of four wavefronts in fp16, one of eight in fp32
+// (125 KB of tables).
+template <typename T, int D> __host__ __device__ constexpr int group_threads() { return D <= 16 ? 768 : sizeof(T) == 4 ? 512 : 256; }
+template <typename T, int D> __host__ __device__ constexpr int groups_per_cu() { return D <= 16 || sizeof(T) == 4 ? 1 : 2; }
 
 // elements of T between table rows in LDS when a workgroup holds the slices of HP heads side by side
 template <typename T, int D, int HP> __host__ __device__ constexpr int table_row_stride_heads()
@@ -439,9 +424,9 @@ template <typename T, int D, int HP> __host__ __device__ constexpr int table_row
 // LDS addresses of a pair do not depend on the head, so two or three heads share that part of the work.
 // kSorted: q, k, v and out rows are in window-sorted order already (no n2n).
 template <typename T, int D, int ND, int HP, bool kSorted>
-__global__ __launch_bounds__((group_threads<T, D, HP>()), (groups_per_cu<T, D, HP>())) void attn_fwd_sweep_kernel(AttnArgs a)
+__global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) void attn_fwd_sweep_kernel(AttnArgs a)
 {
-    constexpr int kThreads = group_threads<T, D, HP>();
+    constexpr int kThreads = group_threads<T, D>();
     // streamed keys per loop iteration: in fp16 at head_dim 16 with one head two interleaved chains hide the LDS round trips
     constexpr int kKeys = sizeof(T) == 2 && D == 16 && HP == 1 ? 2 : 1;
     // lazy softmax reference (see the loop): -4 % for fp16; fp32 measured no gain (head_dim 8) or a loss (16)
@@ -1285,10 +1270,10 @@ int launch_sweep_heads(const AttnArgs &a, hipStream_t stream, int what)
     auto kernel = attn_fwd_sweep_kernel<T, D, ND, HP, kSorted>;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds)) return rc;
     // A workgroup serves one head group for its whole life: as many workgroups per CU as registers and LDS allow.
-    int per_cu = groups_per_cu<T, D, HP>();
+    int per_cu = groups_per_cu<T, D>();
     while (per_cu > 1 && per_cu * lds > 160 * 1024) --per_cu;
     AttnArgs b = a;
-    constexpr int kThreads = group_threads<T, D, HP>();
+    constexpr int kThreads = group_threads<T, D>();
     const int grid = place_groups(b, per_cu * device_cus(), a.H / HP, kThreads);
     b.block_shift = target_shift_for(a.N, a.W, b.target_items);
     if (what & kAttnBuildList) {
