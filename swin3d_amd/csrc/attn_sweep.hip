@@ -381,17 +381,66 @@ void launch_work_list(const AttnArgs &a, hipStream_t stream, bool strips_too = f
     hipLaunchKernelGGL(sweep_place_kernel, grid, dim3(kListThreads), 0, stream, a);
 }
 
-// Which head group a workgroup serves, for its whole life.  Workgroups go to the XCDs in turn: runs of eight consecutive ones serve
+// Which head group a workgroup serves, for its whole life, and which of its workgroups it is.  Workgroups go to the XCDs in turn: runs of eight consecutive ones serve
 // one head group, as far as whole sets of (XCDs x head groups) go, so that every XCD serves every head group and the rows of a
 // unit reach one L2; the head groups take the workgroups behind those in turn.  (All in turn, an even number of head groups meets
 // only some of the XCDs: 199,327 voxels x 6 heads of 8 200 -> 215 us.  Without the ones behind, sixteen of 256 CUs had no workgroup
 // at 6, 10, 12 and 20 heads of 16: with them 149,993 x 10 1036 -> 1018 us, 49,682 x 6 278 -> 271, 37,485 x 20 664 -> 651.  At 24
 // and 40 heads, all of whose workgroups came in turn, 9,000 x 24 285 -> 266, 9,400 x 40 443 -> 432.)
-__device__ __forceinline__ int head_group(const AttnArgs &a, int groups)
-{
-    const int block = static_cast<int>(blockIdx.x);
-    return block < a.set_groups ? block / kQueues % groups : (block - a.set_groups) % groups;
-}
+struct GroupPlace {
+    int head_group, nth, of;       // its workgroups are numbered
+    __device__ __forceinline__ GroupPlace(const AttnArgs &a, int groups)
+    {
+        const int block = static_cast<int>(blockIdx.x), behind = block - a.set_groups;
+        head_group = behind < 0 ? block / kQueues % groups : behind % groups;
+        nth = behind < 0 ? block / (kQueues * groups) * kQueues + block % kQueues : (a.set_groups + behind) / groups;
+        of = static_cast<int>(gridDim.x) / groups;
+    }
+};
+// The units of a head group, by queues, of which a wavefront starts on that of its XCD (as a rule: blocks go to the XCDs in turn).
+// In launches of up to two units a wavefront the first one is the wavefront's own: the first four wavefronts of all workgroups
+// come before their next four, so that all CUs get some, long ones and short ones.  By tickets alone the workgroups that had
+// their tables first took more than their share.  us by tickets / so, 9 axes, fp16: 20,001 voxels x 6 heads of 8 70.1 / 55.7,
+// 50,001 x 6 96.3 / 79.8, 2,003 x 10 49.5 / 42.1, 9,001 x 12 of 16 148.4 / 145.2; fp32 20,001 x 6 of 8 83.4 / 68.2.  Where there are more units,
+// tickets leave those of a window to one CU's wavefronts, whose lines they share: 12,421 x 12 of 16 174, all first units given 185.
+// (One wavefront at a time instead of four 54.6 and 183.5 at the first and the last of these; six 70 and 185.)
+template <int kWaves> struct UnitQueues {
+    static constexpr int kSide = kWaves % 4 == 0 ? 4 : 1;
+    int *counters;
+    int of, total, lane, queue, drawn, tried = 0;      // drawn: the ticket, of lane 0
+    __device__ __forceinline__ UnitQueues(int *head_counters, const GroupPlace &p, int units)
+        : counters(head_counters), of(p.of), total(units), lane(static_cast<int>(threadIdx.x & 63)), queue(p.nth % kQueues)
+    {
+        const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+        drawn = (wave / kSide * places(queue) + p.nth / kQueues) * kSide + wave % kSide;
+        if (given(queue) == 0) draw();
+    }
+    __device__ __forceinline__ int places(int q) const { return (of - q + kQueues - 1) / kQueues; }      // workgroups that start on it
+    // how many of a queue's units have a wavefront of their own
+    __device__ __forceinline__ int given(int q) const
+    {
+        const int waves = kWaves * places(q);
+        return total - q <= 2 * kQueues * waves ? waves : 0;
+    }
+    __device__ __forceinline__ void draw()
+    {
+        const int first = given(queue);
+        if (lane == 0) drawn = first + atomicAdd(counters + queue * kCounterStride, 1);
+    }
+    // the unit drawn, or one of the other queues where there is none; -1: all are empty
+    __device__ __forceinline__ int unit()
+    {
+        int u = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
+        while (u >= total && ++tried < kQueues) {
+            queue = (queue + 1) % kQueues;
+            u = given(queue) * kQueues + queue;
+            if (u >= total) continue;
+            draw();
+            u = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
+        }
+        return u < total ? u : -1;
+    }
+};
 // The grid for `slots` workgroups at a time.  The work list is cut for as many wavefronts as whole sets have, or, where those
 // leave more than a tenth of the slots empty, for all.  (The key-owned sweep of the backward, whose records' lines bound it, stays
 // with whole sets: 370 us, 386 with workgroups behind them, 199,327 voxels x 6 heads of 8 in fp32.)
@@ -451,7 +500,8 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
         for (int n = 0; n < ND; ++n) run += rows[n] = device_rows(a, n, ND, run);
         if (rows_fit_tiles(rows, ND)) return;
     }
-    const int hg = head_group(a, H / HP);
+    const GroupPlace place(a, H / HP);
+    const int hg = place.head_group;
     const int h = hg * HP;   // first head of the group
     // table slices of the heads in the I/O type, interleaved per row: [head][q-side | k-side | v-side]
     constexpr int kRowStride = table_row_stride_heads<T, D, HP>();
@@ -509,18 +559,10 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
         }
     }
 
-    int queue = xcd_id() % kQueues;
-    int tried = 0;       // queues found empty so far
-    int drawn = 0;       // ticket of the next unit
-    if (lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+    UnitQueues<kThreads / 64> queues(counters, place, total_units);
     for (;;) {
-        int unit = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
-        while (unit >= total_units && ++tried < kQueues) {
-            queue = (queue + 1) % kQueues;
-            if (lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
-            unit = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
-        }
-        if (unit >= total_units) break;
+        const int unit = queues.unit();
+        if (unit < 0) break;
         // The unit: 64 >> gshift queries (consecutive in the sorted numbering of their class), each on 2^gshift
         // adjacent lanes that take alternate keys.  The queries lie in at most 64 consecutive entries from the
         // unit's first one; each lane reads one entry and finds its own (the last entry of the class that starts at
@@ -590,7 +632,7 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
         for (int it = 0; it < max_steps; it += kKeys) {
             // the next unit's ticket is drawn during the last iteration: the atomic's round trip overlaps that
             // work, and a unit is not held back (out of reach of idle wavefronts) for longer than one step
-            if (it + kKeys >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+            if (it + kKeys >= max_steps) queues.draw();
             Slice<T, D> v_in[kKeys][HP];
             float logit[kKeys][HP];
             uint32_t off[kKeys][ND];
@@ -888,7 +930,8 @@ __global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T
     if (threadIdx.x == 0) group_exited = 0;
     const int H = a.H;
     const int HD = H * D;
-    const int hg = head_group(a, H / HP);
+    const GroupPlace place(a, H / HP);
+    const int hg = place.head_group;
     const int h = hg * HP;
     constexpr int kRowStride = kKeyOwned ? key_row_stride<T, D, HP>() : table_row_stride_heads<T, D, HP>();
     T *tab = reinterpret_cast<T *>(smem);
@@ -936,18 +979,10 @@ __global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T
         upper[n] = crse_upper(a.rows[n]);
         base_off[n] = __builtin_amdgcn_readfirstlane(tab_addr + a.base[n] * kRowBytes);
     }
-    int queue = xcd_id() % kQueues;
-    int tried = 0;
-    int drawn = 0;
-    if (lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+    UnitQueues<kThreads / 64> queues(counters, place, total_units);
     for (;;) {
-        int unit = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
-        while (unit >= total_units && ++tried < kQueues) {
-            queue = (queue + 1) % kQueues;
-            if (lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
-            unit = __builtin_amdgcn_readfirstlane(drawn) * kQueues + queue;
-        }
-        if (unit >= total_units) break;
+        const int unit = queues.unit();
+        if (unit < 0) break;
         // the unit, as in the forward sweep: 64 >> gshift owned voxels, each on 2^gshift adjacent lanes that take
         // alternate elements of the streamed side
         const int4 info = unit_info[unit];
@@ -1058,7 +1093,7 @@ __global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T
             };
             fetch(0);
             for (int it = 0; it < max_steps; ++it) {
-                if (it + 1 >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+                if (it + 1 >= max_steps) queues.draw();
                 const int st = streamed(it);
                 const bool valid = st < n_w && own_valid && fits;
                 uint32_t off[ND];
@@ -1113,7 +1148,7 @@ __global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T
             continue;
         }
         for (int it = 0; it < max_steps; ++it) {
-            if (it + 1 >= max_steps && lane == 0) drawn = atomicAdd(counters + queue * kCounterStride, 1);
+            if (it + 1 >= max_steps) queues.draw();
             const int st = streamed(it);
             const bool valid = st < n_w && (!kKeyOwned || it < run) && own_valid && fits;
             const int st_in = min(st, n_w - 1);
