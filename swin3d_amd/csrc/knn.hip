@@ -510,8 +510,8 @@ __device__ __forceinline__ float dist2_unfused(float sx, float sy, float sz, flo
 template <int CTRL> __device__ __forceinline__ uint64_t dpp(uint64_t x)
 {
     const int lo = static_cast<int>(x), hi = static_cast<int>(x >> 32);
-    return (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false))) << 32) |
-           static_cast<uint32_t>(__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+    return (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true))) << 32) |
+           static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
 }
 template <int MASK> __device__ __forceinline__ uint64_t lane_xor(uint64_t x)
 {
@@ -526,11 +526,23 @@ template <int MASK> __device__ __forceinline__ uint64_t lane_xor(uint64_t x)
     else return __shfl_xor(x, MASK);
 }
 
-// the smaller of two lanes' values to the lane without HIGH in its number
+// Candidates are ordered as doubles, whose order the words' is: positive and finite (a distance is no NaN, see the kernel; that of a
+// source at the query is a denormal number, which the instruction keeps).  One instruction in place of a comparison and two choices.
+__device__ __forceinline__ uint64_t least(uint64_t a, uint64_t b)
+{
+    uint64_t r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// the smaller of two lanes' values to the lane without HIGH in its number, the larger one to the other: that one takes the least of
+// the negated values
 template <int MASK, int HIGH> __device__ __forceinline__ void exchange(uint64_t &x, int t)
 {
-    const uint64_t other = lane_xor<MASK>(x);
-    x = (other < x) != ((t & HIGH) != 0) ? other : x;
+    static_assert((MASK & HIGH) != 0, "one lane of the two");
+    const uint64_t sign = (t & HIGH) != 0 ? uint64_t(1) << 63 : 0, own = x ^ sign, other = lane_xor<MASK>(own);
+    uint64_t r;
+    asm("v_min_f64 %0, %1, -%2" : "=v"(r) : "v"(own), "v"(other));
+    x = r ^ sign;
 }
 // ascending order of a bitonic sequence over SIZE lanes, and of any sequence (bitonic sort whose first step of a size
 // compares mirrored lanes, so that every run is ascending)
@@ -553,9 +565,9 @@ template <int SIZE> __device__ __forceinline__ void order(uint64_t &x, int t)
 // One query per group of G lanes (G = 4, 8, 16 or 64 >= K).  The group keeps its G best candidates as one sorted list, a
 // candidate per lane: a word of (squared distance, source row), whose order is the result's.  The sources of a run of
 // cells are read G at a time (the next ones while these are worked on), sorted across the lanes and merged: every step
-// is a DPP move and a compare on all lanes, no candidate waits for another.  At K = 16, 199,327 sources, a query for every
-// cell of two voxels: 34 us, and 43 us with each run of cells read by itself, most of a group's lanes idle in its last step;
-// 73 us with candidates inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
+// is a DPP move and a minimum on all lanes, no candidate waits for another.  At K = 16, 199,327 sources, a query for every
+// cell of two voxels: 30 us (33 with a 64-bit comparison and two choices a step, and moves with a copy of their target ahead), and with
+// those 43 us with each run of cells read by itself, most of a group's lanes idle in its last step; 73 us with candidates inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
 //
 // A walk starts with the cube of 3 x 3 x 3 cells: the query's own cell alone never proves its K best.
 // Groups of sixteen for up to eight neighbours, too, where there are few queries: a group then looks up the nine rows of cells
@@ -623,14 +635,14 @@ __global__ __launch_bounds__(kThreads) void knn_query_kernel(
                 const float4 c = p;
                 const bool have = s + t < total;
                 if (s + G < total) p = source(s + G + t);
-                uint64_t found = (static_cast<uint64_t>(__float_as_uint(dist2_unfused(c.x, c.y, c.z, qx, qy, qz))) << 32) |
-                                 __float_as_uint(c.w);
-                found = have ? found : kNone;
+                const float d = dist2_unfused(c.x, c.y, c.z, qx, qy, qz);
+                uint64_t found = (static_cast<uint64_t>(__float_as_uint(d)) << 32) | __float_as_uint(c.w);
+                found = have && d == d ? found : kNone;      // (what is not a number is behind all that is)
                 // (a group of sixteen skips sources that are all behind the last that can count)
                 if (G == 16 && !__any(found < dpp<0x150 + KMAX - 1>(best))) continue;
                 order<G>(found, t);
                 found = lane_xor<G - 1>(found);
-                best = found < best ? found : best;
+                best = least(found, best);
                 order_bitonic<G>(best, t);
             }
         };

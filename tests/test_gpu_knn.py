@@ -177,3 +177,22 @@ def test_max_pool_over_neighbours_matches_gather_and_max(hip_lib, dtype, channel
     if feat.dtype == torch.float16:
         from swin3d_amd.sparse_dl.knn.knn import _max_pool
         assert torch.equal(_max_pool(idx, feat, torch.float32), ref.float())
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 8, 16, 33, 64])
+def test_order_of_the_smallest_distances_and_of_none(oracle_lib, hip_lib, k):
+    """Sources on the query, whose words of (distance, row) are the smallest there are, distances below the least normal number,
+    sources at infinite distance, and queries that are not numbers, of any payload: those have no neighbours."""
+    rng = np.random.default_rng(k)
+    src = np.concatenate([np.zeros((70, 3)), 1e-20 * rng.random((40, 3)), 1e20 * rng.random((40, 3)), rng.random((200, 3))]).astype(np.float32)
+    src = src[rng.permutation(src.shape[0])]
+    qry = np.concatenate([np.zeros((3, 3)), rng.random((60, 3)), np.full((4, 3), 1e-20)]).astype(np.float32)
+    one = lambda n: np.array([n], np.int32)
+    _compare(oracle_lib, k, src, qry, one(src.shape[0]), one(qry.shape[0]))
+    nans = np.array([0x7fffffff, 0xffffffff, 0x7fc00000, 0x7ff00001], np.uint32).view(np.float32)
+    bad = np.repeat(nans[:, None], 3, 1)
+    near = rng.random((200, 3)).astype(np.float32)
+    idx, d2 = _run(k, near, np.concatenate([bad, near[:5]]), one(200), one(9))
+    assert (idx[:4] == -1).all() and (d2[:4] == 2147483648.0).all()
+    ridx, rd2 = oracle_lib.knn(k, near, near[:5], one(200), one(5))
+    assert np.array_equal(idx[4:], ridx) and np.array_equal(d2[4:], rd2)
