@@ -100,8 +100,9 @@ struct BwdPairArgs {
     int64_t pairs;               // capacity of pd per head; windows beyond it are skipped
 };
 int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream);
-// dL and P alone (head_dim 8), with dout_i . o_i made from b.out in place of b.delta
-int launch_attn_bwd_records(const BwdPairArgs &b, int dtype, hipStream_t stream);
+// dL and P alone (head_dim 8), with dout_i . o_i made from b.out in place of b.delta, and the lists of the strips that read them
+namespace tile { struct StripSetup; }
+int launch_attn_bwd_records(const BwdPairArgs &b, const tile::StripSetup &strips, int dtype, hipStream_t stream);
 
 // The backward on tiles or strips (attn_tile_bwd.hip, attn_strip_records.hip): head_dim 16, tables that fit a stage, the pair count known.  Of the
 // arguments it takes the shape, inputs and dq, dk, dv; its own workspace holds records, slots, unit and strip list.

@@ -359,5 +359,56 @@ int launch_strip_records(const RecordsCall &c, void *room, int dtype, hipStream_
 size_t strip_slots_bytes(int H, int nd);
 int launch_strip_gradients(const StripArgs &b, int dtype, hipStream_t stream);
 
+// ---- head_dim 8: what the strips need beside the records of the pair sweep, whose launches of lists make it (attn_sweep.hip) ----
+struct StripSetup {
+    StripArgs b;
+    int64_t *pos_base;          // [N]: at a window's first sorted position, the pairs of the windows before it
+};
+
+// The strip list (workgroup 0) and, for fp32 tables beside fp16 features, the scale of a head's operands of Tq and Tk.
+template <bool kScales>
+__device__ __forceinline__ void strip_setup(const StripArgs &b, int block)
+{
+    const AttnArgs &a = b.f;
+    if (block == 0) {
+        build_list(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(b.list.total), nullptr,
+                   const_cast<int2 *>(b.list.entries), const_cast<int4 *>(b.list.strips));
+        return;
+    }
+    const int job = block - 1, kind = job % 2, h = job / 2;
+    float scale = 1.0f;
+    if constexpr (kScales) {
+        const float *table = static_cast<const float *>(kind == 0 ? a.table_q : a.table_k) + h * a.D;
+        __shared__ int top_s;
+        if (threadIdx.x == 0) top_s = 0;
+        __syncthreads();
+        float top = 0.0f;
+        for (int t = threadIdx.x; t < a.total_rows * a.D; t += kListThreads) {
+            const float x = table[static_cast<int64_t>(t / a.D) * (a.H * a.D) + t % a.D];
+            top = fmaxf(top, finite(x) ? fabsf(x) : 0.0f);
+        }
+        atomicMax(&top_s, __float_as_int(top));
+        __syncthreads();
+        scale = power2(min(100, 14 - exponent_of(__int_as_float(top_s))));
+    }
+    if (threadIdx.x == 0) const_cast<float *>(b.scales)[h * 3 + kind] = 1.0f / scale;
+}
+
+// column t of the strips
+__device__ __forceinline__ void strip_column(const StripSetup &s, int t)
+{
+    const StripArgs &b = s.b;
+    const int u = t / kStrip, c = t % kStrip;
+    if (u >= b.list.total[1]) return;
+    const int4 strip = b.list.strips[u];
+    const int col = strip.z + min(c, strip.w - 1), n = strip.y;
+    const int2 entry = b.list.entries[strip.x + col / n];
+    const int pos = entry.x + col % n, row = b.f.n2n ? b.f.n2n[pos] : pos;
+    const bool fits = static_cast<int64_t>(entry.y) + static_cast<int64_t>(n) * n <= b.pairs;
+    const_cast<int4 *>(b.columns)[t] = make_int4(pos, row, entry.x, fits ? entry.y : -1);
+    const_cast<int32_t *>(b.column_rows)[t] = row;
+    if (pos == entry.x) s.pos_base[pos] = entry.y;
+}
+
 }  // namespace tile
 }  // namespace s3d

@@ -845,56 +845,6 @@ int launch_strips(const StripArgs &b0, hipStream_t stream)
     return S3D_OK;
 }
 
-// ---- head_dim 8: what the strips need beside the records of the pair sweep --------------------------------------------
-struct StripSetup {
-    StripArgs b;
-    int64_t *pos_base;          // [N]: at a window's first sorted position, the pairs of the windows before it
-};
-
-// The strip list (workgroup 0) and, for fp32 tables beside fp16 features, the scale of a head's operands of Tq and Tk.
-template <bool kScales>
-__global__ __launch_bounds__(kListThreads) void strip_setup_kernel(StripArgs b)
-{
-    const AttnArgs &a = b.f;
-    if (blockIdx.x == 0) {
-        build_list(a.w_sizes, a.w2n, static_cast<int>(a.W), const_cast<int32_t *>(b.list.total), nullptr,
-                   const_cast<int2 *>(b.list.entries), const_cast<int4 *>(b.list.strips));
-        return;
-    }
-    const int job = static_cast<int>(blockIdx.x) - 1, kind = job % 2, h = job / 2;
-    float scale = 1.0f;
-    if constexpr (kScales) {
-        const float *table = static_cast<const float *>(kind == 0 ? a.table_q : a.table_k) + h * a.D;
-        __shared__ int top_s;
-        if (threadIdx.x == 0) top_s = 0;
-        __syncthreads();
-        float top = 0.0f;
-        for (int t = threadIdx.x; t < a.total_rows * a.D; t += kListThreads) {
-            const float x = table[static_cast<int64_t>(t / a.D) * (a.H * a.D) + t % a.D];
-            top = fmaxf(top, finite(x) ? fabsf(x) : 0.0f);
-        }
-        atomicMax(&top_s, __float_as_int(top));
-        __syncthreads();
-        scale = power2(min(100, 14 - exponent_of(__int_as_float(top_s))));
-    }
-    if (threadIdx.x == 0) const_cast<float *>(b.scales)[h * 3 + kind] = 1.0f / scale;
-}
-
-__global__ __launch_bounds__(256) void strip_columns_kernel(StripSetup s)
-{
-    const StripArgs &b = s.b;
-    const int t = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x), u = t / kStrip, c = t % kStrip;
-    if (u >= b.list.total[1]) return;
-    const int4 strip = b.list.strips[u];
-    const int col = strip.z + min(c, strip.w - 1), n = strip.y;
-    const int2 entry = b.list.entries[strip.x + col / n];
-    const int pos = entry.x + col % n, row = b.f.n2n ? b.f.n2n[pos] : pos;
-    const bool fits = static_cast<int64_t>(entry.y) + static_cast<int64_t>(n) * n <= b.pairs;
-    const_cast<int4 *>(b.columns)[t] = make_int4(pos, row, entry.x, fits ? entry.y : -1);
-    const_cast<int32_t *>(b.column_rows)[t] = row;
-    if (pos == entry.x) s.pos_base[pos] = entry.y;
-}
-
 }  // namespace
 
 size_t strip_slots_bytes(int H, int nd) { return slot_bytes(H, nd, 2) + slot_bytes(H, nd, 1); }
@@ -963,13 +913,7 @@ int launch_attn_strip8(const BwdPairArgs &p, float *dtq, float *dtk, float *dtv,
     g.grad_stride = static_cast<uint32_t>(p.grad_stride);
     g.dtq = dtq; g.dtk = dtk; g.dtv = dtv;
     s.pos_base = const_cast<int64_t *>(p.pos_base);
-    const dim3 jobs(static_cast<unsigned>(1 + 2 * a.H));
-    if (dtype == S3D_DTYPE_F32_F16_ROWS) hipLaunchKernelGGL(strip_setup_kernel<true>, jobs, dim3(kListThreads), 0, stream, g);
-    else hipLaunchKernelGGL(strip_setup_kernel<false>, jobs, dim3(kListThreads), 0, stream, g);
-    const int64_t columns = static_cast<int64_t>(list_max_strips(a.N)) * kStrip;
-    hipLaunchKernelGGL(strip_columns_kernel, dim3(static_cast<unsigned>(ceil_div(columns, 256))), dim3(256), 0, stream, s);
-    S3D_HIP_CHECK(hipGetLastError());
-    if (int rc = launch_attn_bwd_records(p, dtype, stream)) return rc;
+    if (int rc = launch_attn_bwd_records(p, s, dtype, stream)) return rc;
     return launch_strip_gradients(g, dtype, stream);
 }
 

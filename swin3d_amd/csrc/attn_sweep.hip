@@ -19,8 +19,10 @@
 //   L(i,j)     = sum_c q_i[c] k_j[c] + q_i[c] Tq(i,j)[c] + k_j[c] Tk(i,j)[c]
 //   out_i[c]   = sum_j softmax_j(L(i,j)) (v_j[c] + Tv(i,j)[c])
 #include "attn_kernels.h"
+#include "attn_strip.h"
 #include "sweep_common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -379,6 +381,43 @@ void launch_work_list(const AttnArgs &a, hipStream_t stream, bool strips_too = f
     const dim3 grid(static_cast<unsigned>(want > kListGroups ? kListGroups : want));
     hipLaunchKernelGGL(sweep_count_kernel, grid, dim3(kListThreads), 0, stream, a);
     hipLaunchKernelGGL(sweep_place_kernel, grid, dim3(kListThreads), 0, stream, a);
+}
+
+// The work list of a records sweep beside the lists of the strips that read the records (head_dim 8): the strips' list is one
+// workgroup's for 30 us where windows are many, and the sweep's, two short launches, is made meanwhile.  A call, forward included, us, with
+// launches of their own / so: 199,327 voxels x 6 fp16 1466 / 1457, fp32 beside fp16 rows 1564 / 1555, 60,001 x 10 with six axes 754 / 746.
+template <bool kScales>
+__global__ __launch_bounds__(tile::kListThreads) void records_lists_kernel(tile::StripArgs strips, AttnArgs a, int jobs)
+{
+    const int block = static_cast<int>(blockIdx.x) - jobs, groups = static_cast<int>(gridDim.x) - jobs;
+    if (block < 0) {
+        tile::strip_setup<kScales>(strips, block + jobs);
+        return;
+    }
+    if (threadIdx.x >= kListThreads) return;
+    count_windows(a, block, groups);
+    if (a.W > kFewWindows) return;
+    __threadfence();
+    __syncthreads();
+    place_windows(a, 0, 1);
+}
+__global__ __launch_bounds__(kListThreads) void records_places_kernel(tile::StripSetup strips, AttnArgs a, int groups)
+{
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < groups) place_windows(a, block, groups);
+    else tile::strip_column(strips, (block - groups) * kListThreads + static_cast<int>(threadIdx.x));
+}
+int launch_records_lists(const tile::StripSetup &strips, const AttnArgs &a, bool scales, hipStream_t stream)
+{
+    const int groups = a.W <= kFewWindows ? 1 : static_cast<int>(std::min<int64_t>(ceil_div(a.W, kListThreads), kListGroups));
+    const int jobs = 1 + 2 * a.H, places = a.W <= kFewWindows ? 0 : groups;
+    hipLaunchKernelGGL(scales ? records_lists_kernel<true> : records_lists_kernel<false>, dim3(static_cast<unsigned>(jobs + groups)),
+                       dim3(tile::kListThreads), 0, stream, strips.b, a, jobs);
+    const int64_t columns = static_cast<int64_t>(tile::list_max_strips(a.N)) * tile::kStrip;
+    hipLaunchKernelGGL(records_places_kernel, dim3(static_cast<unsigned>(places + ceil_div(columns, kListThreads))), dim3(kListThreads), 0, stream,
+                       strips, a, places);
+    S3D_HIP_CHECK(hipGetLastError());
+    return S3D_OK;
 }
 
 // Which head group a workgroup serves, for its whole life, and which of its workgroups it is.  Workgroups go to the XCDs in turn: runs of eight consecutive ones serve
@@ -1408,7 +1447,7 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
 }
 
 template <typename T, typename TF, int ND, int HP>
-int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
+int launch_bwd_records(const BwdPairArgs &b0, const tile::StripSetup &strips, hipStream_t stream)
 {
     constexpr int D = 8;
     const AttnArgs &a = b0.f;
@@ -1422,7 +1461,7 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
     BwdPairArgs b = b0;
     const int grid = place_groups(b.f, per_cu * device_cus(), a.H / HP, kThreads);
     b.f.block_shift = target_shift_for(a.N, a.W, b.f.target_items);
-    launch_work_list(b.f, stream);
+    if (int rc = launch_records_lists(strips, b.f, sizeof(T) != sizeof(TF), stream)) return rc;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, stream, b);
     S3D_HIP_CHECK(hipGetLastError());
     return S3D_OK;
@@ -1434,15 +1473,15 @@ int launch_bwd_records(const BwdPairArgs &b0, hipStream_t stream)
 // SIMD 1482 and 1604, of 384 1551 and 1684; before rows and keys were read ahead, 1520 and 1700.  fp32 with 9 axes: 463 us the
 // sweep with one head, 489 with two (then two wavefronts a SIMD); with 6 axes 372 and 339.
 template <typename T, typename TF, int ND>
-int dispatch_bwd_records(const BwdPairArgs &b, hipStream_t stream)
+int dispatch_bwd_records(const BwdPairArgs &b, const tile::StripSetup &strips, hipStream_t stream)
 {
     if constexpr (sizeof(T) == 2 && ND == 9) {
-        if (b.f.H % 3 == 0) return launch_bwd_records<T, TF, ND, 3>(b, stream);
+        if (b.f.H % 3 == 0) return launch_bwd_records<T, TF, ND, 3>(b, strips, stream);
     }
     if constexpr (sizeof(TF) == 2 || ND < 9) {
-        if (b.f.H % 2 == 0) return launch_bwd_records<T, TF, ND, 2>(b, stream);
+        if (b.f.H % 2 == 0) return launch_bwd_records<T, TF, ND, 2>(b, strips, stream);
     }
-    return launch_bwd_records<T, TF, ND, 1>(b, stream);
+    return launch_bwd_records<T, TF, ND, 1>(b, strips, stream);
 }
 
 template <typename T, typename TF>
@@ -1468,13 +1507,13 @@ int launch_attn_bwd_pairs(const BwdPairArgs &b, int dtype, hipStream_t stream)
     }
 }
 
-int launch_attn_bwd_records(const BwdPairArgs &b, int dtype, hipStream_t stream)
+int launch_attn_bwd_records(const BwdPairArgs &b, const tile::StripSetup &strips, int dtype, hipStream_t stream)
 {
 #define S3D_CASE(NN)                                                                                       \
     if (b.f.D == 8 && b.f.nd == NN)                                                                        \
-        return dtype == S3D_DTYPE_F32   ? dispatch_bwd_records<float, float, NN>(b, stream)                \
-               : dtype == S3D_DTYPE_F16 ? dispatch_bwd_records<__half, __half, NN>(b, stream)              \
-                                        : dispatch_bwd_records<float, __half, NN>(b, stream);
+        return dtype == S3D_DTYPE_F32   ? dispatch_bwd_records<float, float, NN>(b, strips, stream)                \
+               : dtype == S3D_DTYPE_F16 ? dispatch_bwd_records<__half, __half, NN>(b, strips, stream)              \
+                                        : dispatch_bwd_records<float, __half, NN>(b, strips, stream);
     S3D_CASE(3) S3D_CASE(6) S3D_CASE(9)
 #undef S3D_CASE
     return fail(S3D_ERR_UNSUPPORTED, "s3d_attn_bwd: head_dim %d, %d axes in the records sweep", b.f.D, b.f.nd);
