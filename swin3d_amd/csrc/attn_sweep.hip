@@ -1349,6 +1349,17 @@ int launch_sweep_heads(const AttnArgs &a, hipStream_t stream, int what)
     AttnArgs b = a;
     constexpr int kThreads = group_threads<T, D>();
     const int grid = place_groups(b, per_cu * device_cus(), a.H / HP, kThreads);
+    if constexpr (D == 8 && HP < 3) {
+        // The list is cut as for sixteen wavefronts a CU: chains of additions no longer than four workgroups of four (in fp32 two of eight)
+        // had them.  Cut for twelve, 60,001 voxels x 10 heads in fp32 were 2.55e-7 from 64 bits for 2.51e-7, in 145.1 us for 146.7; fp16
+        // 100,003 x 10 196.5 for 200.5, 595,677 x 10 879 for 884.
+        constexpr int kWaves = sizeof(T) == 4 && HP == 2 ? 8 : 4;
+        int held = 16 / kWaves;
+        while (held > 1 && held * lds > 160 * 1024) --held;
+        AttnArgs cut = a;
+        place_groups(cut, held * device_cus(), a.H / HP, 64 * kWaves);
+        b.target_items = cut.target_items;
+    }
     b.block_shift = target_shift_for(a.N, a.W, b.target_items);
     if (what & kAttnBuildList) {
         launch_work_list(b, stream, what & kAttnStripList);
