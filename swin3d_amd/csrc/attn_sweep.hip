@@ -639,7 +639,9 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
             qv[hh].load(gq + static_cast<int64_t>(own_row) * a.row_stride + (h + hh) * D);
 #pragma unroll
             for (int c = 0; c < D; ++c) acc[hh][c] = 0.0f;
-            m[hh] = top[hh] = -INFINITY;
+            // (the lowest finite number: a key whose logit is minus infinity has no weight, also where a lane sees it first)
+            m[hh] = -3.4028234663852886e38f;
+            top[hh] = -INFINITY;
             l[hh] = 0.0f;
         }
 #pragma unroll
@@ -761,7 +763,7 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
                             logit[u][hh] = valid[u] ? logit[u][hh] : -INFINITY;
                             m_new = fmaxf(m_new, logit[u][hh]);
                         }
-                        const float scale = __expf(m[hh] - m_new);   // exp(-inf) = 0 on the first key
+                        const float scale = __expf(m[hh] - m_new);   // 0 on the first key
                         l[hh] *= scale;
 #pragma unroll
                         for (int c = 0; c < D; ++c) acc[hh][c] *= scale;
@@ -812,7 +814,7 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
 #pragma unroll
                     for (int hh = 0; hh < HP; ++hh) {
                         const float m_new = fmaxf(m[hh], hi[hh]);
-                        const float scale = __expf(m[hh] - m_new);   // exp(-inf) = 0 on the first key
+                        const float scale = __expf(m[hh] - m_new);   // 0 on the first key
                         l[hh] *= scale;
 #pragma unroll
                         for (int c = 0; c < D; ++c) acc[hh][c] *= scale;
@@ -866,8 +868,11 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
                 }
             }
         }
-        // from the reference exponent to the true maximum (lanes that saw no key: both are -inf, nothing to scale)
-        if constexpr (kLazy) {
+        // from the reference exponent to the true maximum (lanes that saw no key with a weight: that is -inf, nothing to scale)
+        if constexpr (!kLazy) {
+#pragma unroll
+            for (int hh = 0; hh < HP; ++hh) m[hh] = l[hh] == 0.0f ? -INFINITY : m[hh];
+        } else {
 #pragma unroll
             for (int hh = 0; hh < HP; ++hh) {
                 const float scale = top[hh] == -INFINITY ? 1.0f : __expf(m[hh] - top[hh]);

@@ -599,3 +599,36 @@ def test_planned_forward_reuses_one_work_list(oracle_lib, hip_lib):
         attn_coff.REUSE_PLANS = True
     torch.cuda.synchronize()
     assert torch.equal(c, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("heads,dim", [(2, 8), (3, 8), (5, 8), (2, 16), (3, 16), (2, 32)])
+def test_sweep_where_the_first_keys_have_no_weight(oracle_lib, hip_lib, dtype, heads, dim):
+    """Keys masked by a channel of minus infinity in front of a window's others: they leave the result and the softmax's maximum
+    and sum to the others, and a query all of whose keys are masked has none."""
+    from gpu_helpers import assert_attn_close, run_attention
+    from test_gpu_attn_tile import _windows_case
+    sizes = [1, 2, 9, 9, 20, 20, 64, 65, 150, 150, 200]
+    case = _windows_case(oracle_lib, sizes, "XYZ_RGB", heads, seed=13, dim=dim)
+    if dtype == torch.float16:
+        to_half_and_back(case)
+    case.tk[:] = np.abs(case.tk) + 0.01
+    case.q[:, 0, 3] = np.abs(case.q[:, 0, 3]) + 0.1
+    w_sizes, w2n, n2n = (case.index[x] for x in ("w_sizes", "w2n", "n2n"))
+    none = np.zeros(case.N, bool)
+    for w, masked in zip(np.argsort(w_sizes, kind="stable"), (1, 1, 1, 9, 2, 19, 1, 3, 1, 9, 100)):
+        rows = n2n[w2n[w]:w2n[w] + w_sizes[w]]
+        case.k[rows[:masked], 0, 3] = -np.inf
+        none[rows] = masked == rows.size
+    if dtype == torch.float16:
+        to_half_and_back(case)
+    got, gmax, gsum = run_attention(case, dtype, return_stats=True)
+    ref, rmax, rsum, _ = oracle_lib.attn_fwd(*case.oracle_args(), return_stats=True)
+    assert np.isnan(got[none, 0]).all() and np.isnan(ref[none, 0]).all()
+    got[none, 0] = ref[none, 0] = 0
+    assert_attn_close(got, ref, dtype)
+    # logits of up to some tens, off by their roundings
+    some = np.isfinite(rmax)
+    assert (np.isfinite(gmax) == some).all()
+    assert np.abs(gmax - rmax)[some].max() <= (1e-5 if dtype == torch.float32 else 1e-2) * max(1.0, np.abs(rmax[some]).max())
+    assert (np.abs(gsum - rsum)[some] <= (1e-4 if dtype == torch.float32 else 2e-2) * rsum[some]).all()
