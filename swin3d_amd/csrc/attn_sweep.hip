@@ -526,6 +526,12 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
     // 6 of 16 868 / 798, with six axes 60,001 x 12 785 / 746 (two keys at a time before), 199,327 x 6 of 8 327 / 299, 20,001 x 5 83 / 77.
     // Two rows ahead at head_dim 16 in fp16 spills 30 registers (1469), and eight wavefronts with room for it are slower (1111).
     constexpr bool kAhead = D <= 16 && kKeys == 1;
+    // fp32, head_dim 16: a pair's value and its rows of the value table are added before they are weighted, so that the output's sums are
+    // rounded once a key.  One key at a time moves the softmax's reference more often than two did, at 1.0004 times their error against
+    // 64 bits (31 of 33 shapes, voxels 3,001 to 120,001, 3 to 9 axes); summed first it is 0.69 to 0.87 of it, 2.77e-7 -> 2.03e-7 at
+    // 60,001 x 6 with 9 axes, in the same time: 120,001 x 6 in windows of 26 367 / 362 us, of 57 796 / 790 (two keys at a time 404 and 898).
+    constexpr bool kSumFirst = sizeof(T) == 4 && D == 16;
+    static_assert(!kSumFirst || kAhead, "in the loop that reads ahead");
     // 16-byte aligned like the table rows behind it, which are read 16 bytes at a time
     extern __shared__ __align__(16) float smem[];
     __shared__ __align__(16) int group_exit_counter[4];   // [0]: wavefronts of this workgroup that have left their loop
@@ -771,15 +777,17 @@ __global__ __launch_bounds__((group_threads<T, D>()), (groups_per_cu<T, D>())) v
                         for (int u = 0; u < kKeys; ++u) {
                             const float p = __expf(logit[u][hh] - m_new);
                             l[hh] += p;
-                            v_in[u][hh].fma_to(acc[hh], p);
+                            if constexpr (!kSumFirst) v_in[u][hh].fma_to(acc[hh], p);
                             if constexpr (kAhead) {
 #pragma unroll
                                 for (int n = 0; n < ND; ++n) {
                                     const int r = hh * ND + n;
                                     if (r + kOnWay < kRows) read(r + kOnWay);
                                     __builtin_amdgcn_sched_barrier(0);
-                                    rows[r % (kOnWay + 1)].fma_to(acc[hh], p);
+                                    if constexpr (kSumFirst) v_in[u][hh].add(rows[r % (kOnWay + 1)]);
+                                    else rows[r % (kOnWay + 1)].fma_to(acc[hh], p);
                                 }
+                                if constexpr (kSumFirst) v_in[u][hh].fma_to(acc[hh], p);
                             } else
 #pragma unroll
                             for (int n = 0; n < ND; ++n) {

@@ -632,3 +632,21 @@ def test_sweep_where_the_first_keys_have_no_weight(oracle_lib, hip_lib, dtype, h
     assert (np.isfinite(gmax) == some).all()
     assert np.abs(gmax - rmax)[some].max() <= (1e-5 if dtype == torch.float32 else 1e-2) * max(1.0, np.abs(rmax[some]).max())
     assert (np.abs(gsum - rsum)[some] <= (1e-4 if dtype == torch.float32 else 2e-2) * rsum[some]).all()
+
+
+@pytest.mark.parametrize("cRSE", ["XYZ", "XYZ_RGB", "XYZ_RGB_NORM"])
+@pytest.mark.parametrize("heads", [1, 2])
+def test_fp32_sweep_adds_a_pairs_rows_before_the_outputs_sums(oracle_lib, hip_lib, cRSE, heads):
+    """Equal weights of 64 keys, a first value of 2^24 and table rows of 3/4, 3/4 and 1/2 on three axes: a row alone is below half a
+    unit of the sum, the three together are one unit.  Only the first key's own rows may be lost, two in the sum."""
+    from gpu_helpers import run_attention
+    from test_gpu_attn_tile import _windows_case
+    case = _windows_case(oracle_lib, [64] * 12, cRSE, heads, seed=5)
+    for x in (case.q, case.k, case.v, case.tq, case.tk, case.tv):
+        x[:] = 0
+    for axis, value in zip(case.axis_tables(case.tv), (0.75, 0.75, 0.5)):
+        axis[:] = value
+    case.v[case.index["n2n"][case.index["w2n"]]] = 2.0 ** 24
+    got, _, gsum = run_attention(case, torch.float32, return_stats=True)
+    assert (gsum == 64).all()
+    assert np.abs(64 * got - (2.0 ** 24 + 2 * 64)).max() <= 2
