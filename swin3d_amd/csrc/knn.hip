@@ -539,6 +539,14 @@ __device__ __forceinline__ uint64_t least(uint64_t a, uint64_t b)
 template <int MASK, int HIGH> __device__ __forceinline__ void exchange(uint64_t &x, int t)
 {
     static_assert((MASK & HIGH) != 0, "one lane of the two");
+    if constexpr (MASK > 15) {
+        // (a move through LDS, where the comparison is shorter than a change of sign on either side of it: 33 neighbours in one launch,
+        // queries a voxel, 595,677 voxels 984 us, 1029 with the minimum, 946 with the minimum within rows of sixteen lanes only; 64
+        // neighbours 1296, 1297 and 1204, 199,327 voxels 538, 524 and 490)
+        const uint64_t other = lane_xor<MASK>(x);
+        x = (other < x) != ((t & HIGH) != 0) ? other : x;
+        return;
+    }
     const uint64_t sign = (t & HIGH) != 0 ? uint64_t(1) << 63 : 0, own = x ^ sign, other = lane_xor<MASK>(own);
     uint64_t r;
     asm("v_min_f64 %0, %1, -%2" : "=v"(r) : "v"(own), "v"(other));
@@ -566,8 +574,9 @@ template <int SIZE> __device__ __forceinline__ void order(uint64_t &x, int t)
 // candidate per lane: a word of (squared distance, source row), whose order is the result's.  The sources of a run of
 // cells are read G at a time (the next ones while these are worked on), sorted across the lanes and merged: every step
 // is a DPP move and a minimum on all lanes, no candidate waits for another.  At K = 16, 199,327 sources, a query for every
-// cell of two voxels: 30 us (33 with a 64-bit comparison and two choices a step, and moves with a copy of their target ahead), and with
-// those 43 us with each run of cells read by itself, most of a group's lanes idle in its last step; 73 us with candidates inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
+// cell of two voxels: 30 us (33 with a 64-bit comparison and two choices a step, and moves with a copy of their target ahead), and
+// with those 43 us with each run of cells read by itself, most of a group's lanes idle in its last step; 73 us with candidates
+// inserted one by one.  Bound by VALU issue (65 % of the time), most of it the sorting steps.
 //
 // A walk starts with the cube of 3 x 3 x 3 cells: the query's own cell alone never proves its K best.
 // Groups of sixteen for up to eight neighbours, too, where there are few queries: a group then looks up the nine rows of cells
