@@ -1197,132 +1197,131 @@ __global__ __launch_bounds__((kOnlyRecords ? kRecordThreads : bwd_pair_threads<T
                     if (valid) b.pd[head_at + static_cast<int64_t>(min(st, n_w - 1)) * n_w + own_in] = make_float2(dl, p + own_none[hh]);
                 }
             }
-            continue;
-        }
-        for (int it = 0; it < max_steps; ++it) {
-            if (it + 1 >= max_steps) queues.draw();
-            const int st = streamed(it);
-            const bool valid = st < n_w && (!kKeyOwned || it < run) && own_valid && fits;
-            const int st_in = min(st, n_w - 1);
-            const int st_pos = s0 + st_in;
-            const int st_row = row_next;
-            row_next = a.n2n[s0 + min(streamed(it + 1), n_w - 1)];
-            Slice<T, D> st_x[HP], st_y[HP];   // k_j, v_j  or  q_i, dout_i
-#pragma unroll
-            for (int hh = 0; hh < HP; ++hh) {
-                const int64_t at_row = static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D;
-                const int64_t at_grad = static_cast<int64_t>(st_row) * HD + (h + hh) * D;
-                if constexpr (kKeyOwned) {
-                    st_x[hh].load(gq + at_row);
-                    st_y[hh].load(ggo + at_grad);
-                } else {
-                    st_x[hh].load(gk + at_row);
-                    st_y[hh].load(gv + at_row);
-                }
-            }
-            float2 rec[HP];
-            if constexpr (kKeyOwned) {
+        } else {
+            for (int it = 0; it < max_steps; ++it) {
+                if (it + 1 >= max_steps) queues.draw();
+                const int st = streamed(it);
+                const bool valid = st < n_w && (!kKeyOwned || it < run) && own_valid && fits;
+                const int st_in = min(st, n_w - 1);
+                const int st_pos = s0 + st_in;
+                const int st_row = row_next;
+                row_next = a.n2n[s0 + min(streamed(it + 1), n_w - 1)];
+                Slice<T, D> st_x[HP], st_y[HP];   // k_j, v_j  or  q_i, dout_i
 #pragma unroll
                 for (int hh = 0; hh < HP; ++hh) {
-                    rec[hh] = rec_now[hh][0];
-#pragma unroll
-                    for (int e = 0; e + 1 < kRecords; ++e) rec_now[hh][e] = rec_now[hh][e + 1];
+                    const int64_t at_row = static_cast<int64_t>(st_row) * a.row_stride + (h + hh) * D;
+                    const int64_t at_grad = static_cast<int64_t>(st_row) * HD + (h + hh) * D;
+                    if constexpr (kKeyOwned) {
+                        st_x[hh].load(gq + at_row);
+                        st_y[hh].load(ggo + at_grad);
+                    } else {
+                        st_x[hh].load(gk + at_row);
+                        st_y[hh].load(gv + at_row);
+                    }
                 }
-                if (it % kRecords == kRecords - 1) {
+                float2 rec[HP];
+                if constexpr (kKeyOwned) {
 #pragma unroll
-                    for (int hh = 0; hh < HP; ++hh)
+                    for (int hh = 0; hh < HP; ++hh) {
+                        rec[hh] = rec_now[hh][0];
 #pragma unroll
-                        for (int e = 0; e < kRecords; ++e) rec_now[hh][e] = rec_ahead[hh][e];
-                    records(it + 1 + kRecords, rec_ahead);
+                        for (int e = 0; e + 1 < kRecords; ++e) rec_now[hh][e] = rec_now[hh][e + 1];
+                    }
+                    if (it % kRecords == kRecords - 1) {
+#pragma unroll
+                        for (int hh = 0; hh < HP; ++hh)
+#pragma unroll
+                            for (int e = 0; e < kRecords; ++e) rec_now[hh][e] = rec_ahead[hh][e];
+                        records(it + 1 + kRecords, rec_ahead);
+                    }
                 }
-            }
-            uint32_t off[ND];
-            {
-                float cj[ND];
+                uint32_t off[ND];
+                {
+                    float cj[ND];
 #pragma unroll
-                for (int n = 0; n < ND; ++n) cj[n] = a.n_coords[static_cast<int64_t>(st_pos) * ND + n];
+                    for (int n = 0; n < ND; ++n) cj[n] = a.n_coords[static_cast<int64_t>(st_pos) * ND + n];
 #pragma unroll
-                for (int n = 0; n < ND; ++n) {
-                    // row_n(i, j): the query's coordinate first
-                    const float c_i = kKeyOwned ? cj[n] : ci[n], c_j = kKeyOwned ? ci[n] : cj[n];
-                    off[n] = mad_u24(static_cast<uint32_t>(crse_row(c_i, c_j, half_rows[n], upper[n])), row_bytes, base_off[n]);
+                    for (int n = 0; n < ND; ++n) {
+                        // row_n(i, j): the query's coordinate first
+                        const float c_i = kKeyOwned ? cj[n] : ci[n], c_j = kKeyOwned ? ci[n] : cj[n];
+                        off[n] = mad_u24(static_cast<uint32_t>(crse_row(c_i, c_j, half_rows[n], upper[n])), row_bytes, base_off[n]);
+                    }
+                }
+#pragma unroll
+                for (int hh = 0; hh < HP; ++hh) {
+                    const int64_t head_at = static_cast<int64_t>(h + hh) * b.pairs + pair_base;
+                    float logit = 0.0f, dp = 0.0f;
+                    if constexpr (!kKeyOwned) {
+                        logit = own_x[hh].dot(st_x[hh], 0.0f);
+                        dp = own_y[hh].dot(st_y[hh], 0.0f);
+                    }
+                    // sums of three rows of the table that enters the owned gradient as a vector (packed fp16 adds for
+                    // fp16 I/O, as the forward adds its value-table rows)
+                    // (fp32: one sum of all rows - plain adds, no packing to gain, and two sums fewer to hold)
+                    constexpr int kGroup = sizeof(T) == 4 ? ND : 3;
+                    Slice<T, D> vec_sum[(ND + kGroup - 1) / kGroup];
+#pragma unroll
+                    for (int n = 0; n < ND; ++n) {
+                        Slice<T, D> vec_r;       // Tk, or Tq
+                        vec_r.load_lds(off[n] + hh * kHeadBytes);
+                        if constexpr (!kKeyOwned) {
+                            Slice<T, D> tk_r, tv_r;
+                            tk_r.load_lds(off[n] + hh * kHeadBytes + D * sizeof(T));
+                            tv_r.load_lds(off[n] + hh * kHeadBytes + 2 * D * sizeof(T));
+                            if (Slice<T, D>::kChainLogit) logit = st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, logit));
+                            else logit += st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, 0.0f));
+                            if (Slice<T, D>::kChainLogit) dp = own_y[hh].dot(tv_r, dp);
+                            else dp += own_y[hh].dot(tv_r, 0.0f);
+                        }
+                        if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
+                        else vec_sum[n / kGroup].add(vec_r);
+                    }
+                    float p, dl;
+                    if constexpr (kKeyOwned) {
+                        p = valid ? rec[hh].y : 0.0f;
+                        dl = valid ? rec[hh].x : 0.0f;
+                    } else {
+                        p = valid ? __expf(logit - own_m[hh]) * own_inv[hh] : 0.0f;
+                        dl = p * (dp - own_delta[hh]);
+                    }
+                    // dq_i += dL (k_j + Tq)   or   dk_j += dL (q_i + Tk)
+                    st_x[hh].fma_to(res_x[hh], dl);
+#pragma unroll
+                    for (int g = 0; g < (ND + kGroup - 1) / kGroup; ++g) vec_sum[g].fma_to(res_x[hh], dl);
+                    if constexpr (kKeyOwned) st_y[hh].fma_to(res_y[hh], p);     // dv_j += P dout_i
+                    if constexpr (!kKeyOwned) {
+                        if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
+                    }
                 }
             }
 #pragma unroll
             for (int hh = 0; hh < HP; ++hh) {
-                const int64_t head_at = static_cast<int64_t>(h + hh) * b.pairs + pair_base;
-                float logit = 0.0f, dp = 0.0f;
-                if constexpr (!kKeyOwned) {
-                    logit = own_x[hh].dot(st_x[hh], 0.0f);
-                    dp = own_y[hh].dot(st_y[hh], 0.0f);
-                }
-                // sums of three rows of the table that enters the owned gradient as a vector (packed fp16 adds for
-                // fp16 I/O, as the forward adds its value-table rows)
-                // (fp32: one sum of all rows - plain adds, no packing to gain, and two sums fewer to hold)
-                constexpr int kGroup = sizeof(T) == 4 ? ND : 3;
-                Slice<T, D> vec_sum[(ND + kGroup - 1) / kGroup];
+                // lanes that share an owned voxel saw alternate elements of the stream
+                for (int other = 1; other < (1 << gshift); other <<= 1) {
 #pragma unroll
-                for (int n = 0; n < ND; ++n) {
-                    Slice<T, D> vec_r;       // Tk, or Tq
-                    vec_r.load_lds(off[n] + hh * kHeadBytes);
-                    if constexpr (!kKeyOwned) {
-                        Slice<T, D> tk_r, tv_r;
-                        tk_r.load_lds(off[n] + hh * kHeadBytes + D * sizeof(T));
-                        tv_r.load_lds(off[n] + hh * kHeadBytes + 2 * D * sizeof(T));
-                        if (Slice<T, D>::kChainLogit) logit = st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, logit));
-                        else logit += st_x[hh].dot(tk_r, own_x[hh].dot(vec_r, 0.0f));
-                        if (Slice<T, D>::kChainLogit) dp = own_y[hh].dot(tv_r, dp);
-                        else dp += own_y[hh].dot(tv_r, 0.0f);
-                    }
-                    if (n % kGroup == 0) vec_sum[n / kGroup] = vec_r;
-                    else vec_sum[n / kGroup].add(vec_r);
-                }
-                float p, dl;
-                if constexpr (kKeyOwned) {
-                    p = valid ? rec[hh].y : 0.0f;
-                    dl = valid ? rec[hh].x : 0.0f;
-                } else {
-                    p = valid ? __expf(logit - own_m[hh]) * own_inv[hh] : 0.0f;
-                    dl = p * (dp - own_delta[hh]);
-                }
-                // dq_i += dL (k_j + Tq)   or   dk_j += dL (q_i + Tk)
-                st_x[hh].fma_to(res_x[hh], dl);
-#pragma unroll
-                for (int g = 0; g < (ND + kGroup - 1) / kGroup; ++g) vec_sum[g].fma_to(res_x[hh], dl);
-                if constexpr (kKeyOwned) st_y[hh].fma_to(res_y[hh], p);     // dv_j += P dout_i
-                if constexpr (!kKeyOwned) {
-                    if (valid) b.pd[head_at + static_cast<int64_t>(st_in) * n_w + own_in] = make_float2(dl, p);
-                }
-            }
-        }
-        if constexpr (kOnlyRecords) continue;
-#pragma unroll
-        for (int hh = 0; hh < HP; ++hh) {
-            // lanes that share an owned voxel saw alternate elements of the stream
-            for (int other = 1; other < (1 << gshift); other <<= 1) {
-#pragma unroll
-                for (int c = 0; c < D; ++c) res_x[hh][c] += __shfl_xor(res_x[hh][c], other);
-                if constexpr (kKeyOwned) {
-#pragma unroll
-                    for (int c = 0; c < D; ++c) res_y[hh][c] += __shfl_xor(res_y[hh][c], other);
-                }
-            }
-            if (own_valid && sub == 0) {
-                // a window beyond the caller's pair store was skipped: its rows say so
-                if (!fits) {
-#pragma unroll
-                    for (int c = 0; c < D; ++c) res_x[hh][c] = __int_as_float(0x7fc00000);
+                    for (int c = 0; c < D; ++c) res_x[hh][c] += __shfl_xor(res_x[hh][c], other);
                     if constexpr (kKeyOwned) {
 #pragma unroll
-                        for (int c = 0; c < D; ++c) res_y[hh][c] = __int_as_float(0x7fc00000);
+                        for (int c = 0; c < D; ++c) res_y[hh][c] += __shfl_xor(res_y[hh][c], other);
                     }
                 }
-                const int64_t at_row = static_cast<int64_t>(own_row) * b.grad_stride + (h + hh) * D;
-                if constexpr (kKeyOwned) {
-                    store_row<D>(static_cast<TF *>(b.dk) + at_row, res_x[hh]);
-                    store_row<D>(static_cast<TF *>(b.dv) + at_row, res_y[hh]);
-                } else {
-                    store_row<D>(static_cast<TF *>(b.dq) + at_row, res_x[hh]);
+                if (own_valid && sub == 0) {
+                    // a window beyond the caller's pair store was skipped: its rows say so
+                    if (!fits) {
+#pragma unroll
+                        for (int c = 0; c < D; ++c) res_x[hh][c] = __int_as_float(0x7fc00000);
+                        if constexpr (kKeyOwned) {
+#pragma unroll
+                            for (int c = 0; c < D; ++c) res_y[hh][c] = __int_as_float(0x7fc00000);
+                        }
+                    }
+                    const int64_t at_row = static_cast<int64_t>(own_row) * b.grad_stride + (h + hh) * D;
+                    if constexpr (kKeyOwned) {
+                        store_row<D>(static_cast<TF *>(b.dk) + at_row, res_x[hh]);
+                        store_row<D>(static_cast<TF *>(b.dv) + at_row, res_y[hh]);
+                    } else {
+                        store_row<D>(static_cast<TF *>(b.dq) + at_row, res_x[hh]);
+                    }
                 }
             }
         }
