@@ -20,7 +20,7 @@ struct AttnArgs {
     float *out_max, *out_sum;              // [N,H] or null
     void *workspace;                       // the work list: queue counters, unit and window records
     int32_t block_shift;                   // the step target, a lane streams about 2^block_shift keys
-    int32_t target_items;                  // wavefronts that serve one head group (sizes the finer units at the list's end)
+    int32_t target_items;                  // wavefronts a head group's list is cut for (sizes the finer units at its end)
     int32_t leave_to_tiles;                // sizes_dev: the tile or strip kernel was launched too and serves sizes that fit it
     int32_t set_groups;                    // workgroups that come in runs of eight to a head group (the others in turn)
     int32_t H, D, nd, total_rows;

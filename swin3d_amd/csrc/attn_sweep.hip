@@ -420,12 +420,12 @@ int launch_records_lists(const tile::StripSetup &strips, const AttnArgs &a, bool
     return S3D_OK;
 }
 
-// Which head group a workgroup serves, for its whole life, and which of its workgroups it is.  Workgroups go to the XCDs in turn: runs of eight consecutive ones serve
-// one head group, as far as whole sets of (XCDs x head groups) go, so that every XCD serves every head group and the rows of a
-// unit reach one L2; the head groups take the workgroups behind those in turn.  (All in turn, an even number of head groups meets
-// only some of the XCDs: 199,327 voxels x 6 heads of 8 200 -> 215 us.  Without the ones behind, sixteen of 256 CUs had no workgroup
-// at 6, 10, 12 and 20 heads of 16: with them 149,993 x 10 1036 -> 1018 us, 49,682 x 6 278 -> 271, 37,485 x 20 664 -> 651.  At 24
-// and 40 heads, all of whose workgroups came in turn, 9,000 x 24 285 -> 266, 9,400 x 40 443 -> 432.)
+// Which head group a workgroup serves, for its whole life, and which of its workgroups it is.  Workgroups go to the XCDs in turn:
+// runs of eight consecutive ones serve one head group, as far as whole sets of (XCDs x head groups) go, so that every XCD serves
+// every head group and the rows of a unit reach one L2; the head groups take the workgroups behind those in turn.  (All in turn, an
+// even number of head groups meets only some of the XCDs: 199,327 voxels x 6 heads of 8 200 -> 215 us.  Without the ones behind,
+// sixteen of 256 CUs had no workgroup at 6, 10, 12 and 20 heads of 16: with them 149,993 x 10 1036 -> 1018 us, 49,682 x 6 278 -> 271,
+// 37,485 x 20 664 -> 651.  At 24 and 40 heads, all of whose workgroups came in turn, 9,000 x 24 285 -> 266, 9,400 x 40 443 -> 432.)
 struct GroupPlace {
     int head_group, nth, of;       // its workgroups are numbered
     __device__ __forceinline__ GroupPlace(const AttnArgs &a, int groups)
@@ -436,13 +436,19 @@ struct GroupPlace {
         of = static_cast<int>(gridDim.x) / groups;
     }
 };
-// The units of a head group, by queues, of which a wavefront starts on that of its XCD (as a rule: blocks go to the XCDs in turn).
+// The units of a head group, by queues, of which a wavefront starts on that of its workgroup's number: its XCD's, for workgroups of
+// whole sets; those behind them need not meet theirs.  (By the number and not by the XCD's register, so that a wavefront's own unit is
+// one no other has.)
 // In launches of up to two units a wavefront the first one is the wavefront's own: the first four wavefronts of all workgroups
 // come before their next four, so that all CUs get some, long ones and short ones.  By tickets alone the workgroups that had
 // their tables first took more than their share.  us by tickets / so, 9 axes, fp16: 20,001 voxels x 6 heads of 8 70.1 / 55.7,
-// 50,001 x 6 96.3 / 79.8, 2,003 x 10 49.5 / 42.1, 9,001 x 12 of 16 148.4 / 145.2; fp32 20,001 x 6 of 8 83.4 / 68.2.  Where there are more units,
-// tickets leave those of a window to one CU's wavefronts, whose lines they share: 12,421 x 12 of 16 174, all first units given 185.
-// (One wavefront at a time instead of four 54.6 and 183.5 at the first and the last of these; six 70 and 185.)
+// 50,001 x 6 96.3 / 79.8, 2,003 x 10 49.5 / 42.1, 9,001 x 12 of 16 148.4 / 145.2; fp32 20,001 x 6 of 8 83.4 / 68.2.  Where there are
+// more units, tickets leave those of a window to one CU's wavefronts, whose lines they share: 12,421 x 12 of 16 174, all first units
+// given 185.  (One wavefront at a time instead of four 54.6 and 183.5 at the first and the last of these; six 70 and 185.)
+// Another stream's work can keep a workgroup, and its units, from a CU.  Calls on two streams at once, us a pair, by tickets / so: two
+// of 20,001 x 6 87.0 / 83.0, two of 50,001 x 6 146.4 / 149.5, two of 9,001 x 12 of 16 266.0 / 263.8, in fp32 two of 20,001 x 6 107.9 /
+// 112.6; beside products of 50,000 x 192 x 192 50,001 x 6 94.8 / 87.1, 20,001 x 6 71.7 / 71.9; 20,001 x 6 beside copies 96.5 / 88.2,
+// beside 149,993 x 10 of 16 998 / 998, beside a call with gradients 358 / 354.
 template <int kWaves> struct UnitQueues {
     static constexpr int kSide = kWaves % 4 == 0 ? 4 : 1;
     int *counters;
@@ -494,9 +500,11 @@ int place_groups(AttnArgs &a, int slots, int groups, int threads, bool whole_set
 // Workgroup shapes.  A workgroup holds its heads' table slices once: up to head_dim 16 one of twelve wavefronts a CU, three per SIMD
 // with 168 registers (fp16 75 KB of tables for two heads of 16, 45 for three of 8; fp32 65 for two heads of 8, 75 for one of 16).
 // With the rows read ahead three wavefronts hide what four hid, and the tables are staged once: against four workgroups of four
-// wavefronts at head_dim 8 with one and two heads, fp16, 9 axes, us 595,677 voxels x 10 heads 918 / 919, 100,003 x 10 213 / 200, 20,003 x 10
-// 87 / 72, 2,003 x 10 76 / 50, 100,003 x 5 138 / 123, fp32 20,001 x 5 77 / 54; two of eight, three or four per SIMD, 978 and 939 at
-// 595,677; two of eight for pairs of heads in fp32 330 for 299 (199,327 x 6).  Two of six at head_dim 16 25 % slower than one of twelve.
+// wavefronts at head_dim 8 with one and two heads, fp16, 9 axes, us 595,677 voxels x 10 heads 918 / 919, 100,003 x 10 213 / 200,
+// 20,003 x 10 87 / 72, 2,003 x 10 76 / 50, 100,003 x 5 138 / 123, fp32 20,001 x 5 77 / 54; two of eight, three or four per SIMD, 978
+// and 939 at 595,677; two of eight for pairs of heads in fp32 330 for 299 (199,327 x 6).  Two of six at head_dim 16 25 % slower than
+// one of twelve.  fp16, one head of 16 a wavefront, which reads nothing ahead, three workgroups of four / one of twelve: 9,001 x 15
+// 213 / 199, 60,001 x 5 298 / 294, 20,001 x 5 138 / 136, 150,001 x 3 390 / 388, with six axes 150,001 x 5 435 / 434.
 // head_dim 32 (an fp32 query, key, value and output row are 128 registers): two of four wavefronts in fp16, one of eight in fp32
 // (125 KB of tables).
 template <typename T, int D> __host__ __device__ constexpr int group_threads() { return D <= 16 ? 768 : sizeof(T) == 4 ? 512 : 256; }
@@ -1391,7 +1399,7 @@ int launch_sweep(const AttnArgs &a, hipStream_t stream, int what)
     // addresses of a pair are spent once for both.  At head_dim 16 that means one workgroup of twelve wavefronts per
     // CU (75 KB of tables): it measured -10 % at 6 heads.
     if constexpr (sizeof(T) == 2 && D <= 16) {
-        // three heads where they go in threes and fit (head_dim 8: 168 registers, three workgroups of 45 KB of
+        // three heads where they go in threes and fit (head_dim 8: 168 registers, one workgroup with 45 KB of
         // tables per CU): -2 % against pairs at 6 and 12 heads
         if constexpr (D == 8) {
             if (a.H % 3 == 0)
@@ -1447,7 +1455,8 @@ int launch_bwd_pairs(const BwdPairArgs &b0, hipStream_t stream)
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(q_sweep), q_lds)) return rc;
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(k_sweep), k_lds)) return rc;
     const int groups = a.H / HP;
-    // workgroups: as many as registers and the tables in LDS allow, in whole sets as the forward's
+    // workgroups: as many as registers and the tables in LDS allow, the query-owned sweep's placed as the forward's, the key-owned
+    // one's in whole sets
     auto with_grid = [&](BwdPairArgs &b, const void *kernel, size_t lds, int &grid, bool whole_sets) {
         int per_cu = 0;
         S3D_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, lds));
@@ -1493,8 +1502,9 @@ int launch_bwd_records(const BwdPairArgs &b0, const tile::StripSetup &strips, hi
 // Records alone, for the strips of attn_strip_bwd.hip (head_dim 8).  Bound by VALU issue, some 320 instructions a step of two
 // heads.  A call, forward included, us: 199,327 voxels in windows of 26, 6 heads, 9 axes, fp16 1475 with pairs of heads, 1465 with
 // three (6 axes, 60,001 voxels, 467 and 469.5); beside fp16 rows 1570, fp32 tables.  As one workgroup of 256 for each wavefront of a
-// SIMD 1482 and 1604, of 384 1551 and 1684; before rows and keys were read ahead, 1520 and 1700.  fp32 with 9 axes: 463 us the
-// sweep with one head, 489 with two (then two wavefronts a SIMD); with 6 axes 372 and 339.
+// SIMD 1482 and 1604, of 384 1551 and 1684; before rows and keys were read ahead, 1520 and 1700.  fp32, one head / two, 9 axes 40,001 x
+// 6 560 / 602, 20,001 x 6 338 / 385, windows of 57 60,001 x 10 1930 / 2079; 6 axes (two spill two registers) 485 / 473, 290 / 297,
+// 1633 / 1571; 3 axes 20,001 x 6 266 / 265, windows of 57 60,001 x 10 1368 / 1331.
 template <typename T, typename TF, int ND>
 int dispatch_bwd_records(const BwdPairArgs &b, const tile::StripSetup &strips, hipStream_t stream)
 {

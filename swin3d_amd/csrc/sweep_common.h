@@ -14,8 +14,9 @@ namespace sweep {
 // so a single counter per head bounds a launch of 50 000 units to 0.6 ms whatever the units cost.  Every head
 // has kQueues counters, each on a cache line of its own; unit u belongs to queue u % kQueues; a wavefront
 // draws from the queue it starts on and moves to the next one when that is empty.
-// The chip has eight XCDs with an L2 each: a wavefront starts on the queue of the XCD it runs on, so all heads
-// of a unit are served from the same XCD and the unit's q, k, v rows and coordinates reach that L2 once.
+// The chip has eight XCDs with an L2 each: a wavefront starts on the queue of the XCD it runs on (the table-gradient
+// kernels read which, the sweeps go by their workgroup's number, see there), so all heads of a unit are served from the
+// same XCD and the unit's q, k, v rows and coordinates reach that L2 once.
 constexpr int kQueues = 8;
 constexpr int kCounterStride = 64;   // ints between counters (256 bytes)
 
