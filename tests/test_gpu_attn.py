@@ -630,8 +630,8 @@ def test_sweep_where_the_first_keys_have_no_weight(oracle_lib, hip_lib, dtype, h
     # logits of up to some tens, off by their roundings
     some = np.isfinite(rmax)
     assert (np.isfinite(gmax) == some).all()
-    assert np.abs(gmax - rmax)[some].max() <= (1e-5 if dtype == torch.float32 else 1e-2) * max(1.0, np.abs(rmax[some]).max())
-    assert (np.abs(gsum - rsum)[some] <= (1e-4 if dtype == torch.float32 else 2e-2) * rsum[some]).all()
+    assert np.abs(gmax[some] - rmax[some]).max() <= (1e-5 if dtype == torch.float32 else 1e-2) * max(1.0, np.abs(rmax[some]).max())
+    assert (np.abs(gsum[some] - rsum[some]) <= (1e-4 if dtype == torch.float32 else 2e-2) * rsum[some]).all()
 
 
 @pytest.mark.parametrize("cRSE", ["XYZ", "XYZ_RGB", "XYZ_RGB_NORM"])
