@@ -445,6 +445,10 @@ struct GroupPlace {
 // 50,001 x 6 96.3 / 79.8, 2,003 x 10 49.5 / 42.1, 9,001 x 12 of 16 148.4 / 145.2; fp32 20,001 x 6 of 8 83.4 / 68.2.  Where there are
 // more units, tickets leave those of a window to one CU's wavefronts, whose lines they share: 12,421 x 12 of 16 174, all first units
 // given 185.  (One wavefront at a time instead of four 54.6 and 183.5 at the first and the last of these; six 70 and 185.)
+// The line at two: of 113 shapes of up to two units, 64 of them with more than one, 0.55 to 1.01 of the time by tickets, but fp16 with
+// three or six axes at 1.1 to 1.4 units takes 1.01 to 1.07 with 24 heads of 16 (2,701 voxels, six axes 99.9 / 107.1, nine 117.3 /
+// 114.2) and 1.02 to 1.05 with 12 (6,001).  A line at 9/8 for those takes some of that back and loses more elsewhere: 15,001 x 6 with six
+// axes, 1.56 units, 91 -> 102, 5,501 x 12 94 -> 97.5.
 // Another stream's work can keep a workgroup, and its units, from a CU.  Calls on two streams at once, us a pair, by tickets / so: two
 // of 20,001 x 6 87.0 / 83.0, two of 50,001 x 6 146.4 / 149.5, two of 9,001 x 12 of 16 266.0 / 263.8, in fp32 two of 20,001 x 6 107.9 /
 // 112.6; beside products of 50,000 x 192 x 192 50,001 x 6 94.8 / 87.1, 20,001 x 6 71.7 / 71.9; 20,001 x 6 beside copies 96.5 / 88.2,
